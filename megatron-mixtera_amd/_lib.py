@@ -135,6 +135,27 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+_native = None
+
+
+def native():
+    """The extension module ``_native`` (``csrc/host/native.cpp``), loaded and set up once."""
+    global _native
+    if _native is None:
+        load()
+        import torch
+        try:
+            from . import _native as module
+        except ImportError as e:
+            raise LibraryMissingError(
+                f"the native host module cannot be loaded ({e}): build it first (python {PKG_DIR / 'build.py'}); "
+                "there is no fallback path.") from e
+        from . import ops
+        module.setup(KernelError, torch._C._cuda_getCurrentRawStream, ops._grow_workspace)
+        _native = module
+    return _native
+
+
 def check(code: int, what: str) -> None:
     if code != 0:
         msg = load().mi_last_error().decode(errors="replace")

@@ -13,6 +13,7 @@ from typing import Optional, Tuple
 import torch
 from torch import Tensor
 
+from . import ops
 from .flash_attn_interface import (
     flash_attn_varlen_func,
     flash_attn_with_kvcache,
@@ -65,6 +66,13 @@ def flash_decode_and_prefill(q: Tensor, k: Tensor, v: Tensor, max_seqlen_q, max_
                                    k_scales=k_scales, v_scales=v_scales)
 
 
+def _parameter(module: torch.nn.Module, name: str) -> Optional[Tensor]:
+    """``getattr(module, name)``, found in the module's parameters first: the attribute protocol reaches them only
+    after a failed look-up, half a microsecond each."""
+    p = module._parameters.get(name)
+    return p if p is not None else getattr(module, name)
+
+
 class PagedSelfAttentionCore(torch.nn.Module):
     """Everything between ``get_query_key_value_tensors`` and ``linear_proj`` for one layer.
 
@@ -111,10 +119,7 @@ class PagedSelfAttentionCore(torch.nn.Module):
                 softmax_scale=self.softmax_scale, **self._norm_args())
             return out.reshape(out.size(0), out.size(1), -1)
         query = ctx.fused_qkv_norm_rope_append(
-            self.layer_number, mixed_qkv, num_query_heads=num_query_heads, rotary_pos_emb=emb, config=self.config,
-            q_weight=None if self.q_layernorm_weight is None else self.q_layernorm_weight.data,
-            k_weight=None if self.k_layernorm_weight is None else self.k_layernorm_weight.data,
-            norm=self.qk_norm, eps=self.eps)
+            self.layer_number, mixed_qkv, num_query_heads=num_query_heads, rotary_pos_emb=emb, **self._norm_args())
         return self._attend(query, ctx)
 
     def forward(self, query: Tensor, key: Tensor, value: Tensor, inference_context,
@@ -133,11 +138,8 @@ class PagedSelfAttentionCore(torch.nn.Module):
                 return out.reshape(out.size(0), out.size(1), -1)
             ctx.fused_qk_norm_rope_append(
                 self.layer_number, query, key, value, rotary_pos_emb=q_emb if q_emb is not None else k_emb,
-                config=self.config, q_weight=None if self.q_layernorm_weight is None else self.q_layernorm_weight.data,
-                k_weight=None if self.k_layernorm_weight is None else self.k_layernorm_weight.data,
-                norm=self.qk_norm, eps=self.eps)
+                **self._norm_args())
         else:
-            from . import ops
             if self.qk_norm is not None:
                 n = ctx.padded_active_token_count
                 ops.norm_rope_append(query[:n], key[:n], key_out=key[:n], norm=self.qk_norm, eps=self.eps,
@@ -152,8 +154,7 @@ class PagedSelfAttentionCore(torch.nn.Module):
 
     def _norm_args(self) -> dict:
         return dict(config=self.config, norm=self.qk_norm, eps=self.eps,
-                    q_weight=None if self.q_layernorm_weight is None else self.q_layernorm_weight.data,
-                    k_weight=None if self.k_layernorm_weight is None else self.k_layernorm_weight.data)
+                    q_weight=_parameter(self, "q_layernorm_weight"), k_weight=_parameter(self, "k_layernorm_weight"))
 
     def _step_fusable(self, ctx, emb: Optional[Tensor]) -> bool:
         """Decode-only steps over 16-bit caches run norm, RoPE, append and attention as one streaming kernel
@@ -195,14 +196,14 @@ class DecodeLinear(torch.nn.Module):
         self.bias = torch.nn.Parameter(torch.zeros(output_size, dtype=dtype, device=device)) if bias else None
 
     def forward(self, input_: Tensor):
-        from . import ops
-        add = None if (self.bias is None or self.skip_bias_add) else self.bias.data
+        weight, bias = _parameter(self, "weight"), _parameter(self, "bias")
+        add = None if self.skip_bias_add else bias
         rows = input_.numel() // input_.size(-1)
         if rows <= self.DECODE_ROWS:
-            output = ops.linear_decode(input_, self.weight.data, add)
+            output = ops.linear_decode(input_, weight, add)
         else:
-            output = torch.nn.functional.linear(input_, self.weight, add)
-        return output, (self.bias if self.skip_bias_add else None)
+            output = torch.nn.functional.linear(input_, weight, None if add is None else add.data)
+        return output, (bias if self.skip_bias_add else None)
 
 
 class PagedSelfAttentionLayer(torch.nn.Module):

@@ -22,6 +22,9 @@ LIB_PATH = PKG_DIR / LIB_NAME
 # measurement aids of bench.py (a streaming-read kernel); not part of the product library or its ABI
 BENCH_LIB_PATH = PKG_DIR / "libmi355_bench.so"
 
+# the host side of the hot calls: a Python module over the library (torch's headers, the CPython C API)
+NATIVE_PATH = PKG_DIR / "_native.so"
+
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
     "-O3",
@@ -69,10 +72,25 @@ def _hipcc(inputs: list[Path], output: Path, verbose: bool) -> None:
         _run([hipcc_path(), "--offload-arch=gfx950", "-shared", "-fPIC", *map(str, objects), "-o", str(output)], verbose)
 
 
+def _native_module(verbose: bool) -> None:
+    """``csrc/host/native.cpp`` -> ``_native.so``, linked against the library beside it.  Host code only."""
+    import sysconfig
+
+    import torch
+    root = Path(torch.__file__).resolve().parent
+    includes = [INCLUDE, root / "include", root / "include" / "torch" / "csrc" / "api" / "include", sysconfig.get_paths()["include"]]
+    cxx = os.environ.get("CXX") or shutil.which("g++") or "/opt/rocm/llvm/bin/clang++"
+    _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+          *[f"-I{i}" for i in includes], str(CSRC / "host" / "native.cpp"), "-o", str(NATIVE_PATH),
+          f"-L{PKG_DIR}", "-lmi355_decode", "-Wl,-rpath,$ORIGIN", f"-L{root / 'lib'}", "-ltorch", "-ltorch_cpu",
+          "-ltorch_python", "-lc10"], verbose)
+
+
 def build_library(verbose: bool = False) -> Path:
-    """Compile all kernels into ``libmi355_decode.so`` and the benchmark's measurement kernels into
-    ``libmi355_bench.so`` (always recompiles)."""
+    """Compile all kernels into ``libmi355_decode.so``, the host module ``_native.so`` over it and the benchmark's
+    measurement kernels into ``libmi355_bench.so`` (always recompiles)."""
     _hipcc(sources(), LIB_PATH, verbose)
+    _native_module(verbose)
     _hipcc(sorted((CSRC / "bench").glob("*.hip")), BENCH_LIB_PATH, verbose)
     return LIB_PATH
 

@@ -80,6 +80,11 @@ class WarmupEngineMode(Enum):
     NON_DECODE = "non_decode"
 
 
+def _first(rows: Tensor, n: int) -> Tensor:
+    """``rows[:n]``, without a new view when those are all rows."""
+    return rows if rows.size(0) == n else rows[:n]
+
+
 def _ceil_to(value: int, multiple: int) -> int:
     return multiple * int(math.ceil(int(value) / multiple))
 
@@ -411,6 +416,36 @@ class DynamicInferenceContext:
         return int(unfinished.sum().item())
 
     # ------------------------------------------------------------------ per-layer hot path
+    # The cache and its scales are properties so that the views every layer of every step asks for (two index calls of
+    # 2-3 us each) are made once per buffer; whoever assigns another buffer gets views of that one.
+    @property
+    def memory_buffer(self) -> Tensor:
+        return self._memory_buffer
+
+    @memory_buffer.setter
+    def memory_buffer(self, buffer: Tensor) -> None:
+        self._memory_buffer = buffer
+        self._cache_views = None
+
+    @property
+    def kv_scales(self) -> Optional[Tensor]:
+        return self._kv_scales
+
+    @kv_scales.setter
+    def kv_scales(self, scales: Optional[Tensor]) -> None:
+        self._kv_scales = scales
+        self._scale_views = None
+
+    def _layer_cache(self, layer_number: int) -> Tuple[Tensor, Optional[Tensor]]:
+        """Views of the layer's key and value cache (latent cache: its rows and ``None``)."""
+        views = self._cache_views
+        if views is None:
+            buf = self._memory_buffer
+            views = ([(latents, None) for latents in buf.unbind(0)] if self.cache_mla_latent
+                     else list(zip(buf[0].unbind(0), buf[1].unbind(0))))
+            self._cache_views = views
+        return views[layer_number - 1]
+
     def append_key_value_cache(self, layer_number: int, key: Tensor, value: Tensor) -> None:
         """Scatter this step's K/V rows into the layer's chunks (bit-exact copy).
 
@@ -420,36 +455,35 @@ class DynamicInferenceContext:
         n = self.padded_active_token_count
         if self.cache_mla_latent:
             # the caller passes kv_concat as the key; there is no value cache (reference: :533-538)
-            latent = key.squeeze(1) if key.dim() == 3 else key
-            ops.kv_append(latent[:n].unsqueeze(1), None, self.memory_buffer[layer_number - 1].unsqueeze(2), None,
+            latent = key if key.dim() == 3 else key.unsqueeze(1)
+            ops.kv_append(_first(latent, n), None, self._layer_cache(layer_number)[0].unsqueeze(2), None,
                           self.token_to_chunk_idx, self.token_to_local_position_within_kv_chunk)
             return
         assert key.size(1) == 1 and value.size(1) == 1
+        k_cache, v_cache = self._layer_cache(layer_number)
         if self.kv_cache_fp8:
+            k_scales, v_scales = self.key_value_scales(layer_number)
             ops.kv_append_fp8(
-                key[:n], value[:n],
-                self.memory_buffer[0, layer_number - 1], self.memory_buffer[1, layer_number - 1],
-                self.kv_scales[0, layer_number - 1], self.kv_scales[1, layer_number - 1],
+                _first(key, n), _first(value, n), k_cache, v_cache, k_scales, v_scales,
                 self.token_to_chunk_idx, self.token_to_local_position_within_kv_chunk,
                 headroom=self.fp8_append_headroom)
             return
-        ops.kv_append(
-            key[:n], value[:n],
-            self.memory_buffer[0, layer_number - 1], self.memory_buffer[1, layer_number - 1],
-            self.token_to_chunk_idx, self.token_to_local_position_within_kv_chunk)
+        ops.kv_append(_first(key, n), _first(value, n), k_cache, v_cache,
+                      self.token_to_chunk_idx, self.token_to_local_position_within_kv_chunk)
 
     def key_value_cache(self, layer_number: int) -> Tuple[Tensor, Tensor, Tensor]:
         """Views of the layer's key cache, value cache and this step's block table (latent cache: the
         layer's ``[chunks, tokens, rank + rope]`` buffer and ``None``)."""
-        if self.cache_mla_latent:
-            return (self.memory_buffer[layer_number - 1], None, self.block_table)
-        return (self.memory_buffer[0, layer_number - 1], self.memory_buffer[1, layer_number - 1], self.block_table)
+        return (*self._layer_cache(layer_number), self.block_table)
 
     def key_value_scales(self, layer_number: int) -> Tuple[Optional[Tensor], Optional[Tensor]]:
         """fp8 cache: the layer's key and value scales ``[chunks, heads]``; otherwise ``(None, None)``."""
         if not self.kv_cache_fp8:
             return None, None
-        return self.kv_scales[0, layer_number - 1], self.kv_scales[1, layer_number - 1]
+        views = self._scale_views
+        if views is None:
+            views = self._scale_views = list(zip(self._kv_scales[0].unbind(0), self._kv_scales[1].unbind(0)))
+        return views[layer_number - 1]
 
     @staticmethod
     def _rope_flags(config) -> bool:
@@ -507,12 +541,13 @@ class DynamicInferenceContext:
                 faithful_rounding=faithful_rounding)
             self.append_key_value_cache(layer_number, key_out, value[:n])
             return query
+        k_cache, v_cache = self._layer_cache(layer_number)
         ops.norm_rope_append(
-            query[:n], key[:n], value=value[:n], q_weight=q_weight, k_weight=k_weight, eps=eps, norm=norm,
+            _first(query, n), _first(key, n), value=_first(value, n), q_weight=q_weight, k_weight=k_weight, eps=eps, norm=norm,
             rotary_emb=rotary_pos_emb, q_positions=self.token_to_pos_ids,
             k_positions=self.token_to_position_in_request,
             rotary_interleaved=self._rope_flags(config) if config is not None else False, mscale=mscale,
-            k_cache=self.memory_buffer[0, layer_number - 1], v_cache=self.memory_buffer[1, layer_number - 1],
+            k_cache=k_cache, v_cache=v_cache,
             token_to_chunk_idx=self.token_to_chunk_idx,
             token_to_local_pos=self.token_to_local_position_within_kv_chunk,
             faithful_rounding=faithful_rounding)
@@ -556,14 +591,17 @@ class DynamicInferenceContext:
             common.update(k_scales=k_scales, v_scales=v_scales, headroom=self.fp8_append_headroom)
         if mixed_qkv is not None:
             d = self.kv_channels
-            out = torch.empty((mixed_qkv.size(0), 1, num_query_heads, d), dtype=mixed_qkv.dtype, device=mixed_qkv.device)
-            ops.decode_step_attention(None, None, None, k_cache, v_cache, self.kv_seq_lengths, block_table,
-                                      mixed_qkv=mixed_qkv[:n], num_query_heads=num_query_heads,
-                                      num_kv_heads=self.num_kv_heads_per_partition, out=out[:n], **common)
-            return out
+            out = None  # (made by the call when its rows are all of the step's)
+            if mixed_qkv.size(0) != n:
+                out = torch.empty((mixed_qkv.size(0), 1, num_query_heads, d), dtype=mixed_qkv.dtype, device=mixed_qkv.device)
+            got = ops.decode_step_attention(None, None, None, k_cache, v_cache, self.kv_seq_lengths, block_table,
+                                            mixed_qkv=_first(mixed_qkv, n), num_query_heads=num_query_heads,
+                                            num_kv_heads=self.num_kv_heads_per_partition,
+                                            out=None if out is None else out[:n], **common)
+            return got if out is None else out
         out = torch.empty_like(query)
-        ops.decode_step_attention(query[:n], key[:n], value[:n], k_cache, v_cache, self.kv_seq_lengths, block_table,
-                                  out=out[:n], **common)
+        ops.decode_step_attention(_first(query, n), _first(key, n), _first(value, n), k_cache, v_cache, self.kv_seq_lengths,
+                                  block_table, out=_first(out, n), **common)
         return out
 
     def fused_qkv_norm_rope_append(self, layer_number: int, mixed_qkv: Tensor, *, num_query_heads: int,
@@ -598,12 +636,13 @@ class DynamicInferenceContext:
             value = mixed_qkv[:n].reshape(n, hkv, (group + 2) * d)[:, :, (group + 1) * d:].contiguous()
             self.append_key_value_cache(layer_number, key_out, value.unsqueeze(1))
             return query_out
+        k_cache, v_cache = self._layer_cache(layer_number)
         ops.qkv_norm_rope_append(
-            mixed_qkv[:n], num_query_heads=num_query_heads, num_kv_heads=hkv, query_out=query_out[:n],
+            _first(mixed_qkv, n), num_query_heads=num_query_heads, num_kv_heads=hkv, query_out=_first(query_out, n),
             q_weight=q_weight, k_weight=k_weight, eps=eps, norm=norm, rotary_emb=rotary_pos_emb,
             q_positions=self.token_to_pos_ids, k_positions=self.token_to_position_in_request,
             rotary_interleaved=self._rope_flags(config) if config is not None else False, mscale=mscale,
-            k_cache=self.memory_buffer[0, layer_number - 1], v_cache=self.memory_buffer[1, layer_number - 1],
+            k_cache=k_cache, v_cache=v_cache,
             token_to_chunk_idx=self.token_to_chunk_idx,
             token_to_local_pos=self.token_to_local_position_within_kv_chunk,
             faithful_rounding=faithful_rounding)
