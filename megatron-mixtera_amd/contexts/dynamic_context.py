@@ -659,11 +659,11 @@ class DynamicInferenceContext:
         self.cu_kv_seq_lengths = None
         self.kv_seq_lengths = None
         self.block_table = None
-        self.cu_query_seq_lengths_cudagraph_only.fill_(0)
-        self.query_seq_lengths_cudagraph_only.fill_(0)
-        self.cu_kv_seq_lengths_cudagraph_only.fill_(0)
-        self.kv_seq_lengths_cudagraph_only.fill_(0)
-        self.request_to_kv_chunk_ids_cudagraph_only.fill_(0)
+        # (one launch for the five: every step of a serving loop comes through here)
+        torch._foreach_zero_([
+            self.cu_query_seq_lengths_cudagraph_only, self.query_seq_lengths_cudagraph_only,
+            self.cu_kv_seq_lengths_cudagraph_only, self.kv_seq_lengths_cudagraph_only,
+            self.request_to_kv_chunk_ids_cudagraph_only])
 
     def using_cuda_graph_this_step(self) -> bool:
         """Graph sizes exist, the step type may use them, and the batch fits the largest one."""
@@ -791,20 +791,16 @@ class DynamicInferenceContext:
         self.paused_tokens = None
 
         self.request_ids.fill_(-1)
-        self.request_query_lengths.fill_(0)
-        self.request_output_lengths.fill_(0)
-        self.request_kv_length_offsets.fill_(0)
-        self.request_kv_chunk_counts.fill_(0)
         self.request_last_kv_chunk_id.fill_(-1)
-        self.request_last_kv_chunk_offset.fill_(0)
         self.request_to_kv_chunk_ids.fill_(-1)
-
-        self.token_to_input_ids.fill_(0)
-        self.token_to_pos_ids.fill_(0)
         self.token_to_request_idx.fill_(-1)
-        self.token_to_position_in_request.fill_(0)
         self.token_to_chunk_idx.fill_(-1)
-        self.token_to_local_position_within_kv_chunk.fill_(0)
+        torch._foreach_zero_([
+            self.request_query_lengths, self.request_output_lengths, self.request_kv_length_offsets,
+            self.request_kv_chunk_counts, self.request_last_kv_chunk_offset])
+        torch._foreach_zero_([
+            self.token_to_input_ids, self.token_to_pos_ids, self.token_to_position_in_request,
+            self.token_to_local_position_within_kv_chunk])
 
         self.reset_attention_state()
         self.chunk_allocator.reset()
