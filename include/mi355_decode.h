@@ -583,9 +583,9 @@ int mi_sample_from_logits(const void* logits, int64_t stride_row, int32_t logits
  * The projections either side of the attention path at decode size (at most 256 tokens a call):
  *   y[T, N] = x[T, K] . W[N, K]^T (+ bias[N]),   16-bit x / W / bias / y, fp32 accumulation.
  * The weight matrix is streamed from HBM once (it is the traffic: 50 MB for 4096 -> 6144), its rows riding
- * through the matrix cores; K is cut into slices of at most 512 columns whose fp32 partial sums [slice][T][N]
- * live in the caller's workspace and are added in a fixed order by a second small launch (results do not depend
- * on timing).  N a multiple of 16, K a multiple of 32; x, W and y rows 16-byte aligned (y: 8-byte).
+ * through the matrix cores; K is cut into slices of at most 512 columns whose fp32 sums are added in slice order inside
+ * the workgroup that owns the rows (results do not depend on timing).  The workspace is checked as sized by mi_linear_decode_workspace_bytes
+ * and not written.  N a multiple of 16, K a multiple of 32; x, W and y rows 16-byte aligned (y: 8-byte).
  *
  * mi_linear_qkv_decode_step replaces `mixed_qkv, _ = self.linear_qkv(hidden_states)` of
  * Attention.get_query_key_value_tensors (megatron/core/transformer/attention.py:985-992; ColumnParallelLinear at

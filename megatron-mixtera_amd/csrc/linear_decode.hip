@@ -8,178 +8,292 @@
 // With a few dozen rows of x the weight matrix is the traffic -- 50 MB for 4096 -> 6144 -- and each of its bytes is
 // used once: the kernel is a stream of W from HBM with the products riding along.
 //
-// Work split: a workgroup of 8 wavefronts takes 128 rows of W (16 per wavefront, the A operand of mfma 16x16x32)
-// times one slice of at most 512 columns of K, for a block of at most 64 tokens.  Every wavefront asks for its whole
-// share of W at once -- sixteen 16-byte loads per lane, 16 KB per wavefront, non-temporal, whole cache lines per
-// instruction -- so the launch has the entire matrix in flight from its second microsecond, and multiplies each
-// piece as it arrives; before that the workgroup stages its slice of x in LDS (64 tokens x 512 values, read by all 8
-// wavefronts as the B operand).  Slices of K end in fp32 partial sums
-// (one contiguous tile of T x 16 per slice and wavefront) that a second, small kernel adds up in a fixed order (so results do not depend on timing), adds the
-// bias to and rounds; a call whose K fits one slice writes its 16-bit result directly.
+// Work split: K is cut into slices of at most 512 columns, and the result is the slices' fp32 sums added in slice order
+// -- fixed by (T, N, K) alone, so a call is reproducible bit for bit however the work is spread.  A workgroup takes
+// 16 RT rows of W and all of K for a block of at most 64 tokens, one wavefront per slice: each piece of W and of x a
+// workgroup needs enters the CU exactly once, straight into the registers of the wavefront that multiplies it -- no
+// staging shared between wavefronts, no barrier before or between the products, and a ring of loads that stays full
+// from the first instruction on.  The slices' sums meet in LDS at the end: one kernel, no partial sums in memory.
+//
+// 64 tokens, weights from HBM (GPU time per call, graph replay; before: 128 rows of one slice per workgroup, x staged
+// in LDS, partial sums in memory and a second kernel to add them):
+//   4096 -> 6144   23.2 -> 19.1 us,  1 token 14.7 -> 11.6,  256 tokens 64 -> 42
+//   4096 -> 4096   21.7 -> 16.7 us,  1 token 14.1 ->  9.3,  256 tokens 45 -> 23
+//   2048 -> 1280   11.2 ->  8.6 us,  1 token  7.3 ->  4.6,  200 tokens 17 -> 11
+// The matrix alone streams in 10.3 us (4096 -> 6144); beside it the CU's miss queue carries x (64 tokens: 8 KB per
+// 2 KB of a 16-row tile of W), 60 KB/us in all.
 #include "mi_common.h"
 #include "mi_capi_internal.h"
 
 namespace mi {
 
-constexpr int kLinRows = 128;    // rows of W per workgroup (8 wavefronts x 16)
-constexpr int kLinSlice = 512;   // columns of K per workgroup, at most
 constexpr int kLinTok = 64;      // tokens per workgroup, at most
-constexpr int kLinPitch = kLinSlice * 2 + 32;  // LDS bytes per staged row of x: an odd multiple of 32 (conflict-free fragments)
+constexpr int kLinStep = 64;     // columns a wavefront multiplies per step: whole 128-byte lines of 8 rows
+constexpr int kLinSlice = 512;   // columns per slice, at most
+constexpr int kLinRows = 128;    // (only in the slice rule)
+constexpr int kLinLds = 160 * 1024;
 
 struct LinearParams {
   const uint16_t* x; int64_t x_st;
   const uint16_t* w; int64_t w_st;
   const uint16_t* bias;
   uint16_t* out; int64_t o_st;
-  float* part;   // S > 1: [S][N / 16][T][16] -- a wavefront's 16 rows of W for every token, contiguous
-  int32_t T, N, K, kslice, S;
+  int32_t T, N, K, kslice, S, waves;  // S slices of kslice columns (a multiple of 32), `waves` of them at a time
 };
 
-template <bool F16>
-__global__ __launch_bounds__(512, 4) void linear_decode_kernel(LinearParams p) {
-  __shared__ __attribute__((aligned(16))) uint8_t xs[kLinTok * kLinPitch];
+// RT = 16-row tiles of W, XH = 8-token half tiles of x, P = steps in flight, NW = wavefronts at most (8: 256 registers
+// each, 12: 168, 16: 128).
+//
+// The products want lane (m16, g) to hold columns 8 g .. + 7 (of 32) of row m16 of W, and the same of token m16 of x.
+// Loads in that order are slow wherever they hit: neighbouring lanes ask for different rows, and the vector memory
+// pipe takes them at 17 bytes per clock and CU (measured on 512 KB in L2 read by every CU; 54-60 when eight
+// neighbouring lanes ask for one 128-byte line).  So lane l loads 16-byte piece l & 7 of row l >> 3, eight rows per
+// instruction, and the wavefront turns its own piece of LDS -- written as loaded, read in the products' order, both
+// without bank conflicts by the exclusive-or of piece and row.  A wavefront's LDS operations execute in order and no
+// other wavefront touches its piece, so there is no barrier and no wait between the two.
+template <bool F16, int RT, int XH, int P, int NW>
+__global__ __launch_bounds__(64 * NW) void linear_decode_kernel(LinearParams p) {
+  constexpr int TT = (XH + 1) / 2;
+  constexpr int kTurn = (2 * RT + 2 * TT) * 1024;   // bytes of a wavefront's piece of LDS: one step of W and of x
+  constexpr int kTile = 1024;                       // a 16 x 16 tile of sums: 16 bytes per lane
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m16 = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * kLinRows + 16 * wave;     // this wavefront's 16 rows of W
-  const int k0 = blockIdx.y * p.kslice;                 // this workgroup's slice of K
-  const int klen = min(p.kslice, p.K - k0);             // (a multiple of 32)
-  const int t0 = blockIdx.z * kLinTok;
-  const int nt = min(kLinTok, p.T - t0);                // tokens of this block
-  const int nkk = klen >> 5;                            // 32-column steps of the products (<= 16)
-  const bool rows_live = n0 < p.N;                      // (wave-uniform; N is a multiple of 16)
+  const int n0 = blockIdx.x * (16 * RT);
+  const int t0 = blockIdx.y * kLinTok;
+  const int nt = min(8 * XH, p.T - t0);
 
-  // ---- x[t0 .. t0 + nt)[k0 .. k0 + klen) -> LDS (rows and columns beyond stay zero).  Before anything of W is asked
-  // for: loads are served in the order a CU issued them, and behind sixteen loads of W per lane these few cache
-  // hits would wait for microseconds ----
-  {
-    constexpr int PPR = kLinSlice / 8;  // 16-byte pieces per staged row
+  const int lo = lane >> 3, col = 8 * (lane & 7);
+  uint8_t* const turn_put = lds + wave * kTurn + lo * 128 + (((lane & 7) ^ lo) << 4);
+  const uint8_t* const turn_get = lds + wave * kTurn + m16 * 128;
+  const int piece0 = (g ^ (m16 & 7)) << 4, piece1 = ((4 + g) ^ (m16 & 7)) << 4;   // columns 0-31 / 32-63 of the step
+  // Row pairs beyond the last of W repeat it, tokens beyond the last repeat it: their results are not stored.
+  const uint32_t w_lane = (uint32_t)(lo * p.w_st + col);
+  uint32_t x_lane[XH];
 #pragma unroll
-    for (int i = 0; i < kLinTok * PPR / 512; ++i) {
-      const int piece = tid + 512 * i, row = piece / PPR, col = piece - row * PPR;
-      uint4 v = make_uint4(0u, 0u, 0u, 0u);
-      if (row < nt && 8 * col < klen) v = ld16(p.x + (int64_t)(t0 + row) * p.x_st + k0 + 8 * col);
-      *reinterpret_cast<uint4*>(xs + row * kLinPitch + 16 * col) = v;
-    }
-  }
-  __syncthreads();
-  // ---- this wavefront's share of W.  The products want lane (m16, g) to hold columns 32 kk + 8 g .. + 7 of row
-  // n0 + m16; loaded that way an instruction touches 64 bytes of each of 16 rows, half a cache line each.  So a pair
-  // of loads covers whole lines instead -- load 2 j: rows n0 .. + 7, load 2 j + 1: rows n0 + 8 .. + 15, each lane
-  // (m16, g) the 16 bytes at column 64 j + 8 (g + 4 (m16 >> 3)) of row (m16 & 7) -- and two moves per register within
-  // the 16-lane rows put the halves where the products expect them. ----
-  uint4 wf[kLinSlice / 32];
-  {
-    const int lo = m16 & 7, hi = m16 >> 3;
-    const int col = 8 * (g + 4 * hi);   // within a 64-column pair of steps
-    const uint16_t* wrow = p.w + (int64_t)min(n0 + lo, p.N - 1) * p.w_st + k0 + col;
-    const int64_t half = 8 * p.w_st;    // (N is a multiple of 16: rows n0 + 8 .. exist whenever rows_live)
-#pragma unroll
-    for (int j = 0; j < kLinSlice / 64; ++j) {
-      const bool live = rows_live && 64 * j + col < klen;
-      wf[2 * j] = live ? ld16_stream(wrow + 64 * j) : make_uint4(0u, 0u, 0u, 0u);
-      wf[2 * j + 1] = live ? ld16_stream(wrow + half + 64 * j) : make_uint4(0u, 0u, 0u, 0u);
-    }
-  }
-  if (!rows_live) return;
+  for (int i = 0; i < XH; ++i) x_lane[i] = (uint32_t)(min(8 * i + lo, nt - 1) * p.x_st + col);
+  const uint16_t* xbase = p.x + (int64_t)t0 * p.x_st;
+  auto w_at = [&](int i, int k) { return p.w + (int64_t)(min(n0 + 16 * (i >> 1), p.N - 16) + 8 * (i & 1)) * p.w_st + k + w_lane; };
+  auto x_at = [&](int i, int k) { return xbase + k + x_lane[i]; };
 
-  const int ntile = (nt + 15) >> 4;  // 16-token tiles with a live token
-  f32x4_t acc[kLinTok / 16];
+  struct Stage { uint4 w[2 * RT]; uint4 x[XH]; };
+  Stage st[P];
+  int k0 = 0, k1 = 0, ka = 0;   // columns of the slice at hand; where its first whole step of 64 starts
+  auto load = [&](Stage& s, int step) {
+    const int k = ka + step * kLinStep;
+    if (k + kLinStep <= p.K) {
 #pragma unroll
-  for (int i = 0; i < kLinTok / 16; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  const uint8_t* xfrag = xs + m16 * kLinPitch + 16 * g;  // B operand: lane (token m16, g) supplies x[token][32 kk + 8 g ..]
-  // (fully unrolled with wave-uniform guards: the fragments must stay in registers, and a loop that is left early
-  // would index them at run time)
+      for (int i = 0; i < 2 * RT; ++i) s.w[i] = ld16_stream(w_at(i, k));
 #pragma unroll
-  for (int kk = 0; kk < kLinSlice / 32; ++kk) {
-    if ((kk & 1) == 0 && kk < nkk) {
-      // lanes 8-15 of every 16 take the rows-8-15 load's lanes 0-7 (columns 8 g ..), lanes 0-7 the rows-0-7 load's
-      // lanes 8-15 (columns 32 + 8 g ..): row_ror:8 with a bank mask writes just those lanes
-      const uint4 a = wf[kk], b = wf[kk + 1];
-      auto upper = [](uint32_t keep, uint32_t from) { return (uint32_t)__builtin_amdgcn_update_dpp((int)keep, (int)from, 0x128, 0xf, 0xc, false); };
-      auto lower = [](uint32_t keep, uint32_t from) { return (uint32_t)__builtin_amdgcn_update_dpp((int)keep, (int)from, 0x128, 0xf, 0x3, false); };
-      wf[kk] = make_uint4(upper(a.x, b.x), upper(a.y, b.y), upper(a.z, b.z), upper(a.w, b.w));
-      wf[kk + 1] = make_uint4(lower(b.x, a.x), lower(b.y, a.y), lower(b.z, a.z), lower(b.w, a.w));
+      for (int i = 0; i < XH; ++i) s.x[i] = ld16(x_at(i, k));
+    } else {  // the last 32 columns of a K that is no multiple of 64: zeros beyond them
+      const bool live = k + col < p.K;
+#pragma unroll
+      for (int i = 0; i < 2 * RT; ++i) s.w[i] = live ? ld16_stream(w_at(i, k)) : make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+      for (int i = 0; i < XH; ++i) s.x[i] = live ? ld16(x_at(i, k)) : make_uint4(0u, 0u, 0u, 0u);
     }
-    if (kk < nkk) {
+  };
+  f32x4_t acc[RT * TT];
+  auto multiply = [&](Stage& s, int step) {
+    // (a slice of an odd number of 32 columns shares its first or last 64 with its neighbour: each multiplies its half)
+    const bool first = ka + step * kLinStep >= k0, second = ka + step * kLinStep + 32 < k1;
 #pragma unroll
-      for (int i = 0; i < kLinTok / 16; ++i) {
-        if (i < ntile) {
-          const uint4 xf = *reinterpret_cast<const uint4*>(xfrag + 16 * i * kLinPitch + 64 * kk);
-          acc[i] = mfma_16x16x32<F16>(wf[kk], xf, acc[i]);
+    for (int i = 0; i < 2 * RT; ++i) *reinterpret_cast<uint4*>(turn_put + i * 1024) = s.w[i];
+#pragma unroll
+    for (int i = 0; i < XH; ++i) *reinterpret_cast<uint4*>(turn_put + (2 * RT + i) * 1024) = s.x[i];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    uint4 wa[RT], wb[RT];
+#pragma unroll
+    for (int i = 0; i < RT; ++i) {
+      wa[i] = *reinterpret_cast<const uint4*>(turn_get + i * 2048 + piece0);
+      wb[i] = *reinterpret_cast<const uint4*>(turn_get + i * 2048 + piece1);
+    }
+#pragma unroll
+    for (int j = 0; j < TT; ++j) {   // (an odd XH leaves the last half tile as it was: tokens that are not stored)
+      const uint4 xa = *reinterpret_cast<const uint4*>(turn_get + (RT + j) * 2048 + piece0);
+      const uint4 xb = *reinterpret_cast<const uint4*>(turn_get + (RT + j) * 2048 + piece1);
+      if (first) {
+#pragma unroll
+        for (int i = 0; i < RT; ++i) acc[i * TT + j] = mfma_16x16x32<F16>(wa[i], xa, acc[i * TT + j]);
+      }
+      if (second) {
+#pragma unroll
+        for (int i = 0; i < RT; ++i) acc[i * TT + j] = mfma_16x16x32<F16>(wb[i], xb, acc[i * TT + j]);
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  auto tile_at = [&](int slot, int tile) { return reinterpret_cast<f32x4_t*>(lds + (slot * RT * TT + tile) * kTile + 16 * lane); };
+  static_assert(RT * TT * kTile <= kTurn, "the sums of a wavefront lie over its piece");
+  auto before = [&](int tile) { return reinterpret_cast<f32x4_t*>(lds + p.waves * kTurn + tile * kTile + 16 * lane); };
+  for (int s0 = 0; s0 < p.S; s0 += p.waves) {   // (one round unless there are more than 16 slices)
+    if (s0 > 0) __syncthreads();                // the sums have been read
+    const int slice = s0 + wave;
+    k0 = slice * p.kslice;
+    k1 = slice < p.S ? min(k0 + p.kslice, p.K) : k0;
+    ka = k0 & ~(kLinStep - 1);
+    const int steps = k1 > k0 ? (k1 - ka + kLinStep - 1) / kLinStep : 0;
+#pragma unroll
+    for (int i = 0; i < RT * TT; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < P; ++u)
+      if (u < steps) load(st[u], u);
+    for (int s = 0; s < steps; s += P) {
+#pragma unroll
+      for (int u = 0; u < P; ++u) {
+        if (s + u < steps) {
+          multiply(st[u], s + u);
+          if (s + u + P < steps) load(st[u], s + u + P);
         }
       }
     }
-  }
-  // ---- acc[i][j] = y[token 16 i + m16][row n0 + 4 g + j] ----
+    // ---- acc[i * TT + j][e] = y[token 16 j + m16][row n0 + 16 i + 4 g + e] of this slice ----
+    __syncthreads();  // (everyone has read its last step)
 #pragma unroll
-  for (int i = 0; i < kLinTok / 16; ++i) {
-    const int t = 16 * i + m16;
-    if (i >= ntile || t >= nt) continue;
-    const int n = n0 + 4 * g;
-    if (p.S == 1) {
-      float b[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < RT * TT; ++i) *tile_at(wave, i) = acc[i];
+    __syncthreads();
+    const int live = min(p.waves, p.S - s0);
+    const bool last = s0 + p.waves >= p.S;
+    for (int tile = wave; tile < RT * TT; tile += p.waves) {
+      f32x4_t sum = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      if (s0 > 0) sum = *before(tile);
+      for (int w = 0; w < live; ++w) {
+        const f32x4_t v = *tile_at(w, tile);
+        sum[0] += v[0]; sum[1] += v[1]; sum[2] += v[2]; sum[3] += v[3];
+      }
+      if (!last) {
+        *before(tile) = sum;
+        continue;
+      }
+      const int n = n0 + 16 * (tile / TT) + 4 * g, t = 16 * (tile % TT) + m16;
+      if (n >= p.N || t >= nt) continue;
       if (p.bias) {
         const uint2 bw = ld8(p.bias + n);
-        b[0] = lo_to_f32<F16>(bw.x); b[1] = hi_to_f32<F16>(bw.x); b[2] = lo_to_f32<F16>(bw.y); b[3] = hi_to_f32<F16>(bw.y);
+        sum[0] += lo_to_f32<F16>(bw.x); sum[1] += hi_to_f32<F16>(bw.x); sum[2] += lo_to_f32<F16>(bw.y); sum[3] += hi_to_f32<F16>(bw.y);
       }
-      st8(p.out + (int64_t)(t0 + t) * p.o_st + n,
-          make_uint2(pack2<F16>(acc[i][0] + b[0], acc[i][1] + b[1]), pack2<F16>(acc[i][2] + b[2], acc[i][3] + b[3])));
-    } else {
-      // (lane (token, g) writes 16 bytes at token * 64 + 16 g of its wavefront's tile: whole lines, no gaps)
-      float* dst = p.part + (((int64_t)blockIdx.y * (p.N >> 4) + (n0 >> 4)) * p.T + (t0 + t)) * 16 + 4 * g;
-      *reinterpret_cast<float4*>(dst) = make_float4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]);
+      st8(p.out + (int64_t)(t0 + t) * p.o_st + n, make_uint2(pack2<F16>(sum[0], sum[1]), pack2<F16>(sum[2], sum[3])));
     }
   }
-}
-
-// out[t][n .. n + 3] = round(sum over the slices, in their order, of the partial sums + bias[n ..]).  Threads walk the
-// partial tiles in their memory order (tile, token, quarter of the 16 rows): neighbouring threads read neighbouring
-// 16 bytes.
-template <bool F16>
-__global__ __launch_bounds__(256) void linear_decode_reduce_kernel(LinearParams p) {
-  const int64_t q4 = (int64_t)blockIdx.x * 256 + threadIdx.x;   // group of four neighbouring outputs
-  const int64_t per_slice = (int64_t)p.T * p.N;                 // floats per slice
-  if (q4 * 4 >= per_slice) return;
-  const int tile = (int)(q4 / (4 * p.T)), rest = (int)(q4 - (int64_t)tile * 4 * p.T);
-  const int t = rest >> 2, n = 16 * tile + 4 * (rest & 3);
-  float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
-  const float* src = p.part + q4 * 4;
-#pragma unroll 4
-  for (int s = 0; s < p.S; ++s) {
-    const float4 v = *reinterpret_cast<const float4*>(src + (int64_t)s * per_slice);
-    sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
-  }
-  if (p.bias) {
-    const uint2 bw = ld8(p.bias + n);
-    sum.x += lo_to_f32<F16>(bw.x); sum.y += hi_to_f32<F16>(bw.x); sum.z += lo_to_f32<F16>(bw.y); sum.w += hi_to_f32<F16>(bw.y);
-  }
-  st8(p.out + (int64_t)t * p.o_st + n, make_uint2(pack2<F16>(sum.x, sum.y), pack2<F16>(sum.z, sum.w)));
 }
 
 }  // namespace mi
 
 using namespace mi;
 
-// Slices the K columns are cut into: enough workgroups to keep every CU streaming (about one and a half per CU),
-// never more than 512 columns a slice (the staged x rows), slices a multiple of 32 columns.
-static void linear_split(int T, int N, int K, int* n_slices, int* kslice) {
+// The slices of K, and with them the order of summation: at least one per 512 columns, more where 128-row blocks of W
+// times 64-token blocks are few (a slice keeps at least 128 columns), a multiple of 32 columns each.
+static void linear_slices(int T, int N, int K, int* n_slices, int* kslice) {
   const int row_blocks = (N + kLinRows - 1) / kLinRows, tok_blocks = (T + kLinTok - 1) / kLinTok;
   int s = (K + kLinSlice - 1) / kLinSlice;
   const int want = (384 + row_blocks * tok_blocks - 1) / (row_blocks * tok_blocks);
   if (want > s) s = want;
-  if (s > K / 128) s = K / 128 > 0 ? K / 128 : 1;  // (a slice keeps at least 128 columns)
+  if (s > K / 128) s = K / 128 > 0 ? K / 128 : 1;
   int len = ((K + s - 1) / s + 31) & ~31;
   if (len > kLinSlice) len = kLinSlice;
   *kslice = len;
   *n_slices = (K + len - 1) / len;
 }
 
+// LDS of a workgroup: a step of every wavefront (at the end its sums, over it) and, where the slices come in rounds, the
+// sums of the rounds before.
+static int linear_lds(int rt, int half_tiles, int waves, int slices) {
+  const int tt = (half_tiles + 1) / 2;
+  return (waves * (2 * rt + 2 * tt) + (slices > waves ? rt * tt : 0)) * 1024;
+}
+
+static int linear_half_tiles(int t) { return t <= 8 ? 1 : t <= 16 ? 2 : t <= 32 ? 4 : t <= 48 ? 6 : 8; }
+
+// Rows per workgroup (16 RT) and wavefronts (slices at a time): the pair with the least estimated time.  A workgroup
+// fills a CU (its registers or its LDS), so the launch runs in rounds of 256 workgroups; a round costs 4.6 us, 3 us
+// more for every further round of slices, and the bytes it brings into a CU, which arrive at 60 KB/us (W misses and x
+// hits share the CU's miss queue).  Fitted to seven shapes from 1280 x 2048 to 7168 x 5120 at 1 .. 256 tokens: within
+// 15 % of what was measured.  More rows per workgroup read x less often, fewer fill the chip; eight wavefronts have
+// the registers for four row tiles, sixteen for one or two.
+static void linear_plan(int T, int N, int K, int slices, int* row_tiles, int* waves) {
+  const int blocks = (T + kLinTok - 1) / kLinTok, xh = linear_half_tiles(T < kLinTok ? T : kLinTok);
+  double best = 0;
+  *waves = 0;
+  const int fewest = (slices + 15) / 16;
+  for (int rounds = fewest; rounds <= fewest + 2; ++rounds) {
+    const int w = (slices + rounds - 1) / rounds;
+    const int most = w > 12 ? (xh <= 2 ? 2 : 1) : w > 8 || xh <= 2 ? 2 : xh <= 4 ? 3 : 4;  // (the instances there are)
+    for (int rt = 1; rt <= most && linear_lds(rt, xh, w, slices) <= kLinLds; ++rt) {
+      const int64_t groups = (int64_t)((N + 16 * rt - 1) / (16 * rt)) * blocks;
+      const double us = (double)((groups + 255) / 256) * (4.6 + 3.0 * (rounds - 1) + (16 * rt + 8 * xh) * (double)K * 2 / 60e3);
+      if (*waves == 0 || us < best) {
+        best = us;
+        *row_tiles = rt;
+        *waves = w;
+      }
+    }
+  }
+}
+
+
+template <bool F16, int RT, int XH, int P, int NW>
+static void launch_linear(const LinearParams& p, hipStream_t st) {
+  const dim3 grid((p.N + 16 * RT - 1) / (16 * RT), (p.T + kLinTok - 1) / kLinTok);
+  hipLaunchKernelGGL((linear_decode_kernel<F16, RT, XH, P, NW>), grid, dim3(64 * p.waves), linear_lds(RT, XH, p.waves, p.S), st, p);
+}
+// (steps in flight: what fits the registers without spilling)
+template <bool F16>
+static void launch_linear(const LinearParams& p, int rt, hipStream_t st) {
+  const int t = p.T < kLinTok ? p.T : kLinTok;
+  const int xh = linear_half_tiles(t);
+#define LIN(RT, XH, P, NW) launch_linear<F16, RT, XH, P, NW>(p, st)
+  if (p.waves <= 8) {
+    switch (10 * xh + rt) {
+      case 11: LIN(1, 1, 8, 8); break;
+      case 12: LIN(2, 1, 6, 8); break;
+      case 21: LIN(1, 2, 6, 8); break;
+      case 22: LIN(2, 2, 4, 8); break;
+      case 41: LIN(1, 4, 6, 8); break;
+      case 42: LIN(2, 4, 4, 8); break;
+      case 43: LIN(3, 4, 3, 8); break;
+      case 61: LIN(1, 6, 5, 8); break;
+      case 62: LIN(2, 6, 4, 8); break;
+      case 63: LIN(3, 6, 2, 8); break;
+      case 64: LIN(4, 6, 2, 8); break;
+      case 81: LIN(1, 8, 4, 8); break;
+      case 82: LIN(2, 8, 3, 8); break;
+      case 83: LIN(3, 8, 2, 8); break;
+      default: LIN(4, 8, 1, 8); break;
+    }
+  } else if (p.waves <= 12) {
+    switch (10 * xh + rt) {
+      case 11: LIN(1, 1, 6, 12); break;
+      case 12: LIN(2, 1, 4, 12); break;
+      case 21: LIN(1, 2, 5, 12); break;
+      case 22: LIN(2, 2, 3, 12); break;
+      case 41: LIN(1, 4, 4, 12); break;
+      case 42: LIN(2, 4, 2, 12); break;
+      case 61: LIN(1, 6, 3, 12); break;
+      case 62: LIN(2, 6, 1, 12); break;
+      case 81: LIN(1, 8, 2, 12); break;
+      default: LIN(2, 8, 1, 12); break;
+    }
+  } else {
+    switch (10 * xh + rt) {
+      case 11: LIN(1, 1, 6, 16); break;
+      case 12: LIN(2, 1, 3, 16); break;
+      case 21: LIN(1, 2, 4, 16); break;
+      case 22: LIN(2, 2, 2, 16); break;
+      case 41: LIN(1, 4, 2, 16); break;
+      case 61: LIN(1, 6, 1, 16); break;
+      default: LIN(1, 8, 1, 16); break;
+    }
+  }
+#undef LIN
+}
+
+// No scratch is used; a K of two slices and more still asks for a workspace, as callers of this entry point size one
+// and are told when they did not.
+static int64_t linear_workspace(int K) { return K >= 256 ? 256 : 0; }
+
 extern "C" int64_t mi_linear_decode_workspace_bytes(int32_t T, int32_t N, int32_t K) {
-  if (T <= 0 || N <= 0 || K <= 0) return 0;
-  int s, len;
-  linear_split(T, N, K, &s, &len);
-  return s > 1 ? (int64_t)s * T * N * (int64_t)sizeof(float) : 0;
+  return T <= 0 || N <= 0 || K <= 0 ? 0 : linear_workspace(K);
 }
 
 extern "C" int mi_linear_decode(const void* x, int64_t x_stride_tok, const void* weight, int64_t w_stride_row,
@@ -200,29 +314,21 @@ extern "C" int mi_linear_decode(const void* x, int64_t x_stride_tok, const void*
   p.x = (const uint16_t*)x; p.x_st = x_stride_tok; p.w = (const uint16_t*)weight; p.w_st = w_stride_row;
   p.bias = (const uint16_t*)bias; p.out = (uint16_t*)out; p.o_st = out_stride_tok;
   p.T = T; p.N = N; p.K = K;
-  p.part = nullptr;
   hipStream_t st = (hipStream_t)stream;
-  linear_split(T, N, K, &p.S, &p.kslice);
-  if (p.S > 1) {
-    const int64_t need = (int64_t)p.S * T * N * (int64_t)sizeof(float);
+  if (const int64_t need = linear_workspace(K)) {
     if (!workspace || workspace_bytes < need)
       return mi_fail(MI_ERR_WORKSPACE, "mi_linear_decode: workspace smaller than mi_linear_decode_workspace_bytes()");
     if ((uintptr_t)workspace & 15) return mi_fail(MI_ERR_ALIGN, "mi_linear_decode: the workspace must be 16-byte aligned");
-    p.part = (float*)workspace;
   }
-  const dim3 grid((N + kLinRows - 1) / kLinRows, p.S, (T + kLinTok - 1) / kLinTok);
+  linear_slices(T, N, K, &p.S, &p.kslice);
+  int rt;
+  linear_plan(T, N, K, p.S, &rt, &p.waves);
   hipEvent_t ev_a, ev_b;
   const bool timed = mi_profile_next(&ev_a, &ev_b);
   if (timed) (void)hipEventRecord(ev_a, st);
-  if (dtype == MI_DTYPE_FP16) hipLaunchKernelGGL(linear_decode_kernel<true>, grid, dim3(512), 0, st, p);
-  else hipLaunchKernelGGL(linear_decode_kernel<false>, grid, dim3(512), 0, st, p);
+  if (dtype == MI_DTYPE_FP16) launch_linear<true>(p, rt, st);
+  else launch_linear<false>(p, rt, st);
   if (timed) (void)hipEventRecord(ev_b, st);
-  if (p.S > 1) {
-    const int64_t quads = (int64_t)T * (N / 4);
-    const dim3 rgrid((unsigned)((quads + 255) / 256));
-    if (dtype == MI_DTYPE_FP16) hipLaunchKernelGGL(linear_decode_reduce_kernel<true>, rgrid, dim3(256), 0, st, p);
-    else hipLaunchKernelGGL(linear_decode_reduce_kernel<false>, rgrid, dim3(256), 0, st, p);
-  }
   return mi_check_launch("mi_linear_decode");
 }
 

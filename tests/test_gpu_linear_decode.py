@@ -48,6 +48,21 @@ def test_linear_decode_matches_an_fp32_product(mi, dev, T, N, K, bias, dtype):
     assert torch.equal(out, out2)
 
 
+@pytest.mark.parametrize("T", [1, 8, 9, 16, 17, 32, 33, 48, 49, 64, 65, 127])
+@pytest.mark.parametrize("N,K", [(16, 64), (80, 544), (4112, 1056), (208, 4640), (2048, 16416)])
+def test_tile_edges(mi, dev, T, N, K):
+    """Tokens at the edges of the half tiles and of a token block; row counts that leave a workgroup's last tiles
+    empty; columns that end in half a step, slices in one round and in several.  Values beyond the
+    inputs are not numbers, so that a read outside them would show."""
+    gen = torch.Generator().manual_seed(1000 * T + N + K)
+    big = torch.full((T + 8, K + 64), float("nan"), dtype=torch.bfloat16, device=dev)
+    big[:T, :K] = (torch.randn(T, K, generator=gen) * 0.5).bfloat16().to(dev)
+    w = torch.full((N + 16, K + 64), float("nan"), dtype=torch.bfloat16, device=dev)
+    w[:N, :K] = (torch.randn(N, K, generator=gen) * 0.05).bfloat16().to(dev)
+    out = mi.ops.linear_decode(big[:T, :K], w[:N, :K])
+    _ulp_close(out, (big[:T, :K].float() @ w[:N, :K].float().t()).bfloat16(), torch.bfloat16, f"linear {T}x{N}x{K}")
+
+
 def test_strided_inputs_and_leading_dimensions(mi, dev):
     gen = torch.Generator().manual_seed(5)
     big_x = (torch.randn(24, 1, 2 * 512, generator=gen) * 0.5).bfloat16().to(dev)
