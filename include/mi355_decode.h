@@ -580,6 +580,21 @@ int mi_sample_from_logits(const void* logits, int64_t stride_row, int32_t logits
                           uint8_t* active_request_mask, void* stream);
 
 /*
+ * The same call with scratch of mi_sample_workspace_bytes() bytes (256-byte aligned; 0: none is used): rows are then
+ * cut into parts that workgroups of their own read, in up to four launches.  Same samples, masks and cut values.  With
+ * workspace == NULL it is mi_sample_from_logits, one launch.
+ */
+int64_t mi_sample_workspace_bytes(int32_t R, int32_t vocab, int32_t top_k, float top_p);
+
+int mi_sample_from_logits_ws(const void* logits, int64_t stride_row, int32_t logits_dtype, int32_t R,
+                             int32_t vocab, int32_t top_k, float top_p, float temperature,
+                             const float* uniform, int32_t vocab_clamp, int64_t* samples,
+                             float* cut_values, const int32_t* request_kv_length_offsets,
+                             const int32_t* request_query_lengths, const int32_t* request_output_lengths,
+                             int64_t termination_id, uint8_t* active_request_mask, void* workspace,
+                             int64_t workspace_bytes, void* stream);
+
+/*
  * The projections either side of the attention path at decode size (at most 256 tokens a call):
  *   y[T, N] = x[T, K] . W[N, K]^T (+ bias[N]),   16-bit x / W / bias / y, fp32 accumulation.
  * The weight matrix is streamed from HBM once (it is the traffic: 50 MB for 4096 -> 6144), its rows riding

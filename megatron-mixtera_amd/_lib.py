@@ -89,6 +89,9 @@ SIGNATURES = {
     "mi_selected_log_probs": (c_int, [_P, _I64, _I32, _I32, _I32, _P, _P, _P]),
     "mi_sample_from_logits": (
         c_int, [_P, _I64, _I32, _I32, _I32, _I32, _F, _F, _P, _I32, _P, _P, _P, _P, _P, _I64, _P, _P]),
+    "mi_sample_workspace_bytes": (_I64, [_I32, _I32, _I32, _F]),
+    "mi_sample_from_logits_ws": (
+        c_int, [_P, _I64, _I32, _I32, _I32, _I32, _F, _F, _P, _I32, _P, _P, _P, _P, _P, _I64, _P, _P, _I64, _P]),
     "mi_norm_rope_append": (
         c_int,
         [_P, _I64, _P, _I64, _P, _I64, _P, _I64, _P, _I64, _P, _P, _F, _I32, _P, _I64, _I32, _I32, _F,

@@ -791,7 +791,8 @@ PyObject* linear_decode(PyObject* const* a) {
 }
 
 // sample_from_logits(logits, top_k, top_p, temperature, uniform|None, vocab_size, termination_id|None,
-//                    kv_length_offsets|None, query_lengths|None, output_lengths|None, return_cut)
+//                    kv_length_offsets|None, query_lengths|None, output_lengths|None, return_cut,
+//                    override|None)
 //   -> (samples, mask|None[, cut])
 PyObject* sample_from_logits(PyObject* const* a) {
   const Tensor& logits = tensor(a[0], "logits");
@@ -819,10 +820,16 @@ PyObject* sample_from_logits(PyObject* const* a) {
   if (masked) mask = at::empty({R}, logits.options().dtype(at::kByte));
   const bool want_cut = as_bool(a[10]);
   if (want_cut) cut = at::empty({R}, logits.options().dtype(at::kFloat));
-  check(mi_sample_from_logits(logits.data_ptr(), logits.stride(0), code, (int)R, (int)V, (int)top_k, (float)as_float(a[2]),
+  const float top_p = (float)as_float(a[2]);
+  // (a use_workspace buffer that is too small for the parts leaves the rows to one workgroup each)
+  const int64_t need = mi_sample_workspace_bytes((int)R, (int)V, (int)top_k, top_p);
+  Scratch ws;
+  if (a[11] == Py_None || tensor(a[11], "workspace").numel() >= need) ws = scratch(logits, stream, need, Py_None, a[11]);
+  check(mi_sample_from_logits_ws(logits.data_ptr(), logits.stride(0), code, (int)R, (int)V, (int)top_k, top_p,
                               (float)as_float(a[3]), (const float*)ptr(uniform), (int)as_int(a[5]), (int64_t*)samples.data_ptr(),
                               want_cut ? (float*)cut.data_ptr() : nullptr, (const int32_t*)ptr(lens[0]), (const int32_t*)ptr(lens[1]),
-                              (const int32_t*)ptr(lens[2]), masked ? as_int(a[6]) : -1, masked ? (uint8_t*)mask.data_ptr() : nullptr, stream),
+                              (const int32_t*)ptr(lens[2]), masked ? as_int(a[6]) : -1, masked ? (uint8_t*)mask.data_ptr() : nullptr,
+                                 ws.ptr, ws.bytes, stream),
         "mi_sample_from_logits");
   PyObject* m = masked ? wrap(mask) : same(Py_None);
   return want_cut ? Py_BuildValue("NNN", wrap(samples), m, wrap(cut)) : Py_BuildValue("NN", wrap(samples), m);
@@ -919,7 +926,7 @@ PyMethodDef kMethods[] = {
     ABI(mi_update_requests), ABI(mi_add_request), ABI(mi_decode_attention_state), ABI(mi_step_attention_state),
     OP(kv_append, 6), OP(kv_append_fp8, 9), OP(paged_decode_attention, 14), OP(paged_mla_decode_attention, 10),
     OP(paged_prefill_attention, 13), OP(paged_prefill_attention_mla, 11), OP(norm_rope_append, 22), OP(qkv_norm_rope_append, 22), OP(decode_step_attention, 29),
-    OP(linear_decode, 5), OP(sample_from_logits, 11), OP(selected_log_probs, 2), OP(last_token_gather, 3), OP(setup, 3),
+    OP(linear_decode, 5), OP(sample_from_logits, 12), OP(selected_log_probs, 2), OP(last_token_gather, 3), OP(setup, 3),
     OP(set_workspace, 3), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_native", "Host side of the per-layer calls.", -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 

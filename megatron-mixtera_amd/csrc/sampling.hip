@@ -196,12 +196,13 @@ static __device__ __forceinline__ void hist_add(uint64_t* hist, int bin, bool ac
   }
 }
 
-// Wave 0: first bin b (ascending) whose inclusive running sum, started at `above`, exceeds
+// Wave 0: first of the 64 N bins b (ascending) whose inclusive running sum, started at `above`, exceeds
 // `target`.  Writes {bin or -1, running sum before that bin} to res[0..1].
+template <int N = 4>
 static __device__ void find_crossing(const uint64_t* hist, uint64_t above, uint64_t target, uint64_t* res, int lane) {
-  uint64_t h[4], loc = 0;
+  uint64_t h[N], loc = 0;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) { h[j] = hist[4 * lane + j]; loc += h[j]; }
+  for (int j = 0; j < N; ++j) { h[j] = hist[N * lane + j]; loc += h[j]; }
   const uint64_t incl = wave_scan_incl_u64(loc, lane) + above;
   const bool cross = incl > target;
   const uint64_t m = __builtin_amdgcn_ballot_w64(cross);
@@ -211,15 +212,25 @@ static __device__ void find_crossing(const uint64_t* hist, uint64_t above, uint6
   }
   if (lane == __builtin_ctzll(m)) {
     uint64_t run = incl - loc;
-    int b = 4 * lane;
+    int b = N * lane;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < N; ++j) {
       if (run + h[j] > target) break;
       run += h[j];
       ++b;
     }
     res[0] = (uint64_t)b;
     res[1] = run;
+  }
+}
+
+static __device__ __forceinline__ void write_sample(const SampleParams& p, int r, int sample, uint32_t cut_key) {
+  p.samples[r] = sample;
+  if (p.cut_out) p.cut_out[r] = cut_key ? order_key_value(cut_key) : -INFINITY;
+  if (p.active_mask) {
+    bool active = (int64_t)sample != p.termination_id;
+    if (p.kv_off) active = active && (p.kv_off[r] + p.q_len[r] + 1 < p.out_len[r]);
+    p.active_mask[r] = active ? 1 : 0;
   }
 }
 
@@ -281,7 +292,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleParams p) 
       }
       __syncthreads();
       if (wave == 0) {  // the wavefront that reads the bins also clears them for the next digit: two barriers a pass
-        find_crossing(hist, above, target, res, lane);
+        find_crossing<4>(hist, above, target, res, lane);
 #pragma unroll
         for (int j = 0; j < 4; ++j) hist[4 * lane + j] = 0;
       }
@@ -469,7 +480,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleParams p) 
         for (int j = 0; j < 256; ++j) z += hist[j];  // same LDS words for every lane: broadcast reads
         target = (uint64_t)((double)p.top_p * (double)z);
       }
-      if (wave == 0) find_crossing(hist, 0, target, res, lane);
+      if (wave == 0) find_crossing<4>(hist, 0, target, res, lane);
       __syncthreads();
       const int lbin = (int)(int64_t)res[0];
       uint64_t above = res[1];
@@ -514,7 +525,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleParams p) 
             });
           }
           __syncthreads();
-          if (wave == 0) find_crossing(hist, above, target, res, lane);
+          if (wave == 0) find_crossing<4>(hist, above, target, res, lane);
           __syncthreads();
           // the crossing lies inside the chosen bin, so a digit is always found
           const uint32_t digit = 255u - (uint32_t)res[0];
@@ -637,14 +648,489 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleParams p) 
     if (p.vocab_clamp > 0) sample = min(max(sample, 0), p.vocab_clamp - 1);
   }
 
-  if (tid == 0) {
-    p.samples[r] = sample;
-    if (p.cut_out) p.cut_out[r] = cut_key ? order_key_value(cut_key) : -INFINITY;
-    if (p.active_mask) {
-      bool active = (int64_t)sample != p.termination_id;
-      if (p.kv_off) active = active && (p.kv_off[r] + p.q_len[r] + 1 < p.out_len[r]);
-      p.active_mask[r] = active ? 1 : 0;
+  if (tid == 0) write_sample(p, r, sample, cut_key);
+}
+
+// ---- the same over several workgroups per row -------------------------------------------------------------------
+// One workgroup per row leaves most of the chip idle while it walks the row up to five times (64 rows: 64 of 256 CUs;
+// 64 x 128 256 fp32, top-p 0.9 on flat rows: 105 us against 5 us for one read).  Here a row is cut into parts of one
+// workgroup each, and the walk into launches that read the parts once each:
+//   sample_first_kernel : a part's maximum (with its index); top-p: the part's mass in bins, in fp32 below a reference
+//                         that all parts of a row share; top-k: the part's candidates, listed (the elements at or above
+//                         a threshold estimated from 1 024 of them);
+//   sample_mass_kernel  : (top-p and plain draws) the exact masses: the part's total, and per run of elements what lies
+//                         above the bins that hold the cut; the elements in those bins, listed;
+//   sample_pick_kernel  : one workgroup per row: the exact cut among the listed elements, the run of elements the
+//                         uniform number falls into, the element.
+// Every mass is the integer of the one-workgroup form and every sum that decides is exact, so the tokens are the same
+// ones; the estimates only choose what is listed, and the pick checks them.  Where they fail (thousands of equal values,
+// more than the list holds) its workgroup walks the row instead of the list.
+//
+// fp32, 128 256 wide, us per call, one workgroup per row -> parts:
+//   64 rows: greedy 15 -> 12, plain 38 -> 24, top-k 50 39 -> 31, top-p 0.9 105 -> 44 (flat rows), 54 -> 41 (peaked)
+//    1 row : greedy 13 ->  8, plain 35 -> 15, top-k 50 36 -> 18, top-p 0.9 101 -> 25 (flat rows), 51 -> 24 (peaked)
+// 64 rows, top-p: 18 us for the first walk (vector arithmetic: 25 instructions per element), 15 for the second, 11 for
+// the pick (a chain of loads and barriers).
+constexpr int kBins = kSampleThreads; // 1/16 wide, from 24 above the reference to 40 below (and all that is lower)
+constexpr float kBinsAbove = 24.f, kBinsPerUnit = 16.f;
+constexpr int kRuns = kSampleWaves;   // runs of elements per part
+constexpr int kMaxParts = 64;
+constexpr int kPartSample = 1024;
+
+struct SplitParams {
+  SampleParams s;
+  int32_t parts, part_len, run_len;    // elements (multiples of 8); a part is kRuns runs
+  int32_t list_cap;                    // listed elements per part
+  uint32_t* part_key; int32_t* part_idx;  // [R][parts] maximum
+  uint32_t* part_tau;                  // [R][parts] top-k: the threshold of the part's candidates; top-p: the bins' upper edge
+  uint32_t* part_listed;               // [R][parts]
+  float* bins;                         // [R][parts][kBins]
+  uint64_t* part_mass;                 // [R][parts] exact total
+  uint64_t* run_mass;                  // [R][parts][kRuns] exact mass above the listed bins
+  uint2* list;                         // [R][parts][list_cap]: key, vocabulary index
+};
+
+template <int DT, int VEC>
+static __device__ __forceinline__ RowReader<DT, VEC> row_reader(const SampleParams& p, int r) {
+  return RowReader<DT, VEC>{reinterpret_cast<const uint8_t*>(p.logits) + (int64_t)r * p.stride * (DT != 0 ? 2 : 4), p.V,
+                            p.inv_temperature, p.top_k != 1 && p.inv_temperature != 1.0f};
+}
+
+// The row's maximum (lowest index among equals) from its parts', the same in every lane.
+struct RowMax { uint32_t key; int32_t idx; };
+static __device__ __forceinline__ RowMax row_max(const SplitParams& p, int r, int lane) {
+  RowMax m{0, 0x7fffffff};
+  if (lane < p.parts) {
+    const int64_t at = (int64_t)r * p.parts + lane;
+    m = RowMax{p.part_key[at], p.part_idx[at]};
+  }
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) {
+    const uint32_t ok = __shfl_xor(m.key, d, 64); const int oi = __shfl_xor(m.idx, d, 64);
+    if (ok > m.key || (ok == m.key && oi < m.idx)) { m.key = ok; m.idx = oi; }
+  }
+  if (m.idx >= p.s.V) m.idx = 0;  // only when no element compared greater than the start value
+  return m;
+}
+
+// The bin of a value, 0 = largest values; monotone.
+static __device__ __forceinline__ int ref_bin(float x, float top) {
+  const float f = (top - x) * kBinsPerUnit;
+  const int b = f >= (float)(kBins - 1) ? kBins - 1 : (int)f;  // NaN compares false and converts to 0
+  return b < 0 ? 0 : b;
+}
+// The upper edge of the bins: the reference -- the largest finite one of 1 024 elements spread over the row, the same
+// ones for every part -- plus 24.
+template <int DT, int VEC>
+static __device__ __forceinline__ float bins_top(const RowReader<DT, VEC>& rd, float* red, int tid, int lane, int wave) {
+  const int step = rd.V / kSampleThreads;
+  const float x = rd.at(tid * step);
+  float m = fabsf(x) < INFINITY ? x : -3.0e38f;
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) m = fmaxf(m, __shfl_xor(m, d, 64));
+  if (lane == 0) red[wave] = m;
+  __syncthreads();
+  m = red[0];
+#pragma unroll
+  for (int w = 1; w < kSampleWaves; ++w) m = fmaxf(m, red[w]);
+  return m + kBinsAbove;
+}
+
+// Appends one element per lane with `in` set to a list of `cap` entries; `count` goes on counting past it.
+template <typename F>
+static __device__ __forceinline__ void list_append(uint32_t* count, uint32_t cap, bool in, int lane, F store) {
+  const uint64_t m = __builtin_amdgcn_ballot_w64(in);
+  if (m == 0) return;
+  uint32_t base = 0;
+  const int first = __builtin_ctzll(m);
+  if (lane == first) base = atomicAdd(count, (uint32_t)__builtin_popcountll(m));
+  base = __builtin_amdgcn_readlane(base, first);
+  const uint32_t at = base + (uint32_t)__builtin_popcountll(m & (((uint64_t)1 << lane) - 1));
+  if (in && at < cap) store(at);
+}
+
+enum { kPickMax = 0, kPickTopK = 1, kPickTopP = 2 };
+
+template <int DT, int VEC, int MODE>
+__global__ __launch_bounds__(kSampleThreads) void sample_first_kernel(SplitParams p) {
+  __shared__ uint32_t red_key[kSampleWaves];
+  __shared__ int32_t red_idx[kSampleWaves];
+  __shared__ float red[kSampleWaves], red_low[kSampleWaves];
+  __shared__ uint64_t mass[MODE == kPickTopP ? kBins : 1];
+  __shared__ uint32_t sampled[MODE == kPickTopK ? kPartSample : 1];
+  __shared__ uint64_t hist[MODE == kPickTopK ? 256 : 1];
+  __shared__ uint64_t res[2];
+  __shared__ uint32_t listed;
+  const int part = blockIdx.x, r = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const auto rd = row_reader<DT, VEC>(p.s, r);
+  const int a = min(part * p.part_len, p.s.V), b = min(a + p.part_len, p.s.V);
+  const int64_t row_part = (int64_t)r * p.parts + part;
+  uint32_t tau = 0;
+  float top = 0.f;
+  if (MODE == kPickTopK) {
+    // threshold: a rank of the sample that leaves three times this part's share of the top k above it, and twelve
+    // of the sample at least (a dozen of it stand for 8-20 of the same spacing in all but a few of 10^5 parts)
+    const int len = b - a;
+    if (tid < kPartSample / 4) {
+      const int at = a + (int)((int64_t)tid * len / (kPartSample / 4));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) sampled[4 * tid + j] = order_key(rd.at(min(at + j, p.s.V - 1)));
     }
+    if (tid < 256) hist[tid] = 0;
+    if (tid == 0) listed = 0;
+    const int share = (3 * p.s.top_k + p.parts - 1) / p.parts;
+    const int rank = min(kPartSample / 2, max(12, (int)(((int64_t)share * kPartSample + len - 1) / max(len, 1))));
+    __syncthreads();
+    uint32_t pmask = 0;
+    uint64_t above = 0;
+    for (int d = 3; d >= 2; --d) {  // (the upper 16 bits of the key are enough)
+      const uint32_t k = sampled[tid];
+      hist_add(hist, 255 - (int)((k >> (8 * d)) & 255u), (k & pmask) == tau, lane, [&] { return (uint64_t)1; });
+      __syncthreads();
+      if (wave == 0) {
+        find_crossing<4>(hist, above, (uint64_t)(rank - 1), res, lane);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) hist[4 * lane + j] = 0;
+      }
+      __syncthreads();
+      above = res[1];
+      pmask |= 0xffu << (8 * d);
+      tau |= (255u - (uint32_t)res[0]) << (8 * d);
+    }
+  }
+  if (MODE == kPickTopP) {
+    mass[tid] = 0;
+    top = bins_top(rd, red, tid, lane, wave);  // (has the barrier)
+  }
+  const float ref_log2 = 26.f - (top - kBinsAbove) * 1.4426950408889634f;
+  uint2* list = p.list + row_part * p.list_cap;
+  uint32_t bk = 0; int bi = 0x7fffffff;
+  float low = 0.f;   // the last bin's: below it lies most of a flat row, and one address would take it all in turn
+  sweep<(VEC == 8 ? 4 : 8)>(rd, a, b, tid, kSampleThreads, [&](int i, float x, bool in) {
+    const uint32_t k = order_key(x);
+    const bool up = in && k > bk;
+    bk = up ? k : bk; bi = up ? i : bi;
+    if (MODE == kPickTopP && in) {
+      // in units of 2^-26 of the reference's (64-bit integer adds: LDS adds of fp32 ran at a fifth of their rate)
+      const float e = fast_exp2(fminf(__builtin_fmaf(x, 1.4426950408889634f, ref_log2), 62.f)) + 0.5f;
+      const int bin = ref_bin(x, top);
+      if (bin == kBins - 1) {
+        low += e;
+      } else {
+        const uint32_t hi = (uint32_t)(e * 0x1p-32f), lo = (uint32_t)__builtin_fmaf((float)hi, -0x1p32f, e);
+        atomicAdd(reinterpret_cast<unsigned long long*>(&mass[bin]), ((unsigned long long)hi << 32) | lo);
+      }
+    }
+    if (MODE == kPickTopK)
+      list_append(&listed, (uint32_t)p.list_cap, in && k >= tau, lane, [&](uint32_t at) { list[at] = make_uint2(k, (uint32_t)i); });
+  });
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) {
+    const uint32_t ok = __shfl_xor(bk, m, 64); const int oi = __shfl_xor(bi, m, 64);
+    if (ok > bk || (ok == bk && oi < bi)) { bk = ok; bi = oi; }
+  }
+  if (MODE == kPickTopP) {
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) low += __shfl_xor(low, m, 64);
+    if (lane == 0) red_low[wave] = low;
+  }
+  if (lane == 0) { red_key[wave] = bk; red_idx[wave] = bi; }
+  __syncthreads();
+  if (MODE == kPickTopP) {
+    float v = (float)mass[tid];
+    if (tid == kBins - 1)
+      for (int w = 0; w < kSampleWaves; ++w) v += red_low[w];
+    p.bins[row_part * kBins + tid] = v;
+  }
+  if (tid == 0) {
+    for (int w = 1; w < kSampleWaves; ++w) {
+      const uint32_t ok = red_key[w]; const int oi = red_idx[w];
+      if (ok > bk || (ok == bk && oi < bi)) { bk = ok; bi = oi; }
+    }
+    p.part_key[row_part] = bk; p.part_idx[row_part] = bi;
+    p.part_listed[row_part] = MODE == kPickTopK ? listed : 0;
+    p.part_tau[row_part] = MODE == kPickTopK ? tau : __float_as_uint(top);
+  }
+}
+
+// Exact masses.  top-p lists the bins [lo, hi] around the estimated cut; a plain draw (lo = kBins) lists nothing.
+template <int DT, int VEC>
+__global__ __launch_bounds__(kSampleThreads) void sample_mass_kernel(SplitParams p) {
+  __shared__ float red[kSampleWaves];
+  __shared__ int32_t window[2];
+  __shared__ uint64_t wsum[kSampleWaves];
+  __shared__ uint32_t listed;
+  const int part = blockIdx.x, r = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const RowMax m = row_max(p, r, lane);
+  const float mx = order_key_value(m.key), neg_mx = -mx * 1.4426950408889634f;
+  if (!(fabsf(mx) < INFINITY)) return;
+  const auto rd = row_reader<DT, VEC>(p.s, r);
+  const int64_t row_part = (int64_t)r * p.parts + part;
+  const bool filtered = p.s.top_p > 0.f;
+  float top = 0.f;
+  int lo = kBins, hi = kBins;
+  if (filtered) {
+    top = __uint_as_float(p.part_tau[row_part]);
+    // one bin per thread; the bin in which the running sum passes top_p of the total, with a neighbour where it passes
+    // within 3e-4 of the total of the edge
+    float h = 0.f;
+    const float* src = p.bins + (int64_t)r * p.parts * kBins + tid;
+#pragma unroll 4
+    for (int g = 0; g < p.parts; ++g) h += src[(int64_t)g * kBins];
+    float incl = h;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const float v = __shfl_up(incl, d, 64);
+      incl += lane >= d ? v : 0.f;
+    }
+    if (lane == 63) red[wave] = incl;
+    if (tid == 0) { window[0] = kBins - 1; window[1] = 0; listed = 0; }
+    __syncthreads();
+    float total = 0.f;
+#pragma unroll
+    for (int w = 0; w < kSampleWaves; ++w) {
+      incl += w < wave ? red[w] : 0.f;
+      total += red[w];
+    }
+    const float want = p.s.top_p * total, slack = 3e-4f * total;
+    if (incl - h - slack <= want && incl + slack > want && h > 0.f) {
+      atomicMin(&window[0], tid);
+      atomicMax(&window[1], tid);
+    }
+    __syncthreads();
+    lo = window[0]; hi = window[1];
+    if (lo > hi) lo = hi = kBins;   // nothing found (not a number somewhere): the pick walks the row
+  } else {
+    if (tid == 0) listed = 0;
+    __syncthreads();
+  }
+  const int pa = part * p.part_len, a = min(pa + wave * p.run_len, p.s.V), b = min(min(a + p.run_len, pa + p.part_len), p.s.V);
+  uint2* list = p.list + row_part * p.list_cap;
+  uint64_t all = 0, kept = 0;
+  sweep<(VEC == 8 ? 4 : 8)>(rd, a, b, lane, 64, [&](int i, float x, bool in) {
+    const uint64_t w = in ? mass_of(x, neg_mx) : 0;
+    all += w;
+    if (filtered) {
+      const int bin = ref_bin(x, top);
+      kept += bin < lo ? w : 0;
+      list_append(&listed, (uint32_t)p.list_cap, in && bin >= lo && bin <= hi, lane,
+                  [&](uint32_t at) { list[at] = make_uint2(order_key(x), (uint32_t)i); });
+    }
+  });
+  all = wave_sum_u64(all);
+  kept = filtered ? wave_sum_u64(kept) : all;
+  if (lane == 0) {
+    p.run_mass[row_part * kRuns + wave] = kept;
+    wsum[wave] = all;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    for (int w = 1; w < kSampleWaves; ++w) all += wsum[w];
+    p.part_mass[row_part] = all;
+    p.part_listed[row_part] = listed;
+  }
+}
+
+template <int DT, int VEC>
+__global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SplitParams p) {
+  const int r = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  __shared__ uint32_t key[kMemberCap];
+  __shared__ uint32_t mass[kMemberCap];     // (a mass fits 32 bits)
+  __shared__ uint32_t index[kMemberCap];
+  __shared__ uint64_t runs[kMaxParts * kRuns];
+  __shared__ uint64_t hist[512];
+  __shared__ uint64_t res[2];
+  __shared__ uint64_t wsum[3][kSampleWaves];
+  __shared__ uint32_t cut;
+  __shared__ int32_t pick;
+  const bool by_count = p.s.top_k > 1, by_mass = p.s.top_k == 0 && p.s.top_p > 0.f, filtered = by_count || by_mass;
+  const int64_t row = (int64_t)r * p.parts;
+  const int n_runs = p.parts * kRuns;
+  // (everything that does not depend on the maximum is asked for before it is waited for)
+  const int c = filtered && lane < p.parts ? (int)p.part_listed[row + lane] : 0;
+  uint32_t tau = by_count && lane < p.parts ? p.part_tau[row + lane] : 0;   // top-k: the list holds every element at or above it
+  uint64_t z = by_mass && tid < p.parts ? p.part_mass[row + tid] : 0;
+  const uint64_t run0 = p.s.top_k == 0 && tid < n_runs ? p.run_mass[row * kRuns + tid] : 0;
+  const RowMax m = row_max(p, r, lane);
+  const float mx = order_key_value(m.key), neg_mx = -mx * 1.4426950408889634f;
+  if (p.s.top_k == 1 || !(fabsf(mx) < INFINITY)) {
+    if (tid == 0) write_sample(p.s, r, m.idx, 0);
+    return;
+  }
+  const auto rd = row_reader<DT, VEC>(p.s, r);
+  // ---- the lists of the parts, one after the other: every wavefront copies some of them ----
+  int n = 0;
+  bool listed = true;
+  uint64_t in_list = 0;
+  if (filtered) {
+    int incl = c;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int v = __shfl_up(incl, d, 64);
+      incl += lane >= d ? v : 0;
+      tau = max(tau, (uint32_t)__shfl_xor((int)tau, d, 64));
+    }
+    n = __builtin_amdgcn_readlane(incl, 63);
+    listed = __builtin_amdgcn_ballot_w64(c > p.list_cap) == 0 && n <= kMemberCap;
+    for (int g = wave; g < p.parts && listed; g += kSampleWaves) {
+      const int mine = __builtin_amdgcn_readlane(c, g), at = __builtin_amdgcn_readlane(incl, g) - mine;
+      const uint2* src = p.list + (row + g) * p.list_cap;
+      for (int j = lane; j < mine; j += 64) {
+        const uint2 e = src[j];
+        const uint32_t w = (uint32_t)mass_of(order_key_value(e.x), neg_mx);
+        key[at + j] = e.x;
+        index[at + j] = e.y;
+        mass[at + j] = w;
+        in_list += w;
+      }
+    }
+  }
+  runs[tid] = run0;   // (n_runs <= the number of threads)
+  if (tid < 512) hist[tid] = 0;
+  if (tid == 0) { cut = 0; pick = m.idx; }
+  uint64_t above = 0, target = (uint64_t)(p.s.top_k - 1);
+  bool cuts = by_count;   // (a top-p of the whole mass cuts nothing)
+  if (by_mass) {
+    z = wave_sum_u64(z);
+    above = wave_sum_u64(run0);
+    in_list = wave_sum_u64(in_list);
+    if (lane == 0) { wsum[0][wave] = z; wsum[1][wave] = above; wsum[2][wave] = in_list; }
+    __syncthreads();
+    z = above = in_list = 0;
+#pragma unroll
+    for (int w = 0; w < kSampleWaves; ++w) { z += wsum[0][w]; above += wsum[1][w]; in_list += wsum[2][w]; }
+    target = (uint64_t)((double)p.s.top_p * (double)z);
+    cuts = z > target;
+    listed = listed && (!cuts || (above <= target && above + in_list > target));
+  } else {
+    listed = listed && (!by_count || n >= p.s.top_k);
+    __syncthreads();
+  }
+  // ---- the smallest kept key: the one with at most `target` of weight above it and more with itself ----
+  auto digits = [&](bool from_list) {
+    uint32_t pmask = 0, pval = 0;
+    uint64_t before = from_list ? above : 0;
+    for (int d = 3; d >= 0; --d) {
+      auto count = [&](uint32_t k, bool in, auto weight) {
+        hist_add(hist, 255 - (int)((k >> (8 * d)) & 255u), in && (k & pmask) == pval, lane, weight);
+      };
+      if (from_list) {
+        for (int j0 = 0; j0 < n; j0 += kSampleThreads) {
+          const int j = j0 + tid;
+          count(j < n ? key[j] : 0, j < n, [&]() -> uint64_t { return by_count ? 1u : mass[j]; });
+        }
+      } else {
+        sweep<4>(rd, 0, p.s.V, tid, kSampleThreads, [&](int, float x, bool in) {
+          count(order_key(x), in, [&]() -> uint64_t { return by_count ? 1 : mass_of(x, neg_mx); });
+        });
+      }
+      __syncthreads();
+      if (wave == 0) {  // (the wavefront that reads the bins also clears them for the next digit)
+        find_crossing<4>(hist, before, target, res, lane);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) hist[4 * lane + j] = 0;
+      }
+      __syncthreads();
+      before = res[1];
+      pmask |= 0xffu << (8 * d);
+      pval |= (255u - (uint32_t)res[0]) << (8 * d);
+    }
+    if (tid == 0) cut = pval;
+    __syncthreads();
+  };
+  if (cuts && listed) {
+    if (n <= 256) {
+      // every element against every other: 64 elements a wavefront, the wavefronts of the same elements a share of the
+      // others each (one wavefront takes 15 ns per other element)
+      const int blocks = n <= 64 ? 1 : n <= 128 ? 2 : 4, shares = kSampleWaves / blocks;
+      const int at = 64 * (wave % blocks) + lane, share = wave / blocks;
+      const int j1 = (int)((int64_t)n * (share + 1) / shares);
+      const uint32_t mine = at < n ? key[at] : 0;
+      uint64_t over = 0, equal = 0;
+      for (int j = n * share / shares; j < j1; ++j) {   // the same words for every lane: broadcast reads
+        const uint32_t k = key[j], w = by_count ? 1u : mass[j];
+        over += k > mine ? w : 0;
+        equal += k == mine ? w : 0;
+      }
+      if (at < n) {
+        atomicAdd(reinterpret_cast<unsigned long long*>(&hist[at]), (unsigned long long)over);
+        atomicAdd(reinterpret_cast<unsigned long long*>(&hist[256 + at]), (unsigned long long)equal);
+      }
+      __syncthreads();
+      if (tid < n && above + hist[tid] <= target && above + hist[tid] + hist[256 + tid] > target) cut = key[tid];
+      __syncthreads();
+      if (tid < 256) hist[tid] = 0;   // (for the digits, should the threshold turn out too high)
+      __syncthreads();
+    } else {
+      digits(true);
+    }
+    if (by_count && cut < tau) listed = false;   // (every thread sees the same words)
+  }
+  if (cuts && !listed) {
+    __syncthreads();
+    if (tid == 0) cut = 0;
+    digits(false);
+  }
+  const uint32_t cut_key = cuts ? cut : 0;
+  // ---- the kept elements that no run has counted yet join theirs ----
+  auto join = [&](int i, uint64_t w) {
+    const int part = i / p.part_len;
+    atomicAdd(reinterpret_cast<unsigned long long*>(&runs[part * kRuns + (i - part * p.part_len) / p.run_len]), (unsigned long long)w);
+  };
+  if (cuts && listed) {
+    for (int j = tid; j < n; j += kSampleThreads)
+      if (key[j] >= cut_key) join((int)index[j], mass[j]);
+  } else if (filtered) {
+    runs[tid] = 0;
+    __syncthreads();
+    sweep<4>(rd, 0, p.s.V, tid, kSampleThreads, [&](int i, float x, bool in) {
+      if (in && order_key(x) >= cut_key) join(i, mass_of(x, neg_mx));
+    });
+  }
+  __syncthreads();
+  // ---- the run the uniform number falls into: every thread owns one (there are at most 1 024) ----
+  const uint64_t mine = runs[tid];
+  uint64_t incl = wave_scan_incl_u64(mine, lane);
+  if (lane == 63) wsum[0][wave] = incl;
+  __syncthreads();
+  uint64_t total = 0;
+#pragma unroll
+  for (int w = 0; w < kSampleWaves; ++w) {
+    incl += w < wave ? wsum[0][w] : 0;
+    total += wsum[0][w];
+  }
+  // total > 0: the maximum itself is always kept and has the largest mass
+  uint64_t want = (uint64_t)((double)p.s.uniform[r] * (double)total);
+  want = want < total ? want : total - 1;
+  if (incl > want && incl - mine <= want) { res[0] = (uint64_t)tid; res[1] = incl - mine; }
+  __syncthreads();
+  // ---- the element: each thread owns a few neighbours of the run ----
+  const int run = (int)res[0];
+  want -= res[1];
+  const int pa = (run / kRuns) * p.part_len, ra = pa + (run % kRuns) * p.run_len;
+  const int rb = min(min(ra + p.run_len, pa + p.part_len), p.s.V);
+  const int per = (p.run_len + kSampleThreads - 1) / kSampleThreads;
+  auto kept_mass = [&](float x) -> uint64_t { return order_key(x) >= cut_key ? mass_of(x, neg_mx) : 0; };
+  const int a = min(ra + tid * per, rb), b = min(a + per, rb);
+  uint64_t s = 0;
+  for (int i = a; i < b; ++i) s += kept_mass(rd.at(i));
+  incl = wave_scan_incl_u64(s, lane);
+  if (lane == 63) wsum[1][wave] = incl;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kSampleWaves; ++w) incl += w < wave ? wsum[1][w] : 0;
+  if (incl > want && incl - s <= want) {
+    uint64_t at = incl - s;
+    for (int i = a; i < b; ++i) {
+      at += kept_mass(rd.at(i));
+      if (at > want) { pick = i; break; }
+    }
+  }
+  __syncthreads();
+  if (tid == 0) {
+    int sample = pick;
+    if (p.s.vocab_clamp > 0) sample = min(max(sample, 0), p.s.vocab_clamp - 1);
+    write_sample(p.s, r, sample, cut_key);
   }
 }
 
@@ -788,12 +1274,64 @@ extern "C" int mi_last_token_gather(const void* src, int64_t src_stride_row, voi
   return mi_check_launch("mi_last_token_gather");
 }
 
-extern "C" int mi_sample_from_logits(const void* logits, int64_t stride_row, int32_t logits_dtype, int32_t R,
-                                     int32_t vocab, int32_t top_k, float top_p, float temperature,
-                                     const float* uniform, int32_t vocab_clamp, int64_t* samples,
-                                     float* cut_values, const int32_t* request_kv_length_offsets,
-                                     const int32_t* request_query_lengths, const int32_t* request_output_lengths,
-                                     int64_t termination_id, uint8_t* active_request_mask, void* stream) {
+// Parts a row is cut into: enough workgroups for the chip (one per CU), parts of at least 4 096 elements.
+static int sample_parts(int R, int V) {
+  int parts = (256 + R - 1) / R;
+  if (parts > V / 4096) parts = V / 4096;
+  return parts < 1 ? 1 : (parts > kMaxParts ? kMaxParts : parts);
+}
+// Whether the rows are done in parts: while a row has two of them.  From 129 rows on one workgroup per row fills half
+// the chip and more, and its fewer reads count (256 x 128 256 fp32, one workgroup per row / in parts: plain 52 / 60 us,
+// top-k 50 45 / 60, top-p 0.9 70 / 83 on peaked rows).
+static bool sample_in_parts(int R, int V, int top_k) { return V >= kFastMinVocab && R <= 128 && top_k <= kFastTopK; }
+
+static int64_t align256(int64_t n) { return (n + 255) & ~(int64_t)255; }
+static int64_t sample_layout(SplitParams* p, uint8_t* base, int R, int V, int top_k, float top_p) {
+  const int parts = sample_parts(R, V);
+  int run = (V + parts * kRuns - 1) / (parts * kRuns);
+  run = (run + 7) & ~7;
+  int64_t at = 0;
+  auto take = [&](int64_t bytes) { uint8_t* q = base + at; at += align256(bytes); return q; };
+  const int64_t n = (int64_t)R * parts;
+  const bool draws = top_k != 1, by_count = top_k > 1, by_mass = draws && !by_count && top_p > 0.f;
+  p->parts = parts; p->run_len = run; p->part_len = run * kRuns;
+  p->list_cap = kMemberCap;   // (one part's list may hold all that the pick takes)
+  if (parts > 4) p->list_cap = kMemberCap / 4;
+  p->part_key = (uint32_t*)take(4 * n); p->part_idx = (int32_t*)take(4 * n);
+  p->part_tau = (uint32_t*)take(4 * n); p->part_listed = (uint32_t*)take(4 * n);
+  p->bins = (float*)take(by_mass ? n * kBins * 4 : 0);
+  p->part_mass = (uint64_t*)take(draws && !by_count ? n * 8 : 0);
+  p->run_mass = (uint64_t*)take(draws && !by_count ? n * kRuns * 8 : 0);
+  p->list = (uint2*)take(by_count || by_mass ? n * p->list_cap * 8 : 0);
+  return at;
+}
+
+template <int DT, int VEC>
+static void launch_sample(const SampleParams& s, SplitParams* split, hipStream_t st) {
+  if (!split) {
+    hipLaunchKernelGGL((sample_kernel<DT, VEC>), dim3(s.R), dim3(kSampleThreads), 0, st, s);
+    return;
+  }
+  const dim3 grid(split->parts, s.R), block(kSampleThreads);
+  if (s.top_k > 1) hipLaunchKernelGGL((sample_first_kernel<DT, VEC, kPickTopK>), grid, block, 0, st, *split);
+  else if (s.top_k == 0 && s.top_p > 0.f) hipLaunchKernelGGL((sample_first_kernel<DT, VEC, kPickTopP>), grid, block, 0, st, *split);
+  else hipLaunchKernelGGL((sample_first_kernel<DT, VEC, kPickMax>), grid, block, 0, st, *split);
+  if (s.top_k == 0) hipLaunchKernelGGL((sample_mass_kernel<DT, VEC>), grid, block, 0, st, *split);
+  hipLaunchKernelGGL((sample_pick_kernel<DT, VEC>), dim3(s.R), block, 0, st, *split);
+}
+
+extern "C" int64_t mi_sample_workspace_bytes(int32_t R, int32_t vocab, int32_t top_k, float top_p) {
+  SplitParams p;
+  return R > 0 && vocab > 0 && sample_in_parts(R, vocab, top_k) ? sample_layout(&p, nullptr, R, vocab, top_k, top_p) : 0;
+}
+
+extern "C" int mi_sample_from_logits_ws(const void* logits, int64_t stride_row, int32_t logits_dtype, int32_t R,
+                                        int32_t vocab, int32_t top_k, float top_p, float temperature,
+                                        const float* uniform, int32_t vocab_clamp, int64_t* samples,
+                                        float* cut_values, const int32_t* request_kv_length_offsets,
+                                        const int32_t* request_query_lengths, const int32_t* request_output_lengths,
+                                        int64_t termination_id, uint8_t* active_request_mask, void* workspace,
+                                        int64_t workspace_bytes, void* stream) {
   if (R == 0) return MI_OK;
   if (!logits || !samples) return mi_fail(MI_ERR_NULL, "mi_sample_from_logits: null pointer argument");
   if (R < 0 || vocab <= 0 || stride_row < vocab)
@@ -822,19 +1360,37 @@ extern "C" int mi_sample_from_logits(const void* logits, int64_t stride_row, int
   p.termination_id = termination_id; p.active_mask = active_request_mask;
   const int esize = logits_dtype != 0 ? 2 : 4;
   const bool wide = !(((uintptr_t)logits | (uintptr_t)(stride_row * esize)) & 15);  // 16-byte loads
-  const dim3 grid(R), block(kSampleThreads);
+  SplitParams split, *in_parts = nullptr;
+  if (workspace && sample_in_parts(R, vocab, top_k)) {
+    if ((uintptr_t)workspace & 255) return mi_fail(MI_ERR_ALIGN, "mi_sample_from_logits_ws: the workspace must be 256-byte aligned");
+    if (sample_layout(&split, (uint8_t*)workspace, R, vocab, top_k, top_p) > workspace_bytes)
+      return mi_fail(MI_ERR_WORKSPACE, "mi_sample_from_logits_ws: workspace smaller than mi_sample_workspace_bytes()");
+    split.s = p;
+    in_parts = &split;
+  }
   hipStream_t st = (hipStream_t)stream;
   if (logits_dtype == 2) {
-    if (wide) hipLaunchKernelGGL((sample_kernel<2, 8>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((sample_kernel<2, 1>), grid, block, 0, st, p);
+    if (wide) launch_sample<2, 8>(p, in_parts, st);
+    else launch_sample<2, 1>(p, in_parts, st);
   } else if (logits_dtype == 1) {
-    if (wide) hipLaunchKernelGGL((sample_kernel<1, 8>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((sample_kernel<1, 1>), grid, block, 0, st, p);
+    if (wide) launch_sample<1, 8>(p, in_parts, st);
+    else launch_sample<1, 1>(p, in_parts, st);
   } else {
-    if (wide) hipLaunchKernelGGL((sample_kernel<0, 4>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((sample_kernel<0, 1>), grid, block, 0, st, p);
+    if (wide) launch_sample<0, 4>(p, in_parts, st);
+    else launch_sample<0, 1>(p, in_parts, st);
   }
   return mi_check_launch("mi_sample_from_logits");
+}
+
+extern "C" int mi_sample_from_logits(const void* logits, int64_t stride_row, int32_t logits_dtype, int32_t R,
+                                     int32_t vocab, int32_t top_k, float top_p, float temperature,
+                                     const float* uniform, int32_t vocab_clamp, int64_t* samples,
+                                     float* cut_values, const int32_t* request_kv_length_offsets,
+                                     const int32_t* request_query_lengths, const int32_t* request_output_lengths,
+                                     int64_t termination_id, uint8_t* active_request_mask, void* stream) {
+  return mi_sample_from_logits_ws(logits, stride_row, logits_dtype, R, vocab, top_k, top_p, temperature, uniform, vocab_clamp,
+                                  samples, cut_values, request_kv_length_offsets, request_query_lengths,
+                                  request_output_lengths, termination_id, active_request_mask, nullptr, 0, stream);
 }
 
 extern "C" int mi_selected_log_probs(const void* logits, int64_t stride_row, int32_t logits_dtype, int32_t T,

@@ -513,13 +513,13 @@ def sample_from_logits(logits: Tensor, *, top_k: int = 0, top_p: float = 0.0, te
                        termination_id: Optional[int] = None, kv_length_offsets: Optional[Tensor] = None,
                        query_lengths: Optional[Tensor] = None, output_lengths: Optional[Tensor] = None,
                        return_cut: bool = False):
-    """One launch: filter + draw per row of ``logits`` ``[R, V]`` (fp32, bf16 or fp16) and, when
+    """Filter + draw per row of ``logits`` ``[R, V]`` (fp32, bf16 or fp16) and, when
     ``termination_id`` is given, the uint8 mask of requests that go on generating.
 
     Returns ``(samples int64 [R], mask uint8 [R] or None)`` and, with ``return_cut``, also the
     smallest kept value per row (fp32, -inf where nothing was filtered)."""
     return _native().sample_from_logits(logits, top_k, top_p, temperature, uniform, vocab_size or 0, termination_id,
-                                        kv_length_offsets, query_lengths, output_lengths, return_cut)
+                                        kv_length_offsets, query_lengths, output_lengths, return_cut, _override())
 
 
 def linear_decode(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None, out: Optional[Tensor] = None) -> Tensor:

@@ -404,3 +404,37 @@ def test_context_log_probs_through_the_kernel(mi, dev):
         assert (torch.tensor(got_last, dtype=torch.float64).flatten() - want_last).abs().max().item() <= 2e-5
     finally:
         Ctx.TOKEN_ROUNDER, Ctx.REQUEST_ROUNDER = saved
+
+
+@pytest.mark.parametrize("R,V", [(1, 16384), (2, 16389), (5, 50257), (128, 32000), (129, 32000), (1, 260000)])
+@pytest.mark.parametrize("kind", ["flat", "peaked", "equal", "few", "masked", "nan"])
+def test_rows_in_parts_equal_rows_by_one_workgroup(mi, dev, R, V, kind):
+    """Rows cut into parts give the tokens and cut values of the one-workgroup entry point, bit for bit: where the
+    parts' estimates hold, and where they fail (equal values, a handful of values, most of the row masked)."""
+    lib = mi._lib.load()
+    g = torch.Generator().manual_seed(R + V)
+    x = torch.randn(R, V, generator=g) * 3
+    if kind == "peaked":
+        x[:, torch.randint(0, V, (20,), generator=g)] += 15
+    elif kind == "equal":
+        x.fill_(-2.5)
+    elif kind == "few":
+        x = torch.randint(0, 4, (R, V), generator=g).float()
+    elif kind == "masked":
+        x[:, ::2], x[:, 1::3] = float("-inf"), -1e9
+    elif kind == "nan":
+        x[R // 2, V // 3] = float("nan")
+    u = torch.rand(R, generator=g).to(dev)
+    for dtype in (torch.float32, torch.bfloat16):
+        y = x.to(dtype).to(dev)
+        for top_k, top_p in ((1, 0.0), (0, 0.0), (0, 0.5), (0, 0.95), (0, 1.0), (2, 0.0), (50, 0.0), (768, 0.0), (769, 0.0)):
+            got, _, cut = mi.ops.sample_from_logits(y, top_k=top_k, top_p=top_p, temperature=0.7, uniform=u, return_cut=True)
+            want = torch.empty(R, dtype=torch.int64, device=dev)
+            want_cut = torch.empty(R, dtype=torch.float32, device=dev)
+            rc = lib.mi_sample_from_logits(y.data_ptr(), y.stride(0), 0 if dtype == torch.float32 else 1, R, V, top_k, top_p, 0.7,
+                                           u.data_ptr(), 0, want.data_ptr(), want_cut.data_ptr(), None, None, None, -1, None,
+                                           torch.cuda.current_stream().cuda_stream)
+            assert rc == 0, lib.mi_last_error()
+            torch.cuda.synchronize()
+            assert torch.equal(got, want), (dtype, top_k, top_p)
+            assert torch.equal(cut, want_cut), (dtype, top_k, top_p)
