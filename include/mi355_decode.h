@@ -447,7 +447,9 @@ int mi_qkv_norm_rope_append(const void* mixed_qkv, int64_t qkv_stride_tok, void*
  * {total_request_count, paused_request_count, active_token_count, chunk_count_avail,
  *  number of newly paused ids (-1 = none), status (0 ok, 1 mask/count mismatch - nothing was
  *  changed, 2 no active request left, 3 resumed request not at a chunk start), 1 if the context
- *  was emptied, number of finished ids}; the caller copies `counters` to the host after the call.
+ *  was emptied, number of finished ids}; the caller copies `counters` to the host after the call, or hands over pinned
+ *  host memory: the status is written last, behind a fence, so a host that watches it change needs no copy and no wait
+ *  for the stream.
  */
 int mi_update_requests(int32_t* request_ids, int32_t* request_query_lengths,
                        int32_t* request_output_lengths, int32_t* request_kv_length_offsets,
@@ -458,6 +460,22 @@ int mi_update_requests(int32_t* request_ids, int32_t* request_query_lengths,
                        int64_t* token_to_position_in_request, int64_t* token_to_chunk_idx,
                        int64_t* token_to_local_position_within_kv_chunk, int32_t* chunk_bag,
                        const int32_t* active_requests_mask, const int64_t* new_tokens,
+                       int64_t* paused_tokens, int64_t* next_tokens_scratch, int32_t* scratch,
+                       int32_t* newly_paused_request_ids, int32_t* finished_request_ids,
+                       int32_t* counters, int32_t total_request_count, int32_t paused_request_count,
+                       int32_t chunk_count_avail, int32_t gtd_chunk_count, int32_t gtd_request_count,
+                       int32_t chunk_size_tokens, int32_t max_requests, void* stream);
+
+/* The same with a mask of bytes (what mi_sample_from_logits writes). */
+int mi_update_requests_mask8(int32_t* request_ids, int32_t* request_query_lengths,
+                       int32_t* request_output_lengths, int32_t* request_kv_length_offsets,
+                       int32_t* request_kv_chunk_counts, int32_t* request_last_kv_chunk_id,
+                       int32_t* request_last_kv_chunk_offset, int32_t* request_to_kv_chunk_ids,
+                       int64_t table_stride, int32_t max_kv_chunk_count, int64_t* token_to_input_ids,
+                       int64_t* token_to_pos_ids, int64_t* token_to_request_idx,
+                       int64_t* token_to_position_in_request, int64_t* token_to_chunk_idx,
+                       int64_t* token_to_local_position_within_kv_chunk, int32_t* chunk_bag,
+                       const uint8_t* active_requests_mask, const int64_t* new_tokens,
                        int64_t* paused_tokens, int64_t* next_tokens_scratch, int32_t* scratch,
                        int32_t* newly_paused_request_ids, int32_t* finished_request_ids,
                        int32_t* counters, int32_t total_request_count, int32_t paused_request_count,

@@ -73,6 +73,14 @@ def _parameter(module: torch.nn.Module, name: str) -> Optional[Tensor]:
     return p if p is not None else getattr(module, name)
 
 
+def _untouched(module: torch.nn.Module, cls: type) -> bool:
+    """Whether calling ``module`` would run ``cls.forward`` and nothing else (no hooks, no subclass, no replaced
+    forward), so that its work may be folded into another call."""
+    return (type(module) is cls and "forward" not in module.__dict__
+            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
+            and not torch.nn.modules.module._has_any_global_hook())
+
+
 class PagedSelfAttentionCore(torch.nn.Module):
     """Everything between ``get_query_key_value_tensors`` and ``linear_proj`` for one layer.
 
@@ -101,18 +109,23 @@ class PagedSelfAttentionCore(torch.nn.Module):
         else:
             self.q_layernorm_weight = self.k_layernorm_weight = None
 
+    @staticmethod
+    def rotary_table(rotary_pos_emb) -> Optional[Tensor]:
+        """The one table of angles that the fused path takes for query and key."""
+        if rotary_pos_emb is None:
+            return None
+        q_emb, k_emb = rotary_pos_emb if isinstance(rotary_pos_emb, tuple) else (rotary_pos_emb,) * 2
+        assert q_emb is k_emb or q_emb is None or k_emb is None or q_emb.data_ptr() == k_emb.data_ptr(), \
+            "the fused path takes one rotary table for query and key"
+        return q_emb if q_emb is not None else k_emb
+
     def forward_mixed_qkv(self, mixed_qkv: Tensor, num_query_heads: int, inference_context,
                           rotary_pos_emb: Optional[Tuple[Tensor, Tensor]] = None) -> Tensor:
         """Same as :meth:`forward`, starting from the QKV projection's output ``[T, 1, (Hq + 2 Hkv) d]``:
         the split of ``get_query_key_value_tensors`` (attention.py:985-1030) is folded into the fused
         norm / RoPE / append launch, so no per-head q / k / v tensors are materialised."""
         ctx = inference_context
-        emb = None
-        if rotary_pos_emb is not None:
-            q_emb, k_emb = rotary_pos_emb if isinstance(rotary_pos_emb, tuple) else (rotary_pos_emb,) * 2
-            assert q_emb is k_emb or q_emb is None or k_emb is None or q_emb.data_ptr() == k_emb.data_ptr(), \
-                "the fused path takes one rotary table for query and key"
-            emb = q_emb if q_emb is not None else k_emb
+        emb = self.rotary_table(rotary_pos_emb)
         if self.fused and self._step_fusable(ctx, emb):
             out = ctx.fused_decode_step_attention(
                 self.layer_number, mixed_qkv=mixed_qkv, num_query_heads=num_query_heads, rotary_pos_emb=emb,
@@ -231,6 +244,29 @@ class PagedSelfAttentionLayer(torch.nn.Module):
 
     def forward(self, hidden_states: Tensor, inference_context,
                 rotary_pos_emb: Optional[Tuple[Tensor, Tensor]] = None):
+        output = self._decode_in_one_call(hidden_states, inference_context, rotary_pos_emb)
+        if output is not None:
+            proj = self.linear_proj
+            return output, (_parameter(proj, "bias") if proj.skip_bias_add else None)
         mixed_qkv, _ = self.linear_qkv(hidden_states)
         core_attn_out = self.core.forward_mixed_qkv(mixed_qkv, self.num_query_heads, inference_context, rotary_pos_emb)
         return self.linear_proj(core_attn_out)
+
+    def _decode_in_one_call(self, hidden_states: Tensor, ctx, rotary_pos_emb) -> Optional[Tensor]:
+        """The output of a decode-only step by one native call, or ``None`` where the step takes the modules one by
+        one: other steps, a context without that call, hooks or replaced forwards on the parts."""
+        qkv, core, proj = self._modules["linear_qkv"], self._modules["core"], self._modules["linear_proj"]
+        call = getattr(ctx, "fused_decode_layer", None)
+        n = hidden_states.size(0)
+        if (call is None or not core.fused or n > DecodeLinear.DECODE_ROWS or n != ctx.padded_active_token_count
+                or hidden_states.dim() != 3 or hidden_states.size(1) != 1
+                or not (_untouched(qkv, DecodeLinear) and _untouched(core, PagedSelfAttentionCore)
+                        and _untouched(proj, DecodeLinear))):
+            return None
+        emb = core.rotary_table(rotary_pos_emb)
+        if not core._step_fusable(ctx, emb):
+            return None
+        return call(core.layer_number, hidden_states, _parameter(qkv, "weight"),
+                    None if qkv.skip_bias_add else _parameter(qkv, "bias"), _parameter(proj, "weight"),
+                    None if proj.skip_bias_add else _parameter(proj, "bias"), num_query_heads=self.num_query_heads,
+                    rotary_pos_emb=emb, softmax_scale=core.softmax_scale, **core._norm_args())

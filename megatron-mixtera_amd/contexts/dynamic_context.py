@@ -269,12 +269,15 @@ class DynamicInferenceContext:
         self.non_decode_cuda_graphs = use_cuda_graphs_for_non_decode_steps and (num_cuda_graphs is not None)
 
         # ---- fixed-address mirrors consumed by captured graphs ----
-        self.query_seq_lengths_cudagraph_only = torch.zeros(self.max_requests, dtype=torch.int32, device=dev)
-        self.cu_query_seq_lengths_cudagraph_only = torch.zeros(self.max_requests + 1, dtype=torch.int32, device=dev)
-        self.kv_seq_lengths_cudagraph_only = torch.zeros(self.max_requests, dtype=torch.int32, device=dev)
-        self.cu_kv_seq_lengths_cudagraph_only = torch.zeros(self.max_requests + 1, dtype=torch.int32, device=dev)
-        self.request_to_kv_chunk_ids_cudagraph_only = torch.zeros(
-            (self.max_requests, self.max_kv_chunk_count), dtype=torch.int, device=dev)
+        # (views of one buffer, each on a 256-byte line: every step of a serving loop clears them, with one launch)
+        rows = self.max_requests
+        sizes = (rows, rows + 1, rows, rows + 1, rows * self.max_kv_chunk_count)
+        padded_sizes = [_ceil_to(n, 64) for n in sizes]
+        self._mirrors = torch.zeros(sum(padded_sizes), dtype=torch.int32, device=dev)
+        (self.query_seq_lengths_cudagraph_only, self.cu_query_seq_lengths_cudagraph_only,
+         self.kv_seq_lengths_cudagraph_only, self.cu_kv_seq_lengths_cudagraph_only, table) = (
+            part[:n] for part, n in zip(self._mirrors.split(padded_sizes), sizes))
+        self.request_to_kv_chunk_ids_cudagraph_only = table.view(rows, self.max_kv_chunk_count)
 
         # ---- guaranteed-progress reserve (reference: dynamic_context.py:398-401) ----
         reserve = min(int(buffer_guaranteed_fraction * chunk_count_total), chunk_count_total)
@@ -295,14 +298,15 @@ class DynamicInferenceContext:
             self._update_scratch = torch.zeros(4 * self.max_requests, dtype=torch.int32, device=dev)
             self._newly_paused_buf = torch.zeros(self.max_requests, dtype=torch.int32, device=dev)
             self._finished_ids_buf = torch.zeros(self.max_requests, dtype=torch.int32, device=dev)
-            self._counters = torch.zeros(8, dtype=torch.int32, device=dev)
-            self._counters_host = torch.zeros(8, dtype=torch.int32, pin_memory=True)
-            # largest query / kv length of a prefill or mixed step: written by the attention-state kernel,
-            # copied to pinned memory behind an event and only waited for when somebody reads the value
-            self._max_lengths = torch.zeros(2, dtype=torch.int32, device=dev)
-            self._max_lengths_host = torch.zeros(2, dtype=torch.int32, pin_memory=True)
-            self._max_lengths_event = torch.cuda.Event()
-        self._max_lengths_pending = False
+            # The new counters of update_requests, and the largest query / kv length of a prefill or mixed step (only
+            # waited for when somebody reads it), are written by their kernels straight into pinned host memory, where
+            # the host watches one word of each: no copy to enqueue, no wait for the whole stream
+            self._counters = torch.zeros(8, dtype=torch.int32, pin_memory=True)
+            self._counters_host = self._counters.numpy()
+            self._max_lengths = torch.zeros(2, dtype=torch.int32, pin_memory=True)
+            self._max_lengths_host = self._max_lengths.numpy()
+        self._max_lengths_pending = False     # nobody has read the step's maxima yet
+        self._max_lengths_in_flight = False   # their kernel may not have run yet
         # what the host knows without asking the device: the longest prompt admitted since the last
         # update_requests (every other active request has one query token) and a bound on the kv lengths
         self._host_max_query_len = 1
@@ -362,9 +366,21 @@ class DynamicInferenceContext:
     # copy issued by initialize_attention_state; a step that never reads them never waits.
     def _resolve_max_lengths(self) -> None:
         if self._max_lengths_pending:
-            self._max_lengths_event.synchronize()
+            self._land_max_lengths()
             self._max_seqlen_q, self._max_seqlen_k = self._max_lengths_host.tolist()
             self._max_lengths_pending = False
+
+    def _land_max_lengths(self) -> None:
+        """Wait for the maxima of the last prefill / mixed step, if their kernel may still be on its way."""
+        if self._max_lengths_in_flight:
+            self._await(self._max_lengths, 0)
+            self._await(self._max_lengths, 1)
+            self._max_lengths_in_flight = False
+
+    def _await(self, row: Tensor, index: int) -> None:
+        """Wait until a kernel on the current stream has replaced the -1 in ``row[index]`` (pinned host memory)."""
+        if not ops.watch(row, index, -1, 20000):
+            torch.cuda.current_stream(self.device).synchronize()
 
     @property
     def max_seqlen_q(self):
@@ -604,6 +620,23 @@ class DynamicInferenceContext:
                                   block_table, out=_first(out, n), **common)
         return out
 
+    def fused_decode_layer(self, layer_number: int, hidden: Tensor, qkv_weight: Tensor, qkv_bias: Optional[Tensor],
+                           proj_weight: Tensor, proj_bias: Optional[Tensor], *, num_query_heads: int,
+                           rotary_pos_emb: Optional[Tensor] = None, config=None, q_weight: Optional[Tensor] = None,
+                           k_weight: Optional[Tensor] = None, norm: Optional[str] = None, eps: float = 1e-5,
+                           softmax_scale: Optional[float] = None) -> Tensor:
+        """A decode-only step of one attention layer from hidden states to hidden states ``[T, 1, hidden]``, T the
+        padded token count: the QKV projection, :meth:`fused_decode_step_attention` on its output and the output
+        projection in one call."""
+        k_cache, v_cache = self._layer_cache(layer_number)
+        k_scales, v_scales = self.key_value_scales(layer_number)
+        return ops.attention_layer_decode(
+            hidden, qkv_weight, qkv_bias, proj_weight, proj_bias, num_query_heads, self.num_kv_heads_per_partition, k_cache,
+            v_cache, self.kv_seq_lengths, self.block_table, q_weight=q_weight, k_weight=k_weight, eps=eps, norm=norm,
+            rotary_emb=rotary_pos_emb, rotary_interleaved=self._rope_flags(config) if config is not None else False,
+            softmax_scale=softmax_scale, max_kv_len=self.attention_length_bounds()[1], k_scales=k_scales,
+            v_scales=v_scales, headroom=self.fp8_append_headroom)
+
     def fused_qkv_norm_rope_append(self, layer_number: int, mixed_qkv: Tensor, *, num_query_heads: int,
                                    rotary_pos_emb: Optional[Tensor], config=None,
                                    q_weight: Optional[Tensor] = None, k_weight: Optional[Tensor] = None,
@@ -659,11 +692,7 @@ class DynamicInferenceContext:
         self.cu_kv_seq_lengths = None
         self.kv_seq_lengths = None
         self.block_table = None
-        # (one launch for the five: every step of a serving loop comes through here)
-        torch._foreach_zero_([
-            self.cu_query_seq_lengths_cudagraph_only, self.query_seq_lengths_cudagraph_only,
-            self.cu_kv_seq_lengths_cudagraph_only, self.kv_seq_lengths_cudagraph_only,
-            self.request_to_kv_chunk_ids_cudagraph_only])
+        self._mirrors.zero_()
 
     def using_cuda_graph_this_step(self) -> bool:
         """Graph sizes exist, the step type may use them, and the batch fits the largest one."""
@@ -719,7 +748,10 @@ class DynamicInferenceContext:
             # tensors), the padded token rows are pointed at the dummy chunk, and the two maxima follow
             # through pinned memory for whoever reads max_seqlen_q / max_seqlen_k.
             R = self.padded_active_request_count
+            self._land_max_lengths()  # (an earlier step's must not arrive after the reset of the words)
+            self._max_lengths_host[:] = -1
             ops.step_attention_state(self, n_active_req, R, padded)
+            self._max_lengths_in_flight = True
             self.kv_seq_lengths = self.kv_seq_lengths_cudagraph_only[:R]
             self.block_table = self.request_to_kv_chunk_ids_cudagraph_only[:R]
             self.cu_query_seq_lengths = self.cu_query_seq_lengths_cudagraph_only[: R + 1]
@@ -728,8 +760,6 @@ class DynamicInferenceContext:
                 self.max_seqlen_q = padded
                 self.max_seqlen_k = self.max_sequence_length
             else:
-                self._max_lengths_host.copy_(self._max_lengths, non_blocking=True)
-                self._max_lengths_event.record(torch.cuda.current_stream(self.device))
                 self._max_lengths_pending = True
             note_kv_lengths(self.cu_kv_seq_lengths, self.kv_seq_lengths)
             return
@@ -1013,16 +1043,20 @@ class DynamicInferenceContext:
         """``update_requests`` as one kernel + one read-back of the new counters."""
         dev = self.device
         assert active_requests_mask.numel() + self.paused_request_count == self.total_request_count
-        mask = active_requests_mask.to(device=dev, dtype=torch.int32).contiguous()
-        tokens = new_tokens.to(device=dev, dtype=torch.long).contiguous()
+        mask, tokens = active_requests_mask, new_tokens
+        if mask.dtype not in (torch.uint8, torch.int32) or mask.device != dev or not mask.is_contiguous():
+            mask = mask.to(device=dev, dtype=torch.int32).contiguous()
+        if tokens.dtype != torch.long or tokens.device != dev or not tokens.is_contiguous():
+            tokens = tokens.to(device=dev, dtype=torch.long).contiguous()
         assert tokens.numel() >= mask.numel()
         if self.paused_request_count:
             assert self.paused_tokens is not None
             if self.paused_tokens.data_ptr() != self._paused_tokens_buf.data_ptr():
                 self._paused_tokens_buf[: self.paused_request_count] = self.paused_tokens[: self.paused_request_count]
+        self._counters_host[5] = -1
         ops.update_requests(self, mask, tokens)
-        self._counters_host.copy_(self._counters, non_blocking=True)
-        torch.cuda.current_stream(dev).synchronize()
+        self._await(self._counters, 5)
+        self._max_lengths_in_flight = False   # (the stream is in order)
         total, paused, active, avail, n_newly, status, was_reset, n_finished = self._counters_host.tolist()
         assert status != 1, "active + finished + paused requests != total_request_count"
         self.last_finished_request_ids = self._finished_ids_buf[:n_finished].clone()

@@ -25,7 +25,8 @@ struct UpdateParams {
   int32_t* table; int64_t table_stride; int32_t M;
   int64_t* tok_input; int64_t* tok_pos; int64_t* tok_req; int64_t* tok_in_req; int64_t* tok_chunk; int64_t* tok_local;
   int32_t* bag;
-  const int32_t* mask; const int64_t* new_tokens;
+  const void* mask; int32_t mask_bytes;   // int32 or uint8 entries
+  const int64_t* new_tokens;
   int64_t* paused_tokens;    // in: tokens of the paused rows; out: tokens of the rows paused afterwards
   int64_t* next_tokens;      // scratch [max_requests]
   int32_t* scratch;          // scratch [4 * max_requests]
@@ -145,13 +146,27 @@ __global__ __launch_bounds__(kThreads) void update_requests_kernel(UpdateParams 
   int32_t* list_b = p.scratch + p.max_requests;      // [max_requests]
   int32_t* counts = p.scratch + 2 * p.max_requests;  // [max_requests]
 
+  auto mask_at = [&](int i) -> int {
+    return p.mask_bytes == 1 ? static_cast<const uint8_t*>(p.mask)[i] : static_cast<const int32_t*>(p.mask)[i];
+  };
+  // The counters may lie in host memory that the host watches: the status is written last, behind a fence, so that
+  // whoever sees it changed finds the others written.
+  auto report = [&](int status, int total, int paused, int active, int avail, int n_newly, int reset, int n_finished) {
+    if (status != 1) p.counters[7] = n_finished;
+    if (status == 0 || status == 3) {
+      p.counters[0] = total; p.counters[1] = paused; p.counters[2] = active; p.counters[3] = avail;
+      p.counters[4] = n_newly; p.counters[6] = reset;
+    }
+    __threadfence_system();
+    __hip_atomic_store(&p.counters[5], status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  };
   // ---- 1. how many requests continue / finished ---------------------------------------
   if (t < 2) red[t] = 0;
   __syncthreads();
   int c1 = 0, c0 = 0;
   for (int i = t; i < n; i += kThreads) {
-    c1 += p.mask[i] == 1;
-    c0 += p.mask[i] == 0;
+    c1 += mask_at(i) == 1;
+    c0 += mask_at(i) == 0;
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
@@ -168,23 +183,20 @@ __global__ __launch_bounds__(kThreads) void update_requests_kernel(UpdateParams 
   int avail = p.avail;
   int paused = P0;
   if (n_cont + n_fin + P0 != p.total || n < 0) {
-    if (t == 0) { p.counters[5] = 1; }
+    if (t == 0) report(1, 0, 0, 0, 0, 0, 0, 0);
     return;
   }
 
   // ---- 2. nothing left: give everything back --------------------------------------------
   if (n_cont + P0 == 0) {
     if (n_fin > 0) {
-      const int nf = compact(n, P0, list_a, [&](int i) { return p.mask[i] == 0; }, sh);
+      const int nf = compact(n, P0, list_a, [&](int i) { return mask_at(i) == 0; }, sh);
       for (int k = t; k < nf; k += kThreads) p.finished[k] = p.ids[list_a[k]];
       avail = release_rows(p, list_a, nf, avail, counts, sh);
     }
     for (int64_t i = t; i < (int64_t)p.max_requests * p.M; i += kThreads)
       p.table[(i / p.M) * p.table_stride + (i % p.M)] = -1;
-    if (t == 0) {
-      p.counters[0] = 0; p.counters[1] = P0; p.counters[2] = 0; p.counters[3] = avail;
-      p.counters[4] = -1; p.counters[5] = 0; p.counters[6] = 1; p.counters[7] = n_fin;
-    }
+    if (t == 0) report(0, 0, P0, 0, avail, -1, 1, n_fin);
     return;
   }
 
@@ -195,7 +207,7 @@ __global__ __launch_bounds__(kThreads) void update_requests_kernel(UpdateParams 
 
   // ---- 4. finished requests: release chunks, fill their holes from the right ---------------
   if (n_fin > 0) {
-    const int nf = compact(n, P0, list_a, [&](int i) { return p.mask[i] == 0; }, sh);
+    const int nf = compact(n, P0, list_a, [&](int i) { return mask_at(i) == 0; }, sh);
     // their ids, in row order (what the caller of the step reports as finished), before any row moves
     for (int k = t; k < nf; k += kThreads) p.finished[k] = p.ids[list_a[k]];
     avail = release_rows(p, list_a, nf, avail, counts, sh);
@@ -203,8 +215,8 @@ __global__ __launch_bounds__(kThreads) void update_requests_kernel(UpdateParams 
       p.table[(int64_t)list_a[i / p.M] * p.table_stride + (i % p.M)] = -1;
     __syncthreads();
     if (n_cont > 0) {
-      const int nh = compact(n_cont, P0, list_a, [&](int i) { return p.mask[i] == 0; }, sh);
-      compact(n - n_cont, P0 + n_cont, list_b, [&](int i) { return p.mask[n_cont + i] != 0; }, sh);
+      const int nh = compact(n_cont, P0, list_a, [&](int i) { return mask_at(i) == 0; }, sh);
+      compact(n - n_cont, P0 + n_cont, list_b, [&](int i) { return mask_at(n_cont + i) != 0; }, sh);
       for (int k = t; k < nh; k += kThreads) store_row(p, list_a[k], load_row(p, list_b[k]));
       for (int64_t i = t; i < (int64_t)nh * p.M; i += kThreads) {
         const int k = (int)(i / p.M), j = (int)(i % p.M);
@@ -256,7 +268,7 @@ __global__ __launch_bounds__(kThreads) void update_requests_kernel(UpdateParams 
   paused -= n_resume;
   n_cont += n_resume;
   if (n_cont <= 0) {
-    if (t == 0) { p.counters[5] = 2; p.counters[7] = n_fin; }
+    if (t == 0) report(2, 0, 0, 0, 0, 0, 0, n_fin);
     return;
   }
   if (n_newly >= 0 && n_resume > 0) n_newly = max(0, n_newly - n_resume);
@@ -291,10 +303,7 @@ __global__ __launch_bounds__(kThreads) void update_requests_kernel(UpdateParams 
   if (bad) atomicOr(&red[0], 1 << 30);
   __syncthreads();
   avail -= n_resume;
-  if (t == 0) {
-    p.counters[0] = total; p.counters[1] = paused; p.counters[2] = n_cont; p.counters[3] = avail;
-    p.counters[4] = n_newly; p.counters[5] = (red[0] >> 30) ? 3 : 0; p.counters[6] = 0; p.counters[7] = n_fin;
-  }
+  if (t == 0) report((red[0] >> 30) ? 3 : 0, total, paused, n_cont, avail, n_newly, 0, n_fin);
 }
 
 struct DecodeStateParams {
@@ -406,13 +415,13 @@ __global__ __launch_bounds__(1024) void step_attention_state_kernel(StepStatePar
 
 using namespace mi;
 
-extern "C" int mi_update_requests(
+static int update_requests(int mask_bytes,
     int32_t* request_ids, int32_t* request_query_lengths, int32_t* request_output_lengths,
     int32_t* request_kv_length_offsets, int32_t* request_kv_chunk_counts, int32_t* request_last_kv_chunk_id,
     int32_t* request_last_kv_chunk_offset, int32_t* request_to_kv_chunk_ids, int64_t table_stride,
     int32_t max_kv_chunk_count, int64_t* token_to_input_ids, int64_t* token_to_pos_ids,
     int64_t* token_to_request_idx, int64_t* token_to_position_in_request, int64_t* token_to_chunk_idx,
-    int64_t* token_to_local_position_within_kv_chunk, int32_t* chunk_bag, const int32_t* active_requests_mask,
+    int64_t* token_to_local_position_within_kv_chunk, int32_t* chunk_bag, const void* active_requests_mask,
     const int64_t* new_tokens, int64_t* paused_tokens, int64_t* next_tokens_scratch, int32_t* scratch,
     int32_t* newly_paused_request_ids, int32_t* finished_request_ids, int32_t* counters, int32_t total_request_count,
     int32_t paused_request_count, int32_t chunk_count_avail, int32_t gtd_chunk_count,
@@ -435,7 +444,7 @@ extern "C" int mi_update_requests(
   p.tok_input = token_to_input_ids; p.tok_pos = token_to_pos_ids; p.tok_req = token_to_request_idx;
   p.tok_in_req = token_to_position_in_request; p.tok_chunk = token_to_chunk_idx;
   p.tok_local = token_to_local_position_within_kv_chunk;
-  p.bag = chunk_bag; p.mask = active_requests_mask; p.new_tokens = new_tokens;
+  p.bag = chunk_bag; p.mask = active_requests_mask; p.mask_bytes = mask_bytes; p.new_tokens = new_tokens;
   p.paused_tokens = paused_tokens; p.next_tokens = next_tokens_scratch; p.scratch = scratch;
   p.newly_paused = newly_paused_request_ids; p.finished = finished_request_ids; p.counters = counters;
   p.total = total_request_count; p.paused = paused_request_count; p.avail = chunk_count_avail;
@@ -443,6 +452,50 @@ extern "C" int mi_update_requests(
   p.max_requests = max_requests;
   hipLaunchKernelGGL(update_requests_kernel, dim3(1), dim3(kThreads), 0, (hipStream_t)stream, p);
   return mi_check_launch("mi_update_requests");
+}
+
+extern "C" int mi_update_requests(
+    int32_t* request_ids, int32_t* request_query_lengths, int32_t* request_output_lengths,
+    int32_t* request_kv_length_offsets, int32_t* request_kv_chunk_counts, int32_t* request_last_kv_chunk_id,
+    int32_t* request_last_kv_chunk_offset, int32_t* request_to_kv_chunk_ids, int64_t table_stride,
+    int32_t max_kv_chunk_count, int64_t* token_to_input_ids, int64_t* token_to_pos_ids,
+    int64_t* token_to_request_idx, int64_t* token_to_position_in_request, int64_t* token_to_chunk_idx,
+    int64_t* token_to_local_position_within_kv_chunk, int32_t* chunk_bag, const int32_t* active_requests_mask,
+    const int64_t* new_tokens, int64_t* paused_tokens, int64_t* next_tokens_scratch, int32_t* scratch,
+    int32_t* newly_paused_request_ids, int32_t* finished_request_ids, int32_t* counters, int32_t total_request_count,
+    int32_t paused_request_count, int32_t chunk_count_avail, int32_t gtd_chunk_count,
+    int32_t gtd_request_count, int32_t chunk_size_tokens, int32_t max_requests, void* stream) {
+  return update_requests(4, request_ids, request_query_lengths, request_output_lengths, request_kv_length_offsets,
+                         request_kv_chunk_counts, request_last_kv_chunk_id, request_last_kv_chunk_offset,
+                         request_to_kv_chunk_ids, table_stride, max_kv_chunk_count, token_to_input_ids,
+                         token_to_pos_ids, token_to_request_idx, token_to_position_in_request, token_to_chunk_idx,
+                         token_to_local_position_within_kv_chunk, chunk_bag, active_requests_mask, new_tokens,
+                         paused_tokens, next_tokens_scratch, scratch, newly_paused_request_ids,
+                         finished_request_ids, counters, total_request_count, paused_request_count,
+                         chunk_count_avail, gtd_chunk_count, gtd_request_count, chunk_size_tokens, max_requests,
+                         stream);
+}
+
+extern "C" int mi_update_requests_mask8(
+    int32_t* request_ids, int32_t* request_query_lengths, int32_t* request_output_lengths,
+    int32_t* request_kv_length_offsets, int32_t* request_kv_chunk_counts, int32_t* request_last_kv_chunk_id,
+    int32_t* request_last_kv_chunk_offset, int32_t* request_to_kv_chunk_ids, int64_t table_stride,
+    int32_t max_kv_chunk_count, int64_t* token_to_input_ids, int64_t* token_to_pos_ids,
+    int64_t* token_to_request_idx, int64_t* token_to_position_in_request, int64_t* token_to_chunk_idx,
+    int64_t* token_to_local_position_within_kv_chunk, int32_t* chunk_bag, const uint8_t* active_requests_mask,
+    const int64_t* new_tokens, int64_t* paused_tokens, int64_t* next_tokens_scratch, int32_t* scratch,
+    int32_t* newly_paused_request_ids, int32_t* finished_request_ids, int32_t* counters, int32_t total_request_count,
+    int32_t paused_request_count, int32_t chunk_count_avail, int32_t gtd_chunk_count,
+    int32_t gtd_request_count, int32_t chunk_size_tokens, int32_t max_requests, void* stream) {
+  return update_requests(1, request_ids, request_query_lengths, request_output_lengths, request_kv_length_offsets,
+                         request_kv_chunk_counts, request_last_kv_chunk_id, request_last_kv_chunk_offset,
+                         request_to_kv_chunk_ids, table_stride, max_kv_chunk_count, token_to_input_ids,
+                         token_to_pos_ids, token_to_request_idx, token_to_position_in_request, token_to_chunk_idx,
+                         token_to_local_position_within_kv_chunk, chunk_bag, active_requests_mask, new_tokens,
+                         paused_tokens, next_tokens_scratch, scratch, newly_paused_request_ids,
+                         finished_request_ids, counters, total_request_count, paused_request_count,
+                         chunk_count_avail, gtd_chunk_count, gtd_request_count, chunk_size_tokens, max_requests,
+                         stream);
 }
 
 extern "C" int mi_decode_attention_state(

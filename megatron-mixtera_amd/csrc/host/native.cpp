@@ -17,6 +17,7 @@
 #include <ATen/ATen.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <chrono>
 #include <cmath>
 #include <string>
 #include <tuple>
@@ -790,6 +791,29 @@ PyObject* linear_decode(PyObject* const* a) {
   return a[3] == Py_None ? wrap(made) : same(a[3]);
 }
 
+// attention_layer_decode(hidden, qkv_weight, qkv_bias|None, proj_weight, proj_bias|None, num_query_heads, num_kv_heads,
+//                        k_cache, v_cache, kv_lens, block_table, q_weight|None, k_weight|None, eps, norm_kind,
+//                        rotary_emb|None, interleaved, softmax_scale|None, max_kv_len, k_scales|None, v_scales|None,
+//                        headroom, tuning|None, override|None): the three calls of a decode step of a layer in a row
+PyObject* attention_layer_decode(PyObject* const* a) {
+  PyObject* const none = Py_None;
+  PyObject* const linear_qkv[5] = {a[0], a[1], a[2], none, a[23]};
+  PyObject* mixed = linear_decode(linear_qkv);
+  struct Drop {
+    PyObject* o;
+    ~Drop() { Py_XDECREF(o); }
+  };
+  Drop d0{mixed}, d1{PyLong_FromLong(0)}, d2{PyFloat_FromDouble(1.0)};
+  PyObject* const step[29] = {none, none, none, mixed, a[5], a[6], a[7], a[8], a[9], a[10], a[11], a[12], a[13], a[14], a[15],
+                              none, a[16], d2.o, a[17], a[18], d1.o, none, none, Py_True, a[19], a[20], a[21], a[22], a[23]};
+  PyObject* attn = decode_step_attention(step);
+  Drop d3{attn};
+  const Tensor& o = THPVariable_Unpack(attn);   // [R, 1, Hq, d], contiguous
+  Drop d4{wrap(o.view({o.size(0), 1, o.size(2) * o.size(3)}))};
+  PyObject* const linear_proj[5] = {d4.o, a[3], a[4], none, a[23]};
+  return linear_decode(linear_proj);
+}
+
 // sample_from_logits(logits, top_k, top_p, temperature, uniform|None, vocab_size, termination_id|None,
 //                    kv_length_offsets|None, query_lengths|None, output_lengths|None, return_cut,
 //                    override|None)
@@ -900,6 +924,29 @@ PyObject* op(PyObject*, PyObject* const* a, Py_ssize_t n) {
   }
 }
 
+// watch(tensor, index, value, microseconds): whether element `index` of an int32 row in pinned host memory became
+// anything but `value` within the time.  The interpreter lock is free meanwhile.
+PyObject* watch(PyObject* const* a) {
+  const Tensor& t = tensor(a[0], "row");
+  const int64_t index = as_int(a[1]);
+  REQUIRE(t.device().is_cpu() && t.scalar_type() == at::kInt && t.is_contiguous() && index >= 0 && index < t.numel(),
+          "watch takes an int32 row in host memory");
+  const int32_t* word = static_cast<const int32_t*>(t.data_ptr()) + index;
+  const int32_t value = (int32_t)as_int(a[2]);
+  const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(as_int(a[3]));
+  bool changed = false;
+  Py_BEGIN_ALLOW_THREADS
+  for (;;) {
+    for (int i = 0; i < 64 && !changed; ++i) {
+      changed = __atomic_load_n(word, __ATOMIC_ACQUIRE) != value;
+      if (!changed) __builtin_ia32_pause();
+    }
+    if (changed || std::chrono::steady_clock::now() > until) break;
+  }
+  Py_END_ALLOW_THREADS
+  return PyBool_FromLong(changed);
+}
+
 // setup(kernel_error_class, raw_stream(device index), grow(device index, stream, bytes))
 PyObject* setup(PyObject* const* a) {
   for (int i = 0; i < 3; ++i) Py_INCREF(a[i]);
@@ -923,11 +970,11 @@ PyObject* set_workspace(PyObject* const* a) {
 PyMethodDef kMethods[] = {
     ABI(mi_kv_append_decode), ABI(mi_kv_quantize_chunks_fp8), ABI(mi_kv_append_decode_fp8), ABI(mi_decode_workspace_bytes),
     ABI(mi_prefill_workspace_bytes), ABI(mi_paged_decode_attention_noalloc),
-    ABI(mi_update_requests), ABI(mi_add_request), ABI(mi_decode_attention_state), ABI(mi_step_attention_state),
+    ABI(mi_update_requests), ABI(mi_update_requests_mask8), ABI(mi_add_request), ABI(mi_decode_attention_state), ABI(mi_step_attention_state),
     OP(kv_append, 6), OP(kv_append_fp8, 9), OP(paged_decode_attention, 14), OP(paged_mla_decode_attention, 10),
     OP(paged_prefill_attention, 13), OP(paged_prefill_attention_mla, 11), OP(norm_rope_append, 22), OP(qkv_norm_rope_append, 22), OP(decode_step_attention, 29),
-    OP(linear_decode, 5), OP(sample_from_logits, 12), OP(selected_log_probs, 2), OP(last_token_gather, 3), OP(setup, 3),
-    OP(set_workspace, 3), {nullptr, nullptr, 0, nullptr}};
+    OP(linear_decode, 5), OP(attention_layer_decode, 24), OP(sample_from_logits, 12), OP(selected_log_probs, 2), OP(last_token_gather, 3), OP(setup, 3),
+    OP(set_workspace, 3), OP(watch, 4), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_native", "Host side of the per-layer calls.", -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

@@ -425,12 +425,20 @@ def decode_step_attention(query: Optional[Tensor], key: Optional[Tensor], value:
         split_tokens, out, workspace, faithful_rounding, k_scales, v_scales, headroom, _tuning_arg(), _override())
 
 
-def update_requests(ctx, mask_i32: Tensor, new_tokens_i64: Tensor) -> None:
+def watch(row: Tensor, index: int, value: int, microseconds: int) -> bool:
+    """Whether ``row[index]`` (int32 in pinned host memory, written by a kernel) became anything but ``value`` within
+    the time; other Python threads run meanwhile."""
+    return _native().watch(row, index, value, microseconds)
+
+
+def update_requests(ctx, mask: Tensor, new_tokens_i64: Tensor) -> None:
     """Enqueue the single-kernel ``update_requests`` on the state tensors of ``ctx`` (results land in
-    ``ctx._counters`` / ``ctx._newly_paused_buf`` / ``ctx._finished_ids_buf`` / ``ctx._paused_tokens_buf``)."""
+    ``ctx._counters``, pinned host memory, / ``ctx._newly_paused_buf`` / ``ctx._finished_ids_buf`` / ``ctx._paused_tokens_buf``)."""
     table = ctx.request_to_kv_chunk_ids
     _require(table.stride(1) == 1, "request_to_kv_chunk_ids rows must be contiguous")
-    _lib.check(_native().abi_mi_update_requests(
+    native = _native()
+    update = native.abi_mi_update_requests if mask.dtype == torch.int32 else native.abi_mi_update_requests_mask8
+    _lib.check(update(
         ctx.request_ids, ctx.request_query_lengths, ctx.request_output_lengths,
         ctx.request_kv_length_offsets, ctx.request_kv_chunk_counts,
         ctx.request_last_kv_chunk_id, ctx.request_last_kv_chunk_offset,
@@ -438,7 +446,7 @@ def update_requests(ctx, mask_i32: Tensor, new_tokens_i64: Tensor) -> None:
         ctx.token_to_input_ids, ctx.token_to_pos_ids, ctx.token_to_request_idx,
         ctx.token_to_position_in_request, ctx.token_to_chunk_idx,
         ctx.token_to_local_position_within_kv_chunk, ctx.chunk_allocator.chunk_bag,
-        mask_i32, new_tokens_i64, ctx._paused_tokens_buf,
+        mask, new_tokens_i64, ctx._paused_tokens_buf,
         ctx._next_tokens_buf, ctx._update_scratch, ctx._newly_paused_buf,
         ctx._finished_ids_buf, ctx._counters, ctx.total_request_count, ctx.paused_request_count,
         ctx.chunk_allocator.chunk_count_avail, ctx.gtd_chunk_count, ctx.gtd_request_count,
@@ -520,6 +528,23 @@ def sample_from_logits(logits: Tensor, *, top_k: int = 0, top_p: float = 0.0, te
     smallest kept value per row (fp32, -inf where nothing was filtered)."""
     return _native().sample_from_logits(logits, top_k, top_p, temperature, uniform, vocab_size or 0, termination_id,
                                         kv_length_offsets, query_lengths, output_lengths, return_cut, _override())
+
+
+def attention_layer_decode(hidden: Tensor, qkv_weight: Tensor, qkv_bias: Optional[Tensor], proj_weight: Tensor,
+                           proj_bias: Optional[Tensor], num_query_heads: int, num_kv_heads: int, k_cache: Tensor,
+                           v_cache: Tensor, kv_lens: Tensor, block_table: Tensor, *, q_weight: Optional[Tensor] = None,
+                           k_weight: Optional[Tensor] = None, eps: float = 1e-5, norm: Optional[str] = None,
+                           rotary_emb: Optional[Tensor] = None, rotary_interleaved: bool = False,
+                           softmax_scale: Optional[float] = None, max_kv_len: Optional[int] = None,
+                           k_scales: Optional[Tensor] = None, v_scales: Optional[Tensor] = None,
+                           headroom: float = 2.0) -> Tensor:
+    """A decode step of one attention layer, hidden states ``[R, 1, hidden]`` in and out: :func:`linear_decode`,
+    :func:`decode_step_attention` on its output and :func:`linear_decode` again, without returning to Python in
+    between."""
+    return _native().attention_layer_decode(
+        hidden, qkv_weight, qkv_bias, proj_weight, proj_bias, num_query_heads, num_kv_heads, k_cache, v_cache, kv_lens,
+        block_table, q_weight, k_weight, eps, _NORM_KINDS[norm], rotary_emb, rotary_interleaved, softmax_scale, max_kv_len,
+        k_scales, v_scales, headroom, _tuning_arg(), _override())
 
 
 def linear_decode(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None, out: Optional[Tensor] = None) -> Tensor:

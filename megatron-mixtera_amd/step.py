@@ -89,8 +89,9 @@ def generate_output_tokens_dynamic_batch(context, forward_step: ForwardStep, sam
     if with_log_probs:
         log_probs = context.calculate_log_probs(logits, sample, only_last_token_logits=last_rows_only)
 
-    # update_requests works on its own copy of the sample: the caller keeps `sample` as drawn
-    newly_paused = context.update_requests(keep_mask, sample.clone())
+    # the caller keeps `sample` as drawn: the bookkeeping kernel only reads it, the torch op sequence moves its rows
+    newly_paused = context.update_requests(
+        keep_mask, sample if getattr(context, "fused_bookkeeping", False) else sample.clone())
 
     return {
         "active_request_ids": ids_before,
