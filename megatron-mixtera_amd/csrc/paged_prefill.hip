@@ -1105,7 +1105,11 @@ static int launch_paged_prefill(
 
   hipStream_t st = (hipStream_t)stream;
   if (two_phase) {
-    const int sbq_lds = 8 * ((head_dim >= 192 ? 16 : 32) / Gw);  // 8 wavefronts x whole tokens in a wavefront's 32 (wide heads: 16) rows
+    // head_dim 64 and 128: the one-stream tile kernel (measured at every size tried the faster of the two there: 1-3 %
+    // at 128, 8-14 % at 64); the knob asks for the two-phase one
+    const bool woven = tune.prefill_two_phase == 3 && (head_dim == 64 || head_dim == 128);
+    // wavefronts x whole tokens in a wavefront's 32 (wide heads: 16) rows
+    const int sbq_lds = (woven ? prefill_woven_waves(head_dim) : 8) * ((head_dim >= 192 ? 16 : 32) / Gw);
     dim3 lgrid(((T + sbq_lds - 1) / sbq_lds + R) * Hkv * parts);
     hipEvent_t ev_a, ev_b;
     const bool timed = mi_profile_next(&ev_a, &ev_b);
@@ -1126,8 +1130,7 @@ static int launch_paged_prefill(
         workspace_bytes = dec_bytes;
       }
     }
-    // head_dim 128 over a 16-bit cache: the one-stream tile kernel when asked for
-    if (!fp8 && head_dim == 128 && tune.prefill_two_phase == 3) launch_prefill_woven(p, lgrid, f16, st);
+    if (woven) launch_prefill_woven(p, lgrid, head_dim, fp8, f16, st);
     else if (fp8 && head_dim == 64 && f16) MI_PP_LAUNCH(true, 64, 64, true);
     else if (fp8 && head_dim == 64) MI_PP_LAUNCH(true, 64, 64, false);
     else if (fp8 && f16) MI_PP_LAUNCH(true, 128, 128, true);

@@ -2,10 +2,14 @@
 //
 // Serves the same call as the two-phase tile kernel of paged_prefill.hip -- flash_attn_varlen_func(..., causal=True,
 // block_table=...) from Attention.flash_decode_and_prefill (megatron/core/transformer/attention.py:546-557) -- for
-// head_dim 128 over a 16-bit cache whose chunk size is a multiple of 64.
+// head_dim 64 and 128 over a 16-bit or fp8 cache whose chunk size is a multiple of 64.
 //
 // A workgroup of 8 wavefronts (two per SIMD, 256 registers each) takes 256 consecutive (query token, head-in-group)
-// rows of one (request, KV head), 32 rows per wavefront, and walks the keys in staged tiles of 64.  There are no
+// rows of one (request, KV head), 32 rows per wavefront, and walks the keys in staged tiles of 64.  At head_dim 64 the
+// accumulators are half as many and the exponentials per product twice: there workgroups of 4 wavefronts, three per CU
+// (168 registers, 51 KB of LDS each), put a third wavefront on every SIMD to fill the vector pipe, and the work comes
+// in half the pieces (11 ragged prompts of 164-2 911 tokens, fp16: 148 us, the two-phase kernel 170; 8 x 2 048 new
+// tokens beside decoding requests: 754 against 838 us with everything).  There are no
 // matrix / vector phases and no per-phase barriers: every wavefront runs the whole tile pipeline in ONE stream, cut
 // into 32-key steps and software-pipelined so that three independent chains are always open --
 //     products    S^T(step s+1) = K Q^T          and  O^T += V^T P^T(step s-1)     (matrix cores)
@@ -23,6 +27,12 @@
 // (values are multiplied one tile after their keys); the loads of the next pair are issued right after the tile's
 // barrier and are waited for at the next one.
 //
+// An fp8 cache (e4m3 bytes, one scale per chunk and KV head; a tile lies in one chunk) is staged through registers, a
+// tile ahead: 8-byte loads set out after one barrier and are stored, converted, before the next.  Key bytes are
+// converted exactly (four instructions per eight; e4m3 is a subset of both 16-bit types) and their scale multiplies the
+// softmax scale of the tile instead; values are multiplied by theirs and rounded.  (6 prompts of 454-3 766 tokens, head_dim
+// 128: 508 against 516 us with everything; head_dim 64: 329 against 360.)
+//
 // Softmax: exponentials are taken against a per-row reference that moves only when a score exceeds it by a window
 // (2^30 as the largest probability with bf16 operands, 2^8 with fp16); the row sums come out of the matrix cores
 // (an all-ones A fragment).  A move of the reference rescales the accumulators, the sums and the one step of
@@ -36,25 +46,29 @@
 namespace mi {
 
 constexpr int kWvTile = 64;                      // keys per staged tile
-constexpr int kWvPitch = 288;                    // LDS bytes per staged row (256 + 32: conflict-free fragment reads)
-constexpr int kWvPieces = kWvPitch / 16;         // 16-byte pieces per staged row
-constexpr int kWvLoads = kWvTile * kWvPieces / 64;  // direct loads (64 lanes x 16 bytes) per tile: 18
-constexpr int kWvBuf = kWvLoads * 1024;          // bytes per tile buffer
 constexpr int kWvDepth = 1;                      // tiles between the issue of a tile's loads and the barrier that needs them
-constexpr int kWvAhead = 3;                      // fragments requested ahead of their products (the stream: 16 per 32-key slot)
+constexpr int kWvAhead = 3;                      // fragments requested ahead of their products
 constexpr int kWvRing = 4;                       // fragment registers: fragment n lives in slot n % kWvRing
-static_assert(kWvAhead < kWvRing && kWvAhead <= 8 && 16 % kWvRing == 0, "next slot's key fragments are requested after the tile's barrier");
-constexpr bool wv_piece_division_ok() {
-  for (unsigned u = 0; u < 64u * kWvLoads; ++u)
-    if (((u * 3641u) >> 16) != u / 18u) return false;
+// LDS bytes per staged row: the row and 32 bytes of padding (288 or 160: conflict-free fragment reads)
+template <int HD> constexpr int wv_pitch() { return 2 * HD + 32; }
+template <int HD> constexpr int wv_waves() { return HD == 64 ? 4 : 8; }
+// piece u of a tile's line -> its row, by multiplication
+template <int HD> constexpr unsigned wv_magic() { return 65536u / (wv_pitch<HD>() / 16) + 1; }
+template <int HD> constexpr bool wv_piece_division_ok() {
+  for (unsigned u = 0; u < (unsigned)(kWvTile * wv_pitch<HD>() / 16); ++u)
+    if (((u * wv_magic<HD>()) >> 16) != u / (wv_pitch<HD>() / 16)) return false;
   return true;
 }
-static_assert((kWvDepth == 1 || kWvDepth == 2) && kWvPieces == 18 && kWvBuf == kWvTile * kWvPitch && wv_piece_division_ok(), "piece -> (row, column) by multiplication");
+static_assert((kWvDepth == 1 || kWvDepth == 2) && wv_piece_division_ok<128>() && wv_piece_division_ok<64>(), "piece -> (row, column)");
 
-template <bool SPLIT, bool F16>
-__global__ __launch_bounds__(512, 2) void paged_prefill_woven_kernel(PrefillParams p) {
-  constexpr int HD = 128, KS = HD / 32, DV = HD / 16, NQ = 2, WAVES = 8;
-  constexpr int PITCH = kWvPitch, BUF = kWvBuf;
+template <int HD, bool FP8, bool SPLIT, bool F16>
+__global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_prefill_woven_kernel(PrefillParams p) {
+  constexpr int KS = HD / 32, DV = HD / 16, NQ = 2, WAVES = wv_waves<HD>(), THREADS = 64 * WAVES;
+  constexpr int PITCH = wv_pitch<HD>(), PIECES = PITCH / 16, LOADS = kWvTile * PIECES / 64, BUF = LOADS * 1024;
+  constexpr int NKF = 2 * KS, NVF = DV;  // key and value fragments of a 32-key slot
+  constexpr int ESZ = FP8 ? 1 : 2;       // bytes per cache element
+  static_assert(HD == 128 || HD == 64, "head widths");
+  static_assert(kWvAhead < kWvRing && kWvAhead <= NKF && (NKF + NVF) % kWvRing == 0, "next slot's key fragments are requested after the tile's barrier");
   // DEPTH: how many tiles ahead of their barrier the loads of a tile pair are issued.  Key tile t lives in
   // Ks[t % KBUFS], value tile t in Vs[(t + 1) % VBUFS] (values are multiplied one tile after their keys).
   constexpr int DEPTH = kWvDepth, KBUFS = DEPTH + 1, VBUFS = DEPTH + 2;
@@ -76,7 +90,7 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_woven_kernel(PrefillPara
   if (rank == 0 && (!SPLIT || blockIdx.y == 0)) {
     const int tq = p.cu_q[p.R];
     const int per_row = G * HD;
-    for (int64_t i = (int64_t)tid * 8; i < (int64_t)(p.T - tq) * per_row; i += 512 * 8) {
+    for (int64_t i = (int64_t)tid * 8; i < (int64_t)(p.T - tq) * per_row; i += THREADS * 8) {
       const int row = (int)(i / per_row), e = (int)(i - (int64_t)row * per_row);
       st16(p.out + (int64_t)(tq + row) * p.o_st + (int64_t)(hq0 + e / HD) * p.o_sh + (e % HD), make_uint4(0, 0, 0, 0));
     }
@@ -153,36 +167,65 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_woven_kernel(PrefillPara
       return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(x >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((int)x);
     };
     // (48-bit addresses: what a descriptor's second word holds above them are its stride and swizzle fields)
-    const uint64_t kbase = uniform64((uint64_t)(uintptr_t)(p.kc + (int64_t)h * p.kv_sh * 2)) & 0xffffffffffffull;
-    const uint64_t vbase = uniform64((uint64_t)(uintptr_t)(p.vc + (int64_t)h * p.kv_sh * 2)) & 0xffffffffffffull;
+    const uint64_t kbase = uniform64((uint64_t)(uintptr_t)(p.kc + (int64_t)h * p.kv_sh * ESZ)) & 0xffffffffffffull;
+    const uint64_t vbase = uniform64((uint64_t)(uintptr_t)(p.vc + (int64_t)h * p.kv_sh * ESZ)) & 0xffffffffffffull;
     const int last_key = __builtin_amdgcn_readfirstlane(last);
-    const int64_t chunk_bytes = p.kv_sc * 2;
-    const int tok_bytes = p.kv_st * 2;
+    const int64_t chunk_bytes = p.kv_sc * ESZ;
+    const int tok_bytes = p.kv_st * ESZ;
     const int tiles_per_chunk = p.chunk / kWvTile;
     const int tile_bytes = kWvTile * tok_bytes;
     const int32_t* bt_row = p.bt + (int64_t)r * p.bt_stride;
     const uint32_t ks_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)&Ks[0][0];
     const uint32_t vs_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)&Vs[0][0];
 
-    // ---- this wavefront's five direct loads of a tile pair {key tile, value tile} -------------------------------
-    // Load k of the pair's 36 (0-17: the key tile's line, 18-35: the value tile's) belongs to wavefront k % 8; the
-    // fifth load of wavefronts 4-7 repeats their fourth, so that every wavefront issues five per tile.
-    // Loads 0 and 1 are key loads and loads 3 and 4 value loads for every wavefront; load 2 is a key load for
-    // wavefronts 0 and 1 only.
-    static_assert(kWvLoads == 18, "which of a wavefront's five loads belong to the key tile");
+    // ---- 16-bit cache: this wavefront's five direct loads of a tile pair {key tile, value tile} -------------------
+    // Load k of the pair's 2 LOADS (the first half: the key tile's line, the second: the value tile's) belongs to
+    // wavefront k % WAVES; with 36 loads over 8 wavefronts the fifth load of wavefronts 4-7 repeats their fourth, so
+    // that every wavefront issues five per tile.  Loads 0 and 1 are key loads and loads 3 and 4 value loads for every
+    // wavefront; load 2 is a key load for wavefronts 0 and 1 only.
+    static_assert(LOADS == 2 * WAVES + 2, "which of a wavefront's five loads belong to the key tile");
     uint32_t ld_off[5];   // per lane: where its piece of the load comes from, relative to the tile's first row
     uint32_t ld_dst[5];   // scalar: LDS offset of the load's 1 KiB inside its tile buffer
     const bool third_is_key = wave < 2;
+    if constexpr (!FP8) {
 #pragma unroll
-    for (int i = 0; i < 5; ++i) {
-      const int k = wave + 8 * i < 2 * kWvLoads ? wave + 8 * i : wave + 8 * i - 8;
-      const bool is_key = k < kWvLoads;
-      const int kp = is_key ? k : k - kWvLoads;
-      ld_dst[i] = (uint32_t)__builtin_amdgcn_readfirstlane(1024 * kp);
-      const uint32_t u = 64u * (uint32_t)kp + (uint32_t)lane;
-      const uint32_t prow = (u * 3641u) >> 16, pcol = u - 18u * prow;
-      ld_off[i] = prow * (uint32_t)tok_bytes + 16u * min(pcol, 15u);
+      for (int i = 0; i < 5; ++i) {
+        const int k = wave + WAVES * i < 2 * LOADS ? wave + WAVES * i : wave + WAVES * i - WAVES;
+        const bool is_key = k < LOADS;
+        const int kp = is_key ? k : k - LOADS;
+        ld_dst[i] = (uint32_t)__builtin_amdgcn_readfirstlane(1024 * kp);
+        const uint32_t u = 64u * (uint32_t)kp + (uint32_t)lane;
+        const uint32_t prow = (u * wv_magic<HD>()) >> 16, pcol = u - (uint32_t)PIECES * prow;
+        ld_off[i] = prow * (uint32_t)tok_bytes + 16u * min(pcol, (uint32_t)(PIECES - 3));
+      }
     }
+    // ---- fp8 cache: a thread fetches 8 bytes (8 elements) of two rows of a tile into registers, one tile ahead, and
+    // stores them converted.  Keys are converted exactly (e4m3 is a subset of both 16-bit types) and their scale goes
+    // into the softmax scale of their tile; values are multiplied by their scale and rounded.
+    constexpr int PPR8 = HD / 8, RPP8 = THREADS / PPR8;
+    static_assert(2 * RPP8 == kWvTile, "two rows per thread");
+    uint2 kraw[2], vraw[2];
+    const uint32_t f_piece = 8u * (uint32_t)(tid % PPR8), f_row0 = (uint32_t)(tid / PPR8) * (uint32_t)tok_bytes + f_piece,
+                   f_row1 = f_row0 + (uint32_t)RPP8 * (uint32_t)tok_bytes;
+    const int f_lds = (tid / PPR8) * PITCH + 16 * (tid % PPR8);
+    // rows past the request's last key re-read that row (every query row masks them); `nrec`: see tile_nrec
+    auto fetch_fp8 = [&](const uint8_t* cache, int64_t off, uint32_t nrec, uint2 (&reg)[2]) {
+      const uint8_t* src = cache + (int64_t)h * p.kv_sh + off;
+      const uint32_t lim = nrec - (uint32_t)tok_bytes + f_piece;
+      reg[0] = ld8(src + min(f_row0, lim));
+      reg[1] = ld8(src + min(f_row1, lim));
+    };
+    auto store_k_fp8 = [&](uint8_t* buf, int i) {
+      const uint2 lo = fp8x4_to_16x4<F16>(kraw[i].x), hi = fp8x4_to_16x4<F16>(kraw[i].y);
+      *reinterpret_cast<uint4*>(buf + f_lds + i * RPP8 * PITCH) = make_uint4(lo.x, lo.y, hi.x, hi.y);
+    };
+    auto store_v_fp8 = [&](uint8_t* buf, int i, float vscale) {
+      const f32x2_t a = fp8x2_lo_to_f32(vraw[i].x), b = fp8x2_hi_to_f32(vraw[i].x);
+      const f32x2_t c = fp8x2_lo_to_f32(vraw[i].y), d = fp8x2_hi_to_f32(vraw[i].y);
+      *reinterpret_cast<uint4*>(buf + f_lds + i * RPP8 * PITCH) =
+          make_uint4(pack2<F16>(a.x * vscale, a.y * vscale), pack2<F16>(b.x * vscale, b.y * vscale),
+                     pack2<F16>(c.x * vscale, c.y * vscale), pack2<F16>(d.x * vscale, d.y * vscale));
+    };
     // descriptor of a tile: its rows up to the request's last key (reads beyond return zeros)
     auto tile_rsrc = [&](uint64_t base, int64_t off, uint32_t nrec) {
       const uint64_t a = base + (uint64_t)off;
@@ -227,9 +270,24 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_woven_kernel(PrefillPara
       return pc;
     };
     auto bt_arrived = [&](int& pc) { asm volatile("s_waitcnt lgkmcnt(0)" : "+s"(pc)::"memory"); };
+    // fp8: a tile's block-table entry, then its two scales, by vector loads (one address for all lanes) that the
+    // compiler tracks with the other loads into registers: a value in flight across the loop's edge may be copied there
+    int vzero = 0;
+    asm volatile("" : "+v"(vzero));
+    int pc_v = 0;
+    float ks_v = 1.f, vs_v = 1.f;
+    auto scales_request = [&](int pc) {
+      ks_v = p.k_scale[(int64_t)pc * p.Hkv + h + vzero];
+      vs_v = p.v_scale[(int64_t)pc * p.Hkv + h + vzero];
+    };
+    auto uniform_float = [](float x) { return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x))); };
 
-    const float scale = p.scale_log2;
-    const float win = (F16 ? 8.f : 30.f) / scale;
+    // 16-bit: scores and references in raw units, one scale for all.  fp8: references in scaled units, since the scale
+    // belongs to a tile (kept off zero: zero times the -inf of a masked score would be NaN).
+    auto tile_scale = [&](float ks) { return FP8 ? fmaxf(ks * p.scale_log2, 1.17549435e-38f) : p.scale_log2; };
+    float scale_prev = p.scale_log2, scale_cur = p.scale_log2, scale_next = p.scale_log2, vscale = 1.f;
+    const float ref_scale = FP8 ? 1.f : p.scale_log2;   // reference units -> log2 units
+    const float win = (F16 ? 8.f : 30.f) / ref_scale;
     const uint4 ones = make_uint4(ones2<F16>(), ones2<F16>(), ones2<F16>(), ones2<F16>());
     const f32x4_t zero4 = {0.f, 0.f, 0.f, 0.f};
     // per-lane starts of the fragment reads inside a tile buffer
@@ -256,7 +314,7 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_woven_kernel(PrefillPara
       return make_uint4(a.x, a.y, b.x, b.y);
     };
     // probabilities of two scores (chunk c of a step's 8 per lane): rows nt = c >> 2, sub-tile (c >> 1) & 1, pair c & 1
-    auto exp_chunk = [&](const f32x4_t (&Sx)[NQ][2], uint4 (&Px)[NQ], int c) {
+    auto exp_chunk = [&](const f32x4_t (&Sx)[NQ][2], uint4 (&Px)[NQ], int c, float scale) {
       const int nt = c >> 2, u = (c >> 1) & 1, q2 = 2 * (c & 1);
       const float p0 = fast_exp2(__builtin_fmaf(Sx[nt][u][q2], scale, neg_run[nt]));
       const float p1 = fast_exp2(__builtin_fmaf(Sx[nt][u][q2 + 1], scale, neg_run[nt]));
@@ -268,11 +326,11 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_woven_kernel(PrefillPara
     auto move_reference = [&](float (&tmax)[NQ], uint4 (&Ppend)[NQ]) {
 #pragma unroll
       for (int nt = 0; nt < NQ; ++nt) {
-        const float tm = rowgroup_max(tmax[nt]);
+        const float tm = rowgroup_max(tmax[nt]);  // (already in the reference's units)
         const float m_raw = fmaxf(m_run[nt], tm);
         const float m_use = m_raw == -INFINITY ? 0.f : m_raw;
-        const float alpha = fast_exp2((m_run[nt] - m_use) * scale);
-        neg_run[nt] = -m_use * scale;
+        const float alpha = fast_exp2((m_run[nt] - m_use) * ref_scale);
+        neg_run[nt] = -m_use * ref_scale;
         m_run[nt] = m_raw;
         mwin[nt] = m_raw + win;
         if (__builtin_amdgcn_ballot_w64(alpha != 1.f)) {
@@ -292,18 +350,19 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_woven_kernel(PrefillPara
     // fragment starts in the key tile's and the value tile's buffers, ka_next in the next key tile's.  key0: position
     // of the first key of S[H] (MASK only).  at_barrier (H == 1): runs between the two groups of products.
     auto slot = [&](auto Hc, auto Mc, const uint8_t* ka, const uint8_t* ka_next, const uint8_t* va, int key0,
-                    auto&& at_barrier, auto&& under_products) {
+                    auto&& at_barrier, auto&& under_scores, auto&& under_values) {
       constexpr int H = decltype(Hc)::value;
       constexpr bool MASK = decltype(Mc)::value;
       f32x4_t (&Sn)[NQ][2] = S[H];
       const f32x4_t (&Sx)[NQ][2] = S[1 - H];
       uint4 (&Px)[NQ] = P[1 - H];
       const uint4 (&Pv)[NQ] = P[H];
-      // fragment n of the slot's stream: 0-7 key fragments, 8-15 value fragments, from 16 the next slot's first keys
+      const float scale = FP8 ? (H == 0 ? scale_prev : scale_cur) : p.scale_log2;  // of the scores in Sx
+      // fragment n of the slot's stream: NKF key fragments, NVF value fragments, then the next slot's first keys
       auto request = [&](int n) {
-        if (n < 8) fr[n % RING] = read_k(ka, H, n);
-        else if (n < 16) fr[n % RING] = read_v(va, H, n - 8);
-        else fr[n % RING] = H == 0 ? read_k(ka, 1, n - 16) : read_k(ka_next, 0, n - 16);
+        if (n < NKF) fr[n % RING] = read_k(ka, H, n);
+        else if (n < NKF + NVF) fr[n % RING] = read_v(va, H, n - NKF);
+        else fr[n % RING] = H == 0 ? read_k(ka, 1, n - NKF - NVF) : read_k(ka_next, 0, n - NKF - NVF);
       };
       // The probabilities of S[1-H], two scores ("chunk") at a time in three stages -- scale and subtract, exponential,
       // pack -- one stage of three different chunks per position, so that no instruction waits for the one before it:
@@ -326,57 +385,68 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_woven_kernel(PrefillPara
         }
       };
       // scores: sub-tiles alternate, so a product meets its accumulator again four products later
+      constexpr int EPP = 8 / NKF;  // positions of the probabilities' stages per key fragment: 1, or 2 at head width 64
 #pragma unroll
-      for (int n = 0; n < 8; ++n) {
+      for (int n = 0; n < NKF; ++n) {
         request(n + AHEAD);
         MI_SB();
         const int u = n & 1, kk = n >> 1;
         Sn[0][u] = mfma_16x16x32<F16>(fr[n % RING], qf[0][kk], kk ? Sn[0][u] : zero4);
         Sn[1][u] = mfma_16x16x32<F16>(fr[n % RING], qf[1][kk], kk ? Sn[1][u] : zero4);
         MI_SB();
-        exp_stages(n);
+#pragma unroll
+        for (int i = 0; i < EPP; ++i) exp_stages(EPP * n + i);
+        under_scores(n);
         MI_SB();
       }
       if constexpr (H == 1) at_barrier();
       float tmax[NQ];
       int dpos[NQ];
-      // values; beside them the last probabilities, then mask and maximum of the scores just multiplied
-#pragma unroll
-      for (int n = 8; n < 16; ++n) {
-        request(n + AHEAD);
-        MI_SB();
-        const int e = n - 8;
-        acc[0][e] = mfma_16x16x32<F16>(fr[n % RING], Pv[0], acc[0][e]);
-        acc[1][e] = mfma_16x16x32<F16>(fr[n % RING], Pv[1], acc[1][e]);
-        MI_SB();
-        if (n < 10) exp_stages(n);
-        if constexpr (H == 1) under_products(n - 8);
-        if (n == 11 && MASK) {
+      // mask and maximum of the scores just multiplied: step i = rows i >> 1, part i & 1
+      auto max_step = [&](int i) {
+        const int nt = i >> 1, part = i & 1;
+        if (MASK && i == 0) {
           const int tok0 = key0 + 4 * g;
           dpos[0] = qpos[0] - tok0;
           dpos[1] = qpos[1] - tok0;
         }
-        if (n >= 11 && n < 15) {  // rows (n - 11) >> 1 of the scores just multiplied, in two parts
-          const int nt = (n - 11) >> 1, part = (n - 11) & 1;
-          if (MASK && part == 0) {
-            // (every masked score is out of the way before the first maximum is taken: a masked key's score in the
-            // reference would cost fp16 probabilities their precision)
+        if (MASK && part == 0) {
+          // (every masked score is out of the way before the first maximum is taken: a masked key's score in the
+          // reference would cost fp16 probabilities their precision)
 #pragma unroll
-            for (int u = 0; u < 2; ++u)
+          for (int u = 0; u < 2; ++u)
 #pragma unroll
-              for (int i = 0; i < 4; ++i)
-                if (16 * u + i > dpos[nt]) Sn[nt][u][i] = -INFINITY;
-          }
-          // a chain of three-operand maxima
-          if (MASK ? part == 1 : part == 0) {
-            tmax[nt] = fmaxf(fmaxf(Sn[nt][0][0], Sn[nt][0][1]), Sn[nt][0][2]);
-            tmax[nt] = fmaxf(fmaxf(tmax[nt], Sn[nt][0][3]), Sn[nt][1][0]);
-          }
-          if (part == 1) {
-            tmax[nt] = fmaxf(fmaxf(tmax[nt], Sn[nt][1][1]), Sn[nt][1][2]);
-            tmax[nt] = fmaxf(tmax[nt], Sn[nt][1][3]);
-          }
+            for (int i2 = 0; i2 < 4; ++i2)
+              if (16 * u + i2 > dpos[nt]) Sn[nt][u][i2] = -INFINITY;
         }
+        // a chain of three-operand maxima
+        if (MASK ? part == 1 : part == 0) {
+          tmax[nt] = fmaxf(fmaxf(Sn[nt][0][0], Sn[nt][0][1]), Sn[nt][0][2]);
+          tmax[nt] = fmaxf(fmaxf(tmax[nt], Sn[nt][0][3]), Sn[nt][1][0]);
+        }
+        if (part == 1) {
+          tmax[nt] = fmaxf(fmaxf(tmax[nt], Sn[nt][1][1]), Sn[nt][1][2]);
+          tmax[nt] = fmaxf(tmax[nt], Sn[nt][1][3]);
+          if (FP8) tmax[nt] *= scale_cur;
+        }
+      };
+      // values; beside them the last probabilities, then mask and maximum of the scores just multiplied
+#pragma unroll
+      for (int e = 0; e < NVF; ++e) {
+        const int n = NKF + e;
+        request(n + AHEAD);
+        MI_SB();
+        acc[0][e] = mfma_16x16x32<F16>(fr[n % RING], Pv[0], acc[0][e]);
+        acc[1][e] = mfma_16x16x32<F16>(fr[n % RING], Pv[1], acc[1][e]);
+        MI_SB();
+        if (HD == 128) {
+          if (e < 2) exp_stages(8 + e);
+          if (e >= 3 && e < 7) max_step(e - 3);
+        } else {
+          if (e == 0) { exp_stages(8); exp_stages(9); }
+          if (e == 1 || e == 2) { max_step(2 * e - 2); max_step(2 * e - 1); }
+        }
+        under_values(e);
         MI_SB();
       }
       accl[0] = mfma_16x16x32<F16>(ones, Pv[0], accl[0]);
@@ -387,18 +457,28 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_woven_kernel(PrefillPara
     };
 
     // ---- prologue: clear the buffers (the value tile "before the first" must hold zeros), start the first tiles ----
-    for (int i = tid * 16; i < KBUFS * BUF; i += 512 * 16) *reinterpret_cast<uint4*>(&Ks[0][0] + i) = make_uint4(0u, 0u, 0u, 0u);
-    for (int i = tid * 16; i < VBUFS * BUF; i += 512 * 16) *reinterpret_cast<uint4*>(&Vs[0][0] + i) = make_uint4(0u, 0u, 0u, 0u);
+    for (int i = tid * 16; i < KBUFS * BUF; i += THREADS * 16) *reinterpret_cast<uint4*>(&Ks[0][0] + i) = make_uint4(0u, 0u, 0u, 0u);
+    for (int i = tid * 16; i < VBUFS * BUF; i += THREADS * 16) *reinterpret_cast<uint4*>(&Vs[0][0] + i) = make_uint4(0u, 0u, 0u, 0u);
     Cursor cur = cursor_at(tb + DEPTH + 1);
     int64_t off_first[DEPTH + 1];   // tiles tb .. tb + DEPTH, started here
     uint32_t nrec_first[DEPTH + 1];
 #pragma unroll
     for (int i = 0; i <= DEPTH; ++i) {
       const Cursor c = cursor_at(tb + i);
-      off_first[i] = tile_off(c, __builtin_amdgcn_readfirstlane(bt_row[c.ci]));
+      const int pc = __builtin_amdgcn_readfirstlane(bt_row[c.ci]);
+      off_first[i] = tile_off(c, pc);
       nrec_first[i] = tile_nrec(c);
+      if constexpr (FP8) {
+        scales_request(pc);
+        if (i == 0) {
+          scale_prev = scale_cur = tile_scale(uniform_float(ks_v));
+          vscale = uniform_float(vs_v);
+        }
+      }
     }
-    int pc_next = __builtin_amdgcn_readfirstlane(bt_row[cur.ci]);
+    int pc_next = 0;
+    if constexpr (FP8) pc_v = bt_row[cur.ci + vzero];
+    else pc_next = __builtin_amdgcn_readfirstlane(bt_row[cur.ci]);
     // (the query fragments count as used here: the compiler then waits for their loads now and not in the tile
     // loop, where a wait on the vector-memory counter would wait for the direct loads in flight as well)
 #pragma unroll
@@ -409,7 +489,17 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_woven_kernel(PrefillPara
     __syncthreads();  // the cleared buffers are in place before the first direct load can land
     int64_t off_prev;
     uint32_t nrec_prev;
-    {
+    if constexpr (FP8) {
+      static_assert(!FP8 || DEPTH == 1, "fp8 tiles wait in one set of registers");
+      fetch_fp8(p.kc, off_first[0], nrec_first[0], kraw);
+      store_k_fp8(&Ks[0][0], 0);
+      store_k_fp8(&Ks[0][0], 1);
+      fetch_fp8(p.kc, off_first[1], nrec_first[1], kraw);  // stored by iteration 0
+      fetch_fp8(p.vc, off_first[0], nrec_first[0], vraw);
+      off_prev = off_first[1];
+      nrec_prev = nrec_first[1];
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    } else {
       const u32x4_t rk0 = tile_rsrc(kbase, off_first[0], nrec_first[0]);
 #pragma unroll
       for (int i = 0; i < 5; ++i)
@@ -425,8 +515,10 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_woven_kernel(PrefillPara
       nrec_prev = nrec_first[DEPTH];
     }
     // key tile 0 has landed (this wavefront's share): only the DEPTH pairs issued after it may still be on their way
-    if constexpr (DEPTH == 1) asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
+    if constexpr (!FP8) {
+      if constexpr (DEPTH == 1) asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
+      else asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
+    }
     __builtin_amdgcn_s_barrier();
     MI_SB();
 
@@ -449,26 +541,58 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_woven_kernel(PrefillPara
       u32x4_t rs_k, rs_v;
       const uint32_t kdst = ks_lds + (uint32_t)kb;
       const uint32_t vdst = vs_lds + (uint32_t)((vbi == 0 ? VBUFS - 1 : vbi - 1) * BUF);  // (j - 1) % VBUFS
-      slot(std::integral_constant<int, 0>{}, Mc, ka, ka_next, va, key0, [] {}, [](int) {});
+      // fp8: key tile j+1 and value tile j, fetched since the last barrier, go into LDS before this iteration's barrier
+      uint8_t* const kst = &Ks[0][0] + (kbi == KBUFS - 1 ? 0 : kbi + 1) * BUF;
+      uint8_t* const vst = &Vs[0][0] + (vbi == VBUFS - 1 ? 0 : vbi + 1) * BUF;
+      slot(std::integral_constant<int, 0>{}, Mc, ka, ka_next, va, key0, [] {}, [](int) {},
+           [&](int e) {
+             if constexpr (FP8) {
+               if (e == NVF - 2) store_k_fp8(kst, 0);
+               if (e == NVF - 1) store_k_fp8(kst, 1);
+             }
+           });
       slot(std::integral_constant<int, 1>{}, Mc, ka, ka_next, va, key0 + 32,
            [&] {
              // this wavefront's share of key tile j+1 and value tile j has landed: only younger pairs are on their way
-             if constexpr (DEPTH == 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+             if constexpr (FP8) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+             else if constexpr (DEPTH == 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
              else asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
              __builtin_amdgcn_s_barrier();
-             bt_arrived(pc_next);
+             if constexpr (FP8) pc_next = __builtin_amdgcn_readfirstlane(pc_v);
+             else bt_arrived(pc_next);
              const int64_t off = tile_off(cur, pc_next);
              const uint32_t nrec = tile_nrec(cur);
-             rs_k = tile_rsrc(kbase, off, nrec);
-             rs_v = tile_rsrc(vbase, off_prev, nrec_prev);
+             if constexpr (FP8) {
+               scale_next = tile_scale(uniform_float(ks_v));  // (of tile j+1)
+               vscale = uniform_float(vs_v);
+               scales_request(pc_next);
+               fetch_fp8(p.kc, off, nrec, kraw);
+               fetch_fp8(p.vc, off_prev, nrec_prev, vraw);
+             } else {
+               rs_k = tile_rsrc(kbase, off, nrec);
+               rs_v = tile_rsrc(vbase, off_prev, nrec_prev);
+             }
              off_prev = off;
              nrec_prev = nrec;
              cursor_next(cur);
-             pc_next = bt_request(cur.ci);
+             if constexpr (FP8) pc_v = bt_row[cur.ci + vzero];
+             else pc_next = bt_request(cur.ci);
            },
-           [&](int i) {
-             if (i < 5) issue_load(i, rs_k, rs_v, kdst, vdst);
+           [&](int n) {
+             if constexpr (FP8) {
+               if (n < 2) store_v_fp8(vst, n, vscale);
+             }
+           },
+           [&](int e) {
+             if constexpr (!FP8) {
+               if (e < 5) issue_load(e, rs_k, rs_v, kdst, vdst);
+               if (e == NVF - 1 && NVF < 5) issue_load(4, rs_k, rs_v, kdst, vdst);
+             }
            });
+      if constexpr (FP8) {
+        scale_prev = scale_cur;
+        scale_cur = scale_next;
+      }
       ++j;
       kbi = kbi == KBUFS - 1 ? 0 : kbi + 1;
       vbi = vbi == VBUFS - 1 ? 0 : vbi + 1;
@@ -491,7 +615,7 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_woven_kernel(PrefillPara
       };
       values(0, P[0]);
 #pragma unroll
-      for (int c = 0; c < 8; ++c) exp_chunk(S[1], P[1], c);
+      for (int c = 0; c < 8; ++c) exp_chunk(S[1], P[1], c, FP8 ? scale_prev : p.scale_log2);
       values(1, P[1]);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no direct load may still be on its way into this workgroup's LDS
@@ -519,18 +643,29 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_woven_kernel(PrefillPara
         for (int e = 0; e < DV; ++e)
           *reinterpret_cast<float4*>(o + 16 * e) =
               make_float4(acc[nt][e][0] * inv, acc[nt][e][1] * inv, acc[nt][e][2] * inv, acc[nt][e][3] * inv);
-        if (g == 0) p.split_lse[prow] = l_tot > 0.f ? m_run[nt] * p.scale_log2 + fast_log2(l_tot) : -INFINITY;
+        if (g == 0) p.split_lse[prow] = l_tot > 0.f ? m_run[nt] * (FP8 ? 1.f : p.scale_log2) + fast_log2(l_tot) : -INFINITY;
       }
     }
   }
 }
 
-void launch_prefill_woven(const PrefillParams& p, dim3 grid, bool f16, hipStream_t st) {
+int prefill_woven_waves(int head_dim) { return head_dim == 64 ? wv_waves<64>() : wv_waves<128>(); }
+
+void launch_prefill_woven(const PrefillParams& p, dim3 grid, int head_dim, bool fp8, bool f16, hipStream_t st) {
   const bool split = grid.y > 1;
-  if (split && f16) hipLaunchKernelGGL((paged_prefill_woven_kernel<true, true>), grid, dim3(512), 0, st, p);
-  else if (split) hipLaunchKernelGGL((paged_prefill_woven_kernel<true, false>), grid, dim3(512), 0, st, p);
-  else if (f16) hipLaunchKernelGGL((paged_prefill_woven_kernel<false, true>), grid, dim3(512), 0, st, p);
-  else hipLaunchKernelGGL((paged_prefill_woven_kernel<false, false>), grid, dim3(512), 0, st, p);
+#define MI_WV_LAUNCH(HD_, FP8_)                                                                                     \
+  do {                                                                                                              \
+    const dim3 block(64 * wv_waves<HD_>());                                                                         \
+    if (split && f16) hipLaunchKernelGGL((paged_prefill_woven_kernel<HD_, FP8_, true, true>), grid, block, 0, st, p); \
+    else if (split) hipLaunchKernelGGL((paged_prefill_woven_kernel<HD_, FP8_, true, false>), grid, block, 0, st, p); \
+    else if (f16) hipLaunchKernelGGL((paged_prefill_woven_kernel<HD_, FP8_, false, true>), grid, block, 0, st, p);  \
+    else hipLaunchKernelGGL((paged_prefill_woven_kernel<HD_, FP8_, false, false>), grid, block, 0, st, p);          \
+  } while (0)
+  if (head_dim == 64 && fp8) MI_WV_LAUNCH(64, true);
+  else if (head_dim == 64) MI_WV_LAUNCH(64, false);
+  else if (fp8) MI_WV_LAUNCH(128, true);
+  else MI_WV_LAUNCH(128, false);
+#undef MI_WV_LAUNCH
 }
 
 }  // namespace mi
