@@ -67,8 +67,8 @@ typedef struct MiTuning {
   int32_t decode_grid;            /* decode kernels, spans the tile sequence is cut into: 0 = automatic, 1..65535 */
   int32_t decode_waves_per_block; /* decode kernel, KV heads per workgroup: 0 = default (8), 1..8 */
   int32_t prefill_two_phase;      /* prefill tile kernel: 0 = default (3), 1 = two-phase kernel, 2 = the same with its
-                                     wave groups in lock-step, 3 = one-stream kernel where it applies (head_dim 128 over a
-                                     16-bit cache; the two-phase kernel elsewhere), -1 = register-only kernel */
+                                     wave groups in lock-step, 3 = one-stream kernel where it applies (head_dim 64 and 128;
+                                     the two-phase kernel elsewhere), -1 = register-only kernel */
   int32_t prefill_tile_subtiles;  /* register-only prefill kernel, 16-key sub-tiles per iteration: 0 = default (2), 1, 2 */
   int32_t prefill_row_tiles;      /* register-only prefill kernel, 16-row tiles per wavefront: 0 = default (2), 2, 4 */
   int32_t prefill_kv_split;       /* two-phase kernel, key ranges per request: 0 = from T and max_kv_len, -1 = never,
@@ -160,6 +160,15 @@ int mi_kv_append_fp8(const void* key, const void* value, int64_t src_stride_tok,
                      const int64_t* token_to_chunk_idx, const int64_t* token_to_local_pos, int32_t T,
                      int32_t chunk_tokens, int32_t Hkv, int32_t head_dim, float headroom, int32_t dtype,
                      void* stream);
+
+/* The same for keys and values that have strides of their own, between tokens and between heads (elements): the
+ * value rows of a QKV projection's output, for instance. */
+int mi_kv_append_fp8_strided(const void* key, int64_t k_stride_tok, int64_t k_stride_head, const void* value,
+                             int64_t v_stride_tok, int64_t v_stride_head, void* k_cache_fp8, void* v_cache_fp8,
+                             int64_t kv_stride_chunk, int64_t kv_stride_tok, float* k_scales, float* v_scales,
+                             const int64_t* token_to_chunk_idx, const int64_t* token_to_local_pos, int32_t T,
+                             int32_t chunk_tokens, int32_t Hkv, int32_t head_dim, float headroom, int32_t dtype,
+                             void* stream);
 
 /*
  * Bytes of workspace mi_paged_decode_attention needs for these sizes on the current

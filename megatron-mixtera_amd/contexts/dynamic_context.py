@@ -666,7 +666,7 @@ class DynamicInferenceContext:
                 rotary_interleaved=self._rope_flags(config) if config is not None else False, mscale=mscale,
                 faithful_rounding=faithful_rounding)
             group = num_query_heads // hkv
-            value = mixed_qkv[:n].reshape(n, hkv, (group + 2) * d)[:, :, (group + 1) * d:].contiguous()
+            value = mixed_qkv[:n].reshape(n, hkv, (group + 2) * d)[:, :, (group + 1) * d:]
             self.append_key_value_cache(layer_number, key_out, value.unsqueeze(1))
             return query_out
         k_cache, v_cache = self._layer_cache(layer_number)

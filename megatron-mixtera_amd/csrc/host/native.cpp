@@ -343,11 +343,9 @@ PyObject* kv_append_fp8(PyObject* const* a) {
   const Tensor &ks = tensor(a[4], "k_scales"), &vs = tensor(a[5], "v_scales");
   const Tensor &chunk = tensor(a[6], "token_to_chunk_idx"), &local = tensor(a[7], "token_to_local_pos");
   REQUIRE(is_16bit(key) && value.scalar_type() == key.scalar_type(),
-          "K/V must share one 16-bit type and have equal shapes and strides");
+          "K/V must share one 16-bit type and have equal shapes");
   const Rows3 k3 = rows3(key, "key"), v3 = rows3(value, "value");
-  REQUIRE(k3.sh == k3.d && v3.sh == v3.d, "key / value rows must be contiguous");
-  REQUIRE(k3.n == v3.n && k3.h == v3.h && k3.d == v3.d && k3.sn == v3.sn,
-          "K/V must share one 16-bit type and have equal shapes and strides");
+  REQUIRE(k3.n == v3.n && k3.h == v3.h && k3.d == v3.d, "K/V must share one 16-bit type and have equal shapes");
   REQUIRE(kc.element_size() == 1 && vc.element_size() == 1, "fp8 caches hold one byte per element");
   const Cache kcache = cache_of(kc);
   REQUIRE(same_strides(cache_of(vc), kcache) && kcache.sh == kcache.d && k3.h * k3.d == kcache.h * kcache.sh, "cache layout");
@@ -355,10 +353,14 @@ PyObject* kv_append_fp8(PyObject* const* a) {
   REQUIRE(ks.is_contiguous() && vs.is_contiguous(), "scales must be contiguous");
   check_index_row(&chunk, k3.n, "slot rows must be int64 [>=T]");
   check_index_row(&local, k3.n, "slot rows must be int64 [>=T]");
-  check(mi_kv_append_fp8(key.data_ptr(), value.data_ptr(), k3.sn, kc.data_ptr(), vc.data_ptr(), kcache.sc, kcache.st,
-                         (float*)ks.data_ptr(), (float*)vs.data_ptr(), (const int64_t*)chunk.data_ptr(),
-                         (const int64_t*)local.data_ptr(), (int)k3.n, (int)kcache.c, (int)kcache.h, (int)kcache.d,
-                         (float)as_float(a[8]), dtype_code(key), stream),
+  // (rows are split into the cache's heads; a source whose rows are whole may name its heads differently)
+  const bool whole = k3.sh == k3.d && v3.sh == v3.d;
+  REQUIRE(whole || (k3.h == kcache.h && k3.d == kcache.d), "key / value rows must be contiguous or have the cache's heads");
+  check(mi_kv_append_fp8_strided(key.data_ptr(), k3.sn, whole ? kcache.d : k3.sh, value.data_ptr(), v3.sn, whole ? kcache.d : v3.sh,
+                                 kc.data_ptr(), vc.data_ptr(), kcache.sc, kcache.st, (float*)ks.data_ptr(),
+                                 (float*)vs.data_ptr(), (const int64_t*)chunk.data_ptr(), (const int64_t*)local.data_ptr(),
+                                 (int)k3.n, (int)kcache.c, (int)kcache.h, (int)kcache.d, (float)as_float(a[8]),
+                                 dtype_code(key), stream),
         "mi_kv_append_fp8");
   Py_RETURN_NONE;
 }

@@ -32,3 +32,36 @@ def test_fp8_tiles(mi, dev, d, Hq, Hkv, split, dtype):
     ref = oa.paged_varlen_attention(q.cpu(), k8, v8, cu_q, kv_lens, bt, k_scales=ks, v_scales=vs)
     err = (out.float().cpu() - ref).abs()
     assert (err <= 2e-2 + 2e-2 * ref.abs()).all(), f"max err {err.max().item():.4e}"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("d,chunk", [(128, 256), (64, 128), (96, 64), (128, 320)])
+def test_fp8_append_from_strided_rows(mi, dev, d, chunk, dtype):
+    """Values read from a wider row; runs of one token, of two, across workgroups' slices, of whole chunks and of a chunk
+    that does not fit a workgroup's registers; scales beyond the range of the quick quotient; padded rows."""
+    Hkv, N = 3, 24
+    gen = torch.Generator().manual_seed(d + chunk)
+    reqs = [(0, chunk, [3]), (0, 2 * chunk + 17, [7, 1, 12]), (chunk - 5, 60, [5, 9]), (chunk, 2, [2, 14]), (0, 1, [20]),
+            (chunk - 1, 2, [6, 8]), (0, 2, [10]), (0, 31, [11])]
+    slots = [(chunks[pos // chunk], pos % chunk) for first, n, chunks in reqs for pos in range(first, first + n)]
+    real = len(slots)
+    slots += [(N - 1, 0)] * 40
+    T = len(slots)
+    tc, tl = (torch.tensor(x) for x in zip(*slots))
+    key = (torch.randn(T, Hkv, d, generator=gen) * 3).to(dtype)
+    wide = torch.randn(T, Hkv, 3 * d, generator=gen).to(dtype)
+    val = wide[:, :, 2 * d:]
+    key[chunk + 3, 1] = 0
+    val[real - 31:real] *= 1e-4
+    if dtype == torch.bfloat16:
+        key[real - 31:real, 2] *= 1e-30
+        val[0:chunk, 0] *= 1e30
+    k8 = torch.randint(0, 255, (N, chunk, Hkv, d), generator=gen, dtype=torch.uint8)
+    v8 = torch.randint(0, 255, (N, chunk, Hkv, d), generator=gen, dtype=torch.uint8)
+    ks, vs = torch.rand(N, Hkv, generator=gen) + 0.5, torch.rand(N, Hkv, generator=gen) * 1e-3
+    k8d, v8d, ksd, vsd = k8.to(dev), v8.to(dev), ks.to(dev), vs.to(dev)
+    mi.ops.kv_append_fp8(key.to(dev), wide.to(dev)[:, :, 2 * d:], k8d, v8d, ksd, vsd, tc.to(dev), tl.to(dev), headroom=1.5)
+    for cache, scales, rows, got_c, got_s in ((k8, ks, key, k8d, ksd), (v8, vs, val, v8d, vsd)):
+        oa.kv_append_fp8(cache, scales, rows[:real], tc[:real], tl[:real], headroom=1.5)
+        assert torch.equal(got_s.cpu()[:N - 1], scales[:N - 1])
+        assert torch.equal(got_c.cpu()[:N - 1], cache[:N - 1])
