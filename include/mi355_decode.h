@@ -361,6 +361,21 @@ int mi_paged_prefill_attention_fp8(const void* q, int64_t q_stride_tok, int64_t 
                                    void* stream);
 
 /*
+ * The same call (16-bit cache: kv_dtype = MI_KV_16BIT and null scales; or fp8) for a batch without requests of exactly
+ * one query row -- freshly admitted prompts, chunks of prompts: the decode kernels, which would find nothing to do, are
+ * not launched.  One-row requests are served all the same, at the speed of the tile kernel.
+ */
+int mi_paged_prefill_attention_tiles(const void* q, int64_t q_stride_tok, int64_t q_stride_head, const void* k_cache,
+                                     const void* v_cache, int64_t kv_stride_chunk, int64_t kv_stride_tok,
+                                     int64_t kv_stride_head, int32_t kv_dtype, const float* k_scales,
+                                     const float* v_scales, const int32_t* block_table, int64_t bt_stride,
+                                     const int32_t* cu_seqlens_q, const int32_t* kv_lens, void* out,
+                                     int64_t o_stride_tok, int64_t o_stride_head, void* workspace,
+                                     int64_t workspace_bytes, int32_t T, int32_t R, int32_t Hq, int32_t Hkv,
+                                     int32_t head_dim, int32_t chunk_tokens, int32_t max_kv_len, float softmax_scale,
+                                     int32_t dtype, const MiTuning* tuning, void* stream);
+
+/*
  * Paged varlen causal attention with keys wider than values: the prefill / mixed step of
  * multi-latent attention, where the reference decompresses the latent cache into a key cache
  * `[n_chunks, chunk_tokens, H, 192]` (128 + the 64 shared rotary values) and a value cache

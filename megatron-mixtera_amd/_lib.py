@@ -76,6 +76,10 @@ SIGNATURES = {
         c_int,
         [_P, _I64, _I64, _P, _P, _I64, _I64, _I64, _P, _P, _P, _I64, _P, _P, _P, _I64, _I64, _P, _I64,
          _I32, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _F, _I32, _P, _P]),
+    "mi_paged_prefill_attention_tiles": (
+        c_int,
+        [_P, _I64, _I64, _P, _P, _I64, _I64, _I64, _I32, _P, _P, _P, _I64, _P, _P, _P, _I64, _I64, _P, _I64,
+         _I32, _I32, _I32, _I32, _I32, _I32, _I32, _F, _I32, _P, _P]),
     "mi_paged_prefill_attention_mla": (
         c_int,
         [_P, _I64, _I64, _P, _I64, _I64, _I64, _P, _I64, _I64, _I64, _P, _I64, _P, _P, _P, _I64, _I64,

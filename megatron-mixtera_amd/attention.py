@@ -41,20 +41,21 @@ def adjust_key_value_for_inference(inference_context, layer_number: int, query: 
 def flash_decode_and_prefill(q: Tensor, k: Tensor, v: Tensor, max_seqlen_q, max_seqlen_k, cu_seqlens_q,
                              cu_seqlens_k, seqlens_k, block_table, softmax_scale: Optional[float] = None, *,
                              k_scales: Optional[Tensor] = None, v_scales: Optional[Tensor] = None,
-                             mla_head_dim_v: Optional[int] = None) -> Tensor:
+                             mla_head_dim_v: Optional[int] = None, one_row_requests: Optional[bool] = None) -> Tensor:
     """Same contract as ``Attention.flash_decode_and_prefill`` (attention.py:470-601).
 
     ``q`` is ``[T, 1, Hq, d]``; ``k`` / ``v`` are the paged caches.  ``max_seqlen_q == 1``
     selects the decode kernel, anything else the varlen causal kernel.  ``k_scales`` / ``v_scales``
     (an addition) go with byte caches holding e4m3 values.  ``mla_head_dim_v`` (the reference tests
     ``isinstance(self.config, MLATransformerConfig)`` and reads ``config.kv_lora_rank`` instead) selects the
-    absorbed multi-latent decode: ``k`` is then the latent cache and ``v`` is ``None``.
+    absorbed multi-latent decode: ``k`` is then the latent cache and ``v`` is ``None``.  ``one_row_requests`` goes to
+    ``flash_attn_varlen_func``.
     """
     if max_seqlen_q > 1:
         out = flash_attn_varlen_func(q.squeeze(1), k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
                                      softmax_scale=softmax_scale if softmax_scale is not None else q.shape[-1] ** -0.5,
                                      causal=True, block_table=block_table, seqused_k=seqlens_k,
-                                     k_scales=k_scales, v_scales=v_scales)
+                                     k_scales=k_scales, v_scales=v_scales, one_row_requests=one_row_requests)
         return out.unsqueeze(1)
     if mla_head_dim_v is not None:
         metadata, num_splits = get_mla_metadata(seqlens_k, q.size(2), 1)
@@ -182,12 +183,15 @@ class PagedSelfAttentionCore(torch.nn.Module):
             # maxima (cu_query_lengths / cu_kv_lengths, as the reference does) would wait for the device
             cu_q, cu_k, kv_lens = ctx.cu_query_seq_lengths, ctx.cu_kv_seq_lengths, ctx.kv_seq_lengths
             max_q, max_k = ctx.attention_length_bounds()
+            one_row = ctx.one_row_requests_possible()
         else:
+            one_row = True
             cu_q, max_q = ctx.cu_query_lengths()
             cu_k, kv_lens, max_k = ctx.cu_kv_lengths()
         k_scales, v_scales = ctx.key_value_scales(self.layer_number) if hasattr(ctx, "key_value_scales") else (None, None)
         out = flash_decode_and_prefill(query, k_cache, v_cache, max_q, max_k, cu_q, cu_k, kv_lens, block_table,
-                                       softmax_scale=self.softmax_scale, k_scales=k_scales, v_scales=v_scales)
+                                       softmax_scale=self.softmax_scale, k_scales=k_scales, v_scales=v_scales,
+                                       one_row_requests=one_row)
         return out.reshape(out.size(0), out.size(1), -1)
 
 

@@ -301,15 +301,17 @@ class DynamicInferenceContext:
             # The new counters of update_requests, and the largest query / kv length of a prefill or mixed step (only
             # waited for when somebody reads it), are written by their kernels straight into pinned host memory, where
             # the host watches one word of each: no copy to enqueue, no wait for the whole stream
-            self._counters = torch.zeros(8, dtype=torch.int32, pin_memory=True)
+            watched = torch.zeros(64, dtype=torch.int32, pin_memory=True)  # (a line of 128 bytes for each)
+            self._counters = watched[:8]
             self._counters_host = self._counters.numpy()
-            self._max_lengths = torch.zeros(2, dtype=torch.int32, pin_memory=True)
+            self._max_lengths = watched[32:34]
             self._max_lengths_host = self._max_lengths.numpy()
         self._max_lengths_pending = False     # nobody has read the step's maxima yet
         self._max_lengths_in_flight = False   # their kernel may not have run yet
         # what the host knows without asking the device: the longest prompt admitted since the last
         # update_requests (every other active request has one query token) and a bound on the kv lengths
         self._host_max_query_len = 1
+        self._host_one_row_requests = True
         self._host_kv_len_bound = 0
         # ids of the requests that finished in the last update_requests (fused bookkeeping), else None
         self.last_finished_request_ids = None
@@ -414,6 +416,11 @@ class DynamicInferenceContext:
             q_max = max(1, self._host_max_query_len)
         k_bound = min(self.max_sequence_length, max(1, self._host_kv_len_bound))
         return q_max, k_bound
+
+    def one_row_requests_possible(self) -> bool:
+        """Whether some request of this step may have exactly one query row, from what the host knows: requests that
+        an ``update_requests`` has carried over, prompts of one token, and every replay of a graph step."""
+        return self._host_one_row_requests or self.using_cuda_graph_this_step()
 
     def cu_query_lengths(self) -> Tuple[Optional[Tensor], int]:
         return self.cu_query_seq_lengths, self.max_seqlen_q
@@ -835,6 +842,7 @@ class DynamicInferenceContext:
         self.reset_attention_state()
         self.chunk_allocator.reset()
         self._host_max_query_len = 1
+        self._host_one_row_requests = True
         self._host_kv_len_bound = 0
         self.last_finished_request_ids = None
 
@@ -888,8 +896,7 @@ class DynamicInferenceContext:
                             self.chunk_allocator.chunk_count_avail, request_id, length + num_tokens_to_generate)
             self.total_request_count += 1
             self.active_token_count += length
-            self._host_max_query_len = max(self._host_max_query_len, length)
-            self._host_kv_len_bound = max(self._host_kv_len_bound, length)
+            self._note_admitted(length)
             return
         self.request_ids[row] = request_id
         self.request_query_lengths[row] = length
@@ -911,6 +918,12 @@ class DynamicInferenceContext:
 
         self.total_request_count += 1
         self.active_token_count += length
+        self._note_admitted(length)
+
+    def _note_admitted(self, length: int) -> None:
+        """What the host knows about this step's lengths, after a prompt went into the last row."""
+        first = self.total_request_count - self.paused_request_count == 1
+        self._host_one_row_requests = length == 1 or (self._host_one_row_requests and not first)
         self._host_max_query_len = max(self._host_max_query_len, length)
         self._host_kv_len_bound = max(self._host_kv_len_bound, length)
 
@@ -940,6 +953,7 @@ class DynamicInferenceContext:
         """
         # after this call every active request has one query token and one more key
         self._host_max_query_len = 1
+        self._host_one_row_requests = True
         self._host_kv_len_bound = min(self._host_kv_len_bound + 1, self.max_sequence_length)
         if self.fused_bookkeeping:
             return self._update_requests_fused(active_requests_mask, new_tokens)

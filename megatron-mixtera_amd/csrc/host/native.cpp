@@ -442,7 +442,7 @@ PyObject* paged_mla_decode_attention(PyObject* const* a) {
 }
 
 // paged_prefill_attention(q, k_cache, v_cache, cu_seqlens_q, kv_lens, block_table, softmax_scale|None, max_kv_len|None,
-//                         out|None, k_scales|None, v_scales|None, tuning|None, override|None)
+//                         out|None, k_scales|None, v_scales|None, tuning|None, override|None, one_row_requests)
 PyObject* paged_prefill_attention(PyObject* const* a) {
   const Tensor& q = tensor(a[0], "q");
   void* stream = stream_of(q);
@@ -472,7 +472,15 @@ PyObject* paged_prefill_attention(PyObject* const* a) {
   REQUIRE(o3.n == T && o3.h == q3.h && o3.d == q3.d && out.scalar_type() == q.scalar_type(), "out shape / dtype mismatch");
   const auto* tune = (const MiTuning*)host_struct(a[11]);
   const Scratch ws = scratch(q, stream, mi_prefill_workspace_bytes((int)T, (int)R, (int)q3.h, (int)c.h, (int)q3.d, (int)max_len, 0, tune), Py_None, a[12]);
-  if (ks) {
+  if (!as_bool(a[13])) {
+    check(mi_paged_prefill_attention_tiles(q.data_ptr(), q3.sn, q3.sh, kc.data_ptr(), vc.data_ptr(), c.sc, c.st, c.sh,
+                                           ks ? MI_KV_FP8_E4M3 : MI_KV_16BIT, (const float*)ptr(ks), (const float*)ptr(vs),
+                                           (const int32_t*)table.data_ptr(), table.stride(0), (const int32_t*)cu.data_ptr(),
+                                           (const int32_t*)lens.data_ptr(), out.data_ptr(), o3.sn, o3.sh, ws.ptr, ws.bytes,
+                                           (int)T, (int)R, (int)q3.h, (int)c.h, (int)q3.d, (int)c.c, (int)max_len, scale,
+                                           dtype_code(q), tune, stream),
+          "mi_paged_prefill_attention_tiles");
+  } else if (ks) {
     check(mi_paged_prefill_attention_fp8(q.data_ptr(), q3.sn, q3.sh, kc.data_ptr(), vc.data_ptr(), c.sc, c.st, c.sh,
                                          (const float*)ks->data_ptr(), (const float*)vs->data_ptr(),
                                          (const int32_t*)table.data_ptr(), table.stride(0), (const int32_t*)cu.data_ptr(),
@@ -974,7 +982,7 @@ PyMethodDef kMethods[] = {
     ABI(mi_prefill_workspace_bytes), ABI(mi_paged_decode_attention_noalloc),
     ABI(mi_update_requests), ABI(mi_update_requests_mask8), ABI(mi_add_request), ABI(mi_decode_attention_state), ABI(mi_step_attention_state),
     OP(kv_append, 6), OP(kv_append_fp8, 9), OP(paged_decode_attention, 14), OP(paged_mla_decode_attention, 10),
-    OP(paged_prefill_attention, 13), OP(paged_prefill_attention_mla, 11), OP(norm_rope_append, 22), OP(qkv_norm_rope_append, 22), OP(decode_step_attention, 29),
+    OP(paged_prefill_attention, 14), OP(paged_prefill_attention_mla, 11), OP(norm_rope_append, 22), OP(qkv_norm_rope_append, 22), OP(decode_step_attention, 29),
     OP(linear_decode, 5), OP(attention_layer_decode, 24), OP(sample_from_logits, 12), OP(selected_log_probs, 2), OP(last_token_gather, 3), OP(setup, 3),
     OP(set_workspace, 3), OP(watch, 4), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_native", "Host side of the per-layer calls.", -1, kMethods, nullptr, nullptr, nullptr, nullptr};

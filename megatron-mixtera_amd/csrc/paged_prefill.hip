@@ -938,62 +938,77 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_pp_kernel(PrefillParams 
 }
 
 // Rows whose keys were split over several workgroups: o = sum_s 2^(lse_s - max) o_s / sum_s 2^(lse_s - max).
-// Grid (T, Hq), head_dim threads = the output values of one (row, head).
+// A thread takes four neighbouring output values of one (row, head); nx workgroups of 256 threads per row, flattened
+// into grid.x.  Bound by the partials' bytes: 509 rows x 64 heads of 128, 2 ranges, 42 MB: 12 us (one value per thread
+// and a workgroup per (row, head): 29 us, most of it launching workgroups).  Rows of one-row requests that the decode
+// kernels serve have no partials: what is written there from the workspace's old contents they overwrite afterwards.
 template <bool F16>
-__global__ __launch_bounds__(256) void prefill_split_merge_kernel(PrefillParams p, int n_split, int head_dim) {
-  const int row = blockIdx.x, head = blockIdx.y, d = threadIdx.x;
-  if (row >= p.cu_q[p.R]) return;  // padding rows: zeroed by the tile kernel
-  if (p.skip_single) {             // one-row requests were left to the decode kernels
-    int lo = 0, hi = p.R - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (p.cu_q[mid] <= row) lo = mid; else hi = mid - 1;
-    }
-    if (p.cu_q[lo + 1] - p.cu_q[lo] == 1) return;
-  }
-  float mx = -INFINITY, num = 0.f, den = 0.f;
-  for (int s0 = 0; s0 < n_split; s0 += 8) {
-    float lse[8], po[8];
+__global__ __launch_bounds__(256) void prefill_split_merge_kernel(PrefillParams p, int n_split, int head_dim, int nx) {
+  const int row = blockIdx.x / nx, at = 4 * (256 * (blockIdx.x - row * nx) + threadIdx.x);
+  if (row >= p.cu_q[p.R] || at >= p.Hq * head_dim) return;  // padding rows: zeroed by the tile kernel
+  const int head = at / head_dim, d = at - head * head_dim;
+  float mx = -INFINITY, den = 0.f;
+  float4 num = make_float4(0.f, 0.f, 0.f, 0.f);
+  const int64_t step = (int64_t)p.T * p.Hq, prow0 = (int64_t)row * p.Hq + head;
+  for (int s0 = 0; s0 < n_split; s0 += 4) {
+    float lse[4];
+    float4 po[4];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int64_t prow = ((int64_t)min(s0 + j, n_split - 1) * p.T + row) * p.Hq + head;
+    for (int j = 0; j < 4; ++j) {
+      const int64_t prow = min(s0 + j, n_split - 1) * step + prow0;
       lse[j] = p.split_lse[prow];
-      po[j] = p.split_o[prow * head_dim + d];
+      po[j] = *reinterpret_cast<const float4*>(p.split_o + prow * head_dim + d);
     }
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < 4; ++j) {
       if (s0 + j < n_split && lse[j] != -INFINITY) {
         const float m_new = fmaxf(mx, lse[j]);
         const float a = fast_exp2(mx - m_new), wt = fast_exp2(lse[j] - m_new);
-        num = num * a + wt * po[j];
+        num.x = num.x * a + wt * po[j].x; num.y = num.y * a + wt * po[j].y;
+        num.z = num.z * a + wt * po[j].z; num.w = num.w * a + wt * po[j].w;
         den = den * a + wt;
         mx = m_new;
       }
     }
   }
-  p.out[(int64_t)row * p.o_st + (int64_t)head * p.o_sh + d] = f32_to_16<F16>(den > 0.f ? num / den : 0.f);
+  const bool any = den > 0.f;
+  st8(p.out + (int64_t)row * p.o_st + (int64_t)head * p.o_sh + d,
+      any ? make_uint2(pack2<F16>(num.x / den, num.y / den), pack2<F16>(num.z / den, num.w / den)) : make_uint2(0u, 0u));
 }
 
 }  // namespace mi
 
 using namespace mi;
 
-// Ranges the keys of every request are cut into by the two-phase tile kernel.  Few query rows over a
-// long context (a chunk of a prompt, a short turn after a long history) give few workgroups, each
-// with thousands of keys to walk: then the keys are split so that about one workgroup per CU exists,
-// every one keeping at least sixteen 64-key tiles (a 512-token prompt is not worth the merge).  Host-side quantities only (the lengths live on the GPU).
+static void launch_split_merge(const PrefillParams& p, int n_split, int head_dim, bool f16, hipStream_t st) {
+  const int nx = (p.Hq * head_dim / 4 + 255) / 256;
+  if (f16) hipLaunchKernelGGL(prefill_split_merge_kernel<true>, dim3(p.T * nx), dim3(256), 0, st, p, n_split, head_dim, nx);
+  else hipLaunchKernelGGL(prefill_split_merge_kernel<false>, dim3(p.T * nx), dim3(256), 0, st, p, n_split, head_dim, nx);
+}
+
+// Ranges the keys of every request are cut into by the tile kernels.  Few query rows over a long context (a chunk of a
+// prompt, a short turn after a long history) give few workgroups, each with many keys to walk.  The count is the one
+// with the least estimated time: rounds of workgroups over the CUs (one per CU), each 6 us of fixed cost and 1.5 us per
+// 64-key tile (head width 128, measured on one request of 33 to 1 000 tokens), and for more than one range the merge --
+// 4 us of launch and the fp32 partials written and read at 4.5 TB/s, which is what keeps prompts without a context from
+// being split (1 000 tokens x 32 heads in 2 ranges: 40 us against 37).  Host-side quantities only: the lengths live on
+// the GPU, `max_kv_len` is a bound.
 static int prefill_kv_splits(int T, int Hq, int Hkv, int head_dim, int max_kv_len) {
   if (max_kv_len <= 0) return 1;
   const int G = Hq / Hkv, Gw = G < 16 ? G : 16, parts = (G + 15) / 16;
   const int sbq = 8 * ((head_dim >= 192 ? 16 : 32) / Gw);  // query tokens per workgroup (8 wavefronts x 32 or 16 rows)
   const int64_t useful = (int64_t)Hkv * parts * ((T + sbq - 1) / sbq);
-  const int cus = 256;
+  const int64_t cus = 256, tiles = ((int64_t)max_kv_len + 63) / 64;
   if (useful >= cus) return 1;
-  int64_t s = (cus + useful - 1) / useful;
-  const int64_t by_tiles = ((int64_t)max_kv_len + 63) / 64 / 16;
-  if (s > by_tiles) s = by_tiles;
-  if (s > 32) s = 32;  // (more ranges cost more in partials than they win: 64 rows over 131 072 keys, 16-32 is best)
-  return s < 2 ? 1 : (int)s;
+  const float per_tile = 1.5f * (float)head_dim / 128.f, partials = (float)T * (float)Hq * (float)head_dim * 8.f / 4.5e6f;
+  float best = 6.f + (float)tiles * per_tile;
+  int n = 1;
+  // (more than 32 ranges cost more in partials than they win: 64 rows over 131 072 keys, 16-32 is best)
+  for (int64_t s = 2; s <= 32 && 2 * s <= tiles; ++s) {
+    const float t = (float)((useful * s + cus - 1) / cus) * (6.f + (float)((tiles + s - 1) / s) * per_tile) + 4.f + (float)s * partials;
+    if (t < best) { best = t; n = (int)s; }
+  }
+  return n;
 }
 
 // key ranges for these sizes under the caller's knob (1 = automatic, -1 = never, n > 1 = forced)
@@ -1035,7 +1050,7 @@ static int launch_paged_prefill(
     void* workspace, int64_t workspace_bytes, int32_t T, int32_t R, int32_t Hq, int32_t Hkv,
     int32_t head_dim, int32_t chunk_tokens, int32_t max_kv_len, int32_t split_tokens, float softmax_scale,
     int32_t kv_dtype, const float* k_scales, const float* v_scales, int32_t dtype, const MiTuning* tuning,
-    void* stream) {
+    void* stream, bool one_row_requests = true) {
   const bool fp8 = kv_dtype == MI_KV_FP8_E4M3;
   if (T == 0 || R == 0) return MI_OK;
   MiTuning tune;
@@ -1090,14 +1105,15 @@ static int launch_paged_prefill(
   p.chunk = chunk_tokens;
   p.chunk_magic = (((uint64_t)1 << 40) + chunk_tokens - 1) / chunk_tokens;
   p.scale_log2 = softmax_scale * 1.4426950408889634f;
-  // With a workspace, one-row requests go through the bandwidth-optimised decode kernels.
-  p.skip_single = workspace != nullptr;
+  // With a workspace, one-row requests go through the bandwidth-optimised decode kernels -- unless the caller knows
+  // that there are none: two launches that would find nothing to do, 9 us.
+  p.skip_single = workspace != nullptr && one_row_requests;
   p.k_scale = k_scales; p.v_scale = v_scales;
   p.split_o = nullptr; p.split_lse = nullptr;
 
   // The decode part's own argument checks come before the first launch, so that a negative return still means
   // nothing was enqueued (its remaining checks repeat ones made above).
-  if (p.skip_single) {
+  if (workspace) {
     const int rc_w = check_decode_workspace(workspace, workspace_bytes, R, Hq, Hkv, head_dim, split_tokens, tune,
                                             "mi_paged_prefill_attention");
     if (rc_w != MI_OK) return rc_w;
@@ -1147,8 +1163,7 @@ static int launch_paged_prefill(
     else MI_PP_LAUNCH(false, 256, 256, false);
     if (timed) (void)hipEventRecord(ev_b, st);
     if (n_split > 1) {
-      if (f16) hipLaunchKernelGGL(prefill_split_merge_kernel<true>, dim3(T, Hq), dim3(head_dim), 0, st, p, n_split, head_dim);
-      else hipLaunchKernelGGL(prefill_split_merge_kernel<false>, dim3(T, Hq), dim3(head_dim), 0, st, p, n_split, head_dim);
+      launch_split_merge(p, n_split, head_dim, f16, st);
     }
   } else {
     // register-only kernel: any chunk size that is a multiple of 16; 16 or 32 keys per iteration
@@ -1217,6 +1232,19 @@ extern "C" int mi_paged_prefill_attention_fp8(
                               o_stride_tok, o_stride_head, workspace, workspace_bytes, T, R, Hq, Hkv, head_dim,
                               chunk_tokens, max_kv_len, split_tokens, softmax_scale, MI_KV_FP8_E4M3, k_scales, v_scales,
                               dtype, tuning, stream);
+}
+
+extern "C" int mi_paged_prefill_attention_tiles(
+    const void* q, int64_t q_stride_tok, int64_t q_stride_head, const void* k_cache, const void* v_cache,
+    int64_t kv_stride_chunk, int64_t kv_stride_tok, int64_t kv_stride_head, int32_t kv_dtype, const float* k_scales,
+    const float* v_scales, const int32_t* block_table, int64_t bt_stride, const int32_t* cu_seqlens_q,
+    const int32_t* kv_lens, void* out, int64_t o_stride_tok, int64_t o_stride_head, void* workspace,
+    int64_t workspace_bytes, int32_t T, int32_t R, int32_t Hq, int32_t Hkv, int32_t head_dim, int32_t chunk_tokens,
+    int32_t max_kv_len, float softmax_scale, int32_t dtype, const MiTuning* tuning, void* stream) {
+  return launch_paged_prefill(q, q_stride_tok, q_stride_head, k_cache, v_cache, kv_stride_chunk, kv_stride_tok,
+                              kv_stride_head, block_table, bt_stride, cu_seqlens_q, kv_lens, out, o_stride_tok,
+                              o_stride_head, workspace, workspace_bytes, T, R, Hq, Hkv, head_dim, chunk_tokens,
+                              max_kv_len, 0, softmax_scale, kv_dtype, k_scales, v_scales, dtype, tuning, stream, false);
 }
 
 extern "C" int mi_paged_prefill_attention_mla(
@@ -1303,8 +1331,7 @@ extern "C" int mi_paged_prefill_attention_mla(
   }
   if (timed) (void)hipEventRecord(ev_b, st);
   if (n_split > 1) {
-    if (f16) hipLaunchKernelGGL(prefill_split_merge_kernel<true>, dim3(T, Hq), dim3(head_dim_v), 0, st, p, n_split, head_dim_v);
-    else hipLaunchKernelGGL(prefill_split_merge_kernel<false>, dim3(T, Hq), dim3(head_dim_v), 0, st, p, n_split, head_dim_v);
+    launch_split_merge(p, n_split, head_dim_v, f16, st);
   }
   return mi_check_launch("mi_paged_prefill_attention_mla");
 }

@@ -51,6 +51,8 @@ constexpr int kWvAhead = 3;                      // fragments requested ahead of
 constexpr int kWvRing = 4;                       // fragment registers: fragment n lives in slot n % kWvRing
 // LDS bytes per staged row: the row and 32 bytes of padding (288 or 160: conflict-free fragment reads)
 template <int HD> constexpr int wv_pitch() { return 2 * HD + 32; }
+// (half as many at head_dim 128 with few workgroups, one wavefront per SIMD: 5-8 % faster up to one workgroup per CU,
+// slower beyond; two at head_dim 64: slower throughout)
 template <int HD> constexpr int wv_waves() { return HD == 64 ? 4 : 8; }
 // piece u of a tile's line -> its row, by multiplication
 template <int HD> constexpr unsigned wv_magic() { return 65536u / (wv_pitch<HD>() / 16) + 1; }
@@ -178,18 +180,18 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
     const uint32_t ks_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)&Ks[0][0];
     const uint32_t vs_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)&Vs[0][0];
 
-    // ---- 16-bit cache: this wavefront's five direct loads of a tile pair {key tile, value tile} -------------------
+    // ---- 16-bit cache: this wavefront's direct loads of a tile pair {key tile, value tile} ------------------------
     // Load k of the pair's 2 LOADS (the first half: the key tile's line, the second: the value tile's) belongs to
     // wavefront k % WAVES; with 36 loads over 8 wavefronts the fifth load of wavefronts 4-7 repeats their fourth, so
-    // that every wavefront issues five per tile.  Loads 0 and 1 are key loads and loads 3 and 4 value loads for every
-    // wavefront; load 2 is a key load for wavefronts 0 and 1 only.
-    static_assert(LOADS == 2 * WAVES + 2, "which of a wavefront's five loads belong to the key tile");
-    uint32_t ld_off[5];   // per lane: where its piece of the load comes from, relative to the tile's first row
-    uint32_t ld_dst[5];   // scalar: LDS offset of the load's 1 KiB inside its tile buffer
-    const bool third_is_key = wave < 2;
+    // that every wavefront issues as many.  Loads below NKL are key loads and loads above it value loads for every
+    // wavefront; load NKL is a key load for the first LOADS % WAVES wavefronts only.
+    constexpr int NL = (2 * LOADS + WAVES - 1) / WAVES, NKL = LOADS / WAVES;
+    uint32_t ld_off[NL];  // per lane: where its piece of the load comes from, relative to the tile's first row
+    uint32_t ld_dst[NL];  // scalar: LDS offset of the load's 1 KiB inside its tile buffer
+    const bool mid_is_key = wave < LOADS % WAVES;
     if constexpr (!FP8) {
 #pragma unroll
-      for (int i = 0; i < 5; ++i) {
+      for (int i = 0; i < NL; ++i) {
         const int k = wave + WAVES * i < 2 * LOADS ? wave + WAVES * i : wave + WAVES * i - WAVES;
         const bool is_key = k < LOADS;
         const int kp = is_key ? k : k - LOADS;
@@ -199,21 +201,21 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
         ld_off[i] = prow * (uint32_t)tok_bytes + 16u * min(pcol, (uint32_t)(PIECES - 3));
       }
     }
-    // ---- fp8 cache: a thread fetches 8 bytes (8 elements) of two rows of a tile into registers, one tile ahead, and
+    // ---- fp8 cache: a thread fetches 8 bytes (8 elements) of NP8 rows of a tile into registers, one tile ahead, and
     // stores them converted.  Keys are converted exactly (e4m3 is a subset of both 16-bit types) and their scale goes
     // into the softmax scale of their tile; values are multiplied by their scale and rounded.
-    constexpr int PPR8 = HD / 8, RPP8 = THREADS / PPR8;
-    static_assert(2 * RPP8 == kWvTile, "two rows per thread");
-    uint2 kraw[2], vraw[2];
+    constexpr int PPR8 = HD / 8, RPP8 = THREADS / PPR8, NP8 = kWvTile / RPP8;
+    static_assert(NP8 * RPP8 == kWvTile && NP8 <= NKF && NP8 <= NVF, "one row per fragment position");
+    uint2 kraw[NP8], vraw[NP8];
     const uint32_t f_piece = 8u * (uint32_t)(tid % PPR8), f_row0 = (uint32_t)(tid / PPR8) * (uint32_t)tok_bytes + f_piece,
-                   f_row1 = f_row0 + (uint32_t)RPP8 * (uint32_t)tok_bytes;
+                   f_step = (uint32_t)RPP8 * (uint32_t)tok_bytes;
     const int f_lds = (tid / PPR8) * PITCH + 16 * (tid % PPR8);
     // rows past the request's last key re-read that row (every query row masks them); `nrec`: see tile_nrec
-    auto fetch_fp8 = [&](const uint8_t* cache, int64_t off, uint32_t nrec, uint2 (&reg)[2]) {
+    auto fetch_fp8 = [&](const uint8_t* cache, int64_t off, uint32_t nrec, uint2 (&reg)[NP8]) {
       const uint8_t* src = cache + (int64_t)h * p.kv_sh + off;
       const uint32_t lim = nrec - (uint32_t)tok_bytes + f_piece;
-      reg[0] = ld8(src + min(f_row0, lim));
-      reg[1] = ld8(src + min(f_row1, lim));
+#pragma unroll
+      for (int i = 0; i < NP8; ++i) reg[i] = ld8(src + min(f_row0 + (uint32_t)i * f_step, lim));
     };
     auto store_k_fp8 = [&](uint8_t* buf, int i) {
       const uint2 lo = fp8x4_to_16x4<F16>(kraw[i].x), hi = fp8x4_to_16x4<F16>(kraw[i].y);
@@ -237,7 +239,7 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
       return rs;
     };
     auto issue_load = [&](int i, const u32x4_t& rs_k, const u32x4_t& rs_v, uint32_t kdst, uint32_t vdst) {
-      const bool is_key = i < 2 || (i == 2 && third_is_key);
+      const bool is_key = i < NKL || (i == NKL && mid_is_key);
       const u32x4_t rs = is_key ? rs_k : rs_v;
       const uint32_t m0 = (is_key ? kdst : vdst) + ld_dst[i];
       asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(m0), "v"(ld_off[i]), "s"(rs)
@@ -456,9 +458,9 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
       MI_SB();
     };
 
-    // ---- prologue: clear the buffers (the value tile "before the first" must hold zeros), start the first tiles ----
-    for (int i = tid * 16; i < KBUFS * BUF; i += THREADS * 16) *reinterpret_cast<uint4*>(&Ks[0][0] + i) = make_uint4(0u, 0u, 0u, 0u);
-    for (int i = tid * 16; i < VBUFS * BUF; i += THREADS * 16) *reinterpret_cast<uint4*>(&Vs[0][0] + i) = make_uint4(0u, 0u, 0u, 0u);
+    // ---- prologue: clear the buffer of the value tile "before the first" (its probabilities are zeros, and zero times
+    // a stale value must not be NaN; every other buffer is filled whole before it is read), start the first tiles ----
+    for (int i = tid * 16; i < BUF; i += THREADS * 16) *reinterpret_cast<uint4*>(&Vs[0][0] + i) = make_uint4(0u, 0u, 0u, 0u);
     Cursor cur = cursor_at(tb + DEPTH + 1);
     int64_t off_first[DEPTH + 1];   // tiles tb .. tb + DEPTH, started here
     uint32_t nrec_first[DEPTH + 1];
@@ -486,14 +488,14 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
 #pragma unroll
       for (int kk = 0; kk < KS; ++kk)
         asm volatile("" ::"v"(qf[nt][kk].x), "v"(qf[nt][kk].y), "v"(qf[nt][kk].z), "v"(qf[nt][kk].w));
-    __syncthreads();  // the cleared buffers are in place before the first direct load can land
+    __syncthreads();
     int64_t off_prev;
     uint32_t nrec_prev;
     if constexpr (FP8) {
       static_assert(!FP8 || DEPTH == 1, "fp8 tiles wait in one set of registers");
       fetch_fp8(p.kc, off_first[0], nrec_first[0], kraw);
-      store_k_fp8(&Ks[0][0], 0);
-      store_k_fp8(&Ks[0][0], 1);
+#pragma unroll
+      for (int i = 0; i < NP8; ++i) store_k_fp8(&Ks[0][0], i);
       fetch_fp8(p.kc, off_first[1], nrec_first[1], kraw);  // stored by iteration 0
       fetch_fp8(p.vc, off_first[0], nrec_first[0], vraw);
       off_prev = off_first[1];
@@ -502,22 +504,21 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
     } else {
       const u32x4_t rk0 = tile_rsrc(kbase, off_first[0], nrec_first[0]);
 #pragma unroll
-      for (int i = 0; i < 5; ++i)
-        if (i < 2 || (i == 2 && third_is_key)) issue_load(i, rk0, rk0, ks_lds, ks_lds);  // key tile 0 -> Ks[0]
+      for (int i = 0; i < NL; ++i)
+        if (i < NKL || (i == NKL && mid_is_key)) issue_load(i, rk0, rk0, ks_lds, ks_lds);  // key tile 0 -> Ks[0]
 #pragma unroll
       for (int t = 1; t <= DEPTH; ++t) {  // the pairs {key tile t -> Ks[t], value tile t - 1 -> Vs[t]}
         const u32x4_t rk = tile_rsrc(kbase, off_first[t], nrec_first[t]);
         const u32x4_t rv = tile_rsrc(vbase, off_first[t - 1], nrec_first[t - 1]);
 #pragma unroll
-        for (int i = 0; i < 5; ++i) issue_load(i, rk, rv, ks_lds + t * BUF, vs_lds + t * BUF);
+        for (int i = 0; i < NL; ++i) issue_load(i, rk, rv, ks_lds + t * BUF, vs_lds + t * BUF);
       }
       off_prev = off_first[DEPTH];
       nrec_prev = nrec_first[DEPTH];
     }
     // key tile 0 has landed (this wavefront's share): only the DEPTH pairs issued after it may still be on their way
     if constexpr (!FP8) {
-      if constexpr (DEPTH == 1) asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
-      else asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(DEPTH * NL) : "memory");
     }
     __builtin_amdgcn_s_barrier();
     MI_SB();
@@ -547,16 +548,14 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
       slot(std::integral_constant<int, 0>{}, Mc, ka, ka_next, va, key0, [] {}, [](int) {},
            [&](int e) {
              if constexpr (FP8) {
-               if (e == NVF - 2) store_k_fp8(kst, 0);
-               if (e == NVF - 1) store_k_fp8(kst, 1);
+               if (e >= NVF - NP8) store_k_fp8(kst, e - (NVF - NP8));
              }
            });
       slot(std::integral_constant<int, 1>{}, Mc, ka, ka_next, va, key0 + 32,
            [&] {
              // this wavefront's share of key tile j+1 and value tile j has landed: only younger pairs are on their way
              if constexpr (FP8) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-             else if constexpr (DEPTH == 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-             else asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
+             else asm volatile("s_waitcnt vmcnt(%0)" ::"n"((DEPTH - 1) * NL) : "memory");
              __builtin_amdgcn_s_barrier();
              if constexpr (FP8) pc_next = __builtin_amdgcn_readfirstlane(pc_v);
              else bt_arrived(pc_next);
@@ -580,13 +579,13 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
            },
            [&](int n) {
              if constexpr (FP8) {
-               if (n < 2) store_v_fp8(vst, n, vscale);
+               if (n < NP8) store_v_fp8(vst, n, vscale);
              }
            },
            [&](int e) {
              if constexpr (!FP8) {
-               if (e < 5) issue_load(e, rs_k, rs_v, kdst, vdst);
-               if (e == NVF - 1 && NVF < 5) issue_load(4, rs_k, rs_v, kdst, vdst);
+#pragma unroll
+               for (int i = e; i < NL; i += NVF) issue_load(i, rs_k, rs_v, kdst, vdst);
              }
            });
       if constexpr (FP8) {

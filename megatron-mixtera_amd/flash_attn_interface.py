@@ -86,11 +86,13 @@ def flash_attn_varlen_func(q: Tensor, k: Tensor, v: Tensor, cu_seqlens_q: Tensor
                            softcap: float = 0.0, alibi_slopes=None, deterministic: bool = False,
                            return_attn_probs: bool = False, block_table: Optional[Tensor] = None,
                            *, seqused_k: Optional[Tensor] = None, k_scales: Optional[Tensor] = None,
-                           v_scales: Optional[Tensor] = None) -> Tensor:
+                           v_scales: Optional[Tensor] = None, one_row_requests: Optional[bool] = None) -> Tensor:
     """Paged varlen causal attention: ``q`` is ``[T, Hq, d]``, ``k``/``v`` are the paged caches.
 
     Per-request key counts come from ``seqused_k`` if given, else from the differences of
-    ``cu_seqlens_k``.  The mask is flash-attn's bottom-right aligned causal mask.
+    ``cu_seqlens_k``.  The mask is flash-attn's bottom-right aligned causal mask.  ``one_row_requests=False`` says
+    that no request has exactly one query row; without a word from the caller that is known when the rows are more
+    than requests of at most ``max_seqlen_q`` rows could have with one of them at one row.
     """
     _reject(dropout_p=dropout_p, window_size=window_size, softcap=softcap, alibi_slopes=alibi_slopes,
             return_attn_probs=return_attn_probs)
@@ -111,9 +113,11 @@ def flash_attn_varlen_func(q: Tensor, k: Tensor, v: Tensor, cu_seqlens_q: Tensor
         return ops.paged_prefill_attention_mla(
             q, k, v, cu_seqlens_q, kv_lens.to(torch.int32), block_table, max_kv_len=max_seqlen_k,
             softmax_scale=softmax_scale if softmax_scale is not None else q.shape[-1] ** -0.5)
+    if one_row_requests is None:
+        one_row_requests = q.size(0) <= (cu_seqlens_q.numel() - 2) * max_seqlen_q + 1
     return ops.paged_prefill_attention(q, k, v, cu_seqlens_q, kv_lens.to(torch.int32), block_table,
                                        softmax_scale=softmax_scale, max_kv_len=max_seqlen_k,
-                                       k_scales=k_scales, v_scales=v_scales)
+                                       k_scales=k_scales, v_scales=v_scales, one_row_requests=one_row_requests)
 
 
 def _flash_attn_forward(q: Tensor, k: Tensor, v: Tensor, k_new=None, v_new=None, qv=None, out: Optional[Tensor] = None,

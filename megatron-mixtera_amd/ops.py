@@ -345,11 +345,15 @@ def paged_prefill_attention_mla(q: Tensor, k_cache: Tensor, v_cache: Tensor, cu_
 def paged_prefill_attention(q: Tensor, k_cache: Tensor, v_cache: Tensor, cu_seqlens_q: Tensor, kv_lens: Tensor,
                             block_table: Tensor, *, softmax_scale: Optional[float] = None,
                             max_kv_len: Optional[int] = None, out: Optional[Tensor] = None,
-                            k_scales: Optional[Tensor] = None, v_scales: Optional[Tensor] = None) -> Tensor:
+                            k_scales: Optional[Tensor] = None, v_scales: Optional[Tensor] = None,
+                            one_row_requests: bool = True) -> Tensor:
     """Varlen causal attention of new tokens over the paged cache (bottom-right aligned mask).
-    Byte caches with ``k_scales`` / ``v_scales`` ``[N, Hkv]`` select the fp8-e4m3 path."""
+    Byte caches with ``k_scales`` / ``v_scales`` ``[N, Hkv]`` select the fp8-e4m3 path.  ``one_row_requests=False``
+    says that no request has exactly one query row, so the decode kernels need not be launched (a request that has
+    one all the same is served by the tile kernel)."""
     return _native().paged_prefill_attention(q, k_cache, v_cache, cu_seqlens_q, kv_lens, block_table, softmax_scale,
-                                             max_kv_len, out, k_scales, v_scales, _tuning_arg(), _override())
+                                             max_kv_len, out, k_scales, v_scales, _tuning_arg(), _override(),
+                                             one_row_requests)
 
 
 # ---------------------------------------------------------------------------------------------

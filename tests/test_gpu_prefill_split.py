@@ -1,0 +1,27 @@
+"""GPU parity: automatic key ranges and their merge, with and without the decode launches of one-row requests."""
+import pytest
+import torch
+
+from oracle import paged_attention as oa
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("one_row_requests", [True, False])
+@pytest.mark.parametrize("d,Hq,Hkv", [(128, 32, 8), (64, 8, 8), (96, 24, 8), (256, 4, 1)])
+def test_few_rows_over_contexts(mi, dev, d, Hq, Hkv, one_row_requests):
+    """Few rows over a context of more than two ranges; a one-row request among them; padded rows behind."""
+    q_lens, ctx, chunk, pad = [3, 1, 65, 2], [0, 1500, 700, 2100], 64, 5
+    kv_lens = torch.tensor([a + b for a, b in zip(q_lens, ctx)], dtype=torch.int32)
+    cu_q = torch.zeros(len(q_lens) + 1, dtype=torch.int32)
+    cu_q[1:] = torch.cumsum(torch.tensor(q_lens), 0)
+    gen = torch.Generator().manual_seed(d)
+    bt, N = mi.synthetic.build_block_table(kv_lens, chunk, gen)
+    T = int(cu_q[-1])
+    q = torch.randn(T + pad, Hq, d, generator=gen).bfloat16()
+    kc, vc = (torch.randn(N, chunk, Hkv, d, generator=gen).bfloat16() for _ in range(2))
+    out = mi.ops.paged_prefill_attention(q.to(dev), kc.to(dev), vc.to(dev), cu_q.to(dev), kv_lens.to(dev), bt.to(dev),
+                                         max_kv_len=int(kv_lens.max()), one_row_requests=one_row_requests).float().cpu()
+    ref = oa.paged_varlen_attention(q[:T], kc, vc, cu_q, kv_lens, bt)
+    assert (out[:T] - ref).abs().max().item() < 2e-2
+    assert not out[T:].any()
