@@ -1274,16 +1274,25 @@ extern "C" int mi_last_token_gather(const void* src, int64_t src_stride_row, voi
   return mi_check_launch("mi_last_token_gather");
 }
 
-// Parts a row is cut into: enough workgroups for the chip (one per CU), parts of at least 4 096 elements.
+// Parts a row is cut into: as many workgroups as the chip takes at once (one per CU: a second round costs more than
+// larger parts, 83 x 50 304 top-p in 4 parts 45 us, in 3 33), parts of at least 4 096 elements.
 static int sample_parts(int R, int V) {
-  int parts = (256 + R - 1) / R;
+  int parts = 256 / R;
   if (parts > V / 4096) parts = V / 4096;
   return parts < 1 ? 1 : (parts > kMaxParts ? kMaxParts : parts);
 }
-// Whether the rows are done in parts: while a row has two of them.  From 129 rows on one workgroup per row fills half
-// the chip and more, and its fewer reads count (256 x 128 256 fp32, one workgroup per row / in parts: plain 52 / 60 us,
-// top-k 50 45 / 60, top-p 0.9 70 / 83 on peaked rows).
-static bool sample_in_parts(int R, int V, int top_k) { return V >= kFastMinVocab && R <= 128 && top_k <= kFastTopK; }
+// Whether the rows are done in parts: where that was measured the faster (fp32 and bf16, 1-400 rows of 32 768-151 936).
+// The further launches cost 3-6 us, so the walks they shorten have to be long enough; from 129 rows on a row has one
+// part.  Greedy has one walk to shorten (64 x 151 936: 16.5 -> 13.8 us; 64 x 100 352: 11.1 against 12.5); plain draws two
+// (64 x 50 304: 19.7 -> 19.2, x 32 768: 13.6 against 17.3), top-p three; top-k's pick grows with its lists, one from
+// each part, and does not gain from two (128 x 100 352: 34.7 against 38.9).
+static bool sample_in_parts(int R, int V, int top_k, float top_p) {
+  if (V < kFastMinVocab || R > 128 || top_k > kFastTopK) return false;
+  if (top_k == 1) return V >= 1600 * (R > 50 ? R : 50);
+  if (top_k > 1) return R <= 85;
+  if (R > 85) return V >= 65536;
+  return V >= 49152 || (top_p > 0.f && R <= 64);
+}
 
 static int64_t align256(int64_t n) { return (n + 255) & ~(int64_t)255; }
 static int64_t sample_layout(SplitParams* p, uint8_t* base, int R, int V, int top_k, float top_p) {
@@ -1322,7 +1331,7 @@ static void launch_sample(const SampleParams& s, SplitParams* split, hipStream_t
 
 extern "C" int64_t mi_sample_workspace_bytes(int32_t R, int32_t vocab, int32_t top_k, float top_p) {
   SplitParams p;
-  return R > 0 && vocab > 0 && sample_in_parts(R, vocab, top_k) ? sample_layout(&p, nullptr, R, vocab, top_k, top_p) : 0;
+  return R > 0 && vocab > 0 && sample_in_parts(R, vocab, top_k, top_p) ? sample_layout(&p, nullptr, R, vocab, top_k, top_p) : 0;
 }
 
 extern "C" int mi_sample_from_logits_ws(const void* logits, int64_t stride_row, int32_t logits_dtype, int32_t R,
@@ -1361,7 +1370,7 @@ extern "C" int mi_sample_from_logits_ws(const void* logits, int64_t stride_row, 
   const int esize = logits_dtype != 0 ? 2 : 4;
   const bool wide = !(((uintptr_t)logits | (uintptr_t)(stride_row * esize)) & 15);  // 16-byte loads
   SplitParams split, *in_parts = nullptr;
-  if (workspace && sample_in_parts(R, vocab, top_k)) {
+  if (workspace && sample_in_parts(R, vocab, top_k, top_p)) {
     if ((uintptr_t)workspace & 255) return mi_fail(MI_ERR_ALIGN, "mi_sample_from_logits_ws: the workspace must be 256-byte aligned");
     if (sample_layout(&split, (uint8_t*)workspace, R, vocab, top_k, top_p) > workspace_bytes)
       return mi_fail(MI_ERR_WORKSPACE, "mi_sample_from_logits_ws: workspace smaller than mi_sample_workspace_bytes()");

@@ -406,7 +406,7 @@ def test_context_log_probs_through_the_kernel(mi, dev):
         Ctx.TOKEN_ROUNDER, Ctx.REQUEST_ROUNDER = saved
 
 
-@pytest.mark.parametrize("R,V", [(1, 16384), (2, 16389), (5, 50257), (128, 32000), (129, 32000), (1, 260000)])
+@pytest.mark.parametrize("R,V", [(1, 16384), (2, 16389), (5, 50257), (64, 32000), (85, 49152), (128, 65536), (129, 65536), (1, 260000)])
 @pytest.mark.parametrize("kind", ["flat", "peaked", "equal", "few", "masked", "nan"])
 def test_rows_in_parts_equal_rows_by_one_workgroup(mi, dev, R, V, kind):
     """Rows cut into parts give the tokens and cut values of the one-workgroup entry point, bit for bit: where the
