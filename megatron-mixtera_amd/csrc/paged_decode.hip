@@ -68,7 +68,7 @@ struct DecodeParams {
   const float* v_scale;
   float headroom;        // fp8 fused step: scale of a chunk a token opens = headroom * amax(token) / 448
   uint64_t chunk_magic;  // ceil(2^40 / chunk)
-  int32_t R, Hq, Hkv, G, chunk, min_span_tiles, grid;
+  int32_t R, Hq, Hkv, G, chunk, min_span_tiles, grid;  // min_span_tiles: 0 = from the lengths (see walk_segments)
   int32_t parts;  // wavefronts per KV head: each takes up to 16 of the G query heads that share it
   // Fused decode step only (FUSED kernels): `q` holds the raw queries of the step, head h * G + u of a row at
   // h * q_gst + u * d; the step's new key / value rows, norm weights, rotary table and positions.
@@ -776,16 +776,31 @@ static __device__ __forceinline__ void walk_segments(const DecodeParams& p, Seg 
   }
   __syncthreads();
   const int total = cum[p.R - 1];
+  // Tiles per span of a batch that leaves CUs idle.  A span's tiles follow one another, about 1.5 us each (their loads
+  // are one tile ahead, and a trip to memory takes longer than a tile's arithmetic); every further span of a request
+  // costs the merge some 0.04 us.  The sum is least at the square root of a thirtieth of the request's tiles.  When
+  // that gives a span of less than a CU's share, a share of a few tiles is rounded up: the longest span is no longer
+  // for it, and there are fewer.  (64 tokens always, as before, against this, us for a layer's step: four requests of 20-200
+  // tokens 44.5 / 36.4, four of 300-1 200 45.3 / 40.1, one of 777 40.3 / 38.0.)
+  int min_span = p.min_span_tiles;
+  if (min_span <= 0) {
+    // (requests with tiles, among the first 64: padded rows and the prompts of a mixed batch have none)
+    const int n = min(p.R, 64);
+    const bool live = lane < n && cum[lane] > (lane ? cum[lane - 1] : 0);
+    const float share = (float)__builtin_popcountll(__builtin_amdgcn_ballot_w64(live)) / (float)n;
+    min_span = max(1, (int)rintf(__builtin_sqrtf(0.035f * (float)total / fmaxf(share * (float)p.R, 1.f))));
+    if (total > p.grid * min_span && total < 4 * p.grid) min_span = (total + p.grid - 1) / p.grid;
+  }
   // equal spans; the remainder goes one tile each to the first workgroups (rounding the span
   // up instead would leave the last workgroups without work)
   int t0, t1;
-  if (total >= p.grid * p.min_span_tiles) {
+  if (total >= p.grid * min_span) {
     const int per = total / p.grid, rem = total - per * p.grid;
     t0 = (int)blockIdx.x * per + min((int)blockIdx.x, rem);
     t1 = t0 + per + ((int)blockIdx.x < rem ? 1 : 0);
   } else {
-    t0 = blockIdx.x * p.min_span_tiles;
-    t1 = min(t0 + p.min_span_tiles, total);
+    t0 = blockIdx.x * min_span;
+    t1 = min(t0 + min_span, total);
   }
   if (t0 >= t1) return;
 
@@ -1783,9 +1798,6 @@ int mi::launch_paged_decode(
   while (chunk_tokens % (16 * nt)) nt >>= 1;  // a tile must not straddle two chunks
   const int minw = head_dim > 128 ? 2 : tune.decode_min_waves;
   const int tk = 16 * nt;
-  // a small batch is cut finer than a large one needs: 64 tokens per workgroup put a single 8 192-token
-  // request on 128 CUs (17.8 us against 33 us with 256-token spans); large batches get equal spans anyway
-  const int min_span_tokens = split_tokens > 0 ? split_tokens : 64;
 
   DecodeParams p;
   p.q = (const uint16_t*)q; p.q_st = q_stride_tok; p.q_sh = q_stride_head;
@@ -1800,7 +1812,7 @@ int mi::launch_paged_decode(
   p.R = R; p.Hq = Hq; p.Hkv = Hkv; p.G = G; p.chunk = chunk_tokens;
   p.parts = (G + 15) / 16;
   p.chunk_magic = (((uint64_t)1 << 40) + chunk_tokens - 1) / chunk_tokens;
-  p.min_span_tiles = (min_span_tokens + tk - 1) / tk;
+  p.min_span_tiles = split_tokens > 0 ? (split_tokens + tk - 1) / tk : 0;
   p.grid = grid_x;
   p.scale_log2 = softmax_scale * 1.4426950408889634f;
   if (fused) {
