@@ -791,11 +791,18 @@ static __device__ __forceinline__ void walk_segments(const DecodeParams& p, Seg 
     min_span = max(1, (int)rintf(__builtin_sqrtf(0.035f * (float)total / fmaxf(share * (float)p.R, 1.f))));
     if (total > p.grid * min_span && total < 4 * p.grid) min_span = (total + p.grid - 1) / p.grid;
   }
-  // equal spans; the remainder goes one tile each to the first workgroups (rounding the span
+  // Starting a segment costs a workgroup about as much as a tile (its queries, table entries and first tile arrive one
+  // trip after the other), so every request is one unit longer than its tiles where spans are long enough for whole
+  // units to balance: the first `lead` units of a request are its start.  (64 latent-cache requests of 512-8 192
+  // tokens, 17 tiles per span, up to four starts: 72.9 -> 71.1 us; 64 requests of an ordinary cache, the layer: 218.2 -> 216.5.)
+  const int lead = total >= 8 * p.grid && total >= p.grid * min_span ? 1 : 0;
+  auto units = [&](int i) { return cum[i] + lead * (i + 1); };  // of requests 0 .. i
+  const int total_units = units(p.R - 1);
+  // equal spans; the remainder goes one unit each to the first workgroups (rounding the span
   // up instead would leave the last workgroups without work)
   int t0, t1;
   if (total >= p.grid * min_span) {
-    const int per = total / p.grid, rem = total - per * p.grid;
+    const int per = total_units / p.grid, rem = total_units - per * p.grid;
     t0 = (int)blockIdx.x * per + min((int)blockIdx.x, rem);
     t1 = t0 + per + ((int)blockIdx.x < rem ? 1 : 0);
   } else {
@@ -804,21 +811,22 @@ static __device__ __forceinline__ void walk_segments(const DecodeParams& p, Seg 
   }
   if (t0 >= t1) return;
 
-  // first request whose tiles extend beyond t0
+  // first request whose units extend beyond t0
   int lo = 0, hi = p.R - 1;
   while (lo < hi) {
     const int mid = (lo + hi) >> 1;
-    if (cum[mid] > t0) hi = mid; else lo = mid + 1;
+    if (units(mid) > t0) hi = mid; else lo = mid + 1;
   }
   int r = lo;
   while (t0 < t1) {
-    const int rb = r ? cum[r - 1] : 0;
-    const int re = cum[r];
-    if (re > t0) {  // requests without tiles (length 0) are skipped
+    const int rb = r ? units(r - 1) : 0;
+    const int re = units(r);
+    const int ue = min(t1, re);
+    const int tb = max(t0 - rb - lead, 0);   // first tile of the segment, within the request
+    const int te = ue - rb - lead;           // one past its last tile
+    if (te > tb) {  // (requests without tiles, and spans that end within a request's start, are skipped)
       const int len = len_s[r];
-      const int tb = t0 - rb;             // first tile of the segment, within the request
-      const int te = min(t1, re) - rb;    // one past its last tile
-      const bool first = tb == 0, final = te == re - rb;
+      const bool first = tb == 0, final = ue == re;
       if (wave == 0 && lane == 0) {
         if (first) p.seg_info[2 * r] = blockIdx.x;
         if (final) p.seg_info[2 * r + 1] = blockIdx.x;
@@ -826,8 +834,8 @@ static __device__ __forceinline__ void walk_segments(const DecodeParams& p, Seg 
       int row;
       decode_row(p, r, row);
       seg(r, row, len, tb * TK, min(te * TK, len), first && final, final, (int)blockIdx.x + r);
-      t0 = rb + te;
     }
+    t0 = max(t0, ue);
     ++r;
   }
 }
