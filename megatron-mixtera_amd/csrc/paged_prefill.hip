@@ -376,19 +376,9 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_pp_kernel(PrefillParams 
     }
   }
 
-  const int sb = (int)(gridDim.x / HV) - 1 - rank;
-  int lo = 0, hi = p.R - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (p.cu_q[mid] / SBQ + mid <= sb) lo = mid; else hi = mid - 1;
-  }
-  const int r = lo;
-  const int q_begin = p.cu_q[r];
-  const int Lq = p.cu_q[r + 1] - q_begin;
-  const int q0_wg = (sb - (q_begin / SBQ + r)) * SBQ;
-  if (q0_wg >= Lq) return;  // workgroup-uniform
-  if (p.skip_single && Lq == 1) return;
-  const int Lk = p.lens[r];
+  QueryBlock qb;
+  if (!find_query_block(p, SBQ, rank, (int)(gridDim.x / HV), &qb)) return;  // workgroup-uniform
+  const int r = qb.r, q_begin = qb.q_begin, Lq = qb.Lq, Lk = qb.Lk, q0_wg = qb.q0;
   const int shift = Lk - Lq;
   const int last = Lk - 1;
   const int kend_wg = min(Lk, shift + min(q0_wg + SBQ, Lq));

@@ -57,6 +57,127 @@ static __device__ __forceinline__ HeadSlice head_slice(const PrefillParams& p, i
   return s;
 }
 
+// The query block a workgroup of the tile kernels takes.
+struct QueryBlock {
+  int r;              // request
+  int q_begin;        // its first row
+  int Lq, Lk;         // its rows and keys
+  int q0;             // the block's first row within the request
+};
+
+// inclusive sum over the lanes of a wavefront (lane 63: the total), on the vector pipe's lane shifts
+static __device__ __forceinline__ int wave_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8: within 16 lanes
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // lane 15 -> row 1, lane 47 -> row 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // lane 31 -> rows 2 and 3
+  return v;
+}
+
+constexpr int kOrderedRequests = 128;  // requests whose blocks are handed out longest first (two per lane)
+constexpr int kBlockLevels = 16;
+
+// The `rank`-th query block of the batch, blocks of `SBQ` rows; false: there are fewer.  `blocks` is the launch's count
+// (an upper bound).  Every wavefront of the workgroup calls this.
+//
+// The chip takes workgroups in order, so the longest must come first: in the batch's own order the last ones are the
+// first request's, however long its context, and the chip drains while they run.  Blocks are ranked by the keys
+// they see in 16 levels (equal ones side by side: blocks of one request share their keys in L2), which is within a few
+// percent of exact order in a list-scheduling model.  A lane holds one or two requests; how many blocks of a request
+// reach a level is arithmetic, so four steps of bisection and a scan find the block.  11 prompts of 33-3 001 tokens, head width
+// 64: the step 177.2 -> 170.5 us.  With more requests than that -- or one, whose blocks are in order as they are --
+// blocks come last to first: request r's are numbered cu_q[r] / SBQ + r onward.
+static __device__ __forceinline__ bool find_query_block(const PrefillParams& p, int SBQ, int rank, int blocks,
+                                                        QueryBlock* o) {
+  const int lane = threadIdx.x & 63;
+  if (p.R > 1 && p.R <= kOrderedRequests) {
+    const float inv = 1.f / (float)SBQ;
+    auto div = [&](int n) {  // n / SBQ for n >= 0: the estimate is at most one off
+      int q = (int)((float)n * inv);
+      q -= q * SBQ > n ? 1 : 0;
+      return q + ((q + 1) * SBQ <= n ? 1 : 0);
+    };
+    int cq[2], lq[2], lk[2], nb[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int i = lane + 64 * c;
+      cq[c] = lq[c] = lk[c] = nb[c] = 0;
+      if (i < p.R) {
+        cq[c] = p.cu_q[i];
+        lq[c] = p.cu_q[i + 1] - cq[c];
+        lk[c] = p.lens[i];
+        nb[c] = p.skip_single && lq[c] == 1 ? 0 : div(max(lq[c], 0) + SBQ - 1);
+      }
+    }
+    int top = max(nb[0] ? lk[0] : 0, nb[1] ? lk[1] : 0);
+#pragma unroll
+    for (int s = 1; s < 64; s <<= 1) top = max(top, __shfl_xor(top, s, 64));
+    const int step = (__builtin_amdgcn_readfirstlane(top) >> 4) + 1;
+    static_assert(kBlockLevels == 16, "levels of top / 16 keys");
+    // blocks of the lane's request c whose last row sees more than level * step keys
+    auto reach = [&](int c, int level) {
+      if (level <= 0) return nb[c];
+      const int need = level * step + 1 - (lk[c] - lq[c]);  // rows up to the first such one
+      if (level >= kBlockLevels || need > lq[c] || !nb[c]) return 0;
+      return nb[c] - (need > 0 ? div(need - 1) : 0);
+    };
+    auto count = [&](int level) {
+      return __builtin_amdgcn_readlane(wave_scan(reach(0, level) + reach(1, level)), 63);
+    };
+    if (rank >= count(0)) return false;
+    int lo = 0, hi = kBlockLevels, above = 0;  // count(lo) > rank >= count(hi) == above
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int mid = (lo + hi) >> 1, n = count(mid);
+      if (n > rank) {
+        lo = mid;
+      } else {
+        hi = mid;
+        above = n;
+      }
+    }
+    int j = rank - above;  // within the level, request by request
+    const int n0 = reach(0, lo) - reach(0, hi), n1 = reach(1, lo) - reach(1, hi);
+    const int s0 = wave_scan(n0), s1 = wave_scan(n1), all0 = __builtin_amdgcn_readlane(s0, 63);
+    const int c = j < all0 ? 0 : 1;
+    if (c) j -= all0;
+    const int incl = c ? s1 : s0, n = c ? n1 : n0;
+    const int at = __builtin_ctzll(__builtin_amdgcn_ballot_w64(incl > j));
+    const int b = __builtin_amdgcn_readlane((c ? nb[1] : nb[0]) - 1 - (c ? reach(1, hi) : reach(0, hi)) + incl - n, at) - j;
+    o->r = at + 64 * c;
+    o->q_begin = __builtin_amdgcn_readlane(c ? cq[1] : cq[0], at);
+    o->Lq = __builtin_amdgcn_readlane(c ? lq[1] : lq[0], at);
+    o->Lk = __builtin_amdgcn_readlane(c ? lk[1] : lk[0], at);
+    o->q0 = b * SBQ;
+    return true;
+  }
+  // 64 candidates per pass, one per lane (a pass is one trip to memory, and nothing of the workgroup's work can start
+  // before its request is known): the last request whose first block is not past this one.  The same pass fetches
+  // what is needed of that request.
+  const int sb = blocks - 1 - rank;
+  int r = 0;
+  for (int n = p.R;;) {  // the answer lies in [r, r + n)
+    const int stride = (n + 63) >> 6;
+    const int idx = r + lane * stride;
+    const bool in = lane * stride < n;
+    const int cq = in ? p.cu_q[idx] : 0, cq1 = in ? p.cu_q[idx + 1] : 0, len = in ? p.lens[idx] : 0;
+    const int c = __builtin_popcountll(__builtin_amdgcn_ballot_w64(in && cq / SBQ + idx <= sb)) - 1;  // >= 0: the first candidate always qualifies
+    r += c * stride;
+    n = min(stride, n - c * stride);
+    if (stride == 1) {
+      o->r = r;
+      o->q_begin = __builtin_amdgcn_readlane(cq, c);
+      o->Lq = __builtin_amdgcn_readlane(cq1, c) - o->q_begin;
+      o->Lk = __builtin_amdgcn_readlane(len, c);
+      break;
+    }
+  }
+  o->q0 = (sb - (o->q_begin / SBQ + r)) * SBQ;
+  return o->q0 < o->Lq && !(p.skip_single && o->Lq == 1);
+}
+
 // The one-stream ("woven") tile kernel for head_dim 64 and 128 (paged_prefill_woven.hip).  Same grid and request ->
 // workgroup map as the two-phase tile kernel: `grid.x` workgroups of prefill_woven_waves wavefronts, `grid.y` key
 // ranges (with more than one, `p.split_o` / `p.split_lse` receive the partials).

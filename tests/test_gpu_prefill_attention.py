@@ -379,3 +379,23 @@ def test_batches_of_many_requests(mi, dev, R, kernel):
     vc = torch.randn(N, chunk, Hkv, d, generator=gen).bfloat16().to(dev)
     with mi.ops.tuning(prefill_two_phase=kernel):
         _check(mi, q, kc, vc, cu_q.to(dev), kv_lens.to(dev), bt.to(dev))
+
+
+@pytest.mark.parametrize("R", [2, 63, 64, 65, 127, 128, 129])
+@pytest.mark.parametrize("d", [64, 128, 192])
+def test_blocks_handed_out_longest_first(mi, dev, R, d):
+    """Ragged prompts with empty, one-row and many-block requests among them: up to 128 requests (two per lane) a
+    workgroup takes its query block by length, with more in the batch's order."""
+    gen = torch.Generator().manual_seed(1000 * R + d)
+    q_lens = torch.randint(0, 90, (R,), generator=gen)
+    q_lens[0], q_lens[-1] = 1, 517
+    ctx = torch.where(torch.rand(R, generator=gen) < 0.5, 0, torch.randint(0, 900, (R,), generator=gen))
+    Hq, Hkv, chunk = 8, 2, 64
+    kv_lens = (q_lens + ctx).to(torch.int32)
+    cu_q = torch.zeros(R + 1, dtype=torch.int32)
+    cu_q[1:] = torch.cumsum(q_lens, 0)
+    bt, N = mi.synthetic.build_block_table(kv_lens, chunk, gen)
+    q = torch.randn(int(cu_q[-1]), Hq, d, generator=gen).bfloat16().to(dev)
+    kc = torch.randn(N, chunk, Hkv, d, generator=gen).bfloat16().to(dev)
+    vc = torch.randn(N, chunk, Hkv, d, generator=gen).bfloat16().to(dev)
+    _check(mi, q, kc, vc, cu_q.to(dev), kv_lens.to(dev), bt.to(dev))
