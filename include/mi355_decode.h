@@ -376,6 +376,33 @@ int mi_paged_prefill_attention_tiles(const void* q, int64_t q_stride_tok, int64_
                                      int32_t dtype, const MiTuning* tuning, void* stream);
 
 /*
+ * The prompts of a step from the QKV projection's output `[T][(Hq + 2 Hkv) * head_dim]` (rows `qkv_stride_tok` elements
+ * apart; per KV head: its query heads, its key head, its value head) in two calls, without a pass over the queries.
+ *
+ * mi_qkv_key_append: key norm and rotation, keys and values -> their cache rows (and / or the keys -> k_out, for a cache
+ * that is quantised afterwards), and cos | sin of every row's query position -> `cos_sin` `[T][2][head_dim]` in the
+ * tensors' 16-bit type (not touched without rotary_angles).  Angles are head_dim wide; roundings as in
+ * mi_qkv_norm_rope_append with faithful_rounding.
+ * mi_qkv_prefill_attention: mi_paged_prefill_attention_tiles over the raw queries; the tile kernel norms and rotates
+ * them as it loads them (cos_sin NULL: no rotation).  head_dim 64 or 128, chunk_tokens a multiple of 64.
+ */
+int mi_qkv_key_append(const void* mixed_qkv, int64_t qkv_stride_tok, void* k_out, int64_t k_out_stride_tok,
+                      const void* k_weight, float eps, int32_t norm_kind, const float* rotary_angles,
+                      int64_t angles_stride, int32_t rotary_interleaved, float mscale, const int64_t* q_positions,
+                      const int64_t* k_positions, void* k_cache, void* v_cache, int64_t kv_stride_chunk,
+                      int64_t kv_stride_tok, const int64_t* token_to_chunk_idx, const int64_t* token_to_local_pos,
+                      void* cos_sin, int32_t T, int32_t Hq, int32_t Hkv, int32_t head_dim, int32_t dtype, void* stream);
+int mi_qkv_prefill_attention(const void* mixed_qkv, int64_t qkv_stride_tok, const void* q_weight, float eps,
+                             int32_t norm_kind, const void* cos_sin, int32_t rotary_interleaved, const void* k_cache,
+                             const void* v_cache, int64_t kv_stride_chunk, int64_t kv_stride_tok,
+                             int64_t kv_stride_head, int32_t kv_dtype, const float* k_scales, const float* v_scales,
+                             const int32_t* block_table, int64_t bt_stride, const int32_t* cu_seqlens_q,
+                             const int32_t* kv_lens, void* out, int64_t o_stride_tok, int64_t o_stride_head,
+                             void* workspace, int64_t workspace_bytes, int32_t T, int32_t R, int32_t Hq, int32_t Hkv,
+                             int32_t head_dim, int32_t chunk_tokens, int32_t max_kv_len, float softmax_scale,
+                             int32_t dtype, void* stream);
+
+/*
  * Paged varlen causal attention with keys wider than values: the prefill / mixed step of
  * multi-latent attention, where the reference decompresses the latent cache into a key cache
  * `[n_chunks, chunk_tokens, H, 192]` (128 + the 64 shared rotary values) and a value cache

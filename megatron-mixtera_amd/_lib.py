@@ -80,6 +80,13 @@ SIGNATURES = {
         c_int,
         [_P, _I64, _I64, _P, _P, _I64, _I64, _I64, _I32, _P, _P, _P, _I64, _P, _P, _P, _I64, _I64, _P, _I64,
          _I32, _I32, _I32, _I32, _I32, _I32, _I32, _F, _I32, _P, _P]),
+    "mi_qkv_key_append": (
+        c_int, [_P, _I64, _P, _I64, _P, _F, _I32, _P, _I64, _I32, _F, _P, _P, _P, _P, _I64, _I64, _P, _P, _P,
+                _I32, _I32, _I32, _I32, _I32, _P]),
+    "mi_qkv_prefill_attention": (
+        c_int,
+        [_P, _I64, _P, _F, _I32, _P, _I32, _P, _P, _I64, _I64, _I64, _I32, _P, _P, _P, _I64, _P, _P, _P, _I64, _I64, _P, _I64,
+         _I32, _I32, _I32, _I32, _I32, _I32, _I32, _F, _I32, _P]),
     "mi_paged_prefill_attention_mla": (
         c_int,
         [_P, _I64, _I64, _P, _I64, _I64, _I64, _P, _I64, _I64, _I64, _P, _I64, _P, _P, _P, _I64, _I64,

@@ -132,6 +132,12 @@ class PagedSelfAttentionCore(torch.nn.Module):
                 self.layer_number, mixed_qkv=mixed_qkv, num_query_heads=num_query_heads, rotary_pos_emb=emb,
                 softmax_scale=self.softmax_scale, **self._norm_args())
             return out.reshape(out.size(0), out.size(1), -1)
+        fusable = getattr(ctx, "prefill_fusable", None)
+        if self.fused and fusable is not None and fusable(mixed_qkv, self.head_dim, emb):
+            out = ctx.fused_prefill_attention(
+                self.layer_number, mixed_qkv, num_query_heads=num_query_heads, rotary_pos_emb=emb,
+                softmax_scale=self.softmax_scale, **self._norm_args())
+            return out.reshape(out.size(0), out.size(1), -1)
         query = ctx.fused_qkv_norm_rope_append(
             self.layer_number, mixed_qkv, num_query_heads=num_query_heads, rotary_pos_emb=emb, **self._norm_args())
         return self._attend(query, ctx)

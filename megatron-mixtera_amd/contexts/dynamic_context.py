@@ -688,6 +688,45 @@ class DynamicInferenceContext:
             faithful_rounding=faithful_rounding)
         return query_out
 
+    def prefill_fusable(self, mixed_qkv: Tensor, head_dim: int, rotary_pos_emb: Optional[Tensor]) -> bool:
+        """Whether :meth:`fused_prefill_attention` serves this step: every request was just admitted with more than one
+        token, and the tile kernel takes the shapes."""
+        return (not self.cache_mla_latent and not self.one_row_requests_possible() and not self.is_decode_only()
+                and mixed_qkv.is_cuda and mixed_qkv.stride(0) % 8 == 0 and mixed_qkv.data_ptr() % 16 == 0
+                and ops.qkv_prefill_supported(head_dim, self.chunk_size_tokens, rotary_pos_emb))
+
+    def fused_prefill_attention(self, layer_number: int, mixed_qkv: Tensor, *, num_query_heads: int,
+                                rotary_pos_emb: Optional[Tensor], config=None, q_weight: Optional[Tensor] = None,
+                                k_weight: Optional[Tensor] = None, norm: Optional[str] = None, eps: float = 1e-5,
+                                softmax_scale: Optional[float] = None) -> Tensor:
+        """:meth:`fused_qkv_norm_rope_append` and the attention over the cache for a step of prompts, ``[T, 1, Hq, d]``:
+        one launch for keys and values, and the queries are normed and rotated where attention loads them."""
+        n, hkv, d = self.padded_active_token_count, self.num_kv_heads_per_partition, self.kv_channels
+        interleaved = self._rope_flags(config) if config is not None else False
+        k_cache, v_cache = self._layer_cache(layer_number)
+        k_scales, v_scales = self.key_value_scales(layer_number)
+        common = dict(num_query_heads=num_query_heads, num_kv_heads=hkv, eps=eps, norm=norm, rotary_interleaved=interleaved)
+        keys = dict(k_weight=k_weight, rotary_emb=rotary_pos_emb, q_positions=self.token_to_pos_ids,
+                    k_positions=self.token_to_position_in_request, **common)
+        rows = _first(mixed_qkv, n)
+        if self.kv_cache_fp8:
+            key = torch.empty((n, 1, hkv, d), dtype=mixed_qkv.dtype, device=mixed_qkv.device)
+            cos_sin = ops.qkv_key_append(rows, key_out=key, **keys)
+            group = num_query_heads // hkv
+            value = rows.reshape(n, hkv, (group + 2) * d)[:, :, (group + 1) * d:]
+            self.append_key_value_cache(layer_number, key, value.unsqueeze(1))
+        else:
+            cos_sin = ops.qkv_key_append(rows, k_cache=k_cache, v_cache=v_cache, token_to_chunk_idx=self.token_to_chunk_idx,
+                                         token_to_local_pos=self.token_to_local_position_within_kv_chunk, **keys)
+        out = ops.qkv_prefill_attention(rows, k_cache, v_cache, self.cu_query_seq_lengths, self.kv_seq_lengths, self.block_table,
+                                        cos_sin=cos_sin, q_weight=q_weight, softmax_scale=softmax_scale,
+                                        max_kv_len=self.attention_length_bounds()[1], k_scales=k_scales, v_scales=v_scales, **common)
+        if n == mixed_qkv.size(0):
+            return out
+        more = out.new_zeros(mixed_qkv.size(0), *out.shape[1:])   # rows beyond the step's padding
+        more[:n] = out
+        return more
+
     # ------------------------------------------------------------------ per-step attention state
     def reset_attention_state(self) -> None:
         """Forget the per-step attention metadata (the fixed-address mirrors are zeroed)."""

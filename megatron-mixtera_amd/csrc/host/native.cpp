@@ -671,6 +671,77 @@ PyObject* qkv_norm_rope_append(PyObject* const* a) {
   Py_RETURN_NONE;
 }
 
+// qkv_key_append(mixed_qkv, num_query_heads, num_kv_heads, key_out|None, k_weight|None, eps, norm_kind, rotary_emb|None,
+//                q_positions, k_positions, interleaved, mscale, k_cache|None, v_cache|None, token_to_chunk_idx|None,
+//                token_to_local_pos|None) -> cos | sin [T, 2, d] of the query positions (None without rotary_emb)
+PyObject* qkv_key_append(PyObject* const* a) {
+  const Mixed m = mixed_of(a[0], a[1], a[2], "mixed_qkv must be [T, 1, W]");
+  const Tensor& ref = *m.t;
+  Rows3 ko;
+  if (const Tensor* t = opt_tensor(a[3], "key_out")) {
+    ko = rows3(*t, "key_out");
+    REQUIRE(ko.n == m.T && ko.h == m.Hkv && ko.d == m.D && ko.sh == m.D && t->scalar_type() == ref.scalar_type(), "key_out must be [T, Hkv, d]");
+  }
+  const Tensor *kc = opt_tensor(a[12], "k_cache"), *vc = opt_tensor(a[13], "v_cache");
+  REQUIRE(ko.t || kc, "the key needs a destination: key_out and/or the cache");
+  const Angles ang = angles_of(opt_tensor(a[7], "rotary_emb"));
+  REQUIRE(!ang.ptr || ang.rot == m.D, "rotary_emb must be as wide as a head");
+  const Tensor* kw = opt_tensor(a[4], "k_weight");
+  check_norm_weight(kw, ref, m.D);
+  const Tensor *qp = opt_tensor(a[8], "q_positions"), *kp = opt_tensor(a[9], "k_positions");
+  const Tensor *ci = opt_tensor(a[14], "token_to_chunk_idx"), *lp = opt_tensor(a[15], "token_to_local_pos");
+  for (const Tensor* t : {qp, kp, ci, lp}) check_index_row(t, m.T, "index rows must be int64 [>=T]");
+  const CacheSlots s = slots_of(kc, vc, nullptr, nullptr, ref, m.D, "the caches must have the projection's 16-bit type");
+  REQUIRE(!kc || kc->size(2) == m.Hkv, "cache shape mismatch");
+  Tensor angles;
+  if (ang.ptr) angles = at::empty({m.T, 2, m.D}, ref.options());
+  check(mi_qkv_key_append(ref.data_ptr(), m.st, ko.ptr(), ko.sn, ptr(kw), (float)as_float(a[5]), (int)as_int(a[6]), ang.ptr,
+                          ang.stride, as_bool(a[10]), (float)as_float(a[11]), (const int64_t*)ptr(qp), (const int64_t*)ptr(kp),
+                          ptr(kc), ptr(vc), s.sc, s.st, (const int64_t*)ptr(ci), (const int64_t*)ptr(lp),
+                          ang.ptr ? angles.data_ptr() : nullptr, (int)m.T, (int)m.Hq, (int)m.Hkv, (int)m.D, dtype_code(ref),
+                          stream_of(ref)),
+        "mi_qkv_key_append");
+  return ang.ptr ? wrap(angles) : same(Py_None);
+}
+
+// qkv_prefill_attention(mixed_qkv, num_query_heads, num_kv_heads, q_weight|None, eps, norm_kind, cos_sin|None, interleaved,
+//                       k_cache, v_cache, cu_seqlens_q, kv_lens, block_table, softmax_scale|None, max_kv_len, k_scales|None,
+//                       v_scales|None, override|None) -> [T, 1, Hq, d]
+PyObject* qkv_prefill_attention(PyObject* const* a) {
+  const Mixed m = mixed_of(a[0], a[1], a[2], "mixed_qkv must be [T, 1, W]");
+  const Tensor& ref = *m.t;
+  void* stream = stream_of(ref);
+  const Tensor &kc = tensor(a[8], "k_cache"), &vc = tensor(a[9], "v_cache"), &cu = tensor(a[10], "cu_seqlens_q");
+  const Tensor &lens = tensor(a[11], "kv_lens"), &table = tensor(a[12], "block_table");
+  const Tensor *qw = opt_tensor(a[3], "q_weight"), *angles = opt_tensor(a[6], "cos_sin");
+  check_norm_weight(qw, ref, m.D);
+  REQUIRE(kc.dim() == 4 && kc.size(3) == m.D && kc.size(2) == m.Hkv && same_shape(kc, vc), "cache shape mismatch");
+  const Tensor *ks = opt_tensor(a[15], "k_scales"), *vs = opt_tensor(a[16], "v_scales");
+  const Cache c = cache_of(kc);
+  if (ks) {
+    REQUIRE(kc.element_size() == 1 && vc.element_size() == 1, "fp8 caches hold one byte per element");
+    REQUIRE(scales_ok(ks, c.n, c.h) && scales_ok(vs, c.n, c.h), "scales must be contiguous fp32 [N, Hkv]");
+  } else {
+    REQUIRE(kc.scalar_type() == ref.scalar_type() && vc.scalar_type() == ref.scalar_type(), "the cache must have the queries' 16-bit type, or be bytes with scales");
+  }
+  REQUIRE(same_strides(cache_of(vc), c), "k_cache / v_cache strides differ");
+  REQUIRE(cu.scalar_type() == at::kInt && cu.is_contiguous(), "cu_seqlens_q must be contiguous int32");
+  REQUIRE(!angles || (angles->scalar_type() == ref.scalar_type() && angles->is_contiguous() && angles->numel() >= m.T * 2 * m.D),
+          "cos_sin must be [T, 2, d] of the projection's type");
+  const int64_t R = cu.numel() - 1, max_len = as_int(a[14]);
+  check_table(table, lens, R);
+  Tensor out = at::empty({m.T, 1, m.Hq, m.D}, ref.options());
+  const Scratch ws = scratch(ref, stream, mi_prefill_workspace_bytes((int)m.T, (int)R, (int)m.Hq, (int)m.Hkv, (int)m.D, (int)max_len, 0, nullptr), Py_None, a[17]);
+  check(mi_qkv_prefill_attention(ref.data_ptr(), m.st, ptr(qw), (float)as_float(a[4]), (int)as_int(a[5]), angles ? angles->data_ptr() : nullptr,
+                                 as_bool(a[7]), kc.data_ptr(), vc.data_ptr(), c.sc, c.st, c.sh, ks ? MI_KV_FP8_E4M3 : MI_KV_16BIT,
+                                 (const float*)ptr(ks), (const float*)ptr(vs), (const int32_t*)table.data_ptr(), table.stride(0),
+                                 (const int32_t*)cu.data_ptr(), (const int32_t*)lens.data_ptr(), out.data_ptr(), m.Hq * m.D, m.D,
+                                 ws.ptr, ws.bytes, (int)m.T, (int)R, (int)m.Hq, (int)m.Hkv, (int)m.D, (int)c.c, (int)max_len,
+                                 a[13] == Py_None ? default_scale(m.D) : (float)as_float(a[13]), dtype_code(ref), stream),
+        "mi_qkv_prefill_attention");
+  return wrap(out);
+}
+
 // decode_step_attention(query|None, key|None, value|None, mixed_qkv|None, num_query_heads, num_kv_heads, k_cache, v_cache,
 //                       kv_lens, block_table, q_weight|None, k_weight|None, eps, norm_kind, rotary_emb|None,
 //                       positions|None, interleaved, mscale, softmax_scale|None, max_kv_len|None, split_tokens, out|None,
@@ -982,7 +1053,8 @@ PyMethodDef kMethods[] = {
     ABI(mi_prefill_workspace_bytes), ABI(mi_paged_decode_attention_noalloc),
     ABI(mi_update_requests), ABI(mi_update_requests_mask8), ABI(mi_add_request), ABI(mi_decode_attention_state), ABI(mi_step_attention_state),
     OP(kv_append, 6), OP(kv_append_fp8, 9), OP(paged_decode_attention, 14), OP(paged_mla_decode_attention, 10),
-    OP(paged_prefill_attention, 14), OP(paged_prefill_attention_mla, 11), OP(norm_rope_append, 22), OP(qkv_norm_rope_append, 22), OP(decode_step_attention, 29),
+    OP(paged_prefill_attention, 14), OP(paged_prefill_attention_mla, 11), OP(norm_rope_append, 22), OP(qkv_norm_rope_append, 22), OP(qkv_key_append, 16),
+    OP(qkv_prefill_attention, 18), OP(decode_step_attention, 29),
     OP(linear_decode, 5), OP(attention_layer_decode, 24), OP(sample_from_logits, 12), OP(selected_log_probs, 2), OP(last_token_gather, 3), OP(setup, 3),
     OP(set_workspace, 3), OP(watch, 4), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_native", "Host side of the per-layer calls.", -1, kMethods, nullptr, nullptr, nullptr, nullptr};

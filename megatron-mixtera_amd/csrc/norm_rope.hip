@@ -434,6 +434,117 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6, 8))) voi
 
 }  // namespace mi
 
+namespace mi {
+// Keys and values of the QKV projection's output -> cache (or the keys -> k_out), and cos | sin of every query position
+// -> `angles` [T][2][D] in the tensors' 16-bit type (the sine with the sign of its partner term), for the prefill tile
+// kernel, which norms and rotates the queries as it loads them.
+//
+// Bound by memory: per token the keys and values in and out and 4 D bytes of table.  A workgroup takes four tokens so
+// that every lane has a piece of a head vector (one token's eight key heads fill a quarter of it) and evaluates each
+// angle of its tokens once for all heads; pieces are requested before the positions' chain of trips.  Leaving the
+// queries to the tile kernel saves reading and writing them here: 12 348 tokens of 32 / 8 heads of 64.
+constexpr int kKeyTokens = 4;
+template <int D, bool F16>
+__global__ __launch_bounds__(256) void qkv_key_append_kernel(NormRopeParams p, uint16_t* __restrict__ angles) {
+  constexpr int LPV = D / 8, VPB = 256 / LPV;  // lanes per head vector, head vectors per pass
+  __shared__ __align__(16) float cs[kKeyTokens][2][D];
+  const int t0 = blockIdx.x * kKeyTokens, nt = min(kKeyTokens, p.T - t0), nvec = nt * p.Hkv;
+  const int slot = threadIdx.x / LPV, li = threadIdx.x % LPV, e0 = 8 * li;
+  struct Piece {
+    uint4 k, v;
+    int tok, h;
+  };
+  auto load = [&](int vec) {
+    Piece x;
+    x.tok = vec / p.Hkv;
+    x.h = vec - x.tok * p.Hkv;
+    x.k = x.v = make_uint4(0, 0, 0, 0);
+    if (vec < nvec) {
+      x.k = ld16(p.k + (int64_t)(t0 + x.tok) * p.k_st + (int64_t)x.h * p.k_hst + e0);
+      if (p.kc) x.v = ld16(p.v + (int64_t)(t0 + x.tok) * p.v_st + (int64_t)x.h * p.v_hst + e0);
+    }
+    return x;
+  };
+  Piece next = load(slot);
+  if (p.emb) {
+    for (int job = threadIdx.x; job < nt * D; job += 256) {
+      const int tok = job / D, e = job % D;
+      const int64_t qp = p.q_pos[t0 + tok], kp = p.k_pos[t0 + tok];
+      auto eval = [&](int64_t pos, float& c, float& sn) {
+        rotary_sincos(p.emb[pos * p.emb_stride + e], &sn, &c);
+        c = round16<F16>(c * p.mscale);
+        sn = round16<F16>(sn * p.mscale);
+        if (p.interleaved ? (e & 1) == 0 : e < D / 2) sn = -sn;
+      };
+      float c, sn;
+      eval(kp, c, sn);
+      cs[tok][0][e] = c;
+      cs[tok][1][e] = sn;
+      if (qp != kp) eval(qp, c, sn);
+      uint16_t* row = angles + (int64_t)(t0 + tok) * 2 * D;
+      row[e] = f32_to_16<F16>(c);
+      row[D + e] = f32_to_16<F16>(sn);
+    }
+    __syncthreads();
+  }
+  uint4 w_raw = make_uint4(ones2<F16>(), ones2<F16>(), ones2<F16>(), ones2<F16>());
+  if (p.norm == MI_NORM_RMS && p.k_w) w_raw = ld16(p.k_w + e0);
+  for (int vec0 = 0; vec0 < nvec; vec0 += VPB) {
+    const Piece x = next;
+    next = load(vec0 + VPB + slot);
+    float y[8], o[8];
+    {
+      const uint32_t w4[4] = {x.k.x, x.k.y, x.k.z, x.k.w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) { y[2 * j] = lo_to_f32<F16>(w4[j]); y[2 * j + 1] = hi_to_f32<F16>(w4[j]); }
+    }
+    if (p.norm != MI_NORM_NONE) {
+      float ss = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) ss += y[j] * y[j];
+      ss = lane_group_sum<LPV>(ss);
+      const float rstd = rsqrtf(ss * (1.f / D) + p.eps);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) y[j] *= rstd;
+      if (p.norm == MI_NORM_RMS) {
+        const uint32_t w4[4] = {w_raw.x, w_raw.y, w_raw.z, w_raw.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) { y[2 * j] *= lo_to_f32<F16>(w4[j]); y[2 * j + 1] *= hi_to_f32<F16>(w4[j]); }
+      }
+#pragma unroll
+      for (int j = 0; j < 8; j += 2) round16_pair<F16>(y[j], y[j + 1]);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] = y[j];
+    if (p.emb) {
+      float yp[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) yp[j] = p.interleaved ? y[j ^ 1] : lane_xor<LPV / 2>(y[j]);
+      const int tok = min(x.tok, nt - 1);
+#pragma unroll
+      for (int j = 0; j < 8; j += 2) {
+        float a0 = y[j] * cs[tok][0][e0 + j], a1 = y[j + 1] * cs[tok][0][e0 + j + 1];
+        float b0 = yp[j] * cs[tok][1][e0 + j], b1 = yp[j + 1] * cs[tok][1][e0 + j + 1];
+        round16_pair<F16>(a0, a1);
+        round16_pair<F16>(b0, b1);
+        o[j] = a0 + b0;
+        o[j + 1] = a1 + b1;
+      }
+    }
+    if (vec0 + slot < nvec) {
+      const uint4 packed = make_uint4(pack2<F16>(o[0], o[1]), pack2<F16>(o[2], o[3]), pack2<F16>(o[4], o[5]), pack2<F16>(o[6], o[7]));
+      const int t = t0 + x.tok;
+      if (p.k_out) st16(p.k_out + (int64_t)t * p.ko_st + (int64_t)x.h * D + e0, packed);
+      if (p.kc) {
+        const int64_t off = p.tok_chunk[t] * p.chunk_elems + p.tok_local[t] * p.tok_elems + (int64_t)x.h * D + e0;
+        st16(p.kc + off, packed);
+        st16(p.vc + off, x.v);
+      }
+    }
+  }
+}
+}  // namespace mi
+
 using namespace mi;
 
 namespace {
@@ -581,4 +692,48 @@ extern "C" int mi_qkv_norm_rope_append(
   p.norm = norm_kind; p.interleaved = rotary_interleaved; p.faithful = faithful_rounding;
   p.eps = eps; p.mscale = mscale;
   return norm_rope_launch(p, dtype, tuning, (hipStream_t)stream, "mi_qkv_norm_rope_append");
+}
+
+extern "C" int mi_qkv_key_append(
+    const void* mixed_qkv, int64_t qkv_stride_tok, void* k_out, int64_t k_out_stride_tok, const void* k_weight, float eps,
+    int32_t norm_kind, const float* rotary_angles, int64_t angles_stride, int32_t rotary_interleaved, float mscale,
+    const int64_t* q_positions, const int64_t* k_positions, void* k_cache, void* v_cache, int64_t kv_stride_chunk,
+    int64_t kv_stride_tok, const int64_t* token_to_chunk_idx, const int64_t* token_to_local_pos, void* cos_sin, int32_t T,
+    int32_t Hq, int32_t Hkv, int32_t head_dim, int32_t dtype, void* stream) {
+  if (T == 0) return MI_OK;
+  if (dtype != MI_DTYPE_BF16 && dtype != MI_DTYPE_FP16)
+    return mi_fail(MI_ERR_UNSUPPORTED, "mi_qkv_key_append: dtype must be MI_DTYPE_BF16 or MI_DTYPE_FP16");
+  if (norm_kind != MI_NORM_NONE && norm_kind != MI_NORM_RMS && norm_kind != MI_NORM_L2)
+    return mi_fail(MI_ERR_UNSUPPORTED, "mi_qkv_key_append: unknown norm kind");
+  if (T < 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv)
+    return mi_fail(MI_ERR_SHAPE, "mi_qkv_key_append: query heads must be a positive multiple of KV heads");
+  if (head_dim != 64 && head_dim != 128) return mi_fail(MI_ERR_UNSUPPORTED, "mi_qkv_key_append: head_dim must be 64 or 128");
+  if (!mixed_qkv || (!k_cache && !k_out) || (k_cache && (!v_cache || !token_to_chunk_idx || !token_to_local_pos)) ||
+      (rotary_angles && (!q_positions || !k_positions || !cos_sin)))
+    return mi_fail(MI_ERR_NULL, "mi_qkv_key_append: null pointer argument");
+  const int G = Hq / Hkv;
+  const int64_t group = (int64_t)(G + 2) * head_dim;
+  if (qkv_stride_tok < group * Hkv || (rotary_angles && angles_stride < head_dim))
+    return mi_fail(MI_ERR_SHAPE, "mi_qkv_key_append: token stride smaller than (Hq + 2 Hkv) * head_dim, or angles narrower than head_dim");
+  if ((((uintptr_t)mixed_qkv | (uintptr_t)k_out | (uintptr_t)k_weight | (uintptr_t)k_cache | (uintptr_t)v_cache | (uintptr_t)cos_sin) & 15) ||
+      ((qkv_stride_tok | k_out_stride_tok | kv_stride_chunk | kv_stride_tok) & 7))
+    return mi_fail(MI_ERR_ALIGN, "mi_qkv_key_append: rows must be 16-byte aligned");
+  const uint16_t* base = (const uint16_t*)mixed_qkv;
+  NormRopeParams p = {};
+  p.k = base + (int64_t)G * head_dim; p.k_st = qkv_stride_tok; p.k_hst = group;
+  p.v = base + (int64_t)(G + 1) * head_dim; p.v_st = qkv_stride_tok; p.v_hst = group;
+  p.k_out = (uint16_t*)k_out; p.ko_st = k_out_stride_tok;
+  p.k_w = (const uint16_t*)k_weight;
+  p.emb = rotary_angles; p.emb_stride = angles_stride; p.q_pos = q_positions; p.k_pos = k_positions;
+  p.kc = (uint16_t*)k_cache; p.vc = (uint16_t*)v_cache; p.chunk_elems = kv_stride_chunk; p.tok_elems = kv_stride_tok;
+  p.tok_chunk = token_to_chunk_idx; p.tok_local = token_to_local_pos;
+  p.T = T; p.Hkv = Hkv; p.norm = norm_kind; p.interleaved = rotary_interleaved; p.eps = eps; p.mscale = mscale;
+  const dim3 grid((T + kKeyTokens - 1) / kKeyTokens);
+  hipStream_t st = (hipStream_t)stream;
+  const bool f16 = dtype == MI_DTYPE_FP16;
+  if (head_dim == 128 && f16) hipLaunchKernelGGL((qkv_key_append_kernel<128, true>), grid, dim3(256), 0, st, p, (uint16_t*)cos_sin);
+  else if (head_dim == 128) hipLaunchKernelGGL((qkv_key_append_kernel<128, false>), grid, dim3(256), 0, st, p, (uint16_t*)cos_sin);
+  else if (f16) hipLaunchKernelGGL((qkv_key_append_kernel<64, true>), grid, dim3(256), 0, st, p, (uint16_t*)cos_sin);
+  else hipLaunchKernelGGL((qkv_key_append_kernel<64, false>), grid, dim3(256), 0, st, p, (uint16_t*)cos_sin);
+  return mi_check_launch("mi_qkv_key_append");
 }

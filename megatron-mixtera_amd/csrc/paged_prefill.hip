@@ -1032,6 +1032,14 @@ extern "C" int64_t mi_prefill_workspace_bytes(int32_t T, int32_t R, int32_t Hq, 
     else hipLaunchKernelGGL((paged_prefill_pp_kernel<false, FP8_, false, HD_, HDK_, F16_>), lgrid, dim3(512), 0, st, p);                      \
   } while (0)
 
+// queries of the QKV projection's output (see PrefillParams)
+struct RawQueries {
+  int64_t group_stride;
+  const void* angles;
+  const void* weight;
+  float eps;
+  int32_t norm, interleaved;
+};
 static int launch_paged_prefill(
     const void* q, int64_t q_stride_tok, int64_t q_stride_head, const void* k_cache,
     const void* v_cache, int64_t kv_stride_chunk, int64_t kv_stride_tok, int64_t kv_stride_head,
@@ -1040,7 +1048,7 @@ static int launch_paged_prefill(
     void* workspace, int64_t workspace_bytes, int32_t T, int32_t R, int32_t Hq, int32_t Hkv,
     int32_t head_dim, int32_t chunk_tokens, int32_t max_kv_len, int32_t split_tokens, float softmax_scale,
     int32_t kv_dtype, const float* k_scales, const float* v_scales, int32_t dtype, const MiTuning* tuning,
-    void* stream, bool one_row_requests = true) {
+    void* stream, bool one_row_requests = true, const RawQueries* raw = nullptr) {
   const bool fp8 = kv_dtype == MI_KV_FP8_E4M3;
   if (T == 0 || R == 0) return MI_OK;
   MiTuning tune;
@@ -1100,6 +1108,14 @@ static int launch_paged_prefill(
   p.skip_single = workspace != nullptr && one_row_requests;
   p.k_scale = k_scales; p.v_scale = v_scales;
   p.split_o = nullptr; p.split_lse = nullptr;
+  p.q_gst = raw ? raw->group_stride : G * q_stride_head;
+  p.angles = raw ? (const uint16_t*)raw->angles : nullptr;
+  p.q_w = raw ? (const uint16_t*)raw->weight : nullptr;
+  p.eps = raw ? raw->eps : 0.f;
+  p.norm = raw ? raw->norm : MI_NORM_NONE;
+  p.interleaved = raw ? raw->interleaved : 0;
+  if (raw && !(two_phase && tune.prefill_two_phase == 3 && (head_dim == 64 || head_dim == 128)))
+    return mi_fail(MI_ERR_UNSUPPORTED, "mi_qkv_prefill_attention: head_dim 64 or 128 and a chunk size that is a multiple of 64");
 
   // The decode part's own argument checks come before the first launch, so that a negative return still means
   // nothing was enqueued (its remaining checks repeat ones made above).
@@ -1235,6 +1251,28 @@ extern "C" int mi_paged_prefill_attention_tiles(
                               kv_stride_head, block_table, bt_stride, cu_seqlens_q, kv_lens, out, o_stride_tok,
                               o_stride_head, workspace, workspace_bytes, T, R, Hq, Hkv, head_dim, chunk_tokens,
                               max_kv_len, 0, softmax_scale, kv_dtype, k_scales, v_scales, dtype, tuning, stream, false);
+}
+
+extern "C" int mi_qkv_prefill_attention(
+    const void* mixed_qkv, int64_t qkv_stride_tok, const void* q_weight, float eps, int32_t norm_kind, const void* cos_sin,
+    int32_t rotary_interleaved, const void* k_cache, const void* v_cache, int64_t kv_stride_chunk, int64_t kv_stride_tok,
+    int64_t kv_stride_head, int32_t kv_dtype, const float* k_scales, const float* v_scales, const int32_t* block_table,
+    int64_t bt_stride, const int32_t* cu_seqlens_q, const int32_t* kv_lens, void* out, int64_t o_stride_tok,
+    int64_t o_stride_head, void* workspace, int64_t workspace_bytes, int32_t T, int32_t R, int32_t Hq, int32_t Hkv,
+    int32_t head_dim, int32_t chunk_tokens, int32_t max_kv_len, float softmax_scale, int32_t dtype, void* stream) {
+  if (norm_kind != MI_NORM_NONE && norm_kind != MI_NORM_RMS && norm_kind != MI_NORM_L2)
+    return mi_fail(MI_ERR_UNSUPPORTED, "mi_qkv_prefill_attention: unknown norm kind");
+  if (Hq <= 0 || Hkv <= 0 || Hq % Hkv)
+    return mi_fail(MI_ERR_SHAPE, "mi_qkv_prefill_attention: query heads must be a positive multiple of KV heads");
+  if (qkv_stride_tok < (int64_t)(Hq + 2 * Hkv) * head_dim)
+    return mi_fail(MI_ERR_SHAPE, "mi_qkv_prefill_attention: token stride smaller than (Hq + 2 Hkv) * head_dim");
+  if (((uintptr_t)q_weight | (uintptr_t)cos_sin) & 15)
+    return mi_fail(MI_ERR_ALIGN, "mi_qkv_prefill_attention: the norm weight and the angles must be 16-byte aligned");
+  const RawQueries raw = {(int64_t)(Hq / Hkv + 2) * head_dim, cos_sin, q_weight, eps, norm_kind, rotary_interleaved};
+  return launch_paged_prefill(mixed_qkv, qkv_stride_tok, head_dim, k_cache, v_cache, kv_stride_chunk, kv_stride_tok,
+                              kv_stride_head, block_table, bt_stride, cu_seqlens_q, kv_lens, out, o_stride_tok,
+                              o_stride_head, workspace, workspace_bytes, T, R, Hq, Hkv, head_dim, chunk_tokens,
+                              max_kv_len, 0, softmax_scale, kv_dtype, k_scales, v_scales, dtype, nullptr, stream, false, &raw);
 }
 
 extern "C" int mi_paged_prefill_attention_mla(

@@ -33,6 +33,13 @@ struct PrefillParams {
   // log-sum-exps [range][T][Hq] (log2 domain) and a merge kernel finishes the rows.
   float* split_o;
   float* split_lse;
+  // Queries as the QKV projection left them (one-stream tile kernel only): head norm and rotation happen as they are
+  // loaded.  Otherwise q_gst == G * q_sh and the rest is off.
+  int64_t q_gst;           // elements between the query heads of two KV heads
+  const uint16_t* angles;  // [T][2][head_dim]: cos | sin of every row (see qkv_key_append_kernel), or null
+  const uint16_t* q_w;     // RMS norm weight or null
+  float eps;
+  int32_t norm, interleaved;
 };
 
 // The query heads one workgroup serves: with at most 16 query heads per KV head, all G of KV head `hv`; with more,

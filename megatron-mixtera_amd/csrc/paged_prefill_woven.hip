@@ -123,10 +123,78 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
     const int qi = (n * g_magic) >> 16, u = n - qi * G;  // n / G, n % G
     const bool valid = qi < nq;
     qpos[nt] = valid ? shift + q0 + qi : last;
-    const uint16_t* qrow = p.q + (int64_t)(q_begin + q0 + qi) * p.q_st + (int64_t)(hq0 + u) * p.q_sh;
+    const uint16_t* qrow = p.q + (int64_t)(q_begin + q0 + qi) * p.q_st + (int64_t)h * p.q_gst + (int64_t)(hq0 - h * p.G + u) * p.q_sh;
 #pragma unroll
     for (int kk = 0; kk < KS; ++kk)
       qf[nt][kk] = valid ? ld16(qrow + 32 * kk + 8 * g) : make_uint4(0, 0, 0, 0);
+  }
+  // Queries straight from the QKV projection: head norm and rotation in registers, with the roundings of the separate
+  // launch.  A row's values lie in four lanes (g), the partner of a half-split pair KS / 2 fragments away in the same
+  // lane.  It costs a workgroup about a microsecond of its tens and saves the queries' trip through memory.
+  if (p.norm != MI_NORM_NONE || p.angles) {
+#pragma unroll
+    for (int nt = 0; nt < NQ; ++nt) {
+      const int n = 16 * nt + m16;
+      const int qi = (n * g_magic) >> 16;
+      const bool valid = qi < nq;
+      const uint16_t* cs = p.angles + (int64_t)(valid ? q_begin + q0 + qi : q_begin) * (2 * HD) + 8 * g;
+      uint4 cw[KS], sw[KS];
+      if (p.angles) {
+#pragma unroll
+        for (int kk = 0; kk < KS; ++kk) {
+          cw[kk] = ld16(cs + 32 * kk);
+          sw[kk] = ld16(cs + HD + 32 * kk);
+        }
+      }
+      float x[KS][8];
+#pragma unroll
+      for (int kk = 0; kk < KS; ++kk) {
+        const uint32_t w4[4] = {qf[nt][kk].x, qf[nt][kk].y, qf[nt][kk].z, qf[nt][kk].w};
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[kk][j] = (j & 1) ? hi_to_f32<F16>(w4[j >> 1]) : lo_to_f32<F16>(w4[j >> 1]);
+      }
+      if (p.norm != MI_NORM_NONE) {
+        float ss = 0.f;
+#pragma unroll
+        for (int kk = 0; kk < KS; ++kk)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) ss += x[kk][j] * x[kk][j];
+        ss += xor16(ss);
+        ss += xor32(ss);
+        const float rstd = rsqrtf(ss * (1.f / HD) + p.eps);
+#pragma unroll
+        for (int kk = 0; kk < KS; ++kk) {
+          const uint4 w = p.norm == MI_NORM_RMS && p.q_w ? ld16(p.q_w + 32 * kk + 8 * g)
+                                                         : make_uint4(ones2<F16>(), ones2<F16>(), ones2<F16>(), ones2<F16>());
+          const uint32_t w4[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+          for (int j = 0; j < 8; j += 2) {
+            const uint32_t packed = pack2<F16>(x[kk][j] * rstd * lo_to_f32<F16>(w4[j >> 1]),
+                                               x[kk][j + 1] * rstd * hi_to_f32<F16>(w4[j >> 1]));
+            x[kk][j] = lo_to_f32<F16>(packed);
+            x[kk][j + 1] = hi_to_f32<F16>(packed);
+          }
+        }
+      }
+#pragma unroll
+      for (int kk = 0; kk < KS; ++kk) {
+        const uint32_t c4[4] = {cw[kk].x, cw[kk].y, cw[kk].z, cw[kk].w}, s4[4] = {sw[kk].x, sw[kk].y, sw[kk].z, sw[kk].w};
+        uint32_t o4[4];
+#pragma unroll
+        for (int j = 0; j < 8; j += 2) {
+          float o0 = x[kk][j], o1 = x[kk][j + 1];
+          if (p.angles) {
+            const float y0 = p.interleaved ? x[kk][j + 1] : x[kk ^ (KS / 2)][j], y1 = p.interleaved ? x[kk][j] : x[kk ^ (KS / 2)][j + 1];
+            const uint32_t a = pack2<F16>(o0 * lo_to_f32<F16>(c4[j >> 1]), o1 * hi_to_f32<F16>(c4[j >> 1]));
+            const uint32_t b = pack2<F16>(y0 * lo_to_f32<F16>(s4[j >> 1]), y1 * hi_to_f32<F16>(s4[j >> 1]));
+            o0 = lo_to_f32<F16>(a) + lo_to_f32<F16>(b);
+            o1 = hi_to_f32<F16>(a) + hi_to_f32<F16>(b);
+          }
+          o4[j >> 1] = pack2<F16>(o0, o1);
+        }
+        qf[nt][kk] = valid ? make_uint4(o4[0], o4[1], o4[2], o4[3]) : make_uint4(0, 0, 0, 0);
+      }
+    }
   }
 
   float m_run[NQ], neg_run[NQ], mwin[NQ];

@@ -29,7 +29,7 @@ def _stream(t: Tensor) -> int:
     if t.device.type != "cuda":
         raise RuntimeError(
             f"the HIP kernels need device tensors, got a tensor on {t.device}; there is no CPU path")
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def _require(cond: bool, msg: str) -> None:
@@ -393,6 +393,40 @@ def qkv_norm_rope_append(mixed_qkv: Tensor, *, num_query_heads: int, num_kv_head
                                    _NORM_KINDS[norm], rotary_emb, q_positions, k_positions, rotary_interleaved, mscale,
                                    k_cache, v_cache, token_to_chunk_idx, token_to_local_pos, block_table, kv_lens,
                                    faithful_rounding, _tuning_arg())
+
+
+def qkv_prefill_supported(head_dim: int, chunk_tokens: int, rotary_emb: Optional[Tensor]) -> bool:
+    """Whether :func:`qkv_key_append` and :func:`qkv_prefill_attention` take these sizes: the one-stream tile kernel's,
+    and every value of a head rotated (or none).  Tuning overrides ask for the separate calls."""
+    return (head_dim in (64, 128) and chunk_tokens % 64 == 0 and _tuning_arg() is None
+            and (rotary_emb is None or rotary_emb.size(-1) == head_dim))
+
+
+def qkv_key_append(mixed_qkv: Tensor, *, num_query_heads: int, num_kv_heads: int, key_out: Optional[Tensor] = None,
+                   k_weight: Optional[Tensor] = None, eps: float = 1e-5, norm: Optional[str] = None,
+                   rotary_emb: Optional[Tensor] = None, q_positions: Optional[Tensor] = None,
+                   k_positions: Optional[Tensor] = None, rotary_interleaved: bool = False, mscale: float = 1.0,
+                   k_cache: Optional[Tensor] = None, v_cache: Optional[Tensor] = None,
+                   token_to_chunk_idx: Optional[Tensor] = None,
+                   token_to_local_pos: Optional[Tensor] = None) -> Optional[Tensor]:
+    """The key / value half of :func:`qkv_norm_rope_append`.  Returns cos | sin of every row's query position
+    (``None`` without ``rotary_emb``) for :func:`qkv_prefill_attention`, which does the queries' half."""
+    return _native().qkv_key_append(mixed_qkv, num_query_heads, num_kv_heads, key_out, k_weight, eps, _NORM_KINDS[norm],
+                                    rotary_emb, q_positions, k_positions, rotary_interleaved, mscale, k_cache, v_cache,
+                                    token_to_chunk_idx, token_to_local_pos)
+
+
+def qkv_prefill_attention(mixed_qkv: Tensor, k_cache: Tensor, v_cache: Tensor, cu_seqlens_q: Tensor, kv_lens: Tensor,
+                          block_table: Tensor, *, num_query_heads: int, num_kv_heads: int, max_kv_len: int,
+                          cos_sin: Optional[Tensor] = None, q_weight: Optional[Tensor] = None, eps: float = 1e-5,
+                          norm: Optional[str] = None, rotary_interleaved: bool = False,
+                          softmax_scale: Optional[float] = None, k_scales: Optional[Tensor] = None,
+                          v_scales: Optional[Tensor] = None) -> Tensor:
+    """:func:`paged_prefill_attention` without one-row requests over the raw queries of the QKV projection's output:
+    head norm and rotation happen as the tile kernel loads them.  Returns ``[T, 1, Hq, d]``."""
+    return _native().qkv_prefill_attention(mixed_qkv, num_query_heads, num_kv_heads, q_weight, eps, _NORM_KINDS[norm],
+                                           cos_sin, rotary_interleaved, k_cache, v_cache, cu_seqlens_q, kv_lens,
+                                           block_table, softmax_scale, max_kv_len, k_scales, v_scales, _override())
 
 
 # ---------------------------------------------------------------------------------------------

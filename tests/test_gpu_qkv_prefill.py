@@ -1,0 +1,93 @@
+"""Prompts from the QKV projection's output: keys and values appended by one call, queries normed and rotated by the tile
+kernel -- against the separate calls (norm + rotary + append, then attention), whose own tests compare them with the oracle."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+CHUNK = 64
+
+
+def _batch(mi, dev, lens, hq, hkv, d, dtype, pad, seed):
+    gen = torch.Generator().manual_seed(seed)
+    lens = torch.tensor(lens, dtype=torch.int32)
+    T = int(lens.sum()) + pad
+    table, n_chunks = mi.synthetic.build_block_table(lens, CHUNK, gen)
+    cu = torch.zeros(len(lens) + 1, dtype=torch.int32)
+    cu[1:] = torch.cumsum(lens, 0)
+    pos, chunk, local = (x.to(torch.int64) for x in mi.synthetic.prefill_token_rows(cu, lens, table, CHUNK))
+    tail = torch.zeros(pad, dtype=torch.int64)
+    pos, local = torch.cat([pos, tail]), torch.cat([local, torch.arange(pad)])
+    chunk = torch.cat([chunk, tail + n_chunks])           # padded rows: a chunk of their own
+    mixed = torch.randn(T, 1, (hq + 2 * hkv) * d, generator=gen).to(dtype)
+    weights = [(1 + 0.1 * torch.randn(d, generator=gen)).to(dtype).to(dev) for _ in range(2)]
+    caches = [torch.zeros(n_chunks + 1, CHUNK, hkv, d, dtype=dtype, device=dev) for _ in range(2)]
+    return [x.to(dev) for x in (mixed, pos, chunk, local, cu, lens, table)], weights, caches, int(lens.max())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("hq,hkv,norm,interleaved,rope,lens,pad", [
+    (8, 2, "rms", False, True, (2, 31, 33, 257, 300), 7),
+    (6, 2, "l2", True, True, (65, 3, 129), 0),
+    (32, 1, "none", False, True, (2,), 1),
+    (20, 1, "rms", True, True, (515, 64), 0),
+    (8, 8, "rms", False, False, (40, 700), 3),
+    (4, 4, None, False, False, (5, 6, 7), 0),
+])
+def test_equals_the_separate_calls(mi, dev, dtype, d, hq, hkv, norm, interleaved, rope, lens, pad):
+    (mixed, pos, chunk, local, cu, kv, table), (qw, kw), caches, longest = _batch(mi, dev, lens, hq, hkv, d, dtype, pad, d + hq)
+    emb = mi.synthetic.rotary_angle_table(longest, d, base=10000.0).to(dev) if rope else None
+    ref = [c.clone() for c in caches]
+    T = mixed.size(0)
+    query = torch.empty(T, 1, hq, d, dtype=dtype, device=dev)
+    common = dict(num_query_heads=hq, num_kv_heads=hkv, norm=norm, rotary_emb=emb, q_positions=pos, k_positions=pos,
+                  rotary_interleaved=interleaved, k_weight=kw if norm == "rms" else None, token_to_chunk_idx=chunk,
+                  token_to_local_pos=local)
+    qw = qw if norm == "rms" else None
+    with mi.ops.tuning(norm_rope_vectorised=1):
+        mi.ops.qkv_norm_rope_append(mixed, query_out=query, q_weight=qw, k_cache=ref[0], v_cache=ref[1], **common)
+    want = mi.ops.paged_prefill_attention(query.squeeze(1), *ref, cu, kv, table, one_row_requests=False)
+
+    assert mi.ops.qkv_prefill_supported(d, CHUNK, emb)
+    cos_sin = mi.ops.qkv_key_append(mixed, k_cache=caches[0], v_cache=caches[1], **common)
+    got = mi.ops.qkv_prefill_attention(mixed, *caches, cu, kv, table, num_query_heads=hq, num_kv_heads=hkv,
+                                       max_kv_len=longest, cos_sin=cos_sin, q_weight=qw, norm=norm,
+                                       rotary_interleaved=interleaved).squeeze(1)
+    assert torch.equal(caches[1], ref[1])
+    rel = lambda a, b: ((a.float() - b.float()).norm() / b.float().norm()).item()
+    assert rel(caches[0], ref[0]) < 1e-3          # the norm's sum in another order: a rounding here and there
+    assert rel(got, want) < (2e-3 if dtype == torch.bfloat16 else 5e-4)
+    assert (got[int(kv.sum()):] == 0).all()
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+def test_core_takes_it_for_prompts_only(mi, dev, fp8, monkeypatch):
+    """A step of fresh prompts goes through the two calls, one with a one-token prompt through the separate ones, with
+    the same result."""
+    calls = []
+    real = mi.ops.qkv_prefill_attention
+    monkeypatch.setattr(mi.ops, "qkv_prefill_attention", lambda *a, **k: calls.append(1) or real(*a, **k))
+    hq, hkv, d = 8, 2, 128
+    gen = torch.Generator(device=dev).manual_seed(3)
+    emb = mi.synthetic.rotary_angle_table(400, d, base=10000.0).to(dev)
+    core = mi.PagedSelfAttentionCore(1, d, qk_norm="rms", device=dev).requires_grad_(False)
+    outs = {}
+    for name, lens in (("fused", (70, 333)), ("separate", (70, 333)), ("one row", (70, 1))):
+        ctx = mi.DynamicInferenceContext(
+            params_dtype=torch.bfloat16, num_layers=1, kv_channels=d, num_attention_heads=hkv, max_sequence_length=400,
+            buffer_size_gb=0.01, buffer_guaranteed_fraction=0.0, chunk_size_tokens=CHUNK, max_requests_override=4,
+            kv_cache_dtype="fp8_e4m3" if fp8 else None)
+        for i, n in enumerate(lens):
+            ctx.add_request(i, torch.arange(n, device=dev))
+        ctx.initialize_attention_state()
+        gen.manual_seed(3)
+        mixed = torch.randn(ctx.padded_active_token_count, 1, (hq + 2 * hkv) * d, generator=gen, device=dev).bfloat16()
+        before = len(calls)
+        if name == "separate":
+            monkeypatch.setattr(ctx, "prefill_fusable", lambda *a: False)
+        outs[name] = core.forward_mixed_qkv(mixed, hq, ctx, (emb, emb))
+        assert (len(calls) > before) == (name == "fused")
+        assert outs[name].isfinite().all()
+    a, b = outs["fused"].float(), outs["separate"].float()
+    assert ((a - b).norm() / b.norm()).item() < (1e-2 if fp8 else 3e-3)
