@@ -130,22 +130,32 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
   }
   // Queries straight from the QKV projection: head norm and rotation in registers, with the roundings of the separate
   // launch.  A row's values lie in four lanes (g), the partner of a half-split pair KS / 2 fragments away in the same
-  // lane.  It costs a workgroup about a microsecond of its tens and saves the queries' trip through memory.
-  if (p.norm != MI_NORM_NONE || p.angles) {
+  // lane.  What that needs is requested here, together with the queries; the arithmetic (some 900 instructions, three
+  // microseconds of a workgroup's tens) runs while the first tiles are on their way.
+  const bool raw = p.norm != MI_NORM_NONE || p.angles;
+  uint4 cw[NQ][KS], sw[NQ][KS], qw[KS];
+  if (raw) {
 #pragma unroll
-    for (int nt = 0; nt < NQ; ++nt) {
-      const int n = 16 * nt + m16;
-      const int qi = (n * g_magic) >> 16;
-      const bool valid = qi < nq;
-      const uint16_t* cs = p.angles + (int64_t)(valid ? q_begin + q0 + qi : q_begin) * (2 * HD) + 8 * g;
-      uint4 cw[KS], sw[KS];
-      if (p.angles) {
+    for (int kk = 0; kk < KS; ++kk)
+      qw[kk] = p.norm == MI_NORM_RMS && p.q_w ? ld16(p.q_w + 32 * kk + 8 * g)
+                                              : make_uint4(ones2<F16>(), ones2<F16>(), ones2<F16>(), ones2<F16>());
+    if (p.angles) {
+#pragma unroll
+      for (int nt = 0; nt < NQ; ++nt) {
+        const int qi = ((16 * nt + m16) * g_magic) >> 16;
+        const uint16_t* cs = p.angles + (int64_t)(qi < nq ? q_begin + q0 + qi : q_begin) * (2 * HD) + 8 * g;
 #pragma unroll
         for (int kk = 0; kk < KS; ++kk) {
-          cw[kk] = ld16(cs + 32 * kk);
-          sw[kk] = ld16(cs + HD + 32 * kk);
+          cw[nt][kk] = ld16(cs + 32 * kk);
+          sw[nt][kk] = ld16(cs + HD + 32 * kk);
         }
       }
+    }
+  }
+  auto norm_and_rotate = [&] {
+#pragma unroll
+    for (int nt = 0; nt < NQ; ++nt) {
+      const bool valid = (((16 * nt + m16) * g_magic) >> 16) < nq;
       float x[KS][8];
 #pragma unroll
       for (int kk = 0; kk < KS; ++kk) {
@@ -164,9 +174,7 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
         const float rstd = rsqrtf(ss * (1.f / HD) + p.eps);
 #pragma unroll
         for (int kk = 0; kk < KS; ++kk) {
-          const uint4 w = p.norm == MI_NORM_RMS && p.q_w ? ld16(p.q_w + 32 * kk + 8 * g)
-                                                         : make_uint4(ones2<F16>(), ones2<F16>(), ones2<F16>(), ones2<F16>());
-          const uint32_t w4[4] = {w.x, w.y, w.z, w.w};
+          const uint32_t w4[4] = {qw[kk].x, qw[kk].y, qw[kk].z, qw[kk].w};
 #pragma unroll
           for (int j = 0; j < 8; j += 2) {
             const uint32_t packed = pack2<F16>(x[kk][j] * rstd * lo_to_f32<F16>(w4[j >> 1]),
@@ -176,26 +184,36 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
           }
         }
       }
+      auto rotated = [&](auto Ic) {
+        constexpr bool INTERLEAVED = decltype(Ic)::value;
 #pragma unroll
-      for (int kk = 0; kk < KS; ++kk) {
-        const uint32_t c4[4] = {cw[kk].x, cw[kk].y, cw[kk].z, cw[kk].w}, s4[4] = {sw[kk].x, sw[kk].y, sw[kk].z, sw[kk].w};
-        uint32_t o4[4];
+        for (int kk = 0; kk < KS; ++kk) {
+          const uint32_t c4[4] = {cw[nt][kk].x, cw[nt][kk].y, cw[nt][kk].z, cw[nt][kk].w};
+          const uint32_t s4[4] = {sw[nt][kk].x, sw[nt][kk].y, sw[nt][kk].z, sw[nt][kk].w};
+          uint32_t o4[4];
 #pragma unroll
-        for (int j = 0; j < 8; j += 2) {
-          float o0 = x[kk][j], o1 = x[kk][j + 1];
-          if (p.angles) {
-            const float y0 = p.interleaved ? x[kk][j + 1] : x[kk ^ (KS / 2)][j], y1 = p.interleaved ? x[kk][j] : x[kk ^ (KS / 2)][j + 1];
-            const uint32_t a = pack2<F16>(o0 * lo_to_f32<F16>(c4[j >> 1]), o1 * hi_to_f32<F16>(c4[j >> 1]));
+          for (int j = 0; j < 8; j += 2) {
+            const float y0 = INTERLEAVED ? x[kk][j + 1] : x[kk ^ (KS / 2)][j], y1 = INTERLEAVED ? x[kk][j] : x[kk ^ (KS / 2)][j + 1];
+            const uint32_t a = pack2<F16>(x[kk][j] * lo_to_f32<F16>(c4[j >> 1]), x[kk][j + 1] * hi_to_f32<F16>(c4[j >> 1]));
             const uint32_t b = pack2<F16>(y0 * lo_to_f32<F16>(s4[j >> 1]), y1 * hi_to_f32<F16>(s4[j >> 1]));
-            o0 = lo_to_f32<F16>(a) + lo_to_f32<F16>(b);
-            o1 = hi_to_f32<F16>(a) + hi_to_f32<F16>(b);
+            o4[j >> 1] = pack2<F16>(lo_to_f32<F16>(a) + lo_to_f32<F16>(b), hi_to_f32<F16>(a) + hi_to_f32<F16>(b));
           }
-          o4[j >> 1] = pack2<F16>(o0, o1);
+          qf[nt][kk] = valid ? make_uint4(o4[0], o4[1], o4[2], o4[3]) : make_uint4(0, 0, 0, 0);
         }
-        qf[nt][kk] = valid ? make_uint4(o4[0], o4[1], o4[2], o4[3]) : make_uint4(0, 0, 0, 0);
+      };
+      if (!p.angles) {
+#pragma unroll
+        for (int kk = 0; kk < KS; ++kk)
+          qf[nt][kk] = valid ? make_uint4(pack2<F16>(x[kk][0], x[kk][1]), pack2<F16>(x[kk][2], x[kk][3]),
+                                          pack2<F16>(x[kk][4], x[kk][5]), pack2<F16>(x[kk][6], x[kk][7]))
+                             : make_uint4(0, 0, 0, 0);
+      } else if (p.interleaved) {
+        rotated(std::true_type{});
+      } else {
+        rotated(std::false_type{});
       }
     }
-  }
+  };
 
   float m_run[NQ], neg_run[NQ], mwin[NQ];
   f32x4_t acc[NQ][DV], accl[NQ];
@@ -534,12 +552,26 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
 #pragma unroll
       for (int kk = 0; kk < KS; ++kk)
         asm volatile("" ::"v"(qf[nt][kk].x), "v"(qf[nt][kk].y), "v"(qf[nt][kk].z), "v"(qf[nt][kk].w));
+    if (raw) {
+#pragma unroll
+      for (int kk = 0; kk < KS; ++kk) {
+        asm volatile("" ::"v"(qw[kk].x), "v"(qw[kk].y), "v"(qw[kk].z), "v"(qw[kk].w));
+#pragma unroll
+        for (int nt = 0; nt < NQ; ++nt) {
+          asm volatile("" ::"v"(cw[nt][kk].x), "v"(cw[nt][kk].y), "v"(cw[nt][kk].z), "v"(cw[nt][kk].w));
+          asm volatile("" ::"v"(sw[nt][kk].x), "v"(sw[nt][kk].y), "v"(sw[nt][kk].z), "v"(sw[nt][kk].w));
+        }
+      }
+    }
     __syncthreads();
     int64_t off_prev;
     uint32_t nrec_prev;
     if constexpr (FP8) {
       static_assert(!FP8 || DEPTH == 1, "fp8 tiles wait in one set of registers");
       fetch_fp8(p.kc, off_first[0], nrec_first[0], kraw);
+      MI_SB();
+      if (raw) norm_and_rotate();
+      MI_SB();
 #pragma unroll
       for (int i = 0; i < NP8; ++i) store_k_fp8(&Ks[0][0], i);
       fetch_fp8(p.kc, off_first[1], nrec_first[1], kraw);  // stored by iteration 0
@@ -561,6 +593,11 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
       }
       off_prev = off_first[DEPTH];
       nrec_prev = nrec_first[DEPTH];
+    }
+    if constexpr (!FP8) {
+      MI_SB();
+      if (raw) norm_and_rotate();
+      MI_SB();
     }
     // key tile 0 has landed (this wavefront's share): only the DEPTH pairs issued after it may still be on their way
     if constexpr (!FP8) {
