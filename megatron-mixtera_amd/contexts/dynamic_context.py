@@ -300,7 +300,8 @@ class DynamicInferenceContext:
             self._finished_ids_buf = torch.zeros(self.max_requests, dtype=torch.int32, device=dev)
             # The new counters of update_requests, and the largest query / kv length of a prefill or mixed step (only
             # waited for when somebody reads it), are written by their kernels straight into pinned host memory, where
-            # the host watches one word of each: no copy to enqueue, no wait for the whole stream
+            # the host watches one word of each: no copy to enqueue, no wait for the whole stream.  (A launch tells
+            # torch's host allocator, so that a context dropped with one still queued does not hand its words on.)
             watched = torch.zeros(64, dtype=torch.int32, pin_memory=True)  # (a line of 128 bytes for each)
             self._counters = watched[:8]
             self._counters_host = self._counters.numpy()

@@ -15,6 +15,8 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/core/CachingHostAllocator.h>
+#include <c10/core/impl/VirtualGuardImpl.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <chrono>
@@ -1028,6 +1030,19 @@ PyObject* watch(PyObject* const* a) {
   return PyBool_FromLong(changed);
 }
 
+// written_by_kernel(row, device index): a kernel about to go onto the device's current stream stores into `row`, pinned
+// host memory of torch's allocator.  The allocator sees the copies it is told of, not a kernel's stores: noted here, the
+// memory of a dropped `row` is handed out again only once the stream has got past this point.
+PyObject* written_by_kernel(PyObject* const* a) {
+  const Tensor& t = tensor(a[0], "row");
+  const c10::Device device(c10::kCUDA, (c10::DeviceIndex)as_int(a[1]));
+  REQUIRE(t.device().is_cpu(), "written_by_kernel takes a row in host memory");
+  const c10::Stream stream = c10::impl::VirtualGuardImpl(c10::kCUDA).getStream(device);
+  REQUIRE(at::getHostAllocator(c10::kCUDA)->record_event(t.data_ptr(), t.storage().data_ptr().get_context(), stream),
+          "written_by_kernel takes a row in torch's pinned memory");
+  Py_RETURN_NONE;
+}
+
 // setup(kernel_error_class, raw_stream(device index), grow(device index, stream, bytes))
 PyObject* setup(PyObject* const* a) {
   for (int i = 0; i < 3; ++i) Py_INCREF(a[i]);
@@ -1056,7 +1071,7 @@ PyMethodDef kMethods[] = {
     OP(paged_prefill_attention, 14), OP(paged_prefill_attention_mla, 11), OP(norm_rope_append, 22), OP(qkv_norm_rope_append, 22), OP(qkv_key_append, 16),
     OP(qkv_prefill_attention, 18), OP(decode_step_attention, 29),
     OP(linear_decode, 5), OP(attention_layer_decode, 24), OP(sample_from_logits, 12), OP(selected_log_probs, 2), OP(last_token_gather, 3), OP(setup, 3),
-    OP(set_workspace, 3), OP(watch, 4), {nullptr, nullptr, 0, nullptr}};
+    OP(set_workspace, 3), OP(watch, 4), OP(written_by_kernel, 2), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_native", "Host side of the per-layer calls.", -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

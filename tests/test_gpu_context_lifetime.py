@@ -1,0 +1,48 @@
+"""GPU: the pinned words of a context -- written by kernels, watched by the host -- when the context is dropped with a
+step still queued."""
+import weakref
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def make_context(mi, dev):
+    ctx = mi.DynamicInferenceContext(
+        params_dtype=torch.bfloat16, num_layers=1, kv_channels=64, num_attention_heads=2, max_sequence_length=512,
+        buffer_size_gb=0.01, buffer_guaranteed_fraction=0.0, max_requests_override=8, max_tokens_override=1024, device=dev)
+    for i, n in enumerate((5, 300, 77)):
+        ctx.add_request(i, torch.arange(n, device=dev), 20)
+    return ctx
+
+
+def keep_busy(dev, products=200):
+    """Some 100 ms of work on the current stream (products of 1.1 TFLOP)."""
+    a = torch.zeros(8192, 8192, dtype=torch.bfloat16, device=dev)
+    for _ in range(products):
+        torch.mm(a, a)
+
+
+def test_words_of_a_dropped_context_are_not_handed_on(mi, dev):
+    pinned = lambda: [torch.full((64,), 12345, dtype=torch.int32).pin_memory() for _ in range(4)]  # the words' block size
+    ctx, other, spare = make_context(mi, dev), make_context(mi, dev), pinned()
+    keep_busy(dev, 1)
+    torch.cuda.synchronize()
+    del other, spare                   # (what follows finds memory of every kind in the caches: an allocation may wait)
+    keep_busy(dev)
+    done = torch.cuda.Event()
+    ctx.initialize_attention_state()   # its kernel waits behind the products
+    done.record()
+    words = ctx._counters.data_ptr()   # (the block's first; the maxima lie in it too)
+    gone = weakref.ref(ctx)
+    del ctx
+    assert gone() is None
+    rows = pinned()
+    later = make_context(mi, dev)
+    assert not done.query(), "the products ended too early to show anything"
+    assert words not in [later._counters.data_ptr(), *(r.data_ptr() for r in rows)]
+    later.initialize_attention_state()
+    assert (later.max_seqlen_q, later.max_seqlen_k) == (300, 300)
+    torch.cuda.synchronize()
+    assert all((r == 12345).all() for r in rows)
