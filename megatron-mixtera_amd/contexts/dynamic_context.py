@@ -308,7 +308,8 @@ class DynamicInferenceContext:
             self._max_lengths = watched[32:34]
             self._max_lengths_host = self._max_lengths.numpy()
         self._max_lengths_pending = False     # nobody has read the step's maxima yet
-        self._max_lengths_in_flight = False   # their kernel may not have run yet
+        self._max_lengths_in_flight = False   # their kernel, launched on _max_lengths_stream, may not have run yet
+        self._max_lengths_stream = None
         # what the host knows without asking the device: the longest prompt admitted since the last
         # update_requests (every other active request has one query token) and a bound on the kv lengths
         self._host_max_query_len = 1
@@ -376,14 +377,17 @@ class DynamicInferenceContext:
     def _land_max_lengths(self) -> None:
         """Wait for the maxima of the last prefill / mixed step, if their kernel may still be on its way."""
         if self._max_lengths_in_flight:
-            self._await(self._max_lengths, 0)
-            self._await(self._max_lengths, 1)
+            self._await(self._max_lengths, 0, self._max_lengths_stream)
+            self._await(self._max_lengths, 1, self._max_lengths_stream)
             self._max_lengths_in_flight = False
 
-    def _await(self, row: Tensor, index: int) -> None:
-        """Wait until a kernel on the current stream has replaced the -1 in ``row[index]`` (pinned host memory)."""
-        if not ops.watch(row, index, -1, 20000):
-            torch.cuda.current_stream(self.device).synchronize()
+    def _await(self, row: Tensor, index: int, stream) -> None:
+        """Wait until a kernel launched on ``stream`` has replaced the -1 in ``row[index]`` (pinned host memory).
+        ``stream`` is the launch's, which need not be the reader's; it is asked now and then whether it has run dry, so
+        that a launch which never stores its word ends in an error."""
+        while not ops.watch(row, index, -1, 20000):
+            if stream.query() and not ops.watch(row, index, -1, 0):
+                raise RuntimeError("a bookkeeping kernel has ended without its results")
 
     @property
     def max_seqlen_q(self):
@@ -798,6 +802,7 @@ class DynamicInferenceContext:
             self._land_max_lengths()  # (an earlier step's must not arrive after the reset of the words)
             self._max_lengths_host[:] = -1
             ops.step_attention_state(self, n_active_req, R, padded)
+            self._max_lengths_stream = torch.cuda.current_stream(self.device)
             self._max_lengths_in_flight = True
             self.kv_seq_lengths = self.kv_seq_lengths_cudagraph_only[:R]
             self.block_table = self.request_to_kv_chunk_ids_cudagraph_only[:R]
@@ -1109,8 +1114,7 @@ class DynamicInferenceContext:
                 self._paused_tokens_buf[: self.paused_request_count] = self.paused_tokens[: self.paused_request_count]
         self._counters_host[5] = -1
         ops.update_requests(self, mask, tokens)
-        self._await(self._counters, 5)
-        self._max_lengths_in_flight = False   # (the stream is in order)
+        self._await(self._counters, 5, torch.cuda.current_stream(dev))
         total, paused, active, avail, n_newly, status, was_reset, n_finished = self._counters_host.tolist()
         assert status != 1, "active + finished + paused requests != total_request_count"
         self.last_finished_request_ids = self._finished_ids_buf[:n_finished].clone()

@@ -1,5 +1,5 @@
 """GPU: the pinned words of a context -- written by kernels, watched by the host -- when the context is dropped with a
-step still queued."""
+step still queued, and when they are read under another stream than the step's."""
 import weakref
 
 import pytest
@@ -46,3 +46,28 @@ def test_words_of_a_dropped_context_are_not_handed_on(mi, dev):
     assert (later.max_seqlen_q, later.max_seqlen_k) == (300, 300)
     torch.cuda.synchronize()
     assert all((r == 12345).all() for r in rows)
+
+
+def test_maxima_are_awaited_on_the_stream_that_makes_them(mi, dev):
+    """Longer than the host watches a word without asking the stream (20 ms)."""
+    ctx = make_context(mi, dev)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        keep_busy(dev)
+        ctx.initialize_attention_state()
+        done = torch.cuda.Event()
+        done.record()
+    assert not done.query(), "the products ended too early to show anything"
+    assert (ctx.max_seqlen_q, ctx.max_seqlen_k) == (300, 300)
+    torch.cuda.current_stream().wait_stream(side)
+    ctx.update_requests(torch.ones(3, dtype=torch.uint8, device=dev), torch.zeros(3, dtype=torch.long, device=dev))
+    ctx.initialize_attention_state()
+    assert ctx.max_seqlen_q == 1 and ctx.active_token_count == 3
+
+
+def test_a_word_that_never_comes_is_an_error(mi, dev):
+    ctx = make_context(mi, dev)
+    ctx._counters_host[5] = -1
+    with pytest.raises(RuntimeError, match="without its results"):
+        ctx._await(ctx._counters, 5, torch.cuda.current_stream())
