@@ -193,6 +193,11 @@ Scratch scratch(const Tensor& ref, void* stream, int64_t need, PyObject* given, 
   return {it->second.data_ptr(), (int64_t)it->second.numel()};
 }
 
+// Whether a use_workspace buffer serves a call that can do without it.
+bool usable(const Tensor& w, const Tensor& ref, int64_t need, uintptr_t align) {
+  return w.device() == ref.device() && w.numel() >= need && (reinterpret_cast<uintptr_t>(w.data_ptr()) & (align - 1)) == 0;
+}
+
 // ------------------------------------------------------------------------------------------ shared checks
 bool is_16bit(const Tensor& t) { return t.scalar_type() == at::kBFloat16 || t.scalar_type() == at::kHalf; }
 int dtype_code(const Tensor& t) { return t.scalar_type() == at::kHalf ? MI_DTYPE_FP16 : MI_DTYPE_BF16; }
@@ -867,7 +872,11 @@ PyObject* linear_decode(PyObject* const* a) {
   }
   REQUIRE(!bias || (bias->numel() == N && bias->is_contiguous()), "bias must be a contiguous [N] vector");
   void* stream = stream_of(x);
-  const Scratch ws = scratch(x, stream, mi_linear_decode_workspace_bytes((int)T, (int)N, (int)K), Py_None, a[4]);
+  const int64_t need = mi_linear_decode_workspace_bytes((int)T, (int)N, (int)K);
+  Tensor own;  // (the scratch is for results over an input; a use_workspace buffer sized for attention may lack the room)
+  const bool fits = a[4] == Py_None || usable(tensor(a[4], "workspace"), x, need, 16);
+  if (!fits) own = at::empty({need}, x.options().dtype(at::kByte));
+  const Scratch ws = fits ? scratch(x, stream, need, Py_None, a[4]) : Scratch{own.data_ptr(), need};
   check(mi_linear_decode(x2.data_ptr(), st, w.data_ptr(), w.stride(0), ptr(bias), out.data_ptr(), o_st, ws.ptr, ws.bytes, (int)T,
                          (int)N, (int)K, dtype_code(x, "x"), stream),
         "mi_linear_decode");

@@ -178,9 +178,29 @@ __global__ __launch_bounds__(64 * NW) void linear_decode_kernel(LinearParams p) 
   }
 }
 
+// `out` over one of the inputs: workgroups store their rows while others still load, so the results go to the workspace
+// and this launch puts them in place.
+__global__ __launch_bounds__(256) void linear_place_kernel(const uint16_t* from, uint16_t* out, int64_t o_st, int T, int N) {
+  const int quads = N / 4, i = blockIdx.x * 256 + threadIdx.x;   // (T N / 4 fits: T <= 256)
+  if (i >= T * quads) return;
+  const int t = i / quads, n = 4 * (i - t * quads);
+  st8(out + t * o_st + n, ld8(from + (int64_t)t * N + n));
+}
+
 }  // namespace mi
 
 using namespace mi;
+
+// Whether `rows_a` rows of `width_a` values every `st_a` and the same of b share memory.  Columns of one buffer's rows
+// (equal strides) that lie side by side do not; other layouts are taken by their first and last value.
+static bool linear_overlap(const void* a, int64_t rows_a, int64_t width_a, int64_t st_a, const void* b, int64_t rows_b,
+                           int64_t width_b, int64_t st_b) {
+  const intptr_t a0 = (intptr_t)a / 2, b0 = (intptr_t)b / 2;
+  if (a0 + (rows_a - 1) * st_a + width_a <= b0 || b0 + (rows_b - 1) * st_b + width_b <= a0) return false;
+  if (st_a != st_b || rows_a == 1 || rows_b == 1) return true;
+  const intptr_t at = ((b0 - a0) % st_a + st_a) % st_a;   // b's first column, counted from a's
+  return at < width_a || at + width_b > st_a;
+}
 
 // The slices of K, and with them the order of summation: at least one per 512 columns, more where 128-row blocks of W
 // times 64-token blocks are few (a slice keeps at least 128 columns), a multiple of 32 columns each.
@@ -288,12 +308,12 @@ static void launch_linear(const LinearParams& p, int rt, hipStream_t st) {
 #undef LIN
 }
 
-// No scratch is used; a K of two slices and more still asks for a workspace, as callers of this entry point size one
-// and are told when they did not.
-static int64_t linear_workspace(int K) { return K >= 256 ? 256 : 0; }
+// Room for the results, written only where `out` lies over an input.  A K of 256 and more asks for it on every call, so
+// that a caller who sizes none is told at the first.
+static int64_t linear_workspace(int T, int N) { return ((int64_t)T * N * 2 + 255) & ~(int64_t)255; }
 
 extern "C" int64_t mi_linear_decode_workspace_bytes(int32_t T, int32_t N, int32_t K) {
-  return T <= 0 || N <= 0 || K <= 0 ? 0 : linear_workspace(K);
+  return T <= 0 || N <= 0 || K <= 0 ? 0 : linear_workspace(T, N);
 }
 
 extern "C" int mi_linear_decode(const void* x, int64_t x_stride_tok, const void* weight, int64_t w_stride_row,
@@ -315,10 +335,17 @@ extern "C" int mi_linear_decode(const void* x, int64_t x_stride_tok, const void*
   p.bias = (const uint16_t*)bias; p.out = (uint16_t*)out; p.o_st = out_stride_tok;
   p.T = T; p.N = N; p.K = K;
   hipStream_t st = (hipStream_t)stream;
-  if (const int64_t need = linear_workspace(K)) {
-    if (!workspace || workspace_bytes < need)
+  const bool staged = linear_overlap(out, T, N, out_stride_tok, x, T, K, x_stride_tok) ||
+                      linear_overlap(out, T, N, out_stride_tok, weight, N, K, w_stride_row) ||
+                      (bias && linear_overlap(out, T, N, out_stride_tok, bias, 1, N, N));
+  if (staged || K >= 256) {
+    if (!workspace || workspace_bytes < linear_workspace(T, N))
       return mi_fail(MI_ERR_WORKSPACE, "mi_linear_decode: workspace smaller than mi_linear_decode_workspace_bytes()");
     if ((uintptr_t)workspace & 15) return mi_fail(MI_ERR_ALIGN, "mi_linear_decode: the workspace must be 16-byte aligned");
+  }
+  if (staged) {
+    p.out = (uint16_t*)workspace;
+    p.o_st = N;
   }
   linear_slices(T, N, K, &p.S, &p.kslice);
   int rt;
@@ -329,6 +356,8 @@ extern "C" int mi_linear_decode(const void* x, int64_t x_stride_tok, const void*
   if (dtype == MI_DTYPE_FP16) launch_linear<true>(p, rt, st);
   else launch_linear<false>(p, rt, st);
   if (timed) (void)hipEventRecord(ev_b, st);
+  if (staged)
+    hipLaunchKernelGGL(linear_place_kernel, dim3((T * (N / 4) + 255) / 256), dim3(256), 0, st, p.out, (uint16_t*)out, out_stride_tok, T, N);
   return mi_check_launch("mi_linear_decode");
 }
 

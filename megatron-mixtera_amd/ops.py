@@ -590,6 +590,6 @@ def attention_layer_decode(hidden: Tensor, qkv_weight: Tensor, qkv_bias: Optiona
 def linear_decode(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None, out: Optional[Tensor] = None) -> Tensor:
     """``x @ weight.T (+ bias)`` for a decode-sized step (at most 256 rows of ``x``): the weight matrix streams from
     HBM once.  ``x`` is ``[..., K]`` (leading dimensions are flattened to rows), ``weight`` ``[N, K]``; the result
-    has ``x``'s leading dimensions and ``N`` columns.  What ``linear_qkv`` / ``linear_proj`` of the attention layer
+    has ``x``'s leading dimensions and ``N`` columns; ``out`` may lie over ``x``.  What ``linear_qkv`` / ``linear_proj`` of the attention layer
     compute at tensor-parallel size 1 (``mi_linear_decode`` of the header)."""
     return _native().linear_decode(x, weight, bias, out, _override())

@@ -76,6 +76,29 @@ def test_strided_inputs_and_leading_dimensions(mi, dev):
     assert (out[..., 256:] == 7.0).all(), "columns beyond N were touched"
 
 
+@pytest.mark.parametrize("T,N,K", [(64, 2048, 2048), (200, 512, 512), (5, 128, 128), (33, 16, 1024)])
+@pytest.mark.parametrize("place", ["x", "rows before", "part of x", "beside x", "w", "bias"])
+def test_results_over_an_input(mi, dev, T, N, K, place):
+    """Bit for bit what a call with a result of its own gives, also where rows are stored that others still read."""
+    gen = torch.Generator().manual_seed(T + N)
+    buf = torch.randn(T + 8, 2 * K, generator=gen).bfloat16().to(dev)
+    x = buf[8:, :K]
+    w = (torch.randn(max(N, T), K, generator=gen) * 0.05).bfloat16().to(dev)
+    bias = torch.randn(T * N, generator=gen).bfloat16().to(dev)
+    out = {"x": buf[8:, :N], "rows before": buf[:T, :N], "part of x": buf[8:, K - 8:K - 8 + N], "beside x": buf[8:, K:K + N],
+           "w": w.view(-1)[:T * N].view(T, N), "bias": bias.view(T, N)}[place]
+    want = mi.ops.linear_decode(x.clone(), w[:N].clone(), bias[:N].clone())
+    rest = buf.clone()
+    got = mi.ops.linear_decode(x, w[:N], bias[:N], out=out)
+    assert got is out and torch.equal(out, want)
+    if place == "beside x":
+        assert torch.equal(buf[:, :K], rest[:, :K])
+    with mi.ops.use_workspace(torch.empty(256, dtype=torch.uint8, device=dev)):   # (too small to hold the results)
+        buf.copy_(rest)
+        if place in ("x", "rows before", "part of x", "beside x"):
+            assert torch.equal(mi.ops.linear_decode(x, w[:N], bias[:N], out=out), want)
+
+
 def test_rejections(mi, dev):
     x = torch.zeros(300, 64, dtype=torch.bfloat16, device=dev)
     w = torch.zeros(32, 64, dtype=torch.bfloat16, device=dev)
