@@ -316,6 +316,7 @@ PyObject* kv_append(PyObject* const* a) {
     if (size.size() != 3 && size.size() != 4) fail_named(name, "must be [T, Hkv, d]");
     const size_t k = size.size() - 2;
     r.n = size[0]; r.h = size[k]; r.d = size[k + 1]; r.sn = stride[0]; r.sh = stride[k];
+    if (r.h == 1) r.sh = r.d;   // (the stride of a dimension of one says nothing: slices and transposes leave any)
     if (stride[k + 1] != 1 || r.sh != r.d) fail_named(name, "rows must be contiguous");
     return r;
   };

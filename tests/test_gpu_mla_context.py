@@ -79,3 +79,29 @@ def test_mla_context_mixed_then_decode_steps(mi, dev):
         assert ctx.total_request_count == 5
     finally:
         Ctx.TOKEN_ROUNDER, Ctx.REQUEST_ROUNDER = saved
+
+
+@pytest.mark.parametrize("layout", ["wider rows", "transposed", "two dimensions", "heads of one"])
+def test_latent_append_takes_any_layout_of_whole_rows(mi, dev, layout):
+    """The stride of a dimension of one is whatever the slice or transpose left there."""
+    ctx = mi.DynamicInferenceContext(
+        params_dtype=torch.bfloat16, num_layers=1, kv_channels=128, num_attention_heads=H, max_sequence_length=256,
+        buffer_size_gb=40 * (2 * C * (RANK + ROPE)) / 1024**3, buffer_guaranteed_fraction=0.1, chunk_size_tokens=C,
+        max_requests_override=16, max_tokens_override=512, cache_mla_latent=True, kv_lora_rank=RANK,
+        qk_pos_emb_head_dim=ROPE, device=dev)
+    ctx.add_request(0, torch.arange(70, device=dev), num_tokens_to_generate=20)
+    ctx.initialize_attention_state()
+    n, W = ctx.padded_active_token_count, RANK + ROPE
+    want = torch.randn(n, W, generator=torch.Generator().manual_seed(3)).bfloat16().to(dev)
+    if layout == "wider rows":
+        key = torch.zeros(n, 1, 640, dtype=torch.bfloat16, device=dev)[..., :W]
+    elif layout == "transposed":
+        key = torch.zeros(1, n, W, dtype=torch.bfloat16, device=dev).transpose(0, 1)
+    elif layout == "two dimensions":
+        key = torch.zeros(n, 640, dtype=torch.bfloat16, device=dev)[:, :W]
+    else:
+        key = torch.zeros(n, 1, W, dtype=torch.bfloat16, device=dev).as_strided((n, 1, W), (W, 8, 1))
+    key.view(n, W).copy_(want)
+    ctx.append_key_value_cache(1, key, None)
+    ids, loc = ctx.token_to_chunk_idx[:70], ctx.token_to_local_position_within_kv_chunk[:70]
+    assert torch.equal(ctx.memory_buffer[0][ids, loc], want[:70])
