@@ -938,10 +938,11 @@ PyObject* sample_from_logits(PyObject* const* a) {
   const bool want_cut = as_bool(a[10]);
   if (want_cut) cut = at::empty({R}, logits.options().dtype(at::kFloat));
   const float top_p = (float)as_float(a[2]);
-  // (a use_workspace buffer that is too small for the parts leaves the rows to one workgroup each)
+  // (sampling needs no workspace: a use_workspace buffer that does not serve the parts -- too small, on another device, off
+  // a 256-byte line -- leaves the rows to one workgroup each)
   const int64_t need = mi_sample_workspace_bytes((int)R, (int)V, (int)top_k, top_p);
   Scratch ws;
-  if (a[11] == Py_None || tensor(a[11], "workspace").numel() >= need) ws = scratch(logits, stream, need, Py_None, a[11]);
+  if (a[11] == Py_None || usable(tensor(a[11], "workspace"), logits, need, 256)) ws = scratch(logits, stream, need, Py_None, a[11]);
   check(mi_sample_from_logits_ws(logits.data_ptr(), logits.stride(0), code, (int)R, (int)V, (int)top_k, top_p,
                               (float)as_float(a[3]), (const float*)ptr(uniform), (int)as_int(a[5]), (int64_t*)samples.data_ptr(),
                               want_cut ? (float*)cut.data_ptr() : nullptr, (const int32_t*)ptr(lens[0]), (const int32_t*)ptr(lens[1]),

@@ -438,3 +438,18 @@ def test_rows_in_parts_equal_rows_by_one_workgroup(mi, dev, R, V, kind):
             torch.cuda.synchronize()
             assert torch.equal(got, want), (dtype, top_k, top_p)
             assert torch.equal(cut, want_cut), (dtype, top_k, top_p)
+
+
+@pytest.mark.parametrize("buffer", ["whole", "off a line", "too small", "on the host", "empty"])
+def test_sampling_inside_use_workspace(mi, dev, buffer):
+    """A buffer for attention's scratch that does not serve the parts of the rows is passed over, not refused."""
+    gen = torch.Generator().manual_seed(11)
+    logits = torch.randn(8, 65536, generator=gen).to(dev)
+    u = torch.rand(8, generator=gen).to(dev)
+    want, _ = mi.ops.sample_from_logits(logits, top_p=0.9, uniform=u)
+    big = torch.empty(64 << 20, dtype=torch.uint8, device=dev)
+    given = {"whole": big, "off a line": big[16:], "too small": big[:4096], "empty": big[:0],
+             "on the host": torch.empty(64 << 20, dtype=torch.uint8)}[buffer]
+    with mi.ops.use_workspace(given):
+        got, _ = mi.ops.sample_from_logits(logits, top_p=0.9, uniform=u)
+    assert torch.equal(got, want)
