@@ -14,6 +14,7 @@ import torch
 from torch import Tensor
 
 from . import ops
+from .contexts.dynamic_context import DynamicInferenceContext
 from .flash_attn_interface import (
     flash_attn_varlen_func,
     flash_attn_with_kvcache,
@@ -74,10 +75,20 @@ def _parameter(module: torch.nn.Module, name: str) -> Optional[Tensor]:
     return p if p is not None else getattr(module, name)
 
 
-def _untouched(module: torch.nn.Module, cls: type) -> bool:
-    """Whether calling ``module`` would run ``cls.forward`` and nothing else (no hooks, no subclass, no replaced
-    forward), so that its work may be folded into another call."""
-    return (type(module) is cls and "forward" not in module.__dict__
+def _own(obj, cls: type, *names: str) -> bool:
+    """Whether the methods ``names`` of ``obj`` are those that ``cls`` was defined with -- none overridden in a subclass,
+    replaced on the class or on the object -- so that a call which does their work may stand in for them."""
+    kind, here, methods = type(obj), obj.__dict__, _DEFINED[cls]
+    for name in names:
+        if name in here or getattr(kind, name) is not methods[name]:
+            return False
+    return True
+
+
+def _untouched(module: torch.nn.Module, cls: type, *names: str) -> bool:
+    """Whether calling ``module`` (or its methods ``names``) would run what ``cls`` defines and nothing else: no hooks, no
+    subclass, nothing replaced."""
+    return (type(module) is cls and _own(module, cls, "forward", *names)
             and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
             and not torch.nn.modules.module._has_any_global_hook())
 
@@ -132,8 +143,10 @@ class PagedSelfAttentionCore(torch.nn.Module):
                 self.layer_number, mixed_qkv=mixed_qkv, num_query_heads=num_query_heads, rotary_pos_emb=emb,
                 softmax_scale=self.softmax_scale, **self._norm_args())
             return out.reshape(out.size(0), out.size(1), -1)
-        fusable = getattr(ctx, "prefill_fusable", None)
-        if self.fused and fusable is not None and fusable(mixed_qkv, self.head_dim, emb):
+        # (a step of prompts in one call of the context: in place of its append and of _attend below)
+        if (self.fused and isinstance(ctx, DynamicInferenceContext) and _own(self, PagedSelfAttentionCore, "_attend")
+                and _own(ctx, DynamicInferenceContext, "fused_qkv_norm_rope_append")
+                and ctx.prefill_fusable(mixed_qkv, self.head_dim, emb)):
             out = ctx.fused_prefill_attention(
                 self.layer_number, mixed_qkv, num_query_heads=num_query_heads, rotary_pos_emb=emb,
                 softmax_scale=self.softmax_scale, **self._norm_args())
@@ -189,7 +202,7 @@ class PagedSelfAttentionCore(torch.nn.Module):
             # maxima (cu_query_lengths / cu_kv_lengths, as the reference does) would wait for the device
             cu_q, cu_k, kv_lens = ctx.cu_query_seq_lengths, ctx.cu_kv_seq_lengths, ctx.kv_seq_lengths
             max_q, max_k = ctx.attention_length_bounds()
-            one_row = ctx.one_row_requests_possible()
+            one_row = ctx.one_row_requests_possible() if hasattr(ctx, "one_row_requests_possible") else True
         else:
             one_row = True
             cu_q, max_q = ctx.cu_query_lengths()
@@ -264,19 +277,30 @@ class PagedSelfAttentionLayer(torch.nn.Module):
 
     def _decode_in_one_call(self, hidden_states: Tensor, ctx, rotary_pos_emb) -> Optional[Tensor]:
         """The output of a decode-only step by one native call, or ``None`` where the step takes the modules one by
-        one: other steps, a context without that call, hooks or replaced forwards on the parts."""
+        one: other steps, another kind of context, hooks on the parts, or a replaced method whose work the call does."""
         qkv, core, proj = self._modules["linear_qkv"], self._modules["core"], self._modules["linear_proj"]
-        call = getattr(ctx, "fused_decode_layer", None)
         n = hidden_states.size(0)
-        if (call is None or not core.fused or n > DecodeLinear.DECODE_ROWS or n != ctx.padded_active_token_count
-                or hidden_states.dim() != 3 or hidden_states.size(1) != 1
-                or not (_untouched(qkv, DecodeLinear) and _untouched(core, PagedSelfAttentionCore)
-                        and _untouched(proj, DecodeLinear))):
+        if (not (_untouched(qkv, DecodeLinear) and _untouched(proj, DecodeLinear)
+                 and _untouched(core, PagedSelfAttentionCore, "forward_mixed_qkv"))
+                or not isinstance(ctx, DynamicInferenceContext)
+                or not _own(ctx, DynamicInferenceContext, "fused_decode_step_attention")
+                or not core.fused or n > min(qkv.DECODE_ROWS, proj.DECODE_ROWS) or n != ctx.padded_active_token_count
+                or hidden_states.dim() != 3 or hidden_states.size(1) != 1):
             return None
         emb = core.rotary_table(rotary_pos_emb)
         if not core._step_fusable(ctx, emb):
             return None
-        return call(core.layer_number, hidden_states, _parameter(qkv, "weight"),
-                    None if qkv.skip_bias_add else _parameter(qkv, "bias"), _parameter(proj, "weight"),
-                    None if proj.skip_bias_add else _parameter(proj, "bias"), num_query_heads=self.num_query_heads,
-                    rotary_pos_emb=emb, softmax_scale=core.softmax_scale, **core._norm_args())
+        return ctx.fused_decode_layer(
+            core.layer_number, hidden_states, _parameter(qkv, "weight"),
+            None if qkv.skip_bias_add else _parameter(qkv, "bias"), _parameter(proj, "weight"),
+            None if proj.skip_bias_add else _parameter(proj, "bias"), num_query_heads=self.num_query_heads,
+            rotary_pos_emb=emb, softmax_scale=core.softmax_scale, **core._norm_args())
+
+
+# The methods above (and the context's) that a fused call stands in for, as defined: see _own.
+_DEFINED = {
+    DecodeLinear: {"forward": DecodeLinear.forward},
+    PagedSelfAttentionCore: {name: getattr(PagedSelfAttentionCore, name) for name in ("forward", "forward_mixed_qkv", "_attend")},
+    DynamicInferenceContext: {name: getattr(DynamicInferenceContext, name)
+                              for name in ("fused_decode_step_attention", "fused_qkv_norm_rope_append")},
+}

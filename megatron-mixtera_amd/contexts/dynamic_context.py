@@ -640,11 +640,11 @@ class DynamicInferenceContext:
         """A decode-only step of one attention layer from hidden states to hidden states ``[T, 1, hidden]``, T the
         padded token count: the QKV projection, :meth:`fused_decode_step_attention` on its output and the output
         projection in one call."""
-        k_cache, v_cache = self._layer_cache(layer_number)
+        k_cache, v_cache, block_table = self.key_value_cache(layer_number)
         k_scales, v_scales = self.key_value_scales(layer_number)
         return ops.attention_layer_decode(
             hidden, qkv_weight, qkv_bias, proj_weight, proj_bias, num_query_heads, self.num_kv_heads_per_partition, k_cache,
-            v_cache, self.kv_seq_lengths, self.block_table, q_weight=q_weight, k_weight=k_weight, eps=eps, norm=norm,
+            v_cache, self.kv_seq_lengths, block_table, q_weight=q_weight, k_weight=k_weight, eps=eps, norm=norm,
             rotary_emb=rotary_pos_emb, rotary_interleaved=self._rope_flags(config) if config is not None else False,
             softmax_scale=softmax_scale, max_kv_len=self.attention_length_bounds()[1], k_scales=k_scales,
             v_scales=v_scales, headroom=self.fp8_append_headroom)
@@ -708,7 +708,6 @@ class DynamicInferenceContext:
         one launch for keys and values, and the queries are normed and rotated where attention loads them."""
         n, hkv, d = self.padded_active_token_count, self.num_kv_heads_per_partition, self.kv_channels
         interleaved = self._rope_flags(config) if config is not None else False
-        k_cache, v_cache = self._layer_cache(layer_number)
         k_scales, v_scales = self.key_value_scales(layer_number)
         common = dict(num_query_heads=num_query_heads, num_kv_heads=hkv, eps=eps, norm=norm, rotary_interleaved=interleaved)
         keys = dict(k_weight=k_weight, rotary_emb=rotary_pos_emb, q_positions=self.token_to_pos_ids,
@@ -721,9 +720,11 @@ class DynamicInferenceContext:
             value = rows.reshape(n, hkv, (group + 2) * d)[:, :, (group + 1) * d:]
             self.append_key_value_cache(layer_number, key, value.unsqueeze(1))
         else:
+            k_cache, v_cache = self._layer_cache(layer_number)
             cos_sin = ops.qkv_key_append(rows, k_cache=k_cache, v_cache=v_cache, token_to_chunk_idx=self.token_to_chunk_idx,
                                          token_to_local_pos=self.token_to_local_position_within_kv_chunk, **keys)
-        out = ops.qkv_prefill_attention(rows, k_cache, v_cache, self.cu_query_seq_lengths, self.kv_seq_lengths, self.block_table,
+        k_cache, v_cache, block_table = self.key_value_cache(layer_number)
+        out = ops.qkv_prefill_attention(rows, k_cache, v_cache, self.cu_query_seq_lengths, self.kv_seq_lengths, block_table,
                                         cos_sin=cos_sin, q_weight=q_weight, softmax_scale=softmax_scale,
                                         max_kv_len=self.attention_length_bounds()[1], k_scales=k_scales, v_scales=v_scales, **common)
         if n == mixed_qkv.size(0):

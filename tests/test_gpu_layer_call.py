@@ -54,3 +54,64 @@ def test_mask_of_bytes(mi, dev):
         state.append([ctx.total_request_count, ctx.chunk_allocator.chunk_count_avail, ctx.last_finished_request_ids.tolist(),
                       ctx.request_ids.tolist(), ctx.request_to_kv_chunk_ids.tolist(), ctx.token_to_input_ids[:4].tolist()])
     assert state[0] == state[1] and state[0][0] == 3
+
+
+DECODE_PARTS = ["core.forward_mixed_qkv", "class core.forward_mixed_qkv", "linear_qkv.forward", "linear_proj.forward",
+                "ctx.fused_decode_step_attention", "class ctx.fused_decode_step_attention", "ctx.key_value_cache"]
+PROMPT_PARTS = ["core._attend", "class core._attend", "ctx.fused_qkv_norm_rope_append",
+                "class ctx.fused_qkv_norm_rope_append", "ctx.key_value_cache"]
+
+
+@pytest.mark.parametrize("step,part", [("decode", p) for p in DECODE_PARTS] + [("prompts", p) for p in PROMPT_PARTS])
+def test_replaced_parts_are_called(mi, dev, step, part, monkeypatch):
+    """A part replaced on the object, on its class or in a subclass runs in a step that is otherwise folded into fewer
+    calls, and the step's result is what it was."""
+    lens = [3, 256, 40]
+    owner, name = part.split()[-1].split(".")
+    outs, calls = [], []
+    for replaced in (False, True):
+        ctx = _context(mi, dev, lens, None)
+        if step == "decode":
+            ctx.update_requests(torch.ones(3, dtype=torch.uint8, device=dev), torch.zeros(3, dtype=torch.long, device=dev))
+            ctx.initialize_attention_state()
+        gen = torch.Generator(device=dev).manual_seed(2)
+        layer = mi.PagedSelfAttentionLayer(2, 512, 8, 2, 128, qk_norm="rms", device=dev).requires_grad_(False)
+        for p in layer.parameters():
+            p.normal_(0, 0.05, generator=gen)
+        if replaced:
+            target = ctx if owner == "ctx" else getattr(layer, owner)
+            if part.startswith("class"):
+                target = type(target)
+            before = getattr(target, name)
+            monkeypatch.setattr(target, name, lambda *a, **k: (calls.append(1), before(*a, **k))[1])
+        table = mi.synthetic.rotary_angle_table(1024, 128, base=10000.0).to(dev)
+        x = torch.empty(ctx.padded_active_token_count, 1, 512, dtype=torch.bfloat16, device=dev).normal_(generator=gen)
+        outs.append(layer(x, ctx, (table, table))[0][:ctx.active_token_count].float())
+    assert calls, "the replaced part was skipped"
+    # (another kernel may do the step then: a rounding of the 16-bit result apart, a few of them after the projection)
+    torch.testing.assert_close(outs[0], outs[1], rtol=2e-2, atol=2e-2)
+
+
+def test_a_subclass_of_the_context_keeps_its_overrides(mi, dev):
+    class Counting(mi.DynamicInferenceContext):
+        steps = appends = 0
+
+        def fused_decode_step_attention(self, *a, **k):
+            self.steps += 1
+            return super().fused_decode_step_attention(*a, **k)
+
+        def fused_qkv_norm_rope_append(self, *a, **k):
+            self.appends += 1
+            return super().fused_qkv_norm_rope_append(*a, **k)
+
+    ctx = Counting(params_dtype=torch.bfloat16, num_layers=1, kv_channels=128, num_attention_heads=2, max_sequence_length=1024,
+                   buffer_size_gb=0.02, buffer_guaranteed_fraction=0.0, max_requests_override=4, max_tokens_override=1024, device=dev)
+    layer = mi.PagedSelfAttentionLayer(1, 512, 8, 2, 128, device=dev).requires_grad_(False)
+    for p in layer.parameters():
+        p.zero_()
+    ctx.add_request(0, torch.arange(70, device=dev), 20)
+    for _ in range(2):
+        ctx.initialize_attention_state()
+        layer(torch.zeros(ctx.padded_active_token_count, 1, 512, dtype=torch.bfloat16, device=dev), ctx)
+        ctx.update_requests(torch.ones(1, dtype=torch.uint8, device=dev), torch.zeros(1, dtype=torch.long, device=dev))
+    assert (ctx.appends, ctx.steps) == (1, 1)
