@@ -145,7 +145,7 @@ class PagedSelfAttentionCore(torch.nn.Module):
             return out.reshape(out.size(0), out.size(1), -1)
         # (a step of prompts in one call of the context: in place of its append and of _attend below)
         if (self.fused and isinstance(ctx, DynamicInferenceContext) and _own(self, PagedSelfAttentionCore, "_attend")
-                and _own(ctx, DynamicInferenceContext, "fused_qkv_norm_rope_append")
+                and _own(ctx, DynamicInferenceContext, "fused_qkv_norm_rope_append", "key_value_cache")
                 and ctx.prefill_fusable(mixed_qkv, self.head_dim, emb)):
             out = ctx.fused_prefill_attention(
                 self.layer_number, mixed_qkv, num_query_heads=num_query_heads, rotary_pos_emb=emb,
@@ -283,7 +283,7 @@ class PagedSelfAttentionLayer(torch.nn.Module):
         if (not (_untouched(qkv, DecodeLinear) and _untouched(proj, DecodeLinear)
                  and _untouched(core, PagedSelfAttentionCore, "forward_mixed_qkv"))
                 or not isinstance(ctx, DynamicInferenceContext)
-                or not _own(ctx, DynamicInferenceContext, "fused_decode_step_attention")
+                or not _own(ctx, DynamicInferenceContext, "fused_decode_step_attention", "key_value_cache")
                 or not core.fused or n > min(qkv.DECODE_ROWS, proj.DECODE_ROWS) or n != ctx.padded_active_token_count
                 or hidden_states.dim() != 3 or hidden_states.size(1) != 1):
             return None
@@ -302,5 +302,5 @@ _DEFINED = {
     DecodeLinear: {"forward": DecodeLinear.forward},
     PagedSelfAttentionCore: {name: getattr(PagedSelfAttentionCore, name) for name in ("forward", "forward_mixed_qkv", "_attend")},
     DynamicInferenceContext: {name: getattr(DynamicInferenceContext, name)
-                              for name in ("fused_decode_step_attention", "fused_qkv_norm_rope_append")},
+                              for name in ("fused_decode_step_attention", "fused_qkv_norm_rope_append", "key_value_cache")},
 }

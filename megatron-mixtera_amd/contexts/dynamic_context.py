@@ -444,8 +444,8 @@ class DynamicInferenceContext:
         return int(unfinished.sum().item())
 
     # ------------------------------------------------------------------ per-layer hot path
-    # The cache and its scales are properties so that the views every layer of every step asks for (two index calls of
-    # 2-3 us each) are made once per buffer; whoever assigns another buffer gets views of that one.
+    # Every layer of every step needs views of its cache (2-3 us for each index call), so this class keeps a set for its
+    # own calls; whoever assigns another buffer, or puts other memory under it, gets views of that.
     @property
     def memory_buffer(self) -> Tensor:
         return self._memory_buffer
@@ -453,26 +453,16 @@ class DynamicInferenceContext:
     @memory_buffer.setter
     def memory_buffer(self, buffer: Tensor) -> None:
         self._memory_buffer = buffer
-        self._cache_views = None
-
-    @property
-    def kv_scales(self) -> Optional[Tensor]:
-        return self._kv_scales
-
-    @kv_scales.setter
-    def kv_scales(self, scales: Optional[Tensor]) -> None:
-        self._kv_scales = scales
-        self._scale_views = None
+        self._kept_views = None
 
     def _layer_cache(self, layer_number: int) -> Tuple[Tensor, Optional[Tensor]]:
-        """Views of the layer's key and value cache (latent cache: its rows and ``None``)."""
-        views = self._cache_views
-        if views is None:
-            buf = self._memory_buffer
-            views = ([(latents, None) for latents in buf.unbind(0)] if self.cache_mla_latent
-                     else list(zip(buf[0].unbind(0), buf[1].unbind(0))))
-            self._cache_views = views
-        return views[layer_number - 1]
+        """The kept views of the layer's key and value cache (latent cache: its rows and ``None``).  Not to be handed
+        out: what a caller does to the objects (``unsqueeze_`` and the like) must not reach the next step."""
+        buf, kept = self._memory_buffer, self._kept_views
+        if kept is None or kept[0] != buf.data_ptr():
+            pair = not self.cache_mla_latent
+            kept = self._kept_views = (buf.data_ptr(), [ops.layer_views(buf, i, pair) for i in range(buf.size(int(pair)))])
+        return kept[1][layer_number - 1]
 
     def append_key_value_cache(self, layer_number: int, key: Tensor, value: Tensor) -> None:
         """Scatter this step's K/V rows into the layer's chunks (bit-exact copy).
@@ -502,16 +492,13 @@ class DynamicInferenceContext:
     def key_value_cache(self, layer_number: int) -> Tuple[Tensor, Tensor, Tensor]:
         """Views of the layer's key cache, value cache and this step's block table (latent cache: the
         layer's ``[chunks, tokens, rank + rope]`` buffer and ``None``)."""
-        return (*self._layer_cache(layer_number), self.block_table)
+        return (*ops.layer_views(self._memory_buffer, layer_number - 1, not self.cache_mla_latent), self.block_table)
 
     def key_value_scales(self, layer_number: int) -> Tuple[Optional[Tensor], Optional[Tensor]]:
         """fp8 cache: the layer's key and value scales ``[chunks, heads]``; otherwise ``(None, None)``."""
         if not self.kv_cache_fp8:
             return None, None
-        views = self._scale_views
-        if views is None:
-            views = self._scale_views = list(zip(self._kv_scales[0].unbind(0), self._kv_scales[1].unbind(0)))
-        return views[layer_number - 1]
+        return ops.layer_views(self.kv_scales, layer_number - 1, True)
 
     @staticmethod
     def _rope_flags(config) -> bool:
@@ -640,11 +627,11 @@ class DynamicInferenceContext:
         """A decode-only step of one attention layer from hidden states to hidden states ``[T, 1, hidden]``, T the
         padded token count: the QKV projection, :meth:`fused_decode_step_attention` on its output and the output
         projection in one call."""
-        k_cache, v_cache, block_table = self.key_value_cache(layer_number)
+        k_cache, v_cache = self._layer_cache(layer_number)
         k_scales, v_scales = self.key_value_scales(layer_number)
         return ops.attention_layer_decode(
             hidden, qkv_weight, qkv_bias, proj_weight, proj_bias, num_query_heads, self.num_kv_heads_per_partition, k_cache,
-            v_cache, self.kv_seq_lengths, block_table, q_weight=q_weight, k_weight=k_weight, eps=eps, norm=norm,
+            v_cache, self.kv_seq_lengths, self.block_table, q_weight=q_weight, k_weight=k_weight, eps=eps, norm=norm,
             rotary_emb=rotary_pos_emb, rotary_interleaved=self._rope_flags(config) if config is not None else False,
             softmax_scale=softmax_scale, max_kv_len=self.attention_length_bounds()[1], k_scales=k_scales,
             v_scales=v_scales, headroom=self.fp8_append_headroom)
@@ -708,6 +695,7 @@ class DynamicInferenceContext:
         one launch for keys and values, and the queries are normed and rotated where attention loads them."""
         n, hkv, d = self.padded_active_token_count, self.num_kv_heads_per_partition, self.kv_channels
         interleaved = self._rope_flags(config) if config is not None else False
+        k_cache, v_cache = self._layer_cache(layer_number)
         k_scales, v_scales = self.key_value_scales(layer_number)
         common = dict(num_query_heads=num_query_heads, num_kv_heads=hkv, eps=eps, norm=norm, rotary_interleaved=interleaved)
         keys = dict(k_weight=k_weight, rotary_emb=rotary_pos_emb, q_positions=self.token_to_pos_ids,
@@ -720,11 +708,9 @@ class DynamicInferenceContext:
             value = rows.reshape(n, hkv, (group + 2) * d)[:, :, (group + 1) * d:]
             self.append_key_value_cache(layer_number, key, value.unsqueeze(1))
         else:
-            k_cache, v_cache = self._layer_cache(layer_number)
             cos_sin = ops.qkv_key_append(rows, k_cache=k_cache, v_cache=v_cache, token_to_chunk_idx=self.token_to_chunk_idx,
                                          token_to_local_pos=self.token_to_local_position_within_kv_chunk, **keys)
-        k_cache, v_cache, block_table = self.key_value_cache(layer_number)
-        out = ops.qkv_prefill_attention(rows, k_cache, v_cache, self.cu_query_seq_lengths, self.kv_seq_lengths, block_table,
+        out = ops.qkv_prefill_attention(rows, k_cache, v_cache, self.cu_query_seq_lengths, self.kv_seq_lengths, self.block_table,
                                         cos_sin=cos_sin, q_weight=q_weight, softmax_scale=softmax_scale,
                                         max_kv_len=self.attention_length_bounds()[1], k_scales=k_scales, v_scales=v_scales, **common)
         if n == mixed_qkv.size(0):

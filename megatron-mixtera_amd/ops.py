@@ -463,6 +463,13 @@ def decode_step_attention(query: Optional[Tensor], key: Optional[Tensor], value:
         split_tokens, out, workspace, faithful_rounding, k_scales, v_scales, headroom, _tuning_arg(), _override())
 
 
+def layer_views(buffer: Tensor, layer: int, pair: bool) -> Tuple[Tensor, Optional[Tensor]]:
+    """New views ``buffer[0, layer], buffer[1, layer]`` of a buffer of keys and values, or ``buffer[layer], None``."""
+    if not buffer.is_cuda:   # (a context on the host works without the built library)
+        return (buffer[0, layer], buffer[1, layer]) if pair else (buffer[layer], None)
+    return _native().layer_views(buffer, layer, pair)
+
+
 def watch(row: Tensor, index: int, value: int, microseconds: int) -> bool:
     """Whether ``row[index]`` (int32 in pinned host memory, written by a kernel) became anything but ``value`` within
     the time; other Python threads run meanwhile."""

@@ -578,3 +578,28 @@ def test_synthetic_input_helpers_agree_with_the_checker(mi):
             oa.decode_attention_bytes(lens, 32, 8, 128, 256, kv_bytes=kvb, fp8_scales=sc)
     # by hand: one request of 3 tokens, 2/1 heads of 8 values, chunk 2 -> 2 chunks
     assert mi.synthetic.decode_attention_bytes([3], 2, 1, 8, 2) == 3 * 1 * 8 * 2 * 2 + 2 * 8 * 4 + 2 * 4 + 4
+
+
+@pytest.mark.parametrize("latent", [False, True], ids=["pairs", "latents"])
+def test_views_of_the_cache_are_the_callers_own(Ctx, latent):
+    ctx = Ctx(params_dtype=torch.bfloat16, num_layers=2, kv_channels=16, num_attention_heads=2, max_sequence_length=256,
+              buffer_size_gb=0.002, buffer_guaranteed_fraction=0.1, chunk_size_tokens=64, max_requests_override=4,
+              max_tokens_override=64, device="cpu", **(dict(cache_mla_latent=True, kv_lora_rank=32, qk_pos_emb_head_dim=16) if latent else {}))
+    shape = ctx.key_value_cache(2)[0].shape
+    for view in ctx.key_value_cache(2)[:2] + ctx._layer_cache(2):
+        assert view is None or view.shape == shape
+    k, v, _ = ctx.key_value_cache(2)
+    k.unsqueeze_(0)
+    if v is not None:
+        v.squeeze_().transpose_(0, 1)
+    again = ctx.key_value_cache(2)
+    assert again[0].shape == ctx._layer_cache(2)[0].shape == shape and again[0].data_ptr() == k.data_ptr()
+    # a write of something that requires grad, as into any view made by indexing
+    ctx.key_value_cache(1)[0].copy_(torch.ones(shape, dtype=torch.bfloat16, requires_grad=True))
+    # other memory under the same buffer, and another buffer
+    for swap in (lambda t: setattr(ctx.memory_buffer, "data", t), lambda t: setattr(ctx, "memory_buffer", t)):
+        new = torch.full_like(ctx.memory_buffer, 7.0, requires_grad=False).detach()
+        swap(new)
+        assert ctx._layer_cache(1)[0].data_ptr() == ctx.key_value_cache(1)[0].data_ptr() == new.data_ptr()
+    with pytest.raises(IndexError):
+        ctx.key_value_cache(3)

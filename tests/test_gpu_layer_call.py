@@ -115,3 +115,24 @@ def test_a_subclass_of_the_context_keeps_its_overrides(mi, dev):
         layer(torch.zeros(ctx.padded_active_token_count, 1, 512, dtype=torch.bfloat16, device=dev), ctx)
         ctx.update_requests(torch.ones(1, dtype=torch.uint8, device=dev), torch.zeros(1, dtype=torch.long, device=dev))
     assert (ctx.appends, ctx.steps) == (1, 1)
+
+
+@pytest.mark.parametrize("cache", [None, "fp8_e4m3"], ids=["16bit", "fp8"])
+def test_steps_do_not_see_what_callers_do_to_their_views(mi, dev, cache):
+    ctx = _context(mi, dev, [5, 300], cache)
+    for step in range(2):
+        k, v, _ = ctx.key_value_cache(1)
+        assert k.shape == v.shape == ctx.memory_buffer.shape[2:] and k.data_ptr() == ctx.memory_buffer.data_ptr()
+        row = torch.full((ctx.padded_active_token_count, 1, 2, 128), 1.0 + step, dtype=torch.bfloat16, device=dev)
+        ctx.append_key_value_cache(1, row, row)
+        chunk, at = int(ctx.token_to_chunk_idx[0]), int(ctx.token_to_local_position_within_kv_chunk[0])
+        scale = ctx.kv_scales[0, 0, chunk, 0] if cache else 1.0
+        stored = k[chunk, at, 0, 0].view(torch.float8_e4m3fn) if cache else k[chunk, at, 0, 0]
+        assert abs(float(stored) * float(scale) - (1.0 + step)) < 0.1
+        k.unsqueeze_(0)
+        v.transpose_(0, 1)
+        for s in ctx.key_value_scales(1):
+            if s is not None:
+                s.unsqueeze_(0)
+    with pytest.raises(IndexError):
+        ctx.key_value_cache(3)
