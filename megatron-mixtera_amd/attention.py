@@ -75,22 +75,20 @@ def _parameter(module: torch.nn.Module, name: str) -> Optional[Tensor]:
     return p if p is not None else getattr(module, name)
 
 
-def _own(obj, cls: type, *names: str) -> bool:
-    """Whether the methods ``names`` of ``obj`` are those that ``cls`` was defined with -- none overridden in a subclass,
-    replaced on the class or on the object -- so that a call which does their work may stand in for them."""
-    kind, here, methods = type(obj), obj.__dict__, _DEFINED[cls]
-    for name in names:
-        if name in here or getattr(kind, name) is not methods[name]:
+def _own(obj, methods: dict) -> bool:
+    """Whether ``methods`` (name -> function as its class defines it) are what ``obj`` has -- none overridden in a
+    subclass, replaced on the class or on the object -- so that a call which does their work may stand in for them."""
+    kind = type(obj)
+    for name, function in methods.items():
+        if getattr(kind, name) is not function:
             return False
-    return True
+    return obj.__dict__.keys().isdisjoint(methods)
 
 
-def _untouched(module: torch.nn.Module, cls: type, *names: str) -> bool:
-    """Whether calling ``module`` (or its methods ``names``) would run what ``cls`` defines and nothing else: no hooks, no
-    subclass, nothing replaced."""
-    return (type(module) is cls and _own(module, cls, "forward", *names)
-            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks)
-            and not torch.nn.modules.module._has_any_global_hook())
+def _untouched(module: torch.nn.Module, cls: type, methods: dict) -> bool:
+    """Whether ``module`` is a ``cls`` with its own ``methods`` and calling it runs nothing else (no hooks)."""
+    return (type(module) is cls and _own(module, methods)
+            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks))
 
 
 class PagedSelfAttentionCore(torch.nn.Module):
@@ -144,8 +142,8 @@ class PagedSelfAttentionCore(torch.nn.Module):
                 softmax_scale=self.softmax_scale, **self._norm_args())
             return out.reshape(out.size(0), out.size(1), -1)
         # (a step of prompts in one call of the context: in place of its append and of _attend below)
-        if (self.fused and isinstance(ctx, DynamicInferenceContext) and _own(self, PagedSelfAttentionCore, "_attend")
-                and _own(ctx, DynamicInferenceContext, "fused_qkv_norm_rope_append", "key_value_cache")
+        if (self.fused and isinstance(ctx, DynamicInferenceContext) and _own(self, _CORE_ATTEND)
+                and _own(ctx, _CONTEXT_PROMPTS)
                 and ctx.prefill_fusable(mixed_qkv, self.head_dim, emb)):
             out = ctx.fused_prefill_attention(
                 self.layer_number, mixed_qkv, num_query_heads=num_query_heads, rotary_pos_emb=emb,
@@ -280,10 +278,10 @@ class PagedSelfAttentionLayer(torch.nn.Module):
         one: other steps, another kind of context, hooks on the parts, or a replaced method whose work the call does."""
         qkv, core, proj = self._modules["linear_qkv"], self._modules["core"], self._modules["linear_proj"]
         n = hidden_states.size(0)
-        if (not (_untouched(qkv, DecodeLinear) and _untouched(proj, DecodeLinear)
-                 and _untouched(core, PagedSelfAttentionCore, "forward_mixed_qkv"))
-                or not isinstance(ctx, DynamicInferenceContext)
-                or not _own(ctx, DynamicInferenceContext, "fused_decode_step_attention", "key_value_cache")
+        if (not (_untouched(qkv, DecodeLinear, _LINEAR) and _untouched(proj, DecodeLinear, _LINEAR)
+                 and _untouched(core, PagedSelfAttentionCore, _CORE_MIXED))
+                or torch.nn.modules.module._has_any_global_hook()
+                or not isinstance(ctx, DynamicInferenceContext) or not _own(ctx, _CONTEXT_STEP)
                 or not core.fused or n > min(qkv.DECODE_ROWS, proj.DECODE_ROWS) or n != ctx.padded_active_token_count
                 or hidden_states.dim() != 3 or hidden_states.size(1) != 1):
             return None
@@ -297,10 +295,13 @@ class PagedSelfAttentionLayer(torch.nn.Module):
             rotary_pos_emb=emb, softmax_scale=core.softmax_scale, **core._norm_args())
 
 
-# The methods above (and the context's) that a fused call stands in for, as defined: see _own.
-_DEFINED = {
-    DecodeLinear: {"forward": DecodeLinear.forward},
-    PagedSelfAttentionCore: {name: getattr(PagedSelfAttentionCore, name) for name in ("forward", "forward_mixed_qkv", "_attend")},
-    DynamicInferenceContext: {name: getattr(DynamicInferenceContext, name)
-                              for name in ("fused_decode_step_attention", "fused_qkv_norm_rope_append", "key_value_cache")},
-}
+# The methods that a fused call stands in for, as defined: see _own.
+def _defined(cls: type, *names: str) -> dict:
+    return {name: getattr(cls, name) for name in names}
+
+
+_LINEAR = _defined(DecodeLinear, "forward")
+_CORE_MIXED = _defined(PagedSelfAttentionCore, "forward_mixed_qkv")
+_CORE_ATTEND = _defined(PagedSelfAttentionCore, "_attend")
+_CONTEXT_STEP = _defined(DynamicInferenceContext, "fused_decode_step_attention", "key_value_cache")
+_CONTEXT_PROMPTS = _defined(DynamicInferenceContext, "fused_qkv_norm_rope_append", "key_value_cache")

@@ -1009,9 +1009,6 @@ PyObject* op(PyObject*, PyObject* const* a, Py_ssize_t n) {
     PyErr_Clear();
     PyErr_SetString(oom ? oom : PyExc_RuntimeError, e.what_without_backtrace());
     return nullptr;
-  } catch (const c10::IndexError& e) {
-    PyErr_SetString(PyExc_IndexError, e.what_without_backtrace());
-    return nullptr;
   } catch (const c10::Error& e) {
     PyErr_SetString(PyExc_RuntimeError, e.what_without_backtrace());
     return nullptr;
@@ -1022,13 +1019,25 @@ PyObject* op(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // layer_views(buffer, layer, pair) -> new views of one layer: `buffer[0, layer]`, `buffer[1, layer]` of a buffer of keys and
-// values, or `buffer[layer]`, None.  (Indexing from Python takes 2-4 us for each.)
+// values, or `buffer[layer]`, None.  A decode step of a small batch asks for them in every layer, and indexing from Python
+// takes 2-4 us a view, an operation of the dispatcher's 0.5 us: these are made below autograd, which has no business in a
+// cache that kernels write (they take any write, and none makes the buffer itself require grad).
 PyObject* layer_views(PyObject* const* a) {
   const Tensor& buffer = tensor(a[0], "buffer");
-  const int64_t layer = as_int(a[1]);
-  if (!as_bool(a[2])) return Py_BuildValue("NO", wrap(buffer.select(0, layer)), Py_None);
-  const Tensor first = buffer.select(0, 0).select(0, layer), second = buffer.select(0, 1).select(0, layer);
-  return Py_BuildValue("NN", wrap(first), wrap(second));
+  const int lead = as_bool(a[2]) ? 2 : 1;
+  int64_t layer = as_int(a[1]);
+  const int64_t layers = buffer.dim() >= lead ? buffer.size(lead - 1) : 0;
+  if (layer < -layers || layer >= layers) {
+    PyErr_Format(PyExc_IndexError, "layer index %lld is out of range for %lld layers", (long long)layer, (long long)layers);
+    throw PyFailure{};
+  }
+  if (layer < 0) layer += layers;
+  const auto size = buffer.sizes().slice(lead), stride = buffer.strides().slice(lead);
+  const int64_t at = buffer.storage_offset() + layer * buffer.stride(lead - 1);
+  at::AutoDispatchBelowADInplaceOrView below;
+  const Tensor first = buffer.as_strided(size, stride, at);
+  if (lead == 1) return Py_BuildValue("NO", wrap(first), Py_None);
+  return Py_BuildValue("NN", wrap(first), wrap(buffer.as_strided(size, stride, at + buffer.stride(0))));
 }
 
 // watch(tensor, index, value, microseconds): whether element `index` of an int32 row in pinned host memory became
