@@ -27,7 +27,7 @@
 
 namespace mi {
 
-constexpr int kLinTok = 64;      // tokens per workgroup, at most
+constexpr int kLinTok = 64;      // tokens per workgroup, at most (and in the slice rule)
 constexpr int kLinStep = 64;     // columns a wavefront multiplies per step: whole 128-byte lines of 8 rows
 constexpr int kLinSlice = 512;   // columns per slice, at most
 constexpr int kLinRows = 128;    // (only in the slice rule)
@@ -61,7 +61,7 @@ __global__ __launch_bounds__(64 * NW) void linear_decode_kernel(LinearParams p) 
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m16 = lane & 15, g = lane >> 4;
   const int n0 = blockIdx.x * (16 * RT);
-  const int t0 = blockIdx.y * kLinTok;
+  const int t0 = blockIdx.y * (8 * XH);
   const int nt = min(8 * XH, p.T - t0);
 
   const int lo = lane >> 3, col = 8 * (lane & 7);
@@ -223,45 +223,49 @@ static int linear_lds(int rt, int half_tiles, int waves, int slices) {
   return (waves * (2 * rt + 2 * tt) + (slices > waves ? rt * tt : 0)) * 1024;
 }
 
-static int linear_half_tiles(int t) { return t <= 8 ? 1 : t <= 16 ? 2 : t <= 32 ? 4 : t <= 48 ? 6 : 8; }
-
-// Rows per workgroup (16 RT) and wavefronts (slices at a time): the pair with the least estimated time.  A workgroup
-// fills a CU (its registers or its LDS), so the launch runs in rounds of 256 workgroups; a round costs 4.6 us, 3 us
-// more for every further round of slices, and the bytes it brings into a CU, which arrive at 60 KB/us (W misses and x
-// hits share the CU's miss queue).  Fitted to seven shapes from 1280 x 2048 to 7168 x 5120 at 1 .. 256 tokens: within
-// 15 % of what was measured.  More rows per workgroup read x less often, fewer fill the chip; eight wavefronts have
-// the registers for four row tiles, sixteen for one or two.
-static void linear_plan(int T, int N, int K, int slices, int* row_tiles, int* waves) {
-  const int blocks = (T + kLinTok - 1) / kLinTok, xh = linear_half_tiles(T < kLinTok ? T : kLinTok);
+// (the instances there are: eight wavefronts have the registers for four row tiles, sixteen for one or two)
+static bool linear_instance(int rt, int xh, int waves, int slices) {
+  const int most = waves > 12 ? (xh <= 2 ? 2 : 1) : waves > 8 || xh <= 2 ? 2 : xh <= 4 ? 3 : 4;
+  return rt <= most && linear_lds(rt, xh, waves, slices) <= kLinLds;
+}
+// Tokens per workgroup (8 half_tiles), rows (16 row_tiles) and wavefronts (slices at a time): the triple with the least
+// estimated time.  A workgroup fills a CU (its registers or its LDS), so the launch runs in rounds of 256 workgroups; a
+// round costs 4.6 us, 3 us more for every further round of slices, and the bytes it brings into a CU, whose miss queue
+// carries 52 KB/us of W (from HBM) or 68 KB/us of x (from L2).  Fitted to ten shapes from 1280 x 2048 to 7168 x 5120 at 1 ..
+// 256 tokens: the triple taken is within 3 % of the fastest for 100 of the 110, within 13 % for all.  More rows per
+// workgroup read x less often, fewer fill the chip; where W has fewer row blocks than the chip has CUs, smaller token
+// blocks fill it, each with W once more (from the last-level cache): 64 tokens, 2048 x 8192 28.3 -> 19.8 us, 1280 x 5120
+// 22.6 -> 15.5.
+static void linear_plan(int T, int N, int K, int slices, int* half_tiles, int* row_tiles, int* waves) {
   double best = 0;
   *waves = 0;
   const int fewest = (slices + 15) / 16;
-  for (int rounds = fewest; rounds <= fewest + 2; ++rounds) {
-    const int w = (slices + rounds - 1) / rounds;
-    const int most = w > 12 ? (xh <= 2 ? 2 : 1) : w > 8 || xh <= 2 ? 2 : xh <= 4 ? 3 : 4;  // (the instances there are)
-    for (int rt = 1; rt <= most && linear_lds(rt, xh, w, slices) <= kLinLds; ++rt) {
-      const int64_t groups = (int64_t)((N + 16 * rt - 1) / (16 * rt)) * blocks;
-      const double us = (double)((groups + 255) / 256) * (4.6 + 3.0 * (rounds - 1) + (16 * rt + 8 * xh) * (double)K * 2 / 60e3);
-      if (*waves == 0 || us < best) {
-        best = us;
-        *row_tiles = rt;
-        *waves = w;
+  for (const int xh : {1, 2, 4, 6, 8}) {
+    const int blocks = (T + 8 * xh - 1) / (8 * xh);
+    for (int rounds = fewest; rounds <= fewest + 2; ++rounds) {
+      const int w = (slices + rounds - 1) / rounds;
+      for (int rt = 1; linear_instance(rt, xh, w, slices); ++rt) {
+        const int64_t groups = (int64_t)((N + 16 * rt - 1) / (16 * rt)) * blocks;
+        const double us = (double)((groups + 255) / 256) * (4.6 + 3.0 * (rounds - 1) + K * 2 * (16 * rt / 52e3 + 8 * xh / 68e3));
+        if (*waves == 0 || us < best) {
+          best = us;
+          *half_tiles = xh;
+          *row_tiles = rt;
+          *waves = w;
+        }
       }
     }
   }
 }
 
-
 template <bool F16, int RT, int XH, int P, int NW>
 static void launch_linear(const LinearParams& p, hipStream_t st) {
-  const dim3 grid((p.N + 16 * RT - 1) / (16 * RT), (p.T + kLinTok - 1) / kLinTok);
+  const dim3 grid((p.N + 16 * RT - 1) / (16 * RT), (p.T + 8 * XH - 1) / (8 * XH));
   hipLaunchKernelGGL((linear_decode_kernel<F16, RT, XH, P, NW>), grid, dim3(64 * p.waves), linear_lds(RT, XH, p.waves, p.S), st, p);
 }
 // (steps in flight: what fits the registers without spilling)
 template <bool F16>
-static void launch_linear(const LinearParams& p, int rt, hipStream_t st) {
-  const int t = p.T < kLinTok ? p.T : kLinTok;
-  const int xh = linear_half_tiles(t);
+static void launch_linear(const LinearParams& p, int rt, int xh, hipStream_t st) {
 #define LIN(RT, XH, P, NW) launch_linear<F16, RT, XH, P, NW>(p, st)
   if (p.waves <= 8) {
     switch (10 * xh + rt) {
@@ -348,13 +352,13 @@ extern "C" int mi_linear_decode(const void* x, int64_t x_stride_tok, const void*
     p.o_st = N;
   }
   linear_slices(T, N, K, &p.S, &p.kslice);
-  int rt;
-  linear_plan(T, N, K, p.S, &rt, &p.waves);
+  int rt, xh;
+  linear_plan(T, N, K, p.S, &xh, &rt, &p.waves);
   hipEvent_t ev_a, ev_b;
   const bool timed = mi_profile_next(&ev_a, &ev_b);
   if (timed) (void)hipEventRecord(ev_a, st);
-  if (dtype == MI_DTYPE_FP16) launch_linear<true>(p, rt, st);
-  else launch_linear<false>(p, rt, st);
+  if (dtype == MI_DTYPE_FP16) launch_linear<true>(p, rt, xh, st);
+  else launch_linear<false>(p, rt, xh, st);
   if (timed) (void)hipEventRecord(ev_b, st);
   if (staged)
     hipLaunchKernelGGL(linear_place_kernel, dim3((T * (N / 4) + 255) / 256), dim3(256), 0, st, p.out, (uint16_t*)out, out_stride_tok, T, N);

@@ -63,6 +63,19 @@ def test_tile_edges(mi, dev, T, N, K):
     _ulp_close(out, (big[:T, :K].float() @ w[:N, :K].float().t()).bfloat16(), torch.bfloat16, f"linear {T}x{N}x{K}")
 
 
+@pytest.mark.parametrize("T", [8, 16, 24, 33, 64, 65, 96, 200, 256])
+@pytest.mark.parametrize("N,K", [(2048, 8192), (1280, 5120), (48, 512)])
+def test_token_blocks(mi, dev, T, N, K):
+    """Few rows of W: the tokens are spread over more workgroups, with the last block partly empty."""
+    gen = torch.Generator().manual_seed(T + N + K)
+    x = (torch.randn(T, K, generator=gen) * 0.5).bfloat16().to(dev)
+    w = (torch.randn(N, K, generator=gen) * 0.05).bfloat16().to(dev)
+    out = torch.full((T + 2, N), 7.0, dtype=torch.bfloat16, device=dev)
+    mi.ops.linear_decode(x, w, out=out[:T])
+    _ulp_close(out[:T], (x.float() @ w.float().t()).bfloat16(), torch.bfloat16, f"linear {T}x{N}x{K}")
+    assert (out[T:] == 7.0).all(), "rows beyond the tokens were touched"
+
+
 def test_strided_inputs_and_leading_dimensions(mi, dev):
     gen = torch.Generator().manual_seed(5)
     big_x = (torch.randn(24, 1, 2 * 512, generator=gen) * 0.5).bfloat16().to(dev)
