@@ -668,10 +668,11 @@ int mi_sample_from_logits_ws(const void* logits, int64_t stride_row, int32_t log
  *   y[T, N] = x[T, K] . W[N, K]^T (+ bias[N]),   16-bit x / W / bias / y, fp32 accumulation.
  * The weight matrix is streamed from HBM once (it is the traffic: 50 MB for 4096 -> 6144), its rows riding
  * through the matrix cores; K is cut into slices of at most 512 columns whose fp32 sums are added in slice order inside
- * the workgroup that owns the rows (results do not depend on timing).  N a multiple of 16, K a multiple of 32; x, W and y
- * rows 16-byte aligned (y: 8-byte).  y may lie over x (or another input): the results then go to the workspace first and
- * a second launch moves them; otherwise the workspace is not written.  From K = 256 on it is asked for either way, of
- * mi_linear_decode_workspace_bytes() bytes.
+ * the workgroup that owns the rows -- or, where W has too few rows to fill the chip, in up to three parts whose sums a
+ * second launch adds (results depend on the sizes only, not on timing).  N a multiple of 16, K a multiple of 32; x, W and
+ * y rows 16-byte aligned (y: 8-byte).  y may lie over x (or another input): the results then go to the workspace first and
+ * a second launch moves them.  The workspace has mi_linear_decode_workspace_bytes() bytes; from K = 256 on it is asked
+ * for whether or not a call writes it.
  *
  * mi_linear_qkv_decode_step replaces `mixed_qkv, _ = self.linear_qkv(hidden_states)` of
  * Attention.get_query_key_value_tensors (megatron/core/transformer/attention.py:985-992; ColumnParallelLinear at

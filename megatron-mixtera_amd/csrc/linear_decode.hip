@@ -8,12 +8,13 @@
 // With a few dozen rows of x the weight matrix is the traffic -- 50 MB for 4096 -> 6144 -- and each of its bytes is
 // used once: the kernel is a stream of W from HBM with the products riding along.
 //
-// Work split: K is cut into slices of at most 512 columns, and the result is the slices' fp32 sums added in slice order
-// -- fixed by (T, N, K) alone, so a call is reproducible bit for bit however the work is spread.  A workgroup takes
-// 16 RT rows of W and all of K for a block of at most 64 tokens, one wavefront per slice: each piece of W and of x a
+// Work split: K is cut into slices of at most 512 columns, and the result is the slices' fp32 sums added in slice order,
+// part by part -- fixed by (T, N, K) alone, so a call is reproducible bit for bit.  A workgroup takes
+// 16 RT rows of W and all of K (or one of up to three parts) for a block of at most 64 tokens, one wavefront per slice: each piece of W and of x a
 // workgroup needs enters the CU exactly once, straight into the registers of the wavefront that multiplies it -- no
 // staging shared between wavefronts, no barrier before or between the products, and a ring of loads that stays full
-// from the first instruction on.  The slices' sums meet in LDS at the end: one kernel, no partial sums in memory.
+// from the first instruction on.  The slices' sums meet in LDS at the end: one kernel and no partial sums in memory, but
+// for calls whose row blocks alone would not fill the chip (linear_plan).
 //
 // 64 tokens, weights from HBM (GPU time per call, graph replay; before: 128 rows of one slice per workgroup, x staged
 // in LDS, partial sums in memory and a second kernel to add them):
@@ -39,6 +40,8 @@ struct LinearParams {
   const uint16_t* bias;
   uint16_t* out; int64_t o_st;
   int32_t T, N, K, kslice, S, waves;  // S slices of kslice columns (a multiple of 32), `waves` of them at a time
+  int32_t per_part;                   // slices of a part (S: the only one); part z of the grid takes z per_part onward
+  float* part;                        // with several parts their sums, [part][T][N]; else null
 };
 
 // RT = 16-row tiles of W, XH = 8-token half tiles of x, P = steps in flight, NW = wavefronts at most (8: 256 registers
@@ -127,12 +130,13 @@ __global__ __launch_bounds__(64 * NW) void linear_decode_kernel(LinearParams p) 
   };
   auto tile_at = [&](int slot, int tile) { return reinterpret_cast<f32x4_t*>(lds + (slot * RT * TT + tile) * kTile + 16 * lane); };
   static_assert(RT * TT * kTile <= kTurn, "the sums of a wavefront lie over its piece");
+  const int base = blockIdx.z * p.per_part, mine = min(p.per_part, p.S - base);
   auto before = [&](int tile) { return reinterpret_cast<f32x4_t*>(lds + p.waves * kTurn + tile * kTile + 16 * lane); };
-  for (int s0 = 0; s0 < p.S; s0 += p.waves) {   // (one round unless there are more than 16 slices)
-    if (s0 > 0) __syncthreads();                // the sums have been read
-    const int slice = s0 + wave;
+  for (int s0 = 0; s0 < mine; s0 += p.waves) {   // (one round unless there are more than 16 slices)
+    if (s0 > 0) __syncthreads();                 // the sums have been read
+    const int slice = base + s0 + wave;
     k0 = slice * p.kslice;
-    k1 = slice < p.S ? min(k0 + p.kslice, p.K) : k0;
+    k1 = s0 + wave < mine ? min(k0 + p.kslice, p.K) : k0;
     ka = k0 & ~(kLinStep - 1);
     const int steps = k1 > k0 ? (k1 - ka + kLinStep - 1) / kLinStep : 0;
 #pragma unroll
@@ -154,8 +158,8 @@ __global__ __launch_bounds__(64 * NW) void linear_decode_kernel(LinearParams p) 
 #pragma unroll
     for (int i = 0; i < RT * TT; ++i) *tile_at(wave, i) = acc[i];
     __syncthreads();
-    const int live = min(p.waves, p.S - s0);
-    const bool last = s0 + p.waves >= p.S;
+    const int live = min(p.waves, mine - s0);
+    const bool last = s0 + p.waves >= mine;
     for (int tile = wave; tile < RT * TT; tile += p.waves) {
       f32x4_t sum = f32x4_t{0.f, 0.f, 0.f, 0.f};
       if (s0 > 0) sum = *before(tile);
@@ -169,6 +173,10 @@ __global__ __launch_bounds__(64 * NW) void linear_decode_kernel(LinearParams p) 
       }
       const int n = n0 + 16 * (tile / TT) + 4 * g, t = 16 * (tile % TT) + m16;
       if (n >= p.N || t >= nt) continue;
+      if (p.part) {
+        *reinterpret_cast<f32x4_t*>(p.part + ((int64_t)blockIdx.z * p.T + t0 + t) * p.N + n) = sum;
+        continue;
+      }
       if (p.bias) {
         const uint2 bw = ld8(p.bias + n);
         sum[0] += lo_to_f32<F16>(bw.x); sum[1] += hi_to_f32<F16>(bw.x); sum[2] += lo_to_f32<F16>(bw.y); sum[3] += hi_to_f32<F16>(bw.y);
@@ -176,6 +184,25 @@ __global__ __launch_bounds__(64 * NW) void linear_decode_kernel(LinearParams p) 
       st8(p.out + (int64_t)(t0 + t) * p.o_st + n, make_uint2(pack2<F16>(sum[0], sum[1]), pack2<F16>(sum[2], sum[3])));
     }
   }
+}
+
+// The parts' sums added in order, with the bias: a thread takes four values.
+template <bool F16>
+__global__ __launch_bounds__(256) void linear_parts_kernel(LinearParams p, int parts) {
+  const int quads = p.N / 4, i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= p.T * quads) return;
+  const int t = i / quads, n = 4 * (i - t * quads);
+  const float* from = p.part + (int64_t)t * p.N + n;
+  f32x4_t sum = *reinterpret_cast<const f32x4_t*>(from);
+  for (int z = 1; z < parts; ++z) {
+    const f32x4_t v = *reinterpret_cast<const f32x4_t*>(from + (int64_t)z * p.T * p.N);
+    sum[0] += v[0]; sum[1] += v[1]; sum[2] += v[2]; sum[3] += v[3];
+  }
+  if (p.bias) {
+    const uint2 bw = ld8(p.bias + n);
+    sum[0] += lo_to_f32<F16>(bw.x); sum[1] += hi_to_f32<F16>(bw.x); sum[2] += lo_to_f32<F16>(bw.y); sum[3] += hi_to_f32<F16>(bw.y);
+  }
+  st8(p.out + t * p.o_st + n, make_uint2(pack2<F16>(sum[0], sum[1]), pack2<F16>(sum[2], sum[3])));
 }
 
 // `out` over one of the inputs: workgroups store their rows while others still load, so the results go to the workspace
@@ -228,44 +255,61 @@ static bool linear_instance(int rt, int xh, int waves, int slices) {
   const int most = waves > 12 ? (xh <= 2 ? 2 : 1) : waves > 8 || xh <= 2 ? 2 : xh <= 4 ? 3 : 4;
   return rt <= most && linear_lds(rt, xh, waves, slices) <= kLinLds;
 }
-// Tokens per workgroup (8 half_tiles), rows (16 row_tiles) and wavefronts (slices at a time): the triple with the least
-// estimated time.  A workgroup fills a CU (its registers or its LDS), so the launch runs in rounds of 256 workgroups; a
-// round costs 4.6 us, 3 us more for every further round of slices, and the bytes it brings into a CU, whose miss queue
-// carries 52 KB/us of W (from HBM) or 68 KB/us of x (from L2).  Fitted to ten shapes from 1280 x 2048 to 7168 x 5120 at 1 ..
-// 256 tokens: the triple taken is within 3 % of the fastest for 100 of the 110, within 13 % for all.  More rows per
-// workgroup read x less often, fewer fill the chip; where W has fewer row blocks than the chip has CUs, smaller token
-// blocks fill it, each with W once more (from the last-level cache): 64 tokens, 2048 x 8192 28.3 -> 19.8 us, 1280 x 5120
-// 22.6 -> 15.5.
-static void linear_plan(int T, int N, int K, int slices, int* half_tiles, int* row_tiles, int* waves) {
-  double best = 0;
-  *waves = 0;
-  const int fewest = (slices + 15) / 16;
-  for (const int xh : {1, 2, 4, 6, 8}) {
-    const int blocks = (T + 8 * xh - 1) / (8 * xh);
-    for (int rounds = fewest; rounds <= fewest + 2; ++rounds) {
-      const int w = (slices + rounds - 1) / rounds;
-      for (int rt = 1; linear_instance(rt, xh, w, slices); ++rt) {
-        const int64_t groups = (int64_t)((N + 16 * rt - 1) / (16 * rt)) * blocks;
-        const double us = (double)((groups + 255) / 256) * (4.6 + 3.0 * (rounds - 1) + K * 2 * (16 * rt / 52e3 + 8 * xh / 68e3));
-        if (*waves == 0 || us < best) {
-          best = us;
-          *half_tiles = xh;
-          *row_tiles = rt;
-          *waves = w;
+// How a call is spread: tokens per workgroup (8 half_tiles), rows (16 row_tiles), slices at a time (waves), and the parts
+// that the slices are cut into, with workgroups of their own and a second launch that adds their sums.
+struct LinearPlan {
+  int half_tiles, row_tiles, waves, parts;
+};
+// The plan with the least estimated time.  A workgroup fills a CU (its registers or its LDS), so the launch runs in rounds
+// of 256 workgroups; a round costs 4.6 us, 3 us more for every further round of slices, and the bytes it brings into a CU,
+// whose miss queue carries 52 KB/us of W (from HBM) or 60 KB/us of x (from L2); several parts cost 5 us and their sums
+// written and read.  Fitted to ten shapes from 1280 x 2048 to 10240 x 2048 at 1 .. 256 tokens: within 16 % of the fastest
+// plan everywhere, within 4 % for most.  More rows per workgroup read x less often, fewer fill the chip.  Where W has
+// fewer row blocks than the chip has CUs, or a few more, smaller token blocks (W once more for each, from the last-level
+// cache) or parts fill it; 64 tokens, against 64 in a workgroup and one part:
+//   2048 x 8192 28.3 -> 19.1 us,  5120 x 8192 34.7 -> 26.3,  1280 x 5120 22.6 -> 12.7,  2048 x 4096 15.4 -> 12.5
+static LinearPlan linear_plan(int T, int N, int K, int slices) {
+  LinearPlan best{};
+  double least = 0;
+  int64_t undivided = 0;  // workgroups of the best plan of one part
+  for (int z = 1; z <= 3; ++z) {
+    const int per = (slices + z - 1) / z, fewest = (per + 15) / 16;
+    // (as many parts as have slices; none where the chip is filled more than twice as it is: 10240 x 8192, 256 tokens,
+    // two parts 153 us against 149)
+    if ((z - 1) * per >= slices || undivided > 512) break;
+    int covered = 0;
+    const double merge = z > 1 ? 5.0 + z * (double)T * N * 8 / 4.5e6 : 0.0;
+    for (const int xh : {1, 2, 4, 6, 8}) {
+      const int blocks = (T + 8 * xh - 1) / (8 * xh);
+      if (covered >= T) break;  // (the last one held all tokens)
+      covered = 8 * xh;
+      for (int rounds = fewest; rounds <= fewest + 2; ++rounds) {
+        const int w = (per + rounds - 1) / rounds;
+        for (int rt = 1; linear_instance(rt, xh, w, per); ++rt) {
+          const int64_t groups = (int64_t)((N + 16 * rt - 1) / (16 * rt)) * blocks * z;
+          const double us = merge + (double)((groups + 255) / 256) *
+                                        (4.6 + 3.0 * (rounds - 1) + (double)K * 2 * (16 * rt / 52e3 + 8 * xh / 60e3) / z);
+          if (best.waves == 0 || us < least) {
+            least = us;
+            if (z == 1) undivided = groups;
+            best = LinearPlan{xh, rt, w, z};
+          }
         }
       }
     }
   }
+  return best;
 }
 
 template <bool F16, int RT, int XH, int P, int NW>
 static void launch_linear(const LinearParams& p, hipStream_t st) {
-  const dim3 grid((p.N + 16 * RT - 1) / (16 * RT), (p.T + 8 * XH - 1) / (8 * XH));
-  hipLaunchKernelGGL((linear_decode_kernel<F16, RT, XH, P, NW>), grid, dim3(64 * p.waves), linear_lds(RT, XH, p.waves, p.S), st, p);
+  const dim3 grid((p.N + 16 * RT - 1) / (16 * RT), (p.T + 8 * XH - 1) / (8 * XH), (p.S + p.per_part - 1) / p.per_part);
+  hipLaunchKernelGGL((linear_decode_kernel<F16, RT, XH, P, NW>), grid, dim3(64 * p.waves), linear_lds(RT, XH, p.waves, p.per_part), st, p);
 }
 // (steps in flight: what fits the registers without spilling)
 template <bool F16>
-static void launch_linear(const LinearParams& p, int rt, int xh, hipStream_t st) {
+static void launch_linear(const LinearParams& p, const LinearPlan& plan, hipStream_t st) {
+  const int rt = plan.row_tiles, xh = plan.half_tiles;
 #define LIN(RT, XH, P, NW) launch_linear<F16, RT, XH, P, NW>(p, st)
   if (p.waves <= 8) {
     switch (10 * xh + rt) {
@@ -312,12 +356,17 @@ static void launch_linear(const LinearParams& p, int rt, int xh, hipStream_t st)
 #undef LIN
 }
 
-// Room for the results, written only where `out` lies over an input.  A K of 256 and more asks for it on every call, so
-// that a caller who sizes none is told at the first.
-static int64_t linear_workspace(int T, int N) { return ((int64_t)T * N * 2 + 255) & ~(int64_t)255; }
+// Room for the parts' sums, or for the results where `out` lies over an input.  A K of 256 and more asks for it on every
+// call, so that a caller who sizes none is told at the first.
+static int64_t linear_workspace(int T, int N, int parts) {
+  return ((int64_t)T * N * (parts > 1 ? 4 * parts : 2) + 255) & ~(int64_t)255;
+}
 
 extern "C" int64_t mi_linear_decode_workspace_bytes(int32_t T, int32_t N, int32_t K) {
-  return T <= 0 || N <= 0 || K <= 0 ? 0 : linear_workspace(T, N);
+  if (T <= 0 || N <= 0 || K <= 0) return 0;
+  int slices, len;
+  linear_slices(T, N, K, &slices, &len);
+  return linear_workspace(T, N, linear_plan(T, N, K, slices).parts);
 }
 
 extern "C" int mi_linear_decode(const void* x, int64_t x_stride_tok, const void* weight, int64_t w_stride_row,
@@ -338,30 +387,37 @@ extern "C" int mi_linear_decode(const void* x, int64_t x_stride_tok, const void*
   p.x = (const uint16_t*)x; p.x_st = x_stride_tok; p.w = (const uint16_t*)weight; p.w_st = w_stride_row;
   p.bias = (const uint16_t*)bias; p.out = (uint16_t*)out; p.o_st = out_stride_tok;
   p.T = T; p.N = N; p.K = K;
-  hipStream_t st = (hipStream_t)stream;
-  const bool staged = linear_overlap(out, T, N, out_stride_tok, x, T, K, x_stride_tok) ||
-                      linear_overlap(out, T, N, out_stride_tok, weight, N, K, w_stride_row) ||
-                      (bias && linear_overlap(out, T, N, out_stride_tok, bias, 1, N, N));
-  if (staged || K >= 256) {
-    if (!workspace || workspace_bytes < linear_workspace(T, N))
+  linear_slices(T, N, K, &p.S, &p.kslice);
+  const LinearPlan plan = linear_plan(T, N, K, p.S);
+  const bool staged = plan.parts == 1 && (linear_overlap(out, T, N, out_stride_tok, x, T, K, x_stride_tok) ||
+                                          linear_overlap(out, T, N, out_stride_tok, weight, N, K, w_stride_row) ||
+                                          (bias && linear_overlap(out, T, N, out_stride_tok, bias, 1, N, N)));
+  if (staged || plan.parts > 1 || K >= 256) {
+    if (!workspace || workspace_bytes < linear_workspace(T, N, plan.parts))
       return mi_fail(MI_ERR_WORKSPACE, "mi_linear_decode: workspace smaller than mi_linear_decode_workspace_bytes()");
     if ((uintptr_t)workspace & 15) return mi_fail(MI_ERR_ALIGN, "mi_linear_decode: the workspace must be 16-byte aligned");
   }
+  p.waves = plan.waves;
+  p.per_part = (p.S + plan.parts - 1) / plan.parts;
+  p.part = plan.parts > 1 ? (float*)workspace : nullptr;
   if (staged) {
     p.out = (uint16_t*)workspace;
     p.o_st = N;
   }
-  linear_slices(T, N, K, &p.S, &p.kslice);
-  int rt, xh;
-  linear_plan(T, N, K, p.S, &xh, &rt, &p.waves);
+  hipStream_t st = (hipStream_t)stream;
   hipEvent_t ev_a, ev_b;
   const bool timed = mi_profile_next(&ev_a, &ev_b);
   if (timed) (void)hipEventRecord(ev_a, st);
-  if (dtype == MI_DTYPE_FP16) launch_linear<true>(p, rt, xh, st);
-  else launch_linear<false>(p, rt, xh, st);
+  if (dtype == MI_DTYPE_FP16) launch_linear<true>(p, plan, st);
+  else launch_linear<false>(p, plan, st);
   if (timed) (void)hipEventRecord(ev_b, st);
-  if (staged)
-    hipLaunchKernelGGL(linear_place_kernel, dim3((T * (N / 4) + 255) / 256), dim3(256), 0, st, p.out, (uint16_t*)out, out_stride_tok, T, N);
+  const dim3 after((T * (N / 4) + 255) / 256);
+  if (plan.parts > 1) {
+    if (dtype == MI_DTYPE_FP16) hipLaunchKernelGGL(linear_parts_kernel<true>, after, dim3(256), 0, st, p, plan.parts);
+    else hipLaunchKernelGGL(linear_parts_kernel<false>, after, dim3(256), 0, st, p, plan.parts);
+  } else if (staged) {
+    hipLaunchKernelGGL(linear_place_kernel, after, dim3(256), 0, st, p.out, (uint16_t*)out, out_stride_tok, T, N);
+  }
   return mi_check_launch("mi_linear_decode");
 }
 
