@@ -83,19 +83,32 @@ static __device__ __forceinline__ int wave_scan(int v) {
   return v;
 }
 
+// the largest of the lanes' values (none negative)
+static __device__ __forceinline__ int wave_max(int v) {
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
 constexpr int kOrderedRequests = 128;  // requests whose blocks are handed out longest first (two per lane)
-constexpr int kBlockLevels = 16;
+constexpr int kLengthLevels = 16;
 
 // The `rank`-th query block of the batch, blocks of `SBQ` rows; false: there are fewer.  `blocks` is the launch's count
 // (an upper bound).  Every wavefront of the workgroup calls this.
 //
-// The chip takes workgroups in order, so the longest must come first: in the batch's own order the last ones are the
-// first request's, however long its context, and the chip drains while they run.  Blocks are ranked by the keys
-// they see in 16 levels (equal ones side by side: blocks of one request share their keys in L2), which is within a few
-// percent of exact order in a list-scheduling model.  A lane holds one or two requests; how many blocks of a request
-// reach a level is arithmetic, so four steps of bisection and a scan find the block.  11 prompts of 33-3 001 tokens, head width
-// 64: the step 177.2 -> 170.5 us.  With more requests than that -- or one, whose blocks are in order as they are --
-// blocks come last to first: request r's are numbered cu_q[r] / SBQ + r onward.
+// The chip takes workgroups in order, so long ones must not come last: in the batch's own order the last ones are the
+// first request's, however long its context, and the chip drains while they run.  Requests go by their keys, longest
+// first, in 16 levels (within a level by index), and each request's blocks last to first: its shortest end the launch,
+// and blocks that run together share their keys in L2.  (Blocks of all requests ranked by their own length balance no
+// better and spread the reads: equal prompts 1 % slower than in batch order.)  A lane holds one or two requests; four steps
+// of bisection over the levels and a scan find the block.  Steps, against the batch's order: 11 prompts of 33-3 001 tokens,
+// head width 64, 149.9 -> 143.1 us; 8 prompts of 2 048 new tokens each over 0-4 096, 1 271 -> 1 273.  With more
+// requests than that -- or one, whose blocks are in order as they are -- blocks come last to first: request r's are
+// numbered cu_q[r] / SBQ + r onward.
 static __device__ __forceinline__ bool find_query_block(const PrefillParams& p, int SBQ, int rank, int blocks,
                                                         QueryBlock* o) {
   const int lane = threadIdx.x & 63;
@@ -118,23 +131,16 @@ static __device__ __forceinline__ bool find_query_block(const PrefillParams& p, 
         nb[c] = p.skip_single && lq[c] == 1 ? 0 : div(max(lq[c], 0) + SBQ - 1);
       }
     }
-    int top = max(nb[0] ? lk[0] : 0, nb[1] ? lk[1] : 0);
-#pragma unroll
-    for (int s = 1; s < 64; s <<= 1) top = max(top, __shfl_xor(top, s, 64));
-    const int step = (__builtin_amdgcn_readfirstlane(top) >> 4) + 1;
-    static_assert(kBlockLevels == 16, "levels of top / 16 keys");
-    // blocks of the lane's request c whose last row sees more than level * step keys
-    auto reach = [&](int c, int level) {
-      if (level <= 0) return nb[c];
-      const int need = level * step + 1 - (lk[c] - lq[c]);  // rows up to the first such one
-      if (level >= kBlockLevels || need > lq[c] || !nb[c]) return 0;
-      return nb[c] - (need > 0 ? div(need - 1) : 0);
-    };
+    const int top = wave_max(max(nb[0] ? lk[0] : 0, nb[1] ? lk[1] : 0));
+    const int step = (top >> 4) + 1;
+    static_assert(kLengthLevels == 16, "levels of top / 16 keys");
+    // blocks of the lane's request c if it has at least level * step keys
+    auto reach = [&](int c, int level) { return lk[c] >= level * step ? nb[c] : 0; };
     auto count = [&](int level) {
       return __builtin_amdgcn_readlane(wave_scan(reach(0, level) + reach(1, level)), 63);
     };
     if (rank >= count(0)) return false;
-    int lo = 0, hi = kBlockLevels, above = 0;  // count(lo) > rank >= count(hi) == above
+    int lo = 0, hi = kLengthLevels, above = 0;  // count(lo) > rank >= count(hi) == above
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       const int mid = (lo + hi) >> 1, n = count(mid);
@@ -150,9 +156,9 @@ static __device__ __forceinline__ bool find_query_block(const PrefillParams& p, 
     const int s0 = wave_scan(n0), s1 = wave_scan(n1), all0 = __builtin_amdgcn_readlane(s0, 63);
     const int c = j < all0 ? 0 : 1;
     if (c) j -= all0;
-    const int incl = c ? s1 : s0, n = c ? n1 : n0;
+    const int incl = c ? s1 : s0;
     const int at = __builtin_ctzll(__builtin_amdgcn_ballot_w64(incl > j));
-    const int b = __builtin_amdgcn_readlane((c ? nb[1] : nb[0]) - 1 - (c ? reach(1, hi) : reach(0, hi)) + incl - n, at) - j;
+    const int b = __builtin_amdgcn_readlane(incl, at) - 1 - j;  // the request's last block first
     o->r = at + 64 * c;
     o->q_begin = __builtin_amdgcn_readlane(c ? cq[1] : cq[0], at);
     o->Lq = __builtin_amdgcn_readlane(c ? lq[1] : lq[0], at);
