@@ -978,25 +978,31 @@ static void launch_split_merge(const PrefillParams& p, int n_split, int head_dim
 
 // Ranges the keys of every request are cut into by the tile kernels.  Few query rows over a long context (a chunk of a
 // prompt, a short turn after a long history) give few workgroups, each with many keys to walk.  The count is the one
-// with the least estimated time: rounds of workgroups over the CUs (one per CU), each 6 us of fixed cost and 1.5 us per
-// 64-key tile (head width 128, measured on one request of 33 to 1 000 tokens), and for more than one range the merge --
-// 4 us of launch and the fp32 partials written and read at 4.5 TB/s, which is what keeps prompts without a context from
-// being split (1 000 tokens x 32 heads in 2 ranges: 40 us against 37).  Host-side quantities only: the lengths live on
-// the GPU, `max_kv_len` is a bound.
+// with the least estimated time: workgroups over the CUs, and for more than one range the merge -- its launch and the
+// fp32 partials written and read at 4.5 TB/s, which is what keeps prompts without a context from being split (1 000
+// tokens x 32 heads in 2 ranges: 40 us against 37).  Head width 64: three workgroups share a CU, a 64-key tile takes
+// one alone 0.86 us and k of them 0.55 k us, 4 us of fixed cost for every three.  Other widths: one after the other, 6 us
+// and 1.5 us per tile (width 128).  Measured on one request of 33 to 2 000 tokens over 0 to 60 000 keys, 8-64 heads: within
+// 9 % of the best of eleven counts everywhere, within 1 % on average; width 64 counted as eight wavefronts
+// of one workgroup per CU: up to 16 % off.  Host-side quantities only: the lengths live on the GPU, `max_kv_len` is a
+// bound; and not the number of requests, so that a workspace sized for the most of them serves fewer.
 static int prefill_kv_splits(int T, int Hq, int Hkv, int head_dim, int max_kv_len) {
   if (max_kv_len <= 0) return 1;
   const int G = Hq / Hkv, Gw = G < 16 ? G : 16, parts = (G + 15) / 16;
-  const int sbq = 8 * ((head_dim >= 192 ? 16 : 32) / Gw);  // query tokens per workgroup (8 wavefronts x 32 or 16 rows)
+  const bool narrow = head_dim == 64;
+  const int sbq = (narrow ? prefill_woven_waves(64) : 8) * ((head_dim >= 192 ? 16 : 32) / Gw);  // query tokens per workgroup
   const int64_t useful = (int64_t)Hkv * parts * ((T + sbq - 1) / sbq);
   const int64_t cus = 256, tiles = ((int64_t)max_kv_len + 63) / 64;
-  if (useful >= cus) return 1;
-  const float per_tile = 1.5f * (float)head_dim / 128.f, partials = (float)T * (float)Hq * (float)head_dim * 8.f / 4.5e6f;
-  float best = 6.f + (float)tiles * per_tile;
+  if (useful >= (narrow ? 3 * cus : cus)) return 1;
+  const float partials = (float)T * (float)Hq * (float)head_dim * 8.f / 4.5e6f;
+  float best = 0.f;
   int n = 1;
   // (more than 32 ranges cost more in partials than they win: 64 rows over 131 072 keys, 16-32 is best)
-  for (int64_t s = 2; s <= 32 && 2 * s <= tiles; ++s) {
-    const float t = (float)((useful * s + cus - 1) / cus) * (6.f + (float)((tiles + s - 1) / s) * per_tile) + 4.f + (float)s * partials;
-    if (t < best) { best = t; n = (int)s; }
+  for (int64_t s = 1; s <= 32 && (s == 1 || 2 * s <= tiles); ++s) {
+    const float k = (float)((useful * s + cus - 1) / cus), per = (float)((tiles + s - 1) / s);
+    float t = narrow ? 4.f * ceilf(k / 3.f) + per * fmaxf(0.86f, 0.55f * k) : k * (6.f + per * 1.5f * (float)head_dim / 128.f);
+    if (s > 1) t += (narrow ? 2.f : 4.f) + (float)s * partials;
+    if (s == 1 || t < best) { best = t; n = (int)s; }
   }
   return n;
 }
@@ -1132,7 +1138,7 @@ static int launch_paged_prefill(
     const bool woven = tune.prefill_two_phase == 3 && (head_dim == 64 || head_dim == 128);
     // wavefronts x whole tokens in a wavefront's 32 (wide heads: 16) rows
     const int sbq_lds = (woven ? prefill_woven_waves(head_dim) : 8) * ((head_dim >= 192 ? 16 : 32) / Gw);
-    dim3 lgrid(((T + sbq_lds - 1) / sbq_lds + R) * Hkv * parts);
+    dim3 lgrid(prefill_query_blocks(T, R, sbq_lds) * Hkv * parts);
     hipEvent_t ev_a, ev_b;
     const bool timed = mi_profile_next(&ev_a, &ev_b);
     if (timed) (void)hipEventRecord(ev_a, st);
@@ -1336,7 +1342,7 @@ extern "C" int mi_paged_prefill_attention_mla(
   if (timed) (void)hipEventRecord(ev_a, st);
   int n_split = 1;
   if (two_phase) {
-    dim3 lgrid(((T + sbq - 1) / sbq + R) * Hkv * parts);
+    dim3 lgrid(prefill_query_blocks(T, R, sbq) * Hkv * parts);
     const bool stagger = tune.prefill_two_phase != 2;
     // few query rows over long contexts: key ranges per request, partials in the workspace (which holds
     // nothing else here: one-row requests stay in the tile kernel)

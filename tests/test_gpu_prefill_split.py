@@ -25,3 +25,24 @@ def test_few_rows_over_contexts(mi, dev, d, Hq, Hkv, one_row_requests):
     ref = oa.paged_varlen_attention(q[:T], kc, vc, cu_q, kv_lens, bt)
     assert (out[:T] - ref).abs().max().item() < 2e-2
     assert not out[T:].any()
+
+
+@pytest.mark.parametrize("d,Hq,Hkv", [(128, 8, 8), (64, 8, 8), (64, 32, 8), (192, 8, 2)])
+@pytest.mark.parametrize("q_lens", [[64], [40, 0, 0], [1, 65, 0, 16, 17], [0] * 127 + [3], [0, 5] * 65])
+def test_every_query_block_has_a_workgroup(mi, dev, d, Hq, Hkv, q_lens):
+    """As many blocks as a launch of these rows and requests can have: requests of whole blocks and of one row, requests
+    without rows, both forms of numbering (up to 128 requests and more), with and without key ranges."""
+    chunk, kv_lens = 64, torch.tensor([n + 200 if n else 0 for n in q_lens], dtype=torch.int32)
+    cu_q = torch.zeros(len(q_lens) + 1, dtype=torch.int32)
+    cu_q[1:] = torch.cumsum(torch.tensor(q_lens), 0)
+    gen = torch.Generator().manual_seed(d + len(q_lens))
+    bt, N = mi.synthetic.build_block_table(kv_lens.clamp(min=1), chunk, gen)
+    T = int(cu_q[-1])
+    q = torch.randn(T, Hq, d, generator=gen).bfloat16()
+    kc, vc = (torch.randn(N, chunk, Hkv, d, generator=gen).bfloat16() for _ in range(2))
+    ref = oa.paged_varlen_attention(q, kc, vc, cu_q, kv_lens, bt)
+    for split in (-1, 2):
+        with mi.ops.tuning(prefill_kv_split=split):
+            out = mi.ops.paged_prefill_attention(q.to(dev), kc.to(dev), vc.to(dev), cu_q.to(dev), kv_lens.to(dev), bt.to(dev),
+                                                 max_kv_len=int(kv_lens.max()), one_row_requests=False).float().cpu()
+        assert (out - ref).abs().max().item() < 2e-2
