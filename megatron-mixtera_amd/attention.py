@@ -144,7 +144,8 @@ class PagedSelfAttentionCore(torch.nn.Module):
         # (a step of prompts in one call of the context: in place of its append and of _attend below)
         if (self.fused and isinstance(ctx, DynamicInferenceContext) and _own(self, _CORE_ATTEND)
                 and _own(ctx, _CONTEXT_PROMPTS)
-                and ctx.prefill_fusable(mixed_qkv, self.head_dim, emb)):
+                and ctx.prefill_fusable(mixed_qkv, self.head_dim, emb, _parameter(self, "q_layernorm_weight"),
+                                        _parameter(self, "k_layernorm_weight"))):
             out = ctx.fused_prefill_attention(
                 self.layer_number, mixed_qkv, num_query_heads=num_query_heads, rotary_pos_emb=emb,
                 softmax_scale=self.softmax_scale, **self._norm_args())

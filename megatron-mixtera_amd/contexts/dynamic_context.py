@@ -680,11 +680,14 @@ class DynamicInferenceContext:
             faithful_rounding=faithful_rounding)
         return query_out
 
-    def prefill_fusable(self, mixed_qkv: Tensor, head_dim: int, rotary_pos_emb: Optional[Tensor]) -> bool:
+    def prefill_fusable(self, mixed_qkv: Tensor, head_dim: int, rotary_pos_emb: Optional[Tensor],
+                        *norm_weights: Optional[Tensor]) -> bool:
         """Whether :meth:`fused_prefill_attention` serves this step: every request was just admitted with more than one
-        token, and the tile kernel takes the shapes."""
+        token, the tile kernel takes the shapes, and rows and norm weights lie on the 16 bytes that it loads (the
+        separate calls take them anywhere)."""
         return (not self.cache_mla_latent and not self.one_row_requests_possible() and not self.is_decode_only()
                 and mixed_qkv.is_cuda and mixed_qkv.stride(0) % 8 == 0 and mixed_qkv.data_ptr() % 16 == 0
+                and all(w is None or w.data_ptr() % 16 == 0 for w in norm_weights)
                 and ops.qkv_prefill_supported(head_dim, self.chunk_size_tokens, rotary_pos_emb))
 
     def fused_prefill_attention(self, layer_number: int, mixed_qkv: Tensor, *, num_query_heads: int,

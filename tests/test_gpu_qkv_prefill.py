@@ -91,3 +91,24 @@ def test_core_takes_it_for_prompts_only(mi, dev, fp8, monkeypatch):
         assert outs[name].isfinite().all()
     a, b = outs["fused"].float(), outs["separate"].float()
     assert ((a - b).norm() / b.norm()).item() < (1e-2 if fp8 else 3e-3)
+
+
+def test_norm_weights_off_16_bytes_take_the_separate_calls(mi, dev):
+    """A weight in the middle of one flat parameter buffer: taken anywhere by the separate calls, so taken here."""
+    d, hq, hkv = 128, 8, 2
+    outs = []
+    for shift in (0, 1):
+        core = mi.PagedSelfAttentionCore(1, d, qk_norm="rms", device=dev).requires_grad_(False)
+        weights = torch.linspace(0.5, 1.5, 2 * d, device=dev).bfloat16()
+        flat = torch.cat([weights[:shift], weights])
+        core.q_layernorm_weight.data, core.k_layernorm_weight.data = flat[shift:shift + d], flat[shift + d:]
+        assert (core.q_layernorm_weight.data_ptr() % 16 == 0) == (shift == 0)
+        ctx = mi.DynamicInferenceContext(
+            params_dtype=torch.bfloat16, num_layers=1, kv_channels=d, num_attention_heads=hkv, max_sequence_length=400,
+            buffer_size_gb=0.01, buffer_guaranteed_fraction=0.0, chunk_size_tokens=CHUNK, max_requests_override=4)
+        ctx.add_request(0, torch.arange(70, device=dev))
+        ctx.initialize_attention_state()
+        mixed = torch.randn(ctx.padded_active_token_count, 1, (hq + 2 * hkv) * d,
+                            generator=torch.Generator(device=dev).manual_seed(3), device=dev).bfloat16()
+        outs.append(core.forward_mixed_qkv(mixed, hq, ctx)[:70].float())
+    assert ((outs[0] - outs[1]).norm() / outs[0].norm()).item() < 3e-3
