@@ -415,88 +415,49 @@ __global__ __launch_bounds__(1024) void step_attention_state_kernel(StepStatePar
 
 using namespace mi;
 
-static int update_requests(int mask_bytes,
-    int32_t* request_ids, int32_t* request_query_lengths, int32_t* request_output_lengths,
-    int32_t* request_kv_length_offsets, int32_t* request_kv_chunk_counts, int32_t* request_last_kv_chunk_id,
-    int32_t* request_last_kv_chunk_offset, int32_t* request_to_kv_chunk_ids, int64_t table_stride,
-    int32_t max_kv_chunk_count, int64_t* token_to_input_ids, int64_t* token_to_pos_ids,
-    int64_t* token_to_request_idx, int64_t* token_to_position_in_request, int64_t* token_to_chunk_idx,
-    int64_t* token_to_local_position_within_kv_chunk, int32_t* chunk_bag, const void* active_requests_mask,
-    const int64_t* new_tokens, int64_t* paused_tokens, int64_t* next_tokens_scratch, int32_t* scratch,
-    int32_t* newly_paused_request_ids, int32_t* finished_request_ids, int32_t* counters, int32_t total_request_count,
-    int32_t paused_request_count, int32_t chunk_count_avail, int32_t gtd_chunk_count,
-    int32_t gtd_request_count, int32_t chunk_size_tokens, int32_t max_requests, void* stream) {
-  if (!request_ids || !request_query_lengths || !request_output_lengths || !request_kv_length_offsets ||
-      !request_kv_chunk_counts || !request_last_kv_chunk_id || !request_last_kv_chunk_offset ||
-      !request_to_kv_chunk_ids || !token_to_input_ids || !token_to_pos_ids || !token_to_request_idx ||
-      !token_to_position_in_request || !token_to_chunk_idx || !token_to_local_position_within_kv_chunk ||
-      !chunk_bag || !active_requests_mask || !new_tokens || !paused_tokens || !next_tokens_scratch || !scratch ||
-      !newly_paused_request_ids || !finished_request_ids || !counters)
-    return mi_fail(MI_ERR_NULL, "mi_update_requests: null pointer argument");
-  if (total_request_count < 0 || paused_request_count < 0 || paused_request_count > total_request_count ||
-      total_request_count > max_requests || max_kv_chunk_count <= 0 || chunk_size_tokens <= 0)
-    return mi_fail(MI_ERR_SHAPE, "mi_update_requests: inconsistent counts");
-  UpdateParams p;
-  p.ids = request_ids; p.q_len = request_query_lengths; p.out_len = request_output_lengths;
-  p.kv_off = request_kv_length_offsets; p.n_chunks = request_kv_chunk_counts;
-  p.last_chunk = request_last_kv_chunk_id; p.last_off = request_last_kv_chunk_offset;
-  p.table = request_to_kv_chunk_ids; p.table_stride = table_stride; p.M = max_kv_chunk_count;
-  p.tok_input = token_to_input_ids; p.tok_pos = token_to_pos_ids; p.tok_req = token_to_request_idx;
-  p.tok_in_req = token_to_position_in_request; p.tok_chunk = token_to_chunk_idx;
-  p.tok_local = token_to_local_position_within_kv_chunk;
-  p.bag = chunk_bag; p.mask = active_requests_mask; p.mask_bytes = mask_bytes; p.new_tokens = new_tokens;
-  p.paused_tokens = paused_tokens; p.next_tokens = next_tokens_scratch; p.scratch = scratch;
-  p.newly_paused = newly_paused_request_ids; p.finished = finished_request_ids; p.counters = counters;
-  p.total = total_request_count; p.paused = paused_request_count; p.avail = chunk_count_avail;
-  p.gtd_chunks = gtd_chunk_count; p.gtd_requests = gtd_request_count; p.chunk = chunk_size_tokens;
-  p.max_requests = max_requests;
-  hipLaunchKernelGGL(update_requests_kernel, dim3(1), dim3(kThreads), 0, (hipStream_t)stream, p);
-  return mi_check_launch("mi_update_requests");
-}
-
-extern "C" int mi_update_requests(
-    int32_t* request_ids, int32_t* request_query_lengths, int32_t* request_output_lengths,
-    int32_t* request_kv_length_offsets, int32_t* request_kv_chunk_counts, int32_t* request_last_kv_chunk_id,
-    int32_t* request_last_kv_chunk_offset, int32_t* request_to_kv_chunk_ids, int64_t table_stride,
-    int32_t max_kv_chunk_count, int64_t* token_to_input_ids, int64_t* token_to_pos_ids,
-    int64_t* token_to_request_idx, int64_t* token_to_position_in_request, int64_t* token_to_chunk_idx,
-    int64_t* token_to_local_position_within_kv_chunk, int32_t* chunk_bag, const int32_t* active_requests_mask,
-    const int64_t* new_tokens, int64_t* paused_tokens, int64_t* next_tokens_scratch, int32_t* scratch,
-    int32_t* newly_paused_request_ids, int32_t* finished_request_ids, int32_t* counters, int32_t total_request_count,
-    int32_t paused_request_count, int32_t chunk_count_avail, int32_t gtd_chunk_count,
-    int32_t gtd_request_count, int32_t chunk_size_tokens, int32_t max_requests, void* stream) {
-  return update_requests(4, request_ids, request_query_lengths, request_output_lengths, request_kv_length_offsets,
-                         request_kv_chunk_counts, request_last_kv_chunk_id, request_last_kv_chunk_offset,
-                         request_to_kv_chunk_ids, table_stride, max_kv_chunk_count, token_to_input_ids,
-                         token_to_pos_ids, token_to_request_idx, token_to_position_in_request, token_to_chunk_idx,
-                         token_to_local_position_within_kv_chunk, chunk_bag, active_requests_mask, new_tokens,
-                         paused_tokens, next_tokens_scratch, scratch, newly_paused_request_ids,
-                         finished_request_ids, counters, total_request_count, paused_request_count,
-                         chunk_count_avail, gtd_chunk_count, gtd_request_count, chunk_size_tokens, max_requests,
-                         stream);
-}
-
-extern "C" int mi_update_requests_mask8(
-    int32_t* request_ids, int32_t* request_query_lengths, int32_t* request_output_lengths,
-    int32_t* request_kv_length_offsets, int32_t* request_kv_chunk_counts, int32_t* request_last_kv_chunk_id,
-    int32_t* request_last_kv_chunk_offset, int32_t* request_to_kv_chunk_ids, int64_t table_stride,
-    int32_t max_kv_chunk_count, int64_t* token_to_input_ids, int64_t* token_to_pos_ids,
-    int64_t* token_to_request_idx, int64_t* token_to_position_in_request, int64_t* token_to_chunk_idx,
-    int64_t* token_to_local_position_within_kv_chunk, int32_t* chunk_bag, const uint8_t* active_requests_mask,
-    const int64_t* new_tokens, int64_t* paused_tokens, int64_t* next_tokens_scratch, int32_t* scratch,
-    int32_t* newly_paused_request_ids, int32_t* finished_request_ids, int32_t* counters, int32_t total_request_count,
-    int32_t paused_request_count, int32_t chunk_count_avail, int32_t gtd_chunk_count,
-    int32_t gtd_request_count, int32_t chunk_size_tokens, int32_t max_requests, void* stream) {
-  return update_requests(1, request_ids, request_query_lengths, request_output_lengths, request_kv_length_offsets,
-                         request_kv_chunk_counts, request_last_kv_chunk_id, request_last_kv_chunk_offset,
-                         request_to_kv_chunk_ids, table_stride, max_kv_chunk_count, token_to_input_ids,
-                         token_to_pos_ids, token_to_request_idx, token_to_position_in_request, token_to_chunk_idx,
-                         token_to_local_position_within_kv_chunk, chunk_bag, active_requests_mask, new_tokens,
-                         paused_tokens, next_tokens_scratch, scratch, newly_paused_request_ids,
-                         finished_request_ids, counters, total_request_count, paused_request_count,
-                         chunk_count_avail, gtd_chunk_count, gtd_request_count, chunk_size_tokens, max_requests,
-                         stream);
-}
+// One body for the mask of int32 and the mask of bytes.
+#define MI_UPDATE_REQUESTS(NAME_, MASK_)                                                                              \
+  extern "C" int NAME_(                                                                                               \
+      int32_t* request_ids, int32_t* request_query_lengths, int32_t* request_output_lengths,                          \
+      int32_t* request_kv_length_offsets, int32_t* request_kv_chunk_counts, int32_t* request_last_kv_chunk_id,        \
+      int32_t* request_last_kv_chunk_offset, int32_t* request_to_kv_chunk_ids, int64_t table_stride,                  \
+      int32_t max_kv_chunk_count, int64_t* token_to_input_ids, int64_t* token_to_pos_ids,                             \
+      int64_t* token_to_request_idx, int64_t* token_to_position_in_request, int64_t* token_to_chunk_idx,              \
+      int64_t* token_to_local_position_within_kv_chunk, int32_t* chunk_bag, const MASK_* active_requests_mask,        \
+      const int64_t* new_tokens, int64_t* paused_tokens, int64_t* next_tokens_scratch, int32_t* scratch,              \
+      int32_t* newly_paused_request_ids, int32_t* finished_request_ids, int32_t* counters, int32_t total_request_count,\
+      int32_t paused_request_count, int32_t chunk_count_avail, int32_t gtd_chunk_count,                               \
+      int32_t gtd_request_count, int32_t chunk_size_tokens, int32_t max_requests, void* stream) {                     \
+    if (!request_ids || !request_query_lengths || !request_output_lengths || !request_kv_length_offsets ||            \
+        !request_kv_chunk_counts || !request_last_kv_chunk_id || !request_last_kv_chunk_offset ||                     \
+        !request_to_kv_chunk_ids || !token_to_input_ids || !token_to_pos_ids || !token_to_request_idx ||              \
+        !token_to_position_in_request || !token_to_chunk_idx || !token_to_local_position_within_kv_chunk ||           \
+        !chunk_bag || !active_requests_mask || !new_tokens || !paused_tokens || !next_tokens_scratch || !scratch ||   \
+        !newly_paused_request_ids || !finished_request_ids || !counters)                                              \
+      return mi_fail(MI_ERR_NULL, "mi_update_requests: null pointer argument");                                       \
+    if (total_request_count < 0 || paused_request_count < 0 || paused_request_count > total_request_count ||          \
+        total_request_count > max_requests || max_kv_chunk_count <= 0 || chunk_size_tokens <= 0)                      \
+      return mi_fail(MI_ERR_SHAPE, "mi_update_requests: inconsistent counts");                                        \
+    UpdateParams p;                                                                                                   \
+    p.ids = request_ids; p.q_len = request_query_lengths; p.out_len = request_output_lengths;                         \
+    p.kv_off = request_kv_length_offsets; p.n_chunks = request_kv_chunk_counts;                                       \
+    p.last_chunk = request_last_kv_chunk_id; p.last_off = request_last_kv_chunk_offset;                               \
+    p.table = request_to_kv_chunk_ids; p.table_stride = table_stride; p.M = max_kv_chunk_count;                       \
+    p.tok_input = token_to_input_ids; p.tok_pos = token_to_pos_ids; p.tok_req = token_to_request_idx;                 \
+    p.tok_in_req = token_to_position_in_request; p.tok_chunk = token_to_chunk_idx;                                    \
+    p.tok_local = token_to_local_position_within_kv_chunk;                                                            \
+    p.bag = chunk_bag; p.mask = active_requests_mask; p.mask_bytes = (int)sizeof(MASK_); p.new_tokens = new_tokens;   \
+    p.paused_tokens = paused_tokens; p.next_tokens = next_tokens_scratch; p.scratch = scratch;                        \
+    p.newly_paused = newly_paused_request_ids; p.finished = finished_request_ids; p.counters = counters;              \
+    p.total = total_request_count; p.paused = paused_request_count; p.avail = chunk_count_avail;                      \
+    p.gtd_chunks = gtd_chunk_count; p.gtd_requests = gtd_request_count; p.chunk = chunk_size_tokens;                  \
+    p.max_requests = max_requests;                                                                                    \
+    hipLaunchKernelGGL(update_requests_kernel, dim3(1), dim3(kThreads), 0, (hipStream_t)stream, p);                   \
+    return mi_check_launch("mi_update_requests");                                                                     \
+  }
+MI_UPDATE_REQUESTS(mi_update_requests, int32_t)
+MI_UPDATE_REQUESTS(mi_update_requests_mask8, uint8_t)
+#undef MI_UPDATE_REQUESTS
 
 extern "C" int mi_decode_attention_state(
     const int32_t* request_kv_length_offsets, const int32_t* request_query_lengths,
