@@ -216,8 +216,9 @@ static __device__ __forceinline__ float amax8(uint4 w, float m) {
 // key (z = 0) or value (z = 1) rows of each -- and quantises them whole: the run's values stay in registers between
 // the maximum that gives the scale and the conversion, so they are read once and there is no second launch.
 // Bound by memory for long prompts (3 bytes per value) and by the chain of loads (slots -> run -> values) for short
-// ones.  13 900 tokens x 8 heads of 128, key and value: 17 us (scales in a launch of their own, then the rows: 51 us);
-// 1 000 tokens and 24 padded rows: 7 us (53 us: each padded row was a run that a workgroup walked on its own).
+// ones.  13 900 tokens x 8 heads of 128, key and value, kernel time by trace: 27 us as a prompt step runs it, 23 with the
+// rows in the last-level cache (scales in a launch of their own, then the rows: 65 us); 1 000 tokens and 24 padded rows:
+// 12 us (57: each padded row was a run that a workgroup walked on its own).
 //   A run of one token, and a token that continues a chunk opened by an earlier call, need no more than a row: those
 //   of the slice are taken together, the threads spread over rows x pieces.
 //   A longer run is walked by the whole workgroup: the first kFp8Keep pieces (16 bytes each) of every thread -- a
@@ -535,7 +536,7 @@ extern "C" int mi_kv_append_fp8_strided(const void* key, int64_t k_stride_tok, i
                     !(((uintptr_t)k_cache_fp8 | (uintptr_t)v_cache_fp8 | (uintptr_t)kv_stride_chunk | (uintptr_t)kv_stride_tok) & 7);
   const bool f16 = dtype == MI_DTYPE_FP16;
   // Tokens per workgroup: a workgroup without a run start is all latency (13 900 tokens in slices of 32: 43 us), one
-  // with several walks them in turn (256: 28 us, 128: 26) -- 128 while that leaves the chip two workgroups per CU.
+  // with several walks them in turn (256: 28 us, 128: 27) -- 128 while that leaves the chip two workgroups per CU.
   const int64_t want = (int64_t)T * Hkv * 2 / 512;
   p.slice = want >= 128 ? 128 : want >= 64 ? 64 : 32;
   const dim3 grid((T + p.slice - 1) / p.slice, Hkv, 2), block(kFp8Threads);

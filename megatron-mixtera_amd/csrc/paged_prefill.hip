@@ -929,7 +929,7 @@ __global__ __launch_bounds__(512, 2) void paged_prefill_pp_kernel(PrefillParams 
 
 // Rows whose keys were split over several workgroups: o = sum_s 2^(lse_s - max) o_s / sum_s 2^(lse_s - max).
 // A thread takes four neighbouring output values of one (row, head); nx workgroups of 256 threads per row, flattened
-// into grid.x.  Bound by the partials' bytes: 509 rows x 64 heads of 128, 2 ranges, 42 MB: 12 us (one value per thread
+// into grid.x.  Bound by the partials' bytes: 509 rows x 64 heads of 128, 2 ranges, 42 MB: 9 us (one value per thread
 // and a workgroup per (row, head): 29 us, most of it launching workgroups).  Rows of one-row requests that the decode
 // kernels serve have no partials: what is written there from the workspace's old contents they overwrite afterwards.
 template <bool F16>
