@@ -381,11 +381,13 @@ class DynamicInferenceContext:
             self._await(self._max_lengths, 1, self._max_lengths_stream)
             self._max_lengths_in_flight = False
 
-    def _await(self, row: Tensor, index: int, stream) -> None:
-        """Wait until a kernel launched on ``stream`` has replaced the -1 in ``row[index]`` (pinned host memory).
-        ``stream`` is the launch's, which need not be the reader's; it is asked now and then whether it has run dry, so
-        that a launch which never stores its word ends in an error."""
+    def _await(self, row: Tensor, index: int, stream=None) -> None:
+        """Wait until a kernel launched on ``stream`` (default: the current one) has replaced the -1 in ``row[index]``
+        (pinned host memory).  The launch's stream need not be the reader's; it is asked now and then whether it has run
+        dry, so that a launch which never stores its word ends in an error."""
         while not ops.watch(row, index, -1, 20000):
+            if stream is None:
+                stream = torch.cuda.current_stream(self.device)
             if stream.query() and not ops.watch(row, index, -1, 0):
                 raise RuntimeError("a bookkeeping kernel has ended without its results")
 
@@ -1104,7 +1106,7 @@ class DynamicInferenceContext:
                 self._paused_tokens_buf[: self.paused_request_count] = self.paused_tokens[: self.paused_request_count]
         self._counters_host[5] = -1
         ops.update_requests(self, mask, tokens)
-        self._await(self._counters, 5, torch.cuda.current_stream(dev))
+        self._await(self._counters, 5)
         total, paused, active, avail, n_newly, status, was_reset, n_finished = self._counters_host.tolist()
         assert status != 1, "active + finished + paused requests != total_request_count"
         self.last_finished_request_ids = self._finished_ids_buf[:n_finished].clone()

@@ -32,6 +32,7 @@ constexpr int kLinTok = 64;      // tokens per workgroup, at most (and in the sl
 constexpr int kLinStep = 64;     // columns a wavefront multiplies per step: whole 128-byte lines of 8 rows
 constexpr int kLinSlice = 512;   // columns per slice, at most
 constexpr int kLinRows = 128;    // (only in the slice rule)
+constexpr int kLinParts = 3;     // parts of K with workgroups of their own, at most
 constexpr int kLinLds = 160 * 1024;
 
 struct LinearParams {
@@ -270,25 +271,26 @@ struct LinearPlan {
 //   2048 x 8192 28.3 -> 19.1 us,  5120 x 8192 34.7 -> 26.3,  1280 x 5120 22.6 -> 12.7,  2048 x 4096 15.4 -> 12.5
 static LinearPlan linear_plan(int T, int N, int K, int slices) {
   LinearPlan best{};
-  double least = 0;
-  int64_t undivided = 0;  // workgroups of the best plan of one part
-  for (int z = 1; z <= 3; ++z) {
+  float least = 0.f;
+  int undivided = 0;  // workgroups of the best plan of one part
+  const int tiles = (N + 15) / 16;
+  for (int z = 1; z <= kLinParts; ++z) {
     const int per = (slices + z - 1) / z, fewest = (per + 15) / 16;
     // (as many parts as have slices; none where the chip is filled more than twice as it is: 10240 x 8192, 256 tokens,
     // two parts 153 us against 149)
     if ((z - 1) * per >= slices || undivided > 512) break;
+    const float column = (float)K * 2.f / (float)z, merge = z > 1 ? 5.f + (float)z * (float)T * (float)N * (8.f / 4.5e6f) : 0.f;
     int covered = 0;
-    const double merge = z > 1 ? 5.0 + z * (double)T * N * 8 / 4.5e6 : 0.0;
     for (const int xh : {1, 2, 4, 6, 8}) {
-      const int blocks = (T + 8 * xh - 1) / (8 * xh);
+      const int blocks = (T + 8 * xh - 1) / (8 * xh) * z;
       if (covered >= T) break;  // (the last one held all tokens)
       covered = 8 * xh;
       for (int rounds = fewest; rounds <= fewest + 2; ++rounds) {
         const int w = (per + rounds - 1) / rounds;
         for (int rt = 1; linear_instance(rt, xh, w, per); ++rt) {
-          const int64_t groups = (int64_t)((N + 16 * rt - 1) / (16 * rt)) * blocks * z;
-          const double us = merge + (double)((groups + 255) / 256) *
-                                        (4.6 + 3.0 * (rounds - 1) + (double)K * 2 * (16 * rt / 52e3 + 8 * xh / 60e3) / z);
+          const int groups = (tiles + rt - 1) / rt * blocks;
+          const float us = merge + (float)((groups + 255) >> 8) *
+                                       (4.6f + 3.f * (float)(rounds - 1) + column * ((float)rt * (16.f / 52e3f) + (float)xh * (8.f / 60e3f)));
           if (best.waves == 0 || us < least) {
             least = us;
             if (z == 1) undivided = groups;
@@ -356,17 +358,17 @@ static void launch_linear(const LinearParams& p, const LinearPlan& plan, hipStre
 #undef LIN
 }
 
-// Room for the parts' sums, or for the results where `out` lies over an input.  A K of 256 and more asks for it on every
-// call, so that a caller who sizes none is told at the first.
-static int64_t linear_workspace(int T, int N, int parts) {
-  return ((int64_t)T * N * (parts > 1 ? 4 * parts : 2) + 255) & ~(int64_t)255;
+// Room for the sums of as many parts as a plan can have, or for the results where `out` lies over an input.  A K of 256
+// and more asks for it on every call, so that a caller who sizes none is told at the first.
+static int64_t linear_workspace(int T, int N, int slices) {
+  return ((int64_t)T * N * 4 * (slices < kLinParts ? slices : kLinParts) + 255) & ~(int64_t)255;
 }
 
 extern "C" int64_t mi_linear_decode_workspace_bytes(int32_t T, int32_t N, int32_t K) {
   if (T <= 0 || N <= 0 || K <= 0) return 0;
   int slices, len;
   linear_slices(T, N, K, &slices, &len);
-  return linear_workspace(T, N, linear_plan(T, N, K, slices).parts);
+  return linear_workspace(T, N, slices);
 }
 
 extern "C" int mi_linear_decode(const void* x, int64_t x_stride_tok, const void* weight, int64_t w_stride_row,
@@ -393,7 +395,7 @@ extern "C" int mi_linear_decode(const void* x, int64_t x_stride_tok, const void*
                                           linear_overlap(out, T, N, out_stride_tok, weight, N, K, w_stride_row) ||
                                           (bias && linear_overlap(out, T, N, out_stride_tok, bias, 1, N, N)));
   if (staged || plan.parts > 1 || K >= 256) {
-    if (!workspace || workspace_bytes < linear_workspace(T, N, plan.parts))
+    if (!workspace || workspace_bytes < linear_workspace(T, N, p.S))
       return mi_fail(MI_ERR_WORKSPACE, "mi_linear_decode: workspace smaller than mi_linear_decode_workspace_bytes()");
     if ((uintptr_t)workspace & 15) return mi_fail(MI_ERR_ALIGN, "mi_linear_decode: the workspace must be 16-byte aligned");
   }

@@ -21,8 +21,7 @@ from ._lib import (MI_DTYPE_BF16, MI_DTYPE_FP16, MI_KV_16BIT, MI_KV_BF16, MI_KV_
 _NORM_KINDS = {None: MI_NORM_NONE, "none": MI_NORM_NONE, "rms": MI_NORM_RMS, "l2": MI_NORM_L2}
 
 
-def _native():
-    return _lib.native()
+_native = _lib.native
 
 
 def _stream(t: Tensor) -> int:
@@ -465,9 +464,9 @@ def decode_step_attention(query: Optional[Tensor], key: Optional[Tensor], value:
 
 def layer_views(buffer: Tensor, layer: int, pair: bool) -> Tuple[Tensor, Optional[Tensor]]:
     """New views ``buffer[0, layer], buffer[1, layer]`` of a buffer of keys and values, or ``buffer[layer], None``."""
-    if not buffer.is_cuda:   # (a context on the host works without the built library)
-        return (buffer[0, layer], buffer[1, layer]) if pair else (buffer[layer], None)
-    return _native().layer_views(buffer, layer, pair)
+    if buffer.is_cuda:
+        return _native().layer_views(buffer, layer, pair)
+    return (buffer[0, layer], buffer[1, layer]) if pair else (buffer[layer], None)  # (a context on the host: no library)
 
 
 def watch(row: Tensor, index: int, value: int, microseconds: int) -> bool:
