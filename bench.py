@@ -35,18 +35,18 @@ MFMA_BF16_PEAK_TFLOPS = 2500.0  # MI355X dense bf16 matrix peak, published
 # read from inside the benchmark, so the figure is recorded here per workload; None = not collected.
 MEASURED_HBM_TRAFFIC_BYTES = {
     # decode workloads: "<cfg>" = the attention-only streaming kernel, "<cfg>_step" = the one-kernel decode step
-    "cfg2": 1_226_700_000, "cfg2_step": 1_215_000_000, "cfg4": 8_724_700_000, "cfg4_step": 8_634_800_000,
-    "cfg5": 9_070_200_000, "cfg5_step": 9_050_500_000,
+    "cfg2": 1_226_900_000, "cfg2_step": 1_215_100_000, "cfg4": 8_726_200_000, "cfg4_step": 8_635_500_000,
+    "cfg5": 9_072_200_000, "cfg5_step": 9_051_100_000,
     # the mixed step: tile kernel, stream kernel
-    "cfg3_tile": 401_700_000, "cfg3_stream": 2_195_700_000,
+    "cfg3_tile": 401_800_000, "cfg3_stream": 2_195_100_000,
     # multi-latent decode at 128 heads (reads + the partial results it writes)
     "mla_decode_h128": 454_500_000, "mla_decode_h128_long": 1_305_000_000}
 # Where each figure above was read, so that a reader of the JSON line can tell a stale constant from a fresh one:
 # the summary file and the last commit that touched the kernel when the counters were collected.
 _DECODE_TRAFFIC = ("profiles/decode_stream_kernels_hbm_traffic_cfg2_cfg4_cfg5.md (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, "
-                   "library as of commit b54c9eb)")
-_MIXED_TRAFFIC = ("profiles/paged_prefill_woven_kernel_cfg3_mfma.md (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, kernels as of "
-                  "commit e60638b; the one later change of the tile kernel, e3f1ea0, masks two base addresses at its set-up)")
+                   "library as of commit 2060602)")
+_MIXED_TRAFFIC = ("profiles/paged_prefill_woven_kernel_cfg3_mfma.md (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, library as of "
+                  "commit 2060602)")
 _MLA_HEADS_TRAFFIC = ("profiles/paged_mla_decode_heads_kernel_h128_counters.md (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, "
                       "kernel as of commit c8e09ff; the row pitch changed since, the traffic does not depend on it)")
 TRAFFIC_SOURCE = {"mla_decode_h128": _MLA_HEADS_TRAFFIC, "mla_decode_h128_long": _MLA_HEADS_TRAFFIC, "cfg2": _DECODE_TRAFFIC, "cfg2_step": _DECODE_TRAFFIC, "cfg4": _DECODE_TRAFFIC,
@@ -122,7 +122,7 @@ def run_secondary(args, mi, lib, torch, dev):
         pairs = n * (new * ctx + new * (new + 1) // 2)          # (query row, visible key) pairs per head
         flops = 2 * Hq * (dk + dv) * pairs
         nbytes = n * (new + ctx) * Hkv * (dk + dv) * 2 + n * new * Hq * (dk + dv) * 2
-        kernel = ("paged_prefill_woven_kernel" if (not mla and dk == 128 and args.prefill_kernel in (0, 3))
+        kernel = ("paged_prefill_woven_kernel" if (not mla and dk in (64, 128) and args.prefill_kernel in (0, 3))
                   else "paged_prefill_pp_kernel")
         what = (f"paged varlen causal attention, {n} x {new} new tokens over {ctx} cached, {Hq}/{Hkv} heads, "
                 f"keys {dk} / values {dv} wide, chunk 256")
@@ -147,8 +147,8 @@ def run_secondary(args, mi, lib, torch, dev):
         flops = 2 * T * N * K
         kernel = "linear_decode_kernel"
         what = (f"y[{T}, {N}] = x[{T}, {K}] . W[{N}, {K}]^T{' + bias' if prm['bias'] else ''}: the weight matrix streamed "
-                f"once (a ring of {n_w} matrices, so every call reads its weights from HBM), fp32 partial sums over slices "
-                f"of K and their reduction launch included in the step")
+                f"once (a ring of {n_w} matrices, so every call reads its weights from HBM), everything that adds up slices of "
+                f"K included in the step")
         dtype = "bf16 (fp32 accumulate)"
         timed_by_library = True
     elif kind == "sampling":
@@ -163,7 +163,7 @@ def run_secondary(args, mi, lib, torch, dev):
         step = lambda: mi.ops.sample_from_logits(logits, top_k=prm["top_k"], top_p=prm["top_p"], temperature=0.8,
                                                  uniform=u)
         nbytes = R * V * 4 + R * 12
-        kernel = "sample_kernel"
+        kernel = "sample_kernel, or its parts (sample_first / _mass / _pick_kernel)"
         what = (f"sampling of {R} rows of {V} fp32 logits ({'32 tokens 9-15 above a N(0, 2) bulk' if prm.get('peaked') else 'N(0, 3)'}), "
                 f"top_k {prm['top_k']}, top_p {prm['top_p']}, temperature 0.8")
         dtype = "fp32 logits, 2^-32 fixed-point mass"
@@ -233,7 +233,7 @@ def run_secondary(args, mi, lib, torch, dev):
         roofline["library_gemm_ms"] = round(sum(a.elapsed_time(b2) for a, b2 in ev) / args.steps, 5)
         roofline["call_ms"] = round(call_ms, 5)
         # both again as 3 x n_w calls captured in a HIP graph and replayed: GPU time per call without the host's
-        # launch cost (the eager figures above are bound by it: two launches here, one in the library)
+        # launch cost (the eager figures above are bound by it)
         nbytes_ws = lib.mi_linear_decode_workspace_bytes(T, N, K)
         fixed_ws = torch.empty(max(nbytes_ws, 16), dtype=torch.uint8, device=dev)
 
@@ -268,7 +268,7 @@ def run_secondary(args, mi, lib, torch, dev):
 def run_bookkeeping(args, mi, lib, torch, dev):
     """The host-visible bookkeeping of a decode step at serving sizes: mi_add_request per admitted prompt,
     mi_step_attention_state for the first (prefill) step, then per decode step mi_decode_attention_state and
-    mi_update_requests with its read-back of the new counters.  R requests, a chunk table M columns wide."""
+    mi_update_requests, whose counters the host watches in pinned memory.  R requests, a chunk table M columns wide."""
     from importlib import import_module
     ops = mi.ops
     ctx_mod = import_module(mi.__name__ + ".contexts.dynamic_context")
@@ -380,8 +380,8 @@ def run_bookkeeping(args, mi, lib, torch, dev):
         "steps": args.steps, "warmup": args.warmup, "ms_per_step": round(head["decode_step_wall_us"] / 1e3, 5),
         "higher_is_better": False, "scaling": "weak", "vs_baseline": None, "dtype": "int32 / int64", "data": "synthetic",
         "config": {"workload": "request / token bookkeeping of the dynamic context: value = host-visible time of one "
-                               "decode step's initialize_attention_state + update_requests (two launches, one 32-byte "
-                               "read-back) at 1024 requests and a 512-column chunk table; *_us = HIP events around each "
+                               "decode step's initialize_attention_state + update_requests (two launches; the host watches "
+                               "a word of the counters) at 1024 requests and a 512-column chunk table; *_us = HIP events around each "
                                "launch", "sizes": rows},
         "roofline": {"bound": "hbm", "kernel": "decode_attention_state_kernel + update_requests_kernel",
                      "achieved": round(nbytes / step_us / 1e3, 2), "peak": HBM_PEAK_GBPS, "unit": "GB/s",

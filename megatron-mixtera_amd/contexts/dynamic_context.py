@@ -1091,7 +1091,7 @@ class DynamicInferenceContext:
         return newly_paused_request_ids
 
     def _update_requests_fused(self, active_requests_mask: Tensor, new_tokens: Tensor) -> Optional[Tensor]:
-        """``update_requests`` as one kernel + one read-back of the new counters."""
+        """``update_requests`` as one kernel, whose counters the host watches in pinned memory."""
         dev = self.device
         assert active_requests_mask.numel() + self.paused_request_count == self.total_request_count
         mask, tokens = active_requests_mask, new_tokens

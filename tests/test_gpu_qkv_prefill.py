@@ -3,6 +3,9 @@ kernel -- against the separate calls (norm + rotary + append, then attention), w
 import pytest
 import torch
 
+from oracle import paged_attention as oa
+from oracle import rope_norm as orn
+
 pytestmark = pytest.mark.gpu
 
 CHUNK = 64
@@ -59,6 +62,47 @@ def test_equals_the_separate_calls(mi, dev, dtype, d, hq, hkv, norm, interleaved
     assert rel(caches[0], ref[0]) < 1e-3          # the norm's sum in another order: a rounding here and there
     assert rel(got, want) < (2e-3 if dtype == torch.bfloat16 else 5e-4)
     assert (got[int(kv.sum()):] == 0).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("hq,hkv,norm,interleaved,rope,lens,pad", [
+    (8, 2, "rms", False, True, (2, 31, 33, 257, 300), 7),
+    (6, 2, "l2", True, True, (65, 3, 129), 0),
+    (20, 1, "rms", True, True, (515, 64), 0),
+    (8, 8, None, False, False, (40, 200), 3),
+])
+def test_equals_the_oracle(mi, dev, dtype, d, hq, hkv, norm, interleaved, rope, lens, pad):
+    """Values bit for bit; keys as the op-by-op chain (under 1 % differ at all, by at most two units in the last place of
+    the head's largest: see the norm / rotary tests); attention within 2e-2 of fp32 attention over the oracle's cache."""
+    (mixed, pos, chunk, local, cu, kv, table), (qw, kw), caches, longest = _batch(mi, dev, lens, hq, hkv, d, dtype, pad, d + hq)
+    emb = orn.rotary_table(longest, d, interleaved=interleaved) if rope else None
+    qw, kw = (qw, kw) if norm == "rms" else (None, None)
+    eps = 1e-5 if norm == "rms" else 1e-6
+    common = dict(num_query_heads=hq, num_kv_heads=hkv, norm=norm, eps=eps, rotary_interleaved=interleaved)
+    cos_sin = mi.ops.qkv_key_append(mixed, k_cache=caches[0], v_cache=caches[1], k_weight=kw, q_positions=pos, k_positions=pos,
+                                    rotary_emb=emb if emb is None else emb.to(dev), token_to_chunk_idx=chunk,
+                                    token_to_local_pos=local, **common)
+    got = mi.ops.qkv_prefill_attention(mixed, *caches, cu, kv, table, max_kv_len=longest, cos_sin=cos_sin, q_weight=qw,
+                                       **common).squeeze(1).float().cpu()
+    real = int(kv.sum())
+    q, k, v = orn.split_mixed_qkv(mixed[:real].cpu(), hq, hkv)
+    chain = dict(norm=norm, eps=eps, interleaved=interleaved)
+    q = orn.norm_rope(q.reshape(real, hq, d), pos[:real].cpu(), emb, weight=qw if qw is None else qw.cpu(), **chain)
+    k = orn.norm_rope(k.reshape(real, hkv, d), pos[:real].cpu(), emb, weight=kw if kw is None else kw.cpu(), **chain)
+    v = v.reshape(real, hkv, d)
+    at = (chunk[:real].cpu(), local[:real].cpu())
+    assert torch.equal(caches[1].cpu()[at], v)
+    keys = caches[0].cpu()[at]
+    ulp = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)
+    err = (keys.float() - k.float()).abs()
+    assert (keys != k).float().mean().item() < 0.01
+    assert (err <= 2 * ulp * k.float().abs().amax(-1, keepdim=True)).all()
+    kc, vc = (torch.zeros(c.shape, dtype=dtype) for c in caches)
+    oa.kv_append(kc, vc, k, v, *at)
+    ref = oa.paged_varlen_attention(q, kc, vc, cu.cpu(), kv.cpu(), table.cpu())
+    assert (got[:real] - ref).abs().max().item() < 2e-2
+    assert not got[real:].any()
 
 
 @pytest.mark.parametrize("fp8", [False, True])
