@@ -18,11 +18,11 @@
 //
 // 64 tokens, weights from HBM (GPU time per call, graph replay; before: 128 rows of one slice per workgroup, x staged
 // in LDS, partial sums in memory and a second kernel to add them):
-//   4096 -> 6144   23.2 -> 19.1 us,  1 token 14.7 -> 11.6,  256 tokens 64 -> 42
-//   4096 -> 4096   21.7 -> 16.7 us,  1 token 14.1 ->  9.3,  256 tokens 45 -> 23
-//   2048 -> 1280   11.2 ->  8.6 us,  1 token  7.3 ->  4.6,  200 tokens 17 -> 11
-// The matrix alone streams in 10.3 us (4096 -> 6144); beside it the CU's miss queue carries x (64 tokens: 8 KB per
-// 2 KB of a 16-row tile of W), 60 KB/us in all.
+//   4096 -> 6144   23.9 -> 19.9 us,  1 token 16.1 -> 12.8,  256 tokens 65 -> 45
+//   4096 -> 4096   22.0 -> 16.4 us,  1 token 14.5 -> 10.0,  256 tokens 46 -> 25
+//   2048 -> 1280   11.4 ->  6.6 us,  1 token  7.3 ->  4.9,  256 tokens 18 ->  9
+// The matrix alone streams in 10.3 us (4096 -> 6144); beside it the CU's miss queue carries x (32 tokens: 4 KB per 6 KB of
+// a 48-row tile of W), at 52-60 KB/us: 168 MB into the CUs by counter, each request 680 clocks on its way.
 #include "mi_common.h"
 #include "mi_capi_internal.h"
 
