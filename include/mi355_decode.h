@@ -71,7 +71,7 @@ typedef struct MiTuning {
                                      the two-phase kernel elsewhere), -1 = register-only kernel */
   int32_t prefill_tile_subtiles;  /* register-only prefill kernel, 16-key sub-tiles per iteration: 0 = default (2), 1, 2 */
   int32_t prefill_row_tiles;      /* register-only prefill kernel, 16-row tiles per wavefront: 0 = default (2), 2, 4 */
-  int32_t prefill_kv_split;       /* two-phase kernel, key ranges per request: 0 = from T and max_kv_len, -1 = never,
+  int32_t prefill_kv_split;       /* tile kernels, key ranges per request: 0 = from T and max_kv_len, -1 = never,
                                      2..64 = forced where the workspace allows it */
   int32_t norm_rope_vectorised;   /* 16-byte-per-lane norm / rotary kernel: 0 = default (from 256 tokens up, where
                                      alignment and rotary width allow), 1 = wherever they allow, -1 = never */
@@ -189,8 +189,9 @@ int64_t mi_decode_workspace_bytes(int32_t R, int32_t Hq, int32_t Hkv, int32_t he
  *   out[r,h] = softmax(q[r,h] . K_r[:len_r, h/G]^T * softmax_scale) . V_r[:len_r, h/G]
  *   K_r[j] = k_cache[block_table[r, j / chunk_tokens], j % chunk_tokens], G = Hq/Hkv.
  * q/out: bf16 or fp16 `[R, Hq, d]` with the given token / head strides; d 64, 96, 128, 192 or 256 (an fp8 cache:
- * 64 or 128); G any value up to 64 (not only powers of two; every 16 query heads of a KV head take a wavefront).  kv_lens int32 [R] (0 => that row's output is zeros).  `max_kv_len` bounds every kv_lens[r] (the reference
- * passes max_sequence_length here, dynamic_context.py:791); the grid does not depend on
+ * 64 or 128); G any value up to 64 (not only powers of two; every 16 query heads of a KV head take a wavefront).
+ * kv_lens int32 [R] (0 => that row's output is zeros).  `max_kv_len` bounds every kv_lens[r] (the reference passes
+ * max_sequence_length here, dynamic_context.py:791); the grid does not depend on
  * it.  `split_tokens` = minimum tokens one workgroup streams (0 = default 64).
  * kv_dtype MI_KV_FP8_E4M3 reads byte caches with k_scales/v_scales `[n_chunks, Hkv]`.
  */
@@ -411,8 +412,8 @@ int mi_qkv_prefill_attention(const void* mixed_qkv, int64_t qkv_stride_tok, cons
  * attention.py:406-411) and hands them to flash_attn_varlen_func (attention.py:546-557).
  * Same mask and padding rules as mi_paged_prefill_attention; each cache has its own strides
  * (elements); q `[T, Hq, 192]`, out `[T, Hq, 128]`.  One kernel serves every request: the
- * two-phase LDS-tiled kernel when chunk_tokens is a multiple of 64 (and the knob prefill_pingpong
- * is not 0), a register-only kernel otherwise.  `workspace` may be NULL; one of
+ * two-phase LDS-tiled kernel when chunk_tokens is a multiple of 64 (and the knob prefill_two_phase
+ * is not -1), a register-only kernel otherwise.  `workspace` may be NULL; one of
  * mi_prefill_workspace_bytes(T, R, Hq, Hkv, head_dim_v, max_kv_len, 0) bytes (256-byte aligned) lets
  * the two-phase kernel cut the keys of every request into ranges when few query rows meet long
  * contexts, as in mi_paged_prefill_attention (`max_kv_len` bounds every kv_lens[r]; it only sizes

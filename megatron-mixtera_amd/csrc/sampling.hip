@@ -669,8 +669,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleParams p) 
 // fp32, 128 256 wide, us per call, one workgroup per row -> parts:
 //   64 rows: greedy 15 -> 12, plain 38 -> 24, top-k 50 39 -> 31, top-p 0.9 105 -> 44 (flat rows), 54 -> 41 (peaked)
 //    1 row : greedy 13 ->  8, plain 35 -> 15, top-k 50 36 -> 18, top-p 0.9 101 -> 25 (flat rows), 51 -> 24 (peaked)
-// 64 rows, top-p: 18 us for the first walk (38 vector instructions per 64 elements by counter, the pipe half busy), 15 for the second, 11 for
-// the pick (a chain of loads and barriers).
+// 64 rows, top-p: 18 us for the first walk (38 vector instructions per 64 elements by counter, the pipe half busy), 15
+// for the second, 11 for the pick (a chain of loads and barriers).
 constexpr int kBins = kSampleThreads; // 1/16 wide, from 24 above the reference to 40 below (and all that is lower)
 constexpr float kBinsAbove = 24.f, kBinsPerUnit = 16.f;
 constexpr int kRuns = kSampleWaves;   // runs of elements per part
