@@ -10,8 +10,8 @@
 //
 // Work split: K is cut into slices of at most 512 columns, and the result is the slices' fp32 sums added in slice order,
 // part by part -- fixed by (T, N, K) alone, so a call is reproducible bit for bit.  A workgroup takes
-// 16 RT rows of W and all of K (or one of up to three parts) for a block of at most 64 tokens, one wavefront per slice: each piece of W and of x a
-// workgroup needs enters the CU exactly once, straight into the registers of the wavefront that multiplies it -- no
+// 16 RT rows of W and all of K (or one of up to three parts) for a block of at most 64 tokens, one wavefront per slice:
+// each piece of W and of x that a workgroup needs enters the CU exactly once, straight into the registers of the wavefront that multiplies it -- no
 // staging shared between wavefronts, no barrier before or between the products, and a ring of loads that stays full
 // from the first instruction on.  The slices' sums meet in LDS at the end: one kernel and no partial sums in memory, but
 // for calls whose row blocks alone would not fill the chip (linear_plan).
@@ -187,9 +187,10 @@ __global__ __launch_bounds__(64 * NW) void linear_decode_kernel(LinearParams p) 
   }
 }
 
-// The parts' sums added in order, with the bias: a thread takes four values.
+// The parts' sums added in order, with the bias: a thread takes four values, and its four results lie `quad` values past
+// those of the thread before (8, with p.out the workspace: over the first part's sums that it has read).
 template <bool F16>
-__global__ __launch_bounds__(256) void linear_parts_kernel(LinearParams p, int parts) {
+__global__ __launch_bounds__(256) void linear_parts_kernel(LinearParams p, int parts, int quad) {
   const int quads = p.N / 4, i = blockIdx.x * 256 + threadIdx.x;
   if (i >= p.T * quads) return;
   const int t = i / quads, n = 4 * (i - t * quads);
@@ -203,16 +204,16 @@ __global__ __launch_bounds__(256) void linear_parts_kernel(LinearParams p, int p
     const uint2 bw = ld8(p.bias + n);
     sum[0] += lo_to_f32<F16>(bw.x); sum[1] += hi_to_f32<F16>(bw.x); sum[2] += lo_to_f32<F16>(bw.y); sum[3] += hi_to_f32<F16>(bw.y);
   }
-  st8(p.out + t * p.o_st + n, make_uint2(pack2<F16>(sum[0], sum[1]), pack2<F16>(sum[2], sum[3])));
+  st8(p.out + t * p.o_st + (i - t * quads) * quad, make_uint2(pack2<F16>(sum[0], sum[1]), pack2<F16>(sum[2], sum[3])));
 }
 
 // `out` over one of the inputs: workgroups store their rows while others still load, so the results go to the workspace
-// and this launch puts them in place.
-__global__ __launch_bounds__(256) void linear_place_kernel(const uint16_t* from, uint16_t* out, int64_t o_st, int T, int N) {
+// (four of them every `quad` values) and this launch puts them in place.
+__global__ __launch_bounds__(256) void linear_place_kernel(const uint16_t* from, int quad, uint16_t* out, int64_t o_st, int T, int N) {
   const int quads = N / 4, i = blockIdx.x * 256 + threadIdx.x;   // (T N / 4 fits: T <= 256)
   if (i >= T * quads) return;
   const int t = i / quads, n = 4 * (i - t * quads);
-  st8(out + t * o_st + n, ld8(from + (int64_t)t * N + n));
+  st8(out + t * o_st + n, ld8(from + (int64_t)i * quad));
 }
 
 }  // namespace mi
@@ -391,9 +392,10 @@ extern "C" int mi_linear_decode(const void* x, int64_t x_stride_tok, const void*
   p.T = T; p.N = N; p.K = K;
   linear_slices(T, N, K, &p.S, &p.kslice);
   const LinearPlan plan = linear_plan(T, N, K, p.S);
-  const bool staged = plan.parts == 1 && (linear_overlap(out, T, N, out_stride_tok, x, T, K, x_stride_tok) ||
-                                          linear_overlap(out, T, N, out_stride_tok, weight, N, K, w_stride_row) ||
-                                          (bias && linear_overlap(out, T, N, out_stride_tok, bias, 1, N, N)));
+  // (with several parts only the second launch stores, and reads nothing but the bias)
+  const bool staged = (bias && linear_overlap(out, T, N, out_stride_tok, bias, 1, N, N)) ||
+                      (plan.parts == 1 && (linear_overlap(out, T, N, out_stride_tok, x, T, K, x_stride_tok) ||
+                                           linear_overlap(out, T, N, out_stride_tok, weight, N, K, w_stride_row)));
   if (staged || plan.parts > 1 || K >= 256) {
     if (!workspace || workspace_bytes < linear_workspace(T, N, p.S))
       return mi_fail(MI_ERR_WORKSPACE, "mi_linear_decode: workspace smaller than mi_linear_decode_workspace_bytes()");
@@ -402,9 +404,10 @@ extern "C" int mi_linear_decode(const void* x, int64_t x_stride_tok, const void*
   p.waves = plan.waves;
   p.per_part = (p.S + plan.parts - 1) / plan.parts;
   p.part = plan.parts > 1 ? (float*)workspace : nullptr;
+  const int quad = staged && plan.parts > 1 ? 8 : 4;
   if (staged) {
     p.out = (uint16_t*)workspace;
-    p.o_st = N;
+    p.o_st = N / 4 * quad;
   }
   hipStream_t st = (hipStream_t)stream;
   hipEvent_t ev_a, ev_b;
@@ -415,11 +418,11 @@ extern "C" int mi_linear_decode(const void* x, int64_t x_stride_tok, const void*
   if (timed) (void)hipEventRecord(ev_b, st);
   const dim3 after((T * (N / 4) + 255) / 256);
   if (plan.parts > 1) {
-    if (dtype == MI_DTYPE_FP16) hipLaunchKernelGGL(linear_parts_kernel<true>, after, dim3(256), 0, st, p, plan.parts);
-    else hipLaunchKernelGGL(linear_parts_kernel<false>, after, dim3(256), 0, st, p, plan.parts);
-  } else if (staged) {
-    hipLaunchKernelGGL(linear_place_kernel, after, dim3(256), 0, st, p.out, (uint16_t*)out, out_stride_tok, T, N);
+    if (dtype == MI_DTYPE_FP16) hipLaunchKernelGGL(linear_parts_kernel<true>, after, dim3(256), 0, st, p, plan.parts, quad);
+    else hipLaunchKernelGGL(linear_parts_kernel<false>, after, dim3(256), 0, st, p, plan.parts, quad);
   }
+  if (staged)
+    hipLaunchKernelGGL(linear_place_kernel, after, dim3(256), 0, st, p.out, quad, (uint16_t*)out, out_stride_tok, T, N);
   return mi_check_launch("mi_linear_decode");
 }
 

@@ -89,7 +89,7 @@ def test_strided_inputs_and_leading_dimensions(mi, dev):
     assert (out[..., 256:] == 7.0).all(), "columns beyond N were touched"
 
 
-@pytest.mark.parametrize("T,N,K", [(64, 2048, 2048), (200, 512, 512), (5, 128, 128), (33, 16, 1024)])
+@pytest.mark.parametrize("T,N,K", [(64, 2048, 2048), (200, 512, 512), (5, 128, 128), (33, 16, 1024), (64, 2048, 8192)])
 @pytest.mark.parametrize("place", ["x", "rows before", "part of x", "beside x", "w", "bias"])
 def test_results_over_an_input(mi, dev, T, N, K, place):
     """Bit for bit what a call with a result of its own gives, also where rows are stored that others still read."""
