@@ -75,20 +75,23 @@ def _parameter(module: torch.nn.Module, name: str) -> Optional[Tensor]:
     return p if p is not None else getattr(module, name)
 
 
-def _own(obj, methods: dict) -> bool:
-    """Whether ``methods`` (name -> function as its class defines it) are what ``obj`` has -- none overridden in a
-    subclass, replaced on the class or on the object -- so that a call which does their work may stand in for them."""
-    kind = type(obj)
-    for name, function in methods.items():
-        if getattr(kind, name) is not function:
+def _own(obj, methods: tuple) -> bool:
+    """Whether ``methods`` (pairs of name and function as its class defines it) are what ``obj`` has -- none overridden in
+    a subclass, replaced on the class or on the object -- so that a call which does their work may stand in for them."""
+    kind, own = type(obj), obj.__dict__
+    for name, function in methods:
+        if name in own or getattr(kind, name) is not function:
             return False
-    return obj.__dict__.keys().isdisjoint(methods)
+    return True
 
 
-def _untouched(module: torch.nn.Module, cls: type, methods: dict) -> bool:
+def _untouched(module: torch.nn.Module, cls: type, methods: tuple) -> bool:
     """Whether ``module`` is a ``cls`` with its own ``methods`` and calling it runs nothing else (no hooks)."""
-    return (type(module) is cls and _own(module, methods)
-            and not (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks))
+    if type(module) is not cls:
+        return False
+    own = module.__dict__
+    return not (own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or own["_backward_pre_hooks"]
+                ) and _own(module, methods)
 
 
 class PagedSelfAttentionCore(torch.nn.Module):
@@ -279,10 +282,10 @@ class PagedSelfAttentionLayer(torch.nn.Module):
         one: other steps, another kind of context, hooks on the parts, or a replaced method whose work the call does."""
         qkv, core, proj = self._modules["linear_qkv"], self._modules["core"], self._modules["linear_proj"]
         n = hidden_states.size(0)
-        if (not (_untouched(qkv, DecodeLinear, _LINEAR) and _untouched(proj, DecodeLinear, _LINEAR)
-                 and _untouched(core, PagedSelfAttentionCore, _CORE_MIXED))
+        if (not isinstance(ctx, DynamicInferenceContext) or not ctx.is_decode_only() or not _own(ctx, _CONTEXT_STEP)
+                or not (_untouched(qkv, DecodeLinear, _LINEAR) and _untouched(proj, DecodeLinear, _LINEAR)
+                        and _untouched(core, PagedSelfAttentionCore, _CORE_MIXED))
                 or torch.nn.modules.module._has_any_global_hook()
-                or not isinstance(ctx, DynamicInferenceContext) or not _own(ctx, _CONTEXT_STEP)
                 or not core.fused or n > min(qkv.DECODE_ROWS, proj.DECODE_ROWS) or n != ctx.padded_active_token_count
                 or hidden_states.dim() != 3 or hidden_states.size(1) != 1):
             return None
@@ -297,8 +300,8 @@ class PagedSelfAttentionLayer(torch.nn.Module):
 
 
 # The methods that a fused call stands in for, as defined: see _own.
-def _defined(cls: type, *names: str) -> dict:
-    return {name: getattr(cls, name) for name in names}
+def _defined(cls: type, *names: str) -> tuple:
+    return tuple((name, getattr(cls, name)) for name in names)
 
 
 _LINEAR = _defined(DecodeLinear, "forward")

@@ -308,8 +308,9 @@ class DynamicInferenceContext:
             self._max_lengths = watched[32:34]
             self._max_lengths_host = self._max_lengths.numpy()
         self._max_lengths_pending = False     # nobody has read the step's maxima yet
-        self._max_lengths_in_flight = False   # their kernel, launched on _max_lengths_stream, may not have run yet
-        self._max_lengths_stream = None
+        self._max_lengths_in_flight = False   # their kernel may not have run yet
+        # (ids of the streams that the kernels of the watched words were launched on last)
+        self._max_lengths_stream = self._counters_stream = None
         # what the host knows without asking the device: the longest prompt admitted since the last
         # update_requests (every other active request has one query token) and a bound on the kv lengths
         self._host_max_query_len = 1
@@ -381,13 +382,14 @@ class DynamicInferenceContext:
             self._await(self._max_lengths, 1, self._max_lengths_stream)
             self._max_lengths_in_flight = False
 
-    def _await(self, row: Tensor, index: int, stream=None) -> None:
-        """Wait until a kernel launched on ``stream`` (default: the current one) has replaced the -1 in ``row[index]``
-        (pinned host memory).  The launch's stream need not be the reader's; it is asked now and then whether it has run
-        dry, so that a launch which never stores its word ends in an error."""
+    def _await(self, row: Tensor, index: int, stream) -> None:
+        """Wait until a kernel launched on ``stream`` (a stream or its id) has replaced the -1 in ``row[index]`` (pinned
+        host memory).  The launch's stream need not be the reader's; it is asked now and then whether it has run dry, so
+        that a launch which never stores its word ends in an error."""
         while not ops.watch(row, index, -1, 20000):
-            if stream is None:
-                stream = torch.cuda.current_stream(self.device)
+            if isinstance(stream, int):
+                table = self.request_to_kv_chunk_ids
+                stream = torch.cuda.Stream(stream_id=stream, device_index=table.device.index, device_type=1)  # (1: the GPU)
             if stream.query() and not ops.watch(row, index, -1, 0):
                 raise RuntimeError("a bookkeeping kernel has ended without its results")
 
@@ -794,7 +796,6 @@ class DynamicInferenceContext:
             self._land_max_lengths()  # (an earlier step's must not arrive after the reset of the words)
             self._max_lengths_host[:] = -1
             ops.step_attention_state(self, n_active_req, R, padded)
-            self._max_lengths_stream = torch.cuda.current_stream(self.device)
             self._max_lengths_in_flight = True
             self.kv_seq_lengths = self.kv_seq_lengths_cudagraph_only[:R]
             self.block_table = self.request_to_kv_chunk_ids_cudagraph_only[:R]
@@ -1106,7 +1107,9 @@ class DynamicInferenceContext:
                 self._paused_tokens_buf[: self.paused_request_count] = self.paused_tokens[: self.paused_request_count]
         self._counters_host[5] = -1
         ops.update_requests(self, mask, tokens)
-        self._await(self._counters, 5)
+        self._await(self._counters, 5, self._counters_stream)
+        if self._counters_stream == self._max_lengths_stream:
+            self._max_lengths_in_flight = False   # (the stream is in order)
         total, paused, active, avail, n_newly, status, was_reset, n_finished = self._counters_host.tolist()
         assert status != 1, "active + finished + paused requests != total_request_count"
         self.last_finished_request_ids = self._finished_ids_buf[:n_finished].clone()

@@ -1065,7 +1065,7 @@ PyObject* watch(PyObject* const* a) {
 
 // written_by_kernel(row, device index): a kernel about to go onto the device's current stream stores into `row`, pinned
 // host memory of torch's allocator.  The allocator sees the copies it is told of, not a kernel's stores: noted here, the
-// memory of a dropped `row` is handed out again only once the stream has got past this point.
+// memory of a dropped `row` is handed out again only once the stream has got past this point.  Returns the stream's id.
 PyObject* written_by_kernel(PyObject* const* a) {
   const Tensor& t = tensor(a[0], "row");
   const c10::Device device(c10::kCUDA, (c10::DeviceIndex)as_int(a[1]));
@@ -1073,7 +1073,7 @@ PyObject* written_by_kernel(PyObject* const* a) {
   const c10::Stream stream = c10::impl::VirtualGuardImpl(c10::kCUDA).getStream(device);
   REQUIRE(at::getHostAllocator(c10::kCUDA)->record_event(t.data_ptr(), t.storage().data_ptr().get_context(), stream),
           "written_by_kernel takes a row in torch's pinned memory");
-  Py_RETURN_NONE;
+  return PyLong_FromLongLong(stream.id());
 }
 
 // setup(kernel_error_class, raw_stream(device index), grow(device index, stream, bytes))

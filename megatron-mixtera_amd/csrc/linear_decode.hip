@@ -298,6 +298,7 @@ static LinearPlan linear_plan(int T, int N, int K, int slices) {
             best = LinearPlan{xh, rt, w, z};
           }
         }
+        if (w <= 8) break;  // (fewer at a time have no instance more)
       }
     }
   }

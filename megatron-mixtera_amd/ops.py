@@ -481,7 +481,7 @@ def update_requests(ctx, mask: Tensor, new_tokens_i64: Tensor) -> None:
     table = ctx.request_to_kv_chunk_ids
     _require(table.stride(1) == 1, "request_to_kv_chunk_ids rows must be contiguous")
     native = _native()
-    native.written_by_kernel(ctx._counters, table.device.index)
+    ctx._counters_stream = native.written_by_kernel(ctx._counters, table.device.index)
     update = native.abi_mi_update_requests if mask.dtype == torch.int32 else native.abi_mi_update_requests_mask8
     _lib.check(update(
         ctx.request_ids, ctx.request_query_lengths, ctx.request_output_lengths,
@@ -535,7 +535,7 @@ def step_attention_state(ctx, n_active_requests: int, padded_requests: int, padd
     padded token rows and the two maxima (into ``ctx._max_lengths``) in one launch."""
     table = ctx.request_to_kv_chunk_ids
     mirror = ctx.request_to_kv_chunk_ids_cudagraph_only
-    _native().written_by_kernel(ctx._max_lengths, table.device.index)
+    ctx._max_lengths_stream = _native().written_by_kernel(ctx._max_lengths, table.device.index)
     _lib.check(_native().abi_mi_step_attention_state(
         ctx.request_kv_length_offsets, ctx.request_query_lengths, table,
         table.stride(0), table.size(1), ctx.query_seq_lengths_cudagraph_only,
@@ -596,6 +596,6 @@ def attention_layer_decode(hidden: Tensor, qkv_weight: Tensor, qkv_bias: Optiona
 def linear_decode(x: Tensor, weight: Tensor, bias: Optional[Tensor] = None, out: Optional[Tensor] = None) -> Tensor:
     """``x @ weight.T (+ bias)`` for a decode-sized step (at most 256 rows of ``x``): the weight matrix streams from
     HBM once.  ``x`` is ``[..., K]`` (leading dimensions are flattened to rows), ``weight`` ``[N, K]``; the result
-    has ``x``'s leading dimensions and ``N`` columns; ``out`` may lie over ``x``.  What ``linear_qkv`` / ``linear_proj`` of the attention layer
-    compute at tensor-parallel size 1 (``mi_linear_decode`` of the header)."""
+    has ``x``'s leading dimensions and ``N`` columns; ``out`` may lie over ``x``.  What ``linear_qkv`` / ``linear_proj``
+    of the attention layer compute at tensor-parallel size 1 (``mi_linear_decode`` of the header)."""
     return _native().linear_decode(x, weight, bias, out, _override())
