@@ -14,6 +14,7 @@ import torch
 from torch import Tensor
 
 from . import ops
+from ._lib import native
 from .contexts.dynamic_context import DynamicInferenceContext
 from .flash_attn_interface import (
     flash_attn_varlen_func,
@@ -75,25 +76,6 @@ def _parameter(module: torch.nn.Module, name: str) -> Optional[Tensor]:
     return p if p is not None else getattr(module, name)
 
 
-def _own(obj, methods: tuple) -> bool:
-    """Whether ``methods`` (pairs of name and function as its class defines it) are what ``obj`` has -- none overridden in
-    a subclass, replaced on the class or on the object -- so that a call which does their work may stand in for them."""
-    kind, own = type(obj), obj.__dict__
-    for name, function in methods:
-        if name in own or getattr(kind, name) is not function:
-            return False
-    return True
-
-
-def _untouched(module: torch.nn.Module, cls: type, methods: tuple) -> bool:
-    """Whether ``module`` is a ``cls`` with its own ``methods`` and calling it runs nothing else (no hooks)."""
-    if type(module) is not cls:
-        return False
-    own = module.__dict__
-    return not (own["_forward_hooks"] or own["_forward_pre_hooks"] or own["_backward_hooks"] or own["_backward_pre_hooks"]
-                ) and _own(module, methods)
-
-
 class PagedSelfAttentionCore(torch.nn.Module):
     """Everything between ``get_query_key_value_tensors`` and ``linear_proj`` for one layer.
 
@@ -145,8 +127,8 @@ class PagedSelfAttentionCore(torch.nn.Module):
                 softmax_scale=self.softmax_scale, **self._norm_args())
             return out.reshape(out.size(0), out.size(1), -1)
         # (a step of prompts in one call of the context: in place of its append and of _attend below)
-        if (self.fused and isinstance(ctx, DynamicInferenceContext) and _own(self, _CORE_ATTEND)
-                and _own(ctx, _CONTEXT_PROMPTS)
+        if (self.fused and isinstance(ctx, DynamicInferenceContext) and native().as_defined(self, None, _CORE_ATTEND)
+                and native().as_defined(ctx, None, _CONTEXT_PROMPTS)
                 and ctx.prefill_fusable(mixed_qkv, self.head_dim, emb, _parameter(self, "q_layernorm_weight"),
                                         _parameter(self, "k_layernorm_weight"))):
             out = ctx.fused_prefill_attention(
@@ -281,10 +263,11 @@ class PagedSelfAttentionLayer(torch.nn.Module):
         """The output of a decode-only step by one native call, or ``None`` where the step takes the modules one by
         one: other steps, another kind of context, hooks on the parts, or a replaced method whose work the call does."""
         qkv, core, proj = self._modules["linear_qkv"], self._modules["core"], self._modules["linear_proj"]
-        n = hidden_states.size(0)
-        if (not isinstance(ctx, DynamicInferenceContext) or not ctx.is_decode_only() or not _own(ctx, _CONTEXT_STEP)
-                or not (_untouched(qkv, DecodeLinear, _LINEAR) and _untouched(proj, DecodeLinear, _LINEAR)
-                        and _untouched(core, PagedSelfAttentionCore, _CORE_MIXED))
+        if not isinstance(ctx, DynamicInferenceContext) or not ctx.is_decode_only():
+            return None
+        n, as_defined = hidden_states.size(0), native().as_defined
+        if (not (as_defined(qkv, DecodeLinear, _LINEAR) and as_defined(core, PagedSelfAttentionCore, _CORE_MIXED)
+                 and as_defined(proj, DecodeLinear, _LINEAR) and as_defined(ctx, None, _CONTEXT_STEP))
                 or torch.nn.modules.module._has_any_global_hook()
                 or not core.fused or n > min(qkv.DECODE_ROWS, proj.DECODE_ROWS) or n != ctx.padded_active_token_count
                 or hidden_states.dim() != 3 or hidden_states.size(1) != 1):
@@ -299,7 +282,7 @@ class PagedSelfAttentionLayer(torch.nn.Module):
             rotary_pos_emb=emb, softmax_scale=core.softmax_scale, **core._norm_args())
 
 
-# The methods that a fused call stands in for, as defined: see _own.
+# The methods that a fused call stands in for, as defined here: the call is not made where one of them was replaced.
 def _defined(cls: type, *names: str) -> tuple:
     return tuple((name, getattr(cls, name)) for name in names)
 

@@ -1076,6 +1076,41 @@ PyObject* written_by_kernel(PyObject* const* a) {
   return PyLong_FromLongLong(stream.id());
 }
 
+// as_defined(object, class|None, methods): whether `methods` (pairs of a name and the function its class defines) are what
+// the object has: none overridden in a subclass, replaced on the class or on the object.  With a class also whether the
+// object is one of exactly that class and, a torch module, has no hooks on its call.  (A decode step of a small batch asks
+// this of four objects in every layer: 1.9 us from Python.)
+PyObject* as_defined(PyObject* const* a) {
+  static PyObject* const hooks[4] = {
+      PyUnicode_InternFromString("_forward_hooks"), PyUnicode_InternFromString("_forward_pre_hooks"),
+      PyUnicode_InternFromString("_backward_hooks"), PyUnicode_InternFromString("_backward_pre_hooks")};
+  PyObject* const kind = (PyObject*)Py_TYPE(a[0]);
+  if (a[1] != Py_None && kind != a[1]) Py_RETURN_FALSE;
+  PyObject** const slot = _PyObject_GetDictPtr(a[0]);
+  PyObject* const own = slot ? *slot : nullptr;
+  REQUIRE(own && PyTuple_Check(a[2]), "as_defined takes an object with a dictionary and a tuple of pairs");
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(a[2]); ++i) {
+    PyObject* const pair = PyTuple_GET_ITEM(a[2], i);
+    REQUIRE(PyTuple_Check(pair) && PyTuple_GET_SIZE(pair) == 2, "as_defined takes pairs of a name and a function");
+    const int replaced = PyDict_Contains(own, PyTuple_GET_ITEM(pair, 0));
+    if (replaced < 0) throw PyFailure{};
+    if (replaced) Py_RETURN_FALSE;
+    PyObject* const function = PyObject_GetAttr(kind, PyTuple_GET_ITEM(pair, 0));
+    if (!function) throw PyFailure{};
+    Py_DECREF(function);  // (the class holds it)
+    if (function != PyTuple_GET_ITEM(pair, 1)) Py_RETURN_FALSE;
+  }
+  if (a[1] != Py_None)
+    for (PyObject* const name : hooks) {
+      PyObject* const set = PyDict_GetItemWithError(own, name);
+      if (!set && PyErr_Occurred()) throw PyFailure{};
+      const int any = set ? PyObject_IsTrue(set) : 0;
+      if (any < 0) throw PyFailure{};
+      if (any) Py_RETURN_FALSE;
+    }
+  Py_RETURN_TRUE;
+}
+
 // setup(kernel_error_class, raw_stream(device index), grow(device index, stream, bytes))
 PyObject* setup(PyObject* const* a) {
   for (int i = 0; i < 3; ++i) Py_INCREF(a[i]);
@@ -1104,7 +1139,7 @@ PyMethodDef kMethods[] = {
     OP(paged_prefill_attention, 14), OP(paged_prefill_attention_mla, 11), OP(norm_rope_append, 22), OP(qkv_norm_rope_append, 22), OP(qkv_key_append, 16),
     OP(qkv_prefill_attention, 18), OP(decode_step_attention, 29),
     OP(linear_decode, 5), OP(attention_layer_decode, 24), OP(sample_from_logits, 12), OP(selected_log_probs, 2), OP(last_token_gather, 3), OP(setup, 3),
-    OP(set_workspace, 3), OP(layer_views, 3), OP(watch, 4), OP(written_by_kernel, 2), {nullptr, nullptr, 0, nullptr}};
+    OP(set_workspace, 3), OP(layer_views, 3), OP(watch, 4), OP(written_by_kernel, 2), OP(as_defined, 3), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_native", "Host side of the per-layer calls.", -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace
