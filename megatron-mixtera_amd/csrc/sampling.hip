@@ -177,6 +177,13 @@ static __device__ __forceinline__ uint64_t mass_of(float x, float neg_mx_log2e) 
   return (uint64_t)(uint32_t)__builtin_fmaf(e, kMassOne, 0.5f);  // the conversion saturates
 }
 
+// Whether a row with this maximum has a distribution to draw from.  Not where it is not a finite number, and not where it
+// is so large (from some 4e8) that the rounding of the product with log2(e) leaves its own mass at nothing: a total of
+// zero would have no element to fall on.
+static __device__ __forceinline__ bool has_masses(float mx) {
+  return fabsf(mx) < INFINITY && mass_of(mx, -mx * 1.4426950408889634f) > 0;
+}
+
 // Adds weight() to hist[bin] for the active lanes (weight is only evaluated when some lane of the
 // wavefront is active).  When every active lane hits the same bin -- values clustered in one bin
 // would otherwise serialise 64 atomics on one address -- the wavefront adds its sum once.
@@ -384,8 +391,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleParams p) 
   int sample = bi;
   uint32_t cut_key = 0;  // keep everything
 
-  // A maximum that is not a finite number leaves no distribution to draw from: take the argmax.
-  const bool drawable = !greedy && fabsf(mx) < INFINITY;
+  const bool drawable = !greedy && has_masses(mx);   // (otherwise: the argmax)
   const float neg_mx = -mx * 1.4426950408889634f;
   if (drawable) {
     const bool by_count = p.top_k > 1;
@@ -863,7 +869,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_mass_kernel(SplitParams
   const int part = blockIdx.x, r = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const RowMax m = row_max(p, r, lane);
   const float mx = order_key_value(m.key), neg_mx = -mx * 1.4426950408889634f;
-  if (!(fabsf(mx) < INFINITY)) return;
+  if (!has_masses(mx)) return;
   const auto rd = row_reader<DT, VEC>(p.s, r);
   const int64_t row_part = (int64_t)r * p.parts + part;
   const bool filtered = p.s.top_p > 0.f;
@@ -953,7 +959,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SplitParams
   const uint64_t run0 = p.s.top_k == 0 && tid < n_runs ? p.run_mass[row * kRuns + tid] : 0;
   const RowMax m = row_max(p, r, lane);
   const float mx = order_key_value(m.key), neg_mx = -mx * 1.4426950408889634f;
-  if (p.s.top_k == 1 || !(fabsf(mx) < INFINITY)) {
+  if (p.s.top_k == 1 || !has_masses(mx)) {
     if (tid == 0) write_sample(p.s, r, m.idx, 0);
     return;
   }
@@ -1089,6 +1095,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SplitParams
   }
   __syncthreads();
   // ---- the run the uniform number falls into: every thread owns one (there are at most 1 024) ----
+  if (tid == 0) res[0] = res[1] = 0;   // (a run of the row, whatever the masses)
   const uint64_t mine = runs[tid];
   uint64_t incl = wave_scan_incl_u64(mine, lane);
   if (lane == 63) wsum[0][wave] = incl;

@@ -440,6 +440,19 @@ def test_rows_in_parts_equal_rows_by_one_workgroup(mi, dev, R, V, kind):
             assert torch.equal(cut, want_cut), (dtype, top_k, top_p)
 
 
+@pytest.mark.parametrize("V", [1000, 16387, 80001])
+@pytest.mark.parametrize("mode", [dict(top_p=0.3), dict(top_p=0.9), dict(), dict(top_k=5)])
+def test_logits_too_large_for_masses_take_the_argmax(mi, dev, V, mode):
+    """From some 4e8 on, the product with log2(e) rounds by more than the exponent's range and the maximum's own mass may be
+    zero: such rows have no distribution, and no element that a uniform number could fall on."""
+    g = torch.Generator().manual_seed(V)
+    x = (torch.randn(8, V, generator=g) * 1e30).to(dev)
+    u = torch.rand(8, generator=g).to(dev)
+    got, _ = mi.ops.sample_from_logits(x, uniform=u, temperature=0.7, **mode)
+    kept = (x * (1 / 0.7)).amax(-1, keepdim=True) * (1 - 1e-6)   # (a maximum with a mass: itself and what rounds with it)
+    assert (x.gather(1, got[:, None]) * (1 / 0.7) >= kept).all()
+
+
 @pytest.mark.parametrize("buffer", ["whole", "off a line", "too small", "on the host", "empty"])
 def test_sampling_inside_use_workspace(mi, dev, buffer):
     """A buffer for attention's scratch that does not serve the parts of the rows is passed over, not refused."""
