@@ -66,12 +66,45 @@ static __device__ __forceinline__ uint64_t wave_scan_incl_u64(uint64_t v, int /*
   v += dpp_u64<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
   return v;
 }
+template <int CTRL, int ROW_MASK>
+static __device__ __forceinline__ float dpp_f32(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROW_MASK, 0xF, false));
+}
+static __device__ __forceinline__ float wave_scan_incl_f32(float v) {
+  v += dpp_f32<0x111, 0xF>(v);
+  v += dpp_f32<0x112, 0xF>(v);
+  v += dpp_f32<0x114, 0xF>(v);
+  v += dpp_f32<0x118, 0xF>(v);
+  v += dpp_f32<0x142, 0xA>(v);
+  v += dpp_f32<0x143, 0xC>(v);
+  return v;
+}
 // Sum over the 64 lanes, in every lane: the scan above, then its last lane's value.
 static __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
   v = wave_scan_incl_u64(v, 0);
   const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, 63);
   const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), 63);
   return ((uint64_t)hi << 32) | lo;
+}
+
+// Largest of the 64 lanes' values, in every lane, by the same moves.
+template <int CTRL, int ROW_MASK>
+static __device__ __forceinline__ uint32_t dpp_max_u32(uint32_t v) {
+  return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROW_MASK, 0xF, false));
+}
+static __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+  v = dpp_max_u32<0x111, 0xF>(v);
+  v = dpp_max_u32<0x112, 0xF>(v);
+  v = dpp_max_u32<0x114, 0xF>(v);
+  v = dpp_max_u32<0x118, 0xF>(v);
+  v = dpp_max_u32<0x142, 0xA>(v);
+  v = dpp_max_u32<0x143, 0xC>(v);
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// fp32 -> uint32, truncating: NaN and everything below 0 become 0, everything too large 2^32 - 1.
+static __device__ __forceinline__ uint32_t f32_to_u32_sat(float x) {
+  return (uint32_t)fmaxf(x, 0.f);   // (the conversion saturates)
 }
 
 // One row of logits.  DT = element type (0 fp32, 1 bf16, 2 fp16); VEC = elements per 16-byte load (4 fp32,
@@ -88,10 +121,17 @@ struct RowReader {
     }
     return x + 0.0f;
   }
+  // the same with a -0 left as it is, and fp32 multiplied by one where nothing is scaled
+  __device__ __forceinline__ float scaled(float x) const {
+    if (DT == 0 || scale) x *= inv_t;
+    if (DT != 0 && scale) x = to_f32<DT == 2>(f32_to_16<DT == 2>(x));
+    return x;
+  }
   __device__ __forceinline__ float at(int i) const {
     return finish(DT != 0 ? to_f32<DT == 2>(reinterpret_cast<const uint16_t*>(row)[i]) : reinterpret_cast<const float*>(row)[i]);
   }
-  // elements i0 .. i0+VEC-1 (i0 a multiple of VEC), all inside the row
+  // elements i0 .. i0+VEC-1 (i0 a multiple of VEC), all inside the row; ZERO = false: a -0 stays one
+  template <bool ZERO = true>
   __device__ __forceinline__ void load_full(int i0, float (&x)[VEC]) const {
     if (VEC > 1) {
       const uint4 w = ld16(row + (int64_t)i0 * (DT != 0 ? 2 : 4));
@@ -101,7 +141,7 @@ struct RowReader {
         float v;
         if (DT != 0) v = (j & 1) ? hi_to_f32<DT == 2>(u[(j >> 1) & 3]) : lo_to_f32<DT == 2>(u[(j >> 1) & 3]);
         else v = __uint_as_float(u[j & 3]);
-        x[j] = finish(v);
+        x[j] = ZERO ? finish(v) : scaled(v);
       }
     } else {
       x[0] = at(i0);
@@ -169,12 +209,44 @@ static __device__ __forceinline__ void sweep(const RowReader<DT, VEC>& rd, int b
   }
 }
 
+// A thread's next BATCH values of [base, end): U groups of VEC, `nthreads` threads side by side (this one is `t`), all
+// loads in flight together; -inf at and past `end`, and zeros of either sign.  base % VEC == 0, and end is a multiple of VEC
+// or the row's end.
+template <int BATCH, int DT, int VEC>
+static __device__ __forceinline__ void load_batch(const RowReader<DT, VEC>& rd, int base, int end, int t, int nthreads,
+                                                  float (&x)[BATCH / VEC][VEC]) {
+  constexpr int U = BATCH / VEC;
+  const int stride = nthreads * VEC;
+  const int row_end = rd.V - (rd.V % VEC);  // whole groups of the row end here (there is one)
+  if (base + U * stride <= min(end, row_end)) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) rd.template load_full<false>(base + u * stride + t * VEC, x[u]);
+  } else {  // (loads without a branch around them, so that they too are in flight together)
+#pragma unroll
+    for (int u = 0; u < U; ++u) rd.template load_full<false>(min(base + u * stride + t * VEC, row_end - VEC), x[u]);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i0 = base + u * stride + t * VEC;
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) x[u][j] = i0 < min(end, row_end) ? x[u][j] : -INFINITY;
+    }
+    if (VEC > 1 && end > row_end) {  // the row's last values, fewer than a group: one thread's
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (base + u * stride + t * VEC == row_end) {
+#pragma unroll
+          for (int j = 0; j < VEC - 1; ++j)
+            if (row_end + j < end) x[u][j] = rd.at(row_end + j);
+        }
+    }
+  }
+}
+
 // exp(x - mx) as fixed point, rounded to the nearest 2^-32: one 32-bit conversion per element
 // (sums are carried in 64 bits).  0 for anything that is not a number at or below the maximum.
 constexpr float kMassOne = 4294967040.0f;  // largest fp32 below 2^32
 static __device__ __forceinline__ uint64_t mass_of(float x, float neg_mx_log2e) {
-  const float e = fmaxf(fast_exp2(__builtin_fmaf(x, 1.4426950408889634f, neg_mx_log2e)), 0.f);  // NaN -> 0
-  return (uint64_t)(uint32_t)__builtin_fmaf(e, kMassOne, 0.5f);  // the conversion saturates
+  return f32_to_u32_sat(__builtin_fmaf(fast_exp2(__builtin_fmaf(x, 1.4426950408889634f, neg_mx_log2e)), kMassOne, 0.5f));
 }
 
 // Whether a row with this maximum has a distribution to draw from.  Not where it is not a finite number, and not where it
@@ -661,9 +733,9 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleParams p) 
 // One workgroup per row leaves most of the chip idle while it walks the row up to five times (64 rows: 64 of 256 CUs;
 // 64 x 128 256 fp32, top-p 0.9 on flat rows: 105 us against 5 us for one read).  Here a row is cut into parts of one
 // workgroup each, and the walk into launches that read the parts once each:
-//   sample_first_kernel : a part's maximum (with its index); top-p: the part's mass in bins, in fp32 below a reference
-//                         that all parts of a row share; top-k: the part's candidates, listed (the elements at or above
-//                         a threshold estimated from 1 024 of them);
+//   sample_first_kernel : a part's maximum (with its index); top-p: the part's mass in bins of 1/64, counted down from the
+//                         bin of its maximum on a grid that all parts share; top-k: the part's candidates, listed (the
+//                         elements at or above a threshold estimated from 1 024 of them);
 //   sample_mass_kernel  : (top-p and plain draws) the exact masses: the part's total, and per run of elements what lies
 //                         above the bins that hold the cut; the elements in those bins, listed;
 //   sample_pick_kernel  : one workgroup per row: the exact cut among the listed elements, the run of elements the
@@ -673,12 +745,17 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleParams p) 
 // more than the list holds) its workgroup walks the row instead of the list.
 //
 // fp32, 128 256 wide, us per call, one workgroup per row -> parts:
-//   64 rows: greedy 15 -> 12, plain 38 -> 24, top-k 50 39 -> 31, top-p 0.9 105 -> 44 (flat rows), 54 -> 41 (peaked)
-//    1 row : greedy 13 ->  8, plain 35 -> 15, top-k 50 36 -> 18, top-p 0.9 101 -> 25 (flat rows), 51 -> 24 (peaked)
-// 64 rows, top-p: 18 us for the first walk (38 vector instructions per 64 elements by counter, the pipe half busy), 15
-// for the second, 11 for the pick (a chain of loads and barriers).
-constexpr int kBins = kSampleThreads; // 1/16 wide, from 24 above the reference to 40 below (and all that is lower)
-constexpr float kBinsAbove = 24.f, kBinsPerUnit = 16.f;
+//   64 rows: greedy 15 -> 11, plain 38 -> 21, top-k 50 39 -> 30, top-p 0.9 105 -> 27 (flat rows), 54 -> 26 (peaked)
+//    1 row : greedy 13 ->  7, plain 35 -> 13, top-k 50 36 -> 18, top-p 0.9 101 -> 21 (flat rows), 51 -> 20 (peaked)
+// 64 rows, top-p, by trace: 8.4 us for the first walk, 10.6-11.4 for the second, 8.2 for the pick (a chain of loads and
+// barriers).  Both walks are vector arithmetic and one burst of loads: what they gained (18.3, 14.6 and 11.1 us) is fewer
+// instructions per value.  The first took 38, with bins below a sampled reference, an exponential and a 64-bit addition to
+// LDS per value; with the batch in registers its own maximum is the reference, a 32-bit weight within the bin does, and
+// bins a quarter as wide leave a third of the values on the lists.  The second claimed its place on the list for one value
+// of each lane at a time and held the window's comparison against bins; 1.6 of its time are lists, 1.5 what is kept, 1
+// the masses, 3 the bins of the other parts.
+constexpr int kBins = 2048;           // of 1/64, from the bin of the largest value down (all that is lower: none)
+constexpr float kBinsPerUnit = 64.f;
 constexpr int kRuns = kSampleWaves;   // runs of elements per part
 constexpr int kMaxParts = 64;
 constexpr int kPartSample = 1024;
@@ -688,9 +765,10 @@ struct SplitParams {
   int32_t parts, part_len, run_len;    // elements (multiples of 8); a part is kRuns runs
   int32_t list_cap;                    // listed elements per part
   uint32_t* part_key; int32_t* part_idx;  // [R][parts] maximum
-  uint32_t* part_tau;                  // [R][parts] top-k: the threshold of the part's candidates; top-p: the bins' upper edge
+  uint32_t* part_tau;                  // [R][parts] top-k: the threshold of the part's candidates; top-p: its first bin's number
   uint32_t* part_listed;               // [R][parts]
-  float* bins;                         // [R][parts][kBins]
+  uint32_t* bins;                      // [R][parts][kBins]: sums of exp(x - the bin's upper edge), in units of 1 / bin_one
+  float bin_one;                       // (a row of equal values stays below 2^32)
   uint64_t* part_mass;                 // [R][parts] exact total
   uint64_t* run_mass;                  // [R][parts][kRuns] exact mass above the listed bins
   uint2* list;                         // [R][parts][list_cap]: key, vocabulary index
@@ -710,36 +788,11 @@ static __device__ __forceinline__ RowMax row_max(const SplitParams& p, int r, in
     const int64_t at = (int64_t)r * p.parts + lane;
     m = RowMax{p.part_key[at], p.part_idx[at]};
   }
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) {
-    const uint32_t ok = __shfl_xor(m.key, d, 64); const int oi = __shfl_xor(m.idx, d, 64);
-    if (ok > m.key || (ok == m.key && oi < m.idx)) { m.key = ok; m.idx = oi; }
-  }
+  const uint32_t key = wave_max_u32(m.key);
+  m.idx = (int32_t)~wave_max_u32(m.key == key ? ~(uint32_t)m.idx : 0);  // (the lowest of the indices)
+  m.key = key;
   if (m.idx >= p.s.V) m.idx = 0;  // only when no element compared greater than the start value
   return m;
-}
-
-// The bin of a value, 0 = largest values; monotone.
-static __device__ __forceinline__ int ref_bin(float x, float top) {
-  const float f = (top - x) * kBinsPerUnit;
-  const int b = f >= (float)(kBins - 1) ? kBins - 1 : (int)f;  // NaN compares false and converts to 0
-  return b < 0 ? 0 : b;
-}
-// The upper edge of the bins: the reference -- the largest finite one of 1 024 elements spread over the row, the same
-// ones for every part -- plus 24.
-template <int DT, int VEC>
-static __device__ __forceinline__ float bins_top(const RowReader<DT, VEC>& rd, float* red, int tid, int lane, int wave) {
-  const int step = rd.V / kSampleThreads;
-  const float x = rd.at(tid * step);
-  float m = fabsf(x) < INFINITY ? x : -3.0e38f;
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) m = fmaxf(m, __shfl_xor(m, d, 64));
-  if (lane == 0) red[wave] = m;
-  __syncthreads();
-  m = red[0];
-#pragma unroll
-  for (int w = 1; w < kSampleWaves; ++w) m = fmaxf(m, red[w]);
-  return m + kBinsAbove;
 }
 
 // Appends one element per lane with `in` set to a list of `cap` entries; `count` goes on counting past it.
@@ -757,12 +810,11 @@ static __device__ __forceinline__ void list_append(uint32_t* count, uint32_t cap
 
 enum { kPickMax = 0, kPickTopK = 1, kPickTopP = 2 };
 
-template <int DT, int VEC, int MODE>
+template <int DT, int VEC, int MODE, int BATCH>
 __global__ __launch_bounds__(kSampleThreads) void sample_first_kernel(SplitParams p) {
   __shared__ uint32_t red_key[kSampleWaves];
   __shared__ int32_t red_idx[kSampleWaves];
-  __shared__ float red[kSampleWaves], red_low[kSampleWaves];
-  __shared__ uint64_t mass[MODE == kPickTopP ? kBins : 1];
+  __shared__ uint32_t mass[MODE == kPickTopP ? kBins : 1];
   __shared__ uint32_t sampled[MODE == kPickTopK ? kPartSample : 1];
   __shared__ uint64_t hist[MODE == kPickTopK ? 256 : 1];
   __shared__ uint64_t res[2];
@@ -772,7 +824,6 @@ __global__ __launch_bounds__(kSampleThreads) void sample_first_kernel(SplitParam
   const int a = min(part * p.part_len, p.s.V), b = min(a + p.part_len, p.s.V);
   const int64_t row_part = (int64_t)r * p.parts + part;
   uint32_t tau = 0;
-  float top = 0.f;
   if (MODE == kPickTopK) {
     // threshold: a rank of the sample that leaves three times this part's share of the top k above it, and twelve
     // of the sample at least (a dozen of it stand for 8-20 of the same spacing in all but a few of 10^5 parts)
@@ -804,29 +855,75 @@ __global__ __launch_bounds__(kSampleThreads) void sample_first_kernel(SplitParam
       tau |= (255u - (uint32_t)res[0]) << (8 * d);
     }
   }
-  if (MODE == kPickTopP) {
-    mass[tid] = 0;
-    top = bins_top(rd, red, tid, lane, wave);  // (has the barrier)
-  }
-  const float ref_log2 = 26.f - (top - kBinsAbove) * 1.4426950408889634f;
   uint2* list = p.list + row_part * p.list_cap;
   uint32_t bk = 0; int bi = 0x7fffffff;
-  float low = 0.f;   // the last bin's: below it lies most of a flat row, and one address would take it all in turn
+  bool indexed = true;
+  if (MODE == kPickTopP) {
+    // A batch lies in registers while its maximum is found, then goes into bins counted down from the bin of the largest
+    // value so far; where that moves up, the bins move with it.
+    static_assert(kBins == 2 * kSampleThreads, "two bins per thread");
+    float first = -INFINITY;          // number of the first bin: floor(64 x) of the largest value
+    mass[tid] = mass[tid + kSampleThreads] = 0;
+    for (int base = a; base < b; base += BATCH * kSampleThreads) {
+      float x[BATCH / VEC][VEC];
+      load_batch<BATCH>(rd, base, b, tid, kSampleThreads, x);
+      // as integers, numbers from +0 up are in order, NaN above them; among values below 0 the floats' order counts
+      int32_t top_i = INT32_MIN;
+      float top_f = -INFINITY;
+#pragma unroll
+      for (int u = 0; u < BATCH / VEC; ++u)
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) {
+          top_i = max(top_i, __float_as_int(x[u][j]));
+          top_f = fmaxf(top_f, x[u][j]);
+        }
+      bk = max(bk, top_i >= 0 ? (uint32_t)top_i | 0x80000000u : order_key(top_f + 0.f));
+      bk = wave_max_u32(bk);
+      __syncthreads();   // (the batch before has been read and counted)
+      if (lane == 0) red_key[wave] = bk;
+      __syncthreads();
+#pragma unroll
+      for (int w = 0; w < kSampleWaves; ++w) bk = max(bk, red_key[w]);
+      const float now = floorf(order_key_value(bk) * kBinsPerUnit);
+      if (now > first) {
+        if (base > a) {
+          const int by = (int)fminf(now - first, (float)kBins), i0 = tid - by, i1 = i0 + kSampleThreads;
+          const uint32_t m0 = i0 >= 0 ? mass[i0] : 0, m1 = i1 >= 0 ? mass[i1] : 0;
+          __syncthreads();
+          mass[tid] = m0;
+          mass[tid + kSampleThreads] = m1;
+          __syncthreads();
+        }
+        first = now;
+      }
+      const float edge = first + 1.f;
+#pragma unroll
+      for (int u = 0; u < BATCH / VEC; ++u)
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) {
+          // distance from the first bin's upper edge, in bins; exp(-t / 64) by its chord, lowered to within 1.6e-5
+          const float f = __builtin_fmaf(x[u][j], -kBinsPerUnit, edge);
+          const uint32_t bin = f32_to_u32_sat(f);
+          const float w = __builtin_fmaf(__builtin_amdgcn_fractf(f), -0.01550356f * p.bin_one, 0.99998474f * p.bin_one);
+          if (bin < (uint32_t)kBins) atomicAdd(&mass[bin], f32_to_u32_sat(w));
+        }
+    }
+    // The index matters where there may be nothing to draw from: no finite maximum (that of a part of nothing but -inf and
+    // NaN was not found), or one so large that its own mass may round to nothing.
+    indexed = !(fabsf(order_key_value(bk)) < 1e6f);
+    __syncthreads();
+    reinterpret_cast<uint2*>(p.bins + row_part * kBins)[tid] = make_uint2(mass[2 * tid], mass[2 * tid + 1]);
+    if (tid == 0) p.part_tau[row_part] = __float_as_uint(first);
+    if (!indexed) {
+      if (tid == 0) { p.part_key[row_part] = bk; p.part_idx[row_part] = a; p.part_listed[row_part] = 0; }
+      return;
+    }
+    bk = 0;
+  }
   sweep<(VEC == 8 ? 4 : 8)>(rd, a, b, tid, kSampleThreads, [&](int i, float x, bool in) {
     const uint32_t k = order_key(x);
     const bool up = in && k > bk;
     bk = up ? k : bk; bi = up ? i : bi;
-    if (MODE == kPickTopP && in) {
-      // in units of 2^-26 of the reference's (64-bit integer adds: LDS adds of fp32 ran at a fifth of their rate)
-      const float e = fast_exp2(fminf(__builtin_fmaf(x, 1.4426950408889634f, ref_log2), 62.f)) + 0.5f;
-      const int bin = ref_bin(x, top);
-      if (bin == kBins - 1) {
-        low += e;
-      } else {
-        const uint32_t hi = (uint32_t)(e * 0x1p-32f), lo = (uint32_t)__builtin_fmaf((float)hi, -0x1p32f, e);
-        atomicAdd(reinterpret_cast<unsigned long long*>(&mass[bin]), ((unsigned long long)hi << 32) | lo);
-      }
-    }
     if (MODE == kPickTopK)
       list_append(&listed, (uint32_t)p.list_cap, in && k >= tau, lane, [&](uint32_t at) { list[at] = make_uint2(k, (uint32_t)i); });
   });
@@ -835,19 +932,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_first_kernel(SplitParam
     const uint32_t ok = __shfl_xor(bk, m, 64); const int oi = __shfl_xor(bi, m, 64);
     if (ok > bk || (ok == bk && oi < bi)) { bk = ok; bi = oi; }
   }
-  if (MODE == kPickTopP) {
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) low += __shfl_xor(low, m, 64);
-    if (lane == 0) red_low[wave] = low;
-  }
   if (lane == 0) { red_key[wave] = bk; red_idx[wave] = bi; }
   __syncthreads();
-  if (MODE == kPickTopP) {
-    float v = (float)mass[tid];
-    if (tid == kBins - 1)
-      for (int w = 0; w < kSampleWaves; ++w) v += red_low[w];
-    p.bins[row_part * kBins + tid] = v;
-  }
   if (tid == 0) {
     for (int w = 1; w < kSampleWaves; ++w) {
       const uint32_t ok = red_key[w]; const int oi = red_idx[w];
@@ -855,42 +941,81 @@ __global__ __launch_bounds__(kSampleThreads) void sample_first_kernel(SplitParam
     }
     p.part_key[row_part] = bk; p.part_idx[row_part] = bi;
     p.part_listed[row_part] = MODE == kPickTopK ? listed : 0;
-    p.part_tau[row_part] = MODE == kPickTopK ? tau : __float_as_uint(top);
+    if (MODE == kPickTopK) p.part_tau[row_part] = tau;
   }
 }
 
-// Exact masses.  top-p lists the bins [lo, hi] around the estimated cut; a plain draw (lo = kBins) lists nothing.
-template <int DT, int VEC>
+// Exact masses.  top-p lists the values in the bins around the estimated cut; a plain draw lists nothing.
+template <int DT, int VEC, int BATCH>
 __global__ __launch_bounds__(kSampleThreads) void sample_mass_kernel(SplitParams p) {
   __shared__ float red[kSampleWaves];
   __shared__ int32_t window[2];
   __shared__ uint64_t wsum[kSampleWaves];
   __shared__ uint32_t listed;
+  __shared__ uint32_t row_bins[kBins];
   const int part = blockIdx.x, r = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const RowMax m = row_max(p, r, lane);
-  const float mx = order_key_value(m.key), neg_mx = -mx * 1.4426950408889634f;
-  if (!has_masses(mx)) return;
   const auto rd = row_reader<DT, VEC>(p.s, r);
-  const int64_t row_part = (int64_t)r * p.parts + part;
+  const int pa = part * p.part_len, a = min(pa + wave * p.run_len, p.s.V), b = min(min(a + p.run_len, pa + p.part_len), p.s.V);
+  const int64_t row = (int64_t)r * p.parts, row_part = row + part;
   const bool filtered = p.s.top_p > 0.f;
-  float top = 0.f;
-  int lo = kBins, hi = kBins;
+  // (the first batch and the first parts' bins set out before anything is waited for)
+  float x[BATCH / VEC][VEC];
+  load_batch<BATCH>(rd, a, b, lane, 64, x);
+  // (256 bins of one part at a time per wavefront)
+  constexpr int kItems = kBins / 256, kFirstItems = 2;
+  uint4 first_items[kFirstItems];
+  const uint4* const bins_src = reinterpret_cast<const uint4*>(p.bins + row * kBins) + lane;
+  const int n_items = filtered ? p.parts * kItems : 0;
   if (filtered) {
-    top = __uint_as_float(p.part_tau[row_part]);
-    // one bin per thread; the bin in which the running sum passes top_p of the total, with a neighbour where it passes
-    // within 3e-4 of the total of the edge
-    float h = 0.f;
-    const float* src = p.bins + (int64_t)r * p.parts * kBins + tid;
-#pragma unroll 4
-    for (int g = 0; g < p.parts; ++g) h += src[(int64_t)g * kBins];
-    float incl = h;
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const float v = __shfl_up(incl, d, 64);
-      incl += lane >= d ? v : 0.f;
+    for (int n = 0; n < kFirstItems; ++n)
+      first_items[n] = bins_src[64 * min(wave + n * kSampleWaves, n_items - 1)];
+    row_bins[tid] = row_bins[tid + kSampleThreads] = 0;
+  }
+  const uint32_t part_key = lane < p.parts ? p.part_key[row + lane] : 0;
+  float first = lane < p.parts && filtered ? __uint_as_float(p.part_tau[row + lane]) : -INFINITY;
+  const float mx = order_key_value(wave_max_u32(part_key)), neg_mx = -mx * 1.4426950408889634f;
+  if (!has_masses(mx)) return;
+  if (tid == 0) { window[0] = kBins; window[1] = -1; listed = 0; }
+  const float row_first = floorf(mx * kBinsPerUnit);
+  const int down = (int)fminf(row_first - first, (float)kBins);   // by how many bins each part's begin below the row's
+  uint64_t all = 0, kept = 0;
+  auto masses = [&] {
+#pragma unroll
+    for (int u = 0; u < BATCH / VEC; ++u)
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) all += mass_of(x[u][j], neg_mx);
+  };
+  masses();
+  float over = INFINITY, from = INFINITY;   // kept: above `over`; listed: from `from` to `over`
+  if (filtered) {
+    // The parts' bins on the row's scale, two per thread; the bin in which the running sum passes top_p of the total, with
+    // its neighbours where it passes within 1e-4 of the total of the edge (the sums are off by a few 1e-5).
+    auto add_item = [&](int n, uint4 c) {
+      const int at = 256 * (n % kItems) + 4 * lane + __builtin_amdgcn_readlane(down, n / kItems);
+      const uint32_t v[4] = {c.x, c.y, c.z, c.w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (at + j < kBins && v[j]) atomicAdd(&row_bins[at + j], v[j]);
+    };
+    __syncthreads();   // (the bins are cleared)
+#pragma unroll
+    for (int n = 0; n < kFirstItems; ++n)
+      if (wave + n * kSampleWaves < n_items) add_item(wave + n * kSampleWaves, first_items[n]);
+    for (int n0 = wave + kFirstItems * kSampleWaves; n0 < n_items; n0 += 8 * kSampleWaves) {
+      uint4 c[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) c[i] = bins_src[64 * min(n0 + i * kSampleWaves, n_items - 1)];
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (n0 + i * kSampleWaves < n_items) add_item(n0 + i * kSampleWaves, c[i]);
     }
+    __syncthreads();
+    const float h0 = (float)row_bins[2 * tid] * fast_exp2((float)(2 * tid) * (-1.4426950408889634f / kBinsPerUnit));
+    const float h1 = (float)row_bins[2 * tid + 1] * fast_exp2((float)(2 * tid + 1) * (-1.4426950408889634f / kBinsPerUnit));
+    const float h = h0 + h1;
+    float incl = wave_scan_incl_f32(h);
     if (lane == 63) red[wave] = incl;
-    if (tid == 0) { window[0] = kBins - 1; window[1] = 0; listed = 0; }
     __syncthreads();
     float total = 0.f;
 #pragma unroll
@@ -898,31 +1023,64 @@ __global__ __launch_bounds__(kSampleThreads) void sample_mass_kernel(SplitParams
       incl += w < wave ? red[w] : 0.f;
       total += red[w];
     }
-    const float want = p.s.top_p * total, slack = 3e-4f * total;
-    if (incl - h - slack <= want && incl + slack > want && h > 0.f) {
-      atomicMin(&window[0], tid);
-      atomicMax(&window[1], tid);
+    const float want = p.s.top_p * total, slack = 1e-4f * total;
+    const bool in0 = incl - h - slack <= want && incl - h1 + slack > want && h0 > 0.f;
+    const bool in1 = incl - h1 - slack <= want && incl + slack > want && h1 > 0.f;
+    if (in0 || in1) {
+      atomicMin(&window[0], in0 ? 2 * tid : 2 * tid + 1);
+      atomicMax(&window[1], in1 ? 2 * tid + 1 : 2 * tid);
     }
     __syncthreads();
-    lo = window[0]; hi = window[1];
-    if (lo > hi) lo = hi = kBins;   // nothing found (not a number somewhere): the pick walks the row
+    const int lo = window[0], hi = window[1];
+    if (lo <= hi) {   // (nothing found, as where a value is not a number: nothing is listed, and the pick walks the row)
+      over = (row_first + 1.f - (float)lo) * (1.f / kBinsPerUnit);
+      from = (row_first - (float)hi) * (1.f / kBinsPerUnit);
+    }
   } else {
-    if (tid == 0) listed = 0;
     __syncthreads();
   }
-  const int pa = part * p.part_len, a = min(pa + wave * p.run_len, p.s.V), b = min(min(a + p.run_len, pa + p.part_len), p.s.V);
   uint2* list = p.list + row_part * p.list_cap;
-  uint64_t all = 0, kept = 0;
-  sweep<(VEC == 8 ? 4 : 8)>(rd, a, b, lane, 64, [&](int i, float x, bool in) {
-    const uint64_t w = in ? mass_of(x, neg_mx) : 0;
-    all += w;
-    if (filtered) {
-      const int bin = ref_bin(x, top);
-      kept += bin < lo ? w : 0;
-      list_append(&listed, (uint32_t)p.list_cap, in && bin >= lo && bin <= hi, lane,
-                  [&](uint32_t at) { list[at] = make_uint2(order_key(x), (uint32_t)i); });
+  for (int base = a; base < b;) {
+    if (filtered) {   // one claim on the list for sixteen values a lane
+      constexpr int HALF = BATCH / 2;
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        uint64_t in_window[HALF];
+        uint32_t found = 0;
+#pragma unroll
+        for (int n = 0; n < HALF; ++n) {
+          const float v = x[(half * HALF + n) / VEC][(half * HALF + n) % VEC];
+          uint64_t m = __builtin_amdgcn_ballot_w64(v >= from);
+          if (m) {   // (few values are: their mass again is less than holding it)
+            const bool is_over = v > over;
+            kept += is_over ? mass_of(v, neg_mx) : 0;
+            m &= ~__builtin_amdgcn_ballot_w64(is_over);
+            found += (uint32_t)__builtin_popcountll(m);
+          }
+          in_window[n] = m;
+        }
+        if (found == 0) continue;
+        uint32_t at = 0;
+        if (lane == 0) at = atomicAdd(&listed, found);
+        at = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+        for (int n = 0; n < HALF; ++n) {
+          const uint64_t m = in_window[n];
+          if (m == 0) continue;
+          const int u = (half * HALF + n) / VEC, j = (half * HALF + n) % VEC;
+          const uint32_t mine = at + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+          if (((m >> lane) & 1) && mine < (uint32_t)p.list_cap)
+            list[mine] = make_uint2(order_key(x[u][j] + 0.f), (uint32_t)(base + (u * 64 + lane) * VEC + j));
+          at += (uint32_t)__builtin_popcountll(m);
+        }
+      }
     }
-  });
+    base += BATCH * 64;
+    if (base < b) {
+      load_batch<BATCH>(rd, base, b, lane, 64, x);
+      masses();
+    }
+  }
   all = wave_sum_u64(all);
   kept = filtered ? wave_sum_u64(kept) : all;
   if (lane == 0) {
@@ -1315,7 +1473,10 @@ static int64_t sample_layout(SplitParams* p, uint8_t* base, int R, int V, int to
   if (parts > 4) p->list_cap = kMemberCap / 4;
   p->part_key = (uint32_t*)take(4 * n); p->part_idx = (int32_t*)take(4 * n);
   p->part_tau = (uint32_t*)take(4 * n); p->part_listed = (uint32_t*)take(4 * n);
-  p->bins = (float*)take(by_mass ? n * kBins * 4 : 0);
+  p->bins = (uint32_t*)take(by_mass ? n * kBins * 4 : 0);
+  int bits = 0;
+  while (bits < 30 && (V >> bits) > 1) ++bits;   // V < 2^(bits + 1)
+  p->bin_one = (float)(1u << (31 - bits > 16 ? 16 : 31 - bits));
   p->part_mass = (uint64_t*)take(draws && !by_count ? n * 8 : 0);
   p->run_mass = (uint64_t*)take(draws && !by_count ? n * kRuns * 8 : 0);
   p->list = (uint2*)take(by_count || by_mass ? n * p->list_cap * 8 : 0);
@@ -1329,10 +1490,21 @@ static void launch_sample(const SampleParams& s, SplitParams* split, hipStream_t
     return;
   }
   const dim3 grid(split->parts, s.R), block(kSampleThreads);
-  if (s.top_k > 1) hipLaunchKernelGGL((sample_first_kernel<DT, VEC, kPickTopK>), grid, block, 0, st, *split);
-  else if (s.top_k == 0 && s.top_p > 0.f) hipLaunchKernelGGL((sample_first_kernel<DT, VEC, kPickTopP>), grid, block, 0, st, *split);
-  else hipLaunchKernelGGL((sample_first_kernel<DT, VEC, kPickMax>), grid, block, 0, st, *split);
-  if (s.top_k == 0) hipLaunchKernelGGL((sample_mass_kernel<DT, VEC>), grid, block, 0, st, *split);
+  // Values a thread holds at a time: short runs (many parts per row) have few, and what is loaded past their end is worked
+  // on all the same (2 x 138 767 bf16, top-p: 27.0 us with 32, 20.9 with 8; 64 x 128 256 fp32: a second batch costs 3).
+  // Rows off 16 bytes load value by value: 32 of them spill.
+  constexpr int kLarge = VEC == 1 ? 16 : 32, kSmall = 8;
+  const bool small = split->run_len <= 64 * kSmall;
+#define MI_PARTS_LAUNCH(K_, ...)                                                          \
+  do {                                                                                    \
+    if (small) hipLaunchKernelGGL((K_<__VA_ARGS__, kSmall>), grid, block, 0, st, *split); \
+    else hipLaunchKernelGGL((K_<__VA_ARGS__, kLarge>), grid, block, 0, st, *split);       \
+  } while (0)
+  if (s.top_k > 1) hipLaunchKernelGGL((sample_first_kernel<DT, VEC, kPickTopK, kSmall>), grid, block, 0, st, *split);
+  else if (s.top_k == 0 && s.top_p > 0.f) MI_PARTS_LAUNCH(sample_first_kernel, DT, VEC, kPickTopP);
+  else hipLaunchKernelGGL((sample_first_kernel<DT, VEC, kPickMax, kSmall>), grid, block, 0, st, *split);
+  if (s.top_k == 0) MI_PARTS_LAUNCH(sample_mass_kernel, DT, VEC);
+#undef MI_PARTS_LAUNCH
   hipLaunchKernelGGL((sample_pick_kernel<DT, VEC>), dim3(s.R), block, 0, st, *split);
 }
 

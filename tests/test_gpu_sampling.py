@@ -453,6 +453,52 @@ def test_logits_too_large_for_masses_take_the_argmax(mi, dev, V, mode):
     assert (x.gather(1, got[:, None]) * (1 / 0.7) >= kept).all()
 
 
+@pytest.mark.parametrize("R,V,pad", [(3, 16387, 0), (128, 80001, 1), (86, 140000, 4)])
+@pytest.mark.parametrize("kind", ["rising", "negative", "zeros", "huge", "wide", "negative nan", "part masked", "all masked", "infinite"])
+def test_parts_where_the_bins_are_at_their_edges(mi, dev, R, V, pad, kind):
+    """Top-p and plain draws of rows in parts against one workgroup per row: a maximum that rises from batch to batch of a
+    part (the bins move), values whose integer order is not theirs, values that leave the bins' range, parts of nothing but
+    -inf or NaN, rows off 16 bytes."""
+    lib = mi._lib.load()
+    g = torch.Generator().manual_seed(R + V)
+    x = torch.randn(R, V, generator=g) * 3
+    if kind == "rising":
+        x += torch.arange(V) * 1e-3
+    elif kind == "negative":
+        x = -x.abs() - 1e-3
+    elif kind == "zeros":
+        x = torch.where(x > 4, -torch.zeros(1), torch.where(x > 2, torch.zeros(1), -x.abs()))
+    elif kind == "huge":
+        x *= 1e30
+    elif kind == "wide":
+        x *= 200
+    elif kind == "negative nan":
+        x[:, ::7] = torch.tensor(-4194304, dtype=torch.int32).view(torch.float32)   # 0xffc00000
+        x[R // 2] = x[0, 0]
+    elif kind == "part masked":
+        x[:, : V // 2] = float("-inf")
+        x[R // 2, : V // 2] = x.new_tensor(-4194304, dtype=torch.int32).view(torch.float32)
+    elif kind == "all masked":
+        x[::2] = float("-inf")
+    elif kind == "infinite":
+        x[R // 2, V // 3] = float("inf")
+    u = torch.rand(R, generator=g).to(dev)
+    for dtype in (torch.float32, torch.bfloat16):
+        y = torch.zeros(R, V + pad, dtype=dtype, device=dev)[:, :V]
+        y.copy_(x)
+        for top_k, top_p in ((0, 0.0), (0, 0.3), (0, 0.9), (0, 0.999)):
+            got, _, cut = mi.ops.sample_from_logits(y, top_k=top_k, top_p=top_p, temperature=0.7, uniform=u, return_cut=True)
+            want = torch.empty(R, dtype=torch.int64, device=dev)
+            want_cut = torch.empty(R, dtype=torch.float32, device=dev)
+            rc = lib.mi_sample_from_logits(y.data_ptr(), y.stride(0), 0 if dtype == torch.float32 else 1, R, V, top_k, top_p, 0.7,
+                                           u.data_ptr(), 0, want.data_ptr(), want_cut.data_ptr(), None, None, None, -1, None,
+                                           torch.cuda.current_stream().cuda_stream)
+            assert rc == 0, lib.mi_last_error()
+            torch.cuda.synchronize()
+            assert torch.equal(got, want), (dtype, top_k, top_p)
+            assert torch.equal(cut, want_cut), (dtype, top_k, top_p)
+
+
 @pytest.mark.parametrize("buffer", ["whole", "off a line", "too small", "on the host", "empty"])
 def test_sampling_inside_use_workspace(mi, dev, buffer):
     """A buffer for attention's scratch that does not serve the parts of the rows is passed over, not refused."""
