@@ -276,6 +276,17 @@ static __device__ __forceinline__ float lane_group_sum(float x) {
   return x;
 }
 
+// inclusive sum over the lanes of a wavefront (lane 63: the total), on the vector pipe's lane shifts
+static __device__ __forceinline__ int wave_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8: within 16 lanes
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // lane 15 -> row 1, lane 47 -> row 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // lane 31 -> rows 2 and 3
+  return v;
+}
+
 // max over the four lanes {l, l^16, l^32, l^48} with two lane-swap instructions
 static __device__ __forceinline__ float rowgroup_max(float x) {
   const uint32_t u = __float_as_uint(x);

@@ -92,6 +92,11 @@ static __device__ __forceinline__ int chunk_of(int tok, uint64_t magic) {
   return (int)(((uint64_t)(uint32_t)tok * magic) >> 40);
 }
 
+// Fused step: LDS of a wavefront: cos | sin of the request's position and the key row in fp32, then up to 16 query rows.
+static __host__ __device__ __forceinline__ int fused_lds_per_wave(int head_dim, int G) {
+  return 3 * head_dim * 4 + (G < 16 ? G : 16) * (2 * head_dim + 16);
+}
+
 // One segment: tokens [start, end) of request r for KV head h (one wavefront) and the `gq` <= 16 query heads
 // hq0 .. hq0 + gq - 1 that share it.  `whole` = the segment is the entire request (write the 16-bit output, no
 // partial).
@@ -103,8 +108,8 @@ static __device__ __forceinline__ int chunk_of(int tok, uint64_t magic) {
 // launch does (same arithmetic and rounding points as norm_rope_append_kernel): every segment normalises and
 // rotates its query rows in registers; the segment that ends the request (`final_seg`: the only one that reads
 // the step's new token) first normalises and rotates the new key row of its KV head, writes it and the value
-// row into their cache slot, and orders that write before its own reads.  `q_lds` is then this wavefront's
-// piece of LDS for cos / sin of the request's position [2][HDK] and the key row [HDK] (fp32).
+// row into their cache slot, and takes both from LDS for its last tile.  `q_lds` is then this wavefront's
+// piece of LDS for cos / sin of the request's position [2][HDK], the key row [HDK] (fp32) and the query rows.
 template <int HDK, int HDV, int NT, bool FP8, bool F16, bool FUSED = false>
 static __device__ __forceinline__ void decode_segment(const DecodeParams& p, int r, int row, int h, int hq0, int gq,
                                                       int len, int start, int end, bool whole, bool final_seg,
@@ -144,9 +149,10 @@ static __device__ __forceinline__ void decode_segment(const DecodeParams& p, int
   uint4 qf[Q_IN_LDS ? 1 : KS];
   const uint8_t* q_frag = q_lds + m16 * kQPitch + 16 * g;  // this lane's fragment of step kk: + 64 kk
   {
-    const uint16_t* qrow = FUSED ? p.q + (int64_t)row * p.q_st + (int64_t)h * p.q_gst + (int64_t)(hq - h * p.G) * HDK
-                                 : p.q + (int64_t)row * p.q_st + (int64_t)hq * p.q_sh;
-    if (Q_IN_LDS) {
+    const uint16_t* qrow = p.q + (int64_t)row * p.q_st + (int64_t)hq * p.q_sh;
+    if constexpr (FUSED) {
+      // (see fused_queries)
+    } else if (Q_IN_LDS) {
 #pragma unroll
       for (int kk = 0; kk < KS; ++kk)
         *reinterpret_cast<uint4*>(q_lds + m16 * kQPitch + 16 * g + 64 * kk) =
@@ -172,7 +178,8 @@ static __device__ __forceinline__ void decode_segment(const DecodeParams& p, int
   // first element of this lane's 8 of fragment kk (see the query loads above)
   auto frag_d0 = [&](int kk) { return FP8 ? 64 * (kk >> 1) + 16 * g + 8 * (kk & 1) : 32 * kk + 8 * g; };
   float* const cs = reinterpret_cast<float*>(q_lds);  // fused: [2][HDK]: cos | sin at the request's position
-  float* const kx = cs + 2 * HDK;                     // fused: [HDK]: the normalised key row (rotary partners)
+  float* const kx = cs + 2 * HDK;                     // fused: [HDK]: the normalised key row (rotary partners) ...
+  uint8_t* const new_row = reinterpret_cast<uint8_t*>(kx);  // ... then the step's key and value row as the cache holds them
   const bool faithful = FUSED && p.faithful != 0;
   // LDS traffic between the lanes of one wavefront: order it for the compiler, the hardware runs it in order
   auto wave_sync = [] {
@@ -184,18 +191,41 @@ static __device__ __forceinline__ void decode_segment(const DecodeParams& p, int
   // elements lane, lane + 64 at the request's position and the norm weights of this lane's query elements.
   constexpr int NA = (HDK + 63) / 64;
   float ang[NA];
-  uint4 qwr[KS];
+  // fused: the raw query rows, QLR lanes to a head (eight values each), QRP heads at a time, the first two times here
+  constexpr int QLR = HDK / 8, QRP = 64 / QLR;
+  const int q_sub = lane / QLR, q_col = lane - q_sub * QLR;
+  uint8_t* const q_rows = q_lds + 3 * HDK * sizeof(float);   // [gq] rows of kQPitch bytes, normed and rotated
+  auto load_raw = [&](int r0) {
+    const int u = min(r0 + q_sub, G - 1);
+    return ld16(p.q + (int64_t)row * p.q_st + (int64_t)h * p.q_gst + (int64_t)(hq0 - h * p.G + u) * HDK + 8 * q_col);
+  };
+  uint4 q_raw[2], q_wt;
   if constexpr (FUSED) {
+    q_raw[0] = load_raw(0);
+    if (G > QRP) q_raw[1] = load_raw(QRP);
     if (p.emb) {
       // (no position array: the step's token sits at the request's last position, which is already at hand)
       const int64_t pos = p.pos ? p.pos[row] : (int64_t)(len - 1);
 #pragma unroll
       for (int i = 0; i < NA; ++i) ang[i] = lane + 64 * i < p.rot ? p.emb[pos * p.emb_stride + lane + 64 * i] : 0.f;
     }
+    if (p.norm == MI_NORM_RMS && p.q_w) q_wt = ld16(p.q_w + 8 * q_col);
+  }
+  // ... and the step's new key and value rows of this KV head: lane i owns elements i, i + LPV, ...
+  constexpr int LPV = HDK >= 128 ? 64 : 32, EPL = HDK / LPV;
+  const bool on = lane < LPV;   // (widths below 128: the upper lanes repeat the lower ones' loads)
+  uint16_t k_new[EPL], v_new[EPL], k_wt[EPL];
+  if constexpr (FUSED) {
+    if (final_seg) {
+      const uint16_t* ks = p.nk + (int64_t)row * p.nk_st + (int64_t)h * p.nk_hst + (on ? lane : 0);
+      const uint16_t* vs = p.nv + (int64_t)row * p.nv_st + (int64_t)h * p.nv_hst + (on ? lane : 0);
 #pragma unroll
-    for (int kk = 0; kk < KS; ++kk)
-      qwr[kk] = (p.norm == MI_NORM_RMS && p.q_w) ? ld16(p.q_w + frag_d0(kk))
-                                                 : make_uint4(ones2<F16>(), ones2<F16>(), ones2<F16>(), ones2<F16>());
+      for (int w = 0; w < EPL; ++w) {
+        k_new[w] = ks[w * LPV];
+        v_new[w] = vs[w * LPV];
+        if (p.norm == MI_NORM_RMS && p.k_w) k_wt[w] = p.k_w[(on ? lane : 0) + w * LPV];
+      }
+    }
   }
   // fp8 fused step: the scales of the chunk that takes the step's token, as this wavefront knows them after its
   // append (it reads them from these registers, never back from memory: the loads of the cursor below may have
@@ -226,28 +256,30 @@ static __device__ __forceinline__ void decode_segment(const DecodeParams& p, int
     }
   };
   // ---- the step's new key / value rows of this KV head -> their cache slot (the request's last position) ----
-  // (With more than 16 query heads per KV head every wavefront of the head writes the same bytes: each one orders
-  // its own write before its own reads, and none has to wait for another.)
+  // The wavefront's own last tile takes both rows from LDS (see new_token below): its loads set out before the rows are
+  // made, and the stores are waited for by nobody in this launch.
+  // (With more than 16 query heads per KV head every wavefront of the head writes the same bytes and reads none of them.)
   auto fused_append = [&] {
     {
-      constexpr int LPV = HDK >= 128 ? 64 : 32, EPL = HDK / LPV;  // lane i owns elements i, i + LPV, ...
-      const bool on = lane < LPV;
       const int i = on ? lane : 0;
-      const uint16_t* src = p.nk + (int64_t)row * p.nk_st + (int64_t)h * p.nk_hst;
       float y[EPL];
 #pragma unroll
-      for (int w = 0; w < EPL; ++w) y[w] = on ? to_f32<F16>(src[i + w * LPV]) : 0.f;
+      for (int w = 0; w < EPL; ++w) y[w] = on ? to_f32<F16>(k_new[w]) : 0.f;
       if (p.norm != MI_NORM_NONE) {
         float ss = y[0] * y[0] + y[1] * y[1];
 #pragma unroll
         for (int w = 2; w < EPL; ++w) ss += y[w] * y[w];
-#pragma unroll
-        for (int o = LPV / 2; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+        if constexpr (LPV == 64) ss += lane_xor<32>(ss);   // (the order of the separate launch: 32, 16, .. 1)
+        ss += lane_xor<16>(ss);
+        ss += lane_xor<8>(ss);
+        ss += lane_xor<4>(ss);
+        ss += lane_xor<2>(ss);
+        ss += lane_xor<1>(ss);
         const float rstd = rsqrtf(ss * (1.f / HDK) + p.eps);
 #pragma unroll
         for (int w = 0; w < EPL; ++w) {
           y[w] *= rstd;
-          if (p.norm == MI_NORM_RMS && p.k_w) y[w] *= to_f32<F16>(p.k_w[i + w * LPV]);
+          if (p.norm == MI_NORM_RMS && p.k_w) y[w] *= to_f32<F16>(k_wt[w]);
           if (faithful) y[w] = to_f32<F16>(f32_to_16<F16>(y[w]));
         }
       }
@@ -273,6 +305,7 @@ static __device__ __forceinline__ void decode_segment(const DecodeParams& p, int
                             : y[w] * c + yp * sn;
           }
         }
+        wave_sync();   // (the key row is about to take the partners' place)
       }
       const int cpos = len - 1, ci = chunk_of(cpos, p.chunk_magic);
       const int pc_new = p.bt[(int64_t)r * p.bt_stride + ci];
@@ -284,12 +317,11 @@ static __device__ __forceinline__ void decode_segment(const DecodeParams& p, int
         const bool opens = cpos == ci * p.chunk;  // wave-uniform
         float* const ksc_p = const_cast<float*>(p.k_scale) + (int64_t)pc_new * p.Hkv + h;
         float* const vsc_p = const_cast<float*>(p.v_scale) + (int64_t)pc_new * p.Hkv + h;
-        const uint16_t* vsrc = p.nv + (int64_t)row * p.nv_st + (int64_t)h * p.nv_hst;
         float kq[EPL], vq[EPL];
 #pragma unroll
         for (int w = 0; w < EPL; ++w) {
           kq[w] = on ? to_f32<F16>(f32_to_16<F16>(o[w])) : 0.f;
-          vq[w] = on ? to_f32<F16>(vsrc[i + w * LPV]) : 0.f;
+          vq[w] = on ? to_f32<F16>(v_new[w]) : 0.f;
         }
         float ksc, vsc;
         if (opens) {
@@ -322,124 +354,107 @@ static __device__ __forceinline__ void decode_segment(const DecodeParams& p, int
         if (on) {
 #pragma unroll
           for (int w = 0; w < EPL; ++w) {
-            kdst8[i + w * LPV] = (uint8_t)f32_to_e4m3_sat(kq[w] / ksc);
-            vdst8[i + w * LPV] = (uint8_t)f32_to_e4m3_sat(vq[w] / vsc);
+            const uint8_t kb = (uint8_t)f32_to_e4m3_sat(kq[w] / ksc), vb = (uint8_t)f32_to_e4m3_sat(vq[w] / vsc);
+            kdst8[i + w * LPV] = kb;
+            vdst8[i + w * LPV] = vb;
+            new_row[i + w * LPV] = kb;
+            new_row[HDK + i + w * LPV] = vb;
           }
         }
       } else {
       uint16_t* kdst = reinterpret_cast<uint16_t*>(const_cast<uint8_t*>(kbase) + slot_bytes);
+      uint16_t* vdst = reinterpret_cast<uint16_t*>(const_cast<uint8_t*>(vbase) + slot_bytes);
+      uint16_t* k_lds = reinterpret_cast<uint16_t*>(new_row);
       if (on) {
 #pragma unroll
-        for (int w = 0; w < EPL; ++w) kdst[i + w * LPV] = f32_to_16<F16>(o[w]);
+        for (int w = 0; w < EPL; ++w) {
+          const uint16_t kb = f32_to_16<F16>(o[w]);
+          kdst[i + w * LPV] = kb;
+          vdst[i + w * LPV] = v_new[w];
+          k_lds[i + w * LPV] = kb;
+          k_lds[HDK + i + w * LPV] = v_new[w];
+        }
       }
-      const uint32_t* vsrc = reinterpret_cast<const uint32_t*>(p.nv + (int64_t)row * p.nv_st + (int64_t)h * p.nv_hst);
-      uint32_t* vdst = reinterpret_cast<uint32_t*>(const_cast<uint8_t*>(vbase) + slot_bytes);
-      for (int e = lane; e < HDV / 2; e += 64) vdst[e] = vsrc[e];
       }
-      // The rows just written are read back below by other lanes of this same wavefront and by nobody else in
-      // this launch (it owns the request's last tiles): wait until the stores have reached the L2 (their
-      // acknowledgement), then keep the compiler from moving the loads up.  No cache has to be written back or
-      // invalidated for that -- the lines cannot sit in this CU's L1 (nothing read them before), and a wider
-      // scope would flush the L2 of the whole XCD under the other wavefronts' streams.
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      wave_sync();
     }
   };
-  // ---- this wavefront's query rows: lane (m16, g) holds elements 32 kk + 8 g .. + 7 of head m16 ----
+  // ---- this wavefront's query rows -> operand fragments.  In the operand layout 4 of 16 lanes would have work (four query
+  // heads) and 32 values each: some 700 instructions, 2.2 of the 8 us that one tile of a small step takes.  Here a lane has
+  // eight neighbouring values of one head, QRP heads to a pass, and the rows go to their fragments through LDS: 1.2 us, and
+  // code half as long (one request of 777 tokens, the kernel: 10.0 -> 8.6 us with the walk; 64 of 512-8 192: 177.6 -> 175).
   auto fused_queries = [&] {
-    float x[KS][8];
+    const bool active = q_sub < QRP;
+    for (int r0 = 0; r0 < G; r0 += QRP) {
+      const uint4 raw = r0 == 0 ? q_raw[0] : r0 == QRP ? q_raw[1] : load_raw(r0);
+      const uint32_t w4[4] = {raw.x, raw.y, raw.z, raw.w};
+      float x[8];
 #pragma unroll
-    for (int kk = 0; kk < KS; ++kk) {
-      const uint32_t w4[4] = {qf[kk].x, qf[kk].y, qf[kk].z, qf[kk].w};
+      for (int j = 0; j < 8; ++j) x[j] = (j & 1) ? hi_to_f32<F16>(w4[j >> 1]) : lo_to_f32<F16>(w4[j >> 1]);
+      if (p.norm != MI_NORM_NONE) {
+        float ss = 0.f;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        x[kk][2 * j] = lo_to_f32<F16>(w4[j]);
-        x[kk][2 * j + 1] = hi_to_f32<F16>(w4[j]);
-      }
-    }
-    if (p.norm != MI_NORM_NONE) {
-      float ss = 0.f;
-#pragma unroll
-      for (int kk = 0; kk < KS; ++kk)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) ss += x[kk][j] * x[kk][j];
-      ss += xor16(ss);
-      ss += xor32(ss);
-      const float rstd = rsqrtf(ss * (1.f / HDK) + p.eps);
-#pragma unroll
-      for (int kk = 0; kk < KS; ++kk) {
-        const uint32_t w4[4] = {qwr[kk].x, qwr[kk].y, qwr[kk].z, qwr[kk].w};
+        for (int j = 0; j < 8; ++j) ss += x[j] * x[j];
+        ss += lane_xor<1>(ss);
+        ss += lane_xor<2>(ss);
+        if constexpr (QLR % 8 == 0) ss += lane_xor<4>(ss);
+        if constexpr (QLR % 16 == 0) ss += lane_xor<8>(ss);
+        if constexpr (QLR % 32 == 0) ss += lane_xor<16>(ss);
+        if constexpr (QLR % 3 == 0) {  // three groups of 4 or 8 lanes
+          const int base = lane - q_col;
+          const float s1 = __shfl(ss, base + (q_col + QLR / 3) % QLR, 64), s2 = __shfl(ss, base + (q_col + 2 * QLR / 3) % QLR, 64);
+          ss += s1 + s2;
+        }
+        const float rstd = rsqrtf(ss * (1.f / HDK) + p.eps);
+        const uint32_t g4[4] = {q_wt.x, q_wt.y, q_wt.z, q_wt.w};
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-          float v = x[kk][j] * rstd;
-          if (p.norm == MI_NORM_RMS && p.q_w) v *= (j & 1) ? hi_to_f32<F16>(w4[j >> 1]) : lo_to_f32<F16>(w4[j >> 1]);
-          x[kk][j] = faithful ? to_f32<F16>(f32_to_16<F16>(v)) : v;
+          x[j] *= rstd;
+          if (p.norm == MI_NORM_RMS && p.q_w) x[j] *= (j & 1) ? hi_to_f32<F16>(g4[j >> 1]) : lo_to_f32<F16>(g4[j >> 1]);
+        }
+        if (faithful) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) x[j] = to_f32<F16>(f32_to_16<F16>(x[j]));
         }
       }
-    }
-    if (p.emb) {
-      // one rotated element: y cos + (partner, signed) sin, with the op chain's roundings when asked for
-      auto rotated = [&](float y, float yp, float c, float sn) {
-        return faithful ? to_f32<F16>(f32_to_16<F16>(y * c)) + to_f32<F16>(f32_to_16<F16>(yp * sn)) : y * c + yp * sn;
-      };
-      // cos | sin of this lane's elements j .. j + 3 of fragment kk (j = 0 or 4)
-      auto cos_sin = [&](int kk, int j, float (&c)[4], float (&sn)[4]) {
-        const float4 c4 = *reinterpret_cast<const float4*>(&cs[frag_d0(kk) + j]);
-        const float4 s4 = *reinterpret_cast<const float4*>(&cs[HDK + frag_d0(kk) + j]);
-        c[0] = c4.x; c[1] = c4.y; c[2] = c4.z; c[3] = c4.w;
-        sn[0] = s4.x; sn[1] = s4.y; sn[2] = s4.z; sn[3] = s4.w;
-      };
-      // fragments ka < kb whose elements are each other's partners (half-split pairs), rotated in place
-      auto rotate_pair = [&](int ka, int kb) {
+      if (p.emb) {
+        const int e0 = 8 * q_col, half = p.rot >> 1;
+        float c[8], sn[8], y[8];
 #pragma unroll
-        for (int j0 = 0; j0 < 8; j0 += 4) {
-          float ca[4], sa[4], cb[4], sb[4];
-          cos_sin(ka, j0, ca, sa);
-          cos_sin(kb, j0, cb, sb);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const float ya = x[ka][j0 + j], yb = x[kb][j0 + j];
-            x[ka][j0 + j] = rotated(ya, -yb, ca[j], sa[j]);
-            x[kb][j0 + j] = rotated(yb, ya, cb[j], sb[j]);
-          }
+        for (int j = 0; j < 8; j += 4) {
+          const float4 c4 = *reinterpret_cast<const float4*>(&cs[e0 + j]);
+          const float4 s4 = *reinterpret_cast<const float4*>(&cs[HDK + e0 + j]);
+          c[j] = c4.x; c[j + 1] = c4.y; c[j + 2] = c4.z; c[j + 3] = c4.w;
+          sn[j] = s4.x; sn[j + 1] = s4.y; sn[j + 2] = s4.z; sn[j + 3] = s4.w;
         }
-      };
-      if (p.interleaved) {
+        if (p.interleaved) {
 #pragma unroll
-        for (int kk = 0; kk < KS; ++kk) {
-#pragma unroll
-          for (int j0 = 0; j0 < 8; j0 += 4) {
-            float c[4], sn[4];
-            cos_sin(kk, j0, c, sn);
-#pragma unroll
-            for (int j = 0; j < 4; j += 2) {
-              if (frag_d0(kk) + j0 + j < p.rot) {  // (rot_dim is even: a pair lies within it or beyond)
-                const float ya = x[kk][j0 + j], yb = x[kk][j0 + j + 1];
-                x[kk][j0 + j] = rotated(ya, -yb, c[j], sn[j]);
-                x[kk][j0 + j + 1] = rotated(yb, ya, c[j + 1], sn[j + 1]);
-              }
-            }
-          }
-        }
-      } else {
-        // half-split pairs: partners are rot_dim / 2 elements = nf fragments apart (the entry point admits only
-        // whole numbers of fragments); fragments beyond the rotary width pass through
-        const int nf = p.rot >> 6;
-        if (nf == 1) {
-          rotate_pair(0, 1);
-        } else if (nf == 2) {
-          if constexpr (KS >= 4) { rotate_pair(0, 2); rotate_pair(1, 3); }
-        } else if (nf == 3) {
-          if constexpr (KS >= 6) { rotate_pair(0, 3); rotate_pair(1, 4); rotate_pair(2, 5); }
+          for (int j = 0; j < 8; ++j) y[j] = (j & 1) ? x[j ^ 1] : -x[j ^ 1];
         } else {
-          if constexpr (KS >= 8) { rotate_pair(0, 4); rotate_pair(1, 5); rotate_pair(2, 6); rotate_pair(3, 7); }
+          // half-split pairs: rot_dim / 2 elements apart, the entry point admits only multiples of 32: whole lanes
+          const int apart = half >> 3;
+          const int from = lane + (q_col < apart ? apart : -apart);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const float v = __shfl(x[j], from, 64);
+            y[j] = q_col < apart ? -v : v;
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const float v = faithful ? to_f32<F16>(f32_to_16<F16>(x[j] * c[j])) + to_f32<F16>(f32_to_16<F16>(y[j] * sn[j]))
+                                   : x[j] * c[j] + y[j] * sn[j];
+          x[j] = e0 + j < p.rot ? v : x[j];   // (elements beyond the rotary width pass through)
         }
       }
+      if (active && r0 + q_sub < G)
+        *reinterpret_cast<uint4*>(q_rows + (r0 + q_sub) * kQPitch + 16 * q_col) =
+            make_uint4(pack2<F16>(x[0], x[1]), pack2<F16>(x[2], x[3]), pack2<F16>(x[4], x[5]), pack2<F16>(x[6], x[7]));
     }
+    wave_sync();
 #pragma unroll
     for (int kk = 0; kk < KS; ++kk)
-      qf[kk] = make_uint4(pack2<F16>(x[kk][0], x[kk][1]), pack2<F16>(x[kk][2], x[kk][3]),
-                          pack2<F16>(x[kk][4], x[kk][5]), pack2<F16>(x[kk][6], x[kk][7]));
+      qf[kk] = m16 < G ? *reinterpret_cast<const uint4*>(q_rows + m16 * kQPitch + 2 * frag_d0(kk)) : make_uint4(0, 0, 0, 0);
   };
 
   float m_run = -INFINITY, l_run = 0.f;
@@ -561,18 +576,12 @@ static __device__ __forceinline__ void decode_segment(const DecodeParams& p, int
   };
 
   if constexpr (FUSED) {
-    // The segment that ends the request appends before it loads (its tiles hold the new token); every other
-    // segment gets its first loads under way and prepares its queries while they are in flight.
+    // The first loads get under way, and the new rows and the queries are prepared while they are in flight.
     // (The value loads wait until the queries are done: with both tiles in flight the prologue would not fit the
     // registers of three wavefronts per SIMD.)
-    if (final_seg) {
-      fused_cos_sin();
-      fused_append();
-      load_k(start);
-    } else {
-      load_k(start);
-      fused_cos_sin();
-    }
+    load_k(start);
+    fused_cos_sin();
+    if (final_seg) fused_append();
     fused_queries();
     __builtin_amdgcn_sched_barrier(0);
     load_v(start);
@@ -596,6 +605,18 @@ static __device__ __forceinline__ void decode_segment(const DecodeParams& p, int
     // multiplier is positive and wave-uniform, so the maximum is taken over the raw products.
     const float mul = FP8 ? p.scale_log2 * ksc_tile : p.scale_log2;
     const bool ragged = T + 16 * NT > end;  // only the last tile of a segment has masked tokens
+    // Fused step, the request's last tile: what the loads brought for the new token's row (and for the rows past it, which
+    // re-read that one) is replaced.
+    const bool new_token = FUSED && final_seg && T + 16 * NT >= len;
+    if (FUSED && new_token) {
+#pragma unroll
+      for (int u = 0; u < NT; ++u) {
+        if (T + 16 * u + m16 >= len - 1) {
+#pragma unroll
+          for (int kk = 0; kk < (FP8 ? KS / 2 : KS); ++kk) kf[u][kk] = *reinterpret_cast<const uint4*>(new_row + k_col + 64 * kk);
+        }
+      }
+    }
     float sc[NT][4];
     float tmax = -INFINITY;
 #pragma unroll
@@ -657,6 +678,20 @@ static __device__ __forceinline__ void decode_segment(const DecodeParams& p, int
 #pragma unroll
       for (int e = 0; e < DV; ++e) {
         acc[e][0] *= alpha; acc[e][1] *= alpha; acc[e][2] *= alpha; acc[e][3] *= alpha;
+      }
+    }
+
+    if (FUSED && new_token) {
+#pragma unroll
+      for (int u = 0; u < NT; ++u) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if (T + 16 * u + 4 * g + j >= len - 1) {
+#pragma unroll
+            for (int dw = 0; dw < VD; ++dw)
+              vf[u][j][dw] = *reinterpret_cast<const uint32_t*>(new_row + HDK * ESZ + v_col + 4 * dw);
+          }
+        }
       }
     }
 
@@ -745,37 +780,48 @@ static __device__ __forceinline__ bool decode_row(const DecodeParams& p, int r, 
 
 // Span of this workgroup along the flattened sequence of TK-token tiles, then its segments one after
 // the other: seg(r, row, len, first token, one past the last token, whole request?, ends the request?, partial slot).
-// Every wavefront of the workgroup walks the same segments.  Dynamic LDS starts with the inclusive
-// prefix sums of tiles per request [R] and the request lengths [R].
-template <int TK, typename Seg>
+// Every wavefront of the workgroup walks the same segments.  Up to 64 requests lie in the lanes of every wavefront: a
+// load, a scan and lane reads, no LDS and no barrier (one request, one tile per workgroup: 2.0 -> 1.6 us of a step's 9).
+// With more, or without LANES (no register to spare), dynamic LDS starts with the inclusive prefix sums of tiles per request [R] and the request lengths [R].
+template <int TK, bool LANES = true, typename Seg>
 static __device__ __forceinline__ void walk_segments(const DecodeParams& p, Seg seg) {
   extern __shared__ int cum[];
   int* const len_s = cum + p.R;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
+  const bool in_lanes = LANES && p.R <= 64;
 
-  // ---- prefix sum of tiles over the batch (wave 0), shared through LDS -------------
-  if (wave == 0) {
-    int carry = 0;
-    for (int base = 0; base < p.R; base += 64) {
-      const int i = base + lane;
-      int row_unused;
-      const int len_i = i < p.R ? p.lens[i] : 0;
-      int v = (i < p.R && decode_row(p, i, row_unused)) ? tiles_of(len_i, TK) : 0;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int up = __shfl_up(v, o, 64);
-        if (lane >= o) v += up;
+  // ---- prefix sum of tiles over the batch ----
+  int cum_l = 0, len_l = 0;   // lane i: of request i (in_lanes; otherwise of the first 64)
+  auto scan64 = [&](int base) {
+    const int i = base + lane;
+    int row_unused;
+    len_l = i < p.R ? p.lens[i] : 0;
+    cum_l = wave_scan((i < p.R && decode_row(p, i, row_unused)) ? tiles_of(len_l, TK) : 0);
+  };
+  int total;
+  if (in_lanes) {
+    scan64(0);
+    total = __builtin_amdgcn_readlane(cum_l, 63);
+  } else {
+    if (wave == 0) {
+      int carry = 0;
+      for (int base = 0; base < p.R; base += 64) {
+        scan64(base);
+        if (base + lane < p.R) {
+          cum[base + lane] = carry + cum_l;
+          len_s[base + lane] = len_l;  // a segment start then costs no trip to memory for the length
+        }
+        carry += __builtin_amdgcn_readlane(cum_l, 63);
       }
-      if (i < p.R) {
-        cum[i] = carry + v;
-        len_s[i] = len_i;  // a segment start then costs no trip to memory for the length
-      }
-      carry += __shfl(v, 63, 64);
     }
+    __syncthreads();
+    cum_l = cum[lane];
+    total = __builtin_amdgcn_readfirstlane(cum[p.R - 1]);
   }
-  __syncthreads();
-  const int total = cum[p.R - 1];
+  auto cum_of = [&](int i) {   // (i wave-uniform)
+    return in_lanes ? __builtin_amdgcn_readlane(cum_l, i) : __builtin_amdgcn_readfirstlane(cum[i]);
+  };
   // Tiles per span of a batch that leaves CUs idle.  A span's tiles follow one another, about 1.5 us each (their loads
   // are one tile ahead, and a trip to memory takes longer than a tile's arithmetic); every further span of a request
   // costs the merge some 0.04 us.  The sum is least at the square root of a thirtieth of the request's tiles.  When
@@ -786,9 +832,11 @@ static __device__ __forceinline__ void walk_segments(const DecodeParams& p, Seg 
   if (min_span <= 0) {
     // (requests with tiles, among the first 64: padded rows and the prompts of a mixed batch have none)
     const int n = min(p.R, 64);
-    const bool live = lane < n && cum[lane] > (lane ? cum[lane - 1] : 0);
-    const float share = (float)__builtin_popcountll(__builtin_amdgcn_ballot_w64(live)) / (float)n;
-    min_span = max(1, (int)rintf(__builtin_sqrtf(0.035f * (float)total / fmaxf(share * (float)p.R, 1.f))));
+    const int before = __builtin_amdgcn_update_dpp(0, cum_l, 0x138, 0xf, 0xf, false);   // the lane below's, 0 for the first
+    const float live = (float)__builtin_popcountll(__builtin_amdgcn_ballot_w64(lane < n && cum_l > before));
+    const float requests = fmaxf(live * (float)p.R * __builtin_amdgcn_rcpf((float)n), 1.f);
+    min_span = max(1, (int)rintf(__builtin_amdgcn_sqrtf(0.035f * (float)total * __builtin_amdgcn_rcpf(requests))));
+    min_span = __builtin_amdgcn_readfirstlane(min_span);
     if (total > p.grid * min_span && total < 4 * p.grid) min_span = (total + p.grid - 1) / p.grid;
   }
   // Starting a segment costs a workgroup about as much as a tile (its queries, table entries and first tile arrive one
@@ -796,12 +844,12 @@ static __device__ __forceinline__ void walk_segments(const DecodeParams& p, Seg 
   // units to balance: the first `lead` units of a request are its start.  (64 latent-cache requests of 512-8 192
   // tokens, 17 tiles per span, up to four starts: 72.9 -> 71.1 us; 64 requests of an ordinary cache, the layer: 218.2 -> 216.5.)
   const int lead = total >= 8 * p.grid && total >= p.grid * min_span ? 1 : 0;
-  auto units = [&](int i) { return cum[i] + lead * (i + 1); };  // of requests 0 .. i
-  const int total_units = units(p.R - 1);
+  auto units = [&](int i) { return cum_of(i) + lead * (i + 1); };  // of requests 0 .. i
   // equal spans; the remainder goes one unit each to the first workgroups (rounding the span
   // up instead would leave the last workgroups without work)
   int t0, t1;
   if (total >= p.grid * min_span) {
+    const int total_units = total + lead * p.R;
     const int per = total_units / p.grid, rem = total_units - per * p.grid;
     t0 = (int)blockIdx.x * per + min((int)blockIdx.x, rem);
     t1 = t0 + per + ((int)blockIdx.x < rem ? 1 : 0);
@@ -811,13 +859,18 @@ static __device__ __forceinline__ void walk_segments(const DecodeParams& p, Seg 
   }
   if (t0 >= t1) return;
 
-  // first request whose units extend beyond t0
-  int lo = 0, hi = p.R - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (units(mid) > t0) hi = mid; else lo = mid + 1;
+  // first request whose units extend beyond t0 (there is one: t0 lies below the total)
+  int r;
+  if (in_lanes) {
+    r = __builtin_ctzll(__builtin_amdgcn_ballot_w64(lane < p.R && cum_l + lead * (lane + 1) > t0));
+  } else {
+    int lo = 0, hi = p.R - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (units(mid) > t0) hi = mid; else lo = mid + 1;
+    }
+    r = lo;
   }
-  int r = lo;
   while (t0 < t1) {
     const int rb = r ? units(r - 1) : 0;
     const int re = units(r);
@@ -825,7 +878,7 @@ static __device__ __forceinline__ void walk_segments(const DecodeParams& p, Seg 
     const int tb = max(t0 - rb - lead, 0);   // first tile of the segment, within the request
     const int te = ue - rb - lead;           // one past its last tile
     if (te > tb) {  // (requests without tiles, and spans that end within a request's start, are skipped)
-      const int len = len_s[r];
+      const int len = in_lanes ? __builtin_amdgcn_readlane(len_l, r) : __builtin_amdgcn_readfirstlane(len_s[r]);
       const bool first = tb == 0, final = ue == re;
       if (wave == 0 && lane == 0) {
         if (first) p.seg_info[2 * r] = blockIdx.x;
@@ -855,7 +908,7 @@ static __device__ __forceinline__ void decode_stream_body(const DecodeParams& p)
   // behind the two integer arrays, per wavefront: 16 query rows (wide keys) or the fused step's cos / sin / key
   // row (see decode_segment)
   uint8_t* const q_lds = reinterpret_cast<uint8_t*>(cum) + (((size_t)p.R * 8 + 15) & ~(size_t)15) +
-                         (size_t)wave * (FUSED ? 3 * HDK * sizeof(float) : 16 * (HDK * 2 + 16));
+                         (size_t)wave * (FUSED ? (size_t)fused_lds_per_wave(HDK, p.G) : (size_t)(16 * (HDK * 2 + 16)));
   walk_segments<16 * NT>(p, [&](int r, int row, int len, int start, int end, bool whole, bool final_seg, int slot) {
     decode_segment<HDK, HDV, NT, FP8, F16, FUSED>(p, r, row, h, hq0, gq, len, start, end, whole, final_seg, slot, lane,
                                                   q_lds);
@@ -1165,7 +1218,7 @@ __global__ __launch_bounds__(256, 1) void paged_mla_decode_heads_kernel(DecodePa
   const uint4 ones = make_uint4(ones2<F16>(), ones2<F16>(), ones2<F16>(), ones2<F16>());
 #define MI_SB() __builtin_amdgcn_sched_barrier(0)
 
-  walk_segments<TK>(p, [&](int r, int row, int len, int start, int end, bool whole, bool /*final_seg*/, int slot) {
+  walk_segments<TK, false>(p, [&](int r, int row, int len, int start, int end, bool whole, bool /*final_seg*/, int slot) {
     r = __builtin_amdgcn_readfirstlane(r);
     row = __builtin_amdgcn_readfirstlane(row);
     len = __builtin_amdgcn_readfirstlane(len);
@@ -1838,7 +1891,7 @@ int mi::launch_paged_decode(
   const int wpb = pick_waves_per_block(waves, tune);
   dim3 grid(grid_x, waves / wpb), block(64 * wpb);
   // (fused step: per wavefront cos | sin | key row in fp32 behind the per-request arrays)
-  const size_t lds = fused ? (((size_t)R * 2 * sizeof(int32_t) + 15) & ~(size_t)15) + (size_t)wpb * 3 * head_dim * sizeof(float)
+  const size_t lds = fused ? (((size_t)R * 2 * sizeof(int32_t) + 15) & ~(size_t)15) + (size_t)wpb * fused_lds_per_wave(head_dim, G)
                            : (size_t)R * 2 * sizeof(int32_t);
   hipStream_t st = (hipStream_t)stream;
   hipEvent_t ev_a, ev_b;

@@ -72,17 +72,6 @@ struct QueryBlock {
   int q0;             // the block's first row within the request
 };
 
-// inclusive sum over the lanes of a wavefront (lane 63: the total), on the vector pipe's lane shifts
-static __device__ __forceinline__ int wave_scan(int v) {
-  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8: within 16 lanes
-  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // lane 15 -> row 1, lane 47 -> row 3
-  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // lane 31 -> rows 2 and 3
-  return v;
-}
-
 // the largest of the lanes' values (none negative)
 static __device__ __forceinline__ int wave_max(int v) {
   v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));

@@ -1491,7 +1491,7 @@ static void launch_sample(const SampleParams& s, SplitParams* split, hipStream_t
   }
   const dim3 grid(split->parts, s.R), block(kSampleThreads);
   // Values a thread holds at a time: short runs (many parts per row) have few, and what is loaded past their end is worked
-  // on all the same (2 x 138 767 bf16, top-p: 27.0 us with 32, 20.9 with 8; 64 x 128 256 fp32: a second batch costs 3).
+  // on all the same (2 x 138 767 bf16, top-p: 27.0 us with 32, 20.9 with 8).
   // Rows off 16 bytes load value by value: 32 of them spill.
   constexpr int kLarge = VEC == 1 ? 16 : 32, kSmall = 8;
   const bool small = split->run_len <= 64 * kSmall;

@@ -287,3 +287,50 @@ def test_fused_step_more_requests_than_one_launch_takes(mi, dev):
     assert (out_a.float() - out_b.float()).abs().max().item() <= 8e-3
     ref, _, _ = _oracle(case, lens, qw, kw, pos, norm="rms", table=table, interleaved=False)
     _close(out_a, ref, 2e-2, "sliced fused step vs checker")
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("R", [1, 63, 64, 65, 200])
+def test_fused_step_over_a_cache_that_holds_nan_past_the_lengths(mi, dev, R, fp8):
+    """The wavefront that ends a request takes the step's rows from LDS; what its loads find in their slots and past them
+    must not reach the result.  Request counts around the 64 that lie in lanes."""
+    Hq, Hkv, d, chunk = 8, 2, 128, 32
+    lens = [1 + (37 * i) % 131 for i in range(R)]
+    case, lens, qw, kw, pos = _step_case(mi, dev, Hq=Hq, Hkv=Hkv, d=d, chunk=chunk, lens=lens, dtype=torch.bfloat16, seed=R)
+    bt = case.block_table.cpu()
+    caches = [case.k_cache.clone(), case.v_cache.clone()]
+    scales = []
+    if fp8:
+        pairs = [oa.quantize_chunks_fp8(c.cpu()) for c in caches]
+        caches = [c.to(dev) for c, _ in pairs]
+        scales = [s.to(dev) for _, s in pairs]
+    bad = [torch.full_like(c, 0x7f) if fp8 else torch.full_like(c, float("nan")) for c in caches]
+    valid = torch.zeros(caches[0].shape[:2], dtype=torch.bool)
+    for r, n in enumerate(lens.tolist()):
+        for t in range(n - 1):
+            valid[bt[r, t // chunk], t % chunk] = True
+    keep = valid.to(dev)[:, :, None, None]
+    common = dict(q_weight=qw.to(dev), k_weight=kw.to(dev), norm="rms", eps=1e-5, positions=pos.to(dev),
+                  rotary_emb=orn.rotary_table(4096, d, base=500000.0).to(dev), max_kv_len=int(lens.max()))
+    got = []
+    for fill in (bad, [torch.zeros_like(c) for c in caches]):
+        kc, vc = (torch.where(keep, c, f) for c, f in zip(caches, fill))
+        more = dict(k_scales=scales[0].clone(), v_scales=scales[1].clone()) if fp8 else {}
+        got.append(mi.ops.decode_step_attention(case.q, case.k_new, case.v_new, kc, vc, case.kv_lens, case.block_table, **common, **more))
+    assert torch.isfinite(got[0].float()).all()
+    assert torch.equal(got[0], got[1])
+
+
+def test_fused_step_of_the_most_requests_one_launch_takes(mi, dev):
+    """Prefix sums, lengths, angles and the query rows of the widest heads share a workgroup's LDS."""
+    Hq, Hkv, d = 16, 1, 256
+    lens = [1 + i % 3 for i in range(7680)]
+    case, lens, qw, kw, pos = _step_case(mi, dev, Hq=Hq, Hkv=Hkv, d=d, chunk=16, lens=lens, dtype=torch.bfloat16, seed=3)
+    table = orn.rotary_table(4096, d, base=500000.0)
+    (out_a, kc_a, vc_a), (out_b, kc_b, vc_b) = _run_both(mi, dev, case, lens, qw, kw, pos, norm="rms", table=table,
+                                                         interleaved=False, mixed=False, max_kv_len=int(lens.max()))
+    assert torch.equal(kc_a, kc_b) and torch.equal(vc_a, vc_b)
+    # means of one to three values reach 4, where neighbouring bf16 values are 2^-6 apart: one unit in the last place (at
+    # most 2^-7 of the value) on top of what a query's last bit moves
+    a, b = out_a.float(), out_b.float()
+    assert ((a - b).abs() <= 8e-3 + b.abs() / 128).all()
