@@ -10,7 +10,7 @@
 //
 // Work split: K is cut into slices of at most 512 columns, and the result is the slices' fp32 sums added in slice order,
 // part by part -- fixed by (T, N, K) alone, so a call is reproducible bit for bit.  A workgroup takes
-// 16 RT rows of W and all of K (or one of up to three parts) for a block of at most 64 tokens, one wavefront per slice:
+// 8 RH rows of W and all of K (or one of up to three parts) for a block of at most 64 tokens, one wavefront per slice:
 // each piece of W and of x that a workgroup needs enters the CU exactly once, straight into the registers of the wavefront that multiplies it -- no
 // staging shared between wavefronts, no barrier before or between the products, and a ring of loads that stays full
 // from the first instruction on.  The slices' sums meet in LDS at the end: one kernel and no partial sums in memory, but
@@ -45,7 +45,7 @@ struct LinearParams {
   float* part;                        // with several parts their sums, [part][T][N]; else null
 };
 
-// RT = 16-row tiles of W, XH = 8-token half tiles of x, P = steps in flight, NW = wavefronts at most (8: 256 registers
+// RH = 8-row half tiles of W, XH = 8-token half tiles of x, P = steps in flight, NW = wavefronts at most (8: 256 registers
 // each, 12: 168, 16: 128).
 //
 // The products want lane (m16, g) to hold columns 8 g .. + 7 (of 32) of row m16 of W, and the same of token m16 of x.
@@ -55,16 +55,16 @@ struct LinearParams {
 // instruction, and the wavefront turns its own piece of LDS -- written as loaded, read in the products' order, both
 // without bank conflicts by the exclusive-or of piece and row.  A wavefront's LDS operations execute in order and no
 // other wavefront touches its piece, so there is no barrier and no wait between the two.
-template <bool F16, int RT, int XH, int P, int NW>
+template <bool F16, int RH, int XH, int P, int NW>
 __global__ __launch_bounds__(64 * NW) void linear_decode_kernel(LinearParams p) {
-  constexpr int TT = (XH + 1) / 2;
+  constexpr int TT = (XH + 1) / 2, RT = (RH + 1) / 2;
   constexpr int kTurn = (2 * RT + 2 * TT) * 1024;   // bytes of a wavefront's piece of LDS: one step of W and of x
   constexpr int kTile = 1024;                       // a 16 x 16 tile of sums: 16 bytes per lane
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m16 = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * (16 * RT);
+  const int n0 = blockIdx.x * (8 * RH);
   const int t0 = blockIdx.y * (8 * XH);
   const int nt = min(8 * XH, p.T - t0);
 
@@ -72,29 +72,32 @@ __global__ __launch_bounds__(64 * NW) void linear_decode_kernel(LinearParams p) 
   uint8_t* const turn_put = lds + wave * kTurn + lo * 128 + (((lane & 7) ^ lo) << 4);
   const uint8_t* const turn_get = lds + wave * kTurn + m16 * 128;
   const int piece0 = (g ^ (m16 & 7)) << 4, piece1 = ((4 + g) ^ (m16 & 7)) << 4;   // columns 0-31 / 32-63 of the step
-  // Row pairs beyond the last of W repeat it, tokens beyond the last repeat it: their results are not stored.
+  // Rows beyond the last of W repeat its last eight or sixteen, tokens beyond the last repeat it: their results are not stored.
   const uint32_t w_lane = (uint32_t)(lo * p.w_st + col);
   uint32_t x_lane[XH];
 #pragma unroll
   for (int i = 0; i < XH; ++i) x_lane[i] = (uint32_t)(min(8 * i + lo, nt - 1) * p.x_st + col);
   const uint16_t* xbase = p.x + (int64_t)t0 * p.x_st;
-  auto w_at = [&](int i, int k) { return p.w + (int64_t)(min(n0 + 16 * (i >> 1), p.N - 16) + 8 * (i & 1)) * p.w_st + k + w_lane; };
+  auto w_at = [&](int i, int k) {
+    const int row = RH % 2 ? min(n0 + 8 * i, p.N - 8) : min(n0 + 16 * (i >> 1), p.N - 16) + 8 * (i & 1);
+    return p.w + (int64_t)row * p.w_st + k + w_lane;
+  };
   auto x_at = [&](int i, int k) { return xbase + k + x_lane[i]; };
 
-  struct Stage { uint4 w[2 * RT]; uint4 x[XH]; };
+  struct Stage { uint4 w[RH]; uint4 x[XH]; };
   Stage st[P];
   int k0 = 0, k1 = 0, ka = 0;   // columns of the slice at hand; where its first whole step of 64 starts
   auto load = [&](Stage& s, int step) {
     const int k = ka + step * kLinStep;
     if (k + kLinStep <= p.K) {
 #pragma unroll
-      for (int i = 0; i < 2 * RT; ++i) s.w[i] = ld16_stream(w_at(i, k));
+      for (int i = 0; i < RH; ++i) s.w[i] = ld16_stream(w_at(i, k));
 #pragma unroll
       for (int i = 0; i < XH; ++i) s.x[i] = ld16(x_at(i, k));
     } else {  // the last 32 columns of a K that is no multiple of 64: zeros beyond them
       const bool live = k + col < p.K;
 #pragma unroll
-      for (int i = 0; i < 2 * RT; ++i) s.w[i] = live ? ld16_stream(w_at(i, k)) : make_uint4(0u, 0u, 0u, 0u);
+      for (int i = 0; i < RH; ++i) s.w[i] = live ? ld16_stream(w_at(i, k)) : make_uint4(0u, 0u, 0u, 0u);
 #pragma unroll
       for (int i = 0; i < XH; ++i) s.x[i] = live ? ld16(x_at(i, k)) : make_uint4(0u, 0u, 0u, 0u);
     }
@@ -104,7 +107,7 @@ __global__ __launch_bounds__(64 * NW) void linear_decode_kernel(LinearParams p) 
     // (a slice of an odd number of 32 columns shares its first or last 64 with its neighbour: each multiplies its half)
     const bool first = ka + step * kLinStep >= k0, second = ka + step * kLinStep + 32 < k1;
 #pragma unroll
-    for (int i = 0; i < 2 * RT; ++i) *reinterpret_cast<uint4*>(turn_put + i * 1024) = s.w[i];
+    for (int i = 0; i < RH; ++i) *reinterpret_cast<uint4*>(turn_put + i * 1024) = s.w[i];
 #pragma unroll
     for (int i = 0; i < XH; ++i) *reinterpret_cast<uint4*>(turn_put + (2 * RT + i) * 1024) = s.x[i];
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -115,7 +118,7 @@ __global__ __launch_bounds__(64 * NW) void linear_decode_kernel(LinearParams p) 
       wb[i] = *reinterpret_cast<const uint4*>(turn_get + i * 2048 + piece1);
     }
 #pragma unroll
-    for (int j = 0; j < TT; ++j) {   // (an odd XH leaves the last half tile as it was: tokens that are not stored)
+    for (int j = 0; j < TT; ++j) {   // (an odd XH or RH leaves its last half tile as it was: values that are not stored)
       const uint4 xa = *reinterpret_cast<const uint4*>(turn_get + (RT + j) * 2048 + piece0);
       const uint4 xb = *reinterpret_cast<const uint4*>(turn_get + (RT + j) * 2048 + piece1);
       if (first) {
@@ -173,7 +176,7 @@ __global__ __launch_bounds__(64 * NW) void linear_decode_kernel(LinearParams p) 
         continue;
       }
       const int n = n0 + 16 * (tile / TT) + 4 * g, t = 16 * (tile % TT) + m16;
-      if (n >= p.N || t >= nt) continue;
+      if (n >= (RH % 2 ? min(n0 + 8 * RH, p.N) : p.N) || t >= nt) continue;
       if (p.part) {
         *reinterpret_cast<f32x4_t*>(p.part + ((int64_t)blockIdx.z * p.T + t0 + t) * p.N + n) = sum;
         continue;
@@ -252,15 +255,16 @@ static int linear_lds(int rt, int half_tiles, int waves, int slices) {
   return (waves * (2 * rt + 2 * tt) + (slices > waves ? rt * tt : 0)) * 1024;
 }
 
-// (the instances there are: eight wavefronts have the registers for four row tiles, sixteen for one or two)
-static bool linear_instance(int rt, int xh, int waves, int slices) {
-  const int most = waves > 12 ? (xh <= 2 ? 2 : 1) : waves > 8 || xh <= 2 ? 2 : xh <= 4 ? 3 : 4;
-  return rt <= most && linear_lds(rt, xh, waves, slices) <= kLinLds;
+// (the instances there are: eight wavefronts have the registers for four row tiles, sixteen for one or two; 24 rows for few
+// tokens)
+static bool linear_instance(int rh, int xh, int waves, int slices) {
+  const int most = waves > 12 ? (xh <= 2 ? 4 : 2) : waves > 8 || xh <= 2 ? 4 : xh <= 4 ? 6 : 8;
+  return rh <= most && (rh != 3 || xh <= 4) && linear_lds((rh + 1) / 2, xh, waves, slices) <= kLinLds;
 }
-// How a call is spread: tokens per workgroup (8 half_tiles), rows (16 row_tiles), slices at a time (waves), and the parts
+// How a call is spread: tokens per workgroup (8 half_tiles), rows (8 row_halves), slices at a time (waves), and the parts
 // that the slices are cut into, with workgroups of their own and a second launch that adds their sums.
 struct LinearPlan {
-  int half_tiles, row_tiles, waves, parts;
+  int half_tiles, row_halves, waves, parts;
 };
 // The plan with the least estimated time.  A workgroup fills a CU (its registers or its LDS), so the launch runs in rounds
 // of 256 workgroups; a round costs 4.6 us, 3 us more for every further round of slices, and the bytes it brings into a CU,
@@ -270,11 +274,14 @@ struct LinearPlan {
 // fewer row blocks than the chip has CUs, or a few more, smaller token blocks (W once more for each, from the last-level
 // cache) or parts fill it; 64 tokens, against 64 in a workgroup and one part:
 //   2048 x 8192 28.3 -> 19.1 us,  5120 x 8192 34.7 -> 26.3,  1280 x 5120 22.6 -> 12.7,  2048 x 4096 15.4 -> 12.5
+// With few tokens 32 rows leave a quarter of the CUs without any (6144 rows: 192 workgroups) and 16 need a second round:
+// 24 fill the chip.  32 rows -> 24:  6144 x 4096, 16 tokens 13.0 -> 11.8 us, 24 tokens 14.9 -> 13.5;  5120 x 5120, 16 tokens
+// 16.1 -> 14.0;  10240 x 5120, one token 26.4 -> 24.0;  5120 x 8192, one token 18.9 -> 17.4.
 static LinearPlan linear_plan(int T, int N, int K, int slices) {
   LinearPlan best{};
   float least = 0.f;
   int undivided = 0;  // workgroups of the best plan of one part
-  const int tiles = (N + 15) / 16;
+  const int row_halves = N / 8;
   for (int z = 1; z <= kLinParts; ++z) {
     const int per = (slices + z - 1) / z, fewest = (per + 15) / 16;
     // (as many parts as have slices; none where the chip is filled more than twice as it is: 10240 x 8192, 256 tokens,
@@ -288,14 +295,16 @@ static LinearPlan linear_plan(int T, int N, int K, int slices) {
       covered = 8 * xh;
       for (int rounds = fewest; rounds <= fewest + 2; ++rounds) {
         const int w = (per + rounds - 1) / rounds;
-        for (int rt = 1; linear_instance(rt, xh, w, per); ++rt) {
-          const int groups = (tiles + rt - 1) / rt * blocks;
-          const float us = merge + (float)((groups + 255) >> 8) *
-                                       (4.6f + 3.f * (float)(rounds - 1) + column * ((float)rt * (16.f / 52e3f) + (float)xh * (8.f / 60e3f)));
+        for (const int rh : {2, 3, 4, 6, 8}) {
+          if (!linear_instance(rh, xh, w, per)) continue;
+          const int groups = (row_halves + rh - 1) / rh * blocks;
+          float us = merge + (float)((groups + 255) >> 8) *
+                                       (4.6f + 3.f * (float)(rounds - 1) + column * ((float)rh * (8.f / 52e3f) + (float)xh * (8.f / 60e3f)));
+          if (rh == 3) us *= 1.06f;   // (for less than that it is not the faster)
           if (best.waves == 0 || us < least) {
             least = us;
             if (z == 1) undivided = groups;
-            best = LinearPlan{xh, rt, w, z};
+            best = LinearPlan{xh, rh, w, z};
           }
         }
         if (w <= 8) break;  // (fewer at a time have no instance more)
@@ -305,56 +314,64 @@ static LinearPlan linear_plan(int T, int N, int K, int slices) {
   return best;
 }
 
-template <bool F16, int RT, int XH, int P, int NW>
+template <bool F16, int RH, int XH, int P, int NW>
 static void launch_linear(const LinearParams& p, hipStream_t st) {
-  const dim3 grid((p.N + 16 * RT - 1) / (16 * RT), (p.T + 8 * XH - 1) / (8 * XH), (p.S + p.per_part - 1) / p.per_part);
-  hipLaunchKernelGGL((linear_decode_kernel<F16, RT, XH, P, NW>), grid, dim3(64 * p.waves), linear_lds(RT, XH, p.waves, p.per_part), st, p);
+  const dim3 grid((p.N + 8 * RH - 1) / (8 * RH), (p.T + 8 * XH - 1) / (8 * XH), (p.S + p.per_part - 1) / p.per_part);
+  hipLaunchKernelGGL((linear_decode_kernel<F16, RH, XH, P, NW>), grid, dim3(64 * p.waves), linear_lds((RH + 1) / 2, XH, p.waves, p.per_part), st, p);
 }
 // (steps in flight: what fits the registers without spilling)
 template <bool F16>
 static void launch_linear(const LinearParams& p, const LinearPlan& plan, hipStream_t st) {
-  const int rt = plan.row_tiles, xh = plan.half_tiles;
-#define LIN(RT, XH, P, NW) launch_linear<F16, RT, XH, P, NW>(p, st)
+  const int rh = plan.row_halves, xh = plan.half_tiles;
+#define LIN(RH, XH, P, NW) launch_linear<F16, RH, XH, P, NW>(p, st)
   if (p.waves <= 8) {
-    switch (10 * xh + rt) {
-      case 11: LIN(1, 1, 8, 8); break;
-      case 12: LIN(2, 1, 6, 8); break;
-      case 21: LIN(1, 2, 6, 8); break;
-      case 22: LIN(2, 2, 4, 8); break;
-      case 41: LIN(1, 4, 6, 8); break;
-      case 42: LIN(2, 4, 4, 8); break;
-      case 43: LIN(3, 4, 3, 8); break;
-      case 61: LIN(1, 6, 5, 8); break;
-      case 62: LIN(2, 6, 4, 8); break;
-      case 63: LIN(3, 6, 2, 8); break;
-      case 64: LIN(4, 6, 2, 8); break;
-      case 81: LIN(1, 8, 4, 8); break;
-      case 82: LIN(2, 8, 3, 8); break;
-      case 83: LIN(3, 8, 2, 8); break;
-      default: LIN(4, 8, 1, 8); break;
+    switch (10 * xh + rh) {
+      case 12: LIN(2, 1, 8, 8); break;
+      case 13: LIN(3, 1, 7, 8); break;
+      case 14: LIN(4, 1, 6, 8); break;
+      case 22: LIN(2, 2, 6, 8); break;
+      case 23: LIN(3, 2, 5, 8); break;
+      case 24: LIN(4, 2, 4, 8); break;
+      case 42: LIN(2, 4, 6, 8); break;
+      case 43: LIN(3, 4, 4, 8); break;
+      case 44: LIN(4, 4, 4, 8); break;
+      case 46: LIN(6, 4, 3, 8); break;
+      case 62: LIN(2, 6, 5, 8); break;
+      case 64: LIN(4, 6, 4, 8); break;
+      case 66: LIN(6, 6, 2, 8); break;
+      case 68: LIN(8, 6, 2, 8); break;
+      case 82: LIN(2, 8, 4, 8); break;
+      case 84: LIN(4, 8, 3, 8); break;
+      case 86: LIN(6, 8, 2, 8); break;
+      default: LIN(8, 8, 1, 8); break;
     }
   } else if (p.waves <= 12) {
-    switch (10 * xh + rt) {
-      case 11: LIN(1, 1, 6, 12); break;
-      case 12: LIN(2, 1, 4, 12); break;
-      case 21: LIN(1, 2, 5, 12); break;
-      case 22: LIN(2, 2, 3, 12); break;
-      case 41: LIN(1, 4, 4, 12); break;
-      case 42: LIN(2, 4, 2, 12); break;
-      case 61: LIN(1, 6, 3, 12); break;
-      case 62: LIN(2, 6, 1, 12); break;
-      case 81: LIN(1, 8, 2, 12); break;
-      default: LIN(2, 8, 1, 12); break;
+    switch (10 * xh + rh) {
+      case 12: LIN(2, 1, 6, 12); break;
+      case 13: LIN(3, 1, 5, 12); break;
+      case 14: LIN(4, 1, 4, 12); break;
+      case 22: LIN(2, 2, 5, 12); break;
+      case 23: LIN(3, 2, 4, 12); break;
+      case 24: LIN(4, 2, 3, 12); break;
+      case 42: LIN(2, 4, 4, 12); break;
+      case 43: LIN(3, 4, 3, 12); break;
+      case 44: LIN(4, 4, 2, 12); break;
+      case 62: LIN(2, 6, 3, 12); break;
+      case 64: LIN(4, 6, 1, 12); break;
+      case 82: LIN(2, 8, 2, 12); break;
+      default: LIN(4, 8, 1, 12); break;
     }
   } else {
-    switch (10 * xh + rt) {
-      case 11: LIN(1, 1, 6, 16); break;
-      case 12: LIN(2, 1, 3, 16); break;
-      case 21: LIN(1, 2, 4, 16); break;
-      case 22: LIN(2, 2, 2, 16); break;
-      case 41: LIN(1, 4, 2, 16); break;
-      case 61: LIN(1, 6, 1, 16); break;
-      default: LIN(1, 8, 1, 16); break;
+    switch (10 * xh + rh) {
+      case 12: LIN(2, 1, 6, 16); break;
+      case 13: LIN(3, 1, 4, 16); break;
+      case 14: LIN(4, 1, 3, 16); break;
+      case 22: LIN(2, 2, 4, 16); break;
+      case 23: LIN(3, 2, 3, 16); break;
+      case 24: LIN(4, 2, 2, 16); break;
+      case 42: LIN(2, 4, 2, 16); break;
+      case 62: LIN(2, 6, 1, 16); break;
+      default: LIN(2, 8, 1, 16); break;
     }
   }
 #undef LIN

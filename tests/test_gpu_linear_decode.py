@@ -63,6 +63,21 @@ def test_tile_edges(mi, dev, T, N, K):
     _ulp_close(out, (big[:T, :K].float() @ w[:N, :K].float().t()).bfloat16(), torch.bfloat16, f"linear {T}x{N}x{K}")
 
 
+@pytest.mark.parametrize("T", [1, 8, 9, 16, 17, 32])
+@pytest.mark.parametrize("N,K", [(6144, 4096), (6128, 4096), (5120, 5120), (5104, 6144)])
+def test_workgroups_of_24_rows(mi, dev, T, N, K):
+    """Row counts that 32 rows per workgroup would leave on part of the chip: whole workgroups, and a last one of 8 rows.
+    Guards around the weights are not numbers, guards around the result stay as they were."""
+    gen = torch.Generator().manual_seed(T + N)
+    x = (torch.randn(T, K, generator=gen) * 0.5).bfloat16().to(dev)
+    w = torch.full((N + 32, K), float("nan"), dtype=torch.bfloat16, device=dev)
+    w[:N] = (torch.randn(N, K, generator=gen) * 0.05).bfloat16().to(dev)
+    out = torch.full((T, N + 32), 7.0, dtype=torch.bfloat16, device=dev)
+    mi.ops.linear_decode(x, w[:N], out=out[:, :N])
+    _ulp_close(out[:, :N], (x.float() @ w[:N].float().t()).bfloat16(), torch.bfloat16, f"linear {T}x{N}x{K}")
+    assert (out[:, N:] == 7.0).all()
+
+
 @pytest.mark.parametrize("T", [8, 16, 24, 33, 64, 65, 96, 200, 256])
 @pytest.mark.parametrize("N,K", [(2048, 8192), (1280, 5120), (48, 512)])
 def test_token_blocks(mi, dev, T, N, K):
