@@ -262,7 +262,24 @@ int mi_decode_step_attention_fp8(const void* q, int64_t q_stride_tok, int64_t q_
                                  int32_t Hq, int32_t Hkv, int32_t head_dim, int32_t chunk_tokens,
                                  int32_t split_tokens, float softmax_scale, int32_t faithful_rounding,
                                  int32_t dtype, const MiTuning* tuning, void* stream);
-
+/*
+ * Either of the two (kv_dtype MI_KV_16BIT: scales null, headroom any positive number; MI_KV_FP8_E4M3) with the 16-bit matrix
+ * [next_rows][next_columns] of the mi_linear_decode call over R tokens that follows on the stream.  The results are theirs.
+ * Where the batch leaves at least half of the workgroups without a span, those read the matrix meanwhile, so that the
+ * projection finds it in the L2 of the XCDs that will ask for it.  next_weight == NULL: nothing is read.  Otherwise rows and
+ * strides as mi_linear_decode takes them (rows % 16 == 0, columns % 32 == 0 and below 2^20, 16-byte aligned rows).
+ */
+int mi_decode_step_attention_before_linear(
+    const void* q, int64_t q_stride_tok, int64_t q_stride_group, const void* k_new, int64_t k_stride_tok,
+    int64_t k_stride_head, const void* v_new, int64_t v_stride_tok, int64_t v_stride_head, const void* q_weight,
+    const void* k_weight, float eps, int32_t norm_kind, const float* rotary_angles, int64_t angles_stride,
+    int32_t rot_dim, int32_t rotary_interleaved, float mscale, const int64_t* positions, void* k_cache,
+    void* v_cache, int64_t kv_stride_chunk, int64_t kv_stride_tok, int64_t kv_stride_head, int32_t kv_dtype,
+    float* k_scales, float* v_scales, float headroom, const int32_t* block_table, int64_t bt_stride,
+    const int32_t* kv_lens, void* out, int64_t o_stride_tok, int64_t o_stride_head, void* workspace,
+    int64_t workspace_bytes, int32_t R, int32_t Hq, int32_t Hkv, int32_t head_dim, int32_t chunk_tokens,
+    int32_t split_tokens, float softmax_scale, int32_t faithful_rounding, int32_t dtype, const MiTuning* tuning,
+    const void* next_weight, int64_t next_stride_row, int32_t next_rows, int32_t next_columns, void* stream);
 /*
  * mi_paged_decode_attention for callers that cannot allocate device memory: code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc.  It has no counterpart in the

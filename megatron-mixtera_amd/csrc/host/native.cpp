@@ -754,7 +754,9 @@ PyObject* qkv_prefill_attention(PyObject* const* a) {
 //                       kv_lens, block_table, q_weight|None, k_weight|None, eps, norm_kind, rotary_emb|None,
 //                       positions|None, interleaved, mscale, softmax_scale|None, max_kv_len|None, split_tokens, out|None,
 //                       workspace|None, faithful_rounding, k_scales|None, v_scales|None, headroom, tuning|None, override|None)
-PyObject* decode_step_attention(PyObject* const* a) {
+//
+// `next`: the matrix of the projection that follows at once (the layer's step), or null.
+PyObject* decode_step(PyObject* const* a, const Tensor* next) {
   const Tensor &kc = tensor(a[6], "k_cache"), &vc = tensor(a[7], "v_cache"), &lens = tensor(a[8], "kv_lens"), &table = tensor(a[9], "block_table");
   int64_t R, Hq, Hkv, D;
   const uint8_t *qp, *kp, *vp;
@@ -819,7 +821,16 @@ PyObject* decode_step_attention(PyObject* const* a) {
   const Scratch ws = scratch(*ref, stream, mi_decode_workspace_bytes((int)R, (int)Hq, (int)Hkv, (int)D, (int)c.c, (int)max_len, split, tune), a[22], a[28]);
   const float eps = (float)as_float(a[12]), mscale = (float)as_float(a[17]);
   const int norm = (int)as_int(a[13]), inter = as_bool(a[16]), faithful = as_bool(a[23]);
-  if (fp8) {
+  if (next) {
+    check(mi_decode_step_attention_before_linear(
+              qp, q_st, q_gst, kp, k_st, k_hst, vp, v_st, v_hst, ptr(qw), ptr(kw), eps, norm, ang.ptr, ang.stride, ang.rot, inter,
+              mscale, (const int64_t*)ptr(pos), kc.data_ptr(), vc.data_ptr(), c.sc, c.st, c.sh, fp8 ? MI_KV_FP8_E4M3 : MI_KV_16BIT,
+              fp8 ? (float*)ks->data_ptr() : nullptr, fp8 ? (float*)vs->data_ptr() : nullptr, fp8 ? (float)as_float(a[26]) : 1.f,
+              (const int32_t*)table.data_ptr(), table.stride(0), (const int32_t*)lens.data_ptr(), out.data_ptr(), o3.sn, o3.sh,
+              ws.ptr, ws.bytes, (int)R, (int)Hq, (int)Hkv, (int)D, (int)c.c, split, scale, faithful, dtype_code(*ref), tune,
+              next->data_ptr(), next->stride(0), (int)next->size(0), (int)next->size(1), stream),
+          "mi_decode_step_attention_before_linear");
+  } else if (fp8) {
     check(mi_decode_step_attention_fp8(qp, q_st, q_gst, kp, k_st, k_hst, vp, v_st, v_hst, ptr(qw), ptr(kw), eps, norm, ang.ptr,
                                        ang.stride, ang.rot, inter, mscale, (const int64_t*)ptr(pos), kc.data_ptr(), vc.data_ptr(),
                                        c.sc, c.st, c.sh, (float*)ks->data_ptr(), (float*)vs->data_ptr(), (float)as_float(a[26]),
@@ -837,6 +848,8 @@ PyObject* decode_step_attention(PyObject* const* a) {
   }
   return a[21] == Py_None ? wrap(made) : same(a[21]);
 }
+
+PyObject* decode_step_attention(PyObject* const* a) { return decode_step(a, nullptr); }
 
 // linear_decode(x, weight, bias|None, out|None, override|None)
 PyObject* linear_decode(PyObject* const* a) {
@@ -899,7 +912,13 @@ PyObject* attention_layer_decode(PyObject* const* a) {
   Drop d0{mixed}, d1{PyLong_FromLong(0)}, d2{PyFloat_FromDouble(1.0)};
   PyObject* const step[29] = {none, none, none, mixed, a[5], a[6], a[7], a[8], a[9], a[10], a[11], a[12], a[13], a[14], a[15],
                               none, a[16], d2.o, a[17], a[18], d1.o, none, none, Py_True, a[19], a[20], a[21], a[22], a[23]};
-  PyObject* attn = decode_step_attention(step);
+  // (a matrix that the projection below refuses is its to refuse)
+  const Tensor* proj = opt_tensor(a[3], "weight");
+  const bool fetchable = proj && proj->dim() == 2 && proj->stride(1) == 1 && is_16bit(*proj) && proj->device() == tensor(a[7], "k_cache").device() &&
+                         proj->size(0) > 0 && proj->size(0) % 16 == 0 && proj->size(1) > 0 && proj->size(1) % 32 == 0 &&
+                         proj->stride(0) >= proj->size(1) && proj->stride(0) % 8 == 0 && proj->size(0) < (1 << 30) &&
+                         proj->size(1) < (1 << 20) && (reinterpret_cast<uintptr_t>(proj->data_ptr()) & 15) == 0;
+  PyObject* attn = decode_step(step, fetchable ? proj : nullptr);
   Drop d3{attn};
   const Tensor& o = THPVariable_Unpack(attn);   // [R, 1, Hq, d], contiguous
   Drop d4{wrap(o.view({o.size(0), 1, o.size(2) * o.size(3)}))};

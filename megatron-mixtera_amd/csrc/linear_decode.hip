@@ -314,6 +314,15 @@ static LinearPlan linear_plan(int T, int N, int K, int slices) {
   return best;
 }
 
+int mi::linear_rows_per_workgroup(int T, int N, int K) {
+  if (T <= 0 || T > 256) return 0;
+  int slices, len;
+  linear_slices(T, N, K, &slices, &len);
+  const LinearPlan plan = linear_plan(T, N, K, slices);
+  const int rows = 8 * plan.row_halves, across = (N + rows - 1) / rows;
+  return plan.parts == 1 && (T <= 8 * plan.half_tiles || across % 8 == 0) ? rows : 0;
+}
+
 template <bool F16, int RH, int XH, int P, int NW>
 static void launch_linear(const LinearParams& p, hipStream_t st) {
   const dim3 grid((p.N + 8 * RH - 1) / (8 * RH), (p.T + 8 * XH - 1) / (8 * XH), (p.S + p.per_part - 1) / p.per_part);

@@ -42,7 +42,13 @@ struct FusedStepArgs {
   const int64_t* positions;
   int32_t faithful_rounding;
   float fp8_headroom;  // fp8 cache: scale of a chunk the step's token opens = headroom * amax(token) / 448
+  const void* next_weight;  // the matrix of the projection that follows, or null (see mi_decode_step_attention_before_linear)
+  int64_t next_stride_row;
+  int32_t next_rows, next_columns;
 };
+// Rows of the matrix that one workgroup of mi_linear_decode reads, workgroup x of the grid rows [x n, x n + n); 0 where a
+// row is read by workgroups on several XCDs.
+int linear_rows_per_workgroup(int T, int N, int K);
 // Shared by the decode entry point and by the mixed-batch path of the prefill entry point
 // (cu_seqlens_q non-null: only requests with one query row take part, at row cu_seqlens_q[r]).
 // The workspace checks of launch_paged_decode alone (size for R requests, alignment), for callers that must know

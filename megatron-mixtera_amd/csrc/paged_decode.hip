@@ -83,6 +83,10 @@ struct DecodeParams {
   int64_t emb_stride;
   const int64_t* pos;  // [R] rotary position of the step's token
   int32_t rot, norm, interleaved, faithful;
+  // The matrix of the projection that follows (or null): `next_blocks` workgroups of its kernel read `next_rows` rows each.
+  const uint8_t* next_w;
+  int64_t next_st;     // bytes between rows
+  int32_t next_n, next_bytes, next_rows, next_fetch, next_blocks;   // rows, bytes of one, rows per block, of them to fetch, blocks
   float eps, mscale;
   float scale_log2;
 };
@@ -783,8 +787,10 @@ static __device__ __forceinline__ bool decode_row(const DecodeParams& p, int r, 
 // Every wavefront of the workgroup walks the same segments.  Up to 64 requests lie in the lanes of every wavefront: a
 // load, a scan and lane reads, no LDS and no barrier (one request, one tile per workgroup: 2.0 -> 1.6 us of a step's 9).
 // With more, or without LANES (no register to spare), dynamic LDS starts with the inclusive prefix sums of tiles per request [R] and the request lengths [R].
-template <int TK, bool LANES = true, typename Seg>
-static __device__ __forceinline__ void walk_segments(const DecodeParams& p, Seg seg) {
+// A workgroup without a span calls idle(number of those that have one).
+struct NoIdle { __device__ __forceinline__ void operator()(int) const {} };
+template <int TK, bool LANES = true, typename Seg, typename Idle = NoIdle>
+static __device__ __forceinline__ void walk_segments(const DecodeParams& p, Seg seg, Idle idle = Idle()) {
   extern __shared__ int cum[];
   int* const len_s = cum + p.R;
   const int lane = threadIdx.x & 63;
@@ -857,7 +863,10 @@ static __device__ __forceinline__ void walk_segments(const DecodeParams& p, Seg 
     t0 = blockIdx.x * min_span;
     t1 = min(t0 + min_span, total);
   }
-  if (t0 >= t1) return;
+  if (t0 >= t1) {
+    idle((total + min_span - 1) / min_span);
+    return;
+  }
 
   // first request whose units extend beyond t0 (there is one: t0 lies below the total)
   int r;
@@ -893,6 +902,35 @@ static __device__ __forceinline__ void walk_segments(const DecodeParams& p, Seg 
   }
 }
 
+// A workgroup of a decode step that has no span reads its share of the next projection's matrix into the L2 of its XCD,
+// while the others walk a chain of trips to memory that leaves the memory itself idle.  Workgroups are dealt to the eight
+// XCDs in turn, here and in the projection's launch: this one takes the row blocks that workgroups of its own XCD will ask
+// for.  (33.5 MB in 6.2 us; the projection of 4096 x 4096 finds them: 9.9 -> 6.9 us at one token, 10.4 -> 8.0 at 16; the
+// same bytes in another XCD's L2, or in the last-level cache only, are worth nothing.)
+static __device__ __forceinline__ void fetch_next_matrix(int busy) {
+  // (the arguments from where they lie: nothing of this is held in registers by those that have a span)
+  auto* args = (const __attribute__((address_space(4))) DecodeParams*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(args));
+  const auto& p = *args;
+  if (!p.next_w || blockIdx.y || 2 * busy > (int)gridDim.x) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+  const int first = busy + (((int)blockIdx.x - busy) & 7);   // the first workgroup without a span on this XCD
+  const int mine = ((int)blockIdx.x - first) >> 3, all = ((int)gridDim.x - first + 7) >> 3;
+  for (int b = ((int)blockIdx.x & 7) + 8 * mine; b < p.next_blocks; b += 8 * all) {
+    const int row0 = b * p.next_rows, rows = min(p.next_fetch, p.next_n - row0);
+    for (int r = wave; r < rows; r += waves) {
+      const uint8_t* row = p.next_w + (int64_t)(row0 + r) * p.next_st;
+      for (int at = 16 * lane; at < p.next_bytes; at += 8 * 1024) {
+        uint4 v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = ld16(row + min(at + 1024 * i, p.next_bytes - 16));
+#pragma unroll
+        for (int i = 0; i < 8; ++i) asm volatile("" ::"v"(v[i].x), "v"(v[i].y), "v"(v[i].z), "v"(v[i].w));
+      }
+    }
+  }
+}
+
 // The body of the register-streaming kernels: one wavefront per (virtual) KV head.
 template <int HDK, int HDV, int NT, bool FP8, bool F16, bool FUSED = false>
 static __device__ __forceinline__ void decode_stream_body(const DecodeParams& p) {
@@ -912,6 +950,8 @@ static __device__ __forceinline__ void decode_stream_body(const DecodeParams& p)
   walk_segments<16 * NT>(p, [&](int r, int row, int len, int start, int end, bool whole, bool final_seg, int slot) {
     decode_segment<HDK, HDV, NT, FP8, F16, FUSED>(p, r, row, h, hq0, gq, len, start, end, whole, final_seg, slot, lane,
                                                   q_lds);
+  }, [&](int busy) {
+    if constexpr (FUSED) fetch_next_matrix(busy);
   });
 }
 
@@ -1706,6 +1746,11 @@ static void launch_merge(const DecodeParams& p, int grid_x, int R, int Hq, int h
   else hipLaunchKernelGGL((paged_decode_merge_kernel<false>), mgrid, mblock, 0, st, p, ms);
 }
 
+// What a decode step's idle workgroups read of the next projection's matrix, at most: the L2s of eight XCDs.  (A layer of
+// 4096, its 33.5 MB all read: 35.8 -> 34.4 us; with 26 MiB read of it, 35.5.  A matrix of 5120 x 8192, twice the L2s: 57.6
+// -> 56.3 us with 20, 26, 32 or 36 MiB.)
+constexpr int64_t kFetchBytes = (int64_t)32 << 20;
+
 // Requests one launch of the streaming kernels takes: their tile prefix sums and lengths sit in LDS.
 constexpr int kMaxRequestsPerLaunch = 7680;
 
@@ -1885,6 +1930,16 @@ int mi::launch_paged_decode(
     p.rot = fused->rot_dim; p.norm = fused->norm_kind; p.interleaved = fused->rotary_interleaved;
     p.faithful = fused->faithful_rounding; p.eps = fused->eps; p.mscale = fused->mscale;
     p.headroom = fused->fp8_headroom;
+    // (as much of the next projection's matrix as the eight L2s hold, the same share of every workgroup's rows)
+    p.next_w = nullptr;
+    int rows = 0;
+    if (fused->next_weight && (rows = linear_rows_per_workgroup(R, fused->next_rows, fused->next_columns)) > 0) {
+      p.next_w = (const uint8_t*)fused->next_weight; p.next_st = fused->next_stride_row * 2;
+      p.next_n = fused->next_rows; p.next_bytes = fused->next_columns * 2; p.next_rows = rows;
+      p.next_blocks = (p.next_n + rows - 1) / rows;
+      const int64_t fit = kFetchBytes / ((int64_t)p.next_blocks * p.next_bytes);
+      p.next_fetch = fit < rows ? (int)fit : rows;
+    }
   }
 
   const int waves = head_waves(Hq, Hkv);
@@ -1978,7 +2033,8 @@ static int decode_step_entry(
     int64_t bt_stride, const int32_t* kv_lens, void* out, int64_t o_stride_tok, int64_t o_stride_head, void* workspace,
     int64_t workspace_bytes, int32_t R, int32_t Hq, int32_t Hkv, int32_t head_dim, int32_t chunk_tokens,
     int32_t split_tokens, float softmax_scale, int32_t faithful_rounding, int32_t dtype, const MiTuning* tuning,
-    void* stream, int32_t kv_dtype, float* k_scales, float* v_scales, float headroom) {
+    void* stream, int32_t kv_dtype, float* k_scales, float* v_scales, float headroom, const void* next_weight = nullptr,
+    int64_t next_stride_row = 0, int32_t next_rows = 0, int32_t next_columns = 0) {
   const bool fp8 = kv_dtype == MI_KV_FP8_E4M3;
   char msg[160];
   auto fail = [&](int code, const char* what) {
@@ -2022,6 +2078,14 @@ static int decode_step_entry(
   fs.rotary_interleaved = rotary_interleaved; fs.mscale = mscale; fs.positions = positions;
   fs.faithful_rounding = faithful_rounding;
   fs.fp8_headroom = headroom;
+  if (next_weight) {
+    if (next_rows <= 0 || next_columns <= 0 || next_rows % 16 || next_columns % 32 || next_columns >= (1 << 20) ||
+        next_stride_row < next_columns)
+      return fail(MI_ERR_SHAPE, "the next projection needs rows a multiple of 16, columns a multiple of 32 below 2^20 and a row stride that covers them");
+    if (((uintptr_t)next_weight & 15) || next_stride_row % 8)
+      return fail(MI_ERR_ALIGN, "the next projection's rows must be 16-byte aligned");
+  }
+  fs.next_weight = next_weight; fs.next_stride_row = next_stride_row; fs.next_rows = next_rows; fs.next_columns = next_columns;
   // (the remaining checks -- cache strides, chunk size, workspace -- are those of the attention entry point; the
   // head stride of q is not used by the fused kernels)
   return launch_paged_decode(q, q_stride_tok, head_dim, k_cache, v_cache, kv_stride_chunk, kv_stride_tok, kv_stride_head,
@@ -2065,6 +2129,26 @@ extern "C" int mi_decode_step_attention_fp8(
                            o_stride_tok, o_stride_head, workspace, workspace_bytes, R, Hq, Hkv, head_dim, chunk_tokens,
                            split_tokens, softmax_scale, faithful_rounding, dtype, tuning, stream, MI_KV_FP8_E4M3,
                            k_scales, v_scales, headroom);
+}
+
+extern "C" int mi_decode_step_attention_before_linear(
+    const void* q, int64_t q_stride_tok, int64_t q_stride_group, const void* k_new, int64_t k_stride_tok,
+    int64_t k_stride_head, const void* v_new, int64_t v_stride_tok, int64_t v_stride_head, const void* q_weight,
+    const void* k_weight, float eps, int32_t norm_kind, const float* rotary_angles, int64_t angles_stride,
+    int32_t rot_dim, int32_t rotary_interleaved, float mscale, const int64_t* positions, void* k_cache,
+    void* v_cache, int64_t kv_stride_chunk, int64_t kv_stride_tok, int64_t kv_stride_head, int32_t kv_dtype, float* k_scales,
+    float* v_scales, float headroom, const int32_t* block_table, int64_t bt_stride, const int32_t* kv_lens, void* out,
+    int64_t o_stride_tok, int64_t o_stride_head, void* workspace, int64_t workspace_bytes, int32_t R, int32_t Hq,
+    int32_t Hkv, int32_t head_dim, int32_t chunk_tokens, int32_t split_tokens, float softmax_scale,
+    int32_t faithful_rounding, int32_t dtype, const MiTuning* tuning, const void* next_weight, int64_t next_stride_row,
+    int32_t next_rows, int32_t next_columns, void* stream) {
+  return decode_step_entry("mi_decode_step_attention_before_linear", q, q_stride_tok, q_stride_group, k_new, k_stride_tok,
+                           k_stride_head, v_new, v_stride_tok, v_stride_head, q_weight, k_weight, eps, norm_kind,
+                           rotary_angles, angles_stride, rot_dim, rotary_interleaved, mscale, positions, k_cache,
+                           v_cache, kv_stride_chunk, kv_stride_tok, kv_stride_head, block_table, bt_stride, kv_lens, out,
+                           o_stride_tok, o_stride_head, workspace, workspace_bytes, R, Hq, Hkv, head_dim, chunk_tokens,
+                           split_tokens, softmax_scale, faithful_rounding, dtype, tuning, stream, kv_dtype,
+                           k_scales, v_scales, headroom, next_weight, next_stride_row, next_rows, next_columns);
 }
 
 // ---------------------------------------------------------------------------------------------

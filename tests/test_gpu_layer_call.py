@@ -43,6 +43,33 @@ def test_one_call_equals_the_modules(mi, dev, lens, cache):
         assert (a is None and b is None) or torch.equal(a, b)
 
 
+@pytest.mark.parametrize("lens,hidden,heads,cache,pad", [
+    ([5], 6112, 8, None, 0),           # workgroups of 24 rows: the last workgroup's rows end beyond the matrix
+    ([600], 4096, 32, None, 8),        # rows apart, the last one at the end of its storage
+    ([3, 256], 5120, 64, "fp8_e4m3", 0),   # a matrix larger than what is read ahead
+    ([240] * 16, 2048, 16, None, 0),   # half of the workgroups have a span, or all
+])
+def test_reading_the_projection_ahead_changes_nothing(mi, dev, lens, hidden, heads, cache, pad):
+    outs = []
+    for by_module in (False, True):
+        ctx = _context(mi, dev, lens, cache)
+        ctx.update_requests(torch.ones(len(lens), dtype=torch.uint8, device=dev), torch.zeros(len(lens), dtype=torch.long, device=dev))
+        ctx.initialize_attention_state()
+        gen = torch.Generator(device=dev).manual_seed(2)
+        layer = mi.PagedSelfAttentionLayer(2, hidden, heads, 2, 128, qk_norm="rms", device=dev).requires_grad_(False)
+        for p in layer.parameters():
+            p.normal_(0, 0.05, generator=gen)
+        w = layer.linear_proj.weight
+        room = torch.empty(w.numel() + (w.shape[0] - 1) * pad, dtype=w.dtype, device=dev)
+        w.data = room.as_strided(w.shape, (w.shape[1] + pad, 1)).copy_(w.data)
+        if by_module:
+            layer.linear_qkv.register_forward_hook(lambda m, i, o: None)
+        x = torch.empty(ctx.padded_active_token_count, 1, hidden, dtype=torch.bfloat16, device=dev).normal_(generator=gen)
+        outs.append((layer(x, ctx)[0], ctx.memory_buffer))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+
+
 def test_mask_of_bytes(mi, dev):
     lens = [5, 256, 17, 300, 1, 90]
     state = []
