@@ -552,6 +552,26 @@ int mi_update_requests_mask8(int32_t* request_ids, int32_t* request_query_length
                        int32_t chunk_size_tokens, int32_t max_requests, void* stream);
 
 /*
+ * Either of the two (mask_bytes: 4 or 1 per entry) that also zeroes `words_to_clear` words from `rows_to_clear` on (16-byte
+ * aligned, a multiple of 4, at most 2^20) unless the status is 1: the rows of the step that is over.
+ */
+int mi_update_requests_clearing(int32_t* request_ids, int32_t* request_query_lengths,
+                       int32_t* request_output_lengths, int32_t* request_kv_length_offsets,
+                       int32_t* request_kv_chunk_counts, int32_t* request_last_kv_chunk_id,
+                       int32_t* request_last_kv_chunk_offset, int32_t* request_to_kv_chunk_ids,
+                       int64_t table_stride, int32_t max_kv_chunk_count, int64_t* token_to_input_ids,
+                       int64_t* token_to_pos_ids, int64_t* token_to_request_idx,
+                       int64_t* token_to_position_in_request, int64_t* token_to_chunk_idx,
+                       int64_t* token_to_local_position_within_kv_chunk, int32_t* chunk_bag,
+                       const void* active_requests_mask, const int64_t* new_tokens,
+                       int64_t* paused_tokens, int64_t* next_tokens_scratch, int32_t* scratch,
+                       int32_t* newly_paused_request_ids, int32_t* finished_request_ids,
+                       int32_t* counters, int32_t total_request_count, int32_t paused_request_count,
+                       int32_t chunk_count_avail, int32_t gtd_chunk_count, int32_t gtd_request_count,
+                       int32_t chunk_size_tokens, int32_t max_requests,
+                       int32_t mask_bytes, int32_t* rows_to_clear, int64_t words_to_clear, void* stream);
+
+/*
  * The tensor writes of DynamicInferenceContext.add_request (dynamic_context.py:976-1015) as one kernel, after
  * the caller has made the reference's host-side checks (token / request / chunk / sequence-length overflow,
  * dynamic_context.py:945-974) and lowered the allocator's count by `chunk_count`: the request's row of every

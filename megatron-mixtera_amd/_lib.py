@@ -100,6 +100,8 @@ SIGNATURES = {
         c_int, [_P] * 8 + [_I64, _I32] + [_P] * 15 + [_I32] * 7 + [_P]),
     "mi_update_requests_mask8": (
         c_int, [_P] * 8 + [_I64, _I32] + [_P] * 15 + [_I32] * 7 + [_P]),
+    "mi_update_requests_clearing": (
+        c_int, [_P] * 8 + [_I64, _I32] + [_P] * 15 + [_I32] * 8 + [_P, _I64, _P]),
     "mi_step_attention_state": (
         c_int, [_P, _P, _P, _I64, _I32, _P, _P, _P, _P, _P, _I64, _P, _P, _P, _P] + [_I32] * 6 + [_P]),
     "mi_add_request": (c_int, [_P] * 8 + [_I64] + [_P] * 8 + [_I32] * 8 + [_P]),

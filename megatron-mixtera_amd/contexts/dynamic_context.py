@@ -729,6 +729,10 @@ class DynamicInferenceContext:
     # ------------------------------------------------------------------ per-step attention state
     def reset_attention_state(self) -> None:
         """Forget the per-step attention metadata (the fixed-address mirrors are zeroed)."""
+        self._forget_attention_state()
+        self._mirrors.zero_()
+
+    def _forget_attention_state(self) -> None:
         self._max_lengths_pending = False
         note_kv_lengths(getattr(self, 'cu_kv_seq_lengths', None), None)
         self.max_seqlen_q = None
@@ -737,7 +741,6 @@ class DynamicInferenceContext:
         self.cu_kv_seq_lengths = None
         self.kv_seq_lengths = None
         self.block_table = None
-        self._mirrors.zero_()
 
     def using_cuda_graph_this_step(self) -> bool:
         """Graph sizes exist, the step type may use them, and the batch fits the largest one."""
@@ -1106,14 +1109,22 @@ class DynamicInferenceContext:
             if self.paused_tokens.data_ptr() != self._paused_tokens_buf.data_ptr():
                 self._paused_tokens_buf[: self.paused_request_count] = self.paused_tokens[: self.paused_request_count]
         self._counters_host[5] = -1
-        ops.update_requests(self, mask, tokens)
+        # the caller keeps the list of finished requests: one of its own each time, instead of a copy behind the kernel
+        self._finished_ids_buf = torch.empty_like(self._finished_ids_buf)
+        # the kernel zeroes the mirrors itself while the host goes on, unless they are large or the reset is not the one below
+        clears = (self._mirrors.numel() <= ops.UPDATE_CLEARS_AT_MOST and "reset_attention_state" not in self.__dict__ and
+                  type(self).reset_attention_state is DynamicInferenceContext.reset_attention_state)
+        ops.update_requests(self, mask, tokens, self._mirrors if clears else None)
         self._await(self._counters, 5, self._counters_stream)
         if self._counters_stream == self._max_lengths_stream:
             self._max_lengths_in_flight = False   # (the stream is in order)
         total, paused, active, avail, n_newly, status, was_reset, n_finished = self._counters_host.tolist()
         assert status != 1, "active + finished + paused requests != total_request_count"
-        self.last_finished_request_ids = self._finished_ids_buf[:n_finished].clone()
-        self.reset_attention_state()
+        self.last_finished_request_ids = self._finished_ids_buf[:n_finished]
+        if clears:
+            self._forget_attention_state()
+        else:
+            self.reset_attention_state()
         assert status != 2, "active_request_count == 0."
         assert status != 3, (
             "The request_last_kv_chunk_offset should be 0 for the requests that just got resumed this step. ")

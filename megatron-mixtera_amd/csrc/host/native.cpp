@@ -1153,7 +1153,8 @@ PyObject* set_workspace(PyObject* const* a) {
 PyMethodDef kMethods[] = {
     ABI(mi_kv_append_decode), ABI(mi_kv_quantize_chunks_fp8), ABI(mi_kv_append_decode_fp8), ABI(mi_decode_workspace_bytes),
     ABI(mi_prefill_workspace_bytes), ABI(mi_paged_decode_attention_noalloc),
-    ABI(mi_update_requests), ABI(mi_update_requests_mask8), ABI(mi_add_request), ABI(mi_decode_attention_state), ABI(mi_step_attention_state),
+    ABI(mi_update_requests), ABI(mi_update_requests_mask8), ABI(mi_update_requests_clearing),
+    ABI(mi_add_request), ABI(mi_decode_attention_state), ABI(mi_step_attention_state),
     OP(kv_append, 6), OP(kv_append_fp8, 9), OP(paged_decode_attention, 14), OP(paged_mla_decode_attention, 10),
     OP(paged_prefill_attention, 14), OP(paged_prefill_attention_mla, 11), OP(norm_rope_append, 22), OP(qkv_norm_rope_append, 22), OP(qkv_key_append, 16),
     OP(qkv_prefill_attention, 18), OP(decode_step_attention, 29),

@@ -475,14 +475,22 @@ def watch(row: Tensor, index: int, value: int, microseconds: int) -> bool:
     return _native().watch(row, index, value, microseconds)
 
 
-def update_requests(ctx, mask: Tensor, new_tokens_i64: Tensor) -> None:
+# Words that the one workgroup of update_requests zeroes on the side: 256 KB take it 2 us or so, a launch of their own costs
+# the host five; beyond, many workgroups are the faster way.
+UPDATE_CLEARS_AT_MOST = 1 << 16
+
+
+def update_requests(ctx, mask: Tensor, new_tokens_i64: Tensor, clear: Optional[Tensor] = None) -> None:
     """Enqueue the single-kernel ``update_requests`` on the state tensors of ``ctx`` (results land in
-    ``ctx._counters``, pinned host memory, / ``ctx._newly_paused_buf`` / ``ctx._finished_ids_buf`` / ``ctx._paused_tokens_buf``)."""
+    ``ctx._counters``, pinned host memory, / ``ctx._newly_paused_buf`` / ``ctx._finished_ids_buf`` / ``ctx._paused_tokens_buf``).
+    ``clear``: contiguous int32 rows that it zeroes too."""
     table = ctx.request_to_kv_chunk_ids
     _require(table.stride(1) == 1, "request_to_kv_chunk_ids rows must be contiguous")
     native = _native()
     ctx._counters_stream = native.written_by_kernel(ctx._counters, table.device.index)
-    update = native.abi_mi_update_requests if mask.dtype == torch.int32 else native.abi_mi_update_requests_mask8
+    update, more = (native.abi_mi_update_requests if mask.dtype == torch.int32 else native.abi_mi_update_requests_mask8), ()
+    if clear is not None:
+        update, more = native.abi_mi_update_requests_clearing, (mask.element_size(), clear, clear.numel())
     _lib.check(update(
         ctx.request_ids, ctx.request_query_lengths, ctx.request_output_lengths,
         ctx.request_kv_length_offsets, ctx.request_kv_chunk_counts,
@@ -495,7 +503,7 @@ def update_requests(ctx, mask: Tensor, new_tokens_i64: Tensor) -> None:
         ctx._next_tokens_buf, ctx._update_scratch, ctx._newly_paused_buf,
         ctx._finished_ids_buf, ctx._counters, ctx.total_request_count, ctx.paused_request_count,
         ctx.chunk_allocator.chunk_count_avail, ctx.gtd_chunk_count, ctx.gtd_request_count,
-        ctx.chunk_size_tokens, ctx.max_requests, _stream(table)), "mi_update_requests")
+        ctx.chunk_size_tokens, ctx.max_requests, *more, _stream(table)), "mi_update_requests")
 
 
 def add_request(ctx, row: int, token_begin: int, tokens_i64: Tensor, n_chunks: int, stack_first: int,

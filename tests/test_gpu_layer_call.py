@@ -83,6 +83,32 @@ def test_mask_of_bytes(mi, dev):
     assert state[0] == state[1] and state[0][0] == 3
 
 
+@pytest.mark.parametrize("how", ["by the kernel", "large", "overridden"])
+def test_update_leaves_the_mirrors_zero(mi, dev, how, monkeypatch):
+    calls = []
+    if how == "large":
+        monkeypatch.setattr(mi.ops, "UPDATE_CLEARS_AT_MOST", 0)
+    if how == "overridden":
+        before = mi.DynamicInferenceContext.reset_attention_state
+        monkeypatch.setattr(mi.DynamicInferenceContext, "reset_attention_state", lambda c: (calls.append(1), before(c))[1])
+        class Other(mi.DynamicInferenceContext):
+            def reset_attention_state(self):
+                calls.append(2)
+                super().reset_attention_state()
+        monkeypatch.setattr(mi, "DynamicInferenceContext", Other)
+    ctx = _context(mi, dev, [5, 256, 17, 300], None)
+    finished = []
+    for mask in ([1, 0, 1, 1], [1, 0, 1], [0, 0]):      # (the last empties the context)
+        ctx._mirrors.fill_(7)
+        calls.clear()
+        ctx.update_requests(torch.tensor(mask, dtype=torch.uint8, device=dev), torch.arange(len(mask), device=dev))
+        assert not ctx._mirrors.any() and ctx.block_table is None and (calls == [2, 1] or how != "overridden")
+        finished.append(ctx.last_finished_request_ids)
+        if ctx.total_request_count:
+            ctx.initialize_attention_state()
+    assert [f.numel() for f in finished] == [1, 1, 2] and sorted(torch.cat(finished).tolist()) == [0, 1, 2, 3]
+
+
 DECODE_PARTS = ["core.forward_mixed_qkv", "class core.forward_mixed_qkv", "linear_qkv.forward", "linear_proj.forward",
                 "ctx.fused_decode_step_attention", "class ctx.fused_decode_step_attention", "ctx.key_value_cache"]
 PROMPT_PARTS = ["core._attend", "class core._attend", "ctx.fused_qkv_norm_rope_append",
