@@ -277,6 +277,10 @@ struct LinearPlan {
 // With few tokens 32 rows leave a quarter of the CUs without any (6144 rows: 192 workgroups) and 16 need a second round:
 // 24 fill the chip.  32 rows -> 24:  6144 x 4096, 16 tokens 13.0 -> 11.8 us, 24 tokens 14.9 -> 13.5;  5120 x 5120, 16 tokens
 // 16.1 -> 14.0;  10240 x 5120, one token 26.4 -> 24.0;  5120 x 8192, one token 18.9 -> 17.4.
+// Where a few more rows than the chip takes at once would need a second round, a workgroup with room for more tokens than
+// there are has 48 or 64 rows, and one round does: 10240 x 2048, one token 14.9 -> 11.4 us;  8448 x 4096 20.6 -> 17.3;
+// 10240 x 4096, 16 tokens 20.2 -> 18.2;  16384 x 4096, 24 tokens 32.2 -> 27.8.  (Not with up to four wavefronts, two such
+// workgroups share a CU: 16384 x 2048, one token 14.3 -> 16.7.)
 static LinearPlan linear_plan(int T, int N, int K, int slices) {
   LinearPlan best{};
   float least = 0.f;
@@ -291,16 +295,19 @@ static LinearPlan linear_plan(int T, int N, int K, int slices) {
     int covered = 0;
     for (const int xh : {1, 2, 4, 6, 8}) {
       const int blocks = (T + 8 * xh - 1) / (8 * xh) * z;
-      if (covered >= T) break;  // (the last one held all tokens)
+      const bool beyond = covered >= T;  // (the last one held all tokens)
+      if (beyond && z > 1) break;
       covered = 8 * xh;
       for (int rounds = fewest; rounds <= fewest + 2; ++rounds) {
         const int w = (per + rounds - 1) / rounds;
         for (const int rh : {2, 3, 4, 6, 8}) {
           if (!linear_instance(rh, xh, w, per)) continue;
           const int groups = (row_halves + rh - 1) / rh * blocks;
+          if (beyond && (w <= 4 || groups > 256)) continue;
           float us = merge + (float)((groups + 255) >> 8) *
                                        (4.6f + 3.f * (float)(rounds - 1) + column * ((float)rh * (8.f / 52e3f) + (float)xh * (8.f / 60e3f)));
           if (rh == 3) us *= 1.06f;   // (for less than that it is not the faster)
+          if (beyond) us *= 1.1f;     // (nor this)
           if (best.waves == 0 || us < least) {
             least = us;
             if (z == 1) undivided = groups;

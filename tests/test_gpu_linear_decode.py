@@ -64,9 +64,11 @@ def test_tile_edges(mi, dev, T, N, K):
 
 
 @pytest.mark.parametrize("T", [1, 8, 9, 16, 17, 32])
-@pytest.mark.parametrize("N,K", [(6144, 4096), (6128, 4096), (5120, 5120), (5104, 6144)])
+@pytest.mark.parametrize("N,K", [(6144, 4096), (6128, 4096), (5120, 5120), (5104, 6144),
+                                 (8208, 1056), (12288, 2592), (12304, 2592), (16384, 2592)])
 def test_workgroups_of_24_rows(mi, dev, T, N, K):
     """Row counts that 32 rows per workgroup would leave on part of the chip: whole workgroups, and a last one of 8 rows.
+    And those just above what the chip takes at once, in workgroups of 48 or 64 rows with room for more tokens.
     Guards around the weights are not numbers, guards around the result stay as they were."""
     gen = torch.Generator().manual_seed(T + N)
     x = (torch.randn(T, K, generator=gen) * 0.5).bfloat16().to(dev)
