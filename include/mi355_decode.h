@@ -265,7 +265,7 @@ int mi_decode_step_attention_fp8(const void* q, int64_t q_stride_tok, int64_t q_
 /*
  * Either of the two (kv_dtype MI_KV_16BIT: scales null, headroom any positive number; MI_KV_FP8_E4M3) with the 16-bit matrix
  * [next_rows][next_columns] of the mi_linear_decode call over R tokens that follows on the stream.  The results are theirs.
- * Where the batch leaves at least half of the workgroups without a span, those read the matrix meanwhile, so that the
+ * Where the batch leaves at least half of the workgroups without a span (and the cache is 16-bit), those read the matrix meanwhile, so that the
  * projection finds it in the L2 of the XCDs that will ask for it.  next_weight == NULL: nothing is read.  Otherwise rows and
  * strides as mi_linear_decode takes them (rows % 16 == 0, columns % 32 == 0 and below 2^20, 16-byte aligned rows).
  */

@@ -46,7 +46,8 @@ def test_one_call_equals_the_modules(mi, dev, lens, cache):
 @pytest.mark.parametrize("lens,hidden,heads,cache,pad", [
     ([5], 6112, 8, None, 0),           # workgroups of 24 rows: the last workgroup's rows end beyond the matrix
     ([600], 4096, 32, None, 8),        # rows apart, the last one at the end of its storage
-    ([3, 256], 5120, 64, "fp8_e4m3", 0),   # a matrix larger than what is read ahead
+    ([3, 256], 5120, 64, None, 0),     # a matrix larger than what is read ahead
+    ([3, 256], 5120, 64, "fp8_e4m3", 0),   # (nothing is read ahead)
     ([240] * 16, 2048, 16, None, 0),   # half of the workgroups have a span, or all
 ])
 def test_reading_the_projection_ahead_changes_nothing(mi, dev, lens, hidden, heads, cache, pad):
