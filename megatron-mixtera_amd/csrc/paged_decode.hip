@@ -1749,8 +1749,7 @@ static void launch_merge(const DecodeParams& p, int grid_x, int R, int Hq, int h
 }
 
 // What a decode step's idle workgroups read of the next projection's matrix, at most: the L2s of eight XCDs.  (A layer of
-// 4096, its 33.5 MB all read: 35.8 -> 34.4 us; with 26 MiB read of it, 35.5.  A matrix of 5120 x 8192, twice the L2s: 57.6
-// -> 56.3 us with 20, 26, 32 or 36 MiB.)
+// 4096, its 33.5 MB all read: 35.8 -> 34.4 us; with 20 or 26 MiB read of it, 35.5: the rest sets the projection's time.)
 constexpr int64_t kFetchBytes = (int64_t)32 << 20;
 
 // Requests one launch of the streaming kernels takes: their tile prefix sums and lengths sit in LDS.
