@@ -26,6 +26,7 @@ import torch.nn.functional as F
 from torch import Tensor
 
 from .. import ops
+from .._lib import native
 from ..flash_attn_interface import note_kv_lengths
 from .dynamic_chunk_allocator import ChunkAllocator
 
@@ -1111,9 +1112,8 @@ class DynamicInferenceContext:
         self._counters_host[5] = -1
         # the caller keeps the list of finished requests: one of its own each time, instead of a copy behind the kernel
         self._finished_ids_buf = torch.empty_like(self._finished_ids_buf)
-        # the kernel zeroes the mirrors itself while the host goes on, unless they are large or the reset is not the one below
-        clears = (self._mirrors.numel() <= ops.UPDATE_CLEARS_AT_MOST and "reset_attention_state" not in self.__dict__ and
-                  type(self).reset_attention_state is DynamicInferenceContext.reset_attention_state)
+        # the kernel zeroes the mirrors itself while the host goes on, unless they are large or the reset is not the one above
+        clears = self._mirrors.numel() <= ops.UPDATE_CLEARS_AT_MOST and native().as_defined(self, None, _RESET)
         ops.update_requests(self, mask, tokens, self._mirrors if clears else None)
         self._await(self._counters, 5, self._counters_stream)
         if self._counters_stream == self._max_lengths_stream:
@@ -1162,3 +1162,7 @@ class DynamicInferenceContext:
         chosen[q_lens.cumsum(0) - 1] = new_tokens
         picked = pick(chosen)
         return [lp.tolist() for lp in picked.cpu().split(q_lens.tolist(), dim=0)]
+
+
+# The reset that an update's kernel stands in for, as defined here: it is called where it was replaced.
+_RESET = (("reset_attention_state", DynamicInferenceContext.reset_attention_state),)

@@ -110,6 +110,27 @@ def test_update_leaves_the_mirrors_zero(mi, dev, how, monkeypatch):
     assert [f.numel() for f in finished] == [1, 1, 2] and sorted(torch.cat(finished).tolist()) == [0, 1, 2, 3]
 
 
+@pytest.mark.parametrize("where", ["class", "object", "subclass"])
+def test_a_replaced_reset_is_called(mi, dev, where, monkeypatch):
+    """A reset put on the class itself, on one context or in a subclass runs after every update, as the class's own does."""
+    calls = []
+    own = mi.DynamicInferenceContext.reset_attention_state
+    reset = lambda c: (calls.append(1), own(c))[1]
+    if where == "class":
+        monkeypatch.setattr(mi.DynamicInferenceContext, "reset_attention_state", reset)
+    elif where == "subclass":
+        monkeypatch.setattr(mi, "DynamicInferenceContext",
+                            type("Other", (mi.DynamicInferenceContext,), {"reset_attention_state": reset}))
+    ctx = _context(mi, dev, [5, 256, 17], None)
+    if where == "object":
+        ctx.reset_attention_state = lambda: reset(ctx)
+    for mask in ([1, 0, 1], [0, 0]):      # (the last empties the context)
+        ctx._mirrors.fill_(7)
+        calls.clear()
+        ctx.update_requests(torch.tensor(mask, dtype=torch.uint8, device=dev), torch.arange(len(mask), device=dev))
+        assert calls == [1] and not ctx._mirrors.any() and ctx.block_table is None
+
+
 DECODE_PARTS = ["core.forward_mixed_qkv", "class core.forward_mixed_qkv", "linear_qkv.forward", "linear_proj.forward",
                 "ctx.fused_decode_step_attention", "class ctx.fused_decode_step_attention", "ctx.key_value_cache"]
 PROMPT_PARTS = ["core._attend", "class core._attend", "ctx.fused_qkv_norm_rope_append",
