@@ -102,11 +102,6 @@ static __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
-// fp32 -> uint32, truncating: NaN and everything below 0 become 0, everything too large 2^32 - 1.
-static __device__ __forceinline__ uint32_t f32_to_u32_sat(float x) {
-  return (uint32_t)fmaxf(x, 0.f);   // (the conversion saturates)
-}
-
 // One row of logits.  DT = element type (0 fp32, 1 bf16, 2 fp16); VEC = elements per 16-byte load (4 fp32,
 // 8 of a 16-bit type) when the row is 16-byte aligned, 1 otherwise.
 template <int DT, int VEC>
@@ -246,7 +241,10 @@ static __device__ __forceinline__ void load_batch(const RowReader<DT, VEC>& rd, 
 // (sums are carried in 64 bits).  0 for anything that is not a number at or below the maximum.
 constexpr float kMassOne = 4294967040.0f;  // largest fp32 below 2^32
 static __device__ __forceinline__ uint64_t mass_of(float x, float neg_mx_log2e) {
-  return f32_to_u32_sat(__builtin_fmaf(fast_exp2(__builtin_fmaf(x, 1.4426950408889634f, neg_mx_log2e)), kMassOne, 0.5f));
+  const float e = fast_exp2(__builtin_fmaf(x, 1.4426950408889634f, neg_mx_log2e));
+  // (the exponential of a large maximum may round to more than one: what does not fit is no defined conversion.  The median
+  // of 0, e and 1 is 0 for NaN, and a bit of the exponential's instruction.)
+  return (uint32_t)__builtin_fmaf(__builtin_amdgcn_fmed3f(e, 0.f, 1.f), kMassOne, 0.5f);
 }
 
 // Whether a row with this maximum has a distribution to draw from.  Not where it is not a finite number, and not where it
@@ -539,8 +537,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleParams p) 
       const float inv_w = range > 0.f ? 256.f / range : 0.f;
       auto lin_bin = [&](float x) {
         const float f = (mx - x) * inv_w;
-        int b = f >= 255.f ? 255 : (int)f;  // NaN (inf * 0) compares false and converts to 0
-        return b < 0 ? 0 : b;
+        return (int)fminf(fmaxf(f, 0.f), 255.f);  // (NaN, as inf * 0, becomes 0)
       };
       auto weight_of = [&](float x) -> uint64_t { return by_count ? (uint64_t)1 : mass_of(x, neg_mx); };
       if (tid < 256) hist[tid] = 0;
@@ -903,9 +900,9 @@ __global__ __launch_bounds__(kSampleThreads) void sample_first_kernel(SplitParam
         for (int j = 0; j < VEC; ++j) {
           // distance from the first bin's upper edge, in bins; exp(-t / 64) by its chord, lowered to within 1.6e-5
           const float f = __builtin_fmaf(x[u][j], -kBinsPerUnit, edge);
-          const uint32_t bin = f32_to_u32_sat(f);
           const float w = __builtin_fmaf(__builtin_amdgcn_fractf(f), -0.01550356f * p.bin_one, 0.99998474f * p.bin_one);
-          if (bin < (uint32_t)kBins) atomicAdd(&mass[bin], f32_to_u32_sat(w));
+          // (a masked value is an infinite distance away, NaN no distance: both fail the comparison)
+          if (f < (float)kBins) atomicAdd(&mass[(uint32_t)fmaxf(f, 0.f)], (uint32_t)w);
         }
     }
     // The index matters where there may be nothing to draw from: no finite maximum (that of a part of nothing but -inf and
