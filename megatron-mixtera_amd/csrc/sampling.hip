@@ -900,7 +900,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_first_kernel(SplitParam
         for (int j = 0; j < VEC; ++j) {
           // distance from the first bin's upper edge, in bins; exp(-t / 64) by its chord, lowered to within 1.6e-5
           const float f = __builtin_fmaf(x[u][j], -kBinsPerUnit, edge);
-          const float w = __builtin_fmaf(__builtin_amdgcn_fractf(f), -0.01550356f * p.bin_one, 0.99998474f * p.bin_one);
+          const float w = __builtin_fmaf(__builtin_amdgcn_fractf(f), -0.01550356f * p.bin_one, 0.99998474f * p.bin_one + 0.5f);
           // (a masked value is an infinite distance away, NaN no distance: both fail the comparison)
           if (f < (float)kBins) atomicAdd(&mass[(uint32_t)fmaxf(f, 0.f)], (uint32_t)w);
         }
@@ -987,7 +987,9 @@ __global__ __launch_bounds__(kSampleThreads) void sample_mass_kernel(SplitParams
   float over = INFINITY, from = INFINITY;   // kept: above `over`; listed: from `from` to `over`
   if (filtered) {
     // The parts' bins on the row's scale, two per thread; the bin in which the running sum passes top_p of the total, with
-    // its neighbours where it passes within 1e-4 of the total of the edge (the sums are off by a few 1e-5).
+    // its neighbours where it passes within `slack` of the edge.  A value's weight is off by up to 1.6e-5 (the chord) and half
+    // a unit of 1 / bin_one (rounding) of itself, the share of the total that lies above an edge by a quarter of the range of
+    // these: 0.8e-5 + 0.26 / bin_one, 1.6e-5 up to 131 071 values, 4e-5 from 262 144 and 1.3e-4 from 2^20 on.
     auto add_item = [&](int n, uint4 c) {
       const int at = 256 * (n % kItems) + 4 * lane + __builtin_amdgcn_readlane(down, n / kItems);
       const uint32_t v[4] = {c.x, c.y, c.z, c.w};
@@ -1020,7 +1022,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_mass_kernel(SplitParams
       incl += w < wave ? red[w] : 0.f;
       total += red[w];
     }
-    const float want = p.s.top_p * total, slack = 1e-4f * total;
+    const float want = p.s.top_p * total, slack = fmaxf(1e-4f, 3e-5f + 0.3f / p.bin_one) * total;
     const bool in0 = incl - h - slack <= want && incl - h1 + slack > want && h0 > 0.f;
     const bool in1 = incl - h1 - slack <= want && incl + slack > want && h1 > 0.f;
     if (in0 || in1) {

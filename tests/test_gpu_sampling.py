@@ -7,6 +7,7 @@ the checker's decision has a margin (2e-6 of the total mass: the
 kernel's exponentials are fp32), and must in every case satisfy the definition within that margin
 (mass strictly above the cut <= top_p < mass down to the cut; CDF bracket of the drawn index).
 """
+import math
 from types import SimpleNamespace
 
 import pytest
@@ -497,6 +498,39 @@ def test_parts_where_the_bins_are_at_their_edges(mi, dev, R, V, pad, kind):
             torch.cuda.synchronize()
             assert torch.equal(got, want), (dtype, top_k, top_p)
             assert torch.equal(cut, want_cut), (dtype, top_k, top_p)
+
+
+@pytest.mark.parametrize("V", [1 << 18, 1 << 20])
+@pytest.mark.parametrize("first,last", [(0.5028, 5.9754), (0.5183, 5.9913)], ids=["truncated", "rounded"])
+def test_the_window_holds_the_cut_of_a_wide_row(mi, dev, V, first, last):
+    """The wider the row, the coarser the units in which a part's bins are summed (2^-11 of a value at 2^20): most of the mass
+    here lies at two values whose weights would be furthest apart after truncating, or are after rounding, the cut within 1e-5
+    of the edge between two bins that hold 1e-3 each.  Both have to be listed; otherwise one workgroup walks the row several
+    times, for the same token."""
+    lib = mi._lib.load()
+    value = lambda bins: (1.0 - bins) / 64      # `bins` below the upper edge of the first bin, whose number is 0
+    a, c1, c2, d = (value(f) for f in (first, 3.5, 4.5, last))
+    few = V // 1000
+    n_a = int((V - 2 * few) / (1 + math.exp(a - d)))    # as much mass in the first level as in the last
+    x = torch.full((V,), d)
+    x[:n_a], x[n_a:n_a + few], x[n_a + few:n_a + 2 * few] = a, c1, c2
+    w = x.double().exp()
+    top_p = float(w[:n_a + few].sum() / w.sum()) + 1e-5
+    x = x[torch.randperm(V, generator=torch.Generator().manual_seed(V))].view(1, V).to(dev)
+    u = torch.full((1,), 0.37, device=dev)
+    room = torch.zeros(lib.mi_sample_workspace_bytes(1, V, 0, top_p), dtype=torch.uint8, device=dev)
+    got = []
+    for ws, size in ((room.data_ptr(), room.numel()), (None, 0)):
+        token = torch.empty(1, dtype=torch.int64, device=dev)
+        cut = torch.empty(1, dtype=torch.float32, device=dev)
+        rc = lib.mi_sample_from_logits_ws(x.data_ptr(), V, 0, 1, V, 0, top_p, 1.0, u.data_ptr(), 0, token.data_ptr(), cut.data_ptr(),
+                                          None, None, None, -1, None, ws, size, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, lib.mi_last_error()
+        got.append((token.item(), cut.item()))
+    assert got[0] == got[1] and got[0][1] == torch.tensor(c2, dtype=torch.float32).item()
+    # (the workspace: four rows of a word per part, each on a line of 256 bytes; the last counts what the parts listed)
+    parts = min(V // 4096, 64)
+    assert room[768:768 + 4 * parts].view(torch.int32).sum().item() == 2 * few
 
 
 @pytest.mark.parametrize("buffer", ["whole", "off a line", "too small", "on the host", "empty"])
