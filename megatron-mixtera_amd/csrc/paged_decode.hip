@@ -822,7 +822,7 @@ static __device__ __forceinline__ void walk_segments(const DecodeParams& p, Seg 
       }
     }
     __syncthreads();
-    cum_l = cum[lane];
+    cum_l = cum[min(lane, p.R - 1)];
     total = __builtin_amdgcn_readfirstlane(cum[p.R - 1]);
   }
   auto cum_of = [&](int i) {   // (i wave-uniform)
