@@ -912,9 +912,9 @@ PyObject* attention_layer_decode(PyObject* const* a) {
   Drop d0{mixed}, d1{PyLong_FromLong(0)}, d2{PyFloat_FromDouble(1.0)};
   PyObject* const step[29] = {none, none, none, mixed, a[5], a[6], a[7], a[8], a[9], a[10], a[11], a[12], a[13], a[14], a[15],
                               none, a[16], d2.o, a[17], a[18], d1.o, none, none, Py_True, a[19], a[20], a[21], a[22], a[23]};
-  // (a matrix that the projection below refuses is its to refuse)
-  const Tensor* proj = opt_tensor(a[3], "weight");
-  const bool fetchable = proj && proj->dim() == 2 && proj->stride(1) == 1 && is_16bit(*proj) && proj->device() == tensor(a[7], "k_cache").device() &&
+  // (a matrix that the projection below refuses is its to refuse; with an fp8 cache nothing is read ahead)
+  const Tensor *proj = opt_tensor(a[3], "weight"), &cache = tensor(a[7], "k_cache");
+  const bool fetchable = proj && cache.element_size() != 1 && proj->dim() == 2 && proj->stride(1) == 1 && is_16bit(*proj) && proj->device() == cache.device() &&
                          proj->size(0) > 0 && proj->size(0) % 16 == 0 && proj->size(1) > 0 && proj->size(1) % 32 == 0 &&
                          proj->stride(0) >= proj->size(1) && proj->stride(0) % 8 == 0 && proj->size(0) < (1 << 30) &&
                          proj->size(1) < (1 << 20) && (reinterpret_cast<uintptr_t>(proj->data_ptr()) & 15) == 0;

@@ -1934,7 +1934,8 @@ int mi::launch_paged_decode(
     // (as much of the next projection's matrix as the eight L2s hold, the same share of every workgroup's rows)
     p.next_w = nullptr;
     int rows = 0;
-    if (fused->next_weight && (rows = linear_rows_per_workgroup(R, fused->next_rows, fused->next_columns)) > 0) {
+    if (fused->next_weight && kv_dtype != MI_KV_FP8_E4M3 &&   // (that kernel reads nothing ahead)
+        (rows = linear_rows_per_workgroup(R, fused->next_rows, fused->next_columns)) > 0) {
       p.next_w = (const uint8_t*)fused->next_weight; p.next_st = fused->next_stride_row * 2;
       p.next_n = fused->next_rows; p.next_bytes = fused->next_columns * 2; p.next_rows = rows;
       p.next_blocks = (p.next_n + rows - 1) / rows;
