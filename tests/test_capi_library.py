@@ -155,3 +155,51 @@ def test_missing_library_is_an_error(mi, tmp_path, monkeypatch):
     monkeypatch.setattr(mi._lib, "LIB_PATH", tmp_path / "libmi355_decode.so")
     with pytest.raises(mi._lib.LibraryMissingError):
         mi._lib.load()
+
+
+def test_the_matrix_read_ahead_is_refused_where_its_projection_would_be(mi):
+    """mi_decode_step_attention_before_linear: rows a multiple of 16, columns a multiple of 32 below 2^20, rows that do not
+    overlap and start on 16 bytes.  (Host checks: the pointers are never followed; a null matrix passes them and the call ends
+    at the next one, the workspace that is too small.)"""
+    lib = mi._lib.load()
+    one = ctypes.c_void_p(16)
+
+    def call(weight=16, stride=4096, rows=4096, columns=4096, kv_dtype=0):
+        return lib.mi_decode_step_attention_before_linear(
+            one, 1024, 128, one, 1024, 128, one, 1024, 128, None, None, 1e-5, 0, None, 0, 0, 0, 1.0, None, one, one, 2048, 128, 128,
+            kv_dtype, one, one, 2.0, one, 1, one, one, 1024, 128, one, 0, 1, 8, 8, 128, 16, 0, 0.1, 1, 0, None,
+            ctypes.c_void_p(weight), stride, rows, columns, None)
+
+    for kv_dtype in (0, 1):
+        assert call(weight=None, stride=0, rows=0, columns=0, kv_dtype=kv_dtype) == -5
+        assert call(kv_dtype=kv_dtype) == -5 and b"workspace" in lib.mi_last_error()
+        for bad in (dict(rows=0), dict(rows=-16), dict(rows=24), dict(columns=0), dict(columns=-32), dict(columns=48),
+                    dict(columns=1 << 20, stride=1 << 20), dict(stride=4088)):
+            assert call(kv_dtype=kv_dtype, **bad) == -2 and b"next projection" in lib.mi_last_error(), bad
+        for bad in (dict(weight=24), dict(stride=4100)):
+            assert call(kv_dtype=kv_dtype, **bad) == -3 and b"16-byte" in lib.mi_last_error(), bad
+
+
+def test_rows_to_clear_are_refused_where_the_kernel_could_not_zero_them(mi):
+    lib = mi._lib.load()
+    one = ctypes.c_void_p(16)
+
+    def call(mask_bytes=4, rows=16, words=64, requests=0):
+        return lib.mi_update_requests_clearing(*[one] * 8, 4, 4, *[one] * 15, requests, 0, 1, 0, 0, 16, 4, mask_bytes,
+                                               ctypes.c_void_p(rows), words, None)
+
+    assert call(requests=5) == -2 and b"counts" in lib.mi_last_error()      # (more than max_requests)
+    for bad in (dict(mask_bytes=0), dict(mask_bytes=2), dict(mask_bytes=8), dict(words=-4), dict(words=62),
+                dict(words=(1 << 20) + 4), dict(rows=None)):
+        assert call(**bad) == -2 and b"masks of 1 or 4 bytes" in lib.mi_last_error(), bad
+    assert call(rows=20) == -3 and b"16-byte" in lib.mi_last_error()
+
+
+@pytest.mark.parametrize("T,N,K,read", [
+    (1, 6112, 1024, True), (1, 4096, 4096, True), (2, 5120, 8192, True), (16, 2048, 2048, True), (64, 4096, 4096, True),
+    (1, 16, 32, True), (64, 5120, 8192, False), (257, 4096, 4096, False), (0, 4096, 4096, False)])
+def test_which_projections_are_read_ahead(mi, T, N, K, read):
+    """The rows of one workgroup of the projection, which a decode step's idle workgroups read for it; none where K has parts
+    or a row is read by workgroups on several XCDs."""
+    rows = ctypes.CDLL(str(mi._lib.LIB_PATH))._ZN2mi25linear_rows_per_workgroupEiii(T, N, K)
+    assert rows in ((16, 24, 32, 48, 64) if read else (0,))

@@ -334,3 +334,19 @@ def test_fused_step_of_the_most_requests_one_launch_takes(mi, dev):
     # most 2^-7 of the value) on top of what a query's last bit moves
     a, b = out_a.float(), out_b.float()
     assert ((a - b).abs() <= 8e-3 + b.abs() / 128).all()
+
+
+@pytest.mark.parametrize("R", [3, 7680])
+def test_fused_step_of_the_widest_heads_in_eight_wavefronts(mi, dev, R):
+    """Eight wavefronts with sixteen query rows of 256 values each: 92 KB of LDS for any batch, 154 KB with the most requests
+    one launch takes."""
+    Hq, Hkv, d = 68, 4, 256      # (17 query heads per KV head: two wavefronts each, the second with one head)
+    lens = [1 + i % 3 for i in range(R)]
+    case, lens, qw, kw, pos = _step_case(mi, dev, Hq=Hq, Hkv=Hkv, d=d, chunk=16, lens=lens, dtype=torch.bfloat16, seed=R)
+    table = orn.rotary_table(4096, d, base=500000.0)
+    (out_a, kc_a, vc_a), (out_b, kc_b, vc_b) = _run_both(mi, dev, case, lens, qw, kw, pos, norm="rms", table=table,
+                                                         interleaved=False, mixed=False, max_kv_len=int(lens.max()))
+    assert torch.equal(kc_a, kc_b) and torch.equal(vc_a, vc_b)
+    # (the bound of the test above)
+    a, b = out_a.float(), out_b.float()
+    assert ((a - b).abs() <= 8e-3 + b.abs() / 128).all()

@@ -131,6 +131,18 @@ def test_a_replaced_reset_is_called(mi, dev, where, monkeypatch):
         assert calls == [1] and not ctx._mirrors.any() and ctx.block_table is None
 
 
+@pytest.mark.parametrize("dtype", [torch.int32, torch.uint8])
+@pytest.mark.parametrize("words", [0, 4, 4096 + 12])
+def test_update_clears_the_rows_it_is_given_and_no_other(mi, dev, dtype, words):
+    ctx = _context(mi, dev, [5, 256, 17], None)
+    rows = torch.full((words + 8,), 7, dtype=torch.int32, device=dev)
+    mirrors = ctx._mirrors.fill_(3).clone()
+    mi.ops.update_requests(ctx, torch.tensor([1, 0, 1], dtype=dtype, device=dev), torch.arange(3, device=dev), rows[4:4 + words])
+    torch.cuda.synchronize()
+    assert ctx._counters_host.tolist()[:2] == [2, 0] and torch.equal(ctx._mirrors, mirrors)
+    assert (rows[:4] == 7).all() and (rows[4 + words:] == 7).all() and not rows[4:4 + words].any()
+
+
 DECODE_PARTS = ["core.forward_mixed_qkv", "class core.forward_mixed_qkv", "linear_qkv.forward", "linear_proj.forward",
                 "ctx.fused_decode_step_attention", "class ctx.fused_decode_step_attention", "ctx.key_value_cache"]
 PROMPT_PARTS = ["core._attend", "class core._attend", "ctx.fused_qkv_norm_rope_append",
