@@ -35,20 +35,20 @@ MFMA_BF16_PEAK_TFLOPS = 2500.0  # MI355X dense bf16 matrix peak, published
 # read from inside the benchmark, so the figure is recorded here per workload; None = not collected.
 MEASURED_HBM_TRAFFIC_BYTES = {
     # decode workloads: "<cfg>" = the attention-only streaming kernel, "<cfg>_step" = the one-kernel decode step
-    "cfg2": 1_226_900_000, "cfg2_step": 1_215_100_000, "cfg4": 8_726_200_000, "cfg4_step": 8_635_500_000,
-    "cfg5": 9_072_200_000, "cfg5_step": 9_051_100_000,
+    "cfg2": 1_226_700_000, "cfg2_step": 1_214_700_000, "cfg4": 8_726_100_000, "cfg4_step": 8_633_200_000,
+    "cfg5": 9_070_100_000, "cfg5_step": 9_045_200_000,
     # the mixed step: tile kernel, stream kernel
-    "cfg3_tile": 401_800_000, "cfg3_stream": 2_195_100_000,
+    "cfg3_tile": 401_800_000, "cfg3_stream": 2_195_700_000,
     # multi-latent decode at 128 heads (reads + the partial results it writes)
-    "mla_decode_h128": 454_500_000, "mla_decode_h128_long": 1_305_000_000}
+    "mla_decode_h128": 452_800_000, "mla_decode_h128_long": 1_309_900_000}
 # Where each figure above was read, so that a reader of the JSON line can tell a stale constant from a fresh one:
 # the summary file and the last commit that touched the kernel when the counters were collected.
 _DECODE_TRAFFIC = ("profiles/decode_stream_kernels_hbm_traffic_cfg2_cfg4_cfg5.md (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, "
-                   "library as of commit 2060602)")
+                   "library as of commit 18b0bde)")
 _MIXED_TRAFFIC = ("profiles/paged_prefill_woven_kernel_cfg3_mfma.md (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, library as of "
-                  "commit 2060602)")
+                  "commit 18b0bde)")
 _MLA_HEADS_TRAFFIC = ("profiles/paged_mla_decode_heads_kernel_h128_counters.md (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, "
-                      "kernel as of commit c8e09ff; the row pitch changed since, the traffic does not depend on it)")
+                      "library as of commit 18b0bde)")
 TRAFFIC_SOURCE = {"mla_decode_h128": _MLA_HEADS_TRAFFIC, "mla_decode_h128_long": _MLA_HEADS_TRAFFIC, "cfg2": _DECODE_TRAFFIC, "cfg2_step": _DECODE_TRAFFIC, "cfg4": _DECODE_TRAFFIC,
                   "cfg4_step": _DECODE_TRAFFIC, "cfg5": _DECODE_TRAFFIC, "cfg5_step": _DECODE_TRAFFIC, "cfg3_tile": _MIXED_TRAFFIC,
                   "cfg3_stream": _MIXED_TRAFFIC}

@@ -275,11 +275,12 @@ struct LinearPlan {
 // cache) or parts fill it; 64 tokens, against 64 in a workgroup and one part:
 //   2048 x 8192 28.3 -> 19.1 us,  5120 x 8192 34.7 -> 26.3,  1280 x 5120 22.6 -> 12.7,  2048 x 4096 15.4 -> 12.5
 // With few tokens 32 rows leave a quarter of the CUs without any (6144 rows: 192 workgroups) and 16 need a second round:
-// 24 fill the chip.  32 rows -> 24:  6144 x 4096, 16 tokens 13.0 -> 11.8 us, 24 tokens 14.9 -> 13.5;  5120 x 5120, 16 tokens
-// 16.1 -> 14.0;  10240 x 5120, one token 26.4 -> 24.0;  5120 x 8192, one token 18.9 -> 17.4.
+// 24 fill the chip.  Without them -> with them (weights from HBM):  6144 x 4096, 16 tokens 12.9 -> 12.1 us, 24 tokens 15.1 ->
+// 13.8 (1 to 8 tokens 12.1-12.5 either way);  5120 x 5120, one token 14.5 -> 13.1, 16 tokens 15.7 -> 14.1;  10240 x 5120, one
+// token 26.3 -> 23.5;  5120 x 8192, one token 18.7 -> 17.3.
 // Where a few more rows than the chip takes at once would need a second round, a workgroup with room for more tokens than
-// there are has 48 or 64 rows, and one round does: 10240 x 2048, one token 14.9 -> 11.4 us;  8448 x 4096 20.6 -> 17.3;
-// 10240 x 4096, 16 tokens 20.2 -> 18.2;  16384 x 4096, 24 tokens 32.2 -> 27.8.  (Not with up to four wavefronts, two such
+// there are has 48 or 64 rows, and one round does: 10240 x 2048, one token 16.4 -> 12.3 us;  8448 x 4096 19.6 -> 16.0;
+// 10240 x 4096, 16 tokens 20.5 -> 18.3;  16384 x 4096, 24 tokens 32.2 -> 28.3.  (Not with up to four wavefronts, two such
 // workgroups share a CU: 16384 x 2048, one token 14.3 -> 16.7.)
 static LinearPlan linear_plan(int T, int N, int K, int slices) {
   LinearPlan best{};

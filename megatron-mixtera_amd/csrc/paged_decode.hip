@@ -109,8 +109,9 @@ static __host__ __device__ __forceinline__ int fused_lds_per_wave(int head_dim, 
 // shared 576-wide row, the caller points both cache arguments at the same buffer).
 //
 // FUSED: the segment starts from the RAW queries of the step and does what the separate norm / rotary / append
-// launch does (same arithmetic and rounding points as norm_rope_append_kernel): every segment normalises and
-// rotates its query rows in registers; the segment that ends the request (`final_seg`: the only one that reads
+// launch does (same arithmetic and rounding points as norm_rope_append_kernel; a key's sum of squares in its order too, a
+// query's in another, so a query element may differ in its last bit): every segment normalises and
+// rotates its query rows (see fused_queries); the segment that ends the request (`final_seg`: the only one that reads
 // the step's new token) first normalises and rotates the new key row of its KV head, writes it and the value
 // row into their cache slot, and takes both from LDS for its last tile.  `q_lds` is then this wavefront's
 // piece of LDS for cos / sin of the request's position [2][HDK], the key row [HDK] (fp32) and the query rows.
@@ -944,7 +945,7 @@ static __device__ __forceinline__ void decode_stream_body(const DecodeParams& p)
   const int hq0 = h * p.G + 16 * part;
   const int gq = min(16, p.G - 16 * part);
   // behind the two integer arrays, per wavefront: 16 query rows (wide keys) or the fused step's cos / sin / key
-  // row (see decode_segment)
+  // row and its query rows (see decode_segment)
   uint8_t* const q_lds = reinterpret_cast<uint8_t*>(cum) + (((size_t)p.R * 8 + 15) & ~(size_t)15) +
                          (size_t)wave * (FUSED ? (size_t)fused_lds_per_wave(HDK, p.G) : (size_t)(16 * (HDK * 2 + 16)));
   walk_segments<16 * NT>(p, [&](int r, int row, int len, int start, int end, bool whole, bool final_seg, int slot) {
@@ -1947,7 +1948,7 @@ int mi::launch_paged_decode(
   const int waves = head_waves(Hq, Hkv);
   const int wpb = pick_waves_per_block(waves, tune);
   dim3 grid(grid_x, waves / wpb), block(64 * wpb);
-  // (fused step: per wavefront cos | sin | key row in fp32 behind the per-request arrays)
+  // (fused step: per wavefront cos, sin and key row in fp32 and the query rows behind the per-request arrays)
   const size_t lds = fused ? (((size_t)R * 2 * sizeof(int32_t) + 15) & ~(size_t)15) + (size_t)wpb * fused_lds_per_wave(head_dim, G)
                            : (size_t)R * 2 * sizeof(int32_t);
   hipStream_t st = (hipStream_t)stream;
