@@ -240,11 +240,25 @@ static __device__ __forceinline__ void load_batch(const RowReader<DT, VEC>& rd, 
 // exp(x - mx) as fixed point, rounded to the nearest 2^-32: one 32-bit conversion per element
 // (sums are carried in 64 bits).  0 for anything that is not a number at or below the maximum.
 constexpr float kMassOne = 4294967040.0f;  // largest fp32 below 2^32
+static __device__ __forceinline__ float mass_f(float x, float neg_mx_log2e) {
+  return __builtin_fmaf(fast_exp2(__builtin_fmaf(x, 1.4426950408889634f, neg_mx_log2e)), kMassOne, 0.5f);
+}
+// The conversion is the instruction's: truncated, 0 for NaN, and 2^32 - 1 for what does not fit -- a large maximum's
+// exponential rounds to more than one -- where C++ leaves it undefined.  (The compiler's own saturating form is five
+// instructions, a comparison and a selection cost the walks 3-5 %.)  Inline assembly is not moved out of a branch: where a mass
+// may or may not count, it is made first and selected then (200 x 50 304 by one workgroup per row, top-p: 73.2 -> 69.6 us).  Its
+// operand comes from a fused multiply-add: a result of the transcendental unit would need a wait that is not inserted here.
 static __device__ __forceinline__ uint64_t mass_of(float x, float neg_mx_log2e) {
-  const float e = fast_exp2(__builtin_fmaf(x, 1.4426950408889634f, neg_mx_log2e));
-  // (the exponential of a large maximum may round to more than one: what does not fit is no defined conversion.  The median
-  // of 0, e and 1 is 0 for NaN, and a bit of the exponential's instruction.)
-  return (uint32_t)__builtin_fmaf(__builtin_amdgcn_fmed3f(e, 0.f, 1.f), kMassOne, 0.5f);
+  uint32_t m = __float_as_uint(mass_f(x, neg_mx_log2e));
+  asm("v_cvt_u32_f32 %0, %0" : "+v"(m));
+  return m;
+}
+// The same added to a sum {lo, hi}, in one statement: apart, 32 of them at once spill ten registers (64 x 128 256, top-p: 28.0
+// against 30.9 us).
+static __device__ __forceinline__ void add_mass(uint32_t& lo, uint32_t& hi, float x, float neg_mx_log2e) {
+  float m = mass_f(x, neg_mx_log2e);
+  asm("v_cvt_u32_f32 %2, %2\n\tv_add_co_u32 %0, vcc, %0, %2\n\tv_addc_co_u32 %1, vcc, 0, %1, vcc"
+      : "+v"(lo), "+v"(hi), "+v"(m) : : "vcc");
 }
 
 // Whether a row with this maximum has a distribution to draw from.  Not where it is not a finite number, and not where it
@@ -500,13 +514,17 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleParams p) 
 #pragma unroll
         for (int j = 0; j < kSamplesPerThread; ++j) {
           const float x = rd.at(tid * (V / kSampleThreads) + j);
-          below += order_key(x) < tau ? mass_of(x, neg_mx) : 0;
+          const uint64_t w = mass_of(x, neg_mx);
+          below += order_key(x) < tau ? w : 0;
         }
         const double rest = (double)workgroup_sum(below) * ((double)V / kMemberCap) * 1.25;
         usable = (double)c > (double)p.top_p * ((double)c + rest);
         if (usable) {
           uint64_t z = 0;
-          sweep<U>(rd, 0, V, tid, kSampleThreads, [&](int, float x, bool in) { z += in ? mass_of(x, neg_mx) : 0; });
+          sweep<U>(rd, 0, V, tid, kSampleThreads, [&](int, float x, bool in) {
+            const uint64_t w = mass_of(x, neg_mx);
+            z += in ? w : 0;
+          });
           z = workgroup_sum(z);
           target = (uint64_t)((double)p.top_p * (double)z);
           usable = c > target;
@@ -654,7 +672,10 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleParams p) 
         drawn = true;
       }
     }
-    auto kept_mass = [&](float x) -> uint64_t { return order_key(x) >= cut_key ? mass_of(x, neg_mx) : 0; };
+    auto kept_mass = [&](float x) -> uint64_t {
+      const uint64_t w = mass_of(x, neg_mx);
+      return order_key(x) >= cut_key ? w : 0;
+    };
     if (!drawn) {
       const int L1 = ((V + kSampleWaves - 1) / kSampleWaves + 63) & ~63;  // elements per first-level range
       {
@@ -977,12 +998,13 @@ __global__ __launch_bounds__(kSampleThreads) void sample_mass_kernel(SplitParams
   if (tid == 0) { window[0] = kBins; window[1] = -1; listed = 0; }
   const float row_first = floorf(mx * kBinsPerUnit);
   const int down = (int)fminf(row_first - first, (float)kBins);   // by how many bins each part's begin below the row's
-  uint64_t all = 0, kept = 0;
+  uint64_t kept = 0;
+  uint32_t all_lo = 0, all_hi = 0;
   auto masses = [&] {
 #pragma unroll
     for (int u = 0; u < BATCH / VEC; ++u)
 #pragma unroll
-      for (int j = 0; j < VEC; ++j) all += mass_of(x[u][j], neg_mx);
+      for (int j = 0; j < VEC; ++j) add_mass(all_lo, all_hi, x[u][j], neg_mx);
   };
   masses();
   float over = INFINITY, from = INFINITY;   // kept: above `over`; listed: from `from` to `over`
@@ -1053,7 +1075,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_mass_kernel(SplitParams
           uint64_t m = __builtin_amdgcn_ballot_w64(v >= from);
           if (m) {   // (few values are: their mass again is less than holding it)
             const bool is_over = v > over;
-            kept += is_over ? mass_of(v, neg_mx) : 0;
+            const uint64_t w = mass_of(v, neg_mx);
+            kept += is_over ? w : 0;
             m &= ~__builtin_amdgcn_ballot_w64(is_over);
             found += (uint32_t)__builtin_popcountll(m);
           }
@@ -1081,7 +1104,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_mass_kernel(SplitParams
       masses();
     }
   }
-  all = wave_sum_u64(all);
+  uint64_t all = wave_sum_u64(((uint64_t)all_hi << 32) | all_lo);
   kept = filtered ? wave_sum_u64(kept) : all;
   if (lane == 0) {
     p.run_mass[row_part * kRuns + wave] = kept;
@@ -1275,7 +1298,10 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SplitParams
   const int pa = (run / kRuns) * p.part_len, ra = pa + (run % kRuns) * p.run_len;
   const int rb = min(min(ra + p.run_len, pa + p.part_len), p.s.V);
   const int per = (p.run_len + kSampleThreads - 1) / kSampleThreads;
-  auto kept_mass = [&](float x) -> uint64_t { return order_key(x) >= cut_key ? mass_of(x, neg_mx) : 0; };
+  auto kept_mass = [&](float x) -> uint64_t {
+    const uint64_t w = mass_of(x, neg_mx);
+    return order_key(x) >= cut_key ? w : 0;
+  };
   const int a = min(ra + tid * per, rb), b = min(a + per, rb);
   uint64_t s = 0;
   for (int i = a; i < b; ++i) s += kept_mass(rd.at(i));
