@@ -764,9 +764,9 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleParams p) 
 //
 // fp32, 128 256 wide, us per call in a graph, one workgroup per row -> parts (flat rows: N(0, 3); peaked: 32 logits 9-15 above
 // N(0, 2)):
-//   64 rows: greedy 15 -> 12, plain 37 -> 21, top-k 50 39 -> 31, top-p 0.9 100 -> 28 (flat rows), 54 -> 26 (peaked)
-//    1 row : greedy 13 ->  6, plain 34 -> 13, top-k 50 36 -> 18, top-p 0.9  70 -> 20 (flat rows), 50 -> 20 (peaked)
-// 64 flat rows, top-p, by trace: 8.3 us for the first walk, 11.1 for the second, 8.3 for the pick (a chain of loads and
+//   64 rows: greedy 15 -> 12, plain 37 -> 21, top-k 50 39 -> 31, top-p 0.9 102 -> 28 (flat rows), 54 -> 27 (peaked)
+//    1 row : greedy 13 ->  6, plain 34 -> 13, top-k 50 36 -> 18, top-p 0.9  70 -> 21 (flat rows), 50 -> 20 (peaked)
+// 64 flat rows, top-p, by trace: 8.4 us for the first walk, 10.3-11 for the second, 8.4-9 for the pick (a chain of loads and
 // barriers).  Both walks are vector arithmetic and one burst of loads: what they gained (17.9, 14.5 and 11.7 us) is fewer
 // instructions per value.  The first took 38, with bins below a sampled reference, an exponential and a 64-bit addition to
 // LDS per value; with the batch in registers its own maximum is the reference, a 32-bit weight within the bin does, and
@@ -1466,7 +1466,7 @@ extern "C" int mi_last_token_gather(const void* src, int64_t src_stride_row, voi
 }
 
 // Parts a row is cut into: as many workgroups as the chip takes at once (one per CU: a second round costs more than
-// larger parts, 83 x 50 304 top-p in 4 parts 45 us, in 3 33 with the walks of then, 23.6 now), parts of at least 4 096 elements.
+// larger parts, 83 x 50 304 top-p in 4 parts 45 us, in 3 33 with the walks of then, 24 now), parts of at least 4 096 elements.
 static int sample_parts(int R, int V) {
   int parts = 256 / R;
   if (parts > V / 4096) parts = V / 4096;
@@ -1474,13 +1474,13 @@ static int sample_parts(int R, int V) {
 }
 // Whether the rows are done in parts.  The further launches cost 3-6 us, so the walks they shorten have to be long enough; from
 // 129 rows on a row has one part.  fp32 in a graph, us, one workgroup per row against parts:
-//   greedy, one walk to shorten: 64 x 151 936 16.8 / 11.9, 64 x 32 768 below the line 6.2 / 7.5;
-//   plain draws, two: 64 x 50 304 19.3 / 15.7, 64 x 32 768 below it 13.2 / 13.7;
-//   top-k, whose pick grows with its lists: 64 x 128 256 39.1 / 31.1, and does not gain from two: 128 x 100 352 35.1 / 37.3;
-//   top-p, three: 64 x 16 384 30.1 / 19.0, 64 x 128 256 99.7 / 27.9.
+//   greedy, one walk to shorten: 64 x 151 936 16.9 / 12.0, 64 x 32 768 below the line 6.2 / 7.5;
+//   plain draws, two: 64 x 50 304 19.4 / 16.0, 64 x 32 768 below it 13.5 / 13.7;
+//   top-k, whose pick grows with its lists: 64 x 128 256 39.1 / 31.1, and does not gain from two: 128 x 100 352 35.2 / 37.7;
+//   top-p, three: 64 x 16 384 30.0 / 19.4, 64 x 128 256 101.8 / 28.1.
 // Between 65 and 128 rows the lines for draws (49 152 and 65 536 wide) are those of longer walks: today top-p gains below them
-// too (86 x 50 304 65.4 / 23.1, 128 x 16 384 38.0 / 18.3), a plain draw from 50 304 on (128 rows 19.5 / 18.2).  So does greedy
-// from 50 304 on with few rows (1 x 65 536 7.8 / 6.0).
+// too (86 x 50 304 65.4 / 23.1, 128 x 16 384 37.9 / 18.3), a plain draw from 50 304 on (128 rows 20.6 / 18.2).  So does greedy
+// from 50 304 on with few rows (1 x 65 536 7.8 / 6.1).
 static bool sample_in_parts(int R, int V, int top_k, float top_p) {
   if (V < kFastMinVocab || R > 128 || top_k > kFastTopK) return false;
   if (top_k == 1) return V >= 1600 * (R > 50 ? R : 50);
