@@ -17,6 +17,8 @@
 // order of the atomic additions and a replay of the same call gives the same token.  The draw
 // itself is an inverse-CDF lookup in vocabulary order driven by one caller-supplied uniform
 // number per row (three levels: 16 ranges -> 16 sub-ranges -> elements).
+#include <type_traits>
+
 #include "mi_common.h"
 #include "mi_capi_internal.h"
 
@@ -255,10 +257,15 @@ static __device__ __forceinline__ uint64_t mass_of(float x, float neg_mx_log2e) 
 }
 // The same added to a sum {lo, hi}, in one statement: apart, 32 of them at once spill ten registers (64 x 128 256, top-p: 28.0
 // against 30.9 us).
-static __device__ __forceinline__ void add_mass(uint32_t& lo, uint32_t& hi, float x, float neg_mx_log2e) {
+static __device__ __forceinline__ uint32_t add_mass(uint32_t& lo, uint32_t& hi, float x, float neg_mx_log2e) {
   float m = mass_f(x, neg_mx_log2e);
   asm("v_cvt_u32_f32 %2, %2\n\tv_add_co_u32 %0, vcc, %0, %2\n\tv_addc_co_u32 %1, vcc, 0, %1, vcc"
       : "+v"(lo), "+v"(hi), "+v"(m) : : "vcc");
+  return __float_as_uint(m);
+}
+
+static __device__ __forceinline__ void add_u32(uint32_t& lo, uint32_t& hi, uint32_t m) {
+  asm("v_add_co_u32 %0, vcc, %0, %2\n\tv_addc_co_u32 %1, vcc, 0, %1, vcc" : "+v"(lo), "+v"(hi) : "v"(m) : "vcc");
 }
 
 // Whether a row with this maximum has a distribution to draw from.  Not where it is not a finite number, and not where it
@@ -1118,6 +1125,66 @@ __global__ __launch_bounds__(kSampleThreads) void sample_mass_kernel(SplitParams
   }
 }
 
+// The exact cut of a filter, in LDS: the key with at most `target` of weight above it and more with itself.  `hist` has 512
+// cleared words before and after; every thread of the workgroup calls, and every one sees *cut afterwards.
+struct CutShared { uint64_t* hist; uint64_t* res; uint32_t* cut; };
+
+// By four 8-bit digits.  each(count) calls count(key, in, weight) for everything that lies below what `before` counts.
+template <typename Each>
+static __device__ void digit_cut(const CutShared& cs, uint64_t before, uint64_t target, int tid, Each each) {
+  const int lane = tid & 63, wave = tid >> 6;
+  uint32_t pmask = 0, pval = 0;
+  for (int d = 3; d >= 0; --d) {
+    each([&](uint32_t k, bool in, auto weight) {
+      hist_add(cs.hist, 255 - (int)((k >> (8 * d)) & 255u), in && (k & pmask) == pval, lane, weight);
+    });
+    __syncthreads();
+    if (wave == 0) {  // (the wavefront that reads the bins also clears them for the next digit)
+      find_crossing<4>(cs.hist, before, target, cs.res, lane);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) cs.hist[4 * lane + j] = 0;
+    }
+    __syncthreads();
+    before = cs.res[1];
+    pmask |= 0xffu << (8 * d);
+    pval |= (255u - (uint32_t)cs.res[0]) << (8 * d);
+  }
+  if (tid == 0) *cs.cut = pval;
+  __syncthreads();
+}
+template <typename Count>
+static __device__ __forceinline__ void count_list(const uint32_t* key, const uint32_t* mass, int n, bool by_count, int tid, Count count) {
+  for (int j0 = 0; j0 < n; j0 += kSampleThreads) {
+    const int j = j0 + tid;
+    count(j < n ? key[j] : 0, j < n, [&]() -> uint64_t { return by_count ? 1u : mass[j]; });
+  }
+}
+// Of up to 256 listed elements, every one against every other: 64 elements a wavefront, the wavefronts of the same elements
+// a share of the others each (one wavefront takes 15 ns per other element).
+static __device__ __forceinline__ void pair_cut(const CutShared& cs, const uint32_t* key, const uint32_t* mass, int n, bool by_count,
+                                                uint64_t above, uint64_t target, int tid) {
+  const int lane = tid & 63, wave = tid >> 6;
+  const int blocks = n <= 64 ? 1 : n <= 128 ? 2 : 4, shares = kSampleWaves / blocks;
+  const int at = 64 * (wave % blocks) + lane, share = wave / blocks;
+  const int j1 = (int)((int64_t)n * (share + 1) / shares);
+  const uint32_t mine = at < n ? key[at] : 0;
+  uint64_t over = 0, equal = 0;
+  for (int j = n * share / shares; j < j1; ++j) {   // the same words for every lane: broadcast reads
+    const uint32_t k = key[j], w = by_count ? 1u : mass[j];
+    over += k > mine ? w : 0;
+    equal += k == mine ? w : 0;
+  }
+  if (at < n) {
+    atomicAdd(reinterpret_cast<unsigned long long*>(&cs.hist[at]), (unsigned long long)over);
+    atomicAdd(reinterpret_cast<unsigned long long*>(&cs.hist[256 + at]), (unsigned long long)equal);
+  }
+  __syncthreads();
+  if (tid < n && above + cs.hist[tid] <= target && above + cs.hist[tid] + cs.hist[256 + tid] > target) *cs.cut = key[tid];
+  __syncthreads();
+  if (tid < 256) cs.hist[tid] = 0;   // (for the digits, should the list turn out not to hold the cut)
+  __syncthreads();
+}
+
 template <int DT, int VEC>
 __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SplitParams p) {
   const int r = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1193,64 +1260,22 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SplitParams
     listed = listed && (!by_count || n >= p.s.top_k);
     __syncthreads();
   }
-  // ---- the smallest kept key: the one with at most `target` of weight above it and more with itself ----
+  // ---- the smallest kept key ----
+  const CutShared cs{hist, res, &cut};
   auto digits = [&](bool from_list) {
-    uint32_t pmask = 0, pval = 0;
-    uint64_t before = from_list ? above : 0;
-    for (int d = 3; d >= 0; --d) {
-      auto count = [&](uint32_t k, bool in, auto weight) {
-        hist_add(hist, 255 - (int)((k >> (8 * d)) & 255u), in && (k & pmask) == pval, lane, weight);
-      };
+    digit_cut(cs, from_list ? above : 0, target, tid, [&](auto count) {
       if (from_list) {
-        for (int j0 = 0; j0 < n; j0 += kSampleThreads) {
-          const int j = j0 + tid;
-          count(j < n ? key[j] : 0, j < n, [&]() -> uint64_t { return by_count ? 1u : mass[j]; });
-        }
+        count_list(key, mass, n, by_count, tid, count);
       } else {
         sweep<4>(rd, 0, p.s.V, tid, kSampleThreads, [&](int, float x, bool in) {
           count(order_key(x), in, [&]() -> uint64_t { return by_count ? 1 : mass_of(x, neg_mx); });
         });
       }
-      __syncthreads();
-      if (wave == 0) {  // (the wavefront that reads the bins also clears them for the next digit)
-        find_crossing<4>(hist, before, target, res, lane);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) hist[4 * lane + j] = 0;
-      }
-      __syncthreads();
-      before = res[1];
-      pmask |= 0xffu << (8 * d);
-      pval |= (255u - (uint32_t)res[0]) << (8 * d);
-    }
-    if (tid == 0) cut = pval;
-    __syncthreads();
+    });
   };
   if (cuts && listed) {
-    if (n <= 256) {
-      // every element against every other: 64 elements a wavefront, the wavefronts of the same elements a share of the
-      // others each (one wavefront takes 15 ns per other element)
-      const int blocks = n <= 64 ? 1 : n <= 128 ? 2 : 4, shares = kSampleWaves / blocks;
-      const int at = 64 * (wave % blocks) + lane, share = wave / blocks;
-      const int j1 = (int)((int64_t)n * (share + 1) / shares);
-      const uint32_t mine = at < n ? key[at] : 0;
-      uint64_t over = 0, equal = 0;
-      for (int j = n * share / shares; j < j1; ++j) {   // the same words for every lane: broadcast reads
-        const uint32_t k = key[j], w = by_count ? 1u : mass[j];
-        over += k > mine ? w : 0;
-        equal += k == mine ? w : 0;
-      }
-      if (at < n) {
-        atomicAdd(reinterpret_cast<unsigned long long*>(&hist[at]), (unsigned long long)over);
-        atomicAdd(reinterpret_cast<unsigned long long*>(&hist[256 + at]), (unsigned long long)equal);
-      }
-      __syncthreads();
-      if (tid < n && above + hist[tid] <= target && above + hist[tid] + hist[256 + tid] > target) cut = key[tid];
-      __syncthreads();
-      if (tid < 256) hist[tid] = 0;   // (for the digits, should the threshold turn out too high)
-      __syncthreads();
-    } else {
-      digits(true);
-    }
+    if (n <= 256) pair_cut(cs, key, mass, n, by_count, above, target, tid);
+    else digits(true);
     if (by_count && cut < tau) listed = false;   // (every thread sees the same words)
   }
   if (cuts && !listed) {
@@ -1322,6 +1347,414 @@ __global__ __launch_bounds__(kSampleThreads) void sample_pick_kernel(SplitParams
     int sample = pick;
     if (p.s.vocab_clamp > 0) sample = min(max(sample, 0), p.s.vocab_clamp - 1);
     write_sample(p.s, r, sample, cut_key);
+  }
+}
+
+// ---- a row in the registers of one workgroup ---------------------------------------------------------------------
+// elements of a wavefront's run, of `n`
+template <int VEC>
+static __host__ __device__ __forceinline__ int row_run(int n) { return ((n + kSampleWaves - 1) / kSampleWaves + VEC - 1) & ~(VEC - 1); }
+
+// NG groups of VEC elements a lane; a wavefront holds a run of neighbouring elements, group after group.  Rows start on any
+// element (a 16-byte load that is not aligned costs a cache line more now and then); the row's last group, where it is not
+// whole, is read as the last VEC elements, of which the lane before holds the first ones.  V >= VEC.
+template <int DT, int NG>
+struct RowInRegisters {
+  static constexpr int VEC = DT != 0 ? 8 : 4;
+  uint32_t w[NG][4];   // scaled values, two to a word in a 16-bit type; -inf where the lane has no element
+  int at0, last_at;    // the lane's first element; the last group's
+  int groups;          // of the wavefront's run: what lies past them is -inf (wave-uniform)
+
+  __device__ __forceinline__ float value(int g, int j) const {
+    if (DT != 0) return (j & 1) ? hi_to_f32<DT == 2>(w[g][j >> 1]) : lo_to_f32<DT == 2>(w[g][j >> 1]);
+    return __uint_as_float(w[g][j & 3]);
+  }
+  __device__ __forceinline__ int element(int g, int j) const { return min(at0 + g * 64 * VEC, last_at) + j; }
+  // Nothing made of the values lives on from here: conversions of one pass kept for the next spill what they save.
+  __device__ __forceinline__ void forget() {
+#pragma unroll
+    for (int g = 0; g < NG; ++g)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(w[g][i]));
+    asm volatile("" : "+v"(at0));
+  }
+
+  __device__ __forceinline__ void load(const SampleParams& p, int r, int wave, int lane) {
+    typedef std::conditional_t<DT != 0, uint16_t, uint32_t> element_t;
+    constexpr uint32_t kNone = DT == 0 ? 0xff800000u : DT == 1 ? 0xff80ff80u : 0xfc00fc00u;
+    const element_t* row = reinterpret_cast<const element_t*>(p.logits) + (int64_t)r * p.stride;
+    const int run = row_run<VEC>(p.V);   // (at most NG * 64 * VEC)
+    const int end = min((wave + 1) * run, p.V);
+    at0 = wave * run + lane * VEC;
+    last_at = p.V - VEC;
+    groups = __builtin_amdgcn_readfirstlane(max(end - wave * run + 64 * VEC - 1, 0) / (64 * VEC));
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      const uint32_t at = (uint32_t)min(at0 + g * 64 * VEC, last_at);
+      __builtin_memcpy(w[g], row + at, 16);   // (one load, of the element's alignment)
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    asm volatile("" : "+v"(at0));
+    if (p.inv_temperature != 1.0f) {     // (rounded to the logits' type, as RowReader::finish)
+#pragma unroll
+      for (int g = 0; g < NG; ++g)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if (DT == 0) w[g][i] = __float_as_uint(__uint_as_float(w[g][i]) * p.inv_temperature);
+          else w[g][i] = pack2<DT == 2>(lo_to_f32<DT == 2>(w[g][i]) * p.inv_temperature, hi_to_f32<DT == 2>(w[g][i]) * p.inv_temperature);
+          if (i == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+      forget();
+    }
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      const int at = at0 + g * 64 * VEC;
+      const int skip = at >= end ? VEC : at - last_at;   // of the lane's group: not its own
+      if (__builtin_amdgcn_ballot_w64(skip > 0)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if (DT == 0) w[g][i] = skip > i ? kNone : w[g][i];
+          else w[g][i] = skip > 2 * i + 1 ? kNone : skip > 2 * i ? (w[g][i] & 0xffff0000u) | (kNone & 0xffffu) : w[g][i];
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    forget();
+  }
+};
+
+// One workgroup per row, the row read once: maximum, bins around the cut (top-p: the first walk's of the parts; top-k: counts),
+// the members of the bins that hold the cut listed in LDS, the exact cut among them, the wavefront and then the element that the
+// uniform number falls into.  The masses and every sum that decides are those of the other forms; where the list does not
+// hold the cut, four digit passes over the registers find it.
+template <int DT, int NG>
+__global__ __launch_bounds__(kSampleThreads) void sample_row_kernel(SampleParams p) {
+  constexpr int VEC = RowInRegisters<DT, NG>::VEC;
+  __shared__ uint32_t bins[kBins + 64];
+  __shared__ uint32_t key[kMemberCap];
+  __shared__ uint32_t mass[kMemberCap];
+  __shared__ uint32_t index[kMemberCap];
+  __shared__ uint64_t hist[512];
+  __shared__ uint64_t res[2];
+  __shared__ uint64_t wsum[2][kSampleWaves];
+  __shared__ uint64_t runs[kSampleWaves], kept_runs[kSampleWaves];
+  __shared__ uint32_t red[kSampleWaves];
+  __shared__ int32_t window[2];
+  __shared__ uint32_t listed_n;
+  __shared__ uint32_t cut;
+  __shared__ int32_t pick;
+  const int r = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool by_count = p.top_k > 1, by_mass = p.top_k == 0 && p.top_p > 0.f, filtered = by_count || by_mass;
+  const float uniform = p.uniform[r];
+  RowInRegisters<DT, NG> row;
+  row.load(p, r, wave, lane);
+  bins[tid] = bins[tid + kSampleThreads] = 0;
+  if (tid < 512) hist[tid] = 0;
+  if (tid == 0) { window[0] = kBins; window[1] = -1; listed_n = 0; cut = 0; pick = 0; }
+
+  // ---- the maximum: as integers, numbers from +0 up are in order, NaN above them; below 0 the floats' order counts ----
+  int32_t top_i = INT32_MIN;
+  float top_f = -INFINITY;
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    if (g >= row.groups) continue;
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      const float x = row.value(g, j);
+      top_i = max(top_i, __float_as_int(x));
+      top_f = fmaxf(top_f, x);
+    }
+  }
+  uint32_t bk = wave_max_u32(top_i >= 0 ? (uint32_t)top_i | 0x80000000u : order_key(top_f + 0.f));
+  if (lane == 0) red[wave] = bk;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kSampleWaves; ++w) bk = max(bk, red[w]);
+  const float mx = order_key_value(bk), neg_mx = -mx * 1.4426950408889634f;
+  const RowReader<DT, 1> rd = row_reader<DT, 1>(p, r);   // (what is rare reads the row again)
+  if (!has_masses(mx)) {   // nothing to draw from: the argmax, the lowest index among equals
+    uint32_t best = 0, at = 0x7fffffffu;
+    sweep<8>(rd, 0, p.V, tid, kSampleThreads, [&](int i, float x, bool in) {
+      const uint32_t k = order_key(x);
+      const bool up = in && k > best;
+      best = up ? k : best;
+      at = up ? (uint32_t)i : at;
+    });
+    const uint32_t wave_best = wave_max_u32(best);
+    at = ~wave_max_u32(best == wave_best ? ~at : 0);
+    __syncthreads();   // (the maxima have been read)
+    if (lane == 0) { red[wave] = wave_best; key[wave] = at; }
+    __syncthreads();
+    if (tid == 0) {
+      best = 0;
+      for (int w = 0; w < kSampleWaves; ++w) {
+        if (red[w] > best || (red[w] == best && key[w] < at)) { best = red[w]; at = key[w]; }
+      }
+      write_sample(p, r, at < (uint32_t)p.V ? (int)at : 0, 0);
+    }
+    return;
+  }
+
+  row.forget();
+  // ---- the bins, counted down from the maximum's; the bins that hold the cut ----
+  float over = INFINITY, from = INFINITY;   // kept: above `over`; listed: from `from` to `over`
+  if (filtered) {
+    const float row_first = floorf(mx * kBinsPerUnit), edge = row_first + 1.f;
+    int bits = 31 - __builtin_clz(p.V);   // V < 2^(bits + 1)
+    const float bin_one = (float)(1u << (31 - bits > 16 ? 16 : 31 - bits));
+const uint32_t none = (uint32_t)(kBins + lane);   // (a place of its own for what no bin takes: no branch)
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      if (g >= row.groups) continue;
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) {
+        // (the weight of sample_first_kernel)
+        const float f = __builtin_fmaf(row.value(g, j), -kBinsPerUnit, edge);
+        const float wt = __builtin_fmaf(__builtin_amdgcn_fractf(f), -0.01550356f * bin_one, 0.99998474f * bin_one + 0.5f);
+        const bool in = f < (float)kBins;   // (not NaN, nor what is masked)
+        atomicAdd(&bins[in ? (uint32_t)fmaxf(in ? f : 0.f, 0.f) : none], by_count ? 1u : (uint32_t)(in ? wt : 0.f));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();
+    const uint32_t c0 = bins[2 * tid], c1 = bins[2 * tid + 1];
+    if (by_count) {
+      const int h = (int)(c0 + c1);
+      int incl = wave_scan(h);
+      if (lane == 63) red[wave] = (uint32_t)incl;
+      __syncthreads();
+#pragma unroll
+      for (int w = 0; w < kSampleWaves; ++w) incl += w < wave ? (int)red[w] : 0;
+      if (incl >= p.top_k && incl - h < p.top_k) window[0] = window[1] = incl - (int)c1 >= p.top_k ? 2 * tid : 2 * tid + 1;
+    } else {   // (the estimate and its slack: see sample_mass_kernel)
+      const float h0 = (float)c0 * fast_exp2((float)(2 * tid) * (-1.4426950408889634f / kBinsPerUnit));
+      const float h1 = (float)c1 * fast_exp2((float)(2 * tid + 1) * (-1.4426950408889634f / kBinsPerUnit));
+      const float h = h0 + h1;
+      float incl = wave_scan_incl_f32(h);
+      if (lane == 63) red[wave] = __float_as_uint(incl);
+      __syncthreads();
+      float total = 0.f;
+#pragma unroll
+      for (int w = 0; w < kSampleWaves; ++w) {
+        incl += w < wave ? __uint_as_float(red[w]) : 0.f;
+        total += __uint_as_float(red[w]);
+      }
+      const float want = p.top_p * total, slack = fmaxf(1e-4f, 3e-5f + 0.3f / bin_one) * total;
+      const bool in0 = incl - h - slack <= want && incl - h1 + slack > want && h0 > 0.f;
+      const bool in1 = incl - h1 - slack <= want && incl + slack > want && h1 > 0.f;
+      if (in0 || in1) {
+        atomicMin(&window[0], in0 ? 2 * tid : 2 * tid + 1);
+        atomicMax(&window[1], in1 ? 2 * tid + 1 : 2 * tid);
+      }
+    }
+    __syncthreads();
+    const int lo = window[0], hi = window[1];
+    if (lo <= hi) {
+      over = (row_first + 1.f - (float)lo) * (1.f / kBinsPerUnit);
+      from = (row_first - (float)hi) * (1.f / kBinsPerUnit);
+    }
+  }
+
+  // ---- the masses; what lies above the window; its members, listed ----
+  uint32_t all_lo = 0, all_hi = 0;   // top-p: of everything; a plain draw keeps all of it
+  uint32_t kept_lo = 0, kept_hi = 0, kept_n = 0;
+  row.forget();
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    if (g >= row.groups) continue;
+    uint32_t m32[VEC];
+    if (!by_count) {
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) m32[j] = add_mass(all_lo, all_hi, row.value(g, j), neg_mx);
+    }
+    if (!filtered) continue;
+    uint64_t in_window[VEC], any = 0;
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      const float v = row.value(g, j);
+      const bool is_over = v > over;
+      const uint64_t above = __builtin_amdgcn_ballot_w64(is_over);
+      if (above) {
+        if (by_count) kept_n += is_over ? 1u : 0u;
+        else add_u32(kept_lo, kept_hi, is_over ? m32[j] : 0u);
+      }
+      in_window[j] = __builtin_amdgcn_ballot_w64(v >= from) & ~above;
+      any |= in_window[j];
+    }
+    if (any) {
+      uint32_t found = 0, at = 0;
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) found += (uint32_t)__builtin_popcountll(in_window[j]);
+      if (lane == 0) at = atomicAdd(&listed_n, found);
+      at = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) {
+        const uint64_t m = in_window[j];
+        if (m == 0) continue;
+        const uint32_t mine = at + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+        if (((m >> lane) & 1) && mine < (uint32_t)kMemberCap) {
+          const float v = row.value(g, j);
+          key[mine] = order_key(v + 0.f);
+          index[mine] = (uint32_t)row.element(g, j);
+          mass[mine] = (uint32_t)mass_of(v, neg_mx);
+        }
+        at += (uint32_t)__builtin_popcountll(m);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  const uint64_t all = wave_sum_u64(((uint64_t)all_hi << 32) | all_lo);
+  uint64_t kept = by_mass ? wave_sum_u64(((uint64_t)kept_hi << 32) | kept_lo) : by_count ? wave_sum_u64(kept_n) : all;
+  if (lane == 0) { wsum[0][wave] = all; runs[wave] = kept; }
+  __syncthreads();
+  float cut_value = -INFINITY;
+  uint32_t cut_key = 0;
+  uint64_t run_mass = 0;   // lane i: kept members of run i that `of_runs` does not count
+  const uint64_t* of_runs = runs;
+  if (filtered) {
+    const uint64_t z = wave_sum_u64(lane < kSampleWaves ? wsum[0][lane & (kSampleWaves - 1)] : 0);
+    const uint64_t above = wave_sum_u64(lane < kSampleWaves ? runs[lane & (kSampleWaves - 1)] : 0);
+    const uint64_t target = by_count ? (uint64_t)(p.top_k - 1) : (uint64_t)((double)p.top_p * (double)z);
+    const bool cuts = by_count || z > target;   // (a top-p of the whole mass cuts nothing)
+    const int n = __builtin_amdgcn_readfirstlane((int)listed_n);
+    bool listed = n <= kMemberCap, joined = false;
+    if (cuts && n <= 16) {
+      // few members, one a lane: every wavefront works out the cut and the runs' kept masses by itself, without a barrier
+      const bool has = lane < n;
+      const uint32_t k = has ? key[lane] : 0, w = !has ? 0 : by_count ? 1u : mass[lane];
+      listed = above <= target && above + wave_sum_u64(w) > target;
+      if (listed) {
+        uint64_t higher = 0, equal = 0;
+        for (int j = 0; j < n; ++j) {
+          const uint32_t kj = (uint32_t)__builtin_amdgcn_readlane((int)k, j), wj = (uint32_t)__builtin_amdgcn_readlane((int)w, j);
+          higher += kj > k ? wj : 0u;
+          equal += kj == k ? wj : 0u;
+        }
+        const uint64_t hit = __builtin_amdgcn_ballot_w64(has && above + higher <= target && above + higher + equal > target);
+        cut_key = (uint32_t)__builtin_amdgcn_readlane((int)k, __builtin_ctzll(hit));   // (the list holds it)
+        if (by_mass) {
+          const int of_run = has && k >= cut_key ? (int)index[lane] / row_run<VEC>(p.V) : -1;
+          for (int j = 0; j < n; ++j)
+            run_mass += lane == __builtin_amdgcn_readlane(of_run, j) ? (uint32_t)__builtin_amdgcn_readlane((int)w, j) : 0u;
+          joined = true;
+        }
+      }
+    } else if (cuts) {
+      const CutShared cs{hist, res, &cut};
+      if (listed) {   // (does the list hold the cut?)
+        uint64_t in_list = (uint64_t)n;
+        if (by_mass) {
+          in_list = 0;
+          for (int j = tid; j < n; j += kSampleThreads) in_list += mass[j];
+          in_list = wave_sum_u64(in_list);
+          if (lane == 0) wsum[1][wave] = in_list;
+          __syncthreads();
+          in_list = 0;
+#pragma unroll
+          for (int w = 0; w < kSampleWaves; ++w) in_list += wsum[1][w];
+        }
+        listed = above <= target && above + in_list > target;
+      }
+      if (listed) {
+        if (n <= 256) pair_cut(cs, key, mass, n, by_count, above, target, tid);
+        else digit_cut(cs, above, target, tid, [&](auto count) { count_list(key, mass, n, by_count, tid, count); });
+        cut_key = cut;
+      }
+    }
+    if (cuts && !listed) {
+      digit_cut(CutShared{hist, res, &cut}, 0, target, tid, [&](auto count) {
+        sweep<8>(rd, 0, p.V, tid, kSampleThreads, [&](int, float x, bool in) {
+          count(order_key(x), in, [&]() -> uint64_t { return by_count ? 1 : mass_of(x, neg_mx); });
+        });
+      });
+      cut_key = cut;
+    }
+    if (cut_key) cut_value = order_key_value(cut_key);
+    // ---- the kept mass of every wavefront's run ----
+    if (!joined) {
+      if (by_mass && cuts && listed) {   // the kept members join what lies above the window
+        const int run = row_run<VEC>(p.V);
+        for (int j = tid; j < n; j += kSampleThreads)
+          if (key[j] >= cut_key)
+            atomicAdd(reinterpret_cast<unsigned long long*>(&runs[(int)index[j] / run]), (unsigned long long)mass[j]);
+      } else {
+        kept = 0;
+        row.forget();
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+          if (g >= row.groups) continue;
+#pragma unroll
+          for (int j = 0; j < VEC; ++j) {
+            const float v = row.value(g, j);
+            if (__builtin_amdgcn_ballot_w64(v >= cut_value)) {
+              const uint64_t x = mass_of(v, neg_mx);
+              kept += v >= cut_value ? x : 0;
+            }
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        kept = wave_sum_u64(kept);
+        if (lane == 0) kept_runs[wave] = kept;   // (`runs` may still be read)
+        of_runs = kept_runs;
+      }
+      __syncthreads();
+    }
+  }
+  // ---- the wavefront the uniform number falls into (lane i: run i); its group; the lane; the element ----
+  if (lane < kSampleWaves) run_mass += of_runs[lane];
+  const uint64_t runs_incl = wave_scan_incl_u64(run_mass, lane);
+  auto lane_u64 = [](uint64_t v, int at) {
+    return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), at) << 32) |
+           (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, at);
+  };
+  const uint64_t total = lane_u64(runs_incl, 63);
+  // total > 0: the maximum itself is always kept and has the largest mass
+  uint64_t want = (uint64_t)((double)uniform * (double)total);
+  want = want < total ? want : total - 1;
+  const int owner = __builtin_ctzll(__builtin_amdgcn_ballot_w64(runs_incl > want));
+  want -= lane_u64(runs_incl - run_mass, owner);
+  row.forget();
+  if (wave == owner) {
+    bool found = false;
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      if (found || g >= row.groups) continue;
+      if (filtered) {   // (most of a sharp filter's groups hold nothing)
+        uint64_t any = 0;
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) any |= __builtin_amdgcn_ballot_w64(row.value(g, j) >= cut_value);
+        if (!any) continue;
+      }
+      uint64_t m[VEC], sum = 0;
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) {
+        const float v = row.value(g, j);
+        const uint64_t x = mass_of(v, neg_mx);
+        m[j] = v >= cut_value ? x : 0;
+        sum += m[j];
+      }
+      const uint64_t incl = wave_scan_incl_u64(sum, lane), last = lane_u64(incl, 63);
+      if (last <= want) {
+        want -= last;
+        continue;
+      }
+      if (incl > want && incl - sum <= want) {
+        uint64_t at = incl - sum;
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) {
+          if (at <= want && at + m[j] > want) pick = row.element(g, j);
+          at += m[j];
+        }
+      }
+      found = true;
+    }
+  }
+  __syncthreads();
+  if (tid == 0) {
+    int sample = pick;
+    if (p.vocab_clamp > 0) sample = min(max(sample, 0), p.vocab_clamp - 1);
+    write_sample(p, r, sample, cut_key);
   }
 }
 
@@ -1472,17 +1905,21 @@ static int sample_parts(int R, int V) {
   if (parts > V / 4096) parts = V / 4096;
   return parts < 1 ? 1 : (parts > kMaxParts ? kMaxParts : parts);
 }
-// Whether the rows are done in parts.  The further launches cost 3-6 us, so the walks they shorten have to be long enough; from
-// 129 rows on a row has one part.  fp32 in a graph, us, one workgroup per row against parts:
+// Whether the rows are done in parts.  The further launches cost 3-6 us, so the walks they shorten have to be long enough.  fp32 in
+// a graph, us, one workgroup per row (that walks it) against parts:
 //   greedy, one walk to shorten: 64 x 151 936 16.9 / 12.0, 64 x 32 768 below the line 6.2 / 7.5;
 //   plain draws, two: 64 x 50 304 19.4 / 16.0, 64 x 32 768 below it 13.5 / 13.7;
 //   top-k, whose pick grows with its lists: 64 x 128 256 39.1 / 31.1, and does not gain from two: 128 x 100 352 35.2 / 37.7;
 //   top-p, three: 64 x 16 384 30.0 / 19.4, 64 x 128 256 101.8 / 28.1.
-// Between 65 and 128 rows the lines for draws (49 152 and 65 536 wide) are those of longer walks: today top-p gains below them
-// too (86 x 50 304 65.4 / 23.1, 128 x 16 384 37.9 / 18.3), a plain draw from 50 304 on (128 rows 20.6 / 18.2).  So does greedy
-// from 50 304 on with few rows (1 x 65 536 7.8 / 6.1).
+// Rows that fit the registers of a workgroup go there in many of these cases, workspace or not: row_groups.
+// More than 128 rows have one part each, and are done this way for the walks alone: a top-p row that does not fit the registers
+// of a workgroup.  fp32 / bf16: 256 x 128 256 119 / 115 -> 67 / 60, 512 x 151 936 255 / 253 -> 139 / 124; peaked rows 512 x
+// 128 256 130 / 122 -> 115 / 95.  (40 KB of scratch a row)
+constexpr int kManyRows = 1024;
+static bool many_rows_by_walks(int V, int top_k, float top_p) { return top_k == 0 && top_p > 0.f && V > 65536; }
 static bool sample_in_parts(int R, int V, int top_k, float top_p) {
-  if (V < kFastMinVocab || R > 128 || top_k > kFastTopK) return false;
+  if (R > 128) return R <= kManyRows && many_rows_by_walks(V, top_k, top_p);
+  if (V < kFastMinVocab || top_k > kFastTopK) return false;
   if (top_k == 1) return V >= 1600 * (R > 50 ? R : 50);
   if (top_k > 1) return R <= 85;
   if (R > 85) return V >= 65536;
@@ -1513,8 +1950,37 @@ static int64_t sample_layout(SplitParams* p, uint8_t* base, int R, int V, int to
   return at;
 }
 
+// Whether draws from rows of V elements take the registers of one workgroup, and how many groups of 16 bytes a lane: 0 = no.
+// Up to 65 536 elements fit without spilling.  A plain draw is faster than any other form throughout.  A filter's bins and
+// lists are work that parts share: above 32 768 elements parts, where the rows are few enough for them, are level or
+// better.  Without parts the one other form walks the row several times; only top-k over fp32, which it reads once, stays
+// there above 32 768.  In a graph, us, the other form -> this one, fp32 / bf16, N(0, 3):
+//   plain: 16 x 32 000 15.1 / 17.0 -> 7.4 / 9.1, 256 x 32 000 17.4 / 17.9 -> 9.6 / 9.8, 1 x 65 536 12.1 / 12.6 -> 10.7 / 11.0,
+//          256 x 65 536 30.7 / 23.5 -> 20.6 / 12.3;
+//   top-k 50: 16 x 32 000 16.8 / 17.0 -> 13.0 / 15.5, 128 x 32 000 24.0 / 24.3 -> 13.5 / 16.1; 16 x 65 536 17.3 / 17.7, here 21.8 /
+//          20.6; 512 x 50 303 45.4 / 43.7, here 54.7 / 41.6;
+//   top-p 0.9: 16 x 32 000 19.4 / 20.2 -> 16.0 / 18.8, 256 x 32 000 51.4 / 50.0 -> 17.9 / 19.7, 256 x 65 536 82 / 74 -> 33 / 26; 16 x
+//          65 536 22.6 / 23.5, here 24.0 / 25.5.
+template <int DT>
+static int row_groups(const SampleParams& s, bool in_parts) {
+  constexpr int VEC = DT != 0 ? 8 : 4;
+  if (s.top_k == 1 || s.V < VEC || s.V > 65536) return 0;
+  const bool filtered = s.top_k > 1 || s.top_p > 0.f;
+  if (filtered && s.V > 32768 && (in_parts || (s.top_k > 1 && DT == 0))) return 0;
+  return (row_run<VEC>(s.V) + 64 * VEC - 1) / (64 * VEC);
+}
+
 template <int DT, int VEC>
 static void launch_sample(const SampleParams& s, SplitParams* split, hipStream_t st) {
+  const int groups = row_groups<DT>(s, split != nullptr);
+  if (groups > 8) {   // (fp32 only)
+    hipLaunchKernelGGL((sample_row_kernel<DT, DT == 0 ? 16 : 8>), dim3(s.R), dim3(kSampleThreads), 0, st, s);
+    return;
+  }
+  if (groups > 0) {
+    hipLaunchKernelGGL((sample_row_kernel<DT, 8>), dim3(s.R), dim3(kSampleThreads), 0, st, s);
+    return;
+  }
   if (!split) {
     hipLaunchKernelGGL((sample_kernel<DT, VEC>), dim3(s.R), dim3(kSampleThreads), 0, st, s);
     return;
@@ -1579,7 +2045,9 @@ extern "C" int mi_sample_from_logits_ws(const void* logits, int64_t stride_row, 
   const int esize = logits_dtype != 0 ? 2 : 4;
   const bool wide = !(((uintptr_t)logits | (uintptr_t)(stride_row * esize)) & 15);  // 16-byte loads
   SplitParams split, *in_parts = nullptr;
-  if (workspace && sample_in_parts(R, vocab, top_k, top_p)) {
+  // (more than 128 rows do without a workspace that does not serve: for those none is asked for at every size)
+  const bool optional = R > 128 && (((uintptr_t)workspace & 255) || sample_layout(&split, nullptr, R, vocab, top_k, top_p) > workspace_bytes);
+  if (workspace && !optional && sample_in_parts(R, vocab, top_k, top_p)) {
     if ((uintptr_t)workspace & 255) return mi_fail(MI_ERR_ALIGN, "mi_sample_from_logits_ws: the workspace must be 256-byte aligned");
     if (sample_layout(&split, (uint8_t*)workspace, R, vocab, top_k, top_p) > workspace_bytes)
       return mi_fail(MI_ERR_WORKSPACE, "mi_sample_from_logits_ws: workspace smaller than mi_sample_workspace_bytes()");

@@ -546,3 +546,38 @@ def test_sampling_inside_use_workspace(mi, dev, buffer):
     with mi.ops.use_workspace(given):
         got, _ = mi.ops.sample_from_logits(logits, top_p=0.9, uniform=u)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("V", [4, 8, 9, 255, 4097, 16391, 32767, 32768, 32769, 65535, 65536])
+def test_rows_in_the_registers_of_a_workgroup(mi, dev, V, dtype):
+    """Rows that start on any element and end within a group of 16 bytes; wavefronts without elements (short rows), the widest
+    rows of either number of groups; lists of a few members, of many, and none that holds the cut (equal values, a top-k that
+    ends far below the bins)."""
+    R = 86 if V > 32768 else 7     # (the rows of a wide filter that are not done in parts)
+    x = _logits(R, V, V, torch.float32)
+    x[1, V // 2:] = -90.0
+    x[2] = x[2, 0]
+    if V > 200:
+        x[3, 100:180] = x[3].topk(40).values[-1]
+        x[4, ::3] = float("-inf")
+        x[5, V - 1] = 30.0
+    y = torch.zeros(R, V + 3, dtype=dtype, device=dev)[:, 1:V + 1]
+    y.copy_(x)
+    u = torch.rand(R, generator=torch.Generator().manual_seed(V))
+    u[5] = 0.999
+    ud = u.to(dev)
+    xs = osm.scaled_logits(y.cpu(), 0.8)
+    for mode in (dict(), dict(top_k=2), dict(top_k=min(50, V)), dict(top_k=V - 1), dict(top_p=0.5), dict(top_p=0.97)):
+        s, _, cut = mi.ops.sample_from_logits(y, temperature=0.8, uniform=ud, return_cut=True, **mode)
+        s, cut = s.cpu(), cut.cpu()
+        if "top_k" in mode:
+            assert torch.equal(cut, torch.topk(xs, mode["top_k"], dim=-1).values[:, -1]), mode
+        elif "top_p" in mode:
+            pr = osm.kept_probabilities(xs, torch.ones_like(xs, dtype=torch.bool))
+            above = torch.where(xs > cut[:, None], pr, 0).sum(-1)
+            upto = torch.where(xs >= cut[:, None], pr, 0).sum(-1)
+            assert (above <= mode["top_p"] + TOL).all() and (upto > mode["top_p"] - TOL).all(), mode
+        else:
+            assert torch.isinf(cut).all()
+        _check_draw(xs, cut, u, s)
