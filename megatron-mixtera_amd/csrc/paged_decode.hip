@@ -101,6 +101,13 @@ static __host__ __device__ __forceinline__ int fused_lds_per_wave(int head_dim, 
   return 3 * head_dim * 4 + (G < 16 ? G : 16) * (2 * head_dim + 16);
 }
 
+// decode_short_kernel: floats of a query head's partial in LDS (the values, the running maximum, the row sum)
+static __host__ __device__ __forceinline__ constexpr int short_pitch(int head_dim) { return head_dim + 4; }
+static __host__ __device__ __forceinline__ int short_lds_per_wave(int head_dim, int G, bool fused) {
+  const int part = (G < 16 ? G : 16) * short_pitch(head_dim) * 4, prologue = fused ? fused_lds_per_wave(head_dim, G) : 0;
+  return ((part > prologue ? part : prologue) + 15) & ~15;
+}
+
 // One segment: tokens [start, end) of request r for KV head h (one wavefront) and the `gq` <= 16 query heads
 // hq0 .. hq0 + gq - 1 that share it.  `whole` = the segment is the entire request (write the 16-bit output, no
 // partial).
@@ -115,7 +122,8 @@ static __host__ __device__ __forceinline__ int fused_lds_per_wave(int head_dim, 
 // the step's new token) first normalises and rotates the new key row of its KV head, writes it and the value
 // row into their cache slot, and takes both from LDS for its last tile.  `q_lds` is then this wavefront's
 // piece of LDS for cos / sin of the request's position [2][HDK], the key row [HDK] (fp32) and the query rows.
-template <int HDK, int HDV, int NT, bool FP8, bool F16, bool FUSED = false>
+// SHORT: the partial stays in `q_lds` (see decode_short_kernel).
+template <int HDK, int HDV, int NT, bool FP8, bool F16, bool FUSED = false, bool SHORT = false>
 static __device__ __forceinline__ void decode_segment(const DecodeParams& p, int r, int row, int h, int hq0, int gq,
                                                       int len, int start, int end, bool whole, bool final_seg,
                                                       int slot, int lane, uint8_t* q_lds) {
@@ -740,7 +748,15 @@ static __device__ __forceinline__ void decode_segment(const DecodeParams& p, int
   const float inv = 1.f / l_tot;
   if (m16 >= G) return;  // (no barrier follows inside a segment)
   // acc[e][i] holds d = DV*(4g+i) + e: DV*4 contiguous values per lane.
-  if (whole) {
+  if constexpr (SHORT) {
+    float* o = reinterpret_cast<float*>(q_lds) + m16 * short_pitch(HDV) + 4 * DV * g;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int e = 0; e < DV; e += 2)
+        *reinterpret_cast<float2*>(o + DV * i + e) = make_float2(acc[e][i], acc[e + 1][i]);
+    if (g == 0) *reinterpret_cast<float2*>(reinterpret_cast<float*>(q_lds) + m16 * short_pitch(HDV) + HDV) = make_float2(m_run, l_tot);
+  } else if (whole) {
     uint16_t* o = p.out + (int64_t)row * p.o_st + (int64_t)hq * p.o_sh + 4 * DV * g;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -968,6 +984,63 @@ __global__ __launch_bounds__(512, MINW) void paged_decode_stream_kernel(DecodePa
 template <int HD, int NT, bool F16, int MINW = 3, bool FP8 = false>
 __global__ __launch_bounds__(512, MINW) void decode_step_stream_kernel(DecodeParams p) {
   decode_stream_body<HD, HD, NT, FP8, F16, true>(p);
+}
+
+// A few short requests: one workgroup per request and (virtual) KV head, its wavefronts a share of the tokens each, their
+// partials merged in LDS.  The stream above cuts such requests over the chip and needs a second launch to merge them, half as
+// long as the first.
+constexpr int kShortWaves = 8;
+template <int HD, int NT, bool FP8, bool F16, bool FUSED>
+__global__ __launch_bounds__(64 * kShortWaves, 2) void decode_short_kernel(DecodeParams p) {
+  extern __shared__ int cum[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int HV = p.Hkv * p.parts, busy = p.R * HV;
+  if ((int)blockIdx.x >= busy) {
+    if constexpr (FUSED && !FP8) fetch_next_matrix(busy);
+    return;
+  }
+  const int r = blockIdx.x / HV, hv = blockIdx.x - r * HV;
+  const int h = p.parts > 1 ? hv / p.parts : hv, part = hv - h * p.parts;
+  const int hq0 = h * p.G + 16 * part, gq = min(16, p.G - 16 * part);
+  int row;
+  if (!decode_row(p, r, row)) return;
+  constexpr int TK = 16 * NT, PITCH = short_pitch(HD);
+  const int len = __builtin_amdgcn_readfirstlane(p.lens[r]);
+  const int tiles = tiles_of(len, TK);
+  uint8_t* const lds = reinterpret_cast<uint8_t*>(cum);
+  const int per_wave = short_lds_per_wave(HD, p.G, FUSED);
+  // (whole tiles, evenly: a wavefront's tiles follow one another)
+  const int tb = tiles * wave / kShortWaves, te = tiles * (wave + 1) / kShortWaves;
+  if (te > tb) {
+    decode_segment<HD, HD, NT, FP8, F16, FUSED, true>(p, r, row, h, hq0, gq, len, tb * TK, min(te * TK, len), false, te == tiles,
+                                                      0, lane, lds + wave * per_wave);
+  } else if (lane < gq) {
+    *reinterpret_cast<float2*>(lds + wave * per_wave + 4 * (lane * PITCH + HD)) = make_float2(-INFINITY, 0.f);
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < gq * (HD / 4); i += 64 * kShortWaves) {
+    const int m = i / (HD / 4), d = 4 * (i % (HD / 4));
+    float2 ml[kShortWaves];
+    float mx = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < kShortWaves; ++w) {
+      ml[w] = *reinterpret_cast<const float2*>(lds + w * per_wave + 4 * (m * PITCH + HD));
+      mx = fmaxf(mx, ml[w].x);
+    }
+    float4 num = make_float4(0.f, 0.f, 0.f, 0.f);
+    float den = 0.f;
+#pragma unroll
+    for (int w = 0; w < kShortWaves; ++w) {
+      if (ml[w].y == 0.f) continue;   // (no tiles: its values were never written)
+      const float4 v = *reinterpret_cast<const float4*>(lds + w * per_wave + 4 * (m * PITCH + d));
+      const float a = fast_exp2(ml[w].x - mx);
+      num.x += a * v.x; num.y += a * v.y; num.z += a * v.z; num.w += a * v.w;
+      den += a * ml[w].y;
+    }
+    const float inv = den > 0.f ? 1.f / den : 0.f;   // (a request without tokens: zeros)
+    st8(p.out + (int64_t)row * p.o_st + (int64_t)(hq0 + m) * p.o_sh + d,
+        make_uint2(pack2<F16>(num.x * inv, num.y * inv), pack2<F16>(num.z * inv, num.w * inv)));
+  }
 }
 
 // Multi-latent attention, absorbed form: every query head attends to the same 576-wide latent rows
@@ -1829,6 +1902,26 @@ int mi::check_decode_workspace(const void* workspace, int64_t workspace_bytes, i
   return MI_OK;
 }
 
+// Whether a batch goes to decode_short_kernel: `workgroups` of it, requests of at most `most` tokens as far as the table's width
+// tells.  A CU alone takes in some 30 KB/us of a cache in HBM (64-byte pieces of keys, whole rows of values), the second launch
+// and the trip of the partials cost 4-7 us, and with more workgroups than CUs the stream's equal spans balance better.  Us per
+// call in a graph, twelve caches in turn, stream + merge -> short, lengths from a quarter of the bound up, 128 wide, 16-bit:
+//   bound 64 tokens: 1 x 32/8 heads 8.3 -> 4.1, 16 x 32/8 11.8 -> 5.1, 64 x 32/8 12.3 -> 8.3; 256 tokens: 2 x 32/8 12.4 -> 7.3, 16 x
+//   32/8 13.2 -> 8.4, 64 x 32/8 21.3 -> 14.8, 128 x 32/8 28.1 -> 26.9 (the whole step 30.0 -> 36.6: not there);
+//   512 tokens: 16 x 32/8 15.3 -> 13.8, 32 x 32/8 21.4 -> 14.4, 128 x 16/2 21.9 -> 14.1, but 8 x 16/2 9.1 -> 10.9;
+//   1 024 tokens: 32 x 32/8 27.0 -> 24.1, 128 x 16/2 29.2 -> 22.0, but 8 x 32/8 15.2 -> 19.9, 16 x 32/8 step 21.9 -> 23.3.
+// The whole step of a layer, likewise: 16 x 32/8, bound 512: 19.1 -> 15.1.
+constexpr int kShortTile = 2;   // (sub-tiles per iteration; four are 3-8 % slower)
+static bool decode_is_short(int workgroups, int head_dim, int64_t most, int esz, int chunk_tokens, const MiTuning& tune,
+                            int split_tokens) {
+  if ((head_dim != 64 && head_dim != 128) || chunk_tokens % (16 * kShortTile)) return false;
+  if (tune.decode_grid > 0 || tune.decode_tile_subtiles > 0 || split_tokens > 0) return false;   // (the stream's own knobs)
+  const int64_t bytes = most * head_dim * 2 * esz;   // of the longest request's keys and values for one head
+  if (bytes <= 128 << 10) return workgroups <= 512;
+  if (bytes <= 256 << 10) return workgroups >= 64 && workgroups <= 256;
+  return bytes <= 512 << 10 && workgroups >= 192 && workgroups <= 256;
+}
+
 int mi::launch_paged_decode(
     const void* q, int64_t q_stride_tok, int64_t q_stride_head, const void* k_cache,
     const void* v_cache, int64_t kv_stride_chunk, int64_t kv_stride_tok, int64_t kv_stride_head,
@@ -1955,6 +2048,25 @@ int mi::launch_paged_decode(
   hipEvent_t ev_a, ev_b;
   const bool timed = mi_profile_next(&ev_a, &ev_b);
   if (timed) (void)hipEventRecord(ev_a, st);
+  if (decode_is_short(R * waves, head_dim, bt_stride * chunk_tokens, esz, chunk_tokens, tune, split_tokens)) {
+    const dim3 sgrid(p.next_w && fused ? (R * waves > grid_x ? R * waves : grid_x) : R * waves), sblock(64 * kShortWaves);
+    const size_t slds = (size_t)kShortWaves * short_lds_per_wave(head_dim, G, fused != nullptr);
+#define MI_LAUNCH_SHORT(HD_, NT_, FP8_, FUSED_)                                                                         \
+    do {                                                                                                                \
+      if (f16) hipLaunchKernelGGL((decode_short_kernel<HD_, NT_, FP8_, true, FUSED_>), sgrid, sblock, slds, st, p);     \
+      else hipLaunchKernelGGL((decode_short_kernel<HD_, NT_, FP8_, false, FUSED_>), sgrid, sblock, slds, st, p);        \
+    } while (0)
+    if (fused && kv_dtype == MI_KV_FP8_E4M3) MI_LAUNCH_SHORT(128, kShortTile, true, true);
+    else if (fused && head_dim == 128) MI_LAUNCH_SHORT(128, kShortTile, false, true);
+    else if (fused) MI_LAUNCH_SHORT(64, kShortTile, false, true);
+    else if (kv_dtype == MI_KV_FP8_E4M3 && head_dim == 128) MI_LAUNCH_SHORT(128, kShortTile, true, false);
+    else if (kv_dtype == MI_KV_FP8_E4M3) MI_LAUNCH_SHORT(64, kShortTile, true, false);
+    else if (head_dim == 128) MI_LAUNCH_SHORT(128, kShortTile, false, false);
+    else MI_LAUNCH_SHORT(64, kShortTile, false, false);
+#undef MI_LAUNCH_SHORT
+    if (timed) (void)hipEventRecord(ev_b, st);
+    return mi_check_launch("mi_paged_decode_attention");
+  }
 #define MI_LAUNCH_DECODE(HD_, FP8_, F16_)                                                                              \
   do {                                                                                                                 \
     if (nt == 4) hipLaunchKernelGGL((paged_decode_stream_kernel<HD_, 4, FP8_, 2, F16_>), grid, block, lds, st, p);          \

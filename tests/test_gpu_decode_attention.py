@@ -279,3 +279,29 @@ def test_rejects_bad_arguments(mi, dev):
     kc80 = torch.randn(4, 64, 2, 80, device=dev).bfloat16()
     with pytest.raises(mi._lib.KernelError):
         mi.ops.paged_decode_attention(q80, kc80, kc80, case.kv_lens, case.block_table)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("Hq,Hkv,d,chunk", [(8, 8, 64, 32), (32, 8, 128, 64), (16, 1, 128, 256), (20, 1, 64, 256), (24, 8, 128, 128)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_short_requests_by_one_workgroup_per_head(mi, dev, Hq, Hkv, d, chunk, fp8, dtype):
+    """Tables of up to 256 tokens at width 128: one workgroup per request and KV head, against the checker and (16-bit caches)
+    against the stream, which `split_tokens` asks for.  Lengths around the tiles of 32 tokens and the eight wavefronts' shares."""
+    lens = torch.tensor([0, 1, 2, 31, 32, 33, 63, 64, 65, 223, 224, 225, 255, 256], dtype=torch.int32)
+    cfg = mi.synthetic.DecodeConfig("short", lens.numel(), Hq, Hkv, d, 0, 0, chunk=chunk, seed=Hq + d)
+    case = mi.synthetic.make_decode_case(cfg, dev, lens=lens, dtype=dtype)
+    assert case.block_table.stride(0) * chunk <= 256
+    caches, kw, ref_kw = (case.k_cache, case.v_cache), {}, {}
+    if fp8:
+        caches = tuple(torch.empty(case.k_cache.shape, dtype=torch.uint8, device=dev) for _ in range(2))
+        scales = [torch.empty(case.k_cache.size(0), Hkv, dtype=torch.float32, device=dev) for _ in range(2)]
+        for src, pool, scale in zip((case.k_cache, case.v_cache), caches, scales):
+            mi.ops.quantize_chunks_fp8(src, pool, scale)
+        kw = dict(k_scales=scales[0], v_scales=scales[1])
+        ref_kw = {k: v.cpu() for k, v in kw.items()}
+    out = mi.ops.paged_decode_attention(case.q, *caches, case.kv_lens, case.block_table, **kw)
+    ref = oa.paged_decode_attention(case.q.cpu().squeeze(1), caches[0].cpu(), caches[1].cpu(), lens, case.block_table.cpu(), **ref_kw)
+    _close(out.squeeze(1), ref, 2e-2)
+    assert (out[0] == 0).all()
+    stream = mi.ops.paged_decode_attention(case.q, *caches, case.kv_lens, case.block_table, split_tokens=64, **kw)
+    _close(out.squeeze(1), stream.float().cpu().squeeze(1), 8e-3)
