@@ -13,7 +13,7 @@
 // matrix / vector phases and no per-phase barriers: every wavefront runs the whole tile pipeline in ONE stream, cut
 // into 32-key steps and software-pipelined so that three independent chains are always open --
 //     products    S^T(step s+1) = K Q^T          and  O^T += V^T P^T(step s-1)     (matrix cores)
-//     vector ALU  P(step s) = exp2(S(step s) * scale - reference)  and the running maximum of S(step s+1)
+//     vector ALU  P(step s) = exp2(S(step s) * scale - reference)  and the mask of S(step s+1)
 //     LDS         the fragments of the products three fragments ahead
 // -- and the source orders them product pair / fragment read / a few vector instructions, pinned by scheduling
 // barriers.  Whatever one wavefront of a SIMD cannot issue (a product waiting for the matrix core, a wait for LDS),
@@ -33,10 +33,13 @@
 // softmax scale of the tile instead; values are multiplied by theirs and rounded.  (6 prompts of 454-3 766 tokens, head_dim
 // 128: 508 against 516 us with everything; head_dim 64: 329 against 360.)
 //
-// Softmax: exponentials are taken against a per-row reference that moves only when a score exceeds it by a window
-// (2^30 as the largest probability with bf16 operands, 2^8 with fp16); the row sums come out of the matrix cores
-// (an all-ones A fragment).  A move of the reference rescales the accumulators, the sums and the one step of
-// probabilities that is still waiting for its product.
+// Softmax: exponentials are taken against a per-row reference that moves only when a probability leaves a window (a
+// factor of 2^31 with bf16 operands, 2^8 with fp16); the row sums come out of the matrix cores (an all-ones A fragment).
+// No maximum is taken beside the products: the step's finished probabilities are looked at two to a word (5 instructions for
+// 16 scores a lane, where the maximum of the scores took 10), and where one has left the window the scores, still in
+// registers, give the new reference, the accumulators and sums are rescaled and the step's probabilities made again.  (Steps,
+// the maximum of every score -> this: 11 ragged prompts of width 64 147.0 -> 144.4 us, 6 prompts over an fp8 cache 456 -> 446, 8 x 2 048
+// new tokens beside decoding requests 1 307 -> 1 280, 509 new tokens over 61 234 877 -> 854.)
 #include <type_traits>
 
 #include "mi_common.h"
@@ -54,6 +57,11 @@ template <int HD> constexpr int wv_pitch() { return 2 * HD + 32; }
 // (half as many at head_dim 128 with few workgroups, one wavefront per SIMD: 5-8 % faster up to one workgroup per CU,
 // slower beyond; two at head_dim 64: slower throughout)
 template <int HD> constexpr int wv_waves() { return HD == 64 ? 4 : 8; }
+// A row's reference is moved where a probability leaves the window, to where the row's largest one is 2^-headroom: with bf16
+// operands, whose exponents reach far below, 2^-30 under the 2 that the check looks for (one bit of a word); with fp16 1
+// under 2^8.
+template <bool F16> constexpr float kWvHeadroom = F16 ? 0.f : 30.f;
+constexpr float kNoReference = 3e38f;   // any score leaves the window; a masked one (-inf) stays a probability of zero
 // piece u of a tile's line -> its row, by multiplication
 template <int HD> constexpr unsigned wv_magic() { return 65536u / (wv_pitch<HD>() / 16) + 1; }
 template <int HD> constexpr bool wv_piece_division_ok() {
@@ -215,13 +223,11 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
     }
   };
 
-  float m_run[NQ], neg_run[NQ], mwin[NQ];
+  float neg_run[NQ];  // the reference: a probability is 2^(score * scale + neg_run); kNoReference until a row has one
   f32x4_t acc[NQ][DV], accl[NQ];
 #pragma unroll
   for (int nt = 0; nt < NQ; ++nt) {
-    m_run[nt] = -INFINITY;
-    mwin[nt] = -INFINITY;
-    neg_run[nt] = 0.f;
+    neg_run[nt] = kNoReference;
     accl[nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int e = 0; e < DV; ++e) acc[nt][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -348,12 +354,9 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
     };
     auto uniform_float = [](float x) { return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, x))); };
 
-    // 16-bit: scores and references in raw units, one scale for all.  fp8: references in scaled units, since the scale
-    // belongs to a tile (kept off zero: zero times the -inf of a masked score would be NaN).
+    // 16-bit: one scale for all scores.  fp8: a tile's own (kept off zero: zero times the -inf of a masked score would be NaN).
     auto tile_scale = [&](float ks) { return FP8 ? fmaxf(ks * p.scale_log2, 1.17549435e-38f) : p.scale_log2; };
     float scale_prev = p.scale_log2, scale_cur = p.scale_log2, scale_next = p.scale_log2, vscale = 1.f;
-    const float ref_scale = FP8 ? 1.f : p.scale_log2;   // reference units -> log2 units
-    const float win = (F16 ? 8.f : 30.f) / ref_scale;
     const uint4 ones = make_uint4(ones2<F16>(), ones2<F16>(), ones2<F16>(), ones2<F16>());
     const f32x4_t zero4 = {0.f, 0.f, 0.f, 0.f};
     // per-lane starts of the fragment reads inside a tile buffer
@@ -388,27 +391,44 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
       const int d = 2 * u + (c & 1);
       if (d == 0) Px[nt].x = w; else if (d == 1) Px[nt].y = w; else if (d == 2) Px[nt].z = w; else Px[nt].w = w;
     };
-    // the reference of some row has to move (rare): new reference, rescale of everything taken against the old one
-    auto move_reference = [&](float (&tmax)[NQ], uint4 (&Ppend)[NQ]) {
+    // whether one of a step's probabilities has left the window
+    auto leaves_window = [&](const uint4 (&Px)[NQ]) -> bool {
+      if constexpr (F16) {   // 2^8 or more (or NaN): in both halves at once
+        uint32_t t;
+        asm("v_pk_maximum3_f16 %0, %1, %2, %3" : "=v"(t) : "v"(Px[0].x), "v"(Px[0].y), "v"(Px[0].z));
+        asm("v_pk_maximum3_f16 %0, %0, %1, %2" : "+v"(t) : "v"(Px[0].w), "v"(Px[1].x));
+        asm("v_pk_maximum3_f16 %0, %0, %1, %2" : "+v"(t) : "v"(Px[1].y), "v"(Px[1].z));
+        asm("v_pk_maximum3_f16 %0, %0, %1, %1" : "+v"(t) : "v"(Px[1].w));
+        asm("v_pk_add_u16 %0, %0, %1" : "+v"(t) : "v"(0x24002400u));   // (0x5c00, 256.0, becomes the sign)
+        return (t & 0x80008000u) != 0;
+      } else {               // 2 or more: the exponent's highest bit
+        const uint32_t t = ((Px[0].x | Px[0].y | Px[0].z) | (Px[0].w | Px[1].x | Px[1].y)) | (Px[1].z | Px[1].w);
+        return (t & 0x40004000u) != 0;
+      }
+    };
+    // The reference of some row has to move (rare): it goes to the row's largest score of the step, what was summed against the old
+    // one is rescaled, and the step's probabilities are made again.
+    auto move_reference = [&](const f32x4_t (&Sx)[NQ][2], uint4 (&Px)[NQ], float scale) {
 #pragma unroll
       for (int nt = 0; nt < NQ; ++nt) {
-        const float tm = rowgroup_max(tmax[nt]);  // (already in the reference's units)
-        const float m_raw = fmaxf(m_run[nt], tm);
-        const float m_use = m_raw == -INFINITY ? 0.f : m_raw;
-        const float alpha = fast_exp2((m_run[nt] - m_use) * ref_scale);
-        neg_run[nt] = -m_use * ref_scale;
-        m_run[nt] = m_raw;
-        mwin[nt] = m_raw + win;
+        float tm = -INFINITY;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) tm = fmaxf(tm, Sx[nt][u][i]);
+        const float neg = fminf(neg_run[nt], __builtin_fmaf(-rowgroup_max(tm), scale, -kWvHeadroom<F16>));
+        const float alpha = fast_exp2(neg - neg_run[nt]);
+        neg_run[nt] = neg;
         if (__builtin_amdgcn_ballot_w64(alpha != 1.f)) {
 #pragma unroll
           for (int e = 0; e < DV; ++e) {
             acc[nt][e][0] *= alpha; acc[nt][e][1] *= alpha; acc[nt][e][2] *= alpha; acc[nt][e][3] *= alpha;
           }
           accl[nt][0] *= alpha; accl[nt][1] *= alpha; accl[nt][2] *= alpha; accl[nt][3] *= alpha;
-          auto rs = [&](uint32_t w) { return pack2<F16>(lo_to_f32<F16>(w) * alpha, hi_to_f32<F16>(w) * alpha); };
-          Ppend[nt] = make_uint4(rs(Ppend[nt].x), rs(Ppend[nt].y), rs(Ppend[nt].z), rs(Ppend[nt].w));
         }
       }
+#pragma unroll
+      for (int c = 0; c < 8; ++c) exp_chunk(Sx, Px, c, scale);
     };
 
     // ---- one 32-key slot.  H: the half of the key tile whose scores are multiplied (into S[H]); the vector ALU turns
@@ -466,37 +486,17 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
         MI_SB();
       }
       if constexpr (H == 1) at_barrier();
-      float tmax[NQ];
-      int dpos[NQ];
-      // mask and maximum of the scores just multiplied: step i = rows i >> 1, part i & 1
-      auto max_step = [&](int i) {
-        const int nt = i >> 1, part = i & 1;
-        if (MASK && i == 0) {
-          const int tok0 = key0 + 4 * g;
-          dpos[0] = qpos[0] - tok0;
-          dpos[1] = qpos[1] - tok0;
-        }
-        if (MASK && part == 0) {
-          // (every masked score is out of the way before the first maximum is taken: a masked key's score in the
-          // reference would cost fp16 probabilities their precision)
+      // the mask of the scores just multiplied, rows nt
+      auto mask_step = [&](int nt) {
+        if (!MASK) return;
+        const int dpos = qpos[nt] - (key0 + 4 * g);
 #pragma unroll
-          for (int u = 0; u < 2; ++u)
+        for (int u = 0; u < 2; ++u)
 #pragma unroll
-            for (int i2 = 0; i2 < 4; ++i2)
-              if (16 * u + i2 > dpos[nt]) Sn[nt][u][i2] = -INFINITY;
-        }
-        // a chain of three-operand maxima
-        if (MASK ? part == 1 : part == 0) {
-          tmax[nt] = fmaxf(fmaxf(Sn[nt][0][0], Sn[nt][0][1]), Sn[nt][0][2]);
-          tmax[nt] = fmaxf(fmaxf(tmax[nt], Sn[nt][0][3]), Sn[nt][1][0]);
-        }
-        if (part == 1) {
-          tmax[nt] = fmaxf(fmaxf(tmax[nt], Sn[nt][1][1]), Sn[nt][1][2]);
-          tmax[nt] = fmaxf(tmax[nt], Sn[nt][1][3]);
-          if (FP8) tmax[nt] *= scale_cur;
-        }
+          for (int i2 = 0; i2 < 4; ++i2)
+            if (16 * u + i2 > dpos) Sn[nt][u][i2] = -INFINITY;
       };
-      // values; beside them the last probabilities, then mask and maximum of the scores just multiplied
+      // values; beside them the last probabilities, then the mask of the scores just multiplied
 #pragma unroll
       for (int e = 0; e < NVF; ++e) {
         const int n = NKF + e;
@@ -507,10 +507,10 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
         MI_SB();
         if (HD == 128) {
           if (e < 2) exp_stages(8 + e);
-          if (e >= 3 && e < 7) max_step(e - 3);
+          if (e == 3 || e == 5) mask_step((e - 3) / 2);
         } else {
           if (e == 0) { exp_stages(8); exp_stages(9); }
-          if (e == 1 || e == 2) { max_step(2 * e - 2); max_step(2 * e - 1); }
+          if (e == 1 || e == 2) mask_step(e - 1);
         }
         under_values(e);
         MI_SB();
@@ -518,7 +518,7 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
       accl[0] = mfma_16x16x32<F16>(ones, Pv[0], accl[0]);
       accl[1] = mfma_16x16x32<F16>(ones, Pv[1], accl[1]);
       MI_SB();
-      if (__builtin_amdgcn_ballot_w64(tmax[0] > mwin[0] || tmax[1] > mwin[1])) move_reference(tmax, Px);
+      if (__builtin_amdgcn_ballot_w64(leaves_window(Px))) move_reference(Sx, Px, scale);
       MI_SB();
     };
 
@@ -682,7 +682,7 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
     for (; j < jm;) iteration(std::false_type{});
     for (; j < ntl;) iteration(std::true_type{});
 
-    // ---- drain: the last two steps' values (tile ntl - 1 in Vs[ntl % VBUFS]); S[1] is masked and checked already ----
+    // ---- drain: the last two steps' values (tile ntl - 1 in Vs[ntl % VBUFS]); S[1] is masked already ----
     {
       const uint8_t* va = v_lane + vbi * BUF;
       auto values = [&](int half, const uint4 (&Pv)[NQ]) {
@@ -698,6 +698,7 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
       values(0, P[0]);
 #pragma unroll
       for (int c = 0; c < 8; ++c) exp_chunk(S[1], P[1], c, FP8 ? scale_prev : p.scale_log2);
+      if (__builtin_amdgcn_ballot_w64(leaves_window(P[1]))) move_reference(S[1], P[1], FP8 ? scale_prev : p.scale_log2);
       values(1, P[1]);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no direct load may still be on its way into this workgroup's LDS
@@ -725,7 +726,7 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
         for (int e = 0; e < DV; ++e)
           *reinterpret_cast<float4*>(o + 16 * e) =
               make_float4(acc[nt][e][0] * inv, acc[nt][e][1] * inv, acc[nt][e][2] * inv, acc[nt][e][3] * inv);
-        if (g == 0) p.split_lse[prow] = l_tot > 0.f ? m_run[nt] * (FP8 ? 1.f : p.scale_log2) + fast_log2(l_tot) : -INFINITY;
+        if (g == 0) p.split_lse[prow] = l_tot > 0.f ? fast_log2(l_tot) - neg_run[nt] : -INFINITY;
       }
     }
   }
