@@ -164,19 +164,21 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
 #pragma unroll
     for (int nt = 0; nt < NQ; ++nt) {
       const bool valid = (((16 * nt + m16) * g_magic) >> 16) < nq;
-      float x[KS][8];
+      uint32_t y[KS][4];   // the row's values, two to a word
 #pragma unroll
       for (int kk = 0; kk < KS; ++kk) {
-        const uint32_t w4[4] = {qf[nt][kk].x, qf[nt][kk].y, qf[nt][kk].z, qf[nt][kk].w};
-#pragma unroll
-        for (int j = 0; j < 8; ++j) x[kk][j] = (j & 1) ? hi_to_f32<F16>(w4[j >> 1]) : lo_to_f32<F16>(w4[j >> 1]);
+        y[kk][0] = qf[nt][kk].x; y[kk][1] = qf[nt][kk].y; y[kk][2] = qf[nt][kk].z; y[kk][3] = qf[nt][kk].w;
       }
       if (p.norm != MI_NORM_NONE) {
         float ss = 0.f;
 #pragma unroll
         for (int kk = 0; kk < KS; ++kk)
 #pragma unroll
-          for (int j = 0; j < 8; ++j) ss += x[kk][j] * x[kk][j];
+          for (int i = 0; i < 4; ++i) {
+            const float lo = lo_to_f32<F16>(y[kk][i]), hi = hi_to_f32<F16>(y[kk][i]);
+            ss += lo * lo;
+            ss += hi * hi;
+          }
         ss += xor16(ss);
         ss += xor32(ss);
         const float rstd = rsqrtf(ss * (1.f / HD) + p.eps);
@@ -184,14 +186,25 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
         for (int kk = 0; kk < KS; ++kk) {
           const uint32_t w4[4] = {qw[kk].x, qw[kk].y, qw[kk].z, qw[kk].w};
 #pragma unroll
-          for (int j = 0; j < 8; j += 2) {
-            const uint32_t packed = pack2<F16>(x[kk][j] * rstd * lo_to_f32<F16>(w4[j >> 1]),
-                                               x[kk][j + 1] * rstd * hi_to_f32<F16>(w4[j >> 1]));
-            x[kk][j] = lo_to_f32<F16>(packed);
-            x[kk][j + 1] = hi_to_f32<F16>(packed);
-          }
+          for (int i = 0; i < 4; ++i)
+            y[kk][i] = pack2<F16>(lo_to_f32<F16>(y[kk][i]) * rstd * lo_to_f32<F16>(w4[i]),
+                                  hi_to_f32<F16>(y[kk][i]) * rstd * hi_to_f32<F16>(w4[i]));
         }
       }
+      // (fp16 in packed arithmetic, which rounds as the conversions of the 32-bit form do: a product of two fp16 is exact in
+      // fp32, and a sum rounded to fp32 rounds on to fp16 as the exact one would; 3 instructions for two values, not 12)
+      auto rotated_pair = [](uint32_t x, uint32_t partner, uint32_t c, uint32_t sn) -> uint32_t {
+        if constexpr (F16) {
+#pragma clang fp contract(off)
+          const f16x2_t a = __builtin_bit_cast(f16x2_t, x) * __builtin_bit_cast(f16x2_t, c);
+          const f16x2_t b = __builtin_bit_cast(f16x2_t, partner) * __builtin_bit_cast(f16x2_t, sn);
+          return __builtin_bit_cast(uint32_t, a + b);
+        } else {
+          const uint32_t a = pack2<F16>(lo_to_f32<F16>(x) * lo_to_f32<F16>(c), hi_to_f32<F16>(x) * hi_to_f32<F16>(c));
+          const uint32_t b = pack2<F16>(lo_to_f32<F16>(partner) * lo_to_f32<F16>(sn), hi_to_f32<F16>(partner) * hi_to_f32<F16>(sn));
+          return pack2<F16>(lo_to_f32<F16>(a) + lo_to_f32<F16>(b), hi_to_f32<F16>(a) + hi_to_f32<F16>(b));
+        }
+      };
       auto rotated = [&](auto Ic) {
         constexpr bool INTERLEAVED = decltype(Ic)::value;
 #pragma unroll
@@ -200,21 +213,16 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
           const uint32_t s4[4] = {sw[nt][kk].x, sw[nt][kk].y, sw[nt][kk].z, sw[nt][kk].w};
           uint32_t o4[4];
 #pragma unroll
-          for (int j = 0; j < 8; j += 2) {
-            const float y0 = INTERLEAVED ? x[kk][j + 1] : x[kk ^ (KS / 2)][j], y1 = INTERLEAVED ? x[kk][j] : x[kk ^ (KS / 2)][j + 1];
-            const uint32_t a = pack2<F16>(x[kk][j] * lo_to_f32<F16>(c4[j >> 1]), x[kk][j + 1] * hi_to_f32<F16>(c4[j >> 1]));
-            const uint32_t b = pack2<F16>(y0 * lo_to_f32<F16>(s4[j >> 1]), y1 * hi_to_f32<F16>(s4[j >> 1]));
-            o4[j >> 1] = pack2<F16>(lo_to_f32<F16>(a) + lo_to_f32<F16>(b), hi_to_f32<F16>(a) + hi_to_f32<F16>(b));
-          }
+          for (int i = 0; i < 4; ++i)
+            o4[i] = rotated_pair(y[kk][i], INTERLEAVED ? __builtin_amdgcn_alignbit(y[kk][i], y[kk][i], 16) : y[kk ^ (KS / 2)][i],
+                                 c4[i], s4[i]);
           qf[nt][kk] = valid ? make_uint4(o4[0], o4[1], o4[2], o4[3]) : make_uint4(0, 0, 0, 0);
         }
       };
       if (!p.angles) {
 #pragma unroll
         for (int kk = 0; kk < KS; ++kk)
-          qf[nt][kk] = valid ? make_uint4(pack2<F16>(x[kk][0], x[kk][1]), pack2<F16>(x[kk][2], x[kk][3]),
-                                          pack2<F16>(x[kk][4], x[kk][5]), pack2<F16>(x[kk][6], x[kk][7]))
-                             : make_uint4(0, 0, 0, 0);
+          qf[nt][kk] = valid ? make_uint4(y[kk][0], y[kk][1], y[kk][2], y[kk][3]) : make_uint4(0, 0, 0, 0);
       } else if (p.interleaved) {
         rotated(std::true_type{});
       } else {
