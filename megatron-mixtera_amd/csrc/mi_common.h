@@ -304,26 +304,19 @@ static __device__ __forceinline__ f32x2_t fp8x2_lo_to_f32(uint32_t w) {
 static __device__ __forceinline__ f32x2_t fp8x2_hi_to_f32(uint32_t w) {
   return __builtin_amdgcn_cvt_pk_f32_fp8((int)w, true);
 }
-// Four e4m3fn bytes -> two packed bf16 pairs.  gfx950 converts a pair of OCP fp8 values to
-// a packed bf16 pair in one instruction (with a multiplier, 1.0 here); the conversion is
-// exact because every e4m3 value is representable in bf16.
-static __device__ __forceinline__ uint2 fp8x4_to_bf16x4(uint32_t w) {
-  const bf16x2_t lo = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, false);
-  const bf16x2_t hi = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, true);
-  return make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
-}
-
-// The same into the operand type of the kernel: bf16 pairs, or fp16 pairs (exact as well: e4m3 has 3 mantissa bits
-// and its exponents lie inside fp16's).
+// Four e4m3fn bytes -> two packed pairs of the kernel's operand type, times `pow2`, a power of two.  gfx950 converts a pair of OCP
+// fp8 values to a packed pair in one instruction, with the exponent of a float as multiplier; the conversion is exact: e4m3
+// has 3 mantissa bits, and its exponents lie inside bf16's and fp16's.
 template <bool F16>
-static __device__ __forceinline__ uint2 fp8x4_to_16x4(uint32_t w) {
+static __device__ __forceinline__ uint2 fp8x4_to_16x4(uint32_t w, float pow2 = 1.0f) {
   if constexpr (F16) {
-    typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
-    const f16x2_t lo = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, 1.0f, false);
-    const f16x2_t hi = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, 1.0f, true);
+    const f16x2_t lo = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, pow2, false);
+    const f16x2_t hi = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, pow2, true);
     return make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
   } else {
-    return fp8x4_to_bf16x4(w);
+    const bf16x2_t lo = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, pow2, false);
+    const bf16x2_t hi = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, pow2, true);
+    return make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
   }
 }
 

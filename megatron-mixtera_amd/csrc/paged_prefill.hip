@@ -990,7 +990,7 @@ static int prefill_kv_splits(int T, int Hq, int Hkv, int head_dim, int max_kv_le
   if (max_kv_len <= 0) return 1;
   const int G = Hq / Hkv, Gw = G < 16 ? G : 16, parts = (G + 15) / 16;
   const bool narrow = head_dim == 64;
-  const int sbq = (narrow ? prefill_woven_waves(64) : 8) * ((head_dim >= 192 ? 16 : 32) / Gw);  // query tokens per workgroup
+  const int sbq = (narrow ? 4 : 8) * ((head_dim >= 192 ? 16 : 32) / Gw);  // query tokens per workgroup
   const int64_t useful = (int64_t)Hkv * parts * ((T + sbq - 1) / sbq);
   const int64_t cus = 256, tiles = ((int64_t)max_kv_len + 63) / 64;
   if (useful >= (narrow ? 3 * cus : cus)) return 1;
@@ -1027,6 +1027,20 @@ extern "C" int64_t mi_prefill_workspace_bytes(int32_t T, int32_t R, int32_t Hq, 
     if (s > 1) bytes += (int64_t)s * T * Hq * (head_dim + 1) * (int64_t)sizeof(float);
   }
   return bytes;
+}
+
+// Wavefronts of the one-stream tile kernel's workgroups: eight have a CU to themselves and share every staged tile; of four, two
+// share a CU (width 64: three), so that one's start and end -- 11 us of every workgroup: its request, queries and first tiles, the
+// results, the dispatch of the next -- lie under the other's tiles, for twice the tiles' traffic.  That pays where walks are short:
+// prompts that start from nothing (`raw`: their rotation is part of the start) up to some 6 000 tokens, over an fp8 cache, where
+// every tile is converted as well, 4 600; chunks over a context up to some 2 500 keys.  By the host's bound of the keys.  Us, eight
+// wavefronts -> four, 32/8 heads of 128: 12 prompts of 1 000 tokens 214 -> 191, fp8 250 -> 233; one of 600 33.7 -> 26.5, of 2 000 73.5 ->
+// 62.4; six of 454-3 766 395 -> 381, fp8 445 -> 441; 4 x 5 000 826 -> 811, 3 x 6 000 852 -> 843, fp8 4 x 5 000 912 -> 915; 8 x 500 over 0-2 000
+// 113 -> 102, 8 x 512 over 1 536 162 both, 8 x 512 over 2 048 186 -> 188, 8 x 2 048 over 0-2 048 611 -> 620, in ranges 509 over 61 234 838 -> 909.
+static int prefill_woven_waves(int head_dim, bool fp8, bool raw, int n_split, int max_kv_len) {
+  if (head_dim == 64) return 4;
+  const int most = raw ? (fp8 ? 4608 : 6144) : 2560;
+  return n_split == 1 && max_kv_len > 0 && max_kv_len <= most ? 4 : 8;
 }
 
 // The two-phase tile kernel for one combination of (wave groups staggered?, fp8 cache?, keys split?, widths, type).
@@ -1136,12 +1150,6 @@ static int launch_paged_prefill(
     // head_dim 64 and 128: the one-stream tile kernel (measured at every size tried the faster of the two there: 1-3 %
     // at 128, 8-14 % at 64); the knob asks for the two-phase one
     const bool woven = tune.prefill_two_phase == 3 && (head_dim == 64 || head_dim == 128);
-    // wavefronts x whole tokens in a wavefront's 32 (wide heads: 16) rows
-    const int sbq_lds = (woven ? prefill_woven_waves(head_dim) : 8) * ((head_dim >= 192 ? 16 : 32) / Gw);
-    dim3 lgrid(prefill_query_blocks(T, R, sbq_lds) * Hkv * parts);
-    hipEvent_t ev_a, ev_b;
-    const bool timed = mi_profile_next(&ev_a, &ev_b);
-    if (timed) (void)hipEventRecord(ev_a, st);
     const bool stagger = tune.prefill_two_phase != 2;
     // key ranges per request (with a workspace only): partials behind the decode part's scratch
     int n_split = 1;
@@ -1154,11 +1162,17 @@ static int launch_paged_prefill(
       if (n_split > 1) {
         p.split_o = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(workspace) + dec_bytes);
         p.split_lse = p.split_o + (int64_t)n_split * T * Hq * head_dim;
-        lgrid.y = n_split;
         workspace_bytes = dec_bytes;
       }
     }
-    if (woven) launch_prefill_woven(p, lgrid, head_dim, fp8, f16, st);
+    const int waves = woven ? prefill_woven_waves(head_dim, fp8, raw != nullptr, n_split, max_kv_len) : 8;
+    // wavefronts x whole tokens in a wavefront's 32 (wide heads: 16) rows
+    const int sbq_lds = waves * ((head_dim >= 192 ? 16 : 32) / Gw);
+    const dim3 lgrid(prefill_query_blocks(T, R, sbq_lds) * Hkv * parts, n_split);
+    hipEvent_t ev_a, ev_b;
+    const bool timed = mi_profile_next(&ev_a, &ev_b);
+    if (timed) (void)hipEventRecord(ev_a, st);
+    if (woven) launch_prefill_woven(p, lgrid, head_dim, fp8, f16, waves, st);
     else if (fp8 && head_dim == 64 && f16) MI_PP_LAUNCH(true, 64, 64, true);
     else if (fp8 && head_dim == 64) MI_PP_LAUNCH(true, 64, 64, false);
     else if (fp8 && f16) MI_PP_LAUNCH(true, 128, 128, true);

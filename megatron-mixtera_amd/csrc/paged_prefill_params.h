@@ -191,10 +191,8 @@ static inline int prefill_query_blocks(int T, int R, int SBQ) {
 }
 
 // The one-stream ("woven") tile kernel for head_dim 64 and 128 (paged_prefill_woven.hip).  Same grid and request ->
-// workgroup map as the two-phase tile kernel: `grid.x` workgroups of prefill_woven_waves wavefronts, `grid.y` key
-// ranges (with more than one, `p.split_o` / `p.split_lse` receive the partials).
-void launch_prefill_woven(const PrefillParams& p, dim3 grid, int head_dim, bool fp8, bool f16, hipStream_t stream);
-// its wavefronts per workgroup (32 rows each)
-int prefill_woven_waves(int head_dim);
+// workgroup map as the two-phase tile kernel: `grid.x` workgroups of `waves` wavefronts (32 rows each; four or, at head_dim
+// 128, eight), `grid.y` key ranges (with more than one, `p.split_o` / `p.split_lse` receive the partials).
+void launch_prefill_woven(const PrefillParams& p, dim3 grid, int head_dim, bool fp8, bool f16, int waves, hipStream_t stream);
 
 }  // namespace mi

@@ -5,11 +5,11 @@
 // head_dim 64 and 128 over a 16-bit or fp8 cache whose chunk size is a multiple of 64.
 //
 // A workgroup of 8 wavefronts (two per SIMD, 256 registers each) takes 256 consecutive (query token, head-in-group)
-// rows of one (request, KV head), 32 rows per wavefront, and walks the keys in staged tiles of 64.  At head_dim 64 the
-// accumulators are half as many and the exponentials per product twice: there workgroups of 4 wavefronts, three per CU
-// (168 registers, 51 KB of LDS each), put a third wavefront on every SIMD to fill the vector pipe, and the work comes
-// in half the pieces (11 ragged prompts of 164-2 911 tokens, fp16: 148 us, the two-phase kernel 170; 8 x 2 048 new
-// tokens beside decoding requests: 754 against 838 us with everything).  There are no
+// rows of one (request, KV head), 32 rows per wavefront, and walks the keys in staged tiles of 64.  Workgroups of 4
+// wavefronts share a CU by twos (74 KB of LDS each) and cover each other's start and end where walks are short
+// (prefill_woven_waves).  At head_dim 64 the accumulators are half as many and the exponentials per product twice: there
+// workgroups of 4 wavefronts, three per CU (168 registers, 41 KB of LDS each), put a third wavefront on every SIMD to fill
+// the vector pipe (11 ragged prompts of 164-2 911 tokens, fp16: 148 us, the two-phase kernel 170).  There are no
 // matrix / vector phases and no per-phase barriers: every wavefront runs the whole tile pipeline in ONE stream, cut
 // into 32-key steps and software-pipelined so that three independent chains are always open --
 //     products    S^T(step s+1) = K Q^T          and  O^T += V^T P^T(step s-1)     (matrix cores)
@@ -23,15 +23,16 @@
 // registers, no LDS stores), as 18 instructions of 64 lanes x 16 bytes over a line of 64 rows x 18 pieces (288-byte
 // row pitch, the last two pieces of a row are padding).  The loads go through a buffer descriptor that covers the
 // tile's rows up to the request's last key: rows beyond it arrive as zeros (their probabilities are masked to zero,
-// and zero times a stale value must not be NaN).  Key tiles are double-buffered and value tiles triple-buffered
-// (values are multiplied one tile after their keys); the loads of the next pair are issued right after the tile's
-// barrier and are waited for at the next one.
+// and zero times a stale value must not be NaN).  Key and value tiles are double-buffered (values are multiplied one tile
+// after their keys: the second half of a value tile is loaded one barrier after the first, when the half it replaces has
+// been read); loads are issued right after the tile's barrier and are waited for at the next one.
 //
 // An fp8 cache (e4m3 bytes, one scale per chunk and KV head; a tile lies in one chunk) is staged through registers, a
 // tile ahead: 8-byte loads set out after one barrier and are stored, converted, before the next.  Key bytes are
 // converted exactly (four instructions per eight; e4m3 is a subset of both 16-bit types) and their scale multiplies the
-// softmax scale of the tile instead; values are multiplied by theirs and rounded.  (6 prompts of 454-3 766 tokens, head_dim
-// 128: 508 against 516 us with everything; head_dim 64: 329 against 360.)
+// softmax scale of the tile instead.  Value bytes are converted as cheaply, times the power of two of their scale; the rest of
+// the scale, 1 to 2, goes into the exponent of the tile's probabilities and out of their sum, which is kept per tile (values
+// multiplied by their scale and rounded took 48 more vector instructions per tile; 2 x 8 000 tokens 1 081 -> 1 066 us).
 //
 // Softmax: exponentials are taken against a per-row reference that moves only when a probability leaves a window (a
 // factor of 2^31 with bf16 operands, 2^8 with fp16); the row sums come out of the matrix cores (an all-ones A fragment).
@@ -49,14 +50,10 @@
 namespace mi {
 
 constexpr int kWvTile = 64;                      // keys per staged tile
-constexpr int kWvDepth = 1;                      // tiles between the issue of a tile's loads and the barrier that needs them
 constexpr int kWvAhead = 3;                      // fragments requested ahead of their products
 constexpr int kWvRing = 4;                       // fragment registers: fragment n lives in slot n % kWvRing
 // LDS bytes per staged row: the row and 32 bytes of padding (288 or 160: conflict-free fragment reads)
 template <int HD> constexpr int wv_pitch() { return 2 * HD + 32; }
-// (half as many at head_dim 128 with few workgroups, one wavefront per SIMD: 5-8 % faster up to one workgroup per CU,
-// slower beyond; two at head_dim 64: slower throughout)
-template <int HD> constexpr int wv_waves() { return HD == 64 ? 4 : 8; }
 // A row's reference is moved where a probability leaves the window, to where the row's largest one is 2^-headroom: with bf16
 // operands, whose exponents reach far below, 2^-30 under the 2 that the check looks for (one bit of a word); with fp16 1
 // under 2^8.
@@ -69,21 +66,20 @@ template <int HD> constexpr bool wv_piece_division_ok() {
     if (((u * wv_magic<HD>()) >> 16) != u / (wv_pitch<HD>() / 16)) return false;
   return true;
 }
-static_assert((kWvDepth == 1 || kWvDepth == 2) && wv_piece_division_ok<128>() && wv_piece_division_ok<64>(), "piece -> (row, column)");
+static_assert(wv_piece_division_ok<128>() && wv_piece_division_ok<64>(), "piece -> (row, column)");
 
-template <int HD, bool FP8, bool SPLIT, bool F16>
-__global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_prefill_woven_kernel(PrefillParams p) {
-  constexpr int KS = HD / 32, DV = HD / 16, NQ = 2, WAVES = wv_waves<HD>(), THREADS = 64 * WAVES;
+template <int HD, bool FP8, bool SPLIT, bool F16, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, HD == 64 ? 3 : 2) void paged_prefill_woven_kernel(PrefillParams p) {
+  constexpr int KS = HD / 32, DV = HD / 16, NQ = 2, THREADS = 64 * WAVES;
   constexpr int PITCH = wv_pitch<HD>(), PIECES = PITCH / 16, LOADS = kWvTile * PIECES / 64, BUF = LOADS * 1024;
   constexpr int NKF = 2 * KS, NVF = DV;  // key and value fragments of a 32-key slot
   constexpr int ESZ = FP8 ? 1 : 2;       // bytes per cache element
   static_assert(HD == 128 || HD == 64, "head widths");
   static_assert(kWvAhead < kWvRing && kWvAhead <= NKF && (NKF + NVF) % kWvRing == 0, "next slot's key fragments are requested after the tile's barrier");
-  // DEPTH: how many tiles ahead of their barrier the loads of a tile pair are issued.  Key tile t lives in
-  // Ks[t % KBUFS], value tile t in Vs[(t + 1) % VBUFS] (values are multiplied one tile after their keys).
-  constexpr int DEPTH = kWvDepth, KBUFS = DEPTH + 1, VBUFS = DEPTH + 2;
-  __shared__ __attribute__((aligned(16))) uint8_t Ks[KBUFS][BUF];
-  __shared__ __attribute__((aligned(16))) uint8_t Vs[VBUFS][BUF];
+  // Key tile t lives in Ks[t & 1], value tile t in Vs[t & 1], whose halves are filled one barrier apart (see `iteration`).
+  constexpr int HALF = BUF / 2;  // 32 rows of a tile
+  __shared__ __attribute__((aligned(16))) uint8_t Ks[2][BUF];
+  __shared__ __attribute__((aligned(16))) uint8_t Vs[2][BUF];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -233,9 +229,11 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
 
   float neg_run[NQ];  // the reference: a probability is 2^(score * scale + neg_run); kNoReference until a row has one
   f32x4_t acc[NQ][DV], accl[NQ];
+  float row_sum[NQ];  // fp8 only
 #pragma unroll
   for (int nt = 0; nt < NQ; ++nt) {
     neg_run[nt] = kNoReference;
+    row_sum[nt] = 0.f;
     accl[nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int e = 0; e < DV; ++e) acc[nt][e] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -258,19 +256,26 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
     const uint32_t ks_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)&Ks[0][0];
     const uint32_t vs_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)&Vs[0][0];
 
-    // ---- 16-bit cache: this wavefront's direct loads of a tile pair {key tile, value tile} ------------------------
-    // Load k of the pair's 2 LOADS (the first half: the key tile's line, the second: the value tile's) belongs to
-    // wavefront k % WAVES; with 36 loads over 8 wavefronts the fifth load of wavefronts 4-7 repeats their fourth, so
-    // that every wavefront issues as many.  Loads below NKL are key loads and loads above it value loads for every
-    // wavefront; load NKL is a key load for the first LOADS % WAVES wavefronts only.
-    constexpr int NL = (2 * LOADS + WAVES - 1) / WAVES, NKL = LOADS / WAVES;
+    // ---- 16-bit cache: this wavefront's direct loads of an iteration: a key tile's line, then the first half of a value
+    // tile's and the second half of the value tile's before it -------------------------------------------------------
+    // Load k of the 2 LOADS belongs to wavefront k % WAVES; with 36 loads over 8 wavefronts the fifth load of wavefronts 4-7
+    // repeats their fourth, so that every wavefront issues as many.  Where load i of a wavefront is of one kind for some
+    // wavefronts and of the next for the others, the wavefront's number decides.
+    static_assert(LOADS % 2 == 0, "half a tile is whole loads");
+    constexpr int NL = (2 * LOADS + WAVES - 1) / WAVES;
+    auto load_number = [&](int i, int w) { return w + WAVES * i < 2 * LOADS ? w + WAVES * i : w + WAVES * i - WAVES; };
+    // wavefronts (from 0) whose load i lies below `end`: all, none, or some
+    auto below = [&](int i, int end) {
+      if (load_number(i, WAVES - 1) < end && load_number(i, 0) < end) return true;
+      if (WAVES * i >= end + (WAVES * i + WAVES > 2 * LOADS ? WAVES : 0)) return false;
+      return load_number(i, wave) < end;
+    };
     uint32_t ld_off[NL];  // per lane: where its piece of the load comes from, relative to the tile's first row
     uint32_t ld_dst[NL];  // scalar: LDS offset of the load's 1 KiB inside its tile buffer
-    const bool mid_is_key = wave < LOADS % WAVES;
     if constexpr (!FP8) {
 #pragma unroll
       for (int i = 0; i < NL; ++i) {
-        const int k = wave + WAVES * i < 2 * LOADS ? wave + WAVES * i : wave + WAVES * i - WAVES;
+        const int k = load_number(i, wave);
         const bool is_key = k < LOADS;
         const int kp = is_key ? k : k - LOADS;
         ld_dst[i] = (uint32_t)__builtin_amdgcn_readfirstlane(1024 * kp);
@@ -285,27 +290,27 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
     constexpr int PPR8 = HD / 8, RPP8 = THREADS / PPR8, NP8 = kWvTile / RPP8;
     static_assert(NP8 * RPP8 == kWvTile && NP8 <= NKF && NP8 <= NVF, "one row per fragment position");
     uint2 kraw[NP8], vraw[NP8];
-    const uint32_t f_piece = 8u * (uint32_t)(tid % PPR8), f_row0 = (uint32_t)(tid / PPR8) * (uint32_t)tok_bytes + f_piece,
+    const uint32_t f_row0 = (uint32_t)(tid / PPR8) * (uint32_t)tok_bytes + 8u * (uint32_t)(tid % PPR8),
                    f_step = (uint32_t)RPP8 * (uint32_t)tok_bytes;
     const int f_lds = (tid / PPR8) * PITCH + 16 * (tid % PPR8);
-    // rows past the request's last key re-read that row (every query row masks them); `nrec`: see tile_nrec
-    auto fetch_fp8 = [&](const uint8_t* cache, int64_t off, uint32_t nrec, uint2 (&reg)[NP8]) {
-      const uint8_t* src = cache + (int64_t)h * p.kv_sh + off;
-      const uint32_t lim = nrec - (uint32_t)tok_bytes + f_piece;
+    // (through a descriptor of the tile's rows, as the direct loads: rows past the request's last key arrive as zeros)
+    auto fetch_fp8 = [&](uint64_t base, int64_t off, uint32_t nrec, uint2 (&reg)[NP8]) {
+      const auto rs = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(base + (uint64_t)off), 0, (int)nrec, 0x00020000);
 #pragma unroll
-      for (int i = 0; i < NP8; ++i) reg[i] = ld8(src + min(f_row0 + (uint32_t)i * f_step, lim));
+      for (int i = 0; i < NP8; ++i)
+        reg[i] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(rs, (int)(f_row0 + (uint32_t)i * f_step), 0, 0));
     };
     auto store_k_fp8 = [&](uint8_t* buf, int i) {
       const uint2 lo = fp8x4_to_16x4<F16>(kraw[i].x), hi = fp8x4_to_16x4<F16>(kraw[i].y);
       *reinterpret_cast<uint4*>(buf + f_lds + i * RPP8 * PITCH) = make_uint4(lo.x, lo.y, hi.x, hi.y);
     };
-    auto store_v_fp8 = [&](uint8_t* buf, int i, float vscale) {
-      const f32x2_t a = fp8x2_lo_to_f32(vraw[i].x), b = fp8x2_hi_to_f32(vraw[i].x);
-      const f32x2_t c = fp8x2_lo_to_f32(vraw[i].y), d = fp8x2_hi_to_f32(vraw[i].y);
-      *reinterpret_cast<uint4*>(buf + f_lds + i * RPP8 * PITCH) =
-          make_uint4(pack2<F16>(a.x * vscale, a.y * vscale), pack2<F16>(b.x * vscale, b.y * vscale),
-                     pack2<F16>(c.x * vscale, c.y * vscale), pack2<F16>(d.x * vscale, d.y * vscale));
+    auto store_v_fp8 = [&](uint8_t* buf, int i, float vscale) {   // (times the power of two of their scale)
+      const float pow2 = __uint_as_float(__float_as_uint(vscale) & 0x7f800000u);
+      const uint2 lo = fp8x4_to_16x4<F16>(vraw[i].x, pow2), hi = fp8x4_to_16x4<F16>(vraw[i].y, pow2);
+      *reinterpret_cast<uint4*>(buf + f_lds + i * RPP8 * PITCH) = make_uint4(lo.x, lo.y, hi.x, hi.y);
     };
+    // what is left of a value scale, from 1 to 2: it goes into its tile's probabilities (the exponent), and out of their sum
+    auto value_factor = [](float vscale) { return __uint_as_float((__float_as_uint(vscale) & 0x007fffffu) | 0x3f800000u); };
     // descriptor of a tile: its rows up to the request's last key (reads beyond return zeros)
     auto tile_rsrc = [&](uint64_t base, int64_t off, uint32_t nrec) {
       const uint64_t a = base + (uint64_t)off;
@@ -316,10 +321,11 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
       rs.w = 0x00020000u;
       return rs;
     };
-    auto issue_load = [&](int i, const u32x4_t& rs_k, const u32x4_t& rs_v, uint32_t kdst, uint32_t vdst) {
-      const bool is_key = i < NKL || (i == NKL && mid_is_key);
-      const u32x4_t rs = is_key ? rs_k : rs_v;
-      const uint32_t m0 = (is_key ? kdst : vdst) + ld_dst[i];
+    auto issue_load = [&](int i, const u32x4_t& rs_k, const u32x4_t& rs_v0, const u32x4_t& rs_v1, uint32_t kdst, uint32_t v0dst,
+                          uint32_t v1dst) {
+      const bool is_key = below(i, LOADS), first_half = below(i, LOADS + LOADS / 2);
+      const u32x4_t rs = is_key ? rs_k : first_half ? rs_v0 : rs_v1;
+      const uint32_t m0 = (is_key ? kdst : first_half ? v0dst : v1dst) + ld_dst[i];
       asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(m0), "v"(ld_off[i]), "s"(rs)
                    : "memory", "m0");
     };
@@ -365,6 +371,8 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
     // 16-bit: one scale for all scores.  fp8: a tile's own (kept off zero: zero times the -inf of a masked score would be NaN).
     auto tile_scale = [&](float ks) { return FP8 ? fmaxf(ks * p.scale_log2, 1.17549435e-38f) : p.scale_log2; };
     float scale_prev = p.scale_log2, scale_cur = p.scale_log2, scale_next = p.scale_log2, vscale = 1.f;
+    float factor_prev = 1.f, factor_cur = 1.f;   // fp8: value_factor of the tiles whose scales are scale_prev and scale_cur
+    auto value_scale = [&](float vs) { return fmaxf(uniform_float(vs), 1.17549435e-38f); };
     const uint4 ones = make_uint4(ones2<F16>(), ones2<F16>(), ones2<F16>(), ones2<F16>());
     const f32x4_t zero4 = {0.f, 0.f, 0.f, 0.f};
     // per-lane starts of the fragment reads inside a tile buffer
@@ -391,10 +399,10 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
       return make_uint4(a.x, a.y, b.x, b.y);
     };
     // probabilities of two scores (chunk c of a step's 8 per lane): rows nt = c >> 2, sub-tile (c >> 1) & 1, pair c & 1
-    auto exp_chunk = [&](const f32x4_t (&Sx)[NQ][2], uint4 (&Px)[NQ], int c, float scale) {
+    auto exp_chunk = [&](const f32x4_t (&Sx)[NQ][2], uint4 (&Px)[NQ], int c, float scale, const float (&neg)[NQ]) {
       const int nt = c >> 2, u = (c >> 1) & 1, q2 = 2 * (c & 1);
-      const float p0 = fast_exp2(__builtin_fmaf(Sx[nt][u][q2], scale, neg_run[nt]));
-      const float p1 = fast_exp2(__builtin_fmaf(Sx[nt][u][q2 + 1], scale, neg_run[nt]));
+      const float p0 = fast_exp2(__builtin_fmaf(Sx[nt][u][q2], scale, neg[nt]));
+      const float p1 = fast_exp2(__builtin_fmaf(Sx[nt][u][q2 + 1], scale, neg[nt]));
       const uint32_t w = pack2<F16>(p0, p1);
       const int d = 2 * u + (c & 1);
       if (d == 0) Px[nt].x = w; else if (d == 1) Px[nt].y = w; else if (d == 2) Px[nt].z = w; else Px[nt].w = w;
@@ -416,7 +424,8 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
     };
     // The reference of some row has to move (rare): it goes to the row's largest score of the step, what was summed against the old
     // one is rescaled, and the step's probabilities are made again.
-    auto move_reference = [&](const f32x4_t (&Sx)[NQ][2], uint4 (&Px)[NQ], float scale) {
+    auto move_reference = [&](const f32x4_t (&Sx)[NQ][2], uint4 (&Px)[NQ], float scale, float factor) {
+      float shifted[NQ];
 #pragma unroll
       for (int nt = 0; nt < NQ; ++nt) {
         float tm = -INFINITY;
@@ -433,16 +442,19 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
             acc[nt][e][0] *= alpha; acc[nt][e][1] *= alpha; acc[nt][e][2] *= alpha; acc[nt][e][3] *= alpha;
           }
           accl[nt][0] *= alpha; accl[nt][1] *= alpha; accl[nt][2] *= alpha; accl[nt][3] *= alpha;
+          if (FP8) row_sum[nt] *= alpha;
         }
+        shifted[nt] = FP8 ? neg + fast_log2(factor) : neg;
       }
 #pragma unroll
-      for (int c = 0; c < 8; ++c) exp_chunk(Sx, Px, c, scale);
+      for (int c = 0; c < 8; ++c) exp_chunk(Sx, Px, c, scale, shifted);
     };
 
     // ---- one 32-key slot.  H: the half of the key tile whose scores are multiplied (into S[H]); the vector ALU turns
     // S[1-H] into P[1-H]; the value product takes P[H] and half H of the value tile before.  ka / va: this lane's
     // fragment starts in the key tile's and the value tile's buffers, ka_next in the next key tile's.  key0: position
-    // of the first key of S[H] (MASK only).  at_barrier (H == 1): runs between the two groups of products.
+    // of the first key of S[H] (MASK only).  at_barrier (H == 1): runs between the two groups of products, and requests the
+    // first value fragments behind its barrier.
     auto slot = [&](auto Hc, auto Mc, const uint8_t* ka, const uint8_t* ka_next, const uint8_t* va, int key0,
                     auto&& at_barrier, auto&& under_scores, auto&& under_values) {
       constexpr int H = decltype(Hc)::value;
@@ -452,6 +464,10 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
       uint4 (&Px)[NQ] = P[1 - H];
       const uint4 (&Pv)[NQ] = P[H];
       const float scale = FP8 ? (H == 0 ? scale_prev : scale_cur) : p.scale_log2;  // of the scores in Sx
+      const float factor = FP8 ? (H == 0 ? factor_prev : factor_cur) : 1.f;
+      float neg[NQ];
+#pragma unroll
+      for (int nt = 0; nt < NQ; ++nt) neg[nt] = FP8 ? neg_run[nt] + fast_log2(factor) : neg_run[nt];
       // fragment n of the slot's stream: NKF key fragments, NVF value fragments, then the next slot's first keys
       auto request = [&](int n) {
         if (n < NKF) fr[n % RING] = read_k(ka, H, n);
@@ -474,15 +490,15 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
         }
         if (n < 8) {
           const int nt = n >> 2, u = (n >> 1) & 1, q2 = 2 * (n & 1);
-          xs[n][0] = __builtin_fmaf(Sx[nt][u][q2], scale, neg_run[nt]);
-          xs[n][1] = __builtin_fmaf(Sx[nt][u][q2 + 1], scale, neg_run[nt]);
+          xs[n][0] = __builtin_fmaf(Sx[nt][u][q2], scale, neg[nt]);
+          xs[n][1] = __builtin_fmaf(Sx[nt][u][q2 + 1], scale, neg[nt]);
         }
       };
       // scores: sub-tiles alternate, so a product meets its accumulator again four products later
       constexpr int EPP = 8 / NKF;  // positions of the probabilities' stages per key fragment: 1, or 2 at head width 64
 #pragma unroll
       for (int n = 0; n < NKF; ++n) {
-        request(n + AHEAD);
+        if (H == 0 || n + AHEAD < NKF) request(n + AHEAD);   // (the second half of a value tile: behind the barrier)
         MI_SB();
         const int u = n & 1, kk = n >> 1;
         Sn[0][u] = mfma_16x16x32<F16>(fr[n % RING], qf[0][kk], kk ? Sn[0][u] : zero4);
@@ -493,7 +509,13 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
         under_scores(n);
         MI_SB();
       }
-      if constexpr (H == 1) at_barrier();
+      if constexpr (H == 1) {
+        at_barrier([&] {
+#pragma unroll
+          for (int n = 0; n < AHEAD; ++n) request(NKF + n);
+          MI_SB();
+        });
+      }
       // the mask of the scores just multiplied, rows nt
       auto mask_step = [&](int nt) {
         if (!MASK) return;
@@ -523,21 +545,22 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
         under_values(e);
         MI_SB();
       }
-      accl[0] = mfma_16x16x32<F16>(ones, Pv[0], accl[0]);
-      accl[1] = mfma_16x16x32<F16>(ones, Pv[1], accl[1]);
+      // (fp8: the sums of one value tile, whose factor comes out of them in end_of_sums)
+      accl[0] = mfma_16x16x32<F16>(ones, Pv[0], FP8 && H == 0 ? zero4 : accl[0]);
+      accl[1] = mfma_16x16x32<F16>(ones, Pv[1], FP8 && H == 0 ? zero4 : accl[1]);
       MI_SB();
-      if (__builtin_amdgcn_ballot_w64(leaves_window(Px))) move_reference(Sx, Px, scale);
+      if (__builtin_amdgcn_ballot_w64(leaves_window(Px))) move_reference(Sx, Px, scale, factor);
       MI_SB();
     };
 
     // ---- prologue: clear the buffer of the value tile "before the first" (its probabilities are zeros, and zero times
     // a stale value must not be NaN; every other buffer is filled whole before it is read), start the first tiles ----
-    for (int i = tid * 16; i < BUF; i += THREADS * 16) *reinterpret_cast<uint4*>(&Vs[0][0] + i) = make_uint4(0u, 0u, 0u, 0u);
-    Cursor cur = cursor_at(tb + DEPTH + 1);
-    int64_t off_first[DEPTH + 1];   // tiles tb .. tb + DEPTH, started here
-    uint32_t nrec_first[DEPTH + 1];
+    for (int i = tid * 16; i < BUF; i += THREADS * 16) *reinterpret_cast<uint4*>(&Vs[1][0] + i) = make_uint4(0u, 0u, 0u, 0u);
+    Cursor cur = cursor_at(tb + 2);
+    int64_t off_first[2];   // tiles tb and tb + 1, started here
+    uint32_t nrec_first[2];
 #pragma unroll
-    for (int i = 0; i <= DEPTH; ++i) {
+    for (int i = 0; i < 2; ++i) {
       const Cursor c = cursor_at(tb + i);
       const int pc = __builtin_amdgcn_readfirstlane(bt_row[c.ci]);
       off_first[i] = tile_off(c, pc);
@@ -546,7 +569,8 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
         scales_request(pc);
         if (i == 0) {
           scale_prev = scale_cur = tile_scale(uniform_float(ks_v));
-          vscale = uniform_float(vs_v);
+          vscale = value_scale(vs_v);
+          factor_prev = factor_cur = value_factor(vscale);
         }
       }
     }
@@ -572,18 +596,17 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
       }
     }
     __syncthreads();
-    int64_t off_prev;
-    uint32_t nrec_prev;
+    int64_t off_prev, off_prev2 = off_first[0];   // of tiles j+1 and j
+    uint32_t nrec_prev, nrec_prev2 = nrec_first[0];
     if constexpr (FP8) {
-      static_assert(!FP8 || DEPTH == 1, "fp8 tiles wait in one set of registers");
-      fetch_fp8(p.kc, off_first[0], nrec_first[0], kraw);
+      fetch_fp8(kbase, off_first[0], nrec_first[0], kraw);
       MI_SB();
       if (raw) norm_and_rotate();
       MI_SB();
 #pragma unroll
       for (int i = 0; i < NP8; ++i) store_k_fp8(&Ks[0][0], i);
-      fetch_fp8(p.kc, off_first[1], nrec_first[1], kraw);  // stored by iteration 0
-      fetch_fp8(p.vc, off_first[0], nrec_first[0], vraw);
+      fetch_fp8(kbase, off_first[1], nrec_first[1], kraw);  // stored by iteration 0
+      fetch_fp8(vbase, off_first[0], nrec_first[0], vraw);
       off_prev = off_first[1];
       nrec_prev = nrec_first[1];
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -591,25 +614,22 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
       const u32x4_t rk0 = tile_rsrc(kbase, off_first[0], nrec_first[0]);
 #pragma unroll
       for (int i = 0; i < NL; ++i)
-        if (i < NKL || (i == NKL && mid_is_key)) issue_load(i, rk0, rk0, ks_lds, ks_lds);  // key tile 0 -> Ks[0]
+        if (below(i, LOADS)) issue_load(i, rk0, rk0, rk0, ks_lds, ks_lds, ks_lds);  // key tile 0 -> Ks[0]
+      // key tile 1 -> Ks[1], value tile 0 -> Vs[0], whole
+      const u32x4_t rk1 = tile_rsrc(kbase, off_first[1], nrec_first[1]), rv0 = tile_rsrc(vbase, off_first[0], nrec_first[0]);
 #pragma unroll
-      for (int t = 1; t <= DEPTH; ++t) {  // the pairs {key tile t -> Ks[t], value tile t - 1 -> Vs[t]}
-        const u32x4_t rk = tile_rsrc(kbase, off_first[t], nrec_first[t]);
-        const u32x4_t rv = tile_rsrc(vbase, off_first[t - 1], nrec_first[t - 1]);
-#pragma unroll
-        for (int i = 0; i < NL; ++i) issue_load(i, rk, rv, ks_lds + t * BUF, vs_lds + t * BUF);
-      }
-      off_prev = off_first[DEPTH];
-      nrec_prev = nrec_first[DEPTH];
+      for (int i = 0; i < NL; ++i) issue_load(i, rk1, rv0, rv0, ks_lds + BUF, vs_lds, vs_lds);
+      off_prev = off_first[1];
+      nrec_prev = nrec_first[1];
     }
     if constexpr (!FP8) {
       MI_SB();
       if (raw) norm_and_rotate();
       MI_SB();
     }
-    // key tile 0 has landed (this wavefront's share): only the DEPTH pairs issued after it may still be on their way
+    // key tile 0 has landed (this wavefront's share): only the loads issued after it may still be on their way
     if constexpr (!FP8) {
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(DEPTH * NL) : "memory");
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NL) : "memory");
     }
     __builtin_amdgcn_s_barrier();
     MI_SB();
@@ -617,51 +637,62 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
     const int t_mask = max(0, (full_until + 1) >> 6);              // first tile with a masked score for this wavefront
     const int jm = min(max(t_mask - tb, 0), ntl);                  // iterations [0, jm) need no mask
     int j = 0;
-    int kbi = 0, vbi = 0;  // j % KBUFS, j % VBUFS
+    int even = 0;   // BUF where j is odd
 #pragma unroll
     for (int n = 0; n < AHEAD; ++n) fr[n] = read_k(k_lane, 0, n);
 
-    // iteration j: scores of key tile j (Ks[j % KBUFS]), values of tile j-1 (Vs[j % VBUFS]); after its barrier key tile
-    // j+1 and value tile j are in LDS, and the loads of key tile j+DEPTH+1 (into the buffer of key tile j, which every
-    // wavefront has left) and value tile j+DEPTH (into the buffer of value tile j-2) set out under the products that follow.
+    auto end_of_sums = [&](float factor) {
+      const float inv = __builtin_amdgcn_rcpf(factor);
+#pragma unroll
+      for (int nt = 0; nt < NQ; ++nt) row_sum[nt] = __builtin_fmaf(accl[nt][0], inv, row_sum[nt]);
+    };
+    // Iteration j: scores of key tile j, values of tile j-1.  After its barrier, which follows the last score, every wavefront
+    // has left key tile j, the first half of value tile j-1 and the second half of value tile j-2: key tile j+2 and value
+    // tiles j+1 (first half) and j (second half) take their places, under the products that follow, for the next barrier.
     auto iteration = [&](auto Mc) {
-      const int kb = kbi * BUF;
-      const uint8_t* ka = k_lane + kb;
-      const uint8_t* ka_next = k_lane + (kbi == KBUFS - 1 ? 0 : kbi + 1) * BUF;
-      const uint8_t* va = v_lane + vbi * BUF;
+      const uint8_t* ka = k_lane + even;
+      const uint8_t* ka_next = k_lane + (BUF - even);
+      const uint8_t* va = v_lane + (BUF - even);
       const int key0 = (tb + j) * kWvTile;
-      u32x4_t rs_k, rs_v;
-      const uint32_t kdst = ks_lds + (uint32_t)kb;
-      const uint32_t vdst = vs_lds + (uint32_t)((vbi == 0 ? VBUFS - 1 : vbi - 1) * BUF);  // (j - 1) % VBUFS
-      // fp8: key tile j+1 and value tile j, fetched since the last barrier, go into LDS before this iteration's barrier
-      uint8_t* const kst = &Ks[0][0] + (kbi == KBUFS - 1 ? 0 : kbi + 1) * BUF;
-      uint8_t* const vst = &Vs[0][0] + (vbi == VBUFS - 1 ? 0 : vbi + 1) * BUF;
-      slot(std::integral_constant<int, 0>{}, Mc, ka, ka_next, va, key0, [] {}, [](int) {},
+      u32x4_t rs_k, rs_v0, rs_v1;
+      const uint32_t kdst = ks_lds + (uint32_t)even, v0dst = vs_lds + (uint32_t)(BUF - even), v1dst = vs_lds + (uint32_t)even;
+      // fp8: key tile j+1 and the first half of value tile j, fetched since the last barrier, go into LDS before this one
+      uint8_t* const kst = &Ks[0][0] + (BUF - even);
+      uint8_t* const vst = &Vs[0][0] + even;
+      slot(std::integral_constant<int, 0>{}, Mc, ka, ka_next, va, key0, [](auto) {}, [](int) {},
            [&](int e) {
              if constexpr (FP8) {
                if (e >= NVF - NP8) store_k_fp8(kst, e - (NVF - NP8));
              }
            });
       slot(std::integral_constant<int, 1>{}, Mc, ka, ka_next, va, key0 + 32,
-           [&] {
-             // this wavefront's share of key tile j+1 and value tile j has landed: only younger pairs are on their way
+           [&](auto first_values) {
+             // this wavefront's share of key tile j+1 and of the value tiles has landed
              if constexpr (FP8) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-             else asm volatile("s_waitcnt vmcnt(%0)" ::"n"((DEPTH - 1) * NL) : "memory");
+             else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
              __builtin_amdgcn_s_barrier();
+             first_values();
+             if constexpr (FP8) {
+#pragma unroll
+               for (int i = NP8 / 2; i < NP8; ++i) store_v_fp8(vst, i, vscale);
+             }
              if constexpr (FP8) pc_next = __builtin_amdgcn_readfirstlane(pc_v);
              else bt_arrived(pc_next);
              const int64_t off = tile_off(cur, pc_next);
              const uint32_t nrec = tile_nrec(cur);
              if constexpr (FP8) {
                scale_next = tile_scale(uniform_float(ks_v));  // (of tile j+1)
-               vscale = uniform_float(vs_v);
+               vscale = value_scale(vs_v);
                scales_request(pc_next);
-               fetch_fp8(p.kc, off, nrec, kraw);
-               fetch_fp8(p.vc, off_prev, nrec_prev, vraw);
+               fetch_fp8(kbase, off, nrec, kraw);
+               fetch_fp8(vbase, off_prev, nrec_prev, vraw);
              } else {
                rs_k = tile_rsrc(kbase, off, nrec);
-               rs_v = tile_rsrc(vbase, off_prev, nrec_prev);
+               rs_v0 = tile_rsrc(vbase, off_prev, nrec_prev);
+               rs_v1 = tile_rsrc(vbase, off_prev2, nrec_prev2);
              }
+             off_prev2 = off_prev;
+             nrec_prev2 = nrec_prev;
              off_prev = off;
              nrec_prev = nrec;
              cursor_next(cur);
@@ -670,29 +701,32 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
            },
            [&](int n) {
              if constexpr (FP8) {
-               if (n < NP8) store_v_fp8(vst, n, vscale);
+               if (n < NP8 / 2) store_v_fp8(vst, n, vscale);
              }
            },
            [&](int e) {
              if constexpr (!FP8) {
 #pragma unroll
-               for (int i = e; i < NL; i += NVF) issue_load(i, rs_k, rs_v, kdst, vdst);
+               for (int i = e; i < NL; i += NVF) issue_load(i, rs_k, rs_v0, rs_v1, kdst, v0dst, v1dst);
              }
            });
       if constexpr (FP8) {
+        end_of_sums(factor_prev);   // (the values of tile j-1)
         scale_prev = scale_cur;
         scale_cur = scale_next;
+        factor_prev = factor_cur;
+        factor_cur = value_factor(vscale);
       }
       ++j;
-      kbi = kbi == KBUFS - 1 ? 0 : kbi + 1;
-      vbi = vbi == VBUFS - 1 ? 0 : vbi + 1;
+      even = BUF - even;
     };
     for (; j < jm;) iteration(std::false_type{});
     for (; j < ntl;) iteration(std::true_type{});
 
-    // ---- drain: the last two steps' values (tile ntl - 1 in Vs[ntl % VBUFS]); S[1] is masked already ----
+    // ---- drain: the last two steps' values (tile ntl - 1), the second half when it has landed; S[1] is masked already ----
     {
-      const uint8_t* va = v_lane + vbi * BUF;
+      const uint8_t* va = v_lane + (BUF - even);
+      if (FP8) accl[0] = accl[1] = zero4;
       auto values = [&](int half, const uint4 (&Pv)[NQ]) {
 #pragma unroll
         for (int e = 0; e < DV; ++e) {
@@ -704,10 +738,16 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
         accl[1] = mfma_16x16x32<F16>(ones, Pv[1], accl[1]);
       };
       values(0, P[0]);
+      float neg_last[NQ];
 #pragma unroll
-      for (int c = 0; c < 8; ++c) exp_chunk(S[1], P[1], c, FP8 ? scale_prev : p.scale_log2);
-      if (__builtin_amdgcn_ballot_w64(leaves_window(P[1]))) move_reference(S[1], P[1], FP8 ? scale_prev : p.scale_log2);
+      for (int nt = 0; nt < NQ; ++nt) neg_last[nt] = FP8 ? neg_run[nt] + fast_log2(factor_prev) : neg_run[nt];
+#pragma unroll
+      for (int c = 0; c < 8; ++c) exp_chunk(S[1], P[1], c, FP8 ? scale_prev : p.scale_log2, neg_last);
+      if (__builtin_amdgcn_ballot_w64(leaves_window(P[1]))) move_reference(S[1], P[1], FP8 ? scale_prev : p.scale_log2, factor_prev);
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
       values(1, P[1]);
+      if (FP8) end_of_sums(factor_prev);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no direct load may still be on its way into this workgroup's LDS
 #undef MI_SB
@@ -716,7 +756,7 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
   // ---- epilogue: acc[nt][e][i] is output element d = 16e + 4g + i of row (nt, m16) --------------
 #pragma unroll
   for (int nt = 0; nt < NQ; ++nt) {
-    const float l_tot = accl[nt][0];
+    const float l_tot = FP8 ? row_sum[nt] : accl[nt][0];
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
     const int n = 16 * nt + m16;
     const int qi = (n * g_magic) >> 16, u = n - qi * G;  // n / G, n % G
@@ -740,22 +780,23 @@ __global__ __launch_bounds__(64 * wv_waves<HD>(), HD == 64 ? 3 : 2) void paged_p
   }
 }
 
-int prefill_woven_waves(int head_dim) { return head_dim == 64 ? wv_waves<64>() : wv_waves<128>(); }
 
-void launch_prefill_woven(const PrefillParams& p, dim3 grid, int head_dim, bool fp8, bool f16, hipStream_t st) {
+void launch_prefill_woven(const PrefillParams& p, dim3 grid, int head_dim, bool fp8, bool f16, int waves, hipStream_t st) {
   const bool split = grid.y > 1;
-#define MI_WV_LAUNCH(HD_, FP8_)                                                                                     \
+#define MI_WV_LAUNCH(HD_, FP8_, W_)                                                                                  \
   do {                                                                                                              \
-    const dim3 block(64 * wv_waves<HD_>());                                                                         \
-    if (split && f16) hipLaunchKernelGGL((paged_prefill_woven_kernel<HD_, FP8_, true, true>), grid, block, 0, st, p); \
-    else if (split) hipLaunchKernelGGL((paged_prefill_woven_kernel<HD_, FP8_, true, false>), grid, block, 0, st, p); \
-    else if (f16) hipLaunchKernelGGL((paged_prefill_woven_kernel<HD_, FP8_, false, true>), grid, block, 0, st, p);  \
-    else hipLaunchKernelGGL((paged_prefill_woven_kernel<HD_, FP8_, false, false>), grid, block, 0, st, p);          \
+    const dim3 block(64 * W_);                                                                                      \
+    if (split && f16) hipLaunchKernelGGL((paged_prefill_woven_kernel<HD_, FP8_, true, true, W_>), grid, block, 0, st, p); \
+    else if (split) hipLaunchKernelGGL((paged_prefill_woven_kernel<HD_, FP8_, true, false, W_>), grid, block, 0, st, p); \
+    else if (f16) hipLaunchKernelGGL((paged_prefill_woven_kernel<HD_, FP8_, false, true, W_>), grid, block, 0, st, p); \
+    else hipLaunchKernelGGL((paged_prefill_woven_kernel<HD_, FP8_, false, false, W_>), grid, block, 0, st, p);      \
   } while (0)
-  if (head_dim == 64 && fp8) MI_WV_LAUNCH(64, true);
-  else if (head_dim == 64) MI_WV_LAUNCH(64, false);
-  else if (fp8) MI_WV_LAUNCH(128, true);
-  else MI_WV_LAUNCH(128, false);
+  if (head_dim == 64 && fp8) MI_WV_LAUNCH(64, true, 4);
+  else if (head_dim == 64) MI_WV_LAUNCH(64, false, 4);
+  else if (fp8 && waves == 4) MI_WV_LAUNCH(128, true, 4);
+  else if (fp8) MI_WV_LAUNCH(128, true, 8);
+  else if (waves == 4) MI_WV_LAUNCH(128, false, 4);
+  else MI_WV_LAUNCH(128, false, 8);
 #undef MI_WV_LAUNCH
 }
 

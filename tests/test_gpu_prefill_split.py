@@ -46,3 +46,39 @@ def test_every_query_block_has_a_workgroup(mi, dev, d, Hq, Hkv, q_lens):
             out = mi.ops.paged_prefill_attention(q.to(dev), kc.to(dev), vc.to(dev), cu_q.to(dev), kv_lens.to(dev), bt.to(dev),
                                                  max_kv_len=int(kv_lens.max()), one_row_requests=False).float().cpu()
         assert (out - ref).abs().max().item() < 2e-2
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("Hq,Hkv", [(32, 8), (8, 8), (16, 1), (40, 2)])
+def test_four_wavefronts_give_what_eight_do(mi, dev, Hq, Hkv, dtype, fp8):
+    """A row's walk over the tiles does not depend on the rows that share its workgroup: the same bits with the bound of the
+    keys that chooses four wavefronts and with one that chooses eight.  Requests around a tile, a block and two tiles, with and
+    without a context, values whose scale differs from chunk to chunk."""
+    q_lens, ctx, chunk, d = [1, 63, 64, 65, 33, 128, 200, 7], [0, 0, 0, 0, 300, 63, 1, 130], 64, 128
+    kv_lens = torch.tensor([a + b for a, b in zip(q_lens, ctx)], dtype=torch.int32)
+    cu_q = torch.zeros(len(q_lens) + 1, dtype=torch.int32)
+    cu_q[1:] = torch.cumsum(torch.tensor(q_lens), 0)
+    gen = torch.Generator().manual_seed(Hq)
+    bt, N = mi.synthetic.build_block_table(kv_lens, chunk, gen)
+    T = int(cu_q[-1])
+    q = torch.randn(T, Hq, d, generator=gen).to(dtype)
+    kc, vc = ((torch.randn(N, chunk, Hkv, d, generator=gen) * (0.05 + 4 * torch.rand(N, 1, 1, 1, generator=gen))).to(dtype) for _ in range(2))
+    kw, ref_kw, caches = {}, {}, [kc.to(dev), vc.to(dev)]
+    if fp8:
+        pools = [torch.empty(kc.shape, dtype=torch.uint8, device=dev) for _ in range(2)]
+        scales = [torch.empty(N, Hkv, dtype=torch.float32, device=dev) for _ in range(2)]
+        for src, pool, scale in zip(caches, pools, scales):
+            mi.ops.quantize_chunks_fp8(src, pool, scale)
+        caches, kw = pools, dict(k_scales=scales[0], v_scales=scales[1])
+        ref_kw = {k: v.cpu() for k, v in kw.items()}
+    out = [mi.ops.paged_prefill_attention(q.to(dev), *caches, cu_q.to(dev), kv_lens.to(dev), bt.to(dev), max_kv_len=most,
+                                          one_row_requests=False, **kw) for most in (int(kv_lens.max()), 100000)]
+    with mi.ops.tuning(prefill_kv_split=-1):
+        eight = mi.ops.paged_prefill_attention(q.to(dev), *caches, cu_q.to(dev), kv_lens.to(dev), bt.to(dev), max_kv_len=100000,
+                                               one_row_requests=False, **kw)
+    assert torch.equal(out[0], eight)
+    ref = oa.paged_varlen_attention(q, caches[0].cpu(), caches[1].cpu(), cu_q, kv_lens, bt, **ref_kw)
+    bound = 2e-2 + 2e-2 * ref.abs()
+    for o in out:
+        assert ((o.float().cpu() - ref).abs() <= bound).all()
