@@ -70,6 +70,7 @@ struct DecodeParams {
   uint64_t chunk_magic;  // ceil(2^40 / chunk)
   int32_t R, Hq, Hkv, G, chunk, min_span_tiles, grid;  // min_span_tiles: 0 = from the lengths (see walk_segments)
   int32_t parts;  // wavefronts per KV head: each takes up to 16 of the G query heads that share it
+  int32_t splits;  // decode_short_kernel: workgroups per request and KV head
   // Fused decode step only (FUSED kernels): `q` holds the raw queries of the step, head h * G + u of a row at
   // h * q_gst + u * d; the step's new key / value rows, norm weights, rotary table and positions.
   int64_t q_gst;
@@ -986,20 +987,22 @@ __global__ __launch_bounds__(512, MINW) void decode_step_stream_kernel(DecodePar
   decode_stream_body<HD, HD, NT, FP8, F16, true>(p);
 }
 
-// A few short requests: one workgroup per request and (virtual) KV head, its wavefronts a share of the tokens each, their
-// partials merged in LDS.  The stream above cuts such requests over the chip and needs a second launch to merge them, half as
-// long as the first.
+// A few short requests: `splits` workgroups per request and (virtual) KV head, their wavefronts a share of the tokens each, a
+// workgroup's partials merged in LDS.  With one workgroup that is the result.  The stream above cuts such requests over the
+// chip into as many pieces as there are tiles or so and needs a second launch to find and merge them, half as long as the
+// first; here the pieces are few, and decode_short_merge_kernel knows where they are.
 constexpr int kShortWaves = 8;
 template <int HD, int NT, bool FP8, bool F16, bool FUSED>
 __global__ __launch_bounds__(64 * kShortWaves, 2) void decode_short_kernel(DecodeParams p) {
   extern __shared__ int cum[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int HV = p.Hkv * p.parts, busy = p.R * HV;
+  const int HV = p.Hkv * p.parts, busy = p.R * HV * p.splits;
   if ((int)blockIdx.x >= busy) {
     if constexpr (FUSED && !FP8) fetch_next_matrix(busy);
     return;
   }
-  const int r = blockIdx.x / HV, hv = blockIdx.x - r * HV;
+  const int split = blockIdx.x / (p.R * HV), rh = blockIdx.x - split * (p.R * HV);
+  const int r = rh / HV, hv = rh - r * HV;
   const int h = p.parts > 1 ? hv / p.parts : hv, part = hv - h * p.parts;
   const int hq0 = h * p.G + 16 * part, gq = min(16, p.G - 16 * part);
   int row;
@@ -1009,8 +1012,9 @@ __global__ __launch_bounds__(64 * kShortWaves, 2) void decode_short_kernel(Decod
   const int tiles = tiles_of(len, TK);
   uint8_t* const lds = reinterpret_cast<uint8_t*>(cum);
   const int per_wave = short_lds_per_wave(HD, p.G, FUSED);
-  // (whole tiles, evenly: a wavefront's tiles follow one another)
-  const int tb = tiles * wave / kShortWaves, te = tiles * (wave + 1) / kShortWaves;
+  // (whole tiles, evenly over the workgroups, then over the wavefronts: a wavefront's tiles follow one another)
+  const int wb = (int)((int64_t)tiles * split / p.splits), wn = (int)((int64_t)tiles * (split + 1) / p.splits) - wb;
+  const int tb = wb + wn * wave / kShortWaves, te = wb + wn * (wave + 1) / kShortWaves;
   if (te > tb) {
     decode_segment<HD, HD, NT, FP8, F16, FUSED, true>(p, r, row, h, hq0, gq, len, tb * TK, min(te * TK, len), false, te == tiles,
                                                       0, lane, lds + wave * per_wave);
@@ -1037,10 +1041,50 @@ __global__ __launch_bounds__(64 * kShortWaves, 2) void decode_short_kernel(Decod
       num.x += a * v.x; num.y += a * v.y; num.z += a * v.z; num.w += a * v.w;
       den += a * ml[w].y;
     }
-    const float inv = den > 0.f ? 1.f / den : 0.f;   // (a request without tokens: zeros)
-    st8(p.out + (int64_t)row * p.o_st + (int64_t)(hq0 + m) * p.o_sh + d,
-        make_uint2(pack2<F16>(num.x * inv, num.y * inv), pack2<F16>(num.z * inv, num.w * inv)));
+    if (p.splits == 1) {
+      const float inv = den > 0.f ? 1.f / den : 0.f;   // (a request without tokens: zeros)
+      st8(p.out + (int64_t)row * p.o_st + (int64_t)(hq0 + m) * p.o_sh + d,
+          make_uint2(pack2<F16>(num.x * inv, num.y * inv), pack2<F16>(num.z * inv, num.w * inv)));
+    } else {   // (the maximum beside the sum: part_lse holds two floats per head here)
+      const int64_t at = ((int64_t)split * p.R + r) * p.Hq + hq0 + m;
+      *reinterpret_cast<float4*>(p.part_o + at * HD + d) = num;
+      if (d == 0) reinterpret_cast<float2*>(p.part_lse)[at] = make_float2(mx, den);
+    }
   }
+}
+
+// The partials of a request's `splits` workgroups -> its output rows.  A thread has four values of one head; every load it
+// needs is asked for at once.
+constexpr int kShortSplits = 32;
+template <bool F16, int S>
+__global__ __launch_bounds__(256) void decode_short_merge_kernel(DecodeParams p, int head_dim) {
+  const int r = blockIdx.y, i = blockIdx.x * 256 + threadIdx.x, q4 = head_dim >> 2;
+  const int hq = min(i / q4, p.Hq - 1), d = 4 * (i % q4);
+  float2 ml[S];
+  float4 v[S];
+#pragma unroll
+  for (int k = 0; k < S; ++k) {
+    const int64_t at = ((int64_t)min(k, p.splits - 1) * p.R + r) * p.Hq + hq;
+    ml[k] = reinterpret_cast<const float2*>(p.part_lse)[at];
+    v[k] = *reinterpret_cast<const float4*>(p.part_o + at * head_dim + d);
+  }
+  int row;
+  if (!decode_row(p, r, row) || i >= p.Hq * q4) return;   // (a row of another kind: what was read is not its)
+  float mx = -INFINITY, den = 0.f;
+#pragma unroll
+  for (int k = 0; k < S; ++k)
+    if (k < p.splits) mx = fmaxf(mx, ml[k].x);
+  float4 num = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+  for (int k = 0; k < S; ++k) {
+    if (k >= p.splits || ml[k].y == 0.f) continue;   // (no tiles)
+    const float a = fast_exp2(ml[k].x - mx);
+    num.x += a * v[k].x; num.y += a * v[k].y; num.z += a * v[k].z; num.w += a * v[k].w;
+    den += a * ml[k].y;
+  }
+  const float inv = den > 0.f ? 1.f / den : 0.f;
+  st8(p.out + (int64_t)row * p.o_st + (int64_t)hq * p.o_sh + d,
+      make_uint2(pack2<F16>(num.x * inv, num.y * inv), pack2<F16>(num.z * inv, num.w * inv)));
 }
 
 // Multi-latent attention, absorbed form: every query head attends to the same 576-wide latent rows
@@ -1902,24 +1946,34 @@ int mi::check_decode_workspace(const void* workspace, int64_t workspace_bytes, i
   return MI_OK;
 }
 
-// Whether a batch goes to decode_short_kernel: `workgroups` of it, requests of at most `most` tokens as far as the table's width
-// tells.  A CU alone takes in some 30 KB/us of a cache in HBM (64-byte pieces of keys, whole rows of values), the second launch
-// and the trip of the partials cost 4-7 us, and with more workgroups than CUs the stream's equal spans balance better.  Us per
-// call in a graph, twelve caches in turn, stream + merge -> short, lengths from a quarter of the bound up, 128 wide, 16-bit:
-//   bound 64 tokens: 1 x 32/8 heads 8.3 -> 4.1, 16 x 32/8 11.8 -> 5.1, 64 x 32/8 12.3 -> 8.3; 256 tokens: 2 x 32/8 12.4 -> 7.3, 16 x
-//   32/8 13.2 -> 8.4, 64 x 32/8 21.3 -> 14.8, 128 x 32/8 28.1 -> 26.9 (the whole step 30.0 -> 36.6: not there);
-//   512 tokens: 16 x 32/8 15.3 -> 13.8, 32 x 32/8 21.4 -> 14.4, 128 x 16/2 21.9 -> 14.1, but 8 x 16/2 9.1 -> 10.9;
-//   1 024 tokens: 32 x 32/8 27.0 -> 24.1, 128 x 16/2 29.2 -> 22.0, but 8 x 32/8 15.2 -> 19.9, 16 x 32/8 step 21.9 -> 23.3.
-// The whole step of a layer, likewise: 16 x 32/8, bound 512: 19.1 -> 15.1.
+// Workgroups per request and KV head for decode_short_kernel, 0: the stream.  `heads` (virtual) KV heads, requests of at most
+// `most` tokens as far as the table's width tells.
+//
+// A CU alone takes in some 30 KB/us of a cache in HBM, so a request's keys and values of a head go to as many workgroups as the
+// chip has left, from 48 KB each up; the shortest (128 KB in all) to one, without a second launch.  Requests of different
+// lengths get the same number, and the longest decides: with `share` KB of the longest's keys and values per workgroup
+// this takes 7 us and share / 28, the stream, whose spans are equal, 10.5 us and the whole at 6.3 TB/s, lengths taken as
+// three quarters of the bound.  Us per call in a graph, twelve caches in turn, the stream and its merge -> this, 128 wide, 16-bit:
+//   one request, 32/8 heads: 31 tokens 8.3 -> 4.1, 215 12.3 -> 7.5, 687 13.1 -> 8.2, 4 515 19.5 -> 14.5, 14 136 31.4 -> 21.5, 36 122
+//   45.7 -> 36.5; 4 x 16/2 of 12 701-21 684 29.4 -> 23.8; 8 x 32/8 of 1 558-2 896 25.7 -> 22.6, of 3 668-5 861 37.6 / 39.2 (estimated
+//   level); 16 x 32/8 of 577-940 21.9 -> 17.2, of 1 015-1 980 28.4 -> 28.0, of 2 063-3 886 47.2 / 49.5; 32 x 32/8 of 261-1 007 27.0 ->
+//   24.8; up to 256 tokens 64 x 32/8 21.3 -> 14.8, 128 x 32/8 (a whole step) 30.0 / 36.6: not there.
+// The whole step of a layer: 1 x 32/8 of 519 13.3 -> 10.5, 2 of 1 955-2 838 22.4 -> 14.9, 16 of 250-499 19.8 -> 15.2.
 constexpr int kShortTile = 2;   // (sub-tiles per iteration; four are 3-8 % slower)
-static bool decode_is_short(int workgroups, int head_dim, int64_t most, int esz, int chunk_tokens, const MiTuning& tune,
-                            int split_tokens) {
-  if ((head_dim != 64 && head_dim != 128) || chunk_tokens % (16 * kShortTile)) return false;
-  if (tune.decode_grid > 0 || tune.decode_tile_subtiles > 0 || split_tokens > 0) return false;   // (the stream's own knobs)
-  const int64_t bytes = most * head_dim * 2 * esz;   // of the longest request's keys and values for one head
-  if (bytes <= 128 << 10) return workgroups <= 512;
-  if (bytes <= 256 << 10) return workgroups >= 64 && workgroups <= 256;
-  return bytes <= 512 << 10 && workgroups >= 192 && workgroups <= 256;
+static int short_splits(int R, int heads, int head_dim, int64_t most, int esz, int chunk_tokens, int grid, const MiTuning& tune,
+                        int split_tokens) {
+  if ((head_dim != 64 && head_dim != 128) || chunk_tokens % (16 * kShortTile)) return 0;
+  if (tune.decode_grid > 0 || tune.decode_tile_subtiles > 0 || split_tokens > 0) return 0;   // (the stream's own knobs)
+  const int64_t workgroups = (int64_t)R * heads, kb = (most * head_dim * 2 * esz + 1023) >> 10;   // of the longest, one head
+  if (kb <= 128) return workgroups <= 512 ? 1 : 0;
+  if (workgroups > 256) return 0;
+  int64_t n = 256 / workgroups;
+  if (n > kShortSplits) n = kShortSplits;
+  if (n > (kb + 47) / 48) n = (kb + 47) / 48;
+  if (n > (grid + R) / (2 * R)) n = (grid + R) / (2 * R);   // (what the workspace holds: two words per head beside the values)
+  if (n < 1) return 0;
+  const float share = (float)kb / (float)n;
+  return 7.f + share / 28.f < 10.5f + 0.75f * (float)workgroups * (float)kb / 6300.f ? (int)n : 0;
 }
 
 int mi::launch_paged_decode(
@@ -2048,8 +2102,10 @@ int mi::launch_paged_decode(
   hipEvent_t ev_a, ev_b;
   const bool timed = mi_profile_next(&ev_a, &ev_b);
   if (timed) (void)hipEventRecord(ev_a, st);
-  if (decode_is_short(R * waves, head_dim, bt_stride * chunk_tokens, esz, chunk_tokens, tune, split_tokens)) {
-    const dim3 sgrid(p.next_w && fused ? (R * waves > grid_x ? R * waves : grid_x) : R * waves), sblock(64 * kShortWaves);
+  p.splits = short_splits(R, waves, head_dim, bt_stride * chunk_tokens, esz, chunk_tokens, grid_x, tune, split_tokens);
+  if (p.splits > 0) {
+    const int busy = R * waves * p.splits;
+    const dim3 sgrid(p.next_w && fused && busy < grid_x ? grid_x : busy), sblock(64 * kShortWaves);
     const size_t slds = (size_t)kShortWaves * short_lds_per_wave(head_dim, G, fused != nullptr);
 #define MI_LAUNCH_SHORT(HD_, NT_, FP8_, FUSED_)                                                                         \
     do {                                                                                                                \
@@ -2065,6 +2121,19 @@ int mi::launch_paged_decode(
     else MI_LAUNCH_SHORT(64, kShortTile, false, false);
 #undef MI_LAUNCH_SHORT
     if (timed) (void)hipEventRecord(ev_b, st);
+    if (p.splits > 1) {
+      const dim3 mgrid((Hq * head_dim / 4 + 255) / 256, R);
+#define MI_LAUNCH_SHORT_MERGE(S_)                                                                                       \
+      do {                                                                                                              \
+        if (f16) hipLaunchKernelGGL((decode_short_merge_kernel<true, S_>), mgrid, dim3(256), 0, st, p, head_dim);       \
+        else hipLaunchKernelGGL((decode_short_merge_kernel<false, S_>), mgrid, dim3(256), 0, st, p, head_dim);          \
+      } while (0)
+      if (p.splits <= 4) MI_LAUNCH_SHORT_MERGE(4);
+      else if (p.splits <= 8) MI_LAUNCH_SHORT_MERGE(8);
+      else if (p.splits <= 16) MI_LAUNCH_SHORT_MERGE(16);
+      else MI_LAUNCH_SHORT_MERGE(kShortSplits);
+#undef MI_LAUNCH_SHORT_MERGE
+    }
     return mi_check_launch("mi_paged_decode_attention");
   }
 #define MI_LAUNCH_DECODE(HD_, FP8_, F16_)                                                                              \

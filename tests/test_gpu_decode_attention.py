@@ -305,3 +305,29 @@ def test_short_requests_by_one_workgroup_per_head(mi, dev, Hq, Hkv, d, chunk, fp
     assert (out[0] == 0).all()
     stream = mi.ops.paged_decode_attention(case.q, *caches, case.kv_lens, case.block_table, split_tokens=64, **kw)
     _close(out.squeeze(1), stream.float().cpu().squeeze(1), 8e-3)
+
+
+@pytest.mark.parametrize("Hq,Hkv,d,chunk,lens", [
+    (8, 8, 64, 32, [0, 1, 33, 2047, 2048]), (32, 8, 128, 256, [5, 700, 1025]), (16, 1, 128, 64, [0, 31, 64, 65, 900, 1500, 1537, 3]),
+    (20, 1, 64, 256, [7000]), (4, 2, 128, 128, [9001, 12]), (64, 8, 128, 256, [40000])])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_few_requests_by_several_workgroups_per_head(mi, dev, Hq, Hkv, d, chunk, lens, fp8):
+    """Requests cut evenly over workgroups and their merge, against the stream: shares without tiles, without all of their
+    wavefronts' tiles, a request without tokens; as few and as many workgroups as there are; scratch filled with NaN."""
+    lens = torch.tensor(lens, dtype=torch.int32)
+    cfg = mi.synthetic.DecodeConfig("splits", lens.numel(), Hq, Hkv, d, 0, 0, chunk=chunk, seed=Hq + d)
+    case = mi.synthetic.make_decode_case(cfg, dev, lens=lens, on_device_rng=True)
+    caches, kw = (case.k_cache, case.v_cache), {}
+    if fp8:
+        caches = tuple(torch.empty(case.k_cache.shape, dtype=torch.uint8, device=dev) for _ in range(2))
+        scales = [torch.empty(case.k_cache.size(0), Hkv, dtype=torch.float32, device=dev) for _ in range(2)]
+        for src, pool, scale in zip((case.k_cache, case.v_cache), caches, scales):
+            mi.ops.quantize_chunks_fp8(src, pool, scale)
+        kw = dict(k_scales=scales[0], v_scales=scales[1])
+    need = mi.ops.decode_workspace_bytes(lens.numel(), Hq, Hkv, d, chunk, int(lens.max()))
+    scratch = torch.full((need // 4 + 64,), float("nan"), dtype=torch.float32, device=dev).view(torch.uint8)
+    out = mi.ops.paged_decode_attention(case.q, *caches, case.kv_lens, case.block_table, workspace=scratch[:need], **kw)
+    assert torch.isnan(scratch[need:].view(torch.float32)).all()    # nothing beyond what was asked for
+    stream = mi.ops.paged_decode_attention(case.q, *caches, case.kv_lens, case.block_table, split_tokens=64, **kw)
+    _close(out.squeeze(1), stream.float().cpu().squeeze(1), 8e-3)
+    assert (out[(lens == 0).to(dev)] == 0).all()
