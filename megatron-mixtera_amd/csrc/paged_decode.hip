@@ -2445,7 +2445,6 @@ extern "C" int mi_paged_mla_decode_attention(
     int64_t o_stride_tok, int64_t o_stride_head, void* workspace, int64_t workspace_bytes, int32_t R, int32_t Hq,
     int32_t head_dim_k, int32_t head_dim_v, int32_t chunk_tokens, int32_t max_kv_len, float softmax_scale,
     int32_t dtype, const MiTuning* tuning, void* stream) {
-  (void)max_kv_len;
   if (R == 0) return MI_OK;
   if (dtype != MI_DTYPE_BF16 && dtype != MI_DTYPE_FP16)
     return mi_fail(MI_ERR_UNSUPPORTED, "mi_paged_mla_decode_attention: dtype must be MI_DTYPE_BF16 or MI_DTYPE_FP16");
@@ -2492,9 +2491,17 @@ extern "C" int mi_paged_mla_decode_attention(
   const bool shared_tile = chunk_tokens % kMlaTile == 0 && tune.mla_decode_lds > 0 && lds_shared <= 160 * 1024;
   const int parts = (groups % 2 == 0) ? 4 : 8;            // output-column parts per head group
   const int wg_y = shared_tile ? groups / (8 / parts) : 0;  // workgroups per span (shared-tile kernel)
-  // Multiples of 128 heads: four wavefronts with 32 heads each (mla_decode_lds = 2 keeps the kernel above)
+  // Multiples of 128 heads: four wavefronts with 32 heads each (mla_decode_lds = 2 keeps the kernel above).  A segment
+  // costs that kernel some 12 us before and after its tiles (147 KB of queries into one CU, up to 256 KB of partial
+  // sums out of it), so where the call cannot hold more than 256 tokens for every CU that takes 128 heads, the kernel
+  // above spreads its heads over four times as many workgroups.  (128 heads, us for the call, this kernel / the one
+  // above: one request of 900 tokens 25.2 / 16.5, 4 of 300-1 000 39.7 / 21.9, 16 of 300-1 200 48.4 / 30.8, 128 of 2-64
+  // 44.6 / 28.0, 128 of 100-400 70.1 / 61.4, 16 of 4 000 70 / 59; from 60 000 tokens 61.1 / 57.1 they are level,
+  // 122 000 tokens 86.4 / 98.0, 64 requests of 512-8 192 151 / 217.)
   const size_t lds_heads = lds_head + (size_t)4 * kMlaHeadsBuf;
-  const bool heads_tile = mla_heads_kernel_shape(Hq, chunk_tokens) && tune.mla_decode_lds == 1 && lds_heads <= 160 * 1024;
+  const bool few_tokens = shared_tile && (int64_t)R * max_kv_len * (Hq / 128) <= (int64_t)256 * device_cu_count();
+  const bool heads_tile =
+      mla_heads_kernel_shape(Hq, chunk_tokens) && tune.mla_decode_lds == 1 && lds_heads <= 160 * 1024 && !few_tokens;
   int grid_x = mla_grid_size(groups, tune);
   if (heads_tile) {
     grid_x = mla_heads_grid_size(Hq, tune);

@@ -97,6 +97,33 @@ def test_mla_decode_128_heads_scores_that_keep_growing(mi, dev, dtype, choice):
             _check(mi, dev, q, cache, lens, bt, scale=0.07)
 
 
+@pytest.mark.parametrize("Hq,bound", [(128, 0), (128, 1), (256, 0), (256, 1)])
+def test_mla_decode_128_heads_on_both_sides_of_the_token_bound(mi, dev, Hq, bound):
+    """Requests times the bound of their lengths picks the kernel of eight wavefronts (few tokens) or that of four: the
+    results of both, on either side of the line, also where scores grow along the sequence."""
+    lens = [0, 1, 31, 33, 63, 64, 65, 257, 700, 1500]
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    line = 256 * cus // (len(lens) * (Hq // 128))       # the largest bound that counts as few tokens
+    for grow in (False, True):
+        q, cache, lens_t, bt = _case(mi, dev, lens, Hq, 64, seed=31)
+        if grow:
+            cache = cache.float()
+            for r in range(lens_t.numel()):
+                pos = torch.arange(int(lens_t[r]))
+                cache[bt[r, pos // 64].long(), pos % 64, DV:] *= (1.0 + 0.05 * pos)[:, None]
+            cache = cache.bfloat16()
+        assert line >= max(lens)
+        out = mi.ops.paged_mla_decode_attention(q.to(dev), cache.to(dev), lens_t.to(dev), bt.to(dev), softmax_scale=0.07,
+                                                max_kv_len=line + bound)
+        with mi.ops.tuning(mla_decode_lds=2):
+            eight = mi.ops.paged_mla_decode_attention(q.to(dev), cache.to(dev), lens_t.to(dev), bt.to(dev), softmax_scale=0.07)
+        torch.cuda.synchronize()
+        ref = oa.mla_decode_attention(q.squeeze(1), cache, lens_t, bt, 0.07, DV)
+        err = (out.float().cpu().squeeze(1) - ref).abs()
+        assert (err <= 2e-2 + 2e-2 * ref.abs()).all(), f"max err {err.max().item():.4e}"
+        assert torch.equal(out, eight) == (bound == 0)
+
+
 def test_mla_decode_many_requests_fall_back_to_streaming(mi, dev):
     """More requests than the LDS-tile kernel has room for next to its tiles: the call still succeeds."""
     g = torch.Generator().manual_seed(12)
