@@ -24,6 +24,7 @@ bool mi_profile_is_on();
 
 namespace mi {
 int decode_grid_size(int Hq, int Hkv, const MiTuning& tune);
+int device_cu_count();   // of the calling thread's device
 // What a fused decode step hands the streaming kernel beside the attention arguments (see mi_decode_step_attention).
 struct FusedStepArgs {
   int64_t q_stride_group;  // elements between the query-head groups of two KV heads (heads of a group are contiguous)

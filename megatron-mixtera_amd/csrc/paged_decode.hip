@@ -1884,7 +1884,7 @@ static int pick_waves_per_block(int waves, const MiTuning& tune) {
   return 1;
 }
 
-static int device_cu_count() {
+int device_cu_count() {
   static std::atomic<int> cus[64];  // zero-initialised; callers on several host threads may race to fill a slot
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;

@@ -9,7 +9,10 @@
 // wavefronts share a CU by twos (74 KB of LDS each) and cover each other's start and end where walks are short
 // (prefill_woven_waves).  At head_dim 64 the accumulators are half as many and the exponentials per product twice: there
 // workgroups of 4 wavefronts, three per CU (168 registers, 41 KB of LDS each), put a third wavefront on every SIMD to fill
-// the vector pipe (11 ragged prompts of 164-2 911 tokens, fp16: 148 us, the two-phase kernel 170).  There are no
+// the vector pipe (11 ragged prompts of 164-2 911 tokens, fp16: 148 us, the two-phase kernel 170).  Over an fp8 cache 168
+// registers are some ten too few; a call of no more than three workgroups per CU, where the third wavefront would come for a
+// moment only, takes the build for two per CU instead (bf16, 32/8 heads: one prompt of 1 000 tokens 38.4 -> 36.9 us, of 2 200 64.5
+// -> 57.9, of 3 000 83.4 -> 78.0, two of 1 500 60.9 -> 55.0; but one of 4 000, 1 000 workgroups, 113 -> 120).  There are no
 // matrix / vector phases and no per-phase barriers: every wavefront runs the whole tile pipeline in ONE stream, cut
 // into 32-key steps and software-pipelined so that three independent chains are always open --
 //     products    S^T(step s+1) = K Q^T          and  O^T += V^T P^T(step s-1)     (matrix cores)
@@ -32,7 +35,10 @@
 // converted exactly (four instructions per eight; e4m3 is a subset of both 16-bit types) and their scale multiplies the
 // softmax scale of the tile instead.  Value bytes are converted as cheaply, times the power of two of their scale; the rest of
 // the scale, 1 to 2, goes into the exponent of the tile's probabilities and out of their sum, which is kept per tile (values
-// multiplied by their scale and rounded took 48 more vector instructions per tile; 2 x 8 000 tokens 1 081 -> 1 066 us).
+// multiplied by their scale and rounded took 48 more vector instructions per tile; 2 x 8 000 tokens 1 081 -> 1 066 us).  At
+// head_dim 64, half the values for as many probabilities and no registers for it, values are multiplied and rounded (the factor
+// there: 12 prompts of 1 000 tokens 145 -> 148 us, two of 175-2 806 109 -> 111).  After a barrier the next keys set out before the
+// second half of the values is converted (three prompts of 4 000, width 128, 617 -> 607).
 //
 // Softmax: exponentials are taken against a per-row reference that moves only when a probability leaves a window (a
 // factor of 2^31 with bf16 operands, 2^8 with fp16); the row sums come out of the matrix cores (an all-ones A fragment).
@@ -68,9 +74,10 @@ template <int HD> constexpr bool wv_piece_division_ok() {
 }
 static_assert(wv_piece_division_ok<128>() && wv_piece_division_ok<64>(), "piece -> (row, column)");
 
-template <int HD, bool FP8, bool SPLIT, bool F16, int WAVES>
-__global__ __launch_bounds__(64 * WAVES, HD == 64 ? 3 : 2) void paged_prefill_woven_kernel(PrefillParams p) {
+template <int HD, bool FP8, bool SPLIT, bool F16, int WAVES, int PER_SIMD>
+__global__ __launch_bounds__(64 * WAVES, PER_SIMD) void paged_prefill_woven_kernel(PrefillParams p) {
   constexpr int KS = HD / 32, DV = HD / 16, NQ = 2, THREADS = 64 * WAVES;
+  constexpr bool FACTOR = FP8 && HD == 128;   // the value scales' mantissas go into the probabilities (see above)
   constexpr int PITCH = wv_pitch<HD>(), PIECES = PITCH / 16, LOADS = kWvTile * PIECES / 64, BUF = LOADS * 1024;
   constexpr int NKF = 2 * KS, NVF = DV;  // key and value fragments of a 32-key slot
   constexpr int ESZ = FP8 ? 1 : 2;       // bytes per cache element
@@ -229,7 +236,7 @@ __global__ __launch_bounds__(64 * WAVES, HD == 64 ? 3 : 2) void paged_prefill_wo
 
   float neg_run[NQ];  // the reference: a probability is 2^(score * scale + neg_run); kNoReference until a row has one
   f32x4_t acc[NQ][DV], accl[NQ];
-  float row_sum[NQ];  // fp8 only
+  float row_sum[NQ];  // FACTOR only
 #pragma unroll
   for (int nt = 0; nt < NQ; ++nt) {
     neg_run[nt] = kNoReference;
@@ -304,7 +311,15 @@ __global__ __launch_bounds__(64 * WAVES, HD == 64 ? 3 : 2) void paged_prefill_wo
       const uint2 lo = fp8x4_to_16x4<F16>(kraw[i].x), hi = fp8x4_to_16x4<F16>(kraw[i].y);
       *reinterpret_cast<uint4*>(buf + f_lds + i * RPP8 * PITCH) = make_uint4(lo.x, lo.y, hi.x, hi.y);
     };
-    auto store_v_fp8 = [&](uint8_t* buf, int i, float vscale) {   // (times the power of two of their scale)
+    auto store_v_fp8 = [&](uint8_t* buf, int i, float vscale) {   // (FACTOR: times the power of two of their scale)
+      if constexpr (!FACTOR) {
+        const f32x2_t a = fp8x2_lo_to_f32(vraw[i].x), b = fp8x2_hi_to_f32(vraw[i].x);
+        const f32x2_t c = fp8x2_lo_to_f32(vraw[i].y), d = fp8x2_hi_to_f32(vraw[i].y);
+        *reinterpret_cast<uint4*>(buf + f_lds + i * RPP8 * PITCH) =
+            make_uint4(pack2<F16>(a.x * vscale, a.y * vscale), pack2<F16>(b.x * vscale, b.y * vscale),
+                       pack2<F16>(c.x * vscale, c.y * vscale), pack2<F16>(d.x * vscale, d.y * vscale));
+        return;
+      }
       const float pow2 = __uint_as_float(__float_as_uint(vscale) & 0x7f800000u);
       const uint2 lo = fp8x4_to_16x4<F16>(vraw[i].x, pow2), hi = fp8x4_to_16x4<F16>(vraw[i].y, pow2);
       *reinterpret_cast<uint4*>(buf + f_lds + i * RPP8 * PITCH) = make_uint4(lo.x, lo.y, hi.x, hi.y);
@@ -442,9 +457,9 @@ __global__ __launch_bounds__(64 * WAVES, HD == 64 ? 3 : 2) void paged_prefill_wo
             acc[nt][e][0] *= alpha; acc[nt][e][1] *= alpha; acc[nt][e][2] *= alpha; acc[nt][e][3] *= alpha;
           }
           accl[nt][0] *= alpha; accl[nt][1] *= alpha; accl[nt][2] *= alpha; accl[nt][3] *= alpha;
-          if (FP8) row_sum[nt] *= alpha;
+          if (FACTOR) row_sum[nt] *= alpha;
         }
-        shifted[nt] = FP8 ? neg + fast_log2(factor) : neg;
+        shifted[nt] = FACTOR ? neg + fast_log2(factor) : neg;
       }
 #pragma unroll
       for (int c = 0; c < 8; ++c) exp_chunk(Sx, Px, c, scale, shifted);
@@ -464,10 +479,10 @@ __global__ __launch_bounds__(64 * WAVES, HD == 64 ? 3 : 2) void paged_prefill_wo
       uint4 (&Px)[NQ] = P[1 - H];
       const uint4 (&Pv)[NQ] = P[H];
       const float scale = FP8 ? (H == 0 ? scale_prev : scale_cur) : p.scale_log2;  // of the scores in Sx
-      const float factor = FP8 ? (H == 0 ? factor_prev : factor_cur) : 1.f;
+      const float factor = FACTOR ? (H == 0 ? factor_prev : factor_cur) : 1.f;
       float neg[NQ];
 #pragma unroll
-      for (int nt = 0; nt < NQ; ++nt) neg[nt] = FP8 ? neg_run[nt] + fast_log2(factor) : neg_run[nt];
+      for (int nt = 0; nt < NQ; ++nt) neg[nt] = FACTOR ? neg_run[nt] + fast_log2(factor) : neg_run[nt];
       // fragment n of the slot's stream: NKF key fragments, NVF value fragments, then the next slot's first keys
       auto request = [&](int n) {
         if (n < NKF) fr[n % RING] = read_k(ka, H, n);
@@ -546,8 +561,8 @@ __global__ __launch_bounds__(64 * WAVES, HD == 64 ? 3 : 2) void paged_prefill_wo
         MI_SB();
       }
       // (fp8: the sums of one value tile, whose factor comes out of them in end_of_sums)
-      accl[0] = mfma_16x16x32<F16>(ones, Pv[0], FP8 && H == 0 ? zero4 : accl[0]);
-      accl[1] = mfma_16x16x32<F16>(ones, Pv[1], FP8 && H == 0 ? zero4 : accl[1]);
+      accl[0] = mfma_16x16x32<F16>(ones, Pv[0], FACTOR && H == 0 ? zero4 : accl[0]);
+      accl[1] = mfma_16x16x32<F16>(ones, Pv[1], FACTOR && H == 0 ? zero4 : accl[1]);
       MI_SB();
       if (__builtin_amdgcn_ballot_w64(leaves_window(Px))) move_reference(Sx, Px, scale, factor);
       MI_SB();
@@ -672,19 +687,18 @@ __global__ __launch_bounds__(64 * WAVES, HD == 64 ? 3 : 2) void paged_prefill_wo
              else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
              __builtin_amdgcn_s_barrier();
              first_values();
-             if constexpr (FP8) {
-#pragma unroll
-               for (int i = NP8 / 2; i < NP8; ++i) store_v_fp8(vst, i, vscale);
-             }
              if constexpr (FP8) pc_next = __builtin_amdgcn_readfirstlane(pc_v);
              else bt_arrived(pc_next);
              const int64_t off = tile_off(cur, pc_next);
              const uint32_t nrec = tile_nrec(cur);
              if constexpr (FP8) {
                scale_next = tile_scale(uniform_float(ks_v));  // (of tile j+1)
+               const float vscale_last = vscale;
                vscale = value_scale(vs_v);
                scales_request(pc_next);
                fetch_fp8(kbase, off, nrec, kraw);
+#pragma unroll
+               for (int i = NP8 / 2; i < NP8; ++i) store_v_fp8(vst, i, vscale_last);
                fetch_fp8(vbase, off_prev, nrec_prev, vraw);
              } else {
                rs_k = tile_rsrc(kbase, off, nrec);
@@ -711,7 +725,7 @@ __global__ __launch_bounds__(64 * WAVES, HD == 64 ? 3 : 2) void paged_prefill_wo
              }
            });
       if constexpr (FP8) {
-        end_of_sums(factor_prev);   // (the values of tile j-1)
+        if (FACTOR) end_of_sums(factor_prev);   // (the values of tile j-1)
         scale_prev = scale_cur;
         scale_cur = scale_next;
         factor_prev = factor_cur;
@@ -726,7 +740,7 @@ __global__ __launch_bounds__(64 * WAVES, HD == 64 ? 3 : 2) void paged_prefill_wo
     // ---- drain: the last two steps' values (tile ntl - 1), the second half when it has landed; S[1] is masked already ----
     {
       const uint8_t* va = v_lane + (BUF - even);
-      if (FP8) accl[0] = accl[1] = zero4;
+      if (FACTOR) accl[0] = accl[1] = zero4;
       auto values = [&](int half, const uint4 (&Pv)[NQ]) {
 #pragma unroll
         for (int e = 0; e < DV; ++e) {
@@ -740,14 +754,14 @@ __global__ __launch_bounds__(64 * WAVES, HD == 64 ? 3 : 2) void paged_prefill_wo
       values(0, P[0]);
       float neg_last[NQ];
 #pragma unroll
-      for (int nt = 0; nt < NQ; ++nt) neg_last[nt] = FP8 ? neg_run[nt] + fast_log2(factor_prev) : neg_run[nt];
+      for (int nt = 0; nt < NQ; ++nt) neg_last[nt] = FACTOR ? neg_run[nt] + fast_log2(factor_prev) : neg_run[nt];
 #pragma unroll
       for (int c = 0; c < 8; ++c) exp_chunk(S[1], P[1], c, FP8 ? scale_prev : p.scale_log2, neg_last);
       if (__builtin_amdgcn_ballot_w64(leaves_window(P[1]))) move_reference(S[1], P[1], FP8 ? scale_prev : p.scale_log2, factor_prev);
       asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
       values(1, P[1]);
-      if (FP8) end_of_sums(factor_prev);
+      if (FACTOR) end_of_sums(factor_prev);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no direct load may still be on its way into this workgroup's LDS
 #undef MI_SB
@@ -756,7 +770,7 @@ __global__ __launch_bounds__(64 * WAVES, HD == 64 ? 3 : 2) void paged_prefill_wo
   // ---- epilogue: acc[nt][e][i] is output element d = 16e + 4g + i of row (nt, m16) --------------
 #pragma unroll
   for (int nt = 0; nt < NQ; ++nt) {
-    const float l_tot = FP8 ? row_sum[nt] : accl[nt][0];
+    const float l_tot = FACTOR ? row_sum[nt] : accl[nt][0];
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
     const int n = 16 * nt + m16;
     const int qi = (n * g_magic) >> 16, u = n - qi * G;  // n / G, n % G
@@ -783,20 +797,21 @@ __global__ __launch_bounds__(64 * WAVES, HD == 64 ? 3 : 2) void paged_prefill_wo
 
 void launch_prefill_woven(const PrefillParams& p, dim3 grid, int head_dim, bool fp8, bool f16, int waves, hipStream_t st) {
   const bool split = grid.y > 1;
-#define MI_WV_LAUNCH(HD_, FP8_, W_)                                                                                  \
+#define MI_WV_LAUNCH(HD_, FP8_, W_, PS_)                                                                                 \
   do {                                                                                                              \
     const dim3 block(64 * W_);                                                                                      \
-    if (split && f16) hipLaunchKernelGGL((paged_prefill_woven_kernel<HD_, FP8_, true, true, W_>), grid, block, 0, st, p); \
-    else if (split) hipLaunchKernelGGL((paged_prefill_woven_kernel<HD_, FP8_, true, false, W_>), grid, block, 0, st, p); \
-    else if (f16) hipLaunchKernelGGL((paged_prefill_woven_kernel<HD_, FP8_, false, true, W_>), grid, block, 0, st, p); \
-    else hipLaunchKernelGGL((paged_prefill_woven_kernel<HD_, FP8_, false, false, W_>), grid, block, 0, st, p);      \
+    if (split && f16) hipLaunchKernelGGL((paged_prefill_woven_kernel<HD_, FP8_, true, true, W_, PS_>), grid, block, 0, st, p); \
+    else if (split) hipLaunchKernelGGL((paged_prefill_woven_kernel<HD_, FP8_, true, false, W_, PS_>), grid, block, 0, st, p); \
+    else if (f16) hipLaunchKernelGGL((paged_prefill_woven_kernel<HD_, FP8_, false, true, W_, PS_>), grid, block, 0, st, p); \
+    else hipLaunchKernelGGL((paged_prefill_woven_kernel<HD_, FP8_, false, false, W_, PS_>), grid, block, 0, st, p);      \
   } while (0)
-  if (head_dim == 64 && fp8) MI_WV_LAUNCH(64, true, 4);
-  else if (head_dim == 64) MI_WV_LAUNCH(64, false, 4);
-  else if (fp8 && waves == 4) MI_WV_LAUNCH(128, true, 4);
-  else if (fp8) MI_WV_LAUNCH(128, true, 8);
-  else if (waves == 4) MI_WV_LAUNCH(128, false, 4);
-  else MI_WV_LAUNCH(128, false, 8);
+  if (head_dim == 64 && fp8 && (int64_t)grid.x * grid.y <= 3 * device_cu_count()) MI_WV_LAUNCH(64, true, 4, 2);
+  else if (head_dim == 64 && fp8) MI_WV_LAUNCH(64, true, 4, 3);
+  else if (head_dim == 64) MI_WV_LAUNCH(64, false, 4, 3);
+  else if (fp8 && waves == 4) MI_WV_LAUNCH(128, true, 4, 2);
+  else if (fp8) MI_WV_LAUNCH(128, true, 8, 2);
+  else if (waves == 4) MI_WV_LAUNCH(128, false, 4, 2);
+  else MI_WV_LAUNCH(128, false, 8, 2);
 #undef MI_WV_LAUNCH
 }
 

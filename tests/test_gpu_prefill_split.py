@@ -82,3 +82,37 @@ def test_four_wavefronts_give_what_eight_do(mi, dev, Hq, Hkv, dtype, fp8):
     bound = 2e-2 + 2e-2 * ref.abs()
     for o in out:
         assert ((o.float().cpu() - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("splits", [-1, 3])
+def test_a_call_of_few_workgroups_gives_what_a_large_one_does(mi, dev, dtype, splits):
+    """Prompts of width 64 over an fp8 cache: a call of at most three workgroups per CU takes another build of the kernel than
+    a larger one.  The same requests alone and as the first of many: the same bits, and those of the reference."""
+    lens, chunk, d, Hq, Hkv = [1, 33, 64, 65, 190, 257], 64, 64, 32, 8
+    gen = torch.Generator().manual_seed(5)
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    copies = 2 + 3 * cus // (Hkv * sum(-(-n // 32) for n in lens))   # (a block is 128 rows, 32 tokens here)
+    kv_lens = torch.tensor(lens, dtype=torch.int32)
+    bt, N = mi.synthetic.build_block_table(kv_lens, chunk, gen)
+    T = sum(lens)
+    q = torch.randn(T, Hq, d, generator=gen).to(dtype).to(dev)
+    src = [(torch.randn(N, chunk, Hkv, d, generator=gen) * (0.05 + 4 * torch.rand(N, 1, 1, 1, generator=gen))).to(dtype).to(dev) for _ in range(2)]
+    pools = [torch.empty(x.shape, dtype=torch.uint8, device=dev) for x in src]
+    scales = [torch.empty(N, Hkv, dtype=torch.float32, device=dev) for _ in range(2)]
+    for x, pool, scale in zip(src, pools, scales):
+        mi.ops.quantize_chunks_fp8(x, pool, scale)
+    out = []
+    for n in (1, copies):
+        kl = kv_lens.repeat(n)
+        cu_q = torch.zeros(kl.numel() + 1, dtype=torch.int32)
+        cu_q[1:] = torch.cumsum(kl, 0)
+        with mi.ops.tuning(prefill_kv_split=splits):
+            out.append(mi.ops.paged_prefill_attention(q.repeat(n, 1, 1), *pools, cu_q.to(dev), kl.to(dev), bt.repeat(n, 1).to(dev),
+                                                      max_kv_len=int(kl.max()), one_row_requests=False, k_scales=scales[0],
+                                                      v_scales=scales[1]))
+    assert torch.equal(out[0], out[1][:T])
+    cu_q = torch.zeros(len(lens) + 1, dtype=torch.int32)
+    cu_q[1:] = torch.cumsum(kv_lens, 0)
+    ref = oa.paged_varlen_attention(q.cpu(), pools[0].cpu(), pools[1].cpu(), cu_q, kv_lens, bt, k_scales=scales[0].cpu(), v_scales=scales[1].cpu())
+    assert ((out[0].float().cpu() - ref).abs() <= 2e-2 + 2e-2 * ref.abs()).all()
