@@ -9,15 +9,15 @@
 // wavefronts share a CU by twos (74 KB of LDS each) and cover each other's start and end where walks are short
 // (prefill_woven_waves).  At head_dim 64 the accumulators are half as many and the exponentials per product twice: there
 // workgroups of 4 wavefronts, three per CU (168 registers, 41 KB of LDS each), put a third wavefront on every SIMD to fill
-// the vector pipe (11 ragged prompts of 164-2 911 tokens, fp16: 148 us, the two-phase kernel 170).  Over an fp8 cache 168
-// registers are some ten too few; a call of no more than three workgroups per CU, where the third wavefront would come for a
-// moment only, takes the build for two per CU instead (bf16, 32/8 heads: one prompt of 1 000 tokens 38.4 -> 36.9 us, of 2 200 64.5
-// -> 57.9, of 3 000 83.4 -> 78.0, two of 1 500 60.9 -> 55.0; but one of 4 000, 1 000 workgroups, 113 -> 120).  There are no
+// the vector pipe (11 ragged prompts of 164-2 911 tokens, fp16: 148 us, the two-phase kernel 170).  Over an fp8 cache a
+// call of no more than three workgroups per CU, where the third wavefront would come for a moment only, takes a build for
+// two per CU and with more fragments ahead (bf16, 32/8 heads: two prompts of 1 100 tokens 48.0 -> 46.7 us, of 1 500 57 -> 54.5, one
+// of 2 600 67.3 -> 64.5, of 1 000 level; but one of 4 000, 1 000 workgroups, 112 -> 120).  There are no
 // matrix / vector phases and no per-phase barriers: every wavefront runs the whole tile pipeline in ONE stream, cut
 // into 32-key steps and software-pipelined so that three independent chains are always open --
 //     products    S^T(step s+1) = K Q^T          and  O^T += V^T P^T(step s-1)     (matrix cores)
 //     vector ALU  P(step s) = exp2(S(step s) * scale - reference)  and the mask of S(step s+1)
-//     LDS         the fragments of the products three fragments ahead
+//     LDS         the fragments of the products, one or three fragments ahead
 // -- and the source orders them product pair / fragment read / a few vector instructions, pinned by scheduling
 // barriers.  Whatever one wavefront of a SIMD cannot issue (a product waiting for the matrix core, a wait for LDS),
 // the SIMD's other wavefront fills with its own stream; nothing but the one barrier per tile keeps them in step.
@@ -56,8 +56,11 @@
 namespace mi {
 
 constexpr int kWvTile = 64;                      // keys per staged tile
-constexpr int kWvAhead = 3;                      // fragments requested ahead of their products
-constexpr int kWvRing = 4;                       // fragment registers: fragment n lives in slot n % kWvRing
+// Fragment registers: fragment n lives in slot n % ring and is requested ring - 1 fragments ahead of its products.  Width 64 over
+// an fp8 cache at three workgroups per CU: two fragments less are the registers that it lacks, and the SIMD's other two wavefronts
+// cover the wait (with four it spilled nine; 12 prompts of 1 000 tokens 146 -> 136 us, 11 of 33-3 001 176 -> 167, 3 x 6 000 601 -> 568;
+// over a 16-bit cache, which spills nothing, level).
+template <int HD, bool FP8, int PER_SIMD> constexpr int wv_ring() { return FP8 && HD == 64 && PER_SIMD == 3 ? 2 : 4; }
 // LDS bytes per staged row: the row and 32 bytes of padding (288 or 160: conflict-free fragment reads)
 template <int HD> constexpr int wv_pitch() { return 2 * HD + 32; }
 // A row's reference is moved where a probability leaves the window, to where the row's largest one is 2^-headroom: with bf16
@@ -82,7 +85,7 @@ __global__ __launch_bounds__(64 * WAVES, PER_SIMD) void paged_prefill_woven_kern
   constexpr int NKF = 2 * KS, NVF = DV;  // key and value fragments of a 32-key slot
   constexpr int ESZ = FP8 ? 1 : 2;       // bytes per cache element
   static_assert(HD == 128 || HD == 64, "head widths");
-  static_assert(kWvAhead < kWvRing && kWvAhead <= NKF && (NKF + NVF) % kWvRing == 0, "next slot's key fragments are requested after the tile's barrier");
+  static_assert(wv_ring<HD, FP8, PER_SIMD>() - 1 <= NKF && (NKF + NVF) % wv_ring<HD, FP8, PER_SIMD>() == 0, "next slot's key fragments are requested after the tile's barrier");
   // Key tile t lives in Ks[t & 1], value tile t in Vs[t & 1], whose halves are filled one barrier apart (see `iteration`).
   constexpr int HALF = BUF / 2;  // 32 rows of a tile
   __shared__ __attribute__((aligned(16))) uint8_t Ks[2][BUF];
@@ -397,7 +400,7 @@ __global__ __launch_bounds__(64 * WAVES, PER_SIMD) void paged_prefill_woven_kern
     // S[x]: scores of the even (x = 0) / odd (x = 1) 32-key steps, P[x]: their probabilities as the B operand
     f32x4_t S[2][NQ][2];
     uint4 P[2][NQ];
-    constexpr int AHEAD = kWvAhead, RING = kWvRing;
+    constexpr int RING = wv_ring<HD, FP8, PER_SIMD>(), AHEAD = RING - 1;
     uint4 fr[RING];  // fragments in flight: fragment n of the stream lives in fr[n % RING]
 #pragma unroll
     for (int nt = 0; nt < NQ; ++nt) {
