@@ -439,16 +439,16 @@ namespace mi {
 // -> `angles` [T][2][D] in the tensors' 16-bit type (the sine with the sign of its partner term), for the prefill tile
 // kernel, which norms and rotates the queries as it loads them.
 //
-// Bound by memory: per token the keys and values in and out and 4 D bytes of table.  A workgroup takes four tokens so
-// that every lane has a piece of a head vector (one token's eight key heads fill a quarter of it) and evaluates each
-// angle of its tokens once for all heads; pieces are requested before the positions' chain of trips.  Leaving the
-// queries to the tile kernel saves reading and writing them here: 12 348 tokens of 32 / 8 heads of 64.
+// Bound by memory for long prompts: per token the keys and values in and out and 4 D bytes of table.  A workgroup takes
+// `tokens` of them (at most kKeyTokens) and evaluates each angle of its tokens once for all heads; pieces are requested
+// before the positions' chain of trips.  Leaving the queries to the tile kernel saves reading and writing them here:
+// 12 348 tokens of 32 / 8 heads of 64.
 constexpr int kKeyTokens = 4;
 template <int D, bool F16>
-__global__ __launch_bounds__(256) void qkv_key_append_kernel(NormRopeParams p, uint16_t* __restrict__ angles) {
+__global__ __launch_bounds__(256) void qkv_key_append_kernel(NormRopeParams p, uint16_t* __restrict__ angles, int tokens) {
   constexpr int LPV = D / 8, VPB = 256 / LPV;  // lanes per head vector, head vectors per pass
   __shared__ __align__(16) float cs[kKeyTokens][2][D];
-  const int t0 = blockIdx.x * kKeyTokens, nt = min(kKeyTokens, p.T - t0), nvec = nt * p.Hkv;
+  const int t0 = blockIdx.x * tokens, nt = min(tokens, p.T - t0), nvec = nt * p.Hkv;
   const int slot = threadIdx.x / LPV, li = threadIdx.x % LPV, e0 = 8 * li;
   struct Piece {
     uint4 k, v;
@@ -728,12 +728,17 @@ extern "C" int mi_qkv_key_append(
   p.kc = (uint16_t*)k_cache; p.vc = (uint16_t*)v_cache; p.chunk_elems = kv_stride_chunk; p.tok_elems = kv_stride_tok;
   p.tok_chunk = token_to_chunk_idx; p.tok_local = token_to_local_pos;
   p.T = T; p.Hkv = Hkv; p.norm = norm_kind; p.interleaved = rotary_interleaved; p.eps = eps; p.mscale = mscale;
-  const dim3 grid((T + kKeyTokens - 1) / kKeyTokens);
+  // Two tokens where their key heads fill the workgroup's lanes, in one pass, else four.  Short prompts are bound by the chain
+  // of trips and have fewer workgroups than the chip takes at once (the step of one prompt of 500 tokens, 32 / 8 heads of 128,
+  // 25.3 -> 24.2 us, four of 300 32.4 -> 30.6; 8 x 1 000 and 6 x 4 000 level); with lanes idle two are level at best (8 heads of 64: 4 x 800
+  // 37.7 / 38.8), and one token works its angles out on half of the lanes (4 x 500 40.8, 40.0 with two, 41.8).
+  const int tokens = 2 * Hkv * (head_dim / 8) >= 256 ? 2 : kKeyTokens;
+  const dim3 grid((T + tokens - 1) / tokens);
   hipStream_t st = (hipStream_t)stream;
   const bool f16 = dtype == MI_DTYPE_FP16;
-  if (head_dim == 128 && f16) hipLaunchKernelGGL((qkv_key_append_kernel<128, true>), grid, dim3(256), 0, st, p, (uint16_t*)cos_sin);
-  else if (head_dim == 128) hipLaunchKernelGGL((qkv_key_append_kernel<128, false>), grid, dim3(256), 0, st, p, (uint16_t*)cos_sin);
-  else if (f16) hipLaunchKernelGGL((qkv_key_append_kernel<64, true>), grid, dim3(256), 0, st, p, (uint16_t*)cos_sin);
-  else hipLaunchKernelGGL((qkv_key_append_kernel<64, false>), grid, dim3(256), 0, st, p, (uint16_t*)cos_sin);
+  if (head_dim == 128 && f16) hipLaunchKernelGGL((qkv_key_append_kernel<128, true>), grid, dim3(256), 0, st, p, (uint16_t*)cos_sin, tokens);
+  else if (head_dim == 128) hipLaunchKernelGGL((qkv_key_append_kernel<128, false>), grid, dim3(256), 0, st, p, (uint16_t*)cos_sin, tokens);
+  else if (f16) hipLaunchKernelGGL((qkv_key_append_kernel<64, true>), grid, dim3(256), 0, st, p, (uint16_t*)cos_sin, tokens);
+  else hipLaunchKernelGGL((qkv_key_append_kernel<64, false>), grid, dim3(256), 0, st, p, (uint16_t*)cos_sin, tokens);
   return mi_check_launch("mi_qkv_key_append");
 }

@@ -156,3 +156,22 @@ def test_norm_weights_off_16_bytes_take_the_separate_calls(mi, dev):
                             generator=torch.Generator(device=dev).manual_seed(3), device=dev).bfloat16()
         outs.append(core.forward_mixed_qkv(mixed, hq, ctx)[:70].float())
     assert ((outs[0] - outs[1]).norm() / outs[0].norm()).item() < 3e-3
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d,hkv", [(128, 7), (128, 8), (128, 17), (64, 15), (64, 16)])
+@pytest.mark.parametrize("T", [1, 2, 3, 4, 5, 9])
+def test_keys_do_not_depend_on_the_tokens_beside_them(mi, dev, dtype, d, hkv, T):
+    """A workgroup takes two tokens or four, by the heads: either side of that line, whole and partial workgroups give the
+    bits of each token appended by itself."""
+    (mixed, pos, chunk, local, *_), (_, kw), caches, longest = _batch(mi, dev, (T,), hkv, hkv, d, dtype, 0, d + T)
+    emb = mi.synthetic.rotary_angle_table(longest, d, base=10000.0).to(dev)
+    common = dict(num_query_heads=hkv, num_kv_heads=hkv, norm="rms", k_weight=kw, rotary_emb=emb)
+    one, key = [c.clone() for c in caches], torch.empty(T, 1, hkv, d, dtype=dtype, device=dev)
+    slots = lambda a, b: dict(token_to_chunk_idx=chunk[a:b], token_to_local_pos=local[a:b], q_positions=pos[a:b], k_positions=pos[a:b])
+    cos_sin = mi.ops.qkv_key_append(mixed, k_cache=caches[0], v_cache=caches[1], **common, **slots(0, T))
+    alone = [mi.ops.qkv_key_append(mixed[i:i + 1], k_cache=one[0], v_cache=one[1], **common, **slots(i, i + 1)) for i in range(T)]
+    mi.ops.qkv_key_append(mixed, key_out=key, q_positions=pos, k_positions=pos, **common)
+    assert torch.equal(caches[0], one[0]) and torch.equal(caches[1], one[1])
+    assert torch.equal(cos_sin, torch.cat(alone))
+    assert torch.equal(key.squeeze(1), caches[0][chunk, local])
