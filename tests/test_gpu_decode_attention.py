@@ -285,7 +285,7 @@ def test_rejects_bad_arguments(mi, dev):
 @pytest.mark.parametrize("Hq,Hkv,d,chunk", [(8, 8, 64, 32), (32, 8, 128, 64), (16, 1, 128, 256), (20, 1, 64, 256), (24, 8, 128, 128)])
 @pytest.mark.parametrize("fp8", [False, True])
 def test_short_requests_by_one_workgroup_per_head(mi, dev, Hq, Hkv, d, chunk, fp8, dtype):
-    """Tables of up to 256 tokens at width 128: one workgroup per request and KV head, against the checker and (16-bit caches)
+    """Tables of up to 256 tokens at width 128: one workgroup per request and KV head, against the oracle and (16-bit caches)
     against the stream, which `split_tokens` asks for.  Lengths around the tiles of 32 tokens and the eight wavefronts' shares."""
     lens = torch.tensor([0, 1, 2, 31, 32, 33, 63, 64, 65, 223, 224, 225, 255, 256], dtype=torch.int32)
     cfg = mi.synthetic.DecodeConfig("short", lens.numel(), Hq, Hkv, d, 0, 0, chunk=chunk, seed=Hq + d)
