@@ -1670,7 +1670,8 @@ const uint32_t none = (uint32_t)(kBins + lane);   // (a place of its own for wha
       });
       cut_key = cut;
     }
-    if (cut_key) cut_value = order_key_value(cut_key);
+    // (a key below -inf's is a negative NaN's, to which every float compares false: such a cut keeps everything)
+    if (cut_key > order_key(-INFINITY)) cut_value = order_key_value(cut_key);
     // ---- the kept mass of every wavefront's run ----
     if (!joined) {
       if (by_mass && cuts && listed) {   // the kept members join what lies above the window

@@ -26,6 +26,13 @@ def _logits(R, V, seed, dtype=torch.float32, spread=3.0):
     return (torch.randn(R, V, generator=g) * spread).to(dtype)
 
 
+def _with_negative_nan(x, where):
+    """A copy with NaNs whose sign is set (a conversion may drop a NaN's sign, so the bits are written in the type)."""
+    bits = {torch.float32: -0x400000, torch.bfloat16: -0x40, torch.float16: -0x200}[x.dtype]   # 0xffc00000, 0xffc0, 0xfe00
+    whole = torch.int32 if x.dtype == torch.float32 else torch.int16
+    return x.contiguous().view(whole).masked_fill(where, bits).view(x.dtype)
+
+
 # ----------------------------------------------------------------------------------------------
 # last-token gather
 # ----------------------------------------------------------------------------------------------
@@ -581,3 +588,28 @@ def test_rows_in_the_registers_of_a_workgroup(mi, dev, V, dtype):
         else:
             assert torch.isinf(cut).all()
         _check_draw(xs, cut, u, s)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("V", [17, 1000, 16389, 32768, 50000])
+def test_a_top_k_above_the_count_of_numbers_keeps_them_all(mi, dev, V, dtype):
+    """NaNs with their sign set lie below -inf.  Where the top k reach down to them every number is kept, and the token is that of
+    the plain draw from the numbers, masked tokens (the first among them) never."""
+    x = _logits(5, V, V, dtype)
+    x[:, 0] = float("-inf")
+    negative_nan = torch.zeros(5, V, dtype=torch.bool)
+    negative_nan[0, V // 2] = True
+    negative_nan[1, 1::3] = True
+    negative_nan[2, : V - 12] = True
+    negative_nan[3, V // 2:] = True
+    x[3, : V // 4] = float("-inf")
+    x[4, 1:] = x[4, 0]
+    x[4, V // 3] = 1.0
+    u = torch.rand(5, generator=torch.Generator().manual_seed(V)).to(dev)
+    want, _ = mi.ops.sample_from_logits(x.masked_fill(negative_nan, float("-inf")).to(dev), temperature=0.8, uniform=u)
+    y = _with_negative_nan(x, negative_nan).to(dev)
+    numbers = (~negative_nan).sum(-1)
+    for top_k in (V, V - V // 4, 13):
+        got, _ = mi.ops.sample_from_logits(y, top_k=top_k, temperature=0.8, uniform=u)
+        rows = ((numbers < top_k) | ((x > float("-inf")).sum(-1) <= top_k) & (top_k == V)).to(dev)
+        assert torch.equal(got[rows], want[rows]), top_k
