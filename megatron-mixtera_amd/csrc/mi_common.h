@@ -305,8 +305,9 @@ static __device__ __forceinline__ f32x2_t fp8x2_hi_to_f32(uint32_t w) {
   return __builtin_amdgcn_cvt_pk_f32_fp8((int)w, true);
 }
 // Four e4m3fn bytes -> two packed pairs of the kernel's operand type, times `pow2`, a power of two.  gfx950 converts a pair of OCP
-// fp8 values to a packed pair in one instruction, with the exponent of a float as multiplier; the conversion is exact: e4m3
-// has 3 mantissa bits, and its exponents lie inside bf16's and fp16's.
+// fp8 values to a packed pair in one instruction, with the exponent of a float as multiplier.  The conversion is exact where the
+// products, 2^-9 to 448 times `pow2` with e4m3's 3 mantissa bits, lie inside the type: for fp16 with `pow2` from 2^-15 to 2^7, for
+// bf16 (normal numbers) from 2^-117 to 2^119.  Outside, they round to subnormal numbers or overflow.
 template <bool F16>
 static __device__ __forceinline__ uint2 fp8x4_to_16x4(uint32_t w, float pow2 = 1.0f) {
   if constexpr (F16) {

@@ -314,7 +314,23 @@ __global__ __launch_bounds__(64 * WAVES, PER_SIMD) void paged_prefill_woven_kern
       const uint2 lo = fp8x4_to_16x4<F16>(kraw[i].x), hi = fp8x4_to_16x4<F16>(kraw[i].y);
       *reinterpret_cast<uint4*>(buf + f_lds + i * RPP8 * PITCH) = make_uint4(lo.x, lo.y, hi.x, hi.y);
     };
-    auto store_v_fp8 = [&](uint8_t* buf, int i, float vscale) {   // (FACTOR: times the power of two of their scale)
+    // A value scale as sign, power of two and what is left, its factor, which goes into its tile's probabilities (the exponent) and
+    // out of their sum: from 1 to 2, or, where bytes times the power of two round in fp16 (subnormal numbers, below 2^-15), from
+    // 1/2 to 1, so that this error is no larger than that of value times scale.  A scale of zero counts as 2^-126; NaN and
+    // infinite ones are in the factor, and so in all results over the tile.
+    auto scale_bits = [](float vscale) { return max(__float_as_uint(vscale) & 0x7fffffffu, 0x00800000u); };
+    auto factor_below_one = [](uint32_t bits) { return F16 && bits < (uint32_t)(127 - 15) << 23; };
+    auto value_factor = [&](float vscale) {
+      const uint32_t bits = scale_bits(vscale);
+      if (bits >= 0x7f800000u) return __uint_as_float(0x7fc00000u);
+      return __uint_as_float((bits & 0x007fffffu) | (factor_below_one(bits) ? 0x3f000000u : 0x3f800000u));
+    };
+    auto value_pow2 = [&](float vscale) {
+      const uint32_t bits = scale_bits(vscale);
+      return __uint_as_float((bits & 0x7f800000u) + (factor_below_one(bits) ? 0x00800000u : 0u));
+    };
+    auto value_sign = [](float vscale) { return (uint32_t)(__float_as_int(vscale) >> 31) & 0x80808080u; };
+    auto store_v_fp8 = [&](uint8_t* buf, int i, float vscale) {   // (FACTOR: times the sign and the power of two of their scale)
       if constexpr (!FACTOR) {
         const f32x2_t a = fp8x2_lo_to_f32(vraw[i].x), b = fp8x2_hi_to_f32(vraw[i].x);
         const f32x2_t c = fp8x2_lo_to_f32(vraw[i].y), d = fp8x2_hi_to_f32(vraw[i].y);
@@ -323,12 +339,11 @@ __global__ __launch_bounds__(64 * WAVES, PER_SIMD) void paged_prefill_woven_kern
                        pack2<F16>(c.x * vscale, c.y * vscale), pack2<F16>(d.x * vscale, d.y * vscale));
         return;
       }
-      const float pow2 = __uint_as_float(__float_as_uint(vscale) & 0x7f800000u);
-      const uint2 lo = fp8x4_to_16x4<F16>(vraw[i].x, pow2), hi = fp8x4_to_16x4<F16>(vraw[i].y, pow2);
+      const float pow2 = value_pow2(vscale);
+      const uint32_t sign = value_sign(vscale);
+      const uint2 lo = fp8x4_to_16x4<F16>(vraw[i].x ^ sign, pow2), hi = fp8x4_to_16x4<F16>(vraw[i].y ^ sign, pow2);
       *reinterpret_cast<uint4*>(buf + f_lds + i * RPP8 * PITCH) = make_uint4(lo.x, lo.y, hi.x, hi.y);
     };
-    // what is left of a value scale, from 1 to 2: it goes into its tile's probabilities (the exponent), and out of their sum
-    auto value_factor = [](float vscale) { return __uint_as_float((__float_as_uint(vscale) & 0x007fffffu) | 0x3f800000u); };
     // descriptor of a tile: its rows up to the request's last key (reads beyond return zeros)
     auto tile_rsrc = [&](uint64_t base, int64_t off, uint32_t nrec) {
       const uint64_t a = base + (uint64_t)off;
@@ -390,7 +405,6 @@ __global__ __launch_bounds__(64 * WAVES, PER_SIMD) void paged_prefill_woven_kern
     auto tile_scale = [&](float ks) { return FP8 ? fmaxf(ks * p.scale_log2, 1.17549435e-38f) : p.scale_log2; };
     float scale_prev = p.scale_log2, scale_cur = p.scale_log2, scale_next = p.scale_log2, vscale = 1.f;
     float factor_prev = 1.f, factor_cur = 1.f;   // fp8: value_factor of the tiles whose scales are scale_prev and scale_cur
-    auto value_scale = [&](float vs) { return fmaxf(uniform_float(vs), 1.17549435e-38f); };
     const uint4 ones = make_uint4(ones2<F16>(), ones2<F16>(), ones2<F16>(), ones2<F16>());
     const f32x4_t zero4 = {0.f, 0.f, 0.f, 0.f};
     // per-lane starts of the fragment reads inside a tile buffer
@@ -587,7 +601,7 @@ __global__ __launch_bounds__(64 * WAVES, PER_SIMD) void paged_prefill_woven_kern
         scales_request(pc);
         if (i == 0) {
           scale_prev = scale_cur = tile_scale(uniform_float(ks_v));
-          vscale = value_scale(vs_v);
+          vscale = uniform_float(vs_v);
           factor_prev = factor_cur = value_factor(vscale);
         }
       }
@@ -697,7 +711,7 @@ __global__ __launch_bounds__(64 * WAVES, PER_SIMD) void paged_prefill_woven_kern
              if constexpr (FP8) {
                scale_next = tile_scale(uniform_float(ks_v));  // (of tile j+1)
                const float vscale_last = vscale;
-               vscale = value_scale(vs_v);
+               vscale = uniform_float(vs_v);
                scales_request(pc_next);
                fetch_fp8(kbase, off, nrec, kraw);
 #pragma unroll
