@@ -78,8 +78,8 @@ typedef struct MiTuning {
   int32_t mla_decode_lds;         /* multi-latent decode: 0 = default (latent tiles shared through LDS when the chunk
                                      size is a multiple of 64 and the call has at most 768 requests; with a multiple
                                      of 128 query heads and a chunk size that is a multiple of 32, by the kernel of
-                                     four wavefronts with 32 heads each, unless max_kv_len shows that the call
-                                     holds few tokens), 2 = the eight-wavefront LDS kernel at
+                                     four wavefronts with 32 heads each, unless max_kv_len (above 0) shows that the
+                                     call holds few tokens), 2 = the eight-wavefront LDS kernel at
                                      every head count, -1 = one streaming wavefront per 16-head group always */
   int32_t reserved[5];            /* must be 0 */
 } MiTuning;
@@ -315,6 +315,8 @@ int mi_paged_decode_attention_noalloc(const void* q, int64_t q_stride_tok, int64
  *   out[r,h] = softmax(q[r,h] . KV_r[:len_r, :576]^T * softmax_scale) . KV_r[:len_r, :512]
  * q bf16 `[R, Hq, 576]`, out bf16 `[R, Hq, 512]`, kv_cache bf16 `[n_chunks, chunk_tokens, 576]` with
  * the given chunk / token strides (elements).  Hq: 1, 2, 4, 8 or a multiple of 16.
+ * max_kv_len: an upper bound of kv_lens that the host knows, 0 or less: none.  It chooses between kernels (see
+ * mla_decode_lds) and nothing else: results are right for any value, and a bound that is too low only costs time.
  */
 int64_t mi_mla_decode_workspace_bytes(int32_t R, int32_t Hq, int32_t head_dim_v, const MiTuning* tuning);
 

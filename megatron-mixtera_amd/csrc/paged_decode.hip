@@ -2499,7 +2499,7 @@ extern "C" int mi_paged_mla_decode_attention(
   // 44.6 / 28.0, 128 of 100-400 70.1 / 61.4, 16 of 4 000 70 / 59; from 60 000 tokens 61.1 / 57.1 they are level,
   // 122 000 tokens 86.4 / 98.0, 64 requests of 512-8 192 151 / 217.)
   const size_t lds_heads = lds_head + (size_t)4 * kMlaHeadsBuf;
-  const bool few_tokens = shared_tile && (int64_t)R * max_kv_len * (Hq / 128) <= (int64_t)256 * device_cu_count();
+  const bool few_tokens = shared_tile && max_kv_len > 0 && (int64_t)R * max_kv_len * (Hq / 128) <= (int64_t)256 * device_cu_count();
   const bool heads_tile =
       mla_heads_kernel_shape(Hq, chunk_tokens) && tune.mla_decode_lds == 1 && lds_heads <= 160 * 1024 && !few_tokens;
   int grid_x = mla_grid_size(groups, tune);

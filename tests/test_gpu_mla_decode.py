@@ -121,7 +121,17 @@ def test_mla_decode_128_heads_on_both_sides_of_the_token_bound(mi, dev, Hq, boun
         ref = oa.mla_decode_attention(q.squeeze(1), cache, lens_t, bt, 0.07, DV)
         err = (out.float().cpu().squeeze(1) - ref).abs()
         assert (err <= 2e-2 + 2e-2 * ref.abs()).all(), f"max err {err.max().item():.4e}"
-        assert torch.equal(out, eight) == (bound == 0)
+        if bound == 0:
+            assert torch.equal(out, eight)
+
+
+@pytest.mark.parametrize("bound", [0, -1])
+def test_mla_decode_without_a_bound_of_the_lengths_counts_as_many_tokens(mi, dev, bound):
+    """A bound of 0 or less says nothing about the lengths: the kernel of large calls, bit for bit."""
+    q, cache, lens, bt = _case(mi, dev, [1500, 64, 700], 128, 64, seed=5)
+    got, want = (mi.ops.paged_mla_decode_attention(q.to(dev), cache.to(dev), lens.to(dev), bt.to(dev), softmax_scale=0.07,
+                                                   max_kv_len=n) for n in (bound, 1 << 20))
+    assert torch.equal(got, want)
 
 
 def test_mla_decode_many_requests_fall_back_to_streaming(mi, dev):
