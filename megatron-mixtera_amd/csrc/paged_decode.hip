@@ -1950,15 +1950,20 @@ int mi::check_decode_workspace(const void* workspace, int64_t workspace_bytes, i
 // `most` tokens as far as the table's width tells.
 //
 // A CU alone takes in some 30 KB/us of a cache in HBM, so a request's keys and values of a head go to as many workgroups as the
-// chip has left, from 48 KB each up; the shortest (128 KB in all) to one, without a second launch.  Requests of different
-// lengths get the same number, and the longest decides: with `share` KB of the longest's keys and values per workgroup
-// this takes 7 us and share / 28, the stream, whose spans are equal, 10.5 us and the whole at 6.3 TB/s, lengths taken as
-// three quarters of the bound.  Us per call in a graph, twelve caches in turn, the stream and its merge -> this, 128 wide, 16-bit:
-//   one request, 32/8 heads: 31 tokens 8.3 -> 4.1, 215 12.3 -> 7.5, 687 13.1 -> 8.2, 4 515 19.5 -> 14.5, 14 136 31.4 -> 21.5, 36 122
-//   45.7 -> 36.5; 4 x 16/2 of 12 701-21 684 29.4 -> 23.8; 8 x 32/8 of 1 558-2 896 25.7 -> 22.6, of 3 668-5 861 37.6 / 39.2 (estimated
-//   level); 16 x 32/8 of 577-940 21.9 -> 17.2, of 1 015-1 980 28.4 -> 28.0, of 2 063-3 886 47.2 / 49.5; 32 x 32/8 of 261-1 007 27.0 ->
-//   24.8; up to 256 tokens 64 x 32/8 21.3 -> 14.8, 128 x 32/8 (a whole step) 30.0 / 36.6: not there.
-// The whole step of a layer: 1 x 32/8 of 519 13.3 -> 10.5, 2 of 1 955-2 838 22.4 -> 14.9, 16 of 250-499 19.8 -> 15.2.
+// chip has left, from 48 KB each up; the shortest (128 KB in all) to one, without a second launch.  More than 16 (a merge of 32
+// takes 2 us more, also where the requests are far below the bound) only where 16 would have over 128 KB each of a large call.
+// Requests of different lengths get the same number, and the longest decides: with `share` KB of the longest's keys and
+// values per workgroup this takes 7 us and share / 28, the stream, whose spans are equal, 10.5 us and the whole at 6.3 TB/s, lengths
+// taken as three quarters of the bound.  Where lengths differ the stream is faster than that, so `share` has a limit as well.
+// Us per call in a graph, two to twelve caches in turn, the stream and its merge / this, 16-bit caches; every request as long as
+// the bound | from a sixteenth of it up to it | one of it, the others a sixteenth | all of an eighth:
+//   32/8 heads of 128, R x bound: 1 x 100 10.4 / 5.2, 1 x 1 000 13.7 / 9.4, 1 x 16 000 34.0 / 22.4 (an eighth 16.1 / 11.6), 4 x 2 000
+//   19.3 / 12.8 | 16.7 / 11.9 | 15.9 / 11.6 | 12.7 / 7.5, 16 x 500 16.7 / 13.1 | 14.5 / 11.6 | 12.8 / 10.8 | 11.9 / 7.2; above the limit 16 x
+//   2 000 32.8 / 30.2 | 26.8 / 26.4 | 17.2 / 24.0, 32 x 1 000 31.2 / 28.2 | 25.5 / 24.0 | 15.0 / 21.5;
+//   16/2 of 128: 64 x 500 19.2 / 12.7 | 14.9 / 11.1 | 8.9 / 10.5, above it 128 x 1 000 35.8 / 26.7 | 26.7 / 22.5 | 14.4 / 19.4;
+//   8/8 of 64: 4 x 4 000 15.5 / 13.4 | 14.6 / 12.7 | 13.3 / 12.4, above it 4 x 8 000 20.9 / 21.1 | 18.0 / 19.5 | 16.2 / 18.6.
+// An fp8 cache of 8 heads: 4 x 8 000 27.5 / 21.8 | 24.5 / 20.0 | 21.9 / 19.1, above the limit 4 x 16 000 36.7 / 35.4 | 29.5 / 31.7 | 26.4 /
+// 29.8.  32 workgroups to a request where 16 do: 16/2 of 128, 1 x 2 000 at an eighth 8.1 / 10.1.
 constexpr int kShortTile = 2;   // (sub-tiles per iteration; four are 3-8 % slower)
 static int short_splits(int R, int heads, int head_dim, int64_t most, int esz, int chunk_tokens, int grid, const MiTuning& tune,
                         int split_tokens) {
@@ -1970,9 +1975,12 @@ static int short_splits(int R, int heads, int head_dim, int64_t most, int esz, i
   int64_t n = 256 / workgroups;
   if (n > kShortSplits) n = kShortSplits;
   if (n > (kb + 47) / 48) n = (kb + 47) / 48;
+  if (n > 16 && (kb <= 16 * 128 || (heads * head_dim < 512 && workgroups * kb < 32 * 1024))) n = 16;
   if (n > (grid + R) / (2 * R)) n = (grid + R) / (2 * R);   // (what the workspace holds: two words per head beside the values)
   if (n < 1) return 0;
   const float share = (float)kb / (float)n;
+  const bool wide_tokens = head_dim * esz == 256;
+  if (!(n >= 8 && (wide_tokens || heads < 8)) && share > (head_dim == 64 && heads >= 8 ? 192.f : 256.f)) return 0;
   return 7.f + share / 28.f < 10.5f + 0.75f * (float)workgroups * (float)kb / 6300.f ? (int)n : 0;
 }
 
