@@ -329,8 +329,13 @@ __global__ __launch_bounds__(64 * WAVES, PER_SIMD) void paged_prefill_woven_kern
       const uint32_t bits = scale_bits(vscale);
       return __uint_as_float((bits & 0x7f800000u) + (factor_below_one(bits) ? 0x00800000u : 0u));
     };
-    auto value_sign = [](float vscale) { return (uint32_t)(__float_as_int(vscale) >> 31) & 0x80808080u; };
-    auto store_v_fp8 = [&](uint8_t* buf, int i, float vscale) {   // (FACTOR: times the sign and the power of two of their scale)
+    // the sign goes to the fetched bytes, in a branch of its own: as an operation of every store it takes 1.5 % of prompts
+    auto negate_values_fp8 = [&](float vscale) {
+      if (__builtin_expect(__float_as_int(vscale) >= 0, 1)) return;
+#pragma unroll
+      for (int i = 0; i < NP8; ++i) vraw[i] = make_uint2(vraw[i].x ^ 0x80808080u, vraw[i].y ^ 0x80808080u);
+    };
+    auto store_v_fp8 = [&](uint8_t* buf, int i, float vscale) {   // (FACTOR: times the power of two of their scale)
       if constexpr (!FACTOR) {
         const f32x2_t a = fp8x2_lo_to_f32(vraw[i].x), b = fp8x2_hi_to_f32(vraw[i].x);
         const f32x2_t c = fp8x2_lo_to_f32(vraw[i].y), d = fp8x2_hi_to_f32(vraw[i].y);
@@ -340,8 +345,7 @@ __global__ __launch_bounds__(64 * WAVES, PER_SIMD) void paged_prefill_woven_kern
         return;
       }
       const float pow2 = value_pow2(vscale);
-      const uint32_t sign = value_sign(vscale);
-      const uint2 lo = fp8x4_to_16x4<F16>(vraw[i].x ^ sign, pow2), hi = fp8x4_to_16x4<F16>(vraw[i].y ^ sign, pow2);
+      const uint2 lo = fp8x4_to_16x4<F16>(vraw[i].x, pow2), hi = fp8x4_to_16x4<F16>(vraw[i].y, pow2);
       *reinterpret_cast<uint4*>(buf + f_lds + i * RPP8 * PITCH) = make_uint4(lo.x, lo.y, hi.x, hi.y);
     };
     // descriptor of a tile: its rows up to the request's last key (reads beyond return zeros)
@@ -697,6 +701,7 @@ __global__ __launch_bounds__(64 * WAVES, PER_SIMD) void paged_prefill_woven_kern
                if (e >= NVF - NP8) store_k_fp8(kst, e - (NVF - NP8));
              }
            });
+      if constexpr (FACTOR) negate_values_fp8(vscale);
       slot(std::integral_constant<int, 1>{}, Mc, ka, ka_next, va, key0 + 32,
            [&](auto first_values) {
              // this wavefront's share of key tile j+1 and of the value tiles has landed
