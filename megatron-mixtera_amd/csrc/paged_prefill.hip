@@ -1031,16 +1031,29 @@ extern "C" int64_t mi_prefill_workspace_bytes(int32_t T, int32_t R, int32_t Hq, 
 
 // Wavefronts of the one-stream tile kernel's workgroups: eight have a CU to themselves and share every staged tile; of four, two
 // share a CU (width 64: three), so that one's start and end -- 11 us of every workgroup: its request, queries and first tiles, the
-// results, the dispatch of the next -- lie under the other's tiles, for twice the tiles' traffic.  That pays where walks are short:
-// prompts that start from nothing (`raw`: their rotation is part of the start) up to some 6 000 tokens, over an fp8 cache, where
-// every tile is converted as well, 4 600; chunks over a context up to some 2 500 keys.  By the host's bound of the keys.  Us, eight
-// wavefronts -> four, 32/8 heads of 128: 12 prompts of 1 000 tokens 214 -> 191, fp8 250 -> 233; one of 600 33.7 -> 26.5, of 2 000 73.5 ->
-// 62.4; six of 454-3 766 395 -> 381, fp8 445 -> 441; 4 x 5 000 826 -> 811, 3 x 6 000 852 -> 843, fp8 4 x 5 000 912 -> 915; 8 x 500 over 0-2 000
-// 113 -> 102, 8 x 512 over 1 536 162 both, 8 x 512 over 2 048 186 -> 188, 8 x 2 048 over 0-2 048 611 -> 620, in ranges 509 over 61 234 838 -> 909.
-static int prefill_woven_waves(int head_dim, bool fp8, bool raw, int n_split, int max_kv_len) {
+// results, the dispatch of the next -- lie under the other's tiles, for twice the tiles' traffic.  That pays where walks are short,
+// by the host's bound of the keys, and longer for prompts that start from nothing, whose walks are of all lengths and half the
+// bound on average; over an fp8 cache, where every tile is converted as well, shorter.  Most keys are new, as far as sizes tell,
+// where the new tokens fill the longest request and a third of all (up to three requests may be padding).  Requests of at most 128
+// rows on average leave half of eight wavefronts without any: four, whatever the walk (not over an fp8 cache, which all convert; requests of one
+// row, which other kernels serve, hide what the average of the rest is).
+// Four wavefronts' time of eight's, 32/8 | 64/8 | 16/2 heads of 128, `raw` queries:
+//   equal prompts: 8 x 1 500 0.95 | 0.99 | 0.94, 4 x 3 000 0.96 | 0.97 | 1.01, 4 x 5 000 0.99 | 0.99 | 1.01, 1 x 6 000 0.95 (8/8 heads 0.83),
+//   2 x 6 000 1.03 | 1.00 | 1.03, 8 x 6 000 1.01 | 1.00 | 1.00; eleven up to 2 000 0.95 | 0.97 | 0.94, 6 000 0.99 | 0.98 | 1.02; fp8 (32/8 |
+//   64/8) 8 x 1 500 0.94 | 1.04, eleven up to 1 500 0.93 | 0.97, to 2 600 0.99 | 1.03, 1 x 2 600 0.93, 8 x 4 000 0.97 | 0.99, 2 x 5 000 1.06 |
+//   1.00, six of 129-4 097 0.99 (queries done before, without the norm and rotation to cover: 1.06);
+//   chunks over a context: 8 x 512 over 512 0.95 | 0.96 | 1.00, over 1 024 0.99 | 1.04 | 1.01, over 1 536 1.03 | 1.02 | 1.02, over 2 048 1.06 |
+//   1.01 | 1.01, 64 x 64 over 512 0.94 | 0.94 | 0.99, over 1 536 1.16 | 1.07 | 1.08; contexts from 0 up to 1 024 0.94 | 0.90 | 0.87, to 4 096
+//   1.07 | 1.03 | 0.87; fp8 8 x 512 over 256 0.94 | 0.96, over 512 1.01 | 1.01, over 1 024 1.04 | 1.05; 64 x 16 over 4 000 and 16 000, 64/8 heads,
+//   0.69 and 0.72 (fp8, 64 x 8 over 4 000 1.05).
+static int prefill_woven_waves(int head_dim, bool fp8, bool raw, int n_split, int T, int R, int G, bool one_row_requests,
+                                int max_kv_len) {
   if (head_dim == 64) return 4;
-  const int most = raw ? (fp8 ? 4608 : 6144) : 2560;
-  return n_split == 1 && max_kv_len > 0 && max_kv_len <= most ? 4 : 8;
+  if (n_split > 1) return 8;
+  if (!fp8 && !one_row_requests && (int64_t)T * G <= (int64_t)128 * R) return 4;
+  const bool mostly_new = T >= max_kv_len && 3 * (int64_t)T >= (int64_t)(R > 4 ? R - 3 : 1) * max_kv_len;
+  const int most = mostly_new ? (fp8 ? (G > 4 ? 1536 : raw ? 4608 : 2560) : raw ? 6144 : 2560) : (fp8 ? 768 : 1536);
+  return max_kv_len > 0 && max_kv_len <= most ? 4 : 8;
 }
 
 // The two-phase tile kernel for one combination of (wave groups staggered?, fp8 cache?, keys split?, widths, type).
@@ -1165,7 +1178,7 @@ static int launch_paged_prefill(
         workspace_bytes = dec_bytes;
       }
     }
-    const int waves = woven ? prefill_woven_waves(head_dim, fp8, raw != nullptr, n_split, max_kv_len) : 8;
+    const int waves = woven ? prefill_woven_waves(head_dim, fp8, raw != nullptr, n_split, T, R, Gw, one_row_requests, max_kv_len) : 8;
     // wavefronts x whole tokens in a wavefront's 32 (wide heads: 16) rows
     const int sbq_lds = waves * ((head_dim >= 192 ? 16 : 32) / Gw);
     const dim3 lgrid(prefill_query_blocks(T, R, sbq_lds) * Hkv * parts, n_split);

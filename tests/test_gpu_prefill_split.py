@@ -55,7 +55,7 @@ def test_four_wavefronts_give_what_eight_do(mi, dev, Hq, Hkv, dtype, fp8):
     """A row's walk over the tiles does not depend on the rows that share its workgroup: the same bits with the bound of the
     keys that chooses four wavefronts and with one that chooses eight.  Requests around a tile, a block and two tiles, with and
     without a context, values whose scale differs from chunk to chunk."""
-    q_lens, ctx, chunk, d = [1, 63, 64, 65, 33, 128, 200, 7], [0, 0, 0, 0, 300, 63, 1, 130], 64, 128
+    q_lens, ctx, chunk, d = [1, 63, 64, 65, 33, 128, 200, 7, 700], [0, 0, 0, 0, 300, 63, 1, 130, 0], 64, 128
     kv_lens = torch.tensor([a + b for a, b in zip(q_lens, ctx)], dtype=torch.int32)
     cu_q = torch.zeros(len(q_lens) + 1, dtype=torch.int32)
     cu_q[1:] = torch.cumsum(torch.tensor(q_lens), 0)
