@@ -1181,7 +1181,7 @@ static __device__ __forceinline__ void pair_cut(const CutShared& cs, const uint3
   __syncthreads();
   if (tid < n && above + cs.hist[tid] <= target && above + cs.hist[tid] + cs.hist[256 + tid] > target) *cs.cut = key[tid];
   __syncthreads();
-  if (tid < 256) cs.hist[tid] = 0;   // (for the digits, should the list turn out not to hold the cut)
+  if (tid < 512) cs.hist[tid] = 0;   // (for the digits, should the list turn out not to hold the cut)
   __syncthreads();
 }
 
