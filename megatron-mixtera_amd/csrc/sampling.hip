@@ -1503,7 +1503,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_row_kernel(SampleParams
     const float row_first = floorf(mx * kBinsPerUnit), edge = row_first + 1.f;
     int bits = 31 - __builtin_clz(p.V);   // V < 2^(bits + 1)
     const float bin_one = (float)(1u << (31 - bits > 16 ? 16 : 31 - bits));
-const uint32_t none = (uint32_t)(kBins + lane);   // (a place of its own for what no bin takes: no branch)
+    const uint32_t none = (uint32_t)(kBins + lane);   // (a place of its own for what no bin takes: no branch)
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
       if (g >= row.groups) continue;
@@ -1519,14 +1519,18 @@ const uint32_t none = (uint32_t)(kBins + lane);   // (a place of its own for wha
     }
     __syncthreads();
     const uint32_t c0 = bins[2 * tid], c1 = bins[2 * tid + 1];
-    if (by_count) {
-      const int h = (int)(c0 + c1);
+    auto count_window = [&](uint32_t n0, uint32_t n1) {   // (bins 2 tid and 2 tid + 1)
+      const int h = (int)(n0 + n1);
       int incl = wave_scan(h);
       if (lane == 63) red[wave] = (uint32_t)incl;
       __syncthreads();
 #pragma unroll
       for (int w = 0; w < kSampleWaves; ++w) incl += w < wave ? (int)red[w] : 0;
-      if (incl >= p.top_k && incl - h < p.top_k) window[0] = window[1] = incl - (int)c1 >= p.top_k ? 2 * tid : 2 * tid + 1;
+      if (incl >= p.top_k && incl - h < p.top_k) window[0] = window[1] = incl - (int)n1 >= p.top_k ? 2 * tid : 2 * tid + 1;
+      __syncthreads();
+    };
+    if (by_count) {
+      count_window(c0, c1);
     } else {   // (the estimate and its slack: see sample_mass_kernel)
       const float h0 = (float)c0 * fast_exp2((float)(2 * tid) * (-1.4426950408889634f / kBinsPerUnit));
       const float h1 = (float)c1 * fast_exp2((float)(2 * tid + 1) * (-1.4426950408889634f / kBinsPerUnit));
@@ -1547,12 +1551,31 @@ const uint32_t none = (uint32_t)(kBins + lane);   // (a place of its own for wha
         atomicMin(&window[0], in0 ? 2 * tid : 2 * tid + 1);
         atomicMax(&window[1], in1 ? 2 * tid + 1 : 2 * tid);
       }
+      __syncthreads();
     }
-    __syncthreads();
-    const int lo = window[0], hi = window[1];
+    int lo = __builtin_amdgcn_readfirstlane(window[0]), hi = __builtin_amdgcn_readfirstlane(window[1]);
     if (lo <= hi) {
       over = (row_first + 1.f - (float)lo) * (1.f / kBinsPerUnit);
       from = (row_first - (float)hi) * (1.f / kBinsPerUnit);
+    } else if (by_count) {
+      // The k-th value lies below the bins (32 units: a low temperature spreads the values).  Counted again 16 times as wide, in a
+      // walk of the row from memory where the cut's digits would take four (512 x 32 000 bf16, k 50, of them a few such rows:
+      // 58.7 us).
+      constexpr float kWide = kBinsPerUnit / 16.f;
+      bins[2 * tid] = bins[2 * tid + 1] = 0;
+      __syncthreads();
+      const float wide_first = floorf(mx * kWide);
+      sweep<8>(rd, 0, p.V, tid, kSampleThreads, [&](int, float x, bool in) {
+        const float f = __builtin_fmaf(x, -kWide, wide_first + 1.f);
+        if (in && f < (float)kBins) atomicAdd(&bins[(uint32_t)fmaxf(f, 0.f)], 1u);
+      });
+      __syncthreads();
+      count_window(bins[2 * tid], bins[2 * tid + 1]);
+      lo = __builtin_amdgcn_readfirstlane(window[0]);
+      if (lo < kBins) {
+        over = (wide_first + 1.f - (float)lo) * (1.f / kWide);
+        from = (wide_first - (float)lo) * (1.f / kWide);
+      }
     }
   }
 

@@ -563,6 +563,7 @@ def test_rows_in_the_registers_of_a_workgroup(mi, dev, V, dtype):
     ends far below the bins)."""
     R = 86 if V > 32768 else 7     # (the rows of a wide filter that are not done in parts)
     x = _logits(R, V, V, torch.float32)
+    x[6] *= 60 if V % 2 else 3000   # (the k-th value far below the bins, and below the wider ones)
     x[1, V // 2:] = -90.0
     x[2] = x[2, 0]
     if V > 200:
