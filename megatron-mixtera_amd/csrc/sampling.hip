@@ -1929,25 +1929,28 @@ static int sample_parts(int R, int V) {
   if (parts > V / 4096) parts = V / 4096;
   return parts < 1 ? 1 : (parts > kMaxParts ? kMaxParts : parts);
 }
-// Whether the rows are done in parts.  The further launches cost 3-6 us, so the walks they shorten have to be long enough.  fp32 in
-// a graph, us, one workgroup per row (that walks it) against parts:
+// Whether the rows are done in parts, for some type of logits at least.  The further launches cost 3-6 us, so the walks they shorten
+// have to be long enough.  Draws from rows that fit the registers of a workgroup go there, workspace or not, but where row_groups
+// says otherwise; the lines here leave those rows out.  fp32 in a graph, us, one workgroup per row that walks it / parts:
 //   greedy, one walk to shorten: 64 x 151 936 16.9 / 12.0, 64 x 32 768 below the line 6.2 / 7.5;
-//   plain draws, two: 64 x 50 304 19.4 / 16.0, 64 x 32 768 below it 13.5 / 13.7;
+//   plain draws, two: 64 x 128 256 37 / 21;
 //   top-k, whose pick grows with its lists: 64 x 128 256 39.1 / 31.1, and does not gain from two: 128 x 100 352 35.2 / 37.7;
-//   top-p, three: 64 x 16 384 30.0 / 19.4, 64 x 128 256 101.8 / 28.1.
-// Rows that fit the registers of a workgroup go there in many of these cases, workspace or not: row_groups.
+//   top-p, three: 64 x 128 256 101.8 / 28.1.
 // More than 128 rows have one part each, and are done this way for the walks alone: a top-p row that does not fit the registers
 // of a workgroup.  fp32 / bf16: 256 x 128 256 119 / 115 -> 67 / 60, 512 x 151 936 255 / 253 -> 139 / 124; peaked rows 512 x
-// 128 256 130 / 122 -> 115 / 95.  (40 KB of scratch a row)
+// 128 256 130 / 122 -> 115 / 95.  That takes 40 KB of scratch a row, at most 40 MB: more rows are walked.
 constexpr int kManyRows = 1024;
-static bool many_rows_by_walks(int V, int top_k, float top_p) { return top_k == 0 && top_p > 0.f && V > 65536; }
+constexpr int kRowInRegisters = 32768;     // widest row whose filter does not gain from parts
+constexpr int kWidestInRegisters = 65536;
 static bool sample_in_parts(int R, int V, int top_k, float top_p) {
-  if (R > 128) return R <= kManyRows && many_rows_by_walks(V, top_k, top_p);
+  const bool by_mass = top_k == 0 && top_p > 0.f;
+  if (R > 128) return by_mass && R <= kManyRows && V > kWidestInRegisters;
   if (V < kFastMinVocab || top_k > kFastTopK) return false;
   if (top_k == 1) return V >= 1600 * (R > 50 ? R : 50);
-  if (top_k > 1) return R <= 85;
-  if (R > 85) return V >= 65536;
-  return V >= 49152 || (top_p > 0.f && R <= 64);
+  if (top_k > 1) return R <= 85 && V > kRowInRegisters;
+  if (!by_mass) return V > kWidestInRegisters || (R <= 16 && V > 57344);
+  if (V <= kRowInRegisters) return false;
+  return R > 85 ? V >= 65536 : V >= 49152 || R <= 64;
 }
 
 static int64_t align256(int64_t n) { return (n + 255) & ~(int64_t)255; }
@@ -1975,22 +1978,28 @@ static int64_t sample_layout(SplitParams* p, uint8_t* base, int R, int V, int to
 }
 
 // Whether draws from rows of V elements take the registers of one workgroup, and how many groups of 16 bytes a lane: 0 = no.
-// Up to 65 536 elements fit without spilling.  A plain draw is faster than any other form throughout.  A filter's bins and
-// lists are work that parts share: above 32 768 elements parts, where the rows are few enough for them, are level or
-// better.  Without parts the one other form walks the row several times; only top-k over fp32, which it reads once, stays
-// there above 32 768.  In a graph, us, the other form -> this one, fp32 / bf16, N(0, 3):
-//   plain: 16 x 32 000 15.1 / 17.0 -> 7.4 / 9.1, 256 x 32 000 17.4 / 17.9 -> 9.6 / 9.8, 1 x 65 536 12.1 / 12.6 -> 10.7 / 11.0,
-//          256 x 65 536 30.7 / 23.5 -> 20.6 / 12.3;
+// Up to 65 536 elements fit without spilling.  A plain draw is faster than any other form, but for a few of the widest fp32 rows,
+// which parts scale by the temperature.  A filter's bins and lists are work that parts share: above 32 768 elements parts, where
+// the rows are few enough for them, are level or better.  Without parts the one other form walks the row several times; only
+// top-k up to kFastTopK, which it reads once, stays there above 32 768: over fp32, and over a 16-bit type where more than 256
+// rows, which it takes two to a CU, are not the widest.  In a graph, us, the other form -> this one, fp32 / bf16, N(0, 3):
+//   plain: 16 x 32 000 15.1 / 17.0 -> 7.4 / 9.1, 256 x 32 000 17.4 / 17.9 -> 9.6 / 9.8, 1 x 65 536 12.1 / 12.6 -> 10.7 / 11.0 (fp32 with a
+//          temperature 12.8, here 13.7; 1 x 50 257 13.0 -> 11.0), 256 x 65 536 30.7 / 23.5 -> 20.6 / 12.3;
 //   top-k 50: 16 x 32 000 16.8 / 17.0 -> 13.0 / 15.5, 128 x 32 000 24.0 / 24.3 -> 13.5 / 16.1; 16 x 65 536 17.3 / 17.7, here 21.8 /
-//          20.6; 512 x 50 303 45.4 / 43.7, here 54.7 / 41.6;
+//          20.6; bf16 512 x 32 769 34.1, here 38.1, 512 x 50 257 44.1 -> 43.5, 1 024 x 50 257 76.3, here 83.0,
+//          1 024 x 65 536 118 -> 85; k 1 500, bf16: 512 x 50 257 70 -> 51;
 //   top-p 0.9: 16 x 32 000 19.4 / 20.2 -> 16.0 / 18.8, 256 x 32 000 51.4 / 50.0 -> 17.9 / 19.7, 256 x 65 536 82 / 74 -> 33 / 26; 16 x
-//          65 536 22.6 / 23.5, here 24.0 / 25.5.
+//          65 536 22.6 / 23.5, here 24.0 / 25.5; peaked rows 1 x 32 000 18.1 / 18.6 -> 13.4 / 15.3; but top-p 0.999: 7 x 32 000 22.3 / 23.2, here 23.4 / 25.6.
 template <int DT>
 static int row_groups(const SampleParams& s, bool in_parts) {
   constexpr int VEC = DT != 0 ? 8 : 4;
-  if (s.top_k == 1 || s.V < VEC || s.V > 65536) return 0;
-  const bool filtered = s.top_k > 1 || s.top_p > 0.f;
-  if (filtered && s.V > 32768 && (in_parts || (s.top_k > 1 && DT == 0))) return 0;
+  if (s.top_k == 1 || s.V < VEC || s.V > kWidestInRegisters) return 0;
+  if (s.top_k > 1) {
+    const int widest_walked = s.top_k > kFastTopK || s.R <= 256 ? 0 : s.R <= 512 ? 49152 : 57344;
+    if (s.V > kRowInRegisters && (in_parts || DT == 0 || s.V < widest_walked)) return 0;
+  } else if (in_parts) {
+    if (s.top_p > 0.f ? s.V > kRowInRegisters : DT == 0 && s.inv_temperature != 1.0f) return 0;
+  }
   return (row_run<VEC>(s.V) + 64 * VEC - 1) / (64 * VEC);
 }
 

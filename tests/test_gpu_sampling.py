@@ -33,6 +33,24 @@ def _with_negative_nan(x, where):
     return x.contiguous().view(whole).masked_fill(where, bits).view(x.dtype)
 
 
+def _by_one_workgroup(mi, y, u, top_k, top_p, temperature=0.7):
+    """(tokens, cuts) of the form that walks a row with one workgroup: without a workspace, and for draws from rows that would fit
+    the registers of a workgroup as the first part of a wider row, masked from there on."""
+    lib, (R, V) = mi._lib.load(), y.shape
+    if top_k != 1 and V <= 65536:
+        wide = torch.full((R, 65544), float("-inf"), dtype=y.dtype, device=y.device)
+        wide[:, :V] = y
+        y = wide
+    token = torch.empty(R, dtype=torch.int64, device=y.device)
+    cut = torch.empty(R, dtype=torch.float32, device=y.device)
+    code = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}[y.dtype]
+    rc = lib.mi_sample_from_logits(y.data_ptr(), y.stride(0), code, R, y.size(1), top_k, top_p, temperature, u.data_ptr(), 0,
+                                   token.data_ptr(), cut.data_ptr(), None, None, None, -1, None,
+                                   torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, lib.mi_last_error()
+    return token, cut
+
+
 # ----------------------------------------------------------------------------------------------
 # last-token gather
 # ----------------------------------------------------------------------------------------------
@@ -414,12 +432,13 @@ def test_context_log_probs_through_the_kernel(mi, dev):
         Ctx.TOKEN_ROUNDER, Ctx.REQUEST_ROUNDER = saved
 
 
-@pytest.mark.parametrize("R,V", [(1, 16384), (2, 16389), (5, 50257), (64, 32000), (85, 49152), (128, 65536), (129, 65536), (1, 260000)])
+@pytest.mark.parametrize("R,V", [(1, 16384), (2, 16389), (5, 50257), (64, 32000), (85, 49152), (128, 65536), (129, 65536), (1, 260000),
+                                 (32, 24577), (3, 32768), (64, 32769), (16, 57345), (7, 65537), (86, 65539), (257, 57344)])
 @pytest.mark.parametrize("kind", ["flat", "peaked", "equal", "few", "masked", "nan"])
 def test_rows_in_parts_equal_rows_by_one_workgroup(mi, dev, R, V, kind):
-    """Rows cut into parts give the tokens and cut values of the one-workgroup entry point, bit for bit: where the
-    parts' estimates hold, and where they fail (equal values, a handful of values, most of the row masked)."""
-    lib = mi._lib.load()
+    """Rows cut into parts, and rows in the registers of a workgroup, give the tokens and cut values of the workgroup that walks a
+    row, bit for bit: where their estimates hold, and where they fail (equal values, a handful of values, most of the row
+    masked).  Sizes either side of the lines between the forms."""
     g = torch.Generator().manual_seed(R + V)
     x = torch.randn(R, V, generator=g) * 3
     if kind == "peaked":
@@ -437,13 +456,7 @@ def test_rows_in_parts_equal_rows_by_one_workgroup(mi, dev, R, V, kind):
         y = x.to(dtype).to(dev)
         for top_k, top_p in ((1, 0.0), (0, 0.0), (0, 0.5), (0, 0.95), (0, 1.0), (2, 0.0), (50, 0.0), (768, 0.0), (769, 0.0)):
             got, _, cut = mi.ops.sample_from_logits(y, top_k=top_k, top_p=top_p, temperature=0.7, uniform=u, return_cut=True)
-            want = torch.empty(R, dtype=torch.int64, device=dev)
-            want_cut = torch.empty(R, dtype=torch.float32, device=dev)
-            rc = lib.mi_sample_from_logits(y.data_ptr(), y.stride(0), 0 if dtype == torch.float32 else 1, R, V, top_k, top_p, 0.7,
-                                           u.data_ptr(), 0, want.data_ptr(), want_cut.data_ptr(), None, None, None, -1, None,
-                                           torch.cuda.current_stream().cuda_stream)
-            assert rc == 0, lib.mi_last_error()
-            torch.cuda.synchronize()
+            want, want_cut = _by_one_workgroup(mi, y, u, top_k, top_p)
             assert torch.equal(got, want), (dtype, top_k, top_p)
             assert torch.equal(cut, want_cut), (dtype, top_k, top_p)
 
@@ -461,13 +474,12 @@ def test_logits_too_large_for_masses_take_the_argmax(mi, dev, V, mode):
     assert (x.gather(1, got[:, None]) * (1 / 0.7) >= kept).all()
 
 
-@pytest.mark.parametrize("R,V,pad", [(3, 16387, 0), (128, 80001, 1), (86, 140000, 4)])
+@pytest.mark.parametrize("R,V,pad", [(3, 16387, 0), (128, 80001, 1), (86, 140000, 4), (5, 30011, 2), (40, 1003, 3), (6, 50001, 1)])
 @pytest.mark.parametrize("kind", ["rising", "negative", "zeros", "huge", "wide", "negative nan", "part masked", "all masked", "infinite"])
 def test_parts_where_the_bins_are_at_their_edges(mi, dev, R, V, pad, kind):
-    """Top-p and plain draws of rows in parts against one workgroup per row: a maximum that rises from batch to batch of a
-    part (the bins move), values whose integer order is not theirs, values that leave the bins' range, parts of nothing but
-    -inf or NaN, rows off 16 bytes."""
-    lib = mi._lib.load()
+    """Draws from rows in parts, and in the registers of a workgroup, against one workgroup that walks a row: a maximum that rises
+    from batch to batch of a part (the bins move), values whose integer order is not theirs, values that leave the bins'
+    range, parts of nothing but -inf or NaN, rows off 16 bytes."""
     g = torch.Generator().manual_seed(R + V)
     x = torch.randn(R, V, generator=g) * 3
     if kind == "rising":
@@ -480,12 +492,13 @@ def test_parts_where_the_bins_are_at_their_edges(mi, dev, R, V, pad, kind):
         x *= 1e30
     elif kind == "wide":
         x *= 200
-    elif kind == "negative nan":
-        x[:, ::7] = torch.tensor(-4194304, dtype=torch.int32).view(torch.float32)   # 0xffc00000
-        x[R // 2] = x[0, 0]
+    negative_nan = torch.zeros(R, V, dtype=torch.bool)
+    if kind == "negative nan":
+        negative_nan[:, ::7] = True
+        negative_nan[R // 2] = True
     elif kind == "part masked":
         x[:, : V // 2] = float("-inf")
-        x[R // 2, : V // 2] = x.new_tensor(-4194304, dtype=torch.int32).view(torch.float32)
+        negative_nan[R // 2, : V // 2] = True
     elif kind == "all masked":
         x[::2] = float("-inf")
     elif kind == "infinite":
@@ -493,18 +506,15 @@ def test_parts_where_the_bins_are_at_their_edges(mi, dev, R, V, pad, kind):
     u = torch.rand(R, generator=g).to(dev)
     for dtype in (torch.float32, torch.bfloat16):
         y = torch.zeros(R, V + pad, dtype=dtype, device=dev)[:, :V]
-        y.copy_(x)
-        for top_k, top_p in ((0, 0.0), (0, 0.3), (0, 0.9), (0, 0.999)):
+        y.copy_(_with_negative_nan(x.to(dtype), negative_nan))
+        for top_k, top_p in ((0, 0.0), (0, 0.3), (0, 0.9), (0, 0.999), (2, 0.0), (300, 0.0)):
             got, _, cut = mi.ops.sample_from_logits(y, top_k=top_k, top_p=top_p, temperature=0.7, uniform=u, return_cut=True)
-            want = torch.empty(R, dtype=torch.int64, device=dev)
-            want_cut = torch.empty(R, dtype=torch.float32, device=dev)
-            rc = lib.mi_sample_from_logits(y.data_ptr(), y.stride(0), 0 if dtype == torch.float32 else 1, R, V, top_k, top_p, 0.7,
-                                           u.data_ptr(), 0, want.data_ptr(), want_cut.data_ptr(), None, None, None, -1, None,
-                                           torch.cuda.current_stream().cuda_stream)
-            assert rc == 0, lib.mi_last_error()
-            torch.cuda.synchronize()
-            assert torch.equal(got, want), (dtype, top_k, top_p)
-            assert torch.equal(cut, want_cut), (dtype, top_k, top_p)
+            want, want_cut = _by_one_workgroup(mi, y, u, top_k, top_p)
+            # (nothing but NaNs: the masked end of the wider row is above them; the workgroup that walks a row takes negative NaNs
+            # for its largest values where it counts)
+            rows = ~(negative_nan.any(-1) if top_k else negative_nan.all(-1)).to(dev)
+            assert torch.equal(got[rows], want[rows]), (dtype, top_k, top_p)
+            assert torch.equal(cut[rows], want_cut[rows]), (dtype, top_k, top_p)
 
 
 @pytest.mark.parametrize("V", [1 << 18, 1 << 20])
@@ -555,13 +565,57 @@ def test_sampling_inside_use_workspace(mi, dev, buffer):
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("R,V", [(129, 65537), (257, 70001), (1024, 65540), (1025, 65540)])
+def test_top_p_of_many_wide_rows(mi, dev, R, V, dtype):
+    """More than 128 rows that do not fit the registers of a workgroup: one part each up to 1 024 rows, a walk from there on.  The
+    same tokens and cuts as the walk's: flat, peaked and equal rows, half masked ones, rows with a NaN."""
+    lib = mi._lib.load()
+    gen = torch.Generator(device=dev).manual_seed(R)
+    x = torch.empty(R, V, device=dev).normal_(0, 3, generator=gen)
+    x[1::8, 7::997] += 14
+    x[2::8] = -2.5
+    x[3::8, ::2] = float("-inf")
+    x[4::32, V // 3] = float("nan")
+    x[5::8] = x[5::8].round()
+    x[6::8, : V - 9] = float("-inf")
+    y = x.to(dtype)
+    del x
+    u = torch.rand(R, device=dev, generator=gen)
+    assert (lib.mi_sample_workspace_bytes(R, V, 0, 0.9) > 0) == (R <= 1024)
+    for top_p in (0.3, 0.9, 0.999, 1.0):
+        got, _, cut = mi.ops.sample_from_logits(y, top_p=top_p, temperature=0.7, uniform=u, return_cut=True)
+        want, want_cut = _by_one_workgroup(mi, y, u, 0, top_p)
+        assert torch.equal(got, want) and torch.equal(cut, want_cut), top_p
+
+
+@pytest.mark.parametrize("short,off", [(1, 0), (0, 16)], ids=["too small", "off a line"])
+def test_many_rows_pass_over_a_workspace_that_does_not_serve(mi, dev, short, off):
+    """More than 128 rows did without scratch at every size before they had a use for it: a buffer that does not serve is not used
+    and not written.  128 rows refuse it, as they did."""
+    lib, V = mi._lib.load(), 65537
+    gen = torch.Generator(device=dev).manual_seed(3)
+    for R in (128, 129):
+        y = torch.empty(R, V, device=dev).normal_(0, 3, generator=gen)
+        u = torch.rand(R, device=dev, generator=gen)
+        room = torch.full((lib.mi_sample_workspace_bytes(R, V, 0, 0.9) + 256,), 0x5a, dtype=torch.uint8, device=dev)
+        token = torch.empty(R, dtype=torch.int64, device=dev)
+        rc = lib.mi_sample_from_logits_ws(y.data_ptr(), V, 0, R, V, 0, 0.9, 0.7, u.data_ptr(), 0, token.data_ptr(), None, None, None, None,
+                                          -1, None, room.data_ptr() + off, room.numel() - 256 - short,
+                                          torch.cuda.current_stream().cuda_stream)
+        assert (rc == 0) == (R > 128)
+        if rc == 0:
+            assert torch.equal(token, _by_one_workgroup(mi, y, u, 0, 0.9)[0])
+        assert (room == 0x5a).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("V", [4, 8, 9, 255, 4097, 16391, 32767, 32768, 32769, 65535, 65536])
 def test_rows_in_the_registers_of_a_workgroup(mi, dev, V, dtype):
     """Rows that start on any element and end within a group of 16 bytes; wavefronts without elements (short rows), the widest
     rows of either number of groups; lists of a few members, of many, and none that holds the cut (equal values, a top-k that
     ends far below the bins)."""
-    R = 86 if V > 32768 else 7     # (the rows of a wide filter that are not done in parts)
+    R = 129 if V > 32768 else 7     # (the rows of a wide filter that are not done in parts)
     x = _logits(R, V, V, torch.float32)
     x[6] *= 60 if V % 2 else 3000   # (the k-th value far below the bins, and below the wider ones)
     x[1, V // 2:] = -90.0
