@@ -961,7 +961,13 @@ PyObject* sample_from_logits(PyObject* const* a) {
   // a 256-byte line -- leaves the rows to one workgroup each)
   const int64_t need = mi_sample_workspace_bytes((int)R, (int)V, (int)top_k, top_p);
   Scratch ws;
-  if (a[11] == Py_None || usable(tensor(a[11], "workspace"), logits, need, 256)) ws = scratch(logits, stream, need, Py_None, a[11]);
+  Tensor many;   // (scratch of a large batch belongs to the call, or to the graph that captures it: the stream's own is not for capture)
+  if (a[11] == Py_None && R > 128 && need > 0) {
+    many = at::empty({need}, logits.options().dtype(at::kByte));
+    ws = {many.data_ptr(), need};
+  } else if (a[11] == Py_None || usable(tensor(a[11], "workspace"), logits, need, 256)) {
+    ws = scratch(logits, stream, need, Py_None, a[11]);
+  }
   check(mi_sample_from_logits_ws(logits.data_ptr(), logits.stride(0), code, (int)R, (int)V, (int)top_k, top_p,
                               (float)as_float(a[3]), (const float*)ptr(uniform), (int)as_int(a[5]), (int64_t*)samples.data_ptr(),
                               want_cut ? (float*)cut.data_ptr() : nullptr, (const int32_t*)ptr(lens[0]), (const int32_t*)ptr(lens[1]),

@@ -668,3 +668,30 @@ def test_a_top_k_above_the_count_of_numbers_keeps_them_all(mi, dev, V, dtype):
         got, _ = mi.ops.sample_from_logits(y, top_k=top_k, temperature=0.8, uniform=u)
         rows = ((numbers < top_k) | ((x > float("-inf")).sum(-1) <= top_k) & (top_k == V)).to(dev)
         assert torch.equal(got[rows], want[rows]), top_k
+
+
+def test_many_rows_under_capture_leave_the_stream_without_a_workspace(mi, dev):
+    """More than 128 rows needed no scratch before they were done in parts, and could be captured as they are.  The scratch of a
+    captured call is the graph's: replays, with eager calls and the stream's own workspace growing in between, give the eager
+    tokens."""
+    R, V = 129, 65544
+    gen = torch.Generator(device=dev).manual_seed(9)
+    rows = [torch.empty(R, V, device=dev).normal_(0, 3, generator=gen) for _ in range(3)]
+    u = torch.rand(R, device=dev, generator=gen)
+    want = [mi.ops.sample_from_logits(x, top_p=0.9, uniform=u)[0] for x in rows]
+    x = rows[0].clone()
+    stream = torch.cuda.Stream()
+    before = dict(mi.ops._workspace_sizes)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        got, _ = mi.ops.sample_from_logits(x, top_p=0.9, uniform=u)
+    assert mi.ops._workspace_sizes == before
+    for i in (0, 1, 2, 1):
+        x.copy_(rows[i])
+        with torch.cuda.stream(stream):
+            stream.wait_stream(torch.cuda.current_stream(dev))
+            mi.ops.sample_from_logits(rows[2][: 8 << i], top_p=0.9, uniform=u)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want[i])
