@@ -48,7 +48,9 @@ def test_cfg2_shape_reduced_batch(mi, dev):
 def test_head_grouping(mi, dev, Hq, Hkv, d):
     cfg = mi.synthetic.DecodeConfig("g", 5, Hq, Hkv, d, 1, 700, chunk=64, seed=Hq * 131 + Hkv * 7 + d)
     case = mi.synthetic.make_decode_case(cfg, dev)
-    _close(_run_case(mi, case), _ref(case), 2e-2)
+    ref = _ref(case)
+    for split in (0, 64):   # (few short requests by the kernel of their own, and by the stream)
+        _close(_run_case(mi, case, split_tokens=split), ref, 2e-2)
 
 
 @pytest.mark.parametrize("chunk", [16, 48, 128, 256])
@@ -234,14 +236,17 @@ def test_fp8_kv_cache(mi, dev, d):
     assert torch.equal(ks.cpu(), ks_ref) and torch.equal(vs.cpu(), vs_ref), "scales differ"
     assert torch.equal(k8.cpu(), k8_ref) and torch.equal(v8.cpu(), v8_ref), "e4m3 bytes differ"
 
-    out = mi.ops.paged_decode_attention(case.q, k8, v8, case.kv_lens, case.block_table, k_scales=ks, v_scales=vs)
-    torch.cuda.synchronize()
     # reference of record: fp32 attention over the ORIGINAL (unquantised) K/V, tolerance 6e-2
-    _close(out, _ref(case), 6e-2)
+    ref = _ref(case)
     # and tighter against the checker run on the dequantised cache
     ref_q = oa.paged_decode_attention(case.q.cpu().squeeze(1), k8_ref, v8_ref, case.kv_lens.cpu(),
                                       case.block_table.cpu(), k_scales=ks_ref, v_scales=vs_ref)
-    _close(out, ref_q, 2e-2)
+    for split in (0, 64):
+        out = mi.ops.paged_decode_attention(case.q, k8, v8, case.kv_lens, case.block_table, k_scales=ks, v_scales=vs,
+                                            split_tokens=split)
+        torch.cuda.synchronize()
+        _close(out, ref, 6e-2)
+        _close(out, ref_q, 2e-2)
 
 
 def test_fp8_decode_append(mi, dev):
@@ -309,7 +314,8 @@ def test_short_requests_by_one_workgroup_per_head(mi, dev, Hq, Hkv, d, chunk, fp
 
 @pytest.mark.parametrize("Hq,Hkv,d,chunk,lens", [
     (8, 8, 64, 32, [0, 1, 33, 2047, 2048]), (32, 8, 128, 256, [5, 700, 1025]), (16, 1, 128, 64, [0, 31, 64, 65, 900, 1500, 1537, 3]),
-    (20, 1, 64, 256, [7000]), (4, 2, 128, 128, [9001, 12]), (64, 8, 128, 256, [40000])])
+    (20, 1, 64, 256, [7000]), (4, 2, 128, 128, [9001, 12]), (64, 8, 128, 256, [40000]), (20, 1, 64, 256, [3000]),
+    (4, 2, 128, 128, [9001, 12, 0, 4000]), (64, 8, 128, 256, [20000])])
 @pytest.mark.parametrize("fp8", [False, True])
 def test_few_requests_by_several_workgroups_per_head(mi, dev, Hq, Hkv, d, chunk, lens, fp8):
     """Requests cut evenly over workgroups and their merge, against the stream: shares without tiles, without all of their

@@ -76,12 +76,16 @@ def _oracle(case, lens, qw, kw, pos, *, norm, table, interleaved):
 
 LENS = [0, 1, 2, 15, 16, 17, 31, 32, 33, 63, 64, 65, 129, 700, 0, 2049]
 
+# few short requests have a kernel of their own; a span length asks for the stream of the larger batches
+SPANS = pytest.mark.parametrize("split_tokens", [0, 64], ids=["short", "stream"])
 
+
+@SPANS
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("norm", [None, "rms", "l2"])
 @pytest.mark.parametrize("rotary", ["none", "half", "half64", "interleaved", "interleaved40"])
 @pytest.mark.parametrize("Hq,Hkv,d", [(32, 8, 128), (8, 8, 64), (6, 2, 128), (16, 1, 64), (20, 1, 128)])
-def test_fused_step_equals_the_separate_launches(mi, dev, Hq, Hkv, d, rotary, norm, dtype):
+def test_fused_step_equals_the_separate_launches(mi, dev, Hq, Hkv, d, rotary, norm, dtype, split_tokens):
     if rotary == "half64" and d == 64:
         pytest.skip("rot_dim 64 is the full width at head_dim 64")
     rot = {"none": 0, "half": d, "half64": 64, "interleaved": d, "interleaved40": 40}[rotary]
@@ -90,7 +94,7 @@ def test_fused_step_equals_the_separate_launches(mi, dev, Hq, Hkv, d, rotary, no
     case, lens, qw, kw, pos = _step_case(mi, dev, Hq=Hq, Hkv=Hkv, d=d, chunk=64, lens=LENS, dtype=dtype, seed=Hq + d)
     (out_a, kc_a, vc_a), (out_b, kc_b, vc_b) = _run_both(mi, dev, case, lens, qw, kw, pos, norm=norm, table=table,
                                                          interleaved=interleaved, mixed=False,
-                                                         max_kv_len=int(lens.max()))
+                                                         max_kv_len=int(lens.max()), split_tokens=split_tokens)
     dummy = case.k_cache.size(0) - 1   # (rows of length 0 are padding: nothing is appended for them)
     assert torch.equal(kc_a[:dummy], kc_b[:dummy]), "key cache differs from the separate launch"
     assert torch.equal(vc_a[:dummy], vc_b[:dummy]), "value cache differs from the separate launch"
@@ -181,12 +185,13 @@ def test_fused_step_without_faithful_rounding_and_repeated_steps(mi, dev):
     _close(kc[:dummy], kc_ref[:dummy], 2e-2, "key cache after three steps")
 
 
+@SPANS
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("mixed", [False, True])
 @pytest.mark.parametrize("rotary", ["none", "half", "interleaved", "interleaved40"])
 @pytest.mark.parametrize("norm", [None, "rms"])
 @pytest.mark.parametrize("Hq,Hkv", [(32, 8), (6, 2), (20, 1)])
-def test_fused_step_over_an_fp8_cache(mi, dev, Hq, Hkv, norm, rotary, mixed, dtype):
+def test_fused_step_over_an_fp8_cache(mi, dev, Hq, Hkv, norm, rotary, mixed, dtype, split_tokens):
     """The one-kernel step over an fp8-e4m3 cache: bytes and scales equal to the separate launches (norm / rotary
     with key_out, then the quantising append), tokens that open a chunk (lengths 1, 65, 129: they set the scale) and
     tokens that reuse a stored scale; output within 8e-3 of the separate launches and 6e-2 of the unquantised checker."""
@@ -222,17 +227,17 @@ def test_fused_step_over_an_fp8_cache(mi, dev, Hq, Hkv, norm, rotary, mixed, dty
         out_a = mi.ops.decode_step_attention(None, None, None, k8a, v8a, case.kv_lens, case.block_table,
                                              mixed_qkv=grouped.reshape(R, 1, -1).contiguous(), num_query_heads=Hq,
                                              num_kv_heads=Hkv, positions=posd, k_scales=ksa, v_scales=vsa, headroom=1.5,
-                                             max_kv_len=int(lens.max()), **common)
+                                             max_kv_len=int(lens.max()), split_tokens=split_tokens, **common)
     else:
         out_a = mi.ops.decode_step_attention(case.q, case.k_new, case.v_new, k8a, v8a, case.kv_lens, case.block_table,
                                              positions=posd, k_scales=ksa, v_scales=vsa, headroom=1.5,
-                                             max_kv_len=int(lens.max()), **common)
+                                             max_kv_len=int(lens.max()), split_tokens=split_tokens, **common)
     q_b, k_b = torch.empty_like(case.q), torch.empty_like(case.k_new)
     with mi.ops.tuning(norm_rope_vectorised=-1):
         mi.ops.norm_rope_append(case.q, case.k_new, query_out=q_b, key_out=k_b, q_positions=posd, k_positions=posd, **common)
     mi.ops.kv_append_decode_fp8(k_b, case.v_new, k8b, v8b, ksb, vsb, case.block_table, case.kv_lens, headroom=1.5)
     out_b = mi.ops.paged_decode_attention(q_b, k8b, v8b, case.kv_lens, case.block_table, k_scales=ksb, v_scales=vsb,
-                                          max_kv_len=int(lens.max()))
+                                          max_kv_len=int(lens.max()), split_tokens=split_tokens)
     torch.cuda.synchronize()
     assert torch.equal(k8a, k8b) and torch.equal(v8a, v8b), "cache bytes differ from the separate launches"
     assert torch.equal(ksa, ksb) and torch.equal(vsa, vsb), "scales differ from the separate launches"
@@ -289,9 +294,10 @@ def test_fused_step_more_requests_than_one_launch_takes(mi, dev):
     _close(out_a, ref, 2e-2, "sliced fused step vs checker")
 
 
+@SPANS
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("R", [1, 63, 64, 65, 200])
-def test_fused_step_over_a_cache_that_holds_nan_past_the_lengths(mi, dev, R, fp8):
+def test_fused_step_over_a_cache_that_holds_nan_past_the_lengths(mi, dev, R, fp8, split_tokens):
     """The wavefront that ends a request takes the step's rows from LDS; what its loads find in their slots and past them
     must not reach the result.  Request counts around the 64 that lie in lanes."""
     Hq, Hkv, d, chunk = 8, 2, 128, 32
@@ -311,7 +317,7 @@ def test_fused_step_over_a_cache_that_holds_nan_past_the_lengths(mi, dev, R, fp8
             valid[bt[r, t // chunk], t % chunk] = True
     keep = valid.to(dev)[:, :, None, None]
     common = dict(q_weight=qw.to(dev), k_weight=kw.to(dev), norm="rms", eps=1e-5, positions=pos.to(dev),
-                  rotary_emb=orn.rotary_table(4096, d, base=500000.0).to(dev), max_kv_len=int(lens.max()))
+                  rotary_emb=orn.rotary_table(4096, d, base=500000.0).to(dev), max_kv_len=int(lens.max()), split_tokens=split_tokens)
     got = []
     for fill in (bad, [torch.zeros_like(c) for c in caches]):
         kc, vc = (torch.where(keep, c, f) for c, f in zip(caches, fill))

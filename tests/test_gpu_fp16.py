@@ -28,12 +28,13 @@ def _close(got, ref, tol=2e-2, what=""):
 def test_decode_head_groupings(mi, dev, Hq, Hkv, d):
     cfg = mi.synthetic.DecodeConfig("g16", 5, Hq, Hkv, d, 1, 700, chunk=64, seed=Hq * 131 + Hkv * 7 + d)
     case = mi.synthetic.make_decode_case(cfg, dev, dtype=F16)
-    out = mi.ops.paged_decode_attention(case.q, case.k_cache, case.v_cache, case.kv_lens, case.block_table)
-    torch.cuda.synchronize()
-    assert out.dtype == F16
     ref = oa.paged_decode_attention(case.q.cpu().squeeze(1), case.k_cache.cpu(), case.v_cache.cpu(), case.kv_lens.cpu(),
                                     case.block_table.cpu())
-    _close(out, ref, what="decode")
+    for split in (0, 64):   # (few short requests by the kernel of their own, and by the stream)
+        out = mi.ops.paged_decode_attention(case.q, case.k_cache, case.v_cache, case.kv_lens, case.block_table, split_tokens=split)
+        torch.cuda.synchronize()
+        assert out.dtype == F16
+        _close(out, ref, what="decode")
 
 
 @pytest.mark.parametrize("chunk", [16, 128, 256])
@@ -92,16 +93,18 @@ def test_fp16_queries_over_an_fp8_cache(mi, dev, d):
     v8_ref, vs_ref = oa.quantize_chunks_fp8(case.v_cache.cpu())
     assert torch.equal(ks.cpu(), ks_ref) and torch.equal(vs.cpu(), vs_ref), "scales differ"
     assert torch.equal(k8.cpu(), k8_ref) and torch.equal(v8.cpu(), v8_ref), "e4m3 bytes differ"
-    out = mi.ops.paged_decode_attention(case.q, k8, v8, case.kv_lens, case.block_table, k_scales=ks, v_scales=vs)
-    torch.cuda.synchronize()
-    assert out.dtype == F16
     ref_q = oa.paged_decode_attention(case.q.cpu().squeeze(1), k8_ref, v8_ref, case.kv_lens.cpu(), case.block_table.cpu(),
                                       k_scales=ks_ref, v_scales=vs_ref)
-    _close(out, ref_q, what="fp16 over fp8, dequantised cache")
     ref = oa.paged_decode_attention(case.q.cpu().squeeze(1), case.k_cache.cpu(), case.v_cache.cpu(), case.kv_lens.cpu(),
                                     case.block_table.cpu())
-    err = (out.float().cpu().squeeze(1) - ref).abs()
-    assert (err <= 6e-2 + 6e-2 * ref.abs()).all()
+    for split in (0, 64):
+        out = mi.ops.paged_decode_attention(case.q, k8, v8, case.kv_lens, case.block_table, k_scales=ks, v_scales=vs,
+                                            split_tokens=split)
+        torch.cuda.synchronize()
+        assert out.dtype == F16
+        _close(out, ref_q, what="fp16 over fp8, dequantised cache")
+        err = (out.float().cpu().squeeze(1) - ref).abs()
+        assert (err <= 6e-2 + 6e-2 * ref.abs()).all()
     # the step's token, appended by the quantising decode append with fp16 rows
     k8a, v8a, ksa, vsa = k8.clone(), v8.clone(), ks.clone(), vs.clone()
     mi.ops.kv_append_decode_fp8(case.k_new, case.v_new, k8a, v8a, ksa, vsa, case.block_table, case.kv_lens, headroom=2.0)
