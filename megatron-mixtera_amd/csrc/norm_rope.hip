@@ -728,11 +728,14 @@ extern "C" int mi_qkv_key_append(
   p.kc = (uint16_t*)k_cache; p.vc = (uint16_t*)v_cache; p.chunk_elems = kv_stride_chunk; p.tok_elems = kv_stride_tok;
   p.tok_chunk = token_to_chunk_idx; p.tok_local = token_to_local_pos;
   p.T = T; p.Hkv = Hkv; p.norm = norm_kind; p.interleaved = rotary_interleaved; p.eps = eps; p.mscale = mscale;
-  // Two tokens where their key heads fill the workgroup's lanes, in one pass, else four.  Short prompts are bound by the chain
-  // of trips and have fewer workgroups than the chip takes at once (the step of one prompt of 500 tokens, 32 / 8 heads of 128,
-  // 25.3 -> 24.2 us, four of 300 32.4 -> 30.6; 8 x 1 000 and 6 x 4 000 level); with lanes idle two are level at best (8 heads of 64: 4 x 800
-  // 37.7 / 38.8), and one token works its angles out on half of the lanes (4 x 500 40.8, 40.0 with two, 41.8).
-  const int tokens = 2 * Hkv * (head_dim / 8) >= 256 ? 2 : kKeyTokens;
+  // Two tokens where their key heads fill the workgroup's lanes, in one pass, and the call is short, else four.  Short prompts are
+  // bound by the chain of trips and have fewer workgroups than the chip takes at once; long ones by how many workgroups there
+  // are, unless two tokens' heads fill the lanes twice.  Us, four tokens -> two: 32/8 heads of 128, 500 tokens 10.3 -> 9.1, 2 047
+  // 12.9 -> 12.0, 5 000 17.6 / 18.4, 30 000 59.5 / 60.7; 32/16 of 64, 2 047 12.1 -> 11.8, 12 000 25.1 / 28.1; 32/32 of 128, 500 16.8 ->
+  // 12.9, 12 000 93 -> 88.  With lanes idle two are level at best (8 heads of 64, 1 000 tokens 9.4 / 9.7), and one token works
+  // its angles out on half of the lanes (the step of 4 x 500, 32/8 of 128: 40.8, 40.0 with two, 41.8).
+  const int lanes = 2 * Hkv * (head_dim / 8);
+  const int tokens = lanes >= 512 || (lanes >= 256 && T <= 3072) ? 2 : kKeyTokens;
   const dim3 grid((T + tokens - 1) / tokens);
   hipStream_t st = (hipStream_t)stream;
   const bool f16 = dtype == MI_DTYPE_FP16;

@@ -159,11 +159,11 @@ def test_norm_weights_off_16_bytes_take_the_separate_calls(mi, dev):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("d,hkv", [(128, 7), (128, 8), (128, 17), (64, 15), (64, 16)])
-@pytest.mark.parametrize("T", [1, 2, 3, 4, 5, 9])
+@pytest.mark.parametrize("d,hkv", [(128, 7), (128, 8), (128, 17), (64, 15), (64, 16), (128, 32)])
+@pytest.mark.parametrize("T", [1, 2, 3, 4, 5, 9, 3072, 3073])
 def test_keys_do_not_depend_on_the_tokens_beside_them(mi, dev, dtype, d, hkv, T):
-    """A workgroup takes two tokens or four, by the heads: either side of that line, whole and partial workgroups give the
-    bits of each token appended by itself."""
+    """A workgroup takes two tokens or four, by the heads and the call's length: either side of those lines, whole and partial
+    workgroups give the bits of each token appended by itself."""
     (mixed, pos, chunk, local, *_), (_, kw), caches, longest = _batch(mi, dev, (T,), hkv, hkv, d, dtype, 0, d + T)
     emb = mi.synthetic.rotary_angle_table(longest, d, base=10000.0).to(dev)
     common = dict(num_query_heads=hkv, num_kv_heads=hkv, norm="rms", k_weight=kw, rotary_emb=emb)
