@@ -564,7 +564,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleParams p) 
         const float f = (mx - x) * inv_w;
         return (int)fminf(fmaxf(f, 0.f), 255.f);  // (NaN, as inf * 0, becomes 0)
       };
-      auto weight_of = [&](float x) -> uint64_t { return by_count ? (uint64_t)1 : mass_of(x, neg_mx); };
+      // (a NaN, which bin 0 takes, counts for nothing: only ones with their sign set get here, below every number)
+      auto weight_of = [&](float x) -> uint64_t { return by_count ? (uint64_t)(x == x) : mass_of(x, neg_mx); };
       if (tid < 256) hist[tid] = 0;
       if (tid == 0) member_count = 0;
       __syncthreads();
