@@ -38,7 +38,7 @@ MEASURED_HBM_TRAFFIC_BYTES = {
     "cfg2": 1_226_700_000, "cfg2_step": 1_214_700_000, "cfg4": 8_726_100_000, "cfg4_step": 8_633_200_000,
     "cfg5": 9_070_100_000, "cfg5_step": 9_045_200_000,
     # the mixed step: tile kernel, stream kernel
-    "cfg3_tile": 401_800_000, "cfg3_stream": 2_195_700_000,
+    "cfg3_tile": 401_800_000, "cfg3_stream": 2_196_000_000,
     # multi-latent decode at 128 heads (reads + the partial results it writes)
     "mla_decode_h128": 452_800_000, "mla_decode_h128_long": 1_309_900_000}
 # Where each figure above was read, so that a reader of the JSON line can tell a stale constant from a fresh one:
@@ -46,7 +46,7 @@ MEASURED_HBM_TRAFFIC_BYTES = {
 _DECODE_TRAFFIC = ("profiles/decode_stream_kernels_hbm_traffic_cfg2_cfg4_cfg5.md (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, "
                    "library as of commit 18b0bde)")
 _MIXED_TRAFFIC = ("profiles/paged_prefill_woven_kernel_cfg3_mfma.md (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, library as of "
-                  "commit 18b0bde)")
+                  "commit ead4f8c)")
 _MLA_HEADS_TRAFFIC = ("profiles/paged_mla_decode_heads_kernel_h128_counters.md (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, "
                       "library as of commit 18b0bde)")
 TRAFFIC_SOURCE = {"mla_decode_h128": _MLA_HEADS_TRAFFIC, "mla_decode_h128_long": _MLA_HEADS_TRAFFIC, "cfg2": _DECODE_TRAFFIC, "cfg2_step": _DECODE_TRAFFIC, "cfg4": _DECODE_TRAFFIC,
@@ -958,7 +958,8 @@ def run_decode_config(args, mi, lib, torch, dev):
         lib.mi_profile_enable(0)
         sep_kernel_ms = sum(buf[i] for i in range(min(n_sep, args.steps))) / max(1, min(n_sep, args.steps))
         separate = {"ms_per_step": round(sep_ms, 5), "value": round(nbytes / (sep_ms * 1e-3) / 1e9, 1),
-                    "kernel": "paged_decode_stream_kernel", "kernel_ms": round(sep_kernel_ms, 5),
+                    "kernel": "decode_short_kernel" if args.workload == "cfg1" else "paged_decode_stream_kernel",
+                    "kernel_ms": round(sep_kernel_ms, 5),
                     "achieved": round(nbytes / (sep_kernel_ms * 1e-3) / 1e9, 1),
                     "frac": round(nbytes / (sep_kernel_ms * 1e-3) / 1e9 / HBM_PEAK_GBPS, 4),
                     "traffic": MEASURED_HBM_TRAFFIC_BYTES.get(args.workload),
@@ -1040,7 +1041,9 @@ def run_decode_config(args, mi, lib, torch, dev):
         "decode_steps_per_sec": round(1e3 / ms_per_step, 1),
         "roofline": {
             "bound": "hbm",
-            "kernel": "decode_step_stream_kernel" if one_kernel else "paged_decode_stream_kernel",
+            # (cfg1's four requests of up to 1 024 tokens are few and short: the kernel of such calls takes them, not the stream)
+            "kernel": ("decode_short_kernel" if args.workload == "cfg1"
+                       else "decode_step_stream_kernel" if one_kernel else "paged_decode_stream_kernel"),
             "achieved": round(achieved, 1),
             "peak": HBM_PEAK_GBPS,
             "unit": "GB/s",

@@ -692,7 +692,8 @@ int mi_sample_from_logits(const void* logits, int64_t stride_row, int32_t logits
 /*
  * The same call with scratch of mi_sample_workspace_bytes() bytes (256-byte aligned; 0: none is used): rows are then
  * cut into parts that workgroups of their own read, in up to four launches.  Same samples, masks and cut values.  With
- * workspace == NULL it is mi_sample_from_logits, one launch.
+ * workspace == NULL it is mi_sample_from_logits, one launch.  A workspace that does not serve is an error where R is at
+ * most 128 and scratch is asked for; larger batches pass over it.
  */
 int64_t mi_sample_workspace_bytes(int32_t R, int32_t vocab, int32_t top_k, float top_p);
 

@@ -34,7 +34,7 @@
 // tile ahead: 8-byte loads set out after one barrier and are stored, converted, before the next.  Key bytes are
 // converted exactly (four instructions per eight; e4m3 is a subset of both 16-bit types) and their scale multiplies the
 // softmax scale of the tile instead.  Value bytes are converted as cheaply, times the power of two of their scale; the rest of
-// the scale, 1 to 2, goes into the exponent of the tile's probabilities and out of their sum, which is kept per tile (values
+// the scale (value_factor) goes into the exponent of the tile's probabilities and out of their sum, which is kept per tile (values
 // multiplied by their scale and rounded took 48 more vector instructions per tile; 2 x 8 000 tokens 1 081 -> 1 066 us).  At
 // head_dim 64, half the values for as many probabilities and no registers for it, values are multiplied and rounded (the factor
 // there: 12 prompts of 1 000 tokens 145 -> 148 us, two of 175-2 806 109 -> 111).  After a barrier the next keys set out before the
