@@ -324,7 +324,8 @@ static __device__ void find_crossing(const uint64_t* hist, uint64_t above, uint6
 
 static __device__ __forceinline__ void write_sample(const SampleParams& p, int r, int sample, uint32_t cut_key) {
   p.samples[r] = sample;
-  if (p.cut_out) p.cut_out[r] = cut_key ? order_key_value(cut_key) : -INFINITY;
+  // (a cut among NaNs with their sign set, below every number, filters nothing)
+  if (p.cut_out) p.cut_out[r] = cut_key > order_key(-INFINITY) ? order_key_value(cut_key) : -INFINITY;
   if (p.active_mask) {
     bool active = (int64_t)sample != p.termination_id;
     if (p.kv_off) active = active && (p.kv_off[r] + p.q_len[r] + 1 < p.out_len[r]);
@@ -562,10 +563,9 @@ __global__ __launch_bounds__(kSampleThreads) void sample_kernel(SampleParams p) 
       const float inv_w = range > 0.f ? 256.f / range : 0.f;
       auto lin_bin = [&](float x) {
         const float f = (mx - x) * inv_w;
-        return (int)fminf(fmaxf(f, 0.f), 255.f);  // (NaN, as inf * 0, becomes 0)
+        return (int)fmaxf(fminf(f, 255.f), 0.f);  // (NaN, of -inf times 0 or with its sign set: the lowest)
       };
-      // (a NaN, which bin 0 takes, counts for nothing: only ones with their sign set get here, below every number)
-      auto weight_of = [&](float x) -> uint64_t { return by_count ? (uint64_t)(x == x) : mass_of(x, neg_mx); };
+      auto weight_of = [&](float x) -> uint64_t { return by_count ? (uint64_t)1 : mass_of(x, neg_mx); };
       if (tid < 256) hist[tid] = 0;
       if (tid == 0) member_count = 0;
       __syncthreads();

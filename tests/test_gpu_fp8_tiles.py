@@ -39,7 +39,7 @@ def test_fp8_tiles(mi, dev, d, Hq, Hkv, split, dtype):
 @pytest.mark.parametrize("d", [64, 128])
 def test_value_scales_of_every_kind(mi, dev, d, bound, dtype):
     """Value scales below and above what an exact conversion takes, negative, zero, NaN and infinite ones, one to a KV head.  A finite
-    scale: the checker's result, up to roundings of the probabilities and of the products of value and scale (each 2^-9 or
+    scale: the oracle's result, up to roundings of the probabilities and of the products of value and scale (each 2^-9 or
     2^-12 of the largest, the products no finer than the type's: 2^-25, and 2^-126 for what bf16 may flush; doubled for sums).  NaN: NaN.  Infinite: not finite."""
     f16 = dtype == torch.float16
     finite = [1.0, 0.37, -0.7, 0.0, 1.9 * 2.0**-19, 1.3 * 2.0**-16, 300.0 if f16 else 1.7e30, 1.5 * 2.0**-120 if f16 else 1.1 * 2.0**120]

@@ -663,9 +663,10 @@ def test_a_top_k_above_the_count_of_numbers_keeps_them_all(mi, dev, V, dtype):
     y = _with_negative_nan(x, negative_nan).to(dev)
     numbers = (~negative_nan).sum(-1)
     for top_k in (V, V - V // 4, 13):
-        got, _ = mi.ops.sample_from_logits(y, top_k=top_k, temperature=0.8, uniform=u)
+        got, _, cut = mi.ops.sample_from_logits(y, top_k=top_k, temperature=0.8, uniform=u, return_cut=True)
         rows = ((numbers < top_k) | ((x > float("-inf")).sum(-1) <= top_k) & (top_k == V)).to(dev)
         assert torch.equal(got[rows], want[rows]), top_k
+        assert (cut[(numbers < top_k).to(dev)] == float("-inf")).all(), top_k
 
 
 def test_many_rows_under_capture_leave_the_stream_without_a_workspace(mi, dev):
