@@ -330,12 +330,12 @@ __global__ __launch_bounds__(64 * WAVES, PER_SIMD) void paged_prefill_woven_kern
       return __uint_as_float((bits & 0x7f800000u) + (factor_below_one(bits) ? 0x00800000u : 0u));
     };
     // the sign goes to the fetched bytes, in a branch of its own: as an operation of every store it takes 1.5 % of prompts
-    auto negate_values_fp8 = [&](float vscale) {
-      if (__builtin_expect(__float_as_int(vscale) >= 0, 1)) return;
+    auto negate_values_fp8 = [&](int32_t sign) {
+      if (__builtin_expect(sign >= 0, 1)) return;
 #pragma unroll
       for (int i = 0; i < NP8; ++i) vraw[i] = make_uint2(vraw[i].x ^ 0x80808080u, vraw[i].y ^ 0x80808080u);
     };
-    auto store_v_fp8 = [&](uint8_t* buf, int i, float vscale) {   // (FACTOR: times the power of two of their scale)
+    auto store_v_fp8 = [&](uint8_t* buf, int i, float vscale) {   // (FACTOR: their scale's value_pow2)
       if constexpr (!FACTOR) {
         const f32x2_t a = fp8x2_lo_to_f32(vraw[i].x), b = fp8x2_hi_to_f32(vraw[i].x);
         const f32x2_t c = fp8x2_lo_to_f32(vraw[i].y), d = fp8x2_hi_to_f32(vraw[i].y);
@@ -344,8 +344,7 @@ __global__ __launch_bounds__(64 * WAVES, PER_SIMD) void paged_prefill_woven_kern
                        pack2<F16>(c.x * vscale, c.y * vscale), pack2<F16>(d.x * vscale, d.y * vscale));
         return;
       }
-      const float pow2 = value_pow2(vscale);
-      const uint2 lo = fp8x4_to_16x4<F16>(vraw[i].x, pow2), hi = fp8x4_to_16x4<F16>(vraw[i].y, pow2);
+      const uint2 lo = fp8x4_to_16x4<F16>(vraw[i].x, vscale), hi = fp8x4_to_16x4<F16>(vraw[i].y, vscale);
       *reinterpret_cast<uint4*>(buf + f_lds + i * RPP8 * PITCH) = make_uint4(lo.x, lo.y, hi.x, hi.y);
     };
     // descriptor of a tile: its rows up to the request's last key (reads beyond return zeros)
@@ -409,6 +408,15 @@ __global__ __launch_bounds__(64 * WAVES, PER_SIMD) void paged_prefill_woven_kern
     auto tile_scale = [&](float ks) { return FP8 ? fmaxf(ks * p.scale_log2, 1.17549435e-38f) : p.scale_log2; };
     float scale_prev = p.scale_log2, scale_cur = p.scale_log2, scale_next = p.scale_log2, vscale = 1.f;
     float factor_prev = 1.f, factor_cur = 1.f;   // fp8: value_factor of the tiles whose scales are scale_prev and scale_cur
+    float factor_next = 1.f;                     // (and of the tile of `vscale`, whose sign is `vsign`'s)
+    int32_t vsign = 0;
+    auto values_scale = [&](float vs) {          // uniform; vscale: what store_v_fp8 takes
+      vscale = FACTOR ? value_pow2(vs) : vs;
+      if constexpr (FACTOR) {
+        vsign = __float_as_int(vs);
+        factor_next = value_factor(vs);
+      }
+    };
     const uint4 ones = make_uint4(ones2<F16>(), ones2<F16>(), ones2<F16>(), ones2<F16>());
     const f32x4_t zero4 = {0.f, 0.f, 0.f, 0.f};
     // per-lane starts of the fragment reads inside a tile buffer
@@ -605,8 +613,8 @@ __global__ __launch_bounds__(64 * WAVES, PER_SIMD) void paged_prefill_woven_kern
         scales_request(pc);
         if (i == 0) {
           scale_prev = scale_cur = tile_scale(uniform_float(ks_v));
-          vscale = uniform_float(vs_v);
-          factor_prev = factor_cur = value_factor(vscale);
+          values_scale(uniform_float(vs_v));
+          factor_prev = factor_cur = factor_next;
         }
       }
     }
@@ -701,7 +709,7 @@ __global__ __launch_bounds__(64 * WAVES, PER_SIMD) void paged_prefill_woven_kern
                if (e >= NVF - NP8) store_k_fp8(kst, e - (NVF - NP8));
              }
            });
-      if constexpr (FACTOR) negate_values_fp8(vscale);
+      if constexpr (FACTOR) negate_values_fp8(vsign);
       slot(std::integral_constant<int, 1>{}, Mc, ka, ka_next, va, key0 + 32,
            [&](auto first_values) {
              // this wavefront's share of key tile j+1 and of the value tiles has landed
@@ -716,7 +724,7 @@ __global__ __launch_bounds__(64 * WAVES, PER_SIMD) void paged_prefill_woven_kern
              if constexpr (FP8) {
                scale_next = tile_scale(uniform_float(ks_v));  // (of tile j+1)
                const float vscale_last = vscale;
-               vscale = uniform_float(vs_v);
+               values_scale(uniform_float(vs_v));
                scales_request(pc_next);
                fetch_fp8(kbase, off, nrec, kraw);
 #pragma unroll
@@ -751,7 +759,7 @@ __global__ __launch_bounds__(64 * WAVES, PER_SIMD) void paged_prefill_woven_kern
         scale_prev = scale_cur;
         scale_cur = scale_next;
         factor_prev = factor_cur;
-        factor_cur = value_factor(vscale);
+        factor_cur = factor_next;
       }
       ++j;
       even = BUF - even;
