@@ -329,7 +329,8 @@ __global__ __launch_bounds__(64 * WAVES, PER_SIMD) void paged_prefill_woven_kern
       const uint32_t bits = scale_bits(vscale);
       return __uint_as_float((bits & 0x7f800000u) + (factor_below_one(bits) ? 0x00800000u : 0u));
     };
-    // the sign goes to the fetched bytes, in a branch of its own: as an operation of every store it takes 1.5 % of prompts
+    // the sign goes to the fetched bytes, in a branch of its own: as an operation of every store it takes 1.6 % of prompts (six of
+    // 129-4 097 tokens 433.6 -> 440.6 us)
     auto negate_values_fp8 = [&](int32_t sign) {
       if (__builtin_expect(sign >= 0, 1)) return;
 #pragma unroll
